@@ -374,6 +374,21 @@ def decode_linear(x: torch.Tensor, weight: torch.Tensor, bias=None) -> torch.Ten
     return y.view(*shape[:-1], N)
 
 
+def _token_major_like(q):
+    """Output of an attention over (B,H,S,D) queries, laid out (B,S,H,D) so that the caller's
+    transpose back to (B,S,H*D) moves nothing."""
+    B, H, S, D = q.shape
+    return torch.empty(B, S, H, D, dtype=q.dtype, device=q.device).transpose(1, 2)
+
+
+def _extend_on_mfma(q, k_cache):
+    """Several query tokens of a 16-bit model against a cache of the same type: the matrix-core
+    kernel reads each K/V row once for all of them; the decode kernel (one workgroup a query
+    token) serves single tokens, fp32, 8-bit caches and the other head sizes."""
+    return q.shape[2] > 1 and q.shape[3] in (64, 128) and q.dtype == k_cache.dtype \
+        and q.dtype in (torch.bfloat16, torch.float16)
+
+
 def attention_prefill_cached(q, k_cache, v_cache, seq_ids, scale=None,
                              sinks=None, sliding_window: int = 0):
     """Context-encoding attention reading K/V straight from the cache rows
@@ -388,7 +403,7 @@ def attention_prefill_cached(q, k_cache, v_cache, seq_ids, scale=None,
     scale = scale if scale is not None else 1.0 / math.sqrt(q.shape[-1])
     if q.is_cuda:
         c = _require_ext("attention_prefill_cached")
-        out = torch.empty_like(q)
+        out = _token_major_like(q)
         c.flash_prefill_cached(out, q.contiguous(), k_cache, v_cache,
                                seq_ids, float(scale), int(sliding_window),
                                sinks=None if sinks is None else sinks.detach())
@@ -422,6 +437,14 @@ def attention_decode(q, k_cache, v_cache, seq_lens, seq_ids=None, scale=None,
         positions = seq_lens
     if q.is_cuda:
         c = _require_ext("attention_decode")
+        if not ring and _extend_on_mfma(q, k_cache):
+            out = _token_major_like(q)
+            if seq_ids is None:
+                seq_ids = torch.arange(B, device=q.device, dtype=torch.int32)
+            c.flash_extend(out, q.contiguous(), k_cache, v_cache, positions, seq_ids=seq_ids,
+                           scale=float(scale), window=int(sliding_window),
+                           sinks=None if sinks is None else sinks.detach())
+            return out
         Hkv = k_cache.shape[1]
         gq = Hq // max(Hkv, 1)
         if gq > 8:
@@ -626,6 +649,12 @@ def attention_decode_paged(q, k_cache, v_cache, seq_lens, block_table,
         positions = seq_lens
     if q.is_cuda:
         c = _require_ext("attention_decode_paged")
+        if _extend_on_mfma(q, k_cache):
+            out = _token_major_like(q)
+            c.flash_extend(out, q.contiguous(), k_cache, v_cache, positions,
+                           block_table=block_table, scale=float(scale),
+                           window=int(sliding_window))
+            return out
         out = torch.empty_like(q)
         c.attention_decode_paged(
             out, q.contiguous(), k_cache, v_cache,

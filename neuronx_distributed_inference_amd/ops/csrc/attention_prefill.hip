@@ -1,385 +1,585 @@
-// Causal flash-attention prefill for gfx950 (K1/K11-analog; ref
-// nkilib attention_cte called at attention_base.py:722-744 and the in-repo
-// sliding-window NKI kernel modules/sliding_window/attention.py:38-477).
+// Flash attention over many query tokens for gfx950: whole prompts (K1/K11-analog; ref
+// nkilib attention_cte called at attention_base.py:722-744 and the in-repo sliding-window
+// NKI kernel modules/sliding_window/attention.py:38-477) and portions of prompts whose
+// earlier tokens are already in the linear or paged cache.
 //
-// MFMA (16x16x32 bf16/f16) flash forward with online softmax:
-//   * workgroup = 4 waves = one 128-row Q block of one (b, hq); each wave
-//     owns 32 q rows. K/V tiles (KVBLK=32 keys) staged in LDS by the whole
-//     workgroup; V is transposed during staging so the PV B-fragments read
-//     16 contiguous bytes per lane.
-//   * all LDS tiles use padded row strides (row_bytes = data + 16) so the
-//     B-fragment column reads are bank-conflict-free (guide §6 G4: row-major
-//     [KV][128] bf16 is an up-to-16-way conflict).
-//   * P round-trips through LDS between QK^T (C layout) and PV (A layout).
-//   * causal + sliding-window masking on the fp32 scores; GQA native (the
-//     KV head is staged once for the gq query heads that share it —
-//     workgroups differ in hq but hit the same K/V through L2).
+// What bounds it: the matrix cores and, next to them, one exponential per score. Everything
+// else is kept off the vector units:
+//   * A workgroup takes 128 query rows of ONE kv head, 32 a wave. Rows are (token, head of
+//     the group) pairs, so the heads that share K and V share its tiles in LDS, a chunk of
+//     a few tokens still fills the rows, and the causal border is 128/gq tokens wide.
+//   * Scores are made transposed, S^T = K Q^T (mfma 32x32x16): a lane owns ONE query row, so
+//     the running maximum, the sum and the rescaling are plain registers (one exchange with
+//     the other half wave for the maximum of 64 keys, none for the sum until the end).
+//   * P never leaves the registers: the C layout of S^T holds, for a lane, runs of 4
+//     consecutive keys; read as the B operand of O^T = V^T P^T they are the same 16 keys in
+//     another order, and V^T is read in that order. V stays row-major in LDS: ds_read_b64_tr
+//     transposes 4 keys x 16 channels on the way to the registers.
+//   * The accumulator is rescaled only when a row's maximum grew by more than 2^8 since the
+//     last time; probabilities and sums share the stale maximum, so nothing is lost.
+//   * K and V tiles of 64 keys go straight to LDS (global_load_lds, 16 B a lane), two
+//     buffers, one barrier a tile: the next tile flies while this one is computed. Slots of
+//     16 B are XOR-swizzled on the source side so that neither the row reads of K nor the
+//     transposing reads of V meet in a bank.
 //
-// This is the correctness-first structure (guide §5 ladder step ~2-3);
-// planned upgrades: K-tile XOR swizzle (T2), async-stage split (T14),
-// double buffering, exp2 folding.
+// Rows with few tiles to share (short chunks over a long cache) are split over the keys as
+// well: fp32 partial sums per split and a small combining kernel.
+//
+// Measured (MI355X, bf16, 32 query / 8 kv heads; before: 16x16x32 tiles, P through LDS, V
+// transposed by the staging stores; several tokens over a cache: one workgroup a token):
+//   prompt of 8192, head size 128     2168 -> 617 us (891 TFLOP/s; two thirds of it is the
+//                                     matrix pipe, the rest exponentials it does not hide)
+//   prompt of 2048, head size 128/64  179 -> 54 us / 145 -> 42 us
+//   prompt of 512 / 128               40 -> 16 us / 16 -> 9 us
+//   512 tokens over 4000, linear/paged 1772 -> 62 us / 2019 -> 79 us
+//   64 tokens over 4000, linear       237 -> 31 us
+//   32 rows of 6 tokens over 2000     354 -> 47 us (a verification step)
+//   1 row of 2 tokens over 2000       28 -> 17 us
+// No size was found at which several tokens are better off one by one.
 
 #include "common.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+namespace {
 
-template <typename T> struct MfmaTraits;
-template <> struct MfmaTraits<__hip_bfloat16> {
-    using vec8 = bf16x8;
-    static DEV_INLINE f32x4 mfma(vec8 a, vec8 b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+typedef __bf16 fa_bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 fa_f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 fa_bf16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 fa_f16x4 __attribute__((ext_vector_type(4)));
+typedef short fa_s16x4 __attribute__((ext_vector_type(4)));
+typedef float fa_f32x16 __attribute__((ext_vector_type(16)));
+
+template <typename T> struct FaTraits;
+template <> struct FaTraits<__hip_bfloat16> {
+    using vec8 = fa_bf16x8;
+    using vec4 = fa_bf16x4;
+    using elem = __bf16;
+    static DEV_INLINE fa_f32x16 mfma(vec8 a, vec8 b, fa_f32x16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }
 };
-template <> struct MfmaTraits<__half> {
-    using vec8 = f16x8;
-    static DEV_INLINE f32x4 mfma(vec8 a, vec8 b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+template <> struct FaTraits<__half> {
+    using vec8 = fa_f16x8;
+    using vec4 = fa_f16x4;
+    using elem = _Float16;
+    static DEV_INLINE fa_f32x16 mfma(vec8 a, vec8 b, fa_f32x16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
     }
 };
 
-constexpr int QBLK = 128;       // q rows per workgroup
-constexpr int WQ = 32;          // q rows per wave
-constexpr int KVBLK = 64;       // keys per LDS tile
-constexpr float NEG_INF = -1e30f;
+constexpr int QROWS = 128;      // query rows of a workgroup
+constexpr int KT = 64;          // keys of a tile
+constexpr float FA_GROWTH = 8.f;  // log2 growth of a maximum that is put off
 
-template <typename T, int D>
-__global__ __launch_bounds__(256, 2) void flash_prefill_kernel(
-    T* __restrict__ out,       // (B, Hq, S, D)
-    const T* __restrict__ q,   // (B, Hq, S, D)
-    const T* __restrict__ k,   // (B, Hkv, S, D)
-    const T* __restrict__ v,   // (B, Hkv, S, D)
-    const float scale, const int window,
-    const int Hq, const int Hkv, const int S,
-    const float* __restrict__ sinks,   // (Hq,) learned sink logits or null
-    const int* __restrict__ seq_ids,   // non-null: K/V live in the KV cache
-    const int Smax) {                  // cache row capacity (= S when direct)
-    using MT = MfmaTraits<T>;
-    using vec8 = typename MT::vec8;
-    constexpr int DI = D / 16;       // O col fragments per wave
-    constexpr int KS = D / 32;       // K-dim steps for QK^T
-    // padded LDS row strides (bytes)
-    constexpr int K_STRIDE = D * 2 + 16;
-    constexpr int VT_STRIDE = KVBLK * 2 + 16;
-    constexpr int P_STRIDE = KVBLK * 2 + 16;
-    // XOR swizzle on the V^T image in-row offset, keyed by the V^T row (the
-    // head-dim d). The transpose staging writes one b16 per (d, key) from 16
-    // threads whose d differ by 8 at byte stride VT_STRIDE (a multiple of
-    // 16B) — all on one bank without this (measured: SQ_LDS_BANK_CONFLICT
-    // 2.5x SQ_BUSY_CYCLES). The swizzle spreads them over 8 bank slots; the
-    // b128 PV reads stay 16B-aligned and at worst 2-way.
-#define VT_SWZ(row) ((((row) >> 3) & 7) << 4)
+// the other half wave's value
+DEV_INLINE float half_swap(float x) {
+    const unsigned u = __builtin_bit_cast(unsigned, x);
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return __builtin_bit_cast(float, (threadIdx.x & 32) ? r[0] : r[1]);
+}
 
-    __shared__ __attribute__((aligned(16))) char smem[
-        KVBLK * K_STRIDE + D * VT_STRIDE + 4 * WQ * P_STRIDE];
-    char* k_lds = smem;
-    char* vt_lds = smem + KVBLK * K_STRIDE;
-    char* p_lds_all = vt_lds + D * VT_STRIDE;
+// 16 bytes a lane from `src` to the 1 KB of LDS at the wave-uniform `dst`. Written out, because
+// the compiler puts a wait for every such load in flight before each transposing LDS read, of
+// any buffer. It has no register result; the kernel waits (vmcnt) before the barrier that
+// hands the tile over.
+DEV_INLINE void fa_load_lds(const void* src, unsigned dst) {
+    const unsigned at = __builtin_amdgcn_readfirstlane(dst);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 :: "s"(at), "v"(src) : "memory", "m0");
+}
 
-    const int qblk = blockIdx.x;
-    const int hq = blockIdx.y;
-    const int b = blockIdx.z;
-    const int hkv = hq / (Hq / Hkv);
+struct FaArgs {
+    const int* positions;    // (B, S) position of each query (-1: padding), or null: token index
+    const int* seq_ids;      // (B,) cache row, or null: batch row
+    const int* block_table;  // (B, max_blocks), paged caches
+    const float* sinks;      // (Hq,) or null
+    float* o_part;           // (nsplit, B, Hq, S, D), nsplit > 1
+    float* ml_part;          // (nsplit, B, Hq, S, 2)
+    long ob, oh, os;         // element strides of out over (b, head, token)
+    float scale;
+    int window, B, Hq, Hkv, S, cap;   // cap: key rows of a sequence
+    int Smax, block_size, max_blocks; // linear row capacity / paged geometry
+    int nsplit, nqt, clamp_rows;      // clamp_rows: a negative seq_id reads row 0 (else: no keys)
+};
+
+template <typename T, int D, bool PAGED>
+__global__ __launch_bounds__(256, 2) void flash_kernel(
+    T* __restrict__ out, const T* __restrict__ q, const T* __restrict__ k,
+    const T* __restrict__ v, const FaArgs a) {
+    using FT = FaTraits<T>;
+    using vec8 = typename FT::vec8;
+    using vec4 = typename FT::vec4;
+    constexpr int ROWB = D * 2;            // bytes of a key row
+    constexpr int SLOTS = ROWB / 16;       // 16-byte slots of a row: 16 or 8
+    constexpr int RPI = 64 / SLOTS;        // rows that one wave-wide load stages: 4 or 8
+    constexpr int NLD = KT / 4 / RPI;      // loads a wave issues per tile and operand
+    constexpr int TILE_B = KT * ROWB;
+    constexpr int NKS = D / 16;            // k-steps of Q K^T
+    constexpr int NDB = D / 32;            // 32-channel blocks of the output
+
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    // [2 buffers][K tile | V tile], then block bounds and the paged tiles' bad-row marks
+    int* s_bounds = reinterpret_cast<int*>(smem + 4 * TILE_B);
+    int* s_bad = s_bounds + 8;             // [2][1 + KT], paged only
+
+    const int NH = a.B * a.Hkv;
+    int hg, rest;
+    {
+        // kv heads go round the 8 XCDs, so that one L2 serves a head's K and V; the longest
+        // (last) rows of all heads start first
+        const int id = blockIdx.x;
+        if ((NH & 7) == 0) {
+            const int per = NH >> 3, t = id >> 3;
+            hg = (id & 7) + 8 * (t % per);
+            rest = t / per;
+        } else {
+            hg = id % NH;
+            rest = id / NH;
+        }
+    }
+    const int qt = a.nqt - 1 - rest / a.nsplit;
+    const int split = rest % a.nsplit;
+    const int b = hg / a.Hkv, hkv = hg % a.Hkv;
+    const int gq = a.Hq / a.Hkv;
+    const int R = gq * a.S;
+
     const int lane = threadIdx.x & 63;
     const int wid = threadIdx.x >> 6;
-    char* p_lds = p_lds_all + wid * WQ * P_STRIDE;
+    const int half = lane >> 5;
+    const int r_own = qt * QROWS + wid * 32 + (lane & 31);
+    const int rr = min(r_own, R - 1);
+    const int token = rr / gq;
+    const int head = hkv * gq + rr % gq;
+    const int row = a.seq_ids ? a.seq_ids[b] : b;
 
-    const int q_lo = qblk * QBLK;
-    const int wq_lo = q_lo + wid * WQ;          // this wave's first q row
-    const int wq_hi = min(wq_lo + WQ, S) - 1;   // last valid q row (abs)
+    int qpos = a.positions ? a.positions[(long)b * a.S + token] : token;
+    if (r_own >= R || (row < 0 && !a.clamp_rows)) qpos = -1;
+    qpos = min(qpos, a.cap - 1);
 
-    const long q_base = (((long)b * Hq + hq) * S) * D;
-    // seq_ids[b] can be -1 (ModelWrapper pads CTE batches with seq_id -1);
-    // clamp to row 0 so the cached path never reads before the allocation —
-    // pad-row outputs are discarded by the host anyway.
-    const long kv_row = (seq_ids != nullptr) ? max((long)seq_ids[b], 0L) : b;
-    const long kv_base = ((kv_row * Hkv + hkv) * (long)Smax) * D;
-
-    // ---- Q fragments into registers (A layout: row = lane&15, k-elems
-    // (lane>>4)*8 .. +8, per (qi, ks)) ----
-    vec8 q_frag[2][KS];
-    const int qa_row = lane & 15;
-    const int qa_off = (lane >> 4) * 8;
+    // bounds of the wave's and the workgroup's valid rows
+    int wmin = qpos < 0 ? 0x7fffffff : qpos, wmax = qpos;
 #pragma unroll
-    for (int qi = 0; qi < 2; ++qi) {
+    for (int off = 16; off > 0; off >>= 1) {
+        wmin = min(wmin, __shfl_xor(wmin, off, WAVE_SIZE));
+        wmax = max(wmax, __shfl_xor(wmax, off, WAVE_SIZE));
+    }
+    if (lane == 0) {
+        s_bounds[wid * 2] = wmin;
+        s_bounds[wid * 2 + 1] = wmax;
+    }
+    // Q as the B operand: column = the lane's row, 8 channels at half*8 of each k-step
+    vec8 qf[NKS];
+    {
+        const T* qp = q + (((long)b * a.Hq + head) * a.S + token) * D + half * 8;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const int row = min(wq_lo + qi * 16 + qa_row, S - 1);
-            q_frag[qi][ks] = *reinterpret_cast<const vec8*>(
-                q + q_base + (long)row * D + ks * 32 + qa_off);
-        }
+        for (int ks = 0; ks < NKS; ++ks) qf[ks] = *reinterpret_cast<const vec8*>(qp + ks * 16);
+    }
+    // landed before the first tile is on its way: no wait for them inside the loop
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) asm volatile("" : "+v"(qf[ks]));
+    __syncthreads();
+    int bmin = s_bounds[0], bmax = s_bounds[1];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+        bmin = min(bmin, s_bounds[w * 2]);
+        bmax = max(bmax, s_bounds[w * 2 + 1]);
+    }
+    bmin = __builtin_amdgcn_readfirstlane(bmin);
+    bmax = __builtin_amdgcn_readfirstlane(bmax);
+    wmin = __builtin_amdgcn_readfirstlane(wmin);
+    wmax = __builtin_amdgcn_readfirstlane(wmax);
+    const int C = a.window < 0 ? -a.window : 0;
+    int lo = 0;
+    if (a.window > 0) lo = max(0, bmin - a.window + 1);
+    else if (C) lo = (bmin / C) * C;
+    if (bmax < 0) lo = 0;
+    // the wave's own first visible key, and from where on every key is inside all its windows
+    const int w_lo = a.window > 0 ? max(0, wmin - a.window + 1) : (C && wmax >= 0 ? (wmin / C) * C : 0);
+    const int w_in = a.window > 0 ? wmax - a.window + 1 : (C && wmax >= 0 ? (wmax / C) * C : 0);
+
+    // the lane's own first visible key
+    const int key_lo = a.window > 0 ? qpos - a.window + 1 : (C ? (qpos / C) * C : 0);
+
+    int t_lo = lo / KT, t_hi = (bmax + KT) / KT;      // tiles [t_lo, t_hi); none when bmax < 0
+    if (a.nsplit > 1) {
+        const int per = (t_hi - t_lo + a.nsplit - 1) / a.nsplit;
+        t_lo += split * per;
+        t_hi = min(t_hi, t_lo + per);
     }
 
-    f32x4 o_acc[2][DI];
+    const float c0 = a.scale * 1.4426950408889634f;   // scores in log2 units
+    const bool flip = c0 < 0.f;
+    const float c = flip ? -c0 : c0;
+
+    // ---- staging: this lane's rows and source slots ----
+    const int st_row = wid * (KT / 4) + lane / SLOTS;  // + i * RPI
+    const int st_p = lane % SLOTS;
+    const long lin = PAGED ? 0 : ((long)max(row, 0) * a.Hkv + hkv) * (long)a.Smax * D;
+    auto swz_k = [](int r) { return D == 128 ? (r & 15) : ((r >> 1) & 7); };
+    auto swz_v = [](int r) { return D == 128 ? ((r & 3) << 2) : (((r >> 1) & 1) << 2); };
+    const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
+    int blk[NLD];                                      // paged: the next tile's page numbers
+    auto load_blocks = [&](int t) {
+        if constexpr (PAGED) {
 #pragma unroll
-    for (int qi = 0; qi < 2; ++qi)
-#pragma unroll
-        for (int di = 0; di < DI; ++di) o_acc[qi][di] = {0.f, 0.f, 0.f, 0.f};
-    // per-lane softmax state: 4 rows per C fragment, 2 qi fragments
-    float m_run[2][4], l_run[2][4];
-#pragma unroll
-    for (int qi = 0; qi < 2; ++qi)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            m_run[qi][r] = NEG_INF;
-            l_run[qi][r] = 0.f;
+            for (int i = 0; i < NLD; ++i) {
+                const int key = min(t * KT + st_row + i * RPI, bmax);
+                blk[i] = a.block_table[(long)b * a.max_blocks + key / a.block_size];
+            }
         }
-
-    const int kv_hi = min(S, q_lo + QBLK);  // causal: no keys beyond block end
-    int kv_start = 0;
-    if (window > 0) kv_start = max(0, (q_lo - window + 1) / KVBLK * KVBLK);
-    // window < 0: chunked attention (chunk C = -window); the block's first
-    // query bounds the earliest reachable row at its chunk start
-    else if (window < 0) kv_start = (q_lo / -window) * -window / KVBLK * KVBLK;
-
-    // Staging note: occupancy (not staging latency) is the binding
-    // constraint — keep live state minimal so 2 waves/SIMD fit (the
-    // register-prefetch variant measured null because it pushed the kernel
-    // to 329 regs = 1 wave/SIMD).
-    constexpr int NIT = (KVBLK * D) / (256 * 8);
-    const int st_row = (threadIdx.x * 8) / D;        // this thread's key row
-    const int st_d = (threadIdx.x * 8) % D;          // and d offset
-    const int row_step = (256 * 8) / D;
-
-    for (int k0 = kv_start; k0 < kv_hi; k0 += KVBLK) {
+    };
+    auto stage = [&](int t, int buf) {
+        const unsigned kd = lds0 + buf * 2 * TILE_B + wid * (TILE_B / 4);
+        const unsigned vd = kd + TILE_B;
 #pragma unroll
-        for (int it = 0; it < NIT; ++it) {
-            const int row = st_row + it * row_step;
-            const int krow = min(k0 + row, S - 1);
-            Vec8<T> kv8 = load_vec8(k + kv_base + (long)krow * D + st_d);
-            Vec8<T> vv8 = load_vec8(v + kv_base + (long)krow * D + st_d);
-            *reinterpret_cast<int4*>(k_lds + row * K_STRIDE + st_d * 2) =
-                *reinterpret_cast<int4*>(kv8.v);
-#pragma unroll
-            for (int j = 0; j < 8; ++j)  // transpose: V^T[d+j][row]
-                *reinterpret_cast<T*>(
-                    vt_lds + (st_d + j) * VT_STRIDE + ((row * 2) ^ VT_SWZ(st_d + j))) =
-                    vv8.v[j];
+        for (int i = 0; i < NLD; ++i) {
+            const int r = st_row + i * RPI;
+            const int key = min(t * KT + r, bmax);
+            long off;
+            if constexpr (PAGED)
+                off = (((long)max(blk[i], 0) * a.block_size + key % a.block_size) * a.Hkv + hkv) * D;
+            else
+                off = lin + (long)key * D;
+            const T* ks = k + off + (st_p ^ swz_k(r)) * 8;
+            const T* vs = v + off + (st_p ^ swz_v(r)) * 8;
+            fa_load_lds(ks, kd + i * 1024);
+            fa_load_lds(vs, vd + i * 1024);
         }
+        if constexpr (PAGED) {
+            // rows without a page are marked; their values are cleared once they have landed
+            if (st_p == 0) {
+#pragma unroll
+                for (int i = 0; i < NLD; ++i) {
+                    const bool bad = blk[i] < 0;
+                    s_bad[buf * (KT + 1) + 1 + st_row + i * RPI] = bad;
+                    if (bad) s_bad[buf * (KT + 1)] = t;
+                }
+            }
+        }
+    };
+
+    fa_f32x16 o[NDB];
+#pragma unroll
+    for (int i = 0; i < NDB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+    float m = -INFINITY, l = 0.f;      // m: the maximum in use (log2 units); l: this half's sum
+
+    // fragment addresses within a tile
+    const int ka_row = lane & 31;
+    const int vi = lane & 15;
+    const int va_row = half * 4 + (vi >> 2);
+    const int va_d = ((lane >> 4) & 1) * 16 + (vi & 3) * 4;
+
+    if constexpr (PAGED) {
+        if (threadIdx.x < 2) s_bad[threadIdx.x * (KT + 1)] = -1;
         __syncthreads();
-
-        if (k0 <= wq_hi) {  // this wave still has un-masked keys in the tile
-            // ---- QK^T: S_tile[32q][KVBLK k] as 2 x KVBLK/16 fragments ----
-            constexpr int KI = KVBLK / 16;
-            f32x4 s_frag[2][KI];
+    }
+    if (t_lo < t_hi) {
+        load_blocks(t_lo);
+        stage(t_lo, 0);
+        if (t_lo + 1 < t_hi) load_blocks(t_lo + 1);
+    }
+    for (int t = t_lo; t < t_hi; ++t) {
+        const int buf = (t - t_lo) & 1;
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        if constexpr (PAGED) {
+            // a row without a page: its V row (whatever page 0 holds) must not reach 0 * V
 #pragma unroll
-            for (int qi = 0; qi < 2; ++qi)
-#pragma unroll
-                for (int ki = 0; ki < KI; ++ki) {
-                    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int ks = 0; ks < KS; ++ks) {
-                        // B fragment: col = key (lane&15), elems = dims
-                        const vec8 kb = *reinterpret_cast<const vec8*>(
-                            k_lds + (ki * 16 + (lane & 15)) * K_STRIDE +
-                            (ks * 32 + (lane >> 4) * 8) * 2);
-                        acc = MT::mfma(q_frag[qi][ks], kb, acc);
-                    }
-                    s_frag[qi][ki] = acc;
-                }
-
-            // ---- mask + online softmax (C layout: col=lane&15 is the key,
-            // row=(lane>>4)*4+reg is the q) ----
-            // Tiles fully below the causal diagonal (and inside the window /
-            // sequence bounds) skip every per-element mask op — that is most
-            // tiles, and the masking VALU was a large share of wave cycles.
-            const bool full_tile =
-                (k0 + KVBLK - 1 <= wq_lo) && (k0 + KVBLK <= S)
-                && (window <= 0 || k0 >= wq_lo + WQ - window)
-                && (window >= 0 || k0 >= ((wq_lo + WQ - 1) / -window) * -window);
-            float p_new[2][4];  // per-qi per-reg row max of this tile
-#pragma unroll
-            for (int qi = 0; qi < 2; ++qi) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int q_abs = wq_lo + qi * 16 + (lane >> 4) * 4 + r;
-                    float mx = NEG_INF;
-                    if (full_tile) {
-#pragma unroll
-                        for (int ki = 0; ki < KI; ++ki) {
-                            const float sv = s_frag[qi][ki][r] * scale;
-                            s_frag[qi][ki][r] = sv;
-                            mx = fmaxf(mx, sv);
-                        }
-                    } else
-#pragma unroll
-                    for (int ki = 0; ki < KI; ++ki) {
-                        const int k_abs = k0 + ki * 16 + (lane & 15);
-                        float sv = s_frag[qi][ki][r] * scale;
-                        const bool ok = (k_abs <= q_abs) && (k_abs < S) && (q_abs < S)
-                            && (window <= 0 || k_abs > q_abs - window)
-                            && (window >= 0 || k_abs >= (q_abs / -window) * -window);
-                        sv = ok ? sv : NEG_INF;
-                        s_frag[qi][ki][r] = sv;
-                        mx = fmaxf(mx, sv);
-                    }
-                    // row max across the 16 key-columns
-#pragma unroll
-                    for (int off = 8; off > 0; off >>= 1)
-                        mx = fmaxf(mx, __shfl_xor(mx, off, WAVE_SIZE));
-                    p_new[qi][r] = mx;
-                }
+            for (int i = 0; i < NLD; ++i) {
+                const int r = st_row + i * RPI;
+                if (s_bad[buf * (KT + 1) + 1 + r])
+                    *reinterpret_cast<int4*>(smem + buf * 2 * TILE_B + TILE_B + r * ROWB + st_p * 16)
+                        = int4{0, 0, 0, 0};
             }
-#pragma unroll
-            for (int qi = 0; qi < 2; ++qi) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float m_new = fmaxf(m_run[qi][r], p_new[qi][r]);
-                    const float corr = __expf(m_run[qi][r] - m_new);
-                    float row_sum = 0.f;
-                    if (full_tile) {
-#pragma unroll
-                        for (int ki = 0; ki < KI; ++ki) {
-                            const float p = __expf(s_frag[qi][ki][r] - m_new);
-                            s_frag[qi][ki][r] = p;
-                            row_sum += p;
-                        }
-                    } else
-#pragma unroll
-                    for (int ki = 0; ki < KI; ++ki) {
-                        const float sv = s_frag[qi][ki][r];
-                        const float p = (sv <= NEG_INF) ? 0.f : __expf(sv - m_new);
-                        s_frag[qi][ki][r] = p;
-                        row_sum += p;
-                    }
-#pragma unroll
-                    for (int off = 8; off > 0; off >>= 1)
-                        row_sum += __shfl_xor(row_sum, off, WAVE_SIZE);
-                    l_run[qi][r] = l_run[qi][r] * corr + row_sum;
-                    m_run[qi][r] = m_new;
-                    // rescale O rows
-#pragma unroll
-                    for (int di = 0; di < DI; ++di)
-                        o_acc[qi][di][r] *= corr;
-                }
-            }
-
-            // ---- P -> LDS (bf16, A-layout-readable padded rows) ----
-#pragma unroll
-            for (int qi = 0; qi < 2; ++qi)
-#pragma unroll
-                for (int ki = 0; ki < KI; ++ki)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int qrow = qi * 16 + (lane >> 4) * 4 + r;
-                        const int kcol = ki * 16 + (lane & 15);
-                        *reinterpret_cast<T*>(p_lds + qrow * P_STRIDE + kcol * 2) =
-                            VecTraits<T>::from_float(s_frag[qi][ki][r]);
-                    }
-            // lgkmcnt(0): this wave's P writes land before its own reads.
-            // P is per-wave LDS so no workgroup barrier is needed; the
-            // "memory" clobber keeps the compiler from hoisting the reads.
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (t + 1 < t_hi) {
+            stage(t + 1, buf ^ 1);
+            if (t + 2 < t_hi) load_blocks(t + 2);
+        }
+        const int k0 = t * KT;
+        if (k0 > wmax || k0 + KT <= w_lo) continue;     // nothing here for this wave
+        const char* kb = smem + buf * 2 * TILE_B;
+        const char* vb = kb + TILE_B;
 
-            // ---- PV: O[32q][D] += P[32q][KVBLK] * V[KVBLK][D], in 32-key
-            // chunks (one A fragment per chunk) ----
+        fa_f32x16 s[2];
 #pragma unroll
-            for (int kc2 = 0; kc2 < KVBLK / 32; ++kc2) {
+        for (int n = 0; n < 2; ++n) {
 #pragma unroll
-                for (int qi = 0; qi < 2; ++qi) {
-                    const vec8 pa = *reinterpret_cast<const vec8*>(
-                        p_lds + (qi * 16 + (lane & 15)) * P_STRIDE +
-                        (kc2 * 32 + (lane >> 4) * 8) * 2);
+            for (int r = 0; r < 16; ++r) s[n][r] = 0.f;
 #pragma unroll
-                    for (int di = 0; di < DI; ++di) {
-                        const int vrow = di * 16 + (lane & 15);
-                        const vec8 vb = *reinterpret_cast<const vec8*>(
-                            vt_lds + vrow * VT_STRIDE +
-                            (((kc2 * 32 + (lane >> 4) * 8) * 2) ^ VT_SWZ(vrow)));
-                        o_acc[qi][di] = MT::mfma(pa, vb, o_acc[qi][di]);
-                    }
-                }
+            for (int ks = 0; ks < NKS; ++ks) {
+                const int r = n * 32 + ka_row;
+                const vec8 ka = *reinterpret_cast<const vec8*>(
+                    kb + r * ROWB + (((ks * 2 + half) ^ swz_k(r)) << 4));
+                s[n] = FT::mfma(ka, qf[ks], s[n]);
             }
         }
-        __syncthreads();  // compute done before the next write_tile overwrites
+        // four reads ahead of the products, not one (what the compiler does by itself)
+        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+        for (int i = 0; i < 2 * NKS - 4; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+        if (flip) {
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[n][r] = -s[n][r];
+        }
+        bool masked = (k0 + KT - 1 > wmin) || (k0 < w_in);
+        if constexpr (PAGED) masked = masked || s_bad[buf * (KT + 1)] == t;
+        if (masked) {
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int kk = n * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+                    bool ok = k0 + kk <= qpos && k0 + kk >= key_lo;
+                    if constexpr (PAGED) ok = ok && !s_bad[buf * (KT + 1) + 1 + kk];
+                    s[n][r] = ok ? s[n][r] : -INFINITY;
+                }
+        }
+        float mx = s[0][0];
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[n][r]);
+        mx = fmaxf(mx, half_swap(mx)) * c;
+        if (__any(mx > m + FA_GROWTH || (m == -INFINITY && mx > m))) {
+            const float mn = fmaxf(m, mx);
+            const float f = m == -INFINITY ? 0.f : exp2f(m - mn);
+            m = mn;
+            l *= f;
+#pragma unroll
+            for (int i = 0; i < NDB; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[i][r] *= f;
+        }
+        const float mu = m == -INFINITY ? 0.f : m;      // a row that has seen no key yet
+        vec8 p[4];
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float e = __builtin_amdgcn_exp2f(fmaf(s[n][r], c, -mu));
+                l += e;
+                p[n * 2 + (r >> 3)][r & 7] = (typename FT::elem)e;
+            }
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int db = 0; db < NDB; ++db) {
+                vec8 va;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int r = kt * 16 + j * 8 + va_row;
+                    const int d = db * 32 + va_d;
+                    const char* at = vb + r * ROWB + (((d >> 3) ^ swz_v(r)) << 4) + (d & 7) * 2;
+                    const fa_s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (__attribute__((address_space(3))) fa_s16x4*)at);
+                    const vec4 y = __builtin_bit_cast(vec4, x);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) va[j * 4 + e] = y[e];
+                }
+                o[db] = FT::mfma(va, p[kt], o[db]);
+            }
+        __builtin_amdgcn_sched_group_barrier(0x100, 8, 1);
+#pragma unroll
+        for (int i = 0; i < 4 * NDB - 4; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 4, 1);
     }
 
-    // ---- epilogue: normalize and store ----
+    // ---- epilogue: rows of 4 channels from 8*(r>>2) + 4*half ----
+    l += half_swap(l);
+    if (r_own >= R) return;
+    if (qpos < 0) {                    // padding: tiles that are whole for the others ran unmasked
+        m = -INFINITY;
+        l = 0.f;
 #pragma unroll
-    for (int qi = 0; qi < 2; ++qi) {
+        for (int i = 0; i < NDB; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int q_abs = wq_lo + qi * 16 + (lane >> 4) * 4 + r;
-            if (q_abs >= S) continue;
-            float l_tot = l_run[qi][r];
-            if (sinks != nullptr)  // sink joins the denominator only
-                l_tot += __expf(sinks[hq] - m_run[qi][r]);
-            const float inv = (l_tot > 0.f) ? 1.f / l_tot : 0.f;
-#pragma unroll
-            for (int di = 0; di < DI; ++di) {
-                const int dcol = di * 16 + (lane & 15);
-                out[q_base + (long)q_abs * D + dcol] =
-                    VecTraits<T>::from_float(o_acc[qi][di][r] * inv);
-            }
+            for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+    }
+    if (a.nsplit > 1) {
+        const long at = (((long)split * a.B + b) * a.Hq + head) * a.S + token;
+        if (half == 0) {
+            a.ml_part[at * 2] = m;
+            a.ml_part[at * 2 + 1] = l;
         }
+        if (m == -INFINITY) return;                     // nothing seen: the weight is 0
+        float* po = a.o_part + at * D;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *reinterpret_cast<float4*>(po + db * 32 + 8 * g + 4 * half) =
+                    float4{o[db][g * 4], o[db][g * 4 + 1], o[db][g * 4 + 2], o[db][g * 4 + 3]};
+        return;
+    }
+    if (a.sinks != nullptr && m != -INFINITY)           // a sink joins the denominator only
+        l += exp2f(a.sinks[head] * 1.4426950408889634f - m);
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    T* po = out + b * a.ob + head * a.oh + token * a.os;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            vec4 y;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = (typename FT::elem)(o[db][g * 4 + e] * inv);
+            *reinterpret_cast<vec4*>(po + db * 32 + 8 * g + 4 * half) = y;
+        }
+}
+
+// out row = sum over splits of 2^(m_i - m) o_i / l; a wave a row
+template <typename T, int D>
+__global__ __launch_bounds__(256) void flash_combine_kernel(T* __restrict__ out, const FaArgs a) {
+    const long rows = (long)a.B * a.Hq * a.S;
+    const long rowid = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (rowid >= rows) return;
+    const int lane = threadIdx.x & 63;
+    const int token = (int)(rowid % a.S);
+    const int head = (int)(rowid / a.S % a.Hq);
+    const int b = (int)(rowid / a.S / a.Hq);
+    float m = -INFINITY;
+    for (int i = 0; i < a.nsplit; ++i) m = fmaxf(m, a.ml_part[(i * rows + rowid) * 2]);
+    constexpr int PER = D / 64;
+    float acc[PER], L = 0.f;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) acc[j] = 0.f;
+    if (m != -INFINITY) {
+        for (int i = 0; i < a.nsplit; ++i) {
+            const float mi = a.ml_part[(i * rows + rowid) * 2];
+            if (mi == -INFINITY) continue;
+            const float f = exp2f(mi - m);
+            L += f * a.ml_part[(i * rows + rowid) * 2 + 1];
+#pragma unroll
+            for (int j = 0; j < PER; ++j) acc[j] += f * a.o_part[(i * rows + rowid) * D + lane * PER + j];
+        }
+        if (a.sinks != nullptr) L += exp2f(a.sinks[head] * 1.4426950408889634f - m);
+    }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    T* po = out + b * a.ob + head * a.oh + token * a.os + lane * PER;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) po[j] = VecTraits<T>::from_float(acc[j] * inv);
+}
+
+template <typename T, int D, bool PAGED>
+void flash_launch(torch::Tensor& out, const torch::Tensor& q, const torch::Tensor& k,
+                  const torch::Tensor& v, FaArgs& a, hipStream_t stream) {
+    const int gq = a.Hq / a.Hkv;
+    a.nqt = (int)(((long)gq * a.S + QROWS - 1) / QROWS);
+    const size_t lds = 4 * KT * D * 2 + 8 * sizeof(int) + (PAGED ? 2 * (KT + 1) * sizeof(int) : 0);
+    static const bool once = [&] {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_kernel<T, D, PAGED>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        return true;
+    }();
+    (void)once;
+    const long blocks = (long)a.B * a.Hkv * a.nqt * a.nsplit;
+    TORCH_CHECK(blocks < (1l << 31), "flash attention: too many query rows");
+    hipLaunchKernelGGL((flash_kernel<T, D, PAGED>), dim3((unsigned)blocks), dim3(256), lds, stream,
+                       (T*)out.data_ptr(), (const T*)q.data_ptr(), (const T*)k.data_ptr(),
+                       (const T*)v.data_ptr(), a);
+    HIP_CHECK_KERNEL();
+    if (a.nsplit > 1) {
+        const long rows = (long)a.B * a.Hq * a.S;
+        hipLaunchKernelGGL((flash_combine_kernel<T, D>), dim3((unsigned)((rows + 3) / 4)), dim3(256),
+                           0, stream, (T*)out.data_ptr(), a);
+        HIP_CHECK_KERNEL();
     }
 }
 
-// NOTE on the PV B-fragment: mfma_f32_16x16x32 B is a 32(K)x16(N) operand —
-// lane holds col n = lane&15 and k-elems (lane>>4)*8..+7. Our read above
-// loads V^T[n_dim][k] rows, giving lane {d = di*16 + lane&15, k = (lane>>4)*8+j}
-// which matches B[k][n] with n=d. Same shape logic for the QK^T B (K tile).
-
-static void flash_prefill_impl(torch::Tensor& out, torch::Tensor& q,
-                               const torch::Tensor& k, const torch::Tensor& v,
-                               double scale, long window,
-                               c10::optional<torch::Tensor>& sinks_opt,
-                               const int* seq_ids_ptr, int Smax_arg, int Hkv) {
-    const int B = q.size(0), Hq = q.size(1), S = q.size(2), D = q.size(3);
-    TORCH_CHECK(Hq % Hkv == 0, "Hq must divide by Hkv");
-    TORCH_CHECK(D == 64 || D == 128, "flash_prefill: head_dim 64/128 only");
-    dim3 grid((S + QBLK - 1) / QBLK, Hq, B);
-    auto stream = at::hip::getCurrentHIPStream();
+void flash_run(torch::Tensor& out, const torch::Tensor& q, const torch::Tensor& k,
+               const torch::Tensor& v, FaArgs& a, c10::optional<torch::Tensor>& sinks_opt) {
+    const int D = q.size(3);
+    TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4 && out.dim() == 4, "bad shapes");
+    TORCH_CHECK(q.is_contiguous() && k.is_contiguous() && v.is_contiguous(),
+                "contiguous tensors required");
+    TORCH_CHECK(out.sizes() == q.sizes() && out.stride(3) == 1 && out.stride(2) % 4 == 0 &&
+                out.stride(1) % 4 == 0 && out.stride(0) % 4 == 0, "flash attention: bad output layout");
+    TORCH_CHECK(k.sizes() == v.sizes() && k.size(3) == D, "flash attention: K/V shapes differ");
+    TORCH_CHECK(k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type() &&
+                out.scalar_type() == q.scalar_type(), "flash attention: one dtype for q, k, v and out");
+    TORCH_CHECK(a.Hkv > 0 && a.Hq % a.Hkv == 0, "Hq must divide by Hkv");
+    TORCH_CHECK(D == 64 || D == 128, "flash attention: head_dim 64/128 only");
+    if (q.numel() == 0) return;
+    if (k.numel() == 0) {
+        out.zero_();
+        return;
+    }
     torch::Tensor sinks_t;
-    const float* sinks = nullptr;
     if (sinks_opt.has_value()) {
         sinks_t = sinks_opt->to(torch::kFloat32).contiguous();
-        sinks = sinks_t.data_ptr<float>();
+        TORCH_CHECK(sinks_t.numel() == a.Hq, "sinks must be (Hq,)");
+        a.sinks = sinks_t.data_ptr<float>();
     }
-    if (q.scalar_type() == at::ScalarType::BFloat16) {
-        if (D == 128)
-            hipLaunchKernelGGL((flash_prefill_kernel<__hip_bfloat16, 128>), grid, dim3(256), 0,
-                               stream, (__hip_bfloat16*)out.data_ptr(),
-                               (const __hip_bfloat16*)q.data_ptr(),
-                               (const __hip_bfloat16*)k.data_ptr(),
-                               (const __hip_bfloat16*)v.data_ptr(),
-                               (float)scale, (int)window, Hq, Hkv, S, sinks,
-                               seq_ids_ptr, Smax_arg);
-        else
-            hipLaunchKernelGGL((flash_prefill_kernel<__hip_bfloat16, 64>), grid, dim3(256), 0,
-                               stream, (__hip_bfloat16*)out.data_ptr(),
-                               (const __hip_bfloat16*)q.data_ptr(),
-                               (const __hip_bfloat16*)k.data_ptr(),
-                               (const __hip_bfloat16*)v.data_ptr(),
-                               (float)scale, (int)window, Hq, Hkv, S, sinks,
-                               seq_ids_ptr, Smax_arg);
-    } else if (q.scalar_type() == at::ScalarType::Half) {
-        if (D == 128)
-            hipLaunchKernelGGL((flash_prefill_kernel<__half, 128>), grid, dim3(256), 0,
-                               stream, (__half*)out.data_ptr(), (const __half*)q.data_ptr(),
-                               (const __half*)k.data_ptr(), (const __half*)v.data_ptr(),
-                               (float)scale, (int)window, Hq, Hkv, S, sinks,
-                               seq_ids_ptr, Smax_arg);
-        else
-            hipLaunchKernelGGL((flash_prefill_kernel<__half, 64>), grid, dim3(256), 0,
-                               stream, (__half*)out.data_ptr(), (const __half*)q.data_ptr(),
-                               (const __half*)k.data_ptr(), (const __half*)v.data_ptr(),
-                               (float)scale, (int)window, Hq, Hkv, S, sinks,
-                               seq_ids_ptr, Smax_arg);
-    } else {
-        TORCH_CHECK(false, "flash_prefill: bf16/f16 only");
+    a.ob = out.stride(0);
+    a.oh = out.stride(1);
+    a.os = out.stride(2);
+    torch::Tensor o_part, ml_part;
+    if (a.nsplit > 1) {
+        auto opts = torch::TensorOptions().dtype(torch::kFloat32).device(q.device());
+        const long rows = (long)a.nsplit * a.B * a.Hq * a.S;
+        o_part = torch::empty({rows * D}, opts);
+        ml_part = torch::empty({rows * 2}, opts);
+        a.o_part = o_part.data_ptr<float>();
+        a.ml_part = ml_part.data_ptr<float>();
     }
-    HIP_CHECK_KERNEL();
+    auto stream = at::hip::getCurrentHIPStream();
+    const bool paged = a.block_table != nullptr;
+#define FA_GO(T)                                                                 \
+    do {                                                                         \
+        if (D == 128 && paged) flash_launch<T, 128, true>(out, q, k, v, a, stream);  \
+        else if (D == 128) flash_launch<T, 128, false>(out, q, k, v, a, stream); \
+        else if (paged) flash_launch<T, 64, true>(out, q, k, v, a, stream);      \
+        else flash_launch<T, 64, false>(out, q, k, v, a, stream);                \
+    } while (0)
+    if (q.scalar_type() == at::ScalarType::BFloat16) FA_GO(__hip_bfloat16);
+    else if (q.scalar_type() == at::ScalarType::Half) FA_GO(__half);
+    else TORCH_CHECK(false, "flash_prefill: bf16/f16 only");
+#undef FA_GO
 }
+
+FaArgs flash_args(const torch::Tensor& q, double scale, long window) {
+    FaArgs a{};
+    a.scale = (float)scale;
+    a.window = (int)window;
+    a.B = q.size(0);
+    a.Hq = q.size(1);
+    a.S = q.size(2);
+    a.nsplit = 1;
+    return a;
+}
+
+// Splits over the keys: two workgroups fit a CU, so fill 512 places, but leave a split
+// at least 4 tiles (256 keys) of the longest row, below which combining costs more.
+int flash_splits(const FaArgs& a) {
+    const long tiles = ((long)a.Hq / a.Hkv * a.S + QROWS - 1) / QROWS * a.B * a.Hkv;
+    const long most = std::max(1, a.cap / (4 * KT));
+    return (int)std::max(1l, std::min({512 / std::max(1l, tiles), most, 16l}));
+}
+
+}  // namespace
 
 void flash_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k,
                    torch::Tensor v, double scale, long window,
                    c10::optional<torch::Tensor> sinks_opt) {
-    flash_prefill_impl(out, q, k, v, scale, window, sinks_opt, nullptr,
-                       (int)q.size(2), (int)k.size(1));
+    FaArgs a = flash_args(q, scale, window);
+    a.Hkv = k.size(1);
+    a.cap = a.Smax = k.size(2);
+    TORCH_CHECK(k.size(0) == a.B && k.size(2) == a.S, "flash_prefill: K/V must match q");
+    flash_run(out, q, k, v, a, sinks_opt);
 }
 
 void flash_prefill_cached(torch::Tensor out, torch::Tensor q,
@@ -389,7 +589,47 @@ void flash_prefill_cached(torch::Tensor out, torch::Tensor q,
     // K/V read from the (Bc, Hkv, Smax, D) cache rows just written —
     // prefill straight off the cache, no fresh K/V tensors
     auto sid = seq_ids.to(torch::kInt32).contiguous();
-    flash_prefill_impl(out, q, k_cache, v_cache, scale, window, sinks_opt,
-                       sid.data_ptr<int>(), (int)k_cache.size(2),
-                       (int)k_cache.size(1));
+    FaArgs a = flash_args(q, scale, window);
+    a.Hkv = k_cache.size(1);
+    a.Smax = k_cache.size(2);
+    a.cap = std::min(a.S, a.Smax);
+    a.seq_ids = sid.data_ptr<int>();
+    a.clamp_rows = 1;   // rows of -1 are batch padding: read row 0, the host drops the result
+    TORCH_CHECK(sid.numel() == a.B, "seq_ids must be (B,)");
+    flash_run(out, q, k_cache, v_cache, a, sinks_opt);
+}
+
+// Several query tokens a sequence against the cache, each attending the rows up to its own
+// position (chunked prefill, prefix prefill, verification). Linear cache: block_table absent.
+void flash_extend(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
+                  torch::Tensor v_cache, torch::Tensor positions,
+                  c10::optional<torch::Tensor> seq_ids_opt,
+                  c10::optional<torch::Tensor> block_table_opt, double scale, long window,
+                  c10::optional<torch::Tensor> sinks_opt) {
+    FaArgs a = flash_args(q, scale, window);
+    const bool paged = block_table_opt.has_value();
+    a.Hkv = k_cache.size(paged ? 2 : 1);
+    auto pos = positions.to(torch::kInt32).contiguous();
+    TORCH_CHECK(pos.numel() == (long)a.B * a.S, "positions must be (B, Sq)");
+    a.positions = pos.data_ptr<int>();
+    torch::Tensor sid, bt;
+    if (paged) {
+        bt = block_table_opt->to(torch::kInt32).contiguous();
+        TORCH_CHECK(bt.dim() == 2 && bt.size(0) == a.B, "block_table must be (B, blocks)");
+        a.block_table = bt.data_ptr<int>();
+        a.block_size = k_cache.size(1);
+        a.max_blocks = bt.size(1);
+        a.cap = a.max_blocks * a.block_size;
+        if (bt.numel() == 0) {
+            out.zero_();
+            return;
+        }
+    } else {
+        TORCH_CHECK(seq_ids_opt.has_value() && seq_ids_opt->numel() == a.B, "seq_ids must be (B,)");
+        sid = seq_ids_opt->to(torch::kInt32).contiguous();
+        a.seq_ids = sid.data_ptr<int>();
+        a.cap = a.Smax = k_cache.size(2);
+    }
+    a.nsplit = flash_splits(a);
+    flash_run(out, q, k_cache, v_cache, a, sinks_opt);
 }

@@ -27,6 +27,11 @@ void flash_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k,
 void flash_prefill_cached(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
                           torch::Tensor v_cache, torch::Tensor seq_ids, double scale,
                           long window, c10::optional<torch::Tensor> sinks);
+void flash_extend(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
+                  torch::Tensor v_cache, torch::Tensor positions,
+                  c10::optional<torch::Tensor> seq_ids,
+                  c10::optional<torch::Tensor> block_table, double scale, long window,
+                  c10::optional<torch::Tensor> sinks);
 void qkv_rope_update(torch::Tensor q_out, torch::Tensor qkv, torch::Tensor cosb,
                      torch::Tensor sinb, torch::Tensor k_cache, torch::Tensor v_cache,
                      torch::Tensor positions, torch::Tensor seq_ids, long Hq, long Hkv);
@@ -109,6 +114,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           "MFMA causal flash prefill reading K/V from the cache (CDNA4)",
           py::arg("out"), py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
           py::arg("seq_ids"), py::arg("scale"), py::arg("window"),
+          py::arg("sinks") = py::none());
+    m.def("flash_extend", &flash_extend,
+          "MFMA flash attention of several query tokens over the linear or paged cache (CDNA4)",
+          py::arg("out"), py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
+          py::arg("positions"), py::arg("seq_ids") = py::none(),
+          py::arg("block_table") = py::none(), py::arg("scale") = 1.0, py::arg("window") = 0,
           py::arg("sinks") = py::none());
     m.def("qkv_rope_update", &qkv_rope_update, "fused qkv->rope->cache-write (CDNA4)");
     m.def("skinny_gemm", &skinny_gemm, "skinny-M weight-streaming GEMM (CDNA4)",

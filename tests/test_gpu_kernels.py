@@ -1300,3 +1300,85 @@ def test_moe_grouped_tile32_gpu(monkeypatch):
     got = m._forward_grouped(x, w, idx)
     torch.testing.assert_close(got.float(), want.float(),
                                atol=5e-2, rtol=5e-2)
+
+
+def _rel(a, b):
+    return float((a.double().cpu() - b.double().cpu()).norm() / b.double().cpu().norm())
+
+
+@pytest.mark.parametrize("D,gq,Sq,dtype", [
+    (128, 4, 2, torch.bfloat16), (128, 4, 33, torch.bfloat16), (128, 1, 65, torch.float16),
+    (64, 8, 16, torch.bfloat16), (64, 3, 97, torch.float16), (128, 12, 11, torch.bfloat16),
+    (128, 4, 512, torch.bfloat16),
+])
+@pytest.mark.parametrize("window", [0, 100, -64])
+@pytest.mark.parametrize("paged", [False, True])
+def test_attention_extend(D, gq, Sq, dtype, window, paged):
+    """Several query tokens over the cache: positions that start anywhere, trailing pads, a batch
+    row without a cache row, pages in any order with rows that have none, token counts around the
+    128-row tile, splits over the keys, heads that do not divide the tile, sinks. Against the fp32
+    reference on the same rounded inputs the output is off by the rounding of the probabilities
+    and of the result to 16 bits: 2^-8 in bf16, 2^-11 in fp16 (2-norm), with half as much again
+    for the order of the sums."""
+    torch.manual_seed(Sq + D)
+    dev, Hkv, B, cap, bs = _dev(), 2, 3, 1024, 16
+    q = torch.randn(B, Hkv * gq, Sq, D, device=dev).to(dtype)
+    kc = torch.randn(B + 1, Hkv, cap, D, device=dev).to(dtype)
+    vc = torch.randn(B + 1, Hkv, cap, D, device=dev).to(dtype)
+    start = torch.tensor([0, 130, cap - Sq])
+    pos = start.view(B, 1) + torch.arange(Sq).view(1, Sq)
+    pos[1, Sq - Sq // 3:] = -1
+    rows = torch.tensor([2, 0, 3])
+    sinks = torch.randn(Hkv * gq, device=dev) if window == 0 and not paged else None
+    kw = dict(scale=D ** -0.5, sliding_window=window)
+    kr, vr = kc.float().cpu()[rows], vc.float().cpu()[rows]
+    if paged:
+        per = cap // bs
+        perm = torch.randperm(B * per)
+        pk = torch.randn(B * per + 2, bs, Hkv, D, device=dev).to(dtype)
+        pv = torch.full_like(pk, float("nan"))
+        bt = torch.full((B, per), -1, dtype=torch.long)
+        for b in range(B):
+            last = int(pos[b].max())
+            for j in range(last // bs + 1):
+                at = int(perm[b * per + j]) + 2
+                bt[b, j] = at
+                pk[at] = kc[rows[b], :, j * bs:(j + 1) * bs].transpose(0, 1)
+                pv[at] = vc[rows[b], :, j * bs:(j + 1) * bs].transpose(0, 1)
+        out = ops.attention_decode_paged(q, pk, pv, pos.to(dev), bt.to(dev), **kw)
+    else:
+        out = ops.attention_decode(q, kc, vc, pos.to(dev), seq_ids=rows.to(dev), sinks=sinks, **kw)
+    want = ops.attention_decode(q.float().cpu(), kr, vr, pos, sinks=None if sinks is None
+                                else sinks.cpu(), **kw)
+    assert out.shape == want.shape
+    assert torch.equal(out[1, :, Sq - Sq // 3:].float().cpu(), torch.zeros_like(want[1, :, Sq - Sq // 3:]))
+    tol = 1.5 * 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert _rel(out, want) < tol
+
+
+def test_attention_extend_missing_pages_and_rows():
+    """A page missing inside the attended range drops its keys (and nothing of the page that the
+    kernel reads in its place, here NaN, gets through); a negative cache row gives zeros; a
+    negative scale orders the scores the other way round."""
+    torch.manual_seed(0)
+    dev, Hkv, gq, Sq, D, bs, per = _dev(), 2, 4, 40, 128, 32, 8
+    q = torch.randn(1, Hkv * gq, Sq, D, device=dev).to(torch.bfloat16)
+    pk = torch.randn(per, bs, Hkv, D, device=dev).to(torch.bfloat16)
+    pv = torch.randn(per, bs, Hkv, D, device=dev).to(torch.bfloat16)
+    pk[0] = float("nan")
+    pv[0] = float("nan")
+    bt = torch.tensor([[3, -1, 5, 1, 2, 7, -1, -1]])
+    pos = torch.arange(140, 140 + Sq).view(1, Sq)
+    out = ops.attention_decode_paged(q, pk, pv, pos.to(dev), bt.to(dev), scale=-0.05)
+    k, v = ref.paged_gather_kv(pk.float().cpu(), pv.float().cpu(), bt, 180)
+    ar = torch.arange(180)
+    mask = (ar.view(1, 1, 1, -1) <= pos.view(1, 1, Sq, 1)) & ~((ar >= 32) & (ar < 64))
+    k[:, :, 32:64] = 0
+    v[:, :, 32:64] = 0
+    want = ref.sdpa(q.float().cpu(), k, v, mask=mask, scale=-0.05)
+    assert _rel(out, want) < 1.5 * 2.0 ** -8
+    kc = torch.randn(2, Hkv, 128, D, device=dev).to(torch.bfloat16)
+    got = ops.attention_decode(q[:, :, :4].expand(2, -1, -1, -1).contiguous(), kc, kc,
+                               torch.arange(9, 13, device=dev).expand(2, 4),
+                               seq_ids=torch.tensor([-1, 1], device=dev))
+    assert not got[0].any() and bool(got[1].any())
