@@ -13,7 +13,9 @@
 //     the other half wave for the maximum of 64 keys, none for the sum until the end).
 //   * P never leaves the registers: the C layout of S^T holds, for a lane, runs of 4
 //     consecutive keys; read as the B operand of O^T = V^T P^T they are the same 16 keys in
-//     another order, and V^T is read in that order. V stays row-major in LDS: ds_read_b64_tr
+//     another order, and V^T is read in that order. Over a cache P enters the second product
+//     as a high and a low 16-bit part (HILO): single tokens are attended with 32-bit
+//     probabilities, and several must not get less. V stays row-major in LDS: ds_read_b64_tr
 //     transposes 4 keys x 16 channels on the way to the registers.
 //   * The accumulator is rescaled only when a row's maximum grew by more than 2^8 since the
 //     last time; probabilities and sums share the stale maximum, so nothing is lost.
@@ -27,15 +29,17 @@
 //
 // Measured (MI355X, bf16, 32 query / 8 kv heads; before: 16x16x32 tiles, P through LDS, V
 // transposed by the staging stores; several tokens over a cache: one workgroup a token):
-//   prompt of 8192, head size 128     2168 -> 617 us (891 TFLOP/s; two thirds of it is the
+//   prompt of 8192, head size 128     2168 -> 608 us (904 TFLOP/s; two thirds of it is the
 //                                     matrix pipe, the rest exponentials it does not hide)
-//   prompt of 2048, head size 128/64  179 -> 54 us / 145 -> 42 us
+//   prompt of 2048, head size 128/64  179 -> 54 us / 145 -> 39 us
 //   prompt of 512 / 128               40 -> 16 us / 16 -> 9 us
-//   512 tokens over 4000, linear/paged 1772 -> 62 us / 2019 -> 79 us
-//   64 tokens over 4000, linear       237 -> 31 us
-//   32 rows of 6 tokens over 2000     354 -> 47 us (a verification step)
-//   1 row of 2 tokens over 2000       28 -> 17 us
-// No size was found at which several tokens are better off one by one.
+//   512 tokens over 4000, linear/paged 1772 -> 80 us / 2019 -> 95 us (62 / 79 with P in 16 bits)
+//   64 tokens over 4000, linear       237 -> 32 us
+//   32 rows of 6 tokens over 2000     354 -> 49 us (a verification step)
+//   1 row of 2 tokens over 2000       28 -> 19 us
+// No size was found at which several tokens are better off one by one. Error against 64 bits
+// over a cache, bf16, 2-norm: 1.65e-3 (the rounding of the result; one by one 1.65e-3 to
+// 2.35e-3, 2.3e-3 with P in 16 bits), fp16 2.07e-4.
 
 #include "common.h"
 #include <torch/extension.h>
@@ -103,7 +107,7 @@ struct FaArgs {
     int nsplit, nqt, clamp_rows;      // clamp_rows: a negative seq_id reads row 0 (else: no keys)
 };
 
-template <typename T, int D, bool PAGED>
+template <typename T, int D, bool PAGED, bool HILO>
 __global__ __launch_bounds__(256, 2) void flash_kernel(
     T* __restrict__ out, const T* __restrict__ q, const T* __restrict__ k,
     const T* __restrict__ v, const FaArgs a) {
@@ -363,17 +367,23 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
                 for (int r = 0; r < 16; ++r) o[i][r] *= f;
         }
         const float mu = m == -INFINITY ? 0.f : m;      // a row that has seen no key yet
-        vec8 p[4];
 #pragma unroll
         for (int n = 0; n < 2; ++n)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const float e = __builtin_amdgcn_exp2f(fmaf(s[n][r], c, -mu));
                 l += e;
-                p[n * 2 + (r >> 3)][r & 7] = (typename FT::elem)e;
+                s[n][r] = e;
             }
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
+        for (int kt = 0; kt < 4; ++kt) {
+            vec8 p, p_lo;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float e = s[kt >> 1][(kt & 1) * 8 + j];
+                p[j] = (typename FT::elem)e;
+                if constexpr (HILO) p_lo[j] = (typename FT::elem)(e - (float)p[j]);
+            }
 #pragma unroll
             for (int db = 0; db < NDB; ++db) {
                 vec8 va;
@@ -388,15 +398,18 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
 #pragma unroll
                     for (int e = 0; e < 4; ++e) va[j * 4 + e] = y[e];
                 }
-                o[db] = FT::mfma(va, p[kt], o[db]);
+                o[db] = FT::mfma(va, p, o[db]);
+                if constexpr (HILO) o[db] = FT::mfma(va, p_lo, o[db]);
             }
+        }
+        constexpr int PER = HILO ? 2 : 1;
         __builtin_amdgcn_sched_group_barrier(0x100, 8, 1);
 #pragma unroll
         for (int i = 0; i < 4 * NDB - 4; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
+            __builtin_amdgcn_sched_group_barrier(0x008, PER, 1);
             __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 1);
+        __builtin_amdgcn_sched_group_barrier(0x008, 4 * PER, 1);
     }
 
     // ---- epilogue: rows of 4 channels from 8*(r>>2) + 4*half ----
@@ -474,21 +487,21 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(T* __restrict__ out,
     for (int j = 0; j < PER; ++j) po[j] = VecTraits<T>::from_float(acc[j] * inv);
 }
 
-template <typename T, int D, bool PAGED>
+template <typename T, int D, bool PAGED, bool HILO>
 void flash_launch(torch::Tensor& out, const torch::Tensor& q, const torch::Tensor& k,
                   const torch::Tensor& v, FaArgs& a, hipStream_t stream) {
     const int gq = a.Hq / a.Hkv;
     a.nqt = (int)(((long)gq * a.S + QROWS - 1) / QROWS);
     const size_t lds = 4 * KT * D * 2 + 8 * sizeof(int) + (PAGED ? 2 * (KT + 1) * sizeof(int) : 0);
     static const bool once = [&] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_kernel<T, D, PAGED>),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_kernel<T, D, PAGED, HILO>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         return true;
     }();
     (void)once;
     const long blocks = (long)a.B * a.Hkv * a.nqt * a.nsplit;
     TORCH_CHECK(blocks < (1l << 31), "flash attention: too many query rows");
-    hipLaunchKernelGGL((flash_kernel<T, D, PAGED>), dim3((unsigned)blocks), dim3(256), lds, stream,
+    hipLaunchKernelGGL((flash_kernel<T, D, PAGED, HILO>), dim3((unsigned)blocks), dim3(256), lds, stream,
                        (T*)out.data_ptr(), (const T*)q.data_ptr(), (const T*)k.data_ptr(),
                        (const T*)v.data_ptr(), a);
     HIP_CHECK_KERNEL();
@@ -538,17 +551,23 @@ void flash_run(torch::Tensor& out, const torch::Tensor& q, const torch::Tensor& 
     }
     auto stream = at::hip::getCurrentHIPStream();
     const bool paged = a.block_table != nullptr;
-#define FA_GO(T)                                                                 \
-    do {                                                                         \
-        if (D == 128 && paged) flash_launch<T, 128, true>(out, q, k, v, a, stream);  \
-        else if (D == 128) flash_launch<T, 128, false>(out, q, k, v, a, stream); \
-        else if (paged) flash_launch<T, 64, true>(out, q, k, v, a, stream);      \
-        else flash_launch<T, 64, false>(out, q, k, v, a, stream);                \
+    const bool extend = a.positions != nullptr;
+#define FA_D(T, D)                                                                        \
+    do {                                                                                  \
+        if (paged) flash_launch<T, D, true, true>(out, q, k, v, a, stream);               \
+        else if (extend) flash_launch<T, D, false, true>(out, q, k, v, a, stream);        \
+        else flash_launch<T, D, false, false>(out, q, k, v, a, stream);                   \
+    } while (0)
+#define FA_GO(T)                                                                          \
+    do {                                                                                  \
+        if (D == 128) FA_D(T, 128);                                                       \
+        else FA_D(T, 64);                                                                 \
     } while (0)
     if (q.scalar_type() == at::ScalarType::BFloat16) FA_GO(__hip_bfloat16);
     else if (q.scalar_type() == at::ScalarType::Half) FA_GO(__half);
     else TORCH_CHECK(false, "flash_prefill: bf16/f16 only");
 #undef FA_GO
+#undef FA_D
 }
 
 FaArgs flash_args(const torch::Tensor& q, double scale, long window) {
