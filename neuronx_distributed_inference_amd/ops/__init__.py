@@ -447,7 +447,7 @@ def attention_decode(q, k_cache, v_cache, seq_lens, seq_ids=None, scale=None,
             return out
         Hkv = k_cache.shape[1]
         gq = Hq // max(Hkv, 1)
-        if gq > 8:
+        if gq > 8 and (q.dtype == torch.float32 or D not in (64, 128)):
             # odd GQA shards (e.g. 96q/8kv models, replicate-to-TP
             # 70B configs): split the q heads per KV head into <=8-wide
             # groups and run the kernel per group (KV re-read per split;

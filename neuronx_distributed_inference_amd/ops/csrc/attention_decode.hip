@@ -1,7 +1,8 @@
 // Token-generation (decode) attention for gfx950 — the K2-analog
 // (ref attention_block_tkg, modules/attention/attention_base.py:1186-1381).
 //
-// Memory-bound split-KV design for the linear cache (B,Hkv,Smax,D):
+// Memory-bound split-KV design. 16-bit models with head sizes 64 and 128 take the matrix-core
+// kernel further down; fp32 and the other head sizes take this one:
 //  * pass 1: grid (nsplit, Hkv*Sq, B), 256-thread workgroups (4 waves).
 //    Lane groups of D/8 lanes stream K/V rows with 16-B loads (8 bf16 per
 //    lane = one ds-free register path; guide G13). Each group computes the
@@ -29,7 +30,7 @@ constexpr float M_INIT = -1e30f;
 // quantized; the k-scale is folded into the softmax scale by the host and
 // the v-scale applied in pass 2).
 // 2-way packed dot (v_dot2): halves the QK VALU work and the q-register
-// footprint — the GQ=8 (70B TP1) case was occupancy-bound at 178 VGPRs.
+// footprint.
 typedef __bf16 dot2_bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 dot2_f16x2 __attribute__((ext_vector_type(2)));
 template <typename T> struct Dot2 {
@@ -326,46 +327,432 @@ __global__ __launch_bounds__(256) void decode_attn_pass1(
     }
 }
 
+// ---------------------------------------------------------------------------
+// Matrix-core pass 1: 16-bit models, head sizes 64 and 128, cache in the model's type or e4m3.
+//
+// Bound by the stream of K and V. The lane-group kernel above spends about 40 vector
+// instructions a row and query head on products, exponentials and lane sums (129 us where the
+// stream takes 83, 274 us of an 8-bit cache where it takes 33); here a wave takes 32 keys at a
+// time through the matrix pipe and the vector units are left with one exponential a score:
+//   * S^T = K Q^T on 16x16x32 tiles: the rows are keys, the columns up to 16 (query token,
+//     head of the group) pairs, so every K row is used by all of them. The A operand is 16
+//     contiguous bytes of a key row: it comes straight from memory, without LDS.
+//   * O = P V: the C layout of S^T gives a lane 4 consecutive keys of its column in each of
+//     the two 16-key tiles, which is the A operand of P for the same 32 keys in another
+//     order. V rows are loaded in that order, 16 bytes of channels a lane (a whole row for
+//     16 lanes), and turned in registers: one byte permutation makes a B operand word. Which
+//     channels a column of the product stands for is free, so nothing else moves.
+//   * P enters as a high and a low 16-bit part: its error stays below that of 32-bit sums.
+//   * Loads of the next 32 keys are in flight while these are computed (two register
+//     buffers, 16 KB a wave); waves of a workgroup take 32-key tiles in turn and meet in LDS
+//     once at the end.
+//   * The accumulator is rescaled only when a maximum grew by more than 2^8.
+// Measured in a captured graph (MI355X, bf16, 32/8 heads of 128, lengths half to full, before ->
+// now, stream rate): 64 rows of 2048 131 -> 76 us (5.3 TB/s); 16 of 8192 136 -> 73; 128 of 512
+// 68 -> 40; 256 of 168 57 -> 35; 1 of 300 18.2 -> 7.8; 1 of 8192 55 -> 12; 13 rows of 8000, 64/8
+// heads 271 -> 72 us, e4m3 279 -> 48 us. Error against 64 bits, bf16: 1.66e-3 (the rounding of
+// the result), before 1.66e-3 to 3.5e-3 (the scaled query was rounded too).
+typedef __bf16 dm_bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 dm_f16x8 __attribute__((ext_vector_type(8)));
+typedef float dm_f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned dm_u32x4 __attribute__((ext_vector_type(4)));
+
+template <typename T> struct DmTraits;
+template <> struct DmTraits<__hip_bfloat16> {
+    using vec8 = dm_bf16x8;
+    using elem = __bf16;
+    static DEV_INLINE dm_f32x4 mfma(vec8 a, vec8 b, dm_f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    }
+    static DEV_INLINE unsigned cvt2(unsigned w, bool hi) {   // two e4m3 -> two bf16, exact
+        return __builtin_bit_cast(unsigned, hi
+            ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, true)
+            : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, false));
+    }
+};
+template <> struct DmTraits<__half> {
+    using vec8 = dm_f16x8;
+    using elem = _Float16;
+    static DEV_INLINE dm_f32x4 mfma(vec8 a, vec8 b, dm_f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+    }
+    static DEV_INLINE unsigned cvt2(unsigned w, bool hi) {
+        return __builtin_bit_cast(unsigned, hi
+            ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, true)
+            : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, false));
+    }
+};
+
+// NE elements of the cache's type in whole words, and as 16-bit pairs
+template <int NE, bool F8> struct DmRaw {
+    static constexpr int W = NE * (F8 ? 1 : 2) / 4;
+    unsigned w[W];
+    DEV_INLINE void load(const char* p) {
+        if constexpr (W == 4) *reinterpret_cast<int4*>(w) = *reinterpret_cast<const int4*>(p);
+        else if constexpr (W == 2) *reinterpret_cast<int2*>(w) = *reinterpret_cast<const int2*>(p);
+        else w[0] = *reinterpret_cast<const unsigned*>(p);
+    }
+    template <typename T> DEV_INLINE void pairs(unsigned (&o)[NE / 2]) const {
+#pragma unroll
+        for (int i = 0; i < NE / 2; ++i) {
+            if constexpr (F8) o[i] = DmTraits<T>::cvt2(w[i >> 1], i & 1);
+            else o[i] = w[i];
+        }
+    }
+};
+
+constexpr float DM_GROWTH = 8.f;   // log2 growth of a maximum that is put off
+constexpr int DM_TILE = 32;        // keys of a wave's step
+
+template <typename T, typename CT, int D, bool PAGED>
+__global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
+    T* __restrict__ out,               // (B, Hq, Sq, D), written when nsplit == 1
+    float* __restrict__ o_part,        // (B, Hq, Sq, nsplit, D)
+    float* __restrict__ ml_part,       // (B, Hq, Sq, nsplit, 2)
+    const T* __restrict__ q, const CT* __restrict__ k_cache, const CT* __restrict__ v_cache,
+    const int* __restrict__ positions, const int* __restrict__ seq_ids,
+    const int* __restrict__ block_table, const float* __restrict__ sinks,
+    float* __restrict__ lse_out, const float scale, const float v_scale, const int window,
+    const int ring, const int Hkv, const int Sq, const int gq, const int Smax, const int chunk,
+    const int nsplit, const int block_size, const int max_blocks) {
+    using DT = DmTraits<T>;
+    using vec8 = typename DT::vec8;
+    constexpr bool F8 = sizeof(CT) == 1;
+    constexpr int NKS = D / 32;            // k-steps of K Q^T
+    constexpr int DV = D / 16;             // channels a lane holds of a V row
+    constexpr int ES = sizeof(CT);
+
+    const int split = blockIdx.x;
+    const int ncol = gq * Sq;
+    const int nct = (ncol + 15) >> 4;
+    const int hkv = blockIdx.y / nct;
+    const int c0 = (blockIdx.y % nct) * 16;
+    const int nc = min(16, ncol - c0);
+    const int b = blockIdx.z;
+    const int Hq = Hkv * gq;
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: so are the loops
+    const int n = lane & 15, g = lane >> 4;
+
+    const int row = PAGED ? 0 : seq_ids[b];
+    const int col = min(c0 + n, ncol - 1);
+    const int sq = col / gq;
+    const int head = hkv * gq + col % gq;
+    const int qpos = (c0 + n < ncol && row >= 0) ? positions[(long)b * Sq + sq] : -1;
+
+    // keys [k_lo, k_hi) that any column sees; a column's own first key
+    int key_lo = 0, pmax = -1, span = qpos + 1, first = qpos < 0 ? 0x7fffffff : 0;
+    if (ring) {
+        for (int s = 0; s < Sq; ++s) pmax = max(pmax, positions[(long)b * Sq + s]);
+        span = row >= 0 ? min(pmax + 1, Smax) : 0;
+    } else {
+        if (window > 0) key_lo = max(0, qpos - window + 1);
+        else if (window < 0) key_lo = qpos >= 0 ? qpos / -window * -window : 0;
+        if (qpos >= 0) first = key_lo;
+    }
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) {
+        span = max(span, __shfl_xor(span, off, WAVE_SIZE));
+        first = min(first, __shfl_xor(first, off, WAVE_SIZE));
+    }
+    const int k_hi = __builtin_amdgcn_readfirstlane(min(min(span, Smax), (split + 1) * chunk));
+    const int k_lo = __builtin_amdgcn_readfirstlane(max(ring ? 0 : first, split * chunk));
+    const int t_lo = k_lo / DM_TILE, t_hi = k_lo < k_hi ? (k_hi + DM_TILE - 1) / DM_TILE : 0;
+    // position of the key in cache row l: l itself; in a ring the newest one that is l modulo
+    // Smax, which is base + l up to the newest row and base + l - Smax behind it
+    const int ring_base = ring && pmax >= 0 ? pmax - pmax % Smax : 0;
+    const int ring_at = ring && pmax >= 0 ? pmax % Smax : 0x7fffffff;
+    if (ring && window > 0) key_lo = max(0, qpos - window + 1);
+
+    vec8 qf[NKS];
+    {
+        const T* qp = q + (((long)b * Hq + head) * Sq + sq) * D + g * 8;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) qf[ks] = *reinterpret_cast<const vec8*>(qp + ks * 32);
+    }
+
+    const long lin = PAGED ? 0 : ((long)max(row, 0) * Hkv + hkv) * (long)Smax * D * ES;
+    const char* kbase = reinterpret_cast<const char*>(k_cache) + lin;
+    const char* vbase = reinterpret_cast<const char*>(v_cache) + lin;
+    const int last = k_hi - 1;
+
+    // pages: lanes 0..31 each look up a key of the tile, a step ahead of its use
+    auto page_key = [&](int t) -> int { return max(min(t * DM_TILE + (lane & 31), last), 0); };
+    auto page_load = [&](int t) -> int {
+        if constexpr (!PAGED) return 0;
+        return block_table[(long)b * max_blocks + page_key(t) / block_size];
+    };
+    struct Buf {
+        DmRaw<8, F8> k[2][NKS];
+        DmRaw<DV, F8> v[8];
+        unsigned bad;              // bit j: key j of the lane has no page
+    };
+    auto load = [&](Buf& u, int t, int blk) {
+        u.bad = 0;
+        int prow = 0;                  // cache row of the lane's key, -1: no page
+        if constexpr (PAGED) prow = blk < 0 ? -1 : blk * block_size + page_key(t) % block_size;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            const char* p;
+            if constexpr (PAGED) {
+                const int r = __shfl(prow, kb * 16 + n, WAVE_SIZE);
+                p = kbase + ((long)max(r, 0) * Hkv + hkv) * (D * ES);
+            } else {
+                p = kbase + (unsigned)(min(t * DM_TILE + kb * 16 + n, last) * (D * ES));
+            }
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) u.k[kb][ks].load(p + (ks * 32 + g * 8) * ES);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int kk = (j >> 2) * 16 + g * 4 + (j & 3);
+            const char* p;
+            if constexpr (PAGED) {
+                const int r = __shfl(prow, kk, WAVE_SIZE);
+                u.bad |= ((unsigned)r >> 31) << j;
+                p = vbase + ((long)max(r, 0) * Hkv + hkv) * (D * ES);
+            } else {
+                p = vbase + (unsigned)(min(t * DM_TILE + kk, last) * (D * ES));
+            }
+            u.v[j].load(p + n * DV * ES);
+        }
+    };
+
+    dm_f32x4 o[DV];
+#pragma unroll
+    for (int i = 0; i < DV; ++i) o[i] = {0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;          // of column n; l: of this lane's keys
+    const float sc = scale * 1.4426950408889634f;
+
+    auto step = [&](Buf& u, int t) {
+        dm_f32x4 s[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            s[kb] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) {
+                unsigned w[4];
+                u.k[kb][ks].template pairs<T>(w);
+                s[kb] = DT::mfma(__builtin_bit_cast(vec8, dm_u32x4{w[0], w[1], w[2], w[3]}),
+                                 qf[ks], s[kb]);
+            }
+        }
+        float x[8], mx = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int key = t * DM_TILE + (j >> 2) * 16 + g * 4 + (j & 3);
+            const int at = key + ring_base - (key > ring_at ? Smax : 0);
+            bool ok = (key < k_hi) & (key >= k_lo) & (at <= qpos) & (at >= key_lo);
+            if constexpr (PAGED) ok = ok & !((u.bad >> j) & 1);
+            x[j] = ok ? s[j >> 2][j & 3] * sc : -INFINITY;
+            mx = fmaxf(mx, x[j]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE_SIZE));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE_SIZE));
+        if (__any(mx > m + DM_GROWTH || (m == -INFINITY && mx > m))) {
+            const float mn = fmaxf(m, mx);
+            const float f = m == -INFINITY ? 0.f : exp2f(m - mn);
+            m = mn;
+            l *= f;
+            // the accumulator's rows are columns g*4 + r
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float fr = __shfl(f, g * 4 + r, WAVE_SIZE);
+#pragma unroll
+                for (int i = 0; i < DV; ++i) o[i][r] *= fr;
+            }
+        }
+        const float mu = m == -INFINITY ? 0.f : m;
+        vec8 p, p_lo;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float e = __builtin_amdgcn_exp2f(x[j] - mu);
+            l += e;
+            p[j] = (typename DT::elem)e;
+            p_lo[j] = (typename DT::elem)(e - (float)p[j]);
+        }
+        // V: pairs of channels of 8 keys -> for each channel, pairs of keys
+        unsigned vp[8][DV / 2];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) u.v[j].template pairs<T>(vp[j]);
+        if constexpr (PAGED) {             // whatever stands in for a missing page: not 0 * NaN
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const unsigned keep = ((u.bad >> j) & 1) - 1u;
+#pragma unroll
+                for (int i = 0; i < DV / 2; ++i) vp[j][i] &= keep;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < DV; ++i) {
+            dm_u32x4 w;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                w[e] = __builtin_amdgcn_perm(vp[2 * e + 1][i >> 1], vp[2 * e][i >> 1],
+                                             (i & 1) ? 0x07060302u : 0x05040100u);
+            const vec8 vb = __builtin_bit_cast(vec8, w);
+            o[i] = DT::mfma(p, vb, o[i]);
+            o[i] = DT::mfma(p_lo, vb, o[i]);
+        }
+    };
+
+    if (t_lo + wid < t_hi) {
+        Buf u0, u1;
+        int t = t_lo + wid;
+        int blk = page_load(t), next = page_load(t + 4);
+        load(u0, t, blk);
+        for (;;) {
+            // past the end the loads repeat the last key: no branch between them and their use
+            blk = page_load(t + 8);
+            load(u1, t + 4, next);
+            step(u0, t);
+            t += 4;
+            if (t >= t_hi) break;
+            next = page_load(t + 8);
+            load(u0, t + 4, blk);
+            step(u1, t);
+            t += 4;
+            if (t >= t_hi) break;
+        }
+    }
+    l += __shfl_xor(l, 16, WAVE_SIZE);
+    l += __shfl_xor(l, 32, WAVE_SIZE);
+
+    // ---- the four waves meet ----
+    extern __shared__ __attribute__((aligned(16))) float dm_lds[];
+    float* o_lds = dm_lds;                     // [4][nc][D]
+    float* ml_lds = dm_lds + 4 * nc * D;       // [4][16][2]
+    if (g == 0) {
+        ml_lds[(wid * 16 + n) * 2] = m;
+        ml_lds[(wid * 16 + n) * 2 + 1] = l;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (g * 4 + r >= nc) continue;
+        float* p = o_lds + (wid * nc + g * 4 + r) * D + n * DV;
+#pragma unroll
+        for (int i = 0; i < DV; i += 4)
+            *reinterpret_cast<float4*>(p + i) =
+                float4{o[i][r], o[i + 1][r], o[i + 2][r], o[i + 3][r]};
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < nc * (D / 4); idx += 256) {
+        const int cl = idx / (D / 4), d = idx % (D / 4) * 4;
+        const int cc = c0 + cl;
+        const int hh = hkv * gq + cc % gq;
+        float ms = -INFINITY, ls = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) ms = fmaxf(ms, ml_lds[(w * 16 + cl) * 2]);
+        float4 acc = {0.f, 0.f, 0.f, 0.f};
+        if (ms != -INFINITY) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const float f = exp2f(ml_lds[(w * 16 + cl) * 2] - ms);
+                ls += f * ml_lds[(w * 16 + cl) * 2 + 1];
+                const float4 y = *reinterpret_cast<const float4*>(o_lds + (w * nc + cl) * D + d);
+                acc.x += f * y.x;
+                acc.y += f * y.y;
+                acc.z += f * y.z;
+                acc.w += f * y.w;
+            }
+        }
+        const long rowid = ((long)b * Hq + hh) * Sq + cc / gq;
+        const float mn = ms * 0.6931471805599453f;     // natural units from here on
+        if (nsplit > 1) {
+            *reinterpret_cast<float4*>(o_part + (rowid * nsplit + split) * D + d) = acc;
+            if (d == 0) {
+                ml_part[(rowid * nsplit + split) * 2] = mn;
+                ml_part[(rowid * nsplit + split) * 2 + 1] = ls;
+            }
+            continue;
+        }
+        float f = 1.f;
+        if (sinks != nullptr) {        // a sink joins the denominator only
+            const float mt = fmaxf(mn, sinks[hh]);
+            f = __expf(mn - mt);
+            ls = ls * f + __expf(sinks[hh] - mt);
+            if (lse_out != nullptr && d == 0) lse_out[rowid] = mt + __logf(ls);
+        } else if (lse_out != nullptr && d == 0) {
+            lse_out[rowid] = ls > 0.f ? mn + __logf(ls) : -INFINITY;
+        }
+        const float inv = ls > 0.f ? v_scale * f / ls : 0.f;
+        T* po = out + rowid * D + d;
+        po[0] = VecTraits<T>::from_float(acc.x * inv);
+        po[1] = VecTraits<T>::from_float(acc.y * inv);
+        po[2] = VecTraits<T>::from_float(acc.z * inv);
+        po[3] = VecTraits<T>::from_float(acc.w * inv);
+    }
+}
+
+// Pass 2: out row = sum over splits of exp(m_i - m) o_i / L. A group of D/4 lanes takes every
+// G-th split of a row (G: the splits' number rounded up to a power of two, at most all groups of
+// the workgroup) and the groups of a row meet in LDS, so that a row of 64 splits is 8 dependent
+// loads and not 64 (D = 128), and rows of few splits share a workgroup.
 template <typename T, int D>
-__global__ void decode_attn_pass2(
+__global__ __launch_bounds__(256) void decode_attn_pass2(
     T* __restrict__ out,               // (B, Hq, Sq, D)
     const float* __restrict__ o_part,  // (B, Hq, Sq, nsplit, D)
     const float* __restrict__ ml_part, // (B, Hq, Sq, nsplit, 2)
-    const int nsplit, const float v_scale,
+    const int nsplit, const int G, const long rows, const float v_scale,
     const float* __restrict__ sinks,   // (Hq,) learned sink logits or null
     const int Hq, const int Sq,
     float* __restrict__ lse_out) {     // (B,Hq,Sq) log-sum-exp, or null —
                                        // the cross-rank flash-decoding handle
     using VT = VecTraits<T>;
-    const long rowid = blockIdx.x;  // over B*Hq*Sq
-    const int lane = threadIdx.x;
-    // global max over splits
-    float mstar = M_INIT;
-    for (int i = 0; i < nsplit; ++i)
-        mstar = fmaxf(mstar, ml_part[(rowid * nsplit + i) * 2 + 0]);
-    float L = 0.f;
+    constexpr int LPG = D / 4, NG = 256 / LPG;
+    __shared__ float4 s_o[256];
+    __shared__ float s_ml[NG][2];
+    const int grp = threadIdx.x / LPG, c = threadIdx.x % LPG;
+    const long rowid = (long)blockIdx.x * (NG / G) + grp / G;
+    float m = M_INIT, l = 0.f;
+    float4 acc = {0.f, 0.f, 0.f, 0.f};
+    if (rowid < rows) {
+        for (int i = grp % G; i < nsplit; i += G) {
+            const float mi = ml_part[(rowid * nsplit + i) * 2];
+            const float li = ml_part[(rowid * nsplit + i) * 2 + 1];
+            const float4 oi = *reinterpret_cast<const float4*>(o_part + (rowid * nsplit + i) * D + c * 4);
+            const float mn = fmaxf(m, mi);
+            const float f = __expf(m - mn), fi = __expf(mi - mn);
+            m = mn;
+            l = l * f + li * fi;
+            acc.x = acc.x * f + oi.x * fi;
+            acc.y = acc.y * f + oi.y * fi;
+            acc.z = acc.z * f + oi.z * fi;
+            acc.w = acc.w * f + oi.w * fi;
+        }
+    }
+    s_o[threadIdx.x] = acc;
+    if (c == 0) {
+        s_ml[grp][0] = m;
+        s_ml[grp][1] = l;
+    }
+    __syncthreads();
+    if (grp % G != 0 || rowid >= rows) return;
+    float ms = M_INIT, L = 0.f;
+    for (int w = 0; w < G; ++w) ms = fmaxf(ms, s_ml[grp + w][0]);
     if (sinks != nullptr) {  // sink joins the softmax denominator only
         const int h = (int)((rowid / Sq) % Hq);
-        mstar = fmaxf(mstar, sinks[h]);
-        L += __expf(sinks[h] - mstar);
+        ms = fmaxf(ms, sinks[h]);
+        L += __expf(sinks[h] - ms);
     }
-    for (int i = 0; i < nsplit; ++i) {
-        const float mi = ml_part[(rowid * nsplit + i) * 2 + 0];
-        const float li = ml_part[(rowid * nsplit + i) * 2 + 1];
-        L += li * __expf(mi - mstar);
+    acc = {0.f, 0.f, 0.f, 0.f};
+    for (int w = 0; w < G; ++w) {
+        const float f = __expf(s_ml[grp + w][0] - ms);
+        L += s_ml[grp + w][1] * f;
+        const float4 y = s_o[(grp + w) * LPG + c];
+        acc.x += y.x * f;
+        acc.y += y.y * f;
+        acc.z += y.z * f;
+        acc.w += y.w * f;
     }
     const float inv = (L > 0.f) ? v_scale / L : 0.f;
-    if (lse_out != nullptr && lane == 0)
-        lse_out[rowid] = (L > 0.f) ? mstar + __logf(L) : -INFINITY;
-#pragma unroll
-    for (int d = lane; d < D; d += WAVE_SIZE) {
-        float acc = 0.f;
-        for (int i = 0; i < nsplit; ++i) {
-            const float mi = ml_part[(rowid * nsplit + i) * 2 + 0];
-            acc += o_part[(rowid * nsplit + i) * D + d] * __expf(mi - mstar);
-        }
-        out[rowid * D + d] = VT::from_float(acc * inv);
-    }
+    if (lse_out != nullptr && c == 0)
+        lse_out[rowid] = (L > 0.f) ? ms + __logf(L) : -INFINITY;
+    T* po = out + rowid * D + c * 4;
+    po[0] = VT::from_float(acc.x * inv);
+    po[1] = VT::from_float(acc.y * inv);
+    po[2] = VT::from_float(acc.z * inv);
+    po[3] = VT::from_float(acc.w * inv);
 }
 
 // ---------------------------------------------------------------------------
@@ -384,19 +771,56 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
     const int Hkv = paged ? k_cache.size(2) : k_cache.size(1);
     const int max_blocks = paged ? (int)block_table->size(1) : 0;
     const int Smax = paged ? max_blocks * block_size : (int)k_cache.size(2);
-    // split count: fill the chip (>=1024 workgroups when possible), chunks of
-    // >=128 rows so per-split work amortizes.
-    int nsplit = 1024 / std::max(1, B * Hkv * Sq);
-    nsplit = std::max(1, std::min({nsplit, (Smax + 127) / 128, 64}));
-    const int chunk = (Smax + nsplit - 1) / nsplit;
+    constexpr bool MFMA = !std::is_same<T, float>::value && (D == 64 || D == 128);
+    const int nct = (gq * Sq + 15) / 16;
+    // Splits over the keys. Matrix-core kernel: two workgroups fit a CU, so 512 fill the chip;
+    // more only add partial sums to write and combine (64 rows of 2048: 76 us at 512, 84 at
+    // 1024, 87 at 2048; 128 rows of 512: 40 / 40 / 52), as rows of unequal length even out over
+    // the CUs by themselves. A split keeps 128 rows, one step of each wave (1 row of 300: 7.8 us;
+    // 256: 8.4), 256 in long caches where the combining pass weighs more (1 row of 8192: 11.8 us
+    // with 256, 13.5 with 128).
+    // Lane-group kernel: >= 1024 workgroups when possible, chunks of >= 128 rows.
+    int nsplit, chunk;
+    if constexpr (MFMA) {
+        const int least = Smax <= 2048 ? 128 : 256;
+        nsplit = 512 / std::max(1, B * Hkv * nct);
+        nsplit = std::max(1, std::min({nsplit, (Smax + least - 1) / least, 64}));
+        chunk = ((Smax + nsplit - 1) / nsplit + DM_TILE - 1) / DM_TILE * DM_TILE;
+        nsplit = std::max(1, (Smax + chunk - 1) / chunk);
+    } else {
+        nsplit = 1024 / std::max(1, B * Hkv * Sq);
+        nsplit = std::max(1, std::min({nsplit, (Smax + 127) / 128, 64}));
+        chunk = (Smax + nsplit - 1) / nsplit;
+    }
 
     auto opts = torch::TensorOptions().dtype(torch::kFloat32).device(q.device());
-    auto o_part = torch::empty({(long)B * Hq * Sq * nsplit * D}, opts);
-    auto ml_part = torch::empty({(long)B * Hq * Sq * nsplit * 2}, opts);
+    const bool parts = !MFMA || nsplit > 1;
+    auto o_part = torch::empty({parts ? (long)B * Hq * Sq * nsplit * D : 0}, opts);
+    auto ml_part = torch::empty({parts ? (long)B * Hq * Sq * nsplit * 2 : 0}, opts);
     auto stream = at::hip::getCurrentHIPStream();
 
     dim3 grid1(nsplit, Hkv * Sq, B);
-    if (paged) {
+    if constexpr (MFMA) {
+        if (B == 0 || Sq == 0) return;
+        const int nc = std::min(16, gq * Sq);
+        const size_t lds = (4 * nc * D + 4 * 16 * 2) * sizeof(float);
+        dim3 grid(nsplit, Hkv * nct, B);
+#define DM_GO(PG)                                                                           \
+        hipLaunchKernelGGL((decode_mfma_kernel<T, CT, D, PG>), grid, dim3(256), lds, stream, \
+                           (T*)out.data_ptr(), o_part.data_ptr<float>(),                    \
+                           ml_part.data_ptr<float>(), (const T*)q.data_ptr(),               \
+                           (const CT*)k_cache.data_ptr(), (const CT*)v_cache.data_ptr(),    \
+                           seq_lens.data_ptr<int>(), seq_ids.data_ptr<int>(),               \
+                           PG ? block_table->data_ptr<int>() : nullptr,                     \
+                           sinks ? sinks->data_ptr<float>() : nullptr,                      \
+                           lse_out ? lse_out->data_ptr<float>() : nullptr, scale, v_scale,  \
+                           window, ring, Hkv, Sq, gq, Smax, chunk, nsplit, block_size, max_blocks)
+        if (paged) DM_GO(true);
+        else DM_GO(false);
+#undef DM_GO
+        HIP_CHECK_KERNEL();
+        if (nsplit == 1) return;
+    } else if (paged) {
         hipLaunchKernelGGL((decode_attn_pass1<T, CT, D, GQ, true>), grid1, dim3(256), 0, stream,
                            o_part.data_ptr<float>(), ml_part.data_ptr<float>(),
                            (const T*)q.data_ptr(), (const CT*)k_cache.data_ptr(),
@@ -413,10 +837,14 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
                            scale, window, ring, Hkv, Sq, gq, Smax, chunk, nsplit, 0, 0);
     }
     HIP_CHECK_KERNEL();
-    dim3 grid2(B * Hq * Sq);
-    hipLaunchKernelGGL((decode_attn_pass2<T, D>), grid2, dim3(WAVE_SIZE), 0, stream,
+    constexpr int NG = 256 / (D / 4);
+    const long rows = (long)B * Hq * Sq;
+    int G = 1;
+    while (G < nsplit && G < NG) G *= 2;
+    dim3 grid2((unsigned)((rows + NG / G - 1) / (NG / G)));
+    hipLaunchKernelGGL((decode_attn_pass2<T, D>), grid2, dim3(256), 0, stream,
                        (T*)out.data_ptr(), o_part.data_ptr<float>(),
-                       ml_part.data_ptr<float>(), nsplit, v_scale,
+                       ml_part.data_ptr<float>(), nsplit, G, rows, v_scale,
                        sinks ? sinks->data_ptr<float>() : nullptr, Hq, Sq,
                        lse_out ? lse_out->data_ptr<float>() : nullptr);
     HIP_CHECK_KERNEL();
@@ -431,6 +859,18 @@ static void dispatch_gq(torch::Tensor& out, const torch::Tensor& q,
                         float v_scale = 1.0f, const torch::Tensor* sinks = nullptr,
                         torch::Tensor* lse_out = nullptr, int ring = 0) {
     const bool fp8 = k_cache.scalar_type() == at::ScalarType::Float8_e4m3fn;
+    if constexpr (!std::is_same<T, float>::value && (D == 64 || D == 128)) {
+        // the matrix-core kernel takes heads in columns: any ratio
+        TORCH_CHECK(gq <= 8 || (bt == nullptr && lse_out == nullptr),
+                    "GQA ratio > 8 not supported yet (got ", gq, ")");
+        if (fp8)
+            launch_decode<T, __hip_fp8_e4m3, D, 1>(out, q, k_cache, v_cache, seq_lens, seq_ids, scale,
+                                                   window, gq, bt, bs, v_scale, sinks, lse_out, ring);
+        else
+            launch_decode<T, T, D, 1>(out, q, k_cache, v_cache, seq_lens, seq_ids, scale, window, gq,
+                                      bt, bs, v_scale, sinks, lse_out, ring);
+        return;
+    }
 #define GQ_CASE(CT)                                                                     \
     do {                                                                                \
         if (gq <= 1)                                                                    \

@@ -635,6 +635,8 @@ void flash_extend(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
     if (paged) {
         bt = block_table_opt->to(torch::kInt32).contiguous();
         TORCH_CHECK(bt.dim() == 2 && bt.size(0) == a.B, "block_table must be (B, blocks)");
+        TORCH_CHECK(a.Hkv > 0 && a.Hq / a.Hkv <= 8, "GQA ratio > 8 not supported yet (got ",
+                    a.Hkv > 0 ? a.Hq / a.Hkv : 0, ")");
         a.block_table = bt.data_ptr<int>();
         a.block_size = k_cache.size(1);
         a.max_blocks = bt.size(1);

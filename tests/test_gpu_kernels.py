@@ -1308,8 +1308,8 @@ def _rel(a, b):
 
 @pytest.mark.parametrize("D,gq,Sq,dtype", [
     (128, 4, 2, torch.bfloat16), (128, 4, 33, torch.bfloat16), (128, 1, 65, torch.float16),
-    (64, 8, 16, torch.bfloat16), (64, 3, 97, torch.float16), (128, 12, 11, torch.bfloat16),
-    (128, 4, 512, torch.bfloat16),
+    (64, 8, 16, torch.bfloat16), (64, 3, 97, torch.float16), (128, 7, 11, torch.bfloat16),
+    (128, 8, 512, torch.bfloat16),
 ])
 @pytest.mark.parametrize("window", [0, 100, -64])
 @pytest.mark.parametrize("paged", [False, True])
@@ -1382,3 +1382,70 @@ def test_attention_extend_missing_pages_and_rows():
                                torch.arange(9, 13, device=dev).expand(2, 4),
                                seq_ids=torch.tensor([-1, 1], device=dev))
     assert not got[0].any() and bool(got[1].any())
+
+
+@pytest.mark.parametrize("D,gq,Sq,dtype", [
+    (128, 4, 1, torch.bfloat16), (128, 1, 1, torch.float16), (64, 8, 1, torch.bfloat16),
+    (64, 3, 1, torch.float16), (128, 12, 1, torch.bfloat16), (128, 32, 1, torch.bfloat16),
+    (128, 4, 5, torch.bfloat16),
+])
+@pytest.mark.parametrize("window", [0, 100, -64])
+@pytest.mark.parametrize("kind", ["linear", "fp8", "paged", "lse", "ring"])
+def test_attention_decode_mfma(D, gq, Sq, dtype, window, kind):
+    """The matrix-core decode kernel at lengths around its 32-key steps and its splits (1, 31..33,
+    127..129, full), one row of padding, one or two column tiles, missing pages; against the fp32
+    reference on the same rounded inputs. Probabilities are held in two 16-bit parts, so what is
+    left is the rounding of the result: 2^-9 in bf16, 2^-12 in fp16 (2-norm)."""
+    if (kind in ("paged", "lse") and gq > 8) or (kind == "ring" and window < 0):
+        pytest.skip("not a form the entry point takes")
+    torch.manual_seed(gq + D)
+    dev, Hkv, cap, bs = _dev(), 2, 512, 16
+    lens = torch.tensor([1, 31, 32, 33, 127, 128, 129, 300, cap, 200])
+    B = lens.numel()
+    q = torch.randn(B, Hkv * gq, Sq, D, device=dev).to(dtype)
+    pos = (lens.view(B, 1) - Sq + torch.arange(Sq).view(1, Sq)).clamp(min=-1)
+    pos[9] = -1
+    kc = torch.randn(B, Hkv, cap, D, device=dev).to(dtype)
+    vc = torch.randn(B, Hkv, cap, D, device=dev).to(dtype)
+    if kind == "fp8" or (kind == "linear" and Sq > 1):
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    rows = torch.randperm(B)
+    kw = dict(scale=D ** -0.5, sliding_window=window)
+    kr, vr = kc.float().cpu(), vc.float().cpu()
+    lse = None
+    if kind == "paged":
+        per = cap // bs
+        perm = torch.randperm(B * per)
+        pk = torch.randn(B * per + 1, bs, Hkv, D, device=dev).to(dtype)
+        pv = torch.full_like(pk, float("nan"))
+        bt = torch.full((B, per), -1, dtype=torch.long)
+        for b in range(B):
+            for j in range(int(pos[b].max()) // bs + 1):
+                at = bt[b, j] = int(perm[b * per + j]) + 1
+                pk[at] = kc[b, :, j * bs:(j + 1) * bs].transpose(0, 1).to(dtype)
+                pv[at] = vc[b, :, j * bs:(j + 1) * bs].transpose(0, 1).to(dtype)
+        out = ops.attention_decode_paged(q, pk, pv, pos.to(dev), bt.to(dev), **kw)
+        want = ops.attention_decode(q.float().cpu(), kr, vr, pos, **kw)
+    elif kind == "lse":
+        if window < 0:
+            pytest.skip("not a form the entry point takes")
+        out, lse = ops.attention_decode_lse(q, kc, vc, pos.to(dev), **kw)
+        want, want_lse = ops.attention_decode_lse(q.float().cpu(), kr, vr, pos, **kw)
+    else:
+        sinks = torch.randn(Hkv * gq, device=dev) if window == 100 else None
+        if kind == "ring":
+            pos = torch.where(pos >= 0, pos + 700 * (torch.arange(B).view(B, 1) % 2), pos)
+            kw["ring"] = True
+        inv = torch.empty_like(rows)
+        inv[rows] = torch.arange(B)
+        out = ops.attention_decode(q, kc[inv].contiguous(), vc[inv].contiguous(), pos.to(dev),
+                                   seq_ids=rows.to(dev), sinks=sinks, **kw)
+        want = ops.attention_decode(q.float().cpu(), kr, vr, pos,
+                                    sinks=None if sinks is None else sinks.cpu(), **kw)
+    assert not out[9].any()
+    tol = 2.0 ** (-9 if dtype == torch.bfloat16 else -12)
+    assert _rel(out, want) < tol
+    if lse is not None:
+        ok = torch.isfinite(want_lse)
+        assert torch.equal(ok, torch.isfinite(lse.cpu()))
+        torch.testing.assert_close(lse.cpu()[ok], want_lse[ok], atol=2e-5, rtol=2e-5)
