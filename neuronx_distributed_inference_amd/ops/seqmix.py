@@ -356,6 +356,14 @@ def window_bias_attention(q, k_cache, v_cache, step: StepLayout, block_table,
                            gate=gate, out_dtype=out_dtype)
 
 
+# Portions of at least this many tokens run in chunks; shorter ones token by token. At 32 tokens
+# of 16 heads of 128 the two are even (31 and 33 us for one row, 36 and 38 for 4, 78 and 77 for
+# 16); at 128 tokens the chunks take 57 us for the scan's 81 (4 rows) and 163 for 227 (16 rows).
+DELTA_CHUNK_MIN_TOKENS = 64
+# bytes of chunk operands kept between the two chunk kernels (they stay in the last-level cache)
+DELTA_CHUNK_WORKSPACE = 128 << 20
+
+
 def gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps: float,
                      state, step: StepLayout, kv_heads: int, dim: int, vdim: int,
                      out_dtype=torch.float32, gate_act: str = "sigmoid"):
@@ -375,7 +383,15 @@ def gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps: float,
         out = torch.empty(B, S, H * vdim, dtype=out_dtype, device=qkv.device)
         obuf = torch.empty(B, S, H * vdim, dtype=torch.float32, device=qkv.device)
         PS = (2 * kv_heads + H) * dim + H + kv_heads
-        prep = torch.empty(B, S, PS, dtype=torch.float32, device=qkv.device)
+        prep = ws = None
+        unit = 49 * dim + 16 * vdim + 256          # floats of one 16-token chunk of a head
+        if S >= DELTA_CHUNK_MIN_TOKENS and dim in (64, 128) and vdim % 16 == 0 \
+                and _rows_view(qkv) % 4 == 0 and qkv.data_ptr() % 16 == 0 \
+                and state.data_ptr() % 16 == 0:
+            span = max(1, min(-(-S // 16), DELTA_CHUNK_WORKSPACE // (4 * B * H * unit)))
+            ws = torch.empty(span * B * H * unit, dtype=torch.float32, device=qkv.device)
+        else:
+            prep = torch.empty(B, S, PS, dtype=torch.float32, device=qkv.device)
         _check(lib.nx_gated_delta(
             _p(qkv), ctypes.c_long(_rows_view(qkv)), _p(beta),
             ctypes.c_long(_rows_view(beta)), _p(a), ctypes.c_long(_rows_view(a)),
@@ -384,8 +400,8 @@ def gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps: float,
             _p(step.positions), _p(step.seq_ids), _p(step.nvalid), _p(prep),
             ctypes.c_long(PS), _p(obuf), _p(out),
             _is_bf16(beta), B, S, H, kv_heads, dim, vdim, int(per_head),
-            int(gate_act == "silu"), _stream()),
-            "gated_delta_rule")
+            int(gate_act == "silu"), _p(ws), ctypes.c_long(0 if ws is None else ws.numel()),
+            _stream()), "gated_delta_rule")
         return out
     return ref.gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps,
                                 state, step.positions, step.seq_ids, kv_heads,

@@ -1449,3 +1449,68 @@ def test_attention_decode_mfma(D, gq, Sq, dtype, window, kind):
         ok = torch.isfinite(want_lse)
         assert torch.equal(ok, torch.isfinite(lse.cpu()))
         torch.testing.assert_close(lse.cpu()[ok], want_lse[ok], atol=2e-5, rtol=2e-5)
+
+
+@pytest.mark.parametrize("S,D,Dv,H,G,per_head,dtype", [
+    (32, 128, 128, 2, 2, False, torch.bfloat16), (33, 64, 16, 3, 1, False, torch.float32),
+    (47, 128, 48, 4, 2, True, torch.float32), (100, 128, 128, 2, 1, False, torch.float32),
+    (257, 64, 80, 2, 2, False, torch.bfloat16), (400, 128, 16, 1, 1, True, torch.bfloat16),
+])
+@pytest.mark.parametrize("span", ["one", "all"])
+def test_gated_delta_chunks(S, D, Dv, H, G, per_head, dtype, span, monkeypatch):
+    """The delta rule in 16-token chunks, against the recurrence in 64 bits: rows of every length
+    around a chunk, a carried and a fresh state, a row without a slot, heads that share keys,
+    decays from next to none to total, one chunk a span and all in one. Products and sums are
+    32-bit: what a token's result is off by grows with the chain of 128 additions and the
+    16 substitutions, not with the length; 4e-6 (2-norm) is four times what the token-by-token
+    kernel shows. In bf16 the result's own rounding (2^-9) comes on top."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    torch.manual_seed(S + D)
+    monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN_TOKENS", 1)
+    if span == "one":
+        monkeypatch.setattr(seqmix, "DELTA_CHUNK_WORKSPACE", 1)
+    dev, f64 = _dev(), torch.float64
+    lens = [S, max(1, S - 17), 31, 16, 1, 0, S]
+    B = len(lens)
+    pos = torch.full((B, S), -1)
+    for b, n in enumerate(lens):
+        pos[b, :n] = torch.arange(n) + (5 * b if b % 2 else 0)
+    slots = torch.tensor([3, 0, 5, 1, 2, 4, -1])
+    qkv = torch.randn(B, S, 2 * G * D + H * Dv)
+    beta = torch.randn(B, S, H).to(dtype)
+    a = (torch.randn(B, S, H if per_head else H * D) * 2).to(dtype)
+    gate = torch.randn(B, S, H * Dv).to(dtype)
+    A_log = torch.linspace(-3, 4, H) if H > 1 else torch.tensor([0.5])
+    dt_bias = torch.randn(a.shape[-1])
+    w = torch.randn(Dv)
+    state = torch.randn(7, H, Dv, D) * 0.3
+    st = state.to(dev)
+    step = seqmix.StepLayout(pos.to(dev), slots.to(dev))
+    out = seqmix.gated_delta_rule(qkv.to(dev), beta.to(dev), a.to(dev), dt_bias.to(dev),
+                                  A_log.to(dev), gate.to(dev), w.to(dev), 1e-5, st, step, G, D, Dv,
+                                  out_dtype=dtype)
+    want, wstate = torch.zeros(B, S, H, Dv, dtype=f64), state.to(f64)
+    for b, n in enumerate(lens):
+        if slots[b] < 0 or n == 0:
+            continue
+        x = qkv[b, :n].to(f64)
+        unit = lambda t: t * torch.rsqrt(t.square().sum(-1, keepdim=True) + 1e-6)  # noqa: E731
+        q = unit(x[:, :G * D].view(n, G, D)).repeat_interleave(H // G, 1) * D ** -0.5
+        k = unit(x[:, G * D:2 * G * D].view(n, G, D)).repeat_interleave(H // G, 1)
+        v = x[:, 2 * G * D:].view(n, H, Dv)
+        dt = torch.nn.functional.softplus(a[b, :n].to(f64) + dt_bias.to(f64)).view(n, H, -1)
+        dec = torch.exp(-A_log.to(f64).exp().view(1, H, 1) * dt).expand(n, H, D)
+        M = wstate[slots[b]].transpose(-1, -2) if pos[b, 0] > 0 else torch.zeros(H, D, Dv, dtype=f64)
+        for t in range(n):
+            M = dec[t].unsqueeze(-1) * M
+            u = torch.sigmoid(beta[b, t].to(f64)).unsqueeze(-1) * (
+                v[t] - torch.einsum("hdv,hd->hv", M, k[t]))
+            M = M + k[t].unsqueeze(-1) * u.unsqueeze(1)
+            want[b, t] = torch.einsum("hdv,hd->hv", M, q[t])
+        wstate[slots[b]] = M.transpose(-1, -2)
+    want = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + 1e-5) * w.to(f64)
+    want = want.reshape(B, S, H * Dv) * torch.sigmoid(gate.to(f64)) * (pos >= 0).unsqueeze(-1)
+    assert _rel(st, wstate) < 4e-6
+    assert _rel(out, want) < (1e-5 if dtype == torch.float32 else 2.0 ** -9)
+    assert not out[6].any() and torch.equal(st[6].cpu(), state[6])
