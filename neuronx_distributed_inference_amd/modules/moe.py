@@ -178,17 +178,18 @@ class ExpertMLPs(nn.Module):
         El = self.num_local_experts
         gates = torch.zeros(T, El, dtype=x.dtype, device=x.device)
         gates = gates.scatter(1, idx, weights.to(x.dtype))
-        gte = gates.t().unsqueeze(-1)                      # (E, T, 1)
+        gte = gates.t().unsqueeze(1)                       # (E, 1, T)
+        # weights on the left: the right operand of a 16-bit batched product is contiguous
+        xe = x.t().unsqueeze(0)
         if self.scale_input:
-            xe = x.unsqueeze(0) * gte                      # Llama4: gate input
-        else:
-            xe = x.unsqueeze(0).expand(El, T, H)
-        g = torch.bmm(xe, self.w_gate.transpose(1, 2))
-        u = torch.bmm(xe, self.w_up.transpose(1, 2))
-        y = torch.bmm(self.act_mul(g, u), self.w_down.transpose(1, 2))
+            xe = xe * gte                                  # Llama4: gate input
+        xe = xe.expand(El, H, T).contiguous()
+        g = torch.bmm(self.w_gate, xe)
+        u = torch.bmm(self.w_up, xe)
+        y = torch.bmm(self.w_down, self.act_mul(g, u))
         if not self.scale_input:
             y = y * gte
-        return y.sum(dim=0)
+        return y.sum(dim=0).t().contiguous()
 
     def _forward_grouped(self, x: torch.Tensor, weights: torch.Tensor,
                          idx: torch.Tensor) -> torch.Tensor:
@@ -203,11 +204,18 @@ class ExpertMLPs(nn.Module):
         El = self.num_local_experts
         offset = self._local_offset()
         top_k = idx.shape[1]
+        fp8 = getattr(self, "fp8", False)
+        mx4 = getattr(self, "mx4", False)
+        if x.is_cuda and not mx4:
+            ws = [getattr(self, n + ("_q" if fp8 else "")) for n in ("w_gate", "w_up", "w_down")]
+            return ops.moe_routed_experts(
+                x, weights, idx, *ws,
+                scales=(self.w_gate_s, self.w_up_s, self.w_down_s) if fp8 else None,
+                first=offset, num_experts=self.num_experts,
+                gelu=self.act_mul is not ops.silu_mul, scale_input=self.scale_input)
         flat = (idx - offset).view(-1)
         local = (flat >= 0) & (flat < El)
         flat_routed = torch.where(local, flat, torch.full_like(flat, El))
-        fp8 = getattr(self, "fp8", False)
-        mx4 = getattr(self, "mx4", False)
         # fine-grained MoE (few tokens per expert): a 32-row tile halves
         # the padded-row waste. bf16 kernel only (quantized kernels are
         # 64-row); opt-in via NXDI_MOE_TILE32=1 while it soaks.
@@ -231,21 +239,6 @@ class ExpertMLPs(nn.Module):
         gatew = weights.view(-1)[order]
         lmask = local[order]
 
-        # widest column tile that still yields >= ~2 blocks/CU — wide
-        # tiles cut x re-reads 4x but run at occupancy 1, so a small
-        # grid (TP-sharded N or small batch) must fall back to narrower
-        # tiles to fill the chip
-        def _bn(N, ntiles=Mpad // tile):
-            if tile == 32:
-                return 256 if (N % 256 == 0
-                               and (N // 256) * ntiles >= 256) else 128
-            # occupancy is 1 block/CU at bn>=192 (120 KB LDS), 2 below
-            for cand in (256, 192, 128):
-                occ = 1 if cand >= 192 else 2
-                if N % cand == 0 and (N // cand) * ntiles >= 256 * occ:
-                    return cand
-            return 64
-
         if fp8 or mx4:
             I, Hn = self.w_gate_q.shape[1], self.w_down_q.shape[1]
         else:
@@ -267,20 +260,14 @@ class ExpertMLPs(nn.Module):
             u = ops.moe_grouped_gemm_mx4(x_in, self.w_up_q, self.w_up_s,
                                          expert_ids, x_gather=xg)
         elif fp8:
-            # fp8 column tiles are 128/256 only
-            def _bn8(N, ntiles=Mpad // 64):
-                if N % 256 == 0 and (N // 256) * ntiles >= 256:
-                    return 256
-                return 128
-
             g = ops.moe_grouped_gemm_fp8(x_in, self.w_gate_q, self.w_gate_s,
-                                         expert_ids, bn=_bn8(I), x_gather=xg)
+                                         expert_ids, x_gather=xg)
             u = ops.moe_grouped_gemm_fp8(x_in, self.w_up_q, self.w_up_s,
-                                         expert_ids, bn=_bn8(I), x_gather=xg)
+                                         expert_ids, x_gather=xg)
         else:
-            g = ops.moe_grouped_gemm(x_in, self.w_gate, expert_ids, bn=_bn(I),
+            g = ops.moe_grouped_gemm(x_in, self.w_gate, expert_ids,
                                      x_gather=xg, mt=tile)
-            u = ops.moe_grouped_gemm(x_in, self.w_up, expert_ids, bn=_bn(I),
+            u = ops.moe_grouped_gemm(x_in, self.w_up, expert_ids,
                                      x_gather=xg, mt=tile)
         h = self.act_mul(g, u)
         # routing-weighted combine fuses into the down epilogue (fp32
@@ -298,11 +285,11 @@ class ExpertMLPs(nn.Module):
                                      combine_gather=gtab)
         elif fp8:
             ops.moe_grouped_gemm_fp8(h, self.w_down_q, self.w_down_s,
-                                     expert_ids, bn=_bn8(Hn),
+                                     expert_ids,
                                      combine_out=out32, combine_scale=gw_tab,
                                      combine_gather=gtab)
         else:
-            ops.moe_grouped_gemm(h, self.w_down, expert_ids, bn=_bn(Hn),
+            ops.moe_grouped_gemm(h, self.w_down, expert_ids,
                                  combine_out=out32, combine_scale=gw_tab,
                                  combine_gather=gtab, mt=tile)
         return out32.to(x.dtype)
@@ -311,29 +298,22 @@ class ExpertMLPs(nn.Module):
         """x: (T, H); weights/idx: (T, top_k) over GLOBAL expert ids.
         Returns (T, H) partial (summed by the caller's TP all-reduce)."""
         T, H = x.shape
-        # Grouped expert GEMM is the GPU DEFAULT (opt out with
-        # NXDI_MOE_GROUPED=0). With wide column tiles (bn=256: 4x fewer
-        # x re-reads) and the fused one-launch segment-table kernel
-        # (142 -> 13 us of launch latency), grouped beats the dense bmm
-        # path on Mixtral decode T=256 top-2 (826 vs 877 us/layer;
-        # profiles/r02_bench_summary.md) on top of removing the top_k/E
-        # redundant FLOPs.
+        # The routed kernels are the GPU default at every size (opt out with
+        # NXDI_MOE_GROUPED=0): they read the chosen experts' weights once,
+        # the dense products all experts' and compute E/top_k times as much.
+        # 8 experts of 4096 x 14336: 250 us for a token, 529-567 for 16-191;
+        # one pass over all the weights alone takes 577.
         import os as _os
 
         if getattr(self, "fp8", False) or getattr(self, "mx4", False):
             return self._forward_grouped(x, weights, idx)
         grouped_env = _os.environ.get("NXDI_MOE_GROUPED")
-        # small batches leave too few 64-row tiles to fill 256 CUs at the
-        # wide-tile occupancy (measured: Mixtral T=64 grouped 27.7 vs
-        # dense 23.7 ms/step; T=256 grouped 31.2 vs dense 32.0) — dense
-        # bmm keeps those
-        big_enough = x.shape[0] * idx.shape[1] >= 384
         use_grouped = (
             x.is_cuda and ops.extension_available()
             and x.dtype in (torch.bfloat16, torch.float16)
             and self.w_gate.shape[2] % 64 == 0 and self.w_gate.shape[1] % 64 == 0
             and H % 64 == 0
-            and (grouped_env == "1" or (grouped_env != "0" and big_enough))
+            and grouped_env != "0"
         )
         if use_grouped:
             return self._forward_grouped(x, weights, idx)

@@ -818,6 +818,50 @@ def moe_grouped_gemm(x_sorted: torch.Tensor, w: torch.Tensor,
     return out if out is not None else y
 
 
+# bytes of fp32 products that the routed down projection keeps at a time
+MOE_WORKSPACE = 1 << 30
+
+
+def moe_routed_experts(x: torch.Tensor, weights: torch.Tensor, idx: torch.Tensor, w_gate, w_up,
+                       w_down, scales=None, first: int = 0, num_experts: int = 0,
+                       gelu: bool = False, scale_input: bool = False) -> torch.Tensor:
+    """sum_j weights[t, j] * down_e(act(gate_e(x[t])) * up_e(x[t])), e = idx[t, j] - first, over
+    the local experts of (E, I, H) / (E, H, I) stacks (uint8 e4m3fn with ``scales`` = fp32 (E, N)
+    of gate, up and down). ``num_experts`` is the number the router chooses from. With
+    ``scale_input`` the weights scale the experts' inputs and the outputs are added as they are.
+    GPU only; x bf16/f16 (T, H)."""
+    c = _require_ext("moe_routed_experts")
+    T, H = x.shape
+    E, I = w_gate.shape[0], w_gate.shape[1]
+    n, dev = idx.numel(), x.device
+    out = torch.empty(T, H, dtype=x.dtype, device=dev)
+    if n == 0:
+        return out.zero_()
+    # rows of a tile by the rows an expert has on average (measured beside the kernel: taller
+    # tiles read weights less often, lower ones leave more workgroups)
+    mean = n / max(num_experts, E)
+    mt = 128 if mean > 64 else 64 if mean > 32 else 32
+    tiles_max = (n + min(n, E) * (mt - 1)) // mt
+    rows = tiles_max * mt
+    tabs = torch.empty(1 + 2 * tiles_max + rows + n, dtype=torch.int32, device=dev)
+    tiles, gather, inv = tabs.split([1 + 2 * tiles_max, rows, n])
+    c.moe_route(tiles, gather, inv, idx.contiguous(), E, first, mt)
+    weights = weights.float().contiguous()
+    s = scales or (None, None, None)
+    h = torch.empty(rows, I, dtype=x.dtype, device=dev)
+    if scale_input:
+        # inv is -1 for another rank's choices: their rows end in the extra last one
+        xs = torch.empty(rows + 1, H, dtype=x.dtype, device=dev)
+        xs[inv.long()] = (x.unsqueeze(1) * weights.view(T, -1, 1).to(x.dtype)).reshape(n, H)
+        c.moe_routed_glu(h, xs, w_gate, w_up, s[0], s[1], tiles, None, mt, int(gelu))
+    else:
+        c.moe_routed_glu(h, x.contiguous(), w_gate, w_up, s[0], s[1], tiles, gather, mt, int(gelu))
+    cols = min(H, max(256, MOE_WORKSPACE // (4 * rows) // 256 * 256))
+    ws = torch.empty(rows * cols, dtype=torch.float32, device=dev)
+    c.moe_routed_down(out, ws, h, w_down, s[2], tiles, inv, None if scale_input else weights, mt)
+    return out
+
+
 def fp8_moe_quantize(w: torch.Tensor):
     """Per-output-channel e4m3fn quantization of stacked expert weights
     (E, N, K) -> (wq (E, N, K) uint8, scale (E, N) fp32). e4m3fn max

@@ -81,6 +81,14 @@ void moe_grouped_gemm_mx4(torch::Tensor y, torch::Tensor x, torch::Tensor wq,
                           c10::optional<torch::Tensor> combine_out,
                           c10::optional<torch::Tensor> combine_scale,
                           c10::optional<torch::Tensor> combine_gather);
+void moe_route(torch::Tensor tiles, torch::Tensor gather, torch::Tensor inv, torch::Tensor idx,
+               long num_local, long first, long mt);
+void moe_routed_glu(torch::Tensor h, torch::Tensor x, torch::Tensor w_gate, torch::Tensor w_up,
+                    c10::optional<torch::Tensor> s_gate, c10::optional<torch::Tensor> s_up,
+                    torch::Tensor tiles, c10::optional<torch::Tensor> gather, long mt, long gelu);
+void moe_routed_down(torch::Tensor out, torch::Tensor ws, torch::Tensor h, torch::Tensor w_down,
+                     c10::optional<torch::Tensor> s_down, torch::Tensor tiles, torch::Tensor inv,
+                     c10::optional<torch::Tensor> weights, long mt);
 void router_topk(torch::Tensor vals, torch::Tensor idx, torch::Tensor logits,
                  long top_k, long act_sigmoid, long pre_softmax,
                  long normalize);
@@ -149,6 +157,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("fp8_epilogue", &fp8_epilogue, "scaled-mm row-scale epilogue (CDNA4)",
           py::arg("out"), py::arg("y32"), py::arg("w_scale"),
           py::arg("bias") = py::none());
+    m.def("moe_route", &moe_route, "row tiles of the routed experts");
+    m.def("moe_routed_glu", &moe_routed_glu, "gated expert projections over row tiles");
+    m.def("moe_routed_down", &moe_routed_down, "expert down projection and weighted sum");
     m.def("moe_grouped_tables", &moe_grouped_tables_gpu,
           "fused MoE segment tables: one launch vs the torch op chain",
           py::arg("order"), py::arg("dest"), py::arg("expert_ids"),

@@ -1514,3 +1514,57 @@ def test_gated_delta_chunks(S, D, Dv, H, G, per_head, dtype, span, monkeypatch):
     assert _rel(st, wstate) < 4e-6
     assert _rel(out, want) < (1e-5 if dtype == torch.float32 else 2.0 ** -9)
     assert not out[6].any() and torch.equal(st[6].cpu(), state[6])
+
+
+@pytest.mark.parametrize("T,E,k,H,I,dtype,f8,local,gelu,scale_input,ws", [
+    (1, 4, 2, 256, 128, torch.bfloat16, False, None, False, False, None),
+    (33, 16, 8, 128, 192, torch.float16, False, None, True, False, None),
+    (70, 8, 3, 64, 64, torch.bfloat16, False, (2, 4), False, False, None),
+    (300, 8, 2, 320, 192, torch.bfloat16, False, None, False, True, None),
+    (300, 8, 2, 576, 320, torch.float16, False, (4, 4), False, False, 1),
+    (257, 65, 8, 1024, 64, torch.bfloat16, False, None, False, False, 4 << 20),
+    (40, 8, 2, 256, 384, torch.bfloat16, True, None, False, False, None),
+    (130, 8, 4, 384, 128, torch.float16, True, None, True, False, None),
+    (600, 8, 2, 256, 512, torch.bfloat16, True, (0, 2), False, True, None),
+])
+def test_moe_routed_experts(T, E, k, H, I, dtype, f8, local, gelu, scale_input, ws, monkeypatch):
+    """Routed experts against 64 bits, from the same rounded weights: every row tile (32, 64, 128),
+    remainders of rows, columns and slabs, an expert that nobody chose, experts of other ranks.
+    The activations between the projections and the result are rounded to the 16-bit type (half
+    a unit each), sums are 32-bit: the 2-norm of the error stays below a unit, 2^-8 or 2^-11
+    (the scaled input is rounded as well, half a unit more)."""
+    torch.manual_seed(T + H)
+    if ws:
+        monkeypatch.setattr(ops, "MOE_WORKSPACE", ws)
+    dev, f64 = _dev(), torch.float64
+    first, El = local or (0, E)
+    x = (torch.randn(T, H, device=dev)).to(dtype)
+    logits = torch.randn(T, E, device=dev)
+    logits[:, first] = -9.                                    # chosen by nobody
+    wt, idx = torch.softmax(logits, -1).topk(k, dim=-1)
+    if T > 8:
+        idx[:, 0] = first + 1                                 # one expert has many rows
+        idx[:, 1:] = torch.where(idx[:, 1:] == first + 1, (first + 2) % E, idx[:, 1:])
+    w = [(torch.randn(El, *s, device=dev) * 0.1).to(dtype) for s in ((I, H), (I, H), (H, I))]
+    scales, ref = None, [v.to(f64) for v in w]
+    if f8:
+        w, scales = zip(*[ops.fp8_moe_quantize(v) for v in w])
+        ref = [ops.fp8_moe_dequant(v, s).to(f64) for v, s in zip(w, scales)]
+    got = ops.moe_routed_experts(x, wt, idx, *w, scales=scales, first=first, num_experts=E,
+                                 gelu=gelu, scale_input=scale_input)
+    want = torch.zeros(T, H, dtype=f64, device=dev)
+    act = (lambda g: torch.nn.functional.gelu(g, approximate="tanh")) if gelu \
+        else torch.nn.functional.silu
+    for e in range(El):
+        for j in range(k):
+            t = (idx[:, j] == first + e).nonzero().view(-1)
+            xe, s = x[t].to(f64), wt[t, j].to(f64).unsqueeze(1)
+            xe = xe * s if scale_input else xe
+            y = (act(xe @ ref[0][e].t()) * (xe @ ref[1][e].t())) @ ref[2][e].t()
+            want[t] += y if scale_input else y * s
+    unit = 2 ** -8 if dtype == torch.bfloat16 else 2 ** -11
+    assert torch.isfinite(got).all()
+    assert _rel(got, want) < unit * (1.5 if scale_input else 1)
+    again = ops.moe_routed_experts(x, wt, idx, *w, scales=scales, first=first, num_experts=E,
+                                   gelu=gelu, scale_input=scale_input)
+    assert torch.equal(got, again)
