@@ -27,6 +27,7 @@ from neuronx_distributed_inference_amd.modules.attention.gqa import (
     GroupQueryAttentionO,
     GroupQueryAttentionQKV,
 )
+from neuronx_distributed_inference_amd.modules.norm import RMSNorm
 from neuronx_distributed_inference_amd.modules.rope import RotaryEmbedding
 from neuronx_distributed_inference_amd.parallel import state as ps
 
@@ -159,6 +160,19 @@ class AttentionBase(nn.Module):
             q = (q * self.q_scale_fn(position_ids).unsqueeze(1).unsqueeze(-1)).to(q.dtype)
         return q, k, v
 
+    def _front_norms(self, hidden):
+        """What the fused front end needs of the q/k norms: () without any, (q weight, k weight,
+        eps), or None for norms that it does not take in."""
+        if self.q_norm is None and self.k_norm is None:
+            return ()
+        norms = (self.q_norm, self.k_norm)
+        if (hidden.is_cuda and self.head_dim in (64, 128)
+                and all(type(n) is RMSNorm and n.weight.numel() == self.head_dim
+                        and n.weight.dtype == hidden.dtype for n in norms)
+                and norms[0].variance_epsilon == norms[1].variance_epsilon):
+            return (norms[0].weight, norms[1].weight, norms[0].variance_epsilon)
+        return None
+
     # ------------------------------------------------------------------
     def forward(
         self,
@@ -185,23 +199,30 @@ class AttentionBase(nn.Module):
             active_mask = attention_mask
 
         # Fused TKG front end (K2-analog): one GEMM -> one kernel doing
-        # RoPE + cache write + q relayout. Skipped when per-head qk-norms or
-        # clip_qkv need the unfused path.
+        # RoPE (and plain per-head qk-norms) + cache write, into rows or pages,
+        # + q relayout. Other norms and clip_qkv need the unfused path.
+        norms = self._front_norms(hidden) if self.qkv_proj.fused else None
+        paged = getattr(kv_mgr, "is_paged", False)
         if (
             phase == PHASE_TKG
             and self.qkv_proj.fused
-            and self.q_norm is None
+            and norms is not None
             and self.clip_qkv is None
             and cos is not None
-            and not getattr(kv_mgr, "is_paged", False)
+            and not (paged and (not hidden.is_cuda or self.head_dim not in (64, 128)
+                                or self.kv_shard_degree > 1))
+            and not ((norms or paged) and self.dp_degree > 1)
             and not self.rope_interleaved
             and self.qk_norm_post_rope is None
             and self.q_scale_fn is None
         ):
             y = self.qkv_proj.qkv(hidden)
-            kc, vc = kv_mgr.get_cache(self.layer_idx)
             import neuronx_distributed_inference_amd.ops as _ops
 
+            if paged:
+                kc, vc = kv_mgr.k_caches[self.layer_idx], kv_mgr.v_caches[self.layer_idx]
+            else:
+                kc, vc = kv_mgr.get_cache(self.layer_idx)
             wpos = position_ids
             if self.kv_shard_degree > 1:
                 from neuronx_distributed_inference_amd.modules.attention import (
@@ -217,6 +238,7 @@ class AttentionBase(nn.Module):
                 vc.data if hasattr(vc, "data") else vc,
                 wpos, seq_ids,
                 self.num_heads_per_rank, self.num_kv_heads_per_rank,
+                norms=norms or None, slots=kv_mgr.slot_mapping if paged else None,
             )
             out = self._decode(q, kv_mgr, position_ids, seq_ids, active_mask)
             out = out.transpose(1, 2).reshape(B, S, -1)
@@ -231,7 +253,7 @@ class AttentionBase(nn.Module):
         if (
             phase == PHASE_CTE
             and self.qkv_proj.fused
-            and self.q_norm is None
+            and norms is not None
             and self.clip_qkv is None
             and cos is not None
             and seq_ids is not None
@@ -256,7 +278,7 @@ class AttentionBase(nn.Module):
                 y = self.qkv_proj.qkv(hidden)
                 q = _ops.qkv_rope_update(
                     y, cos, sin, kc, vc, position_ids, seq_ids,
-                    self.num_heads_per_rank, self.num_kv_heads_per_rank,
+                    self.num_heads_per_rank, self.num_kv_heads_per_rank, norms=norms or None,
                 )
                 out = _ops.attention_prefill_cached(
                     q, kc, vc, seq_ids, scale=self.scale, sinks=self.sinks,

@@ -580,22 +580,28 @@ def topk_topp_sample(logits, top_k, top_p, temperature, rand, global_topk: int =
     return ref.topk_topp_sample(logits, top_k, top_p, temperature, rand, global_topk)
 
 
-def qkv_rope_update(qkv, cos, sin, k_cache, v_cache, positions, seq_ids, Hq, Hkv):
+def qkv_rope_update(qkv, cos, sin, k_cache, v_cache, positions, seq_ids, Hq, Hkv,
+                    norms=None, slots=None):
     """Fused qkv-GEMM output -> RoPE(q,k) -> cache write(k,v) -> q (B,Hq,S,D).
 
-    qkv: (B, S, (Hq+2Hkv)*D) contiguous; cos/sin (B,S,D) fp32.
+    qkv: (B, S, (Hq+2Hkv)*D) contiguous; cos/sin (B,S,D) fp32. ``norms`` = (q weight, k weight,
+    eps) of per-head RMS norms before the rope. With ``slots`` (B*S flat slots) the caches are
+    pages (blocks, block size, Hkv, D) and positions and seq_ids are not read.
     """
     B, S, _ = qkv.shape
     D = k_cache.shape[3]
     if qkv.is_cuda:
         c = _require_ext("qkv_rope_update")
         q_out = torch.empty(B, Hq, S, D, dtype=qkv.dtype, device=qkv.device)
-        if seq_ids is None:
+        if slots is not None:
+            slots = seq_ids = positions = slots.to(torch.int32).contiguous()
+        elif seq_ids is None:
             seq_ids = torch.arange(B, device=qkv.device, dtype=torch.int32)
+        qw, kw, eps = norms or (None, None, 0.0)
         c.qkv_rope_update(
             q_out, qkv.contiguous(), cos.contiguous(), sin.contiguous(),
             k_cache, v_cache, positions.to(torch.int32).contiguous(),
-            seq_ids.to(torch.int32).contiguous(), Hq, Hkv,
+            seq_ids.to(torch.int32).contiguous(), Hq, Hkv, qw, kw, eps, slots,
         )
         return q_out
     # CPU reference composition
@@ -603,8 +609,15 @@ def qkv_rope_update(qkv, cos, sin, k_cache, v_cache, positions, seq_ids, Hq, Hkv
     q = q.reshape(B, S, Hq, D).transpose(1, 2)
     k = k.reshape(B, S, Hkv, D).transpose(1, 2)
     v = v.reshape(B, S, Hkv, D).transpose(1, 2)
+    if norms is not None:
+        q = ref.rms_norm(q, norms[0], norms[2])[0]
+        k = ref.rms_norm(k, norms[1], norms[2])[0]
     q, k = ref.rope_apply(q, k, cos, sin)
-    ref.kv_cache_update(k_cache, v_cache, k, v, positions, seq_ids)
+    if slots is not None:
+        ref.block_kv_cache_update(k_cache, v_cache, k.transpose(1, 2).reshape(B * S, Hkv, D),
+                                  v.transpose(1, 2).reshape(B * S, Hkv, D), slots)
+    else:
+        ref.kv_cache_update(k_cache, v_cache, k, v, positions, seq_ids)
     return q.contiguous()
 
 

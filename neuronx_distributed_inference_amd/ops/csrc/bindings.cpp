@@ -34,7 +34,9 @@ void flash_extend(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
                   c10::optional<torch::Tensor> sinks);
 void qkv_rope_update(torch::Tensor q_out, torch::Tensor qkv, torch::Tensor cosb,
                      torch::Tensor sinb, torch::Tensor k_cache, torch::Tensor v_cache,
-                     torch::Tensor positions, torch::Tensor seq_ids, long Hq, long Hkv);
+                     torch::Tensor positions, torch::Tensor seq_ids, long Hq, long Hkv,
+                     c10::optional<torch::Tensor> q_norm, c10::optional<torch::Tensor> k_norm,
+                     double eps, c10::optional<torch::Tensor> slots);
 void silu_mul_fused(torch::Tensor out, torch::Tensor gate_up);
 void skinny_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                  c10::optional<torch::Tensor> bias);

@@ -1568,3 +1568,60 @@ def test_moe_routed_experts(T, E, k, H, I, dtype, f8, local, gelu, scale_input, 
     again = ops.moe_routed_experts(x, wt, idx, *w, scales=scales, first=first, num_experts=E,
                                    gelu=gelu, scale_input=scale_input)
     assert torch.equal(got, again)
+
+
+@pytest.mark.parametrize("B,S,Hq,Hkv,D,dtype,norms,paged,fp8", [
+    (1, 1, 1, 1, 64, torch.bfloat16, True, False, False),
+    (3, 37, 5, 2, 128, torch.float16, True, True, False),
+    (2, 9, 8, 1, 32, torch.float32, False, True, False),
+    (2, 70, 3, 3, 256, torch.bfloat16, True, False, True),
+    (2, 5, 4, 2, 80, torch.bfloat16, False, False, False),
+])
+def test_qkv_rope_update_norms_and_pages(B, S, Hq, Hkv, D, dtype, norms, paged, fp8):
+    """The fused front end against the composition in 64 bits: head norms, rows and pages, dropped
+    tokens, slots nobody wrote. One rounding to the stored type (half a unit of the value) after
+    32-bit arithmetic."""
+    torch.manual_seed(D)
+    dev, f64 = _dev(), torch.float64
+    qkv = torch.randn(B, S, (Hq + 2 * Hkv) * D).to(dtype)
+    ang = torch.rand(B, S, D // 2) * 6
+    cos, sin = (torch.cat([f(ang)] * 2, -1) for f in (torch.cos, torch.sin))
+    w = [(torch.rand(D) + 0.5).to(dtype) for _ in range(2)]
+    cdt = torch.float8_e4m3fn if fp8 else dtype
+    shape = (4, 64, Hkv, D) if paged else (B + 1, Hkv, S + 3, D)
+    caches = [torch.full(shape, 2.0).to(cdt) for _ in range(2)]
+    got_c = [c.to(dev) for c in caches]
+    pos = torch.arange(S).repeat(B, 1) + 2
+    pos[-1, S // 2:] = -1
+    seq = torch.arange(B).flip(0).int()
+    slots = torch.randperm(256)[:B * S].int() if paged else None
+    if paged:
+        slots[::5] = -1
+    got = ops.qkv_rope_update(qkv.to(dev), cos.to(dev), sin.to(dev), *got_c, pos.to(dev),
+                              seq.to(dev), Hq, Hkv,
+                              norms=(w[0].to(dev), w[1].to(dev), 1e-6) if norms else None,
+                              slots=None if slots is None else slots.to(dev))
+    x = qkv.to(f64).view(B, S, Hq + 2 * Hkv, D)
+    q, k, v = x.split([Hq, Hkv, Hkv], 2)
+    if norms:
+        q, k = (t * torch.rsqrt(t.square().mean(-1, keepdim=True) + 1e-6) * u.to(f64)
+                for t, u in zip((q, k), w))
+
+    def rope(t):
+        a, b = t.chunk(2, -1)
+        return t * cos.to(f64).unsqueeze(2) + torch.cat([-b, a], -1) * sin.to(f64).unsqueeze(2)
+
+    q, k = rope(q), rope(k)
+    unit = {torch.float32: 2 ** -20, torch.float16: 2 ** -11, torch.bfloat16: 2 ** -8}[dtype]
+    torch.testing.assert_close(got.to(f64).cpu(), q.transpose(1, 2), rtol=unit, atol=1e-5)
+    for c, c0, t in zip(got_c, caches, (k, v)):
+        want = c0.to(f64)
+        for b in range(B):
+            for s in range(S):
+                if paged and slots[b * S + s] >= 0:
+                    want.view(-1, Hkv, D)[slots[b * S + s]] = t[b, s]
+                elif not paged and pos[b, s] >= 0:
+                    want[seq[b], :, pos[b, s]] = t[b, s]
+        u = 2 ** -4 if fp8 else unit
+        torch.testing.assert_close(c.to(f64 if not fp8 else torch.float32).to(f64).cpu(), want,
+                                   rtol=u, atol=2 ** -9 if fp8 else 1e-5)
