@@ -853,7 +853,10 @@ def moe_routed_experts(x: torch.Tensor, weights: torch.Tensor, idx: torch.Tensor
     # rows of a tile by the rows an expert has on average (measured beside the kernel: taller
     # tiles read weights less often, lower ones leave more workgroups)
     mean = n / max(num_experts, E)
-    mt = 128 if mean > 64 else 64 if mean > 32 else 32
+    if scales:
+        mt = 64 if mean > 32 else 32
+    else:
+        mt = 128 if mean >= 48 else 64 if mean >= 24 else 32
     tiles_max = (n + min(n, E) * (mt - 1)) // mt
     rows = tiles_max * mt
     tabs = torch.empty(1 + 2 * tiles_max + rows + n, dtype=torch.int32, device=dev)

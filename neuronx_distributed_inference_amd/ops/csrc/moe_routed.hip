@@ -5,9 +5,8 @@
 // Bounds: with few rows an expert the weight stream (every chosen expert's weights once from
 // HBM); with many the matrix cores, and before those the LDS (128 B/clk a CU).
 //
-//   * Workgroup = 8 waves, MT rows of one expert x 256 columns (128 with 8-bit weights and
-//     MT = 128: their steps are 128 deep). K goes in steps of 128 B of a weight row through a
-//     ring of three LDS buffers, global_load_lds throughout, one raw barrier a step and a
+//   * Workgroup = 8 waves, MT rows of one expert x 256 columns. K goes in steps of 128 B of a
+//     weight row (128 deep with 8-bit weights, and then 64 rows at most) through a ring of three LDS buffers, global_load_lds throughout, one raw barrier a step and a
 //     counted vmcnt: two steps are in flight while one is computed.
 //   * The row tiles of an expert want the same weights: the list of workgroups (8 row tiles x
 //     all column tiles, rows fastest) is cut into 8 contiguous parts, one for each XCD, so that
@@ -29,7 +28,8 @@
 //     376 -> 309 (288).
 // Row tiles (32, 64, 128), gate + up and down with its sum: 32 rows an expert 164+102, 144+92,
 // 144+100 (64 rows 224+138, 172+118, 150+118); 128 rows 358+234, 237+185, 202+164;
-// 8 experts in 8 bits, 32 rows: 198+117, 185+143, 219+128 (32 fills more of the chip).
+// 8 experts in 8 bits, 32 rows: 198+117, 185+143 (32 fills more of the chip); 128 rows 474+280,
+//   380+267 (128 rows x 128 columns: 440+258).
 
 #include "common.h"
 #include <torch/extension.h>
@@ -89,7 +89,8 @@ DEV_INLINE float mr_act(float g, int gelu) {
 
 template <bool F8, int MT>
 struct MrTile {
-    static constexpr int BN = (F8 && MT == 128) ? 128 : 256;
+    static_assert(!F8 || MT < 128, "the ring would not fit");
+    static constexpr int BN = 256;
     static constexpr int BK = F8 ? 128 : 64;          // 128 B of a weight row
     static constexpr int XH = BK / 64;                // 128 B images of x a step
     static constexpr int WM = MT == 128 ? 2 : 1;      // waves along the rows
@@ -374,21 +375,24 @@ void mr_dispatch(void* y, const torch::Tensor& x, const torch::Tensor& w0,
     const bool f8 = s0 != nullptr, bf = x.scalar_type() == at::ScalarType::BFloat16;
 #define MR(TT, FF, MM) mr_launch<TT, FF, GLU, MM>(y, x, w0, w1, s0, s1, tiles, gather, max_tiles, \
                                                   col0, ncols, gelu, st)
-#define MR_M(TT, FF)                                                                              \
+#define MR_M(TT)                                                                                  \
     do {                                                                                          \
-        if (mt == 128) MR(TT, FF, 128);                                                           \
-        else if (mt == 64) MR(TT, FF, 64);                                                        \
-        else MR(TT, FF, 32);                                                                      \
+        if (f8 && mt == 64) MR(TT, true, 64);                                                     \
+        else if (f8) MR(TT, true, 32);                                                            \
+        else if (mt == 128) MR(TT, false, 128);                                                   \
+        else if (mt == 64) MR(TT, false, 64);                                                     \
+        else MR(TT, false, 32);                                                                   \
     } while (0)
-    if (bf) { if (f8) MR_M(__hip_bfloat16, true); else MR_M(__hip_bfloat16, false); }
-    else { if (f8) MR_M(__half, true); else MR_M(__half, false); }
+    if (bf) MR_M(__hip_bfloat16);
+    else MR_M(__half);
 #undef MR_M
 #undef MR
 }
 
 void mr_check(const torch::Tensor& x, const torch::Tensor& w, const c10::optional<torch::Tensor>& s,
               const torch::Tensor& tiles, long mt) {
-    TORCH_CHECK(mt == 32 || mt == 64 || mt == 128, "moe_routed: mt must be 32, 64 or 128");
+    TORCH_CHECK(mt == 32 || mt == 64 || (mt == 128 && !s.has_value()),
+                "moe_routed: mt must be 32, 64 or, with 16-bit weights, 128");
     TORCH_CHECK(x.dim() == 2 && w.dim() == 3 && x.size(1) == w.size(2), "moe_routed: shapes");
     TORCH_CHECK(x.is_contiguous() && w.is_contiguous() && tiles.is_contiguous(),
                 "moe_routed: contiguous tensors required");
