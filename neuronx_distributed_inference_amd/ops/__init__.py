@@ -831,6 +831,38 @@ def moe_grouped_gemm(x_sorted: torch.Tensor, w: torch.Tensor,
     return out if out is not None else y
 
 
+ROW_TOPK_MAX = 2048
+
+
+def row_max(x: torch.Tensor):
+    """(values, indices) of the last dim's largest elements, x.max(-1)."""
+    if x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32) and x.size(-1) > 0:
+        c = _require_ext("row_max")
+        rows = x.reshape(-1, x.size(-1))
+        rows = rows if rows.stride(1) == 1 else rows.contiguous()
+        vals = torch.empty(x.shape[:-1], dtype=x.dtype, device=x.device)
+        idx = torch.empty(x.shape[:-1], dtype=torch.long, device=x.device)
+        c.row_max(vals, idx, rows)
+        return vals, idx
+    return x.max(dim=-1)
+
+
+def row_topk(x: torch.Tensor, k: int):
+    """(values, indices) of the last dim's k largest elements in order, x.topk(k)."""
+    if (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32)
+            and 1 <= k <= min(ROW_TOPK_MAX, x.size(-1)) and x.numel() // x.size(-1) < 65536):
+        c = _require_ext("row_topk")
+        rows = x.reshape(-1, x.size(-1))
+        rows = rows if rows.stride(1) == 1 else rows.contiguous()
+        vals = torch.empty(*x.shape[:-1], k, dtype=x.dtype, device=x.device)
+        idx = torch.empty(*x.shape[:-1], k, dtype=torch.long, device=x.device)
+        ws = torch.empty(2 * rows.size(0) * k * -(-x.size(-1) // 4096), dtype=torch.long,
+                         device=x.device)
+        c.row_topk(vals, idx, rows, ws, k)
+        return vals, idx
+    return x.topk(k, dim=-1)
+
+
 # bytes of fp32 products that the routed down projection keeps at a time
 MOE_WORKSPACE = 1 << 30
 

@@ -91,6 +91,8 @@ void moe_routed_glu(torch::Tensor h, torch::Tensor x, torch::Tensor w_gate, torc
 void moe_routed_down(torch::Tensor out, torch::Tensor ws, torch::Tensor h, torch::Tensor w_down,
                      c10::optional<torch::Tensor> s_down, torch::Tensor tiles, torch::Tensor inv,
                      c10::optional<torch::Tensor> weights, long mt);
+void row_max(torch::Tensor val, torch::Tensor idx, torch::Tensor x);
+void row_topk(torch::Tensor val, torch::Tensor idx, torch::Tensor x, torch::Tensor ws, long k);
 void router_topk(torch::Tensor vals, torch::Tensor idx, torch::Tensor logits,
                  long top_k, long act_sigmoid, long pre_softmax,
                  long normalize);
@@ -159,6 +161,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("fp8_epilogue", &fp8_epilogue, "scaled-mm row-scale epilogue (CDNA4)",
           py::arg("out"), py::arg("y32"), py::arg("w_scale"),
           py::arg("bias") = py::none());
+    m.def("row_max", &row_max, "largest element of each row");
+    m.def("row_topk", &row_topk, "k largest elements of each row, in order");
     m.def("moe_route", &moe_route, "row tiles of the routed experts");
     m.def("moe_routed_glu", &moe_routed_glu, "gated expert projections over row tiles");
     m.def("moe_routed_down", &moe_routed_down, "expert down projection and weighted sum");

@@ -12,6 +12,7 @@ from __future__ import annotations
 import torch
 import torch.distributed as dist
 
+from neuronx_distributed_inference_amd import ops
 from neuronx_distributed_inference_amd.parallel import state as ps
 
 
@@ -25,7 +26,8 @@ def _group_info(group):
 def distributed_argmax(logits: torch.Tensor, dim: int = -1, group=None) -> torch.Tensor:
     """Greedy argmax over the full (sharded) vocab; returns global indices."""
     group, world, rank = _group_info(group)
-    local_max, local_idx = logits.max(dim=dim)
+    last = dim in (-1, logits.dim() - 1)
+    local_max, local_idx = ops.row_max(logits) if last else logits.max(dim=dim)
     if world == 1:
         return local_idx
     shard = logits.size(dim)
@@ -45,7 +47,9 @@ def distributed_topk(logits: torch.Tensor, k: int, dim: int = -1, group=None):
     """Top-k (values, global indices) over the sharded vocab dim."""
     group, world, rank = _group_info(group)
     k_local = min(k, logits.size(dim))
-    vals, idxs = logits.topk(k_local, dim=dim)
+    last = dim in (-1, logits.dim() - 1)
+    topk = ops.row_topk if last else lambda x, n: x.topk(n, dim=dim)
+    vals, idxs = topk(logits, k_local)
     if world == 1:
         return vals, idxs
     shard = logits.size(dim)
@@ -56,6 +60,6 @@ def distributed_topk(logits: torch.Tensor, k: int, dim: int = -1, group=None):
     dist.all_gather(gi, idxs.contiguous(), group=group)
     all_vals = torch.cat(gv, dim=dim)
     all_idxs = torch.cat(gi, dim=dim)
-    top_vals, pos = all_vals.topk(min(k, all_vals.size(dim)), dim=dim)
+    top_vals, pos = topk(all_vals, min(k, all_vals.size(dim)))
     top_idxs = all_idxs.gather(dim, pos)
     return top_vals, top_idxs

@@ -1625,3 +1625,74 @@ def test_qkv_rope_update_norms_and_pages(B, S, Hq, Hkv, D, dtype, norms, paged, 
         u = 2 ** -4 if fp8 else unit
         torch.testing.assert_close(c.to(f64 if not fp8 else torch.float32).to(f64).cpu(), want,
                                    rtol=u, atol=2 ** -9 if fp8 else 1e-5)
+
+
+@pytest.mark.parametrize("rows,n,k,dtype,stride", [
+    (1, 1, 1, torch.bfloat16, 0), (3, 7, 7, torch.float32, 0), (64, 4096, 50, torch.bfloat16, 0),
+    (2, 4097, 256, torch.float16, 0), (5, 32001, 256, torch.float32, 3),
+    (2, 128256, 256, torch.bfloat16, 8), (2, 151936, 2048, torch.float32, 0),
+])
+def test_row_topk(rows, n, k, dtype, stride):
+    """Row maximum and top-k are exact: values as torch's, equal values and signed zeros by index,
+    NaN first, rows of the lowest value, strided and misaligned rows, replays of a captured call."""
+    torch.manual_seed(n)
+    x = torch.randn(rows, n + stride).to(dtype)
+    if n > 6:
+        x[0, 3:6] = x[0].max() + 1                            # ties
+        x[-1, 1], x[-1, 4] = float("inf"), float("-inf")
+    if rows > 2:
+        x[1] = float("-inf")
+        x[2] = torch.where(torch.arange(n + stride) % 2 == 0, 0.0, -0.0)
+    if rows > 4:
+        x[3, 5] = float("nan")
+    xd = x.to(_dev())[:, :n]
+    x = x[:, :n]
+    key = torch.where(torch.isnan(x.float()), float("inf"), x.float())
+    order = torch.sort(key + 0.0, dim=-1, descending=True, stable=True).indices
+    if rows > 4:                                              # NaN before infinity
+        order[3] = torch.cat([torch.tensor([5]), order[3][order[3] != 5]])
+    vals, idx = ops.row_max(xd)
+    assert torch.equal(idx.cpu(), order[:, 0])
+    torch.testing.assert_close(vals.cpu(), x.gather(1, order[:, :1])[:, 0], rtol=0, atol=0,
+                               equal_nan=True)
+
+    def check(v, i):
+        assert torch.equal(i.cpu(), order[:, :k])
+        torch.testing.assert_close(v.cpu(), x.gather(1, order[:, :k]), rtol=0, atol=0,
+                                   equal_nan=True)
+
+    check(*ops.row_topk(xd, k))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        gv, gi = ops.row_topk(xd, k)
+    for _ in range(3):
+        gv.zero_(), gi.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        check(gv, gi)
+
+
+def test_captured_sampling_replays():
+    """A captured sampling step over a wide vocabulary replays: rows with top_k = 1 give the
+    largest logit of each replay's input, the others one of their top_k."""
+    from neuronx_distributed_inference_amd.config import OnDeviceSamplingConfig
+    from neuronx_distributed_inference_amd.modules.generation.sampling import create_sampler
+
+    torch.manual_seed(3)
+    sampler = create_sampler(OnDeviceSamplingConfig(do_sample=True, top_k=5), 128256)
+    logits = torch.randn(4, 128256, dtype=torch.bfloat16, device=_dev())
+    params = torch.tensor([[1, 1.0, 1.0], [5, 1.0, 1.0], [1, 0.9, 0.7], [5, 1.0, 1.0]],
+                          device=_dev())
+    sampler(logits, params)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        tok = sampler(logits, params)
+    for _ in range(3):
+        logits.copy_(torch.randn(4, 128256, device=_dev()))
+        graph.replay()
+        torch.cuda.synchronize()
+        five = logits.float().cpu().topk(5, -1)
+        for r in range(4):
+            value = logits[r, tok[r]].float().cpu()
+            assert value == five.values[r, 0] if r % 2 == 0 else value >= five.values[r, 4]
