@@ -1230,7 +1230,8 @@ __global__ void latent_decode_merge_kernel(const float* __restrict__ ws,
 }
 
 // ------------------------------------------------------- gated delta rule
-// Three kernels per step of few tokens (portions of 64 and more go in chunks, below).
+// Three kernels per step of few tokens (portions of 64 and more go in chunks, single tokens in
+// one launch, both below).
 // (1) delta_prep_kernel, fully parallel over tokens: unit q and k per KV head
 //     (q also scaled by D^-1/2), decay exp(-exp(A_log) softplus(a + dt_bias))
 //     per head and key channel, beta = sigmoid(.), all fp32, into one row per
@@ -1844,6 +1845,118 @@ __global__ void gated_rmsnorm_kernel(const float* __restrict__ o, const T* __res
     for (int c = lane; c < Dv; c += WAVE) {
         const float gv = ldf<T>(gp + c);
         stf<T>(op + c, ip[c] * inv * w[c] * (gate_silu ? gv * sigmoidf_(gv) : sigmoidf_(gv)));
+    }
+}
+
+// ---- the recurrence and its norm for one token a row, all in one launch
+// Bound by the state, once in and once out. A workgroup per (head, row): its 8 waves have the whole
+// state of the head (D <= 128, Dv <= 128) on the way before they prepare q, k and the decays (each
+// 16 lanes for themselves, 8 key channels a lane, four value channels a wave at a time), so the
+// small chains of the preparation hide behind it; the norm over the value channels goes through
+// LDS. 48 rows of 16 heads of 128 x 128 (101 MB): 26 us; the three kernels above took 56.
+template <typename T, int D>
+__global__ void __launch_bounds__(512)
+delta_step_kernel(const float* __restrict__ qkv, long cstride, const T* __restrict__ beta,
+                  long bstride, const T* __restrict__ a, long astride,
+                  const float* __restrict__ dt_bias, const float* __restrict__ a_log,
+                  const T* __restrict__ gate, long gstride, const float* __restrict__ norm_w,
+                  float eps, float* __restrict__ state, const int* __restrict__ pos,
+                  const int* __restrict__ seq, T* __restrict__ out, int H, int G, int Dv,
+                  int per_head, int gate_silu) {
+    constexpr int F = D / 64, NI = 4;            // float4s of a lane in a state row; rows of a lane
+    __shared__ float os[32 * NI];
+    const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
+    const int slot = seq[b], p = pos[b];
+    T* op = out + ((long)b * H + h) * Dv;
+    if (slot < 0 || p < 0) {                     // uniform over the workgroup
+        if (tid < Dv) stf<T>(op + tid, 0.f);
+        return;
+    }
+    const int lane = tid & 63, part = lane & 15, row0 = (tid >> 6) * 4 + (lane >> 4);
+    const int g = h / (H / G);
+    float* st = state + ((long)slot * H + h) * Dv * D + part * 4;
+    const float* vp = qkv + (long)b * cstride + 2L * G * D + (long)h * Dv;
+    float4 s[NI][F];
+    float v[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int r = min(row0 + 32 * i, Dv - 1);
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+            s[i][f] = *reinterpret_cast<const float4*>(st + (long)r * D + f * 64);
+        v[i] = vp[r];
+    }
+    float4 q[F], k[F], dec[F];
+    const float* qp = qkv + (long)b * cstride + (long)g * D + part * 4;
+    const T* ap = a + (long)b * astride + (per_head ? h : (long)h * D + part * 4);
+    const float* bp = dt_bias + (per_head ? h : h * D + part * 4);
+    float av[4 * F], bv[4 * F];
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        q[f] = *reinterpret_cast<const float4*>(qp + f * 64);
+        k[f] = *reinterpret_cast<const float4*>(qp + (long)G * D + f * 64);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            av[4 * f + e] = ldf<T>(ap + (per_head ? 0 : f * 64 + e));
+            bv[4 * f + e] = bp[per_head ? 0 : f * 64 + e];
+        }
+    }
+    const float bt = sigmoidf_(ldf<T>(beta + (long)b * bstride + h));
+    const float neg_rate = -expf(a_log[h]);
+    asm volatile("" ::: "memory");               // all of the above in flight
+    float sq = 0.f, sk = 0.f, qk = 0.f;
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        sq += q[f].x * q[f].x + q[f].y * q[f].y + q[f].z * q[f].z + q[f].w * q[f].w;
+        sk += k[f].x * k[f].x + k[f].y * k[f].y + k[f].z * k[f].z + k[f].w * k[f].w;
+        float* d = &dec[f].x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (per_head && (f || e)) d[e] = dec[0].x;
+            else d[e] = expf(neg_rate * softplusf_(av[4 * f + e] + bv[4 * f + e]));
+    }
+    const float iq = 1.f / sqrtf(part_sum<16>(sq) + 1e-6f) * (1.f / sqrtf((float)D));
+    const float ik = 1.f / sqrtf(part_sum<16>(sk) + 1e-6f);
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        q[f].x *= iq; q[f].y *= iq; q[f].z *= iq; q[f].w *= iq;
+        k[f].x *= ik; k[f].y *= ik; k[f].z *= ik; k[f].w *= ik;
+        qk += q[f].x * k[f].x + q[f].y * k[f].y + q[f].z * k[f].z + q[f].w * k[f].w;
+    }
+    qk = part_sum<16>(qk);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        float dot = 0.f, oq = 0.f;
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            float4& x = s[i][f];
+            if (p == 0) x = float4{0.f, 0.f, 0.f, 0.f};      // a sequence's first token
+            x.x *= dec[f].x; dot += x.x * k[f].x; oq += x.x * q[f].x;
+            x.y *= dec[f].y; dot += x.y * k[f].y; oq += x.y * q[f].y;
+            x.z *= dec[f].z; dot += x.z * k[f].z; oq += x.z * q[f].z;
+            x.w *= dec[f].w; dot += x.w * k[f].w; oq += x.w * q[f].w;
+        }
+        dot = part_sum<16>(dot);
+        oq = part_sum<16>(oq);
+        const float u = bt * (v[i] - dot);
+        const int r = row0 + 32 * i;
+        if (r < Dv) {
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                float4 x = s[i][f];
+                x.x += k[f].x * u; x.y += k[f].y * u; x.z += k[f].z * u; x.w += k[f].w * u;
+                *reinterpret_cast<float4*>(st + (long)r * D + f * 64) = x;
+            }
+            if (part == 0) os[r] = oq + u * qk;
+        }
+    }
+    __syncthreads();
+    float ss = 0.f;
+    for (int c = lane; c < Dv; c += WAVE) ss += os[c] * os[c];
+    const float inv = 1.f / sqrtf(wave_sum(ss) / Dv + eps);
+    if (tid < Dv) {
+        const float gv = ldf<T>(gate + (long)b * gstride + (long)h * Dv + tid);
+        stf<T>(op + tid, os[tid] * inv * norm_w[tid] * (gate_silu ? gv * sigmoidf_(gv) : sigmoidf_(gv)));
     }
 }
 
@@ -4776,6 +4889,20 @@ int nx_gated_delta(const float* qkv, long cstride, const void* beta, long bstrid
                    int Dv, int per_head, int gate_silu, float* ws, long ws_floats,
                    hipStream_t st) {
     if (B <= 0 || S <= 0) return 0;
+    if (!ws && !prep) {
+        // one token a row
+        if (S != 1 || (D != 64 && D != 128) || Dv > 128 || cstride % 4 || H % G || B > 65535)
+            return -1;
+        dim3 gs(H, B), bs(512);
+#define DST(TT, DD) delta_step_kernel<TT, DD><<<gs, bs, 0, st>>>( \
+        qkv, cstride, (const TT*)beta, bstride, (const TT*)a, astride, dt_bias, a_log, \
+        (const TT*)gate, gstride, norm_w, eps, state, pos, seq, (TT*)out, H, G, Dv, per_head, \
+        gate_silu)
+        if (in_bf16) { if (D == 64) DST(bf16, 64); else DST(bf16, 128); }
+        else { if (D == 64) DST(float, 64); else DST(float, 128); }
+#undef DST
+        return (int)hipGetLastError();
+    }
     if (D > 256 || H % G != 0 || (!ws && PS < (long)(2 * G + H) * D + H + G)) return -1;
     const long ntok = (long)B * S;
     if (ws) {

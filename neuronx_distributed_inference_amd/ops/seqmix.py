@@ -381,13 +381,17 @@ def gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps: float,
         assert qkv.dtype == torch.float32 and state.dtype == torch.float32
         assert beta.dtype == a.dtype == gate.dtype == out_dtype
         out = torch.empty(B, S, H * vdim, dtype=out_dtype, device=qkv.device)
-        obuf = torch.empty(B, S, H * vdim, dtype=torch.float32, device=qkv.device)
         PS = (2 * kv_heads + H) * dim + H + kv_heads
-        prep = ws = None
+        obuf = prep = ws = None
         unit = 49 * dim + 16 * vdim + 256          # floats of one 16-token chunk of a head
-        if S >= DELTA_CHUNK_MIN_TOKENS and dim in (64, 128) and vdim % 16 == 0 \
-                and _rows_view(qkv) % 4 == 0 and qkv.data_ptr() % 16 == 0 \
-                and state.data_ptr() % 16 == 0:
+        wide = (dim in (64, 128) and _rows_view(qkv) % 4 == 0 and qkv.data_ptr() % 16 == 0
+                and state.data_ptr() % 16 == 0)
+        one = wide and S == 1 and vdim <= 128 and B < 65536
+        if not one:
+            obuf = torch.empty(B, S, H * vdim, dtype=torch.float32, device=qkv.device)
+        if one:
+            pass                                   # one launch, nothing in between
+        elif wide and S >= DELTA_CHUNK_MIN_TOKENS and vdim % 16 == 0:
             span = max(1, min(-(-S // 16), DELTA_CHUNK_WORKSPACE // (4 * B * H * unit)))
             ws = torch.empty(span * B * H * unit, dtype=torch.float32, device=qkv.device)
         else:

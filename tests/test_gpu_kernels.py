@@ -1696,3 +1696,56 @@ def test_captured_sampling_replays():
         for r in range(4):
             value = logits[r, tok[r]].float().cpu()
             assert value == five.values[r, 0] if r % 2 == 0 else value >= five.values[r, 4]
+
+
+@pytest.mark.parametrize("B,H,G,D,Dv,per_head,silu,dtype", [
+    (1, 1, 1, 128, 128, False, False, torch.bfloat16), (5, 4, 2, 128, 72, True, True, torch.float32),
+    (7, 3, 3, 64, 128, False, False, torch.float32), (6, 16, 16, 64, 33, True, False, torch.bfloat16),
+])
+def test_gated_delta_one_token(B, H, G, D, Dv, per_head, silu, dtype):
+    """One token a row against 64 bits: first tokens over a slot of NaN, carried states, rows
+    without a token or a slot, value channels that do not fill the waves. 32-bit sums of 128
+    terms: 2e-6 (2-norm); in bf16 the result's own rounding comes on top."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    torch.manual_seed(D + Dv)
+    dev, f64 = _dev(), torch.float64
+    pos = (torch.arange(B) * 3 % 7).view(B, 1)
+    slots = torch.randperm(B + 1)[:B]
+    if B > 2:
+        pos[1], slots[2] = -1, -1
+    qkv = torch.randn(B, 1, 2 * G * D + H * Dv)
+    beta, gate = torch.randn(B, 1, H).to(dtype), torch.randn(B, 1, H * Dv).to(dtype)
+    a = (torch.randn(B, 1, H if per_head else H * D) * 2).to(dtype)
+    A_log, dt_bias, w = torch.linspace(-3, 3, H), torch.randn(a.shape[-1]), torch.randn(Dv)
+    state = torch.randn(B + 1, H, Dv, D) * 0.3
+    state[slots[0]] = float("nan")                            # position 0
+    st = state.to(dev)
+    step = seqmix.StepLayout(pos.to(dev), slots.to(dev))
+    out = seqmix.gated_delta_rule(qkv.to(dev), beta.to(dev), a.to(dev), dt_bias.to(dev),
+                                  A_log.to(dev), gate.to(dev), w.to(dev), 1e-5, st, step, G, D, Dv,
+                                  out_dtype=dtype, gate_act="silu" if silu else "sigmoid")
+    want, wstate = torch.zeros(B, 1, H * Dv, dtype=f64), state.to(f64)
+    for b in range(B):
+        if pos[b] < 0 or slots[b] < 0:
+            continue
+        x = qkv[b, 0].to(f64)
+        unit = lambda t: t * torch.rsqrt(t.square().sum(-1, keepdim=True) + 1e-6)  # noqa: E731
+        q = unit(x[:G * D].view(G, D)).repeat_interleave(H // G, 0) * D ** -0.5
+        k = unit(x[G * D:2 * G * D].view(G, D)).repeat_interleave(H // G, 0)
+        v = x[2 * G * D:].view(H, Dv)
+        dec = torch.exp(-A_log.to(f64).exp().view(H, 1) * torch.nn.functional.softplus(
+            a[b, 0].to(f64) + dt_bias.to(f64)).view(H, -1)).expand(H, D)
+        M = wstate[slots[b]] if pos[b] > 0 else torch.zeros(H, Dv, D, dtype=f64)
+        M = M * dec.unsqueeze(1)
+        u = torch.sigmoid(beta[b, 0].to(f64)).view(H, 1) * (v - (M * k.unsqueeze(1)).sum(-1))
+        M = M + u.unsqueeze(-1) * k.unsqueeze(1)
+        o = (M * q.unsqueeze(1)).sum(-1)
+        o = o * torch.rsqrt(o.square().mean(-1, keepdim=True) + 1e-5) * w.to(f64)
+        gv = gate[b, 0].to(f64)
+        want[b, 0] = o.reshape(-1) * torch.sigmoid(gv) * (gv if silu else 1)
+        wstate[slots[b]] = M
+    assert _rel(st, wstate) < 2e-6
+    assert _rel(out, want) < (4e-6 if dtype == torch.float32 else 2.0 ** -9)
+    if B > 2:
+        assert not out[1].any() and not out[2].any()
