@@ -459,7 +459,33 @@ window_attn_kernel(const T* __restrict__ q, long qstride, const T* __restrict__ 
                 slot = (long)(blk < 0 ? 0 : blk) * bsz + (j % bsz);
             }
             const T* kp = kc + slot * ktok + (long)g * khead;
-            if (kvec) {
+            constexpr int E16 = 16 / sizeof(T), LINE = 8 * E16;
+            if (MAXR <= 4 && kvec && Dk % LINE == 0) {     // (wider values leave no registers)
+                // a lane's whole 128 B line at once: 16 waves of 64 rows are far more than L1
+                // holds, and a line fetched 16 B at a time comes again from L2 (with the value
+                // loads below 47 -> 41 us: 48 rows, 16 heads of 128 on 4 KV heads, 700 keys)
+                for (int d = 0; d < Dk; d += LINE) {
+                    uint4 raw[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        raw[u] = *reinterpret_cast<const uint4*>(kp + d + u * E16);
+                    asm volatile("" ::: "memory");       // all eight in flight
+#pragma unroll
+                    for (int u = 0; u < 8; u += 8 / E16) {
+                        float kv[8];
+                        load8<T>(reinterpret_cast<const T*>(raw + u), kv);
+#pragma unroll
+                        for (int r = 0; r < ATT_NQ; ++r) {
+                            if (rpos[r] < 0) continue;   // uniform
+                            const float* qr = qs + r * DkP + d + u * E16;
+                            const float4 qa = *reinterpret_cast<const float4*>(qr);
+                            const float4 qb = *reinterpret_cast<const float4*>(qr + 4);
+                            sc[r] += kv[0] * qa.x + kv[1] * qa.y + kv[2] * qa.z + kv[3] * qa.w +
+                                     kv[4] * qb.x + kv[5] * qb.y + kv[6] * qb.z + kv[7] * qb.w;
+                        }
+                    }
+                }
+            } else if (kvec) {
                 for (int d = 0; d < Dk; d += 8) {
                     float kv[8];
                     load8<T>(kp + d, kv);
@@ -528,19 +554,37 @@ window_attn_kernel(const T* __restrict__ q, long qstride, const T* __restrict__ 
                     done = true;
                     const int ksub = WAVE / lpr;
                     const int sub = lane / lpr, ch = (lane % lpr) * 8;
-                    for (int it = 0; it * ksub < cnt; ++it) {
-                        const int mm = it * ksub + sub;
-                        const long sj = __shfl(sl, mm < cnt ? mm : 0, WAVE);
-                        if (mm < cnt) {
+                    // several key groups' loads in flight; keys past the tile's last count 0
+                    constexpr int U = MAXR <= 4 ? 4 : 1;
+                    for (int it = 0; it * ksub < cnt; it += U) {
+                        T vr[U][8];
+                        float4 pp[U];
+#pragma unroll
+                        for (int u = 0; u < U; ++u) {
+                            const int mm = (it + u) * ksub + sub;
+                            const bool in = mm < cnt;
+                            const long sj = __shfl(sl, in ? mm : 0, WAVE);
+                            const uint4* vp = reinterpret_cast<const uint4*>(
+                                vc + sj * vtok + (long)g * vhead + ch);
+#pragma unroll
+                            for (int x = 0; x < (int)sizeof(T) / 2; ++x)
+                                *reinterpret_cast<uint4*>(&vr[u][x * (16 / sizeof(T))]) = vp[x];
+                            pp[u] = *reinterpret_cast<const float4*>(myp + (in ? mm : 0) * ATT_NQ);
+                            if (!in) pp[u] = float4{0.f, 0.f, 0.f, 0.f};
+                        }
+                        asm volatile("" ::: "memory");
+#pragma unroll
+                        for (int u = 0; u < U; ++u) {
                             float vv[8];
-                            load8<T>(vc + sj * vtok + (long)g * vhead + ch, vv);
-                            const float4 pp = *reinterpret_cast<const float4*>(myp + mm * ATT_NQ);
+                            load8<T>(vr[u], vv);
+                            const bool in = (it + u) * ksub + sub < cnt;
 #pragma unroll
                             for (int e = 0; e < 8; ++e) {
-                                acc8[0][e] += pp.x * vv[e];
-                                acc8[1][e] += pp.y * vv[e];
-                                acc8[2][e] += pp.z * vv[e];
-                                acc8[3][e] += pp.w * vv[e];
+                                const float v = in ? vv[e] : 0.f;
+                                acc8[0][e] += pp[u].x * v;
+                                acc8[1][e] += pp[u].y * v;
+                                acc8[2][e] += pp[u].z * v;
+                                acc8[3][e] += pp[u].w * v;
                             }
                         }
                     }

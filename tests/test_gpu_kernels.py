@@ -1749,3 +1749,47 @@ def test_gated_delta_one_token(B, H, G, D, Dv, per_head, silu, dtype):
     assert _rel(out, want) < (4e-6 if dtype == torch.float32 else 2.0 ** -9)
     if B > 2:
         assert not out[1].any() and not out[2].any()
+
+
+@pytest.mark.parametrize("S,H,G,Dk,Dv,dtype,window,keep", [
+    (1, 4, 1, 128, 128, torch.bfloat16, 300, 3), (1, 6, 2, 64, 64, torch.float32, None, 0),
+    (1, 2, 2, 72, 256, torch.bfloat16, None, 0), (1, 3, 1, 96, 40, torch.float32, 70, 0),
+    (3, 4, 2, 64, 128, torch.float32, 130, 1),
+])
+def test_window_attention_key_and_value_loads(S, H, G, Dk, Dv, dtype, window, keep):
+    """Windowed paged attention against 64 bits: key rows of whole 128-byte lines and others,
+    one key to several tiles, pages that nobody wrote hold NaN. fp32 scores and sums: 2e-6; in
+    bf16 the result's rounding, 2^-9, and as much for a hardware logarithm (2^-8)."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    torch.manual_seed(Dk + Dv)
+    dev, f64, bs = _dev(), torch.float64, 16
+    lens = [1, 63, 64, 65, 1100, 517]
+    B, nb = len(lens), 80
+    lens = [max(n, S) for n in lens]
+    kc = torch.full((B * nb, bs, G, Dk), float("nan"), dtype=dtype)
+    vc = torch.full((B * nb, bs, G, Dv), float("nan"), dtype=dtype)
+    table = torch.randperm(B * nb).view(B, nb).int()
+    q = torch.randn(B, S, H * Dk).to(dtype)
+    r1, r2 = torch.rand(H), torch.rand(H) * 0.1
+    pos = torch.stack([torch.arange(n - S, n) for n in lens])
+    want = torch.zeros(B, S, H, Dv, dtype=f64)
+    for b, n in enumerate(lens):
+        k, v = torch.randn(n, G, Dk).to(dtype), torch.randn(n, G, Dv).to(dtype)
+        rows = table[b].long()[torch.arange(n) // bs]
+        kc[rows, torch.arange(n) % bs], vc[rows, torch.arange(n) % bs] = k, v
+        for page in table[b].long()[:-(-n // bs)]:            # a written page is finite
+            kc[page], vc[page] = kc[page].nan_to_num(0.0), vc[page].nan_to_num(0.0)
+        for s in range(S):
+            i, j = n - S + s, torch.arange(n - S + s + 1)
+            x = torch.einsum("hd,jhd->hj", q[b, s].view(H, Dk).to(f64),
+                             k[j].to(f64).repeat_interleave(H // G, 1)) * Dk ** -0.5
+            x -= r1.to(f64).view(H, 1) * torch.log1p(r2.to(f64).view(H, 1) * (i - j))
+            if window:
+                x[:, ~((i - j < window) | (j < keep))] = float("-inf")
+            want[b, s] = torch.einsum("hj,jhd->hd", torch.softmax(x, -1),
+                                      v[j].to(f64).repeat_interleave(H // G, 1))
+    step = seqmix.StepLayout(pos.to(dev), torch.arange(B, device=dev))
+    out = seqmix.paged_attention(q.to(dev), kc.to(dev), vc.to(dev), step, table.to(dev), Dk ** -0.5,
+                                 H, window=window, keep_first=keep, r1=r1.to(dev), r2=r2.to(dev))
+    assert _rel(out, want.reshape(B, S, -1)) < (2e-6 if dtype == torch.float32 else 2.0 ** -8)
