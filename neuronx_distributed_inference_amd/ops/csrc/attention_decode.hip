@@ -771,6 +771,7 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
     const int Hkv = paged ? k_cache.size(2) : k_cache.size(1);
     const int max_blocks = paged ? (int)block_table->size(1) : 0;
     const int Smax = paged ? max_blocks * block_size : (int)k_cache.size(2);
+    if (Smax == 0) ring = 0;               // the kernels divide by a ring's size
     constexpr bool MFMA = !std::is_same<T, float>::value && (D == 64 || D == 128);
     const int nct = (gq * Sq + 15) / 16;
     // Splits over the keys. Matrix-core kernel: two workgroups fit a CU, so 512 fill the chip;
@@ -785,7 +786,8 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
         const int least = Smax <= 2048 ? 128 : 256;
         nsplit = 512 / std::max(1, B * Hkv * nct);
         nsplit = std::max(1, std::min({nsplit, (Smax + least - 1) / least, 64}));
-        chunk = ((Smax + nsplit - 1) / nsplit + DM_TILE - 1) / DM_TILE * DM_TILE;
+        // (a cache of no rows has one split, which reads nothing and writes zeros)
+        chunk = std::max(DM_TILE, ((Smax + nsplit - 1) / nsplit + DM_TILE - 1) / DM_TILE * DM_TILE);
         nsplit = std::max(1, (Smax + chunk - 1) / chunk);
     } else {
         nsplit = 1024 / std::max(1, B * Hkv * Sq);

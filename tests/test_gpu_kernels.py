@@ -1793,3 +1793,25 @@ def test_window_attention_key_and_value_loads(S, H, G, Dk, Dv, dtype, window, ke
     out = seqmix.paged_attention(q.to(dev), kc.to(dev), vc.to(dev), step, table.to(dev), Dk ** -0.5,
                                  H, window=window, keep_first=keep, r1=r1.to(dev), r2=r2.to(dev))
     assert _rel(out, want.reshape(B, S, -1)) < (2e-6 if dtype == torch.float32 else 2.0 ** -8)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.float16, 64), (torch.float32, 64)])
+@pytest.mark.parametrize("Sq", [1, 3])
+@pytest.mark.parametrize("kind", ["linear", "ring", "paged", "lse"])
+def test_attention_decode_empty_cache(dtype, D, Sq, kind):
+    """A cache without rows (a block table without columns): zeros, and -inf for the log-sum-exp."""
+    dev, B, Hkv, gq = _dev(), 2, 2, 4
+    q = torch.randn(B, Hkv * gq, Sq, D, device=dev).to(dtype)
+    pos = torch.zeros(B, Sq, dtype=torch.int32, device=dev)
+    if kind == "paged":
+        pages = torch.randn(3, 16, Hkv, D, device=dev).to(dtype)
+        out = ops.attention_decode_paged(q, pages, pages, pos,
+                                         torch.empty(B, 0, dtype=torch.int32, device=dev))
+    else:
+        cache = torch.empty(B, Hkv, 0, D, device=dev, dtype=dtype)
+        if kind == "lse":
+            out, lse = ops.attention_decode_lse(q, cache, cache, pos)
+            assert torch.equal(lse.cpu(), torch.full((B, Hkv * gq, Sq), float("-inf")))
+        else:
+            out = ops.attention_decode(q, cache, cache, pos, ring=kind == "ring")
+    assert out.shape == q.shape and not out.any()
