@@ -342,7 +342,14 @@ __global__ __launch_bounds__(256) void decode_attn_pass1(
 //     order. V rows are loaded in that order, 16 bytes of channels a lane (a whole row for
 //     16 lanes), and turned in registers: one byte permutation makes a B operand word. Which
 //     channels a column of the product stands for is free, so nothing else moves.
-//   * P enters as a high and a low 16-bit part: its error stays below that of 32-bit sums.
+//   * P enters as three 16-bit parts that add up to its 24 bits. (Two parts: 64 rows of 2048 73.1
+//     us for 73.9, of an 8-bit cache 38.6 for 40.7. 32-bit matrix instructions, which need no
+//     parts: 81 and 55.) fp16 has no exponents for small parts: there P is lifted by 2^7, and its
+//     reference follows a 32-key step down that stays more than 2^8 below it, so that P at each
+//     step's largest lies in [2^-1, 2^15]. The accumulator is scaled up meanwhile, by 2^64 at
+//     most: far from overflow, and what lies deeper is less than a 32-bit sum keeps. One key
+//     whose values are 10^-4 of the others' ahead of 60000 at e^-19, fp16, error 2-norm: 1.9e-4
+//     (two parts and one reference 4.2e-3, 32-bit multiply-adds of scaled queries 5.1e-4).
 //   * Loads of the next 32 keys are in flight while these are computed (two register
 //     buffers, 16 KB a wave); waves of a workgroup take 32-key tiles in turn and meet in LDS
 //     once at the end.
@@ -364,6 +371,16 @@ template <> struct DmTraits<__hip_bfloat16> {
     static DEV_INLINE dm_f32x4 mfma(vec8 a, vec8 b, dm_f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
     }
+    // a 16-bit part of each value, taken off it
+    static DEV_INLINE vec8 part(float (&e)[8]) {
+        vec8 p;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            p[j] = (__bf16)e[j];
+            e[j] -= (float)p[j];
+        }
+        return p;
+    }
     static DEV_INLINE unsigned cvt2(unsigned w, bool hi) {   // two e4m3 -> two bf16, exact
         return __builtin_bit_cast(unsigned, hi
             ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, true)
@@ -375,6 +392,17 @@ template <> struct DmTraits<__half> {
     using elem = _Float16;
     static DEV_INLINE dm_f32x4 mfma(vec8 a, vec8 b, dm_f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+    }
+    static DEV_INLINE vec8 part(float (&e)[8]) {
+        dm_u32x4 p;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {          // towards zero: in pairs, what is left is exact
+            const auto h = __builtin_amdgcn_cvt_pkrtz(e[2 * j], e[2 * j + 1]);
+            p[j] = __builtin_bit_cast(unsigned, h);
+            e[2 * j] -= (float)h[0];
+            e[2 * j + 1] -= (float)h[1];
+        }
+        return __builtin_bit_cast(vec8, p);
     }
     static DEV_INLINE unsigned cvt2(unsigned w, bool hi) {
         return __builtin_bit_cast(unsigned, hi
@@ -402,6 +430,7 @@ template <int NE, bool F8> struct DmRaw {
 };
 
 constexpr float DM_GROWTH = 8.f;   // log2 growth of a maximum that is put off
+constexpr float DM_DEPTH = 64.f;   // and how far below the largest score P may count from (fp16)
 constexpr int DM_TILE = 32;        // keys of a wave's step
 
 template <typename T, typename CT, int D, bool PAGED>
@@ -418,6 +447,8 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
     using DT = DmTraits<T>;
     using vec8 = typename DT::vec8;
     constexpr bool F8 = sizeof(CT) == 1;
+    constexpr bool F16 = std::is_same<T, __half>::value;
+    constexpr float LIFT = F16 ? 7.f : 0.f;
     constexpr int NKS = D / 32;            // k-steps of K Q^T
     constexpr int DV = D / 16;             // channels a lane holds of a V row
     constexpr int ES = sizeof(CT);
@@ -521,7 +552,8 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
     dm_f32x4 o[DV];
 #pragma unroll
     for (int i = 0; i < DV; ++i) o[i] = {0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;          // of column n; l: of this lane's keys
+    // of column n; what P counts from, l: of this lane's keys, largest score so far (fp16)
+    float m = -INFINITY, l = 0.f, top = -INFINITY;
     const float sc = scale * 1.4426950408889634f;
 
     auto step = [&](Buf& u, int t) {
@@ -549,8 +581,16 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
         }
         mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE_SIZE));
         mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE_SIZE));
-        if (__any(mx > m + DM_GROWTH || (m == -INFINITY && mx > m))) {
-            const float mn = fmaxf(m, mx);
+        bool move = mx > m + DM_GROWTH || (m == -INFINITY && mx > m);
+        float mn = fmaxf(m, mx);
+        if constexpr (F16) {               // and down to a step that stays far below
+            top = fmaxf(top, mx);
+            if (mx < m - DM_GROWTH && mx != -INFINITY) {
+                mn = fmaxf(mx, top - DM_DEPTH);
+                move = mn < m;
+            }
+        }
+        if (__any(move)) {
             const float f = m == -INFINITY ? 0.f : exp2f(m - mn);
             m = mn;
             l *= f;
@@ -562,15 +602,16 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
                 for (int i = 0; i < DV; ++i) o[i][r] *= fr;
             }
         }
-        const float mu = m == -INFINITY ? 0.f : m;
-        vec8 p, p_lo;
+        const float mu = m == -INFINITY ? 0.f : m - LIFT;
+        float e[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const float e = __builtin_amdgcn_exp2f(x[j] - mu);
-            l += e;
-            p[j] = (typename DT::elem)e;
-            p_lo[j] = (typename DT::elem)(e - (float)p[j]);
+            e[j] = __builtin_amdgcn_exp2f(x[j] - mu);
+            l += e[j];
         }
+        vec8 p[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) p[c] = DT::part(e);
         // V: pairs of channels of 8 keys -> for each channel, pairs of keys
         unsigned vp[8][DV / 2];
 #pragma unroll
@@ -591,8 +632,8 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
                 w[e] = __builtin_amdgcn_perm(vp[2 * e + 1][i >> 1], vp[2 * e][i >> 1],
                                              (i & 1) ? 0x07060302u : 0x05040100u);
             const vec8 vb = __builtin_bit_cast(vec8, w);
-            o[i] = DT::mfma(p, vb, o[i]);
-            o[i] = DT::mfma(p_lo, vb, o[i]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) o[i] = DT::mfma(p[c], vb, o[i]);
         }
     };
 
@@ -617,6 +658,7 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
     }
     l += __shfl_xor(l, 16, WAVE_SIZE);
     l += __shfl_xor(l, 32, WAVE_SIZE);
+    m -= LIFT;
 
     // ---- the four waves meet ----
     extern __shared__ __attribute__((aligned(16))) float dm_lds[];

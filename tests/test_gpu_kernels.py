@@ -1815,3 +1815,37 @@ def test_attention_decode_empty_cache(dtype, D, Sq, kind):
         else:
             out = ops.attention_decode(q, cache, cache, pos, ring=kind == "ring")
     assert out.shape == q.shape and not out.any()
+
+
+def _peaked(n, Sq, dtype, lead, at, seed=0):
+    """Queries and a cache of n rows whose scores are about equal but for one row, `lead` ahead (nats), whose
+    values are 10^-4 of the others': what the result owes to the tail is not small."""
+    g = torch.Generator().manual_seed(seed)
+    q = (1 + 0.01 * torch.randn(1, 4, Sq, 128, generator=g)).to(dtype)
+    k = 0.02 * torch.randn(1, 1, n, 128, generator=g)
+    v = 1 + torch.randn(1, 1, n, 128, generator=g)
+    k[:, :, at], v[:, :, at] = lead * 128 ** -0.5, 1e-4
+    k, v = k.to(dtype), v.to(dtype)
+    pos = (n - Sq + torch.arange(Sq)).view(1, Sq)
+    s = (q.double() @ k.double().transpose(2, 3)) * 128 ** -0.5
+    s = s.masked_fill(torch.arange(n).view(1, 1, 1, n) > pos.view(1, 1, Sq, 1), float("-inf"))
+    return q, k, v, pos, torch.softmax(s, -1) @ v.double()
+
+
+@pytest.mark.parametrize("lead,at,fp8", [(16, 5, False), (19, 5, False), (19, 7001, False),
+                                         (28, 3000, False), (40, 5, False), (16, 5, True),
+                                         (19, 3000, True)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_attention_decode_keeps_the_tail(dtype, lead, at, fp8):
+    """Probabilities far below the largest are not lost: 7002 keys at e^-lead of one. What is left is
+    the rounding of the result: results of about one value, 1.4e-4, just above a power of two, where
+    errors spread evenly over half a unit, 2^-8 in bf16 and 2^-11 in fp16, have a 2-norm of that by
+    the root of 3; and 2^-20 for the 32-bit sums (2^-24, a few dozen terms of one size each). An
+    8-bit cache holds 16 times the values, so that the result is one that fp16 has."""
+    q, k, v, pos, want = _peaked(7002, 1, dtype, lead, at)
+    if fp8:
+        k, v = k.to(torch.float8_e4m3fn), (16 * v.float()).to(torch.float8_e4m3fn)
+        s = (q.double() @ k.double().transpose(2, 3)) * 128 ** -0.5
+        want = torch.softmax(s, -1) @ v.double()
+    got = ops.attention_decode(q.to(_dev()), k.to(_dev()), v.to(_dev()), pos.to(_dev()))
+    assert _rel(got, want) < 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * 3 ** -0.5 + 2.0 ** -20
