@@ -13,10 +13,15 @@
 //     the other half wave for the maximum of 64 keys, none for the sum until the end).
 //   * P never leaves the registers: the C layout of S^T holds, for a lane, runs of 4
 //     consecutive keys; read as the B operand of O^T = V^T P^T they are the same 16 keys in
-//     another order, and V^T is read in that order. Over a cache P enters the second product
-//     as a high and a low 16-bit part (HILO): single tokens are attended with 32-bit
-//     probabilities, and several must not get less. V stays row-major in LDS: ds_read_b64_tr
+//     another order, and V^T is read in that order. V stays row-major in LDS: ds_read_b64_tr
 //     transposes 4 keys x 16 channels on the way to the registers.
+//   * Over a cache P enters the second product as three 16-bit parts (HILO), which add up to its
+//     24 bits: single tokens are attended with 32-bit probabilities, and several do not get less.
+//     (One part more than the two that random inputs need for the same measured error: 512 tokens
+//     over 4000, linear 69 -> 81 us, paged 83 -> 98.) In fp16, which has no exponents for small
+//     parts, P is lifted by 2^7 and its reference follows a tile that stays more than 2^8 below
+//     it, so that P at each tile's largest lies in [2^-1, 2^15]; the accumulator is scaled up
+//     meanwhile, by 2^64 at most. Prompts from an empty cache: one 16-bit part, as ever.
 //   * The accumulator is rescaled only when a row's maximum grew by more than 2^8 since the
 //     last time; probabilities and sums share the stale maximum, so nothing is lost.
 //   * K and V tiles of 64 keys go straight to LDS (global_load_lds, 16 B a lane), two
@@ -33,13 +38,14 @@
 //                                     matrix pipe, the rest exponentials it does not hide)
 //   prompt of 2048, head size 128/64  179 -> 54 us / 145 -> 39 us
 //   prompt of 512 / 128               40 -> 16 us / 16 -> 9 us
-//   512 tokens over 4000, linear/paged 1772 -> 80 us / 2019 -> 95 us (62 / 79 with P in 16 bits)
-//   64 tokens over 4000, linear       237 -> 32 us
-//   32 rows of 6 tokens over 2000     354 -> 49 us (a verification step)
-//   1 row of 2 tokens over 2000       28 -> 19 us
+//   512 tokens over 4000, linear/paged 1574 -> 81 us / 1749 -> 98 us
+//   64 tokens over 4000, linear       237 -> 34 us
+//   32 rows of 6 tokens over 2000     351 -> 50 us (a verification step)
+//   1 row of 2 tokens over 2000       28 -> 18 us
 // No size was found at which several tokens are better off one by one. Error against 64 bits
-// over a cache, bf16, 2-norm: 1.65e-3 (the rounding of the result; one by one 1.65e-3 to
-// 2.35e-3, 2.3e-3 with P in 16 bits), fp16 2.07e-4.
+// over a cache, bf16, 2-norm: 1.7e-3 (the rounding of the result; one by one 2.4e-3, fp16 2.1e-4
+// and 3.0e-4); with one key far ahead of 60000 at e^-19 whose values are 10^-4 of the others',
+// fp16: 2.0e-4 (one by one 4.0e-4; with two parts and one reference 6.2e-2).
 
 #include "common.h"
 #include <torch/extension.h>
@@ -52,6 +58,7 @@ typedef _Float16 fa_f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 fa_bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 fa_f16x4 __attribute__((ext_vector_type(4)));
 typedef short fa_s16x4 __attribute__((ext_vector_type(4)));
+typedef unsigned fa_u32x4 __attribute__((ext_vector_type(4)));
 typedef float fa_f32x16 __attribute__((ext_vector_type(16)));
 
 template <typename T> struct FaTraits;
@@ -62,6 +69,16 @@ template <> struct FaTraits<__hip_bfloat16> {
     static DEV_INLINE fa_f32x16 mfma(vec8 a, vec8 b, fa_f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }
+    // a 16-bit part of each value, taken off it
+    static DEV_INLINE vec8 part(float (&e)[8]) {
+        vec8 p;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            p[j] = (elem)e[j];
+            e[j] -= (float)p[j];
+        }
+        return p;
+    }
 };
 template <> struct FaTraits<__half> {
     using vec8 = fa_f16x8;
@@ -70,11 +87,23 @@ template <> struct FaTraits<__half> {
     static DEV_INLINE fa_f32x16 mfma(vec8 a, vec8 b, fa_f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
     }
+    static DEV_INLINE vec8 part(float (&e)[8]) {
+        fa_u32x4 p;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {          // towards zero: in pairs, what is left is exact
+            const auto h = __builtin_amdgcn_cvt_pkrtz(e[2 * j], e[2 * j + 1]);
+            p[j] = __builtin_bit_cast(unsigned, h);
+            e[2 * j] -= (float)h[0];
+            e[2 * j + 1] -= (float)h[1];
+        }
+        return __builtin_bit_cast(vec8, p);
+    }
 };
 
 constexpr int QROWS = 128;      // query rows of a workgroup
 constexpr int KT = 64;          // keys of a tile
 constexpr float FA_GROWTH = 8.f;  // log2 growth of a maximum that is put off
+constexpr float FA_DEPTH = 64.f;  // and how far below the largest score P may count from (fp16)
 
 // the other half wave's value
 DEV_INLINE float half_swap(float x) {
@@ -121,6 +150,9 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
     constexpr int TILE_B = KT * ROWB;
     constexpr int NKS = D / 16;            // k-steps of Q K^T
     constexpr int NDB = D / 32;            // 32-channel blocks of the output
+    constexpr int NP = HILO ? 3 : 1;       // 16-bit parts of P
+    constexpr bool FOLLOW = HILO && std::is_same<T, __half>::value;
+    constexpr float LIFT = FOLLOW ? 7.f : 0.f;
 
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // [2 buffers][K tile | V tile], then block bounds and the paged tiles' bad-row marks
@@ -268,7 +300,8 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
     for (int i = 0; i < NDB; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
-    float m = -INFINITY, l = 0.f;      // m: the maximum in use (log2 units); l: this half's sum
+    // m: what P counts from (log2 units); l: this half's sum; top: the largest score (FOLLOW)
+    float m = -INFINITY, l = 0.f, top = -INFINITY;
 
     // fragment addresses within a tile
     const int ka_row = lane & 31;
@@ -356,8 +389,16 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[n][r]);
         mx = fmaxf(mx, half_swap(mx)) * c;
-        if (__any(mx > m + FA_GROWTH || (m == -INFINITY && mx > m))) {
-            const float mn = fmaxf(m, mx);
+        bool move = mx > m + FA_GROWTH || (m == -INFINITY && mx > m);
+        float mn = fmaxf(m, mx);
+        if constexpr (FOLLOW) {                         // and down to a tile that stays far below
+            top = fmaxf(top, mx);
+            if (mx < m - FA_GROWTH && mx != -INFINITY) {
+                mn = fmaxf(mx, top - FA_DEPTH);
+                move = mn < m;
+            }
+        }
+        if (__any(move)) {
             const float f = m == -INFINITY ? 0.f : exp2f(m - mn);
             m = mn;
             l *= f;
@@ -366,7 +407,7 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
 #pragma unroll
                 for (int r = 0; r < 16; ++r) o[i][r] *= f;
         }
-        const float mu = m == -INFINITY ? 0.f : m;      // a row that has seen no key yet
+        const float mu = m == -INFINITY ? 0.f : m - LIFT;   // (0: a row that has seen no key yet)
 #pragma unroll
         for (int n = 0; n < 2; ++n)
 #pragma unroll
@@ -377,12 +418,18 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
             }
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
-            vec8 p, p_lo;
+            vec8 p[NP];
+            {
+                float e[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float e = s[kt >> 1][(kt & 1) * 8 + j];
-                p[j] = (typename FT::elem)e;
-                if constexpr (HILO) p_lo[j] = (typename FT::elem)(e - (float)p[j]);
+                for (int j = 0; j < 8; ++j) e[j] = s[kt >> 1][(kt & 1) * 8 + j];
+                if constexpr (HILO) {
+#pragma unroll
+                    for (int c = 0; c < NP; ++c) p[c] = FT::part(e);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) p[0][j] = (typename FT::elem)e[j];
+                }
             }
 #pragma unroll
             for (int db = 0; db < NDB; ++db) {
@@ -398,22 +445,22 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
 #pragma unroll
                     for (int e = 0; e < 4; ++e) va[j * 4 + e] = y[e];
                 }
-                o[db] = FT::mfma(va, p, o[db]);
-                if constexpr (HILO) o[db] = FT::mfma(va, p_lo, o[db]);
+#pragma unroll
+                for (int c = 0; c < NP; ++c) o[db] = FT::mfma(va, p[c], o[db]);
             }
         }
-        constexpr int PER = HILO ? 2 : 1;
         __builtin_amdgcn_sched_group_barrier(0x100, 8, 1);
 #pragma unroll
         for (int i = 0; i < 4 * NDB - 4; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, PER, 1);
+            __builtin_amdgcn_sched_group_barrier(0x008, NP, 1);
             __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, 4 * PER, 1);
+        __builtin_amdgcn_sched_group_barrier(0x008, 4 * NP, 1);
     }
 
     // ---- epilogue: rows of 4 channels from 8*(r>>2) + 4*half ----
     l += half_swap(l);
+    m -= LIFT;
     if (r_own >= R) return;
     if (qpos < 0) {                    // padding: tiles that are whole for the others ran unmasked
         m = -INFINITY;
@@ -439,9 +486,13 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
                     float4{o[db][g * 4], o[db][g * 4 + 1], o[db][g * 4 + 2], o[db][g * 4 + 3]};
         return;
     }
-    if (a.sinks != nullptr && m != -INFINITY)           // a sink joins the denominator only
-        l += exp2f(a.sinks[head] * 1.4426950408889634f - m);
-    const float inv = l > 0.f ? 1.f / l : 0.f;
+    float f = 1.f;
+    if (a.sinks != nullptr && m != -INFINITY) {         // a sink joins the denominator only
+        const float sk = a.sinks[head] * 1.4426950408889634f, mt = fmaxf(m, sk);
+        f = exp2f(m - mt);
+        l = l * f + exp2f(sk - mt);
+    }
+    const float inv = l > 0.f ? f / l : 0.f;
     T* po = out + b * a.ob + head * a.oh + token * a.os;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
@@ -466,6 +517,7 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(T* __restrict__ out,
     const int b = (int)(rowid / a.S / a.Hq);
     float m = -INFINITY;
     for (int i = 0; i < a.nsplit; ++i) m = fmaxf(m, a.ml_part[(i * rows + rowid) * 2]);
+    if (a.sinks != nullptr && m != -INFINITY) m = fmaxf(m, a.sinks[head] * 1.4426950408889634f);
     constexpr int PER = D / 64;
     float acc[PER], L = 0.f;
 #pragma unroll

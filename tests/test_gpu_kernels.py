@@ -1849,3 +1849,19 @@ def test_attention_decode_keeps_the_tail(dtype, lead, at, fp8):
         want = torch.softmax(s, -1) @ v.double()
     got = ops.attention_decode(q.to(_dev()), k.to(_dev()), v.to(_dev()), pos.to(_dev()))
     assert _rel(got, want) < 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * 3 ** -0.5 + 2.0 ** -20
+
+
+@pytest.mark.parametrize("lead,at", [(16, 5), (19, 5), (19, 6999), (28, 3000), (40, 5)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("paged", [False, True])
+def test_attention_extend_keeps_the_tail(dtype, lead, at, paged):
+    """As for single tokens, for several; one workgroup's range holds the leading key, or none does."""
+    q, k, v, pos, want = _peaked(7008, 3, dtype, lead, at)
+    dev = _dev()
+    if paged:
+        pk, pv = (t.view(438, 16, 1, 128).to(dev) for t in (k, v))
+        got = ops.attention_decode_paged(q.to(dev), pk, pv, pos.to(dev),
+                                         torch.arange(438, device=dev).view(1, -1))
+    else:
+        got = ops.attention_decode(q.to(dev), k.to(dev), v.to(dev), pos.to(dev))
+    assert _rel(got, want) < 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * 3 ** -0.5 + 2.0 ** -20
