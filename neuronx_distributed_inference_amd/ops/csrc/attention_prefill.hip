@@ -245,8 +245,8 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
     }
 
     const float c0 = a.scale * 1.4426950408889634f;   // scores in log2 units
-    const bool flip = c0 < 0.f;
-    const float c = flip ? -c0 : c0;
+    // c multiplies masked scores too, which are -inf: positive, so that they stay it
+    const float sign = c0 == 0.f ? 0.f : c0 < 0.f ? -1.f : 1.f, c = c0 == 0.f ? 1.f : fabsf(c0);
 
     // ---- staging: this lane's rows and source slots ----
     const int st_row = wid * (KT / 4) + lane / SLOTS;  // + i * RPI
@@ -364,11 +364,11 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
         __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-        if (flip) {
+        if (sign != 1.f) {
 #pragma unroll
             for (int n = 0; n < 2; ++n)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s[n][r] = -s[n][r];
+                for (int r = 0; r < 16; ++r) s[n][r] *= sign;
         }
         bool masked = (k0 + KT - 1 > wmin) || (k0 < w_in);
         if constexpr (PAGED) masked = masked || s_bad[buf * (KT + 1)] == t;

@@ -1865,3 +1865,34 @@ def test_attention_extend_keeps_the_tail(dtype, lead, at, paged):
     else:
         got = ops.attention_decode(q.to(dev), k.to(dev), v.to(dev), pos.to(dev))
     assert _rel(got, want) < 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * 3 ** -0.5 + 2.0 ** -20
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16)])
+@pytest.mark.parametrize("kind", ["prompt", "cached", "extend", "split", "paged", "decode"])
+@pytest.mark.parametrize("scale", [0.0, -0.0, -0.1])
+def test_attention_scale_zero_and_below(D, dtype, kind, scale):
+    """A scale of zero is the uniform average of the visible values, a negative one turns the order
+    of the scores; masked keys stay out. Rounding of the probabilities (prompts) and of the result,
+    half a unit each of 2^-7 and 2^-10, and half as much again for the sums."""
+    torch.manual_seed(D)
+    dev, B, Hkv, gq = _dev(), 2, 2, 2
+    S = {"split": 4, "decode": 1}.get(kind, 130)
+    cap = 1024 if kind == "split" else 144
+    q = torch.randn(B, Hkv * gq, S, D).to(dtype)
+    k, v = (torch.randn(B, Hkv, cap, D).to(dtype) for _ in range(2))
+    first = 0 if kind in ("prompt", "cached") else cap - S - 3
+    pos = first + torch.arange(S).expand(B, S)
+    mask = torch.arange(cap).view(1, 1, 1, cap) <= pos.view(B, 1, S, 1)
+    want = ref.sdpa(q.float(), k.float(), v.float(), mask=mask, scale=scale)
+    qd, kd, vd, pd = (t.to(dev) for t in (q, k, v, pos))
+    if kind == "prompt":
+        got = ops.attention_prefill(qd, kd[:, :, :S], vd[:, :, :S], scale=scale)
+    elif kind == "cached":
+        got = ops.attention_prefill_cached(qd, kd, vd, torch.arange(B, device=dev), scale=scale)
+    elif kind == "paged":
+        pages = [t.transpose(1, 2).reshape(B * cap // 16, 16, Hkv, D).contiguous() for t in (kd, vd)]
+        got = ops.attention_decode_paged(qd, *pages, pd, torch.arange(B * cap // 16, device=dev)
+                                         .view(B, -1), scale=scale)
+    else:
+        got = ops.attention_decode(qd, kd, vd, pd, scale=scale)
+    assert _rel(got, want) < 1.5 * 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
