@@ -686,17 +686,18 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
 #pragma unroll
         for (int w = 0; w < 4; ++w) ms = fmaxf(ms, ml_lds[(w * 16 + cl) * 2]);
         float4 acc = {0.f, 0.f, 0.f, 0.f};
-        if (ms != -INFINITY) {
 #pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                const float f = exp2f(ml_lds[(w * 16 + cl) * 2] - ms);
-                ls += f * ml_lds[(w * 16 + cl) * 2 + 1];
-                const float4 y = *reinterpret_cast<const float4*>(o_lds + (w * nc + cl) * D + d);
-                acc.x += f * y.x;
-                acc.y += f * y.y;
-                acc.z += f * y.z;
-                acc.w += f * y.w;
-            }
+        for (int w = 0; w < 4; ++w) {
+            const float lw = ml_lds[(w * 16 + cl) * 2 + 1];
+            if (lw == 0.f) continue;       // no key seen
+            // (no maximum, but a sum: it is NaN, as of a query that is, and stays)
+            const float f = ms == -INFINITY ? 1.f : exp2f(ml_lds[(w * 16 + cl) * 2] - ms);
+            ls += f * lw;
+            const float4 y = *reinterpret_cast<const float4*>(o_lds + (w * nc + cl) * D + d);
+            acc.x += f * y.x;
+            acc.y += f * y.y;
+            acc.z += f * y.z;
+            acc.w += f * y.w;
         }
         const long rowid = ((long)b * Hq + hh) * Sq + cc / gq;
         const float mn = ms * 0.6931471805599453f;     // natural units from here on

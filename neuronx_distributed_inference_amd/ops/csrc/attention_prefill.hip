@@ -462,7 +462,9 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
     l += half_swap(l);
     m -= LIFT;
     if (r_own >= R) return;
-    if (qpos < 0) {                    // padding: tiles that are whole for the others ran unmasked
+    // padding (tiles that are whole for the others ran unmasked), or no key seen. A sum that is
+    // NaN, as of a query that is, has no maximum either and stays
+    if (qpos < 0 || l == 0.f) {
         m = -INFINITY;
         l = 0.f;
 #pragma unroll
@@ -476,7 +478,7 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
             a.ml_part[at * 2] = m;
             a.ml_part[at * 2 + 1] = l;
         }
-        if (m == -INFINITY) return;                     // nothing seen: the weight is 0
+        if (l == 0.f) return;                           // nothing seen: the weight is 0
         float* po = a.o_part + at * D;
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
@@ -522,17 +524,16 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(T* __restrict__ out,
     float acc[PER], L = 0.f;
 #pragma unroll
     for (int j = 0; j < PER; ++j) acc[j] = 0.f;
-    if (m != -INFINITY) {
-        for (int i = 0; i < a.nsplit; ++i) {
-            const float mi = a.ml_part[(i * rows + rowid) * 2];
-            if (mi == -INFINITY) continue;
-            const float f = exp2f(mi - m);
-            L += f * a.ml_part[(i * rows + rowid) * 2 + 1];
+    for (int i = 0; i < a.nsplit; ++i) {
+        const float mi = a.ml_part[(i * rows + rowid) * 2];
+        const float li = a.ml_part[(i * rows + rowid) * 2 + 1];
+        if (li == 0.f) continue;
+        const float f = mi == -INFINITY ? 1.f : exp2f(mi - m);      // (1: a sum of NaN)
+        L += f * li;
 #pragma unroll
-            for (int j = 0; j < PER; ++j) acc[j] += f * a.o_part[(i * rows + rowid) * D + lane * PER + j];
-        }
-        if (a.sinks != nullptr) L += exp2f(a.sinks[head] * 1.4426950408889634f - m);
+        for (int j = 0; j < PER; ++j) acc[j] += f * a.o_part[(i * rows + rowid) * D + lane * PER + j];
     }
+    if (a.sinks != nullptr && m != -INFINITY) L += exp2f(a.sinks[head] * 1.4426950408889634f - m);
     const float inv = L > 0.f ? 1.f / L : 0.f;
     T* po = out + b * a.ob + head * a.oh + token * a.os + lane * PER;
 #pragma unroll

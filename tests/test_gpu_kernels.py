@@ -1896,3 +1896,37 @@ def test_attention_scale_zero_and_below(D, dtype, kind, scale):
     else:
         got = ops.attention_decode(qd, kd, vd, pd, scale=scale)
     assert _rel(got, want) < 1.5 * 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16)])
+@pytest.mark.parametrize("cap,Sq", [(96, 1), (4096, 1), (96, 5), (4096, 5), (4096, 1200)])
+@pytest.mark.parametrize("kind", ["linear", "fp8", "paged", "sinks"])
+def test_attention_nan_query_stays(D, dtype, cap, Sq, kind):
+    """A query (or the keys it meets) that is NaN gives NaN, with one split over the keys or many;
+    the other rows are what they are without it."""
+    torch.manual_seed(cap + Sq)
+    dev, B, Hkv, gq, n = _dev(), 2, 2, 3, min(cap, 3000) - 10
+    if Sq > n:
+        pytest.skip("more tokens than rows")
+    q = torch.randn(B, Hkv * gq, Sq, D, device=dev).to(dtype)
+    k, v = (torch.randn(B, Hkv, cap, D, device=dev).to(dtype) for _ in range(2))
+    if kind == "fp8":
+        k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+    pos = (n - Sq + torch.arange(Sq, device=dev)).expand(B, Sq)
+    sinks = torch.randn(Hkv * gq, device=dev) if kind == "sinks" else None
+
+    def run(q):
+        if kind == "paged":
+            pages = [t.transpose(1, 2).reshape(B * cap // 16, 16, Hkv, D).contiguous()
+                     for t in (k, v)]
+            return ops.attention_decode_paged(q, *pages, pos, torch.arange(
+                B * cap // 16, device=dev).view(B, -1))
+        return ops.attention_decode(q, k, v, pos, sinks=sinks)
+
+    want = run(q)
+    bad = q.clone()
+    bad[1, 2, Sq // 2] = float("nan")
+    got = run(bad)
+    assert bool(torch.isnan(got[1, 2, Sq // 2]).all())
+    got[1, 2, Sq // 2] = want[1, 2, Sq // 2]
+    assert torch.isfinite(want).all() and torch.equal(got, want)
