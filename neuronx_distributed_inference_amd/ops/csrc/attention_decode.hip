@@ -17,6 +17,7 @@
 // structure flash-decoding (seq-sharded KV, ref C5) extends across GPUs.
 
 #include "common.h"
+#include "attention_row.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -678,7 +679,10 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
                 float4{o[i][r], o[i + 1][r], o[i + 2][r], o[i + 3][r]};
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < nc * (D / 4); idx += 256) {
+    // (whole waves, for the rows that are done again: a column is 32 or 16 lanes of one)
+    for (int base = wid * 64; base < nc * (D / 4); base += 256) {
+        const bool in = base + lane < nc * (D / 4);
+        const int idx = in ? base + lane : base;
         const int cl = idx / (D / 4), d = idx % (D / 4) * 4;
         const int cc = c0 + cl;
         const int hh = hkv * gq + cc % gq;
@@ -699,6 +703,37 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
             acc.z += f * y.z;
             acc.w += f * y.w;
         }
+        // columns whose sums are finite and whose values are not: see attention_row.h
+        const bool lost = !((acc.x + acc.y) * 0.f + (acc.z + acc.w) * 0.f == 0.f) && ls == ls;
+        unsigned long long bad = __ballot(lost);
+        while (bad) {
+            const int first_lane = __ffsll(bad) - 1, cb = (base + first_lane) / (D / 4);
+            const int cq = (c0 + cb) / gq, pos = row >= 0 ? positions[(long)b * Sq + cq] : -1;
+            int from = 0;
+            if (window > 0) from = max(0, pos - window + 1);
+            else if (window < 0 && !ring) from = pos >= 0 ? pos / -window * -window : 0;
+            float mr, lr, y[D / 64];
+            attend_row<D>(q + (((long)b * Hq + hkv * gq + (c0 + cb) % gq) * Sq + cq) * D,
+                          k_cache, v_cache, k_lo, k_hi, sc, [&](int key) -> long {
+                const int at = key + ring_base - (key > ring_at ? Smax : 0);
+                if (at > pos || at < from) return -1;
+                if constexpr (PAGED) {
+                    const int p = block_table[(long)b * max_blocks + key / block_size];
+                    return p < 0 ? -1 : (((long)p * block_size + key % block_size) * Hkv + hkv) * D;
+                }
+                return (((long)max(row, 0) * Hkv + hkv) * (long)Smax + key) * D;
+            }, mr, lr, y);
+            float z[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z[e] = __shfl(y[e % (D / 64)], (d + e) / (D / 64), WAVE_SIZE);
+            if (cl == cb) {
+                ms = mr;
+                ls = lr;
+                acc = float4{z[0], z[1], z[2], z[3]};
+            }
+            bad &= ~__ballot(cl == cb);
+        }
+        if (!in) continue;
         const long rowid = ((long)b * Hq + hh) * Sq + cc / gq;
         const float mn = ms * 0.6931471805599453f;     // natural units from here on
         if (nsplit > 1) {

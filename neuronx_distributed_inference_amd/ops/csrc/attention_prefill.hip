@@ -48,6 +48,7 @@
 // fp16: 2.0e-4 (one by one 4.0e-4; with two parts and one reference 6.2e-2).
 
 #include "common.h"
+#include "attention_row.h"
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -461,6 +462,50 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
     // ---- epilogue: rows of 4 channels from 8*(r>>2) + 4*half ----
     l += half_swap(l);
     m -= LIFT;
+    if constexpr (HILO) {
+        // rows whose sums are finite and whose values are not: see attention_row.h
+        float z[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NDB; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) z[r & 3] += o[i][r] * 0.f;
+        const bool lost = !((z[0] + z[1]) + (z[2] + z[3]) == 0.f);
+        const unsigned long long bad =
+            __ballot(lost && l == l && l != 0.f && qpos >= 0 && r_own < R);
+        for (unsigned rest = (unsigned)bad | (unsigned)(bad >> 32); rest; rest &= rest - 1) {
+            const int own = __ffs(rest) - 1;
+            const long at = ((long)b * a.Hq + __shfl(head, own, WAVE_SIZE)) * a.S +
+                            __shfl(token, own, WAVE_SIZE);
+            float mr, lr, acc[D / 64];
+            attend_row<D>(q + at * D, k, v, max(__shfl(key_lo, own, WAVE_SIZE), t_lo * KT),
+                          min(__shfl(qpos, own, WAVE_SIZE) + 1, t_hi * KT), c0,
+                          [&](int key) -> long {
+                if constexpr (PAGED) {
+                    const int p = a.block_table[(long)b * a.max_blocks + key / a.block_size];
+                    return p < 0 ? -1 : (((long)p * a.block_size + key % a.block_size) * a.Hkv + hkv) * D;
+                }
+                return lin + (long)key * D;
+            }, mr, lr, acc);
+            // through the tile buffer that the last tile did not use, a part for each wave
+            float* row_lds = reinterpret_cast<float*>(smem + ((t_hi - t_lo) & 1) * 2 * TILE_B +
+                                                      wid * (TILE_B / 2));
+#pragma unroll
+            for (int e = 0; e < D / 64; ++e) row_lds[lane * (D / 64) + e] = acc[e];
+            __builtin_amdgcn_wave_barrier();
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if ((lane & 31) == own) {
+                m = mr;
+                l = lr;
+#pragma unroll
+                for (int i = 0; i < NDB; ++i)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        o[i][r] = row_lds[i * 32 + 8 * (r >> 2) + 4 * half + (r & 3)];
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
     if (r_own >= R) return;
     // padding (tiles that are whole for the others ran unmasked), or no key seen. A sum that is
     // NaN, as of a query that is, has no maximum either and stays

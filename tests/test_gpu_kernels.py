@@ -1930,3 +1930,98 @@ def test_attention_nan_query_stays(D, dtype, cap, Sq, kind):
     assert bool(torch.isnan(got[1, 2, Sq // 2]).all())
     got[1, 2, Sq // 2] = want[1, 2, Sq // 2]
     assert torch.isfinite(want).all() and torch.equal(got, want)
+
+
+def _attend_visible(q, k, v, pos, window=0, scale=None):
+    """Attention in 64 bits that reads the visible keys of each row alone; pos (B, S), -1: no row."""
+    B, H, S, D = q.shape
+    out = torch.zeros(B, H, S, D, dtype=torch.float64)
+    g = H // k.shape[1]
+    for b in range(B):
+        for s in range(S):
+            p = int(pos[b, s])
+            if p < 0:
+                continue
+            lo = max(0, p - window + 1) if window > 0 else p // -window * -window if window else 0
+            kk = k[b, :, lo:p + 1].double().repeat_interleave(g, 0)
+            vv = v[b, :, lo:p + 1].double().repeat_interleave(g, 0)
+            x = (kk * q[b, :, s].double().unsqueeze(1)).sum(-1) * (scale or D ** -0.5)
+            out[b, :, s] = (torch.softmax(x, -1).unsqueeze(-1) * vv).sum(1)
+    return out
+
+
+def _same_but_not_finite(got, want, tol):
+    """Infinities and NaN where the reference has them, the rest within tol (2-norm)."""
+    got = got.double().cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.where(torch.isinf(got), got, 0.0), torch.where(torch.isinf(want), want, 0.0))
+    ok = torch.isfinite(want)
+    assert bool(ok.any()) and _rel(got[ok], want[ok]) < tol
+
+
+@pytest.mark.parametrize("D,gq,dtype", [(128, 4, torch.bfloat16), (64, 1, torch.float16)])
+@pytest.mark.parametrize("start,Sq", [(0, 40), (500, 6), (200, 70)])
+@pytest.mark.parametrize("window", [0, 50, -64])
+@pytest.mark.parametrize("paged", [False, True])
+def test_attention_extend_values_not_finite(D, gq, dtype, start, Sq, window, paged):
+    """Values of a token that are not finite reach that token and later ones, and none before it (or
+    past their window): NaN, and infinities as infinities. The rounding of the result, 2^-9 and 2^-12."""
+    torch.manual_seed(start + D)
+    dev, B, Hkv, cap = _dev(), 2, 2, 640
+    q = torch.randn(B, Hkv * gq, Sq, D).to(dtype)
+    k, v = (torch.randn(B, Hkv, cap, D).to(dtype) for _ in range(2))
+    pos = start + torch.arange(Sq).expand(B, Sq)
+    inf = float("inf")
+    v[0, 0, start + Sq // 2, 3] = float("nan")
+    v[0, 1, start + Sq // 2, 5:9] = inf
+    v[1, 0, start + Sq - 1, 7] = -inf
+    v[1, 0, start + Sq:] = float("nan")
+    if start:
+        v[1, 1, start - 20, 1] = inf                          # in no window of the last tokens
+    want = _attend_visible(q, k, v, pos, window)
+    qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
+    kw = dict(sliding_window=window)
+    if paged:
+        pages = [t.transpose(1, 2).reshape(B * cap // 16, 16, Hkv, D).contiguous() for t in (kd, vd)]
+        table = torch.arange(B * cap // 16, device=dev).view(B, -1)
+        got = ops.attention_decode_paged(qd, *pages, pos.to(dev), table, **kw)
+    else:
+        got = ops.attention_decode(qd, kd, vd, pos.to(dev), **kw)
+    _same_but_not_finite(got, want, 2.0 ** (-8.5 if dtype == torch.bfloat16 else -11.5))
+
+
+@pytest.mark.parametrize("D,gq,dtype", [(128, 4, torch.bfloat16), (64, 3, torch.float16)])
+@pytest.mark.parametrize("Sq", [1, 5])
+@pytest.mark.parametrize("window", [0, 50])
+@pytest.mark.parametrize("kind", ["linear", "fp8", "paged", "lse", "ring"])
+def test_attention_decode_values_not_finite(D, gq, dtype, Sq, window, kind):
+    """Values that are not finite in rows that a token does not see (before its window, behind it,
+    of later tokens of the same step) do not reach it; those that it sees do."""
+    torch.manual_seed(D + Sq)
+    dev, B, Hkv, cap = _dev(), 3, 2, 640
+    fp8 = kind == "fp8"
+    q = torch.randn(B, Hkv * gq, Sq, D).to(dtype)
+    k, v = (torch.randn(B, Hkv, cap, D).to(dtype) for _ in range(2))
+    last = torch.tensor([70, 333, 600])
+    pos = last.view(B, 1) - Sq + 1 + torch.arange(Sq)
+    nan, inf = float("nan"), float("nan") if fp8 else float("inf")
+    for b in range(B):
+        n = int(last[b])
+        v[b, 0, n - 50 - Sq:n - 49 - Sq + 1, ::3] = nan      # around the first window's start
+        v[b, 0, n, 4], v[b, :, n + 1:] = inf, nan
+        v[b, 1, n - 5, 6] = -inf
+    if fp8:
+        k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+    kd, vd, qd, pd = k.to(dev), v.to(dev), q.to(dev), pos.to(dev)
+    want = _attend_visible(q, k.float(), v.float(), pos, window)
+    kw = dict(sliding_window=window)
+    if kind == "paged":
+        pages = [t.transpose(1, 2).reshape(B * cap // 16, 16, Hkv, D).contiguous() for t in (kd, vd)]
+        got = ops.attention_decode_paged(qd, *pages, pd, torch.arange(B * cap // 16, device=dev)
+                                         .view(B, -1), **kw)
+    elif kind == "lse":
+        got, lse = ops.attention_decode_lse(qd, kd, vd, pd, **kw)
+        assert torch.isfinite(lse).all()
+    else:
+        got = ops.attention_decode(qd, kd, vd, pd, ring=kind == "ring", **kw)
+    _same_but_not_finite(got, want, 2.0 ** (-8.5 if dtype == torch.bfloat16 else -11.5))
