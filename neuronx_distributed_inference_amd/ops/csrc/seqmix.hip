@@ -1732,6 +1732,24 @@ delta_chunk_scan_kernel(const float* __restrict__ ws, float* __restrict__ state,
             dc_f32x4 oo = exo[c & 1][0][lane];
 #pragma unroll
             for (int w = 1; w < 4; ++w) oo += exo[c & 1][w][lane];
+            if (__any(!((uu[0] + uu[1]) * 0.f + (uu[2] + uu[3]) * 0.f == 0.f))) {
+                // a token whose update is not finite: P is 0 for the tokens before it, but
+                // 0 * NaN is not. Row by row, over the tokens that each one sees
+                for (int w = 0; w < 4; ++w)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float us = __shfl(uu[e], r16 + 16 * w, WAVE);
+                        // (an infinite update makes infinities of both signs in the state)
+                        const float later = us + us * 0.f;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const float ps = __shfl(prev.p[e], g * 4 + r + 16 * w, WAVE);
+                            const int over = g * 4 + r - (w * 4 + e);
+                            if (over >= 0) oo[r] += ps * (over ? later : us);
+                        }
+                    }
+                return oo;
+            }
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 oo = __builtin_amdgcn_mfma_f32_16x16x4f32(prev.p[r], uu[r], oo, 0, 0, 0);

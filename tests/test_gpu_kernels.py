@@ -2025,3 +2025,39 @@ def test_attention_decode_values_not_finite(D, gq, dtype, Sq, window, kind):
     else:
         got = ops.attention_decode(qd, kd, vd, pd, ring=kind == "ring", **kw)
     _same_but_not_finite(got, want, 2.0 ** (-8.5 if dtype == torch.bfloat16 else -11.5))
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float32)])
+@pytest.mark.parametrize("part,bad", [("v", 0), ("v", 37), ("v", 99), ("q", 37), ("k", 50), ("a", 64),
+                                      ("beta", 15), ("gate", 16)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_gated_delta_chunks_not_finite(D, dtype, part, bad, value, monkeypatch):
+    """A token that is not finite reaches itself and later tokens, none before it in its chunk:
+    NaN where the token-by-token kernel has it, the rest as there, within twice the 2-norm of the
+    rounding to the output's type (or 1e-5 for the order of 32-bit sums)."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    torch.manual_seed(D)
+    dev, S, H, Dv, B = _dev(), 100, 2, 32, 2
+    pos = torch.arange(S, device=dev).expand(B, S)
+    t = {"qkv": torch.randn(B, S, 2 * H * D + H * Dv, device=dev),
+         "beta": torch.randn(B, S, H, device=dev).to(dtype),
+         "a": torch.randn(B, S, H * D, device=dev).to(dtype),
+         "gate": torch.randn(B, S, H * Dv, device=dev).to(dtype)}
+    name, at = {"q": ("qkv", 3), "k": ("qkv", H * D + 3), "v": ("qkv", 2 * H * D + 3)}.get(part, (part, 1))
+    t[name][0, bad, at] = value
+    A_log, dt_bias, w = (torch.randn(n, device=dev) for n in (H, H * D, Dv))
+    state = torch.randn(B, H, Dv, D, device=dev) * 0.3
+    res = []
+    for least in (1, 1 << 30):
+        monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN_TOKENS", least)
+        st = state.clone()
+        step = seqmix.StepLayout(pos, torch.arange(B, device=dev))
+        out = seqmix.gated_delta_rule(t["qkv"], t["beta"], t["a"], dt_bias, A_log, t["gate"], w, 1e-5,
+                                      st, step, H, D, Dv, out_dtype=dtype)
+        res.append((out.double().cpu(), st.double().cpu()))
+    for got, want in zip(*res):
+        fin = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got), fin)
+        assert _rel(got[fin], want[fin]) < (1e-5 if dtype == torch.float32 else 2.0 ** -8)
+    assert torch.isfinite(res[0][0][0, :bad]).all() and torch.isfinite(res[0][0][1]).all()
