@@ -268,6 +268,7 @@ class AttentionBase(nn.Module):
             and not (getattr(kv_mgr, "ring_layers", None)
                      and kv_mgr.is_ring(self.layer_idx))
             and (not hidden.is_cuda or self.head_dim in (64, 128))
+            and not (norms and hidden.dtype == torch.float32)
         ):
             kc, vc = kv_mgr.get_cache(self.layer_idx)
             kc = kc.data if hasattr(kc, "data") else kc
@@ -280,10 +281,18 @@ class AttentionBase(nn.Module):
                     y, cos, sin, kc, vc, position_ids, seq_ids,
                     self.num_heads_per_rank, self.num_kv_heads_per_rank, norms=norms or None,
                 )
-                out = _ops.attention_prefill_cached(
-                    q, kc, vc, seq_ids, scale=self.scale, sinks=self.sinks,
-                    sliding_window=self.sliding_window,
-                )
+                if norms and attention_mask is not None:
+                    # by position, which counts the mask's tokens wherever they stand, with
+                    # probabilities in 32 bits as on the masked path
+                    out = _ops.attention_decode(
+                        q, kc, vc, position_ids, seq_ids=seq_ids, scale=self.scale,
+                        sinks=self.sinks, sliding_window=self.sliding_window,
+                    )
+                else:
+                    out = _ops.attention_prefill_cached(
+                        q, kc, vc, seq_ids, scale=self.scale, sinks=self.sinks,
+                        sliding_window=self.sliding_window,
+                    )
                 out = out.transpose(1, 2).reshape(B, S, -1)
                 return self.o_proj(out)
 

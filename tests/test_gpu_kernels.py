@@ -2061,3 +2061,64 @@ def test_gated_delta_chunks_not_finite(D, dtype, part, bad, value, monkeypatch):
         assert torch.equal(torch.isfinite(got), fin)
         assert _rel(got[fin], want[fin]) < (1e-5 if dtype == torch.float32 else 2.0 ** -8)
     assert torch.isfinite(res[0][0][0, :bad]).all() and torch.isfinite(res[0][0][1]).all()
+
+
+def _normed_attention(dtype, S, B):
+    """An attention layer with head norms, its rotary table and a cache, on the GPU."""
+    from neuronx_distributed_inference_amd.config import EngineConfig
+    from neuronx_distributed_inference_amd.models.qwen3.modeling_qwen3 import (
+        Qwen3ForCausalLM, Qwen3InferenceConfig)
+
+    name = str(dtype).split(".")[1]
+    ec = EngineConfig(batch_size=B, max_batch_size=B, seq_len=S + 8, max_length=S + 8,
+                      torch_dtype=name, tp_degree=1, fused_qkv=True)
+    cfg = Qwen3InferenceConfig(
+        neuron_config=ec, vocab_size=64, hidden_size=256, intermediate_size=256, head_dim=64,
+        num_hidden_layers=1, num_attention_heads=4, num_key_value_heads=2,
+        max_position_embeddings=S + 8, rms_norm_eps=1e-5, hidden_act="silu")
+    with torch.device("cuda"):
+        lm = Qwen3ForCausalLM(cfg).eval()
+    for p in lm.parameters():
+        if p.requires_grad:
+            p.data.normal_(0, 0.06)
+    att = lm.model.layers[0].self_attn
+    for n in (att.q_norm, att.k_norm):
+        n.weight.data.uniform_(0.5, 1.5)
+    return lm.model, att
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("kind", ["right", "left", "holes"])
+def test_normed_prompt_with_a_mask(dtype, kind, monkeypatch):
+    """A masked prompt of a model with head norms: the fused front end gives what the unfused,
+    masked path gives, wherever the mask's zeros stand. Both round q and k (the unfused one twice),
+    the result and the projection: six roundings of half a unit, in fp32 the order of sums."""
+    torch.manual_seed(1)
+    dev, B, S = _dev(), 3, 90
+    model, att = _normed_attention(dtype, S, B)
+    h = torch.randn(B, S, 256, device=dev).to(dtype)
+    mask = torch.ones(B, S, dtype=torch.long, device=dev)
+    if kind == "right":
+        mask[1, 40:], mask[2, 1:] = 0, 0
+    elif kind == "left":
+        mask[1, :40], mask[2, :1] = 0, 0
+    else:
+        mask[1, 20:50], mask[2, ::3] = 0, 0
+    pos = torch.where(mask > 0, mask.cumsum(-1) - 1, -1)
+    cos, sin = model.rotary.get_cos_sin(pos, device=dev)
+    seq = torch.tensor([2, 0, 1], device=dev, dtype=torch.int32)
+
+    def run():
+        with torch.inference_mode():
+            return att(h, cos, sin, model.kv_mgr, pos.int(), "context_encoding",
+                       attention_mask=mask, seq_ids=seq)
+
+    got = run()
+    rows = [c.clone() for c in model.kv_mgr.get_cache(0)]
+    monkeypatch.setattr(type(att), "_front_norms", lambda *a: None)
+    want = run()
+    keep = mask > 0
+    tol = {torch.float32: 1e-5, torch.float16: 6 * 2.0 ** -11, torch.bfloat16: 6 * 2.0 ** -8}[dtype]
+    assert _rel(got[keep], want[keep]) < tol
+    for a, b in zip(rows, model.kv_mgr.get_cache(0)):
+        assert _rel(a, b) < tol
