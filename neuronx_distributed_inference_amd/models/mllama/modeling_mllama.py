@@ -320,7 +320,7 @@ class _MllamaTextCrossAttention(nn.Module):
             # the HIP decode kernel
             pos = torch.full((B, S), k.shape[2] - 1, device=x.device,
                              dtype=torch.int32)
-            a = ops.attention_decode(q, k, v, pos, scale=self.scale)
+            a = ops.attention_decode(q, k, v, pos, scale=self.scale, token_major=True)
         return self.o_proj(a.transpose(1, 2).reshape(B, S, -1))
 
 

@@ -91,7 +91,8 @@ class _WhisperAttention(nn.Module):
         causal self cache and the static cross-attention K/V."""
         B, S, _ = x.shape
         q = self._shape(self.q_proj(x))
-        out = ops.attention_decode(q, k_cache, v_cache, eff_lens, scale=self.scale)
+        out = ops.attention_decode(q, k_cache, v_cache, eff_lens, scale=self.scale,
+                                   token_major=True)
         return self.out_proj(out.transpose(1, 2).reshape(B, S, -1))
 
 

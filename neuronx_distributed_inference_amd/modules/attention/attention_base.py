@@ -287,11 +287,12 @@ class AttentionBase(nn.Module):
                     out = _ops.attention_decode(
                         q, kc, vc, position_ids, seq_ids=seq_ids, scale=self.scale,
                         sinks=self.sinks, sliding_window=self.sliding_window,
+                        token_major=True,
                     )
                 else:
                     out = _ops.attention_prefill_cached(
                         q, kc, vc, seq_ids, scale=self.scale, sinks=self.sinks,
-                        sliding_window=self.sliding_window,
+                        sliding_window=self.sliding_window, token_major=True,
                     )
                 out = out.transpose(1, 2).reshape(B, S, -1)
                 return self.o_proj(out)
@@ -466,7 +467,7 @@ class AttentionBase(nn.Module):
         out = ops.attention_decode(
             q_shard, k_cache, v_cache, position_ids[lo:lo + per],
             seq_ids=local_rows[lo:lo + per], scale=self.scale, sinks=self.sinks,
-            sliding_window=self.sliding_window,
+            sliding_window=self.sliding_window, token_major=True,
         )
         out = out.transpose(1, 2).reshape(per, S, -1)
         out = self.tkg_o_proj(out)                  # reduce over decode-TP
@@ -522,7 +523,7 @@ class AttentionBase(nn.Module):
         if getattr(kv_mgr, "is_paged", False):
             return ops.attention_decode_paged(
                 q, k_cache.data, v_cache.data, position_ids, kv_mgr.block_table,
-                scale=self.scale, sliding_window=self.sliding_window,
+                scale=self.scale, sliding_window=self.sliding_window, token_major=True,
             )
         if self.kv_shard_degree > 1 and self.sinks is None and self.sliding_window == 0:
             from neuronx_distributed_inference_amd.modules.attention import (
@@ -538,5 +539,5 @@ class AttentionBase(nn.Module):
         ring = bool(getattr(kv_mgr, "ring_layers", None)) and kv_mgr.is_ring(self.layer_idx)
         return ops.attention_decode(
             q, k_cache, v_cache, position_ids, seq_ids=seq_ids, scale=self.scale,
-            sinks=self.sinks, sliding_window=self.sliding_window, ring=ring,
+            sinks=self.sinks, sliding_window=self.sliding_window, ring=ring, token_major=True,
         )

@@ -374,9 +374,11 @@ def decode_linear(x: torch.Tensor, weight: torch.Tensor, bias=None) -> torch.Ten
     return y.view(*shape[:-1], N)
 
 
-def _token_major_like(q):
-    """Output of an attention over (B,H,S,D) queries, laid out (B,S,H,D) so that the caller's
-    transpose back to (B,S,H*D) moves nothing."""
+def _attention_out(q, token_major):
+    """Output of an attention over (B,H,S,D) queries; with ``token_major`` laid out (B,S,H,D), so
+    that the transpose to (B,S,H*D) moves nothing."""
+    if not token_major:
+        return torch.empty(q.shape, dtype=q.dtype, device=q.device)
     B, H, S, D = q.shape
     return torch.empty(B, S, H, D, dtype=q.dtype, device=q.device).transpose(1, 2)
 
@@ -390,7 +392,7 @@ def _extend_on_mfma(q, k_cache):
 
 
 def attention_prefill_cached(q, k_cache, v_cache, seq_ids, scale=None,
-                             sinks=None, sliding_window: int = 0):
+                             sinks=None, sliding_window: int = 0, token_major: bool = False):
     """Context-encoding attention reading K/V straight from the cache rows
     that `qkv_rope_update` just wrote (no fresh K/V tensors, no copies).
 
@@ -398,12 +400,13 @@ def attention_prefill_cached(q, k_cache, v_cache, seq_ids, scale=None,
     rows. Causal by *row index* — valid for right-padded batches because
     pad positions (-1) were skipped by the cache scatter, so cache rows
     0..i are always the real prefix for any real query at row i. Fuses the
-    reference's CTE attention + cache update (SURVEY §2 K1+K5)."""
+    reference's CTE attention + cache update (SURVEY §2 K1+K5). ``token_major``
+    allows a result laid out (B,S,Hq,D)."""
     import math
     scale = scale if scale is not None else 1.0 / math.sqrt(q.shape[-1])
     if q.is_cuda:
         c = _require_ext("attention_prefill_cached")
-        out = _token_major_like(q)
+        out = _attention_out(q, token_major)
         c.flash_prefill_cached(out, q.contiguous(), k_cache, v_cache,
                                seq_ids, float(scale), int(sliding_window),
                                sinks=None if sinks is None else sinks.detach())
@@ -417,13 +420,15 @@ def attention_prefill_cached(q, k_cache, v_cache, seq_ids, scale=None,
 
 
 def attention_decode(q, k_cache, v_cache, seq_lens, seq_ids=None, scale=None,
-                     sinks=None, sliding_window: int = 0, ring: bool = False):
+                     sinks=None, sliding_window: int = 0, ring: bool = False,
+                     token_major: bool = False):
     """Token-generation attention against the linear KV cache.
 
     q: (B,Hq,Sq,D) with small Sq (1 or spec_len); k_cache/v_cache:
     (B_cache,Hkv,Smax,D). `seq_lens` is either (B,) valid lengths (queries
     assumed to be the last Sq positions) or (B,Sq) per-query absolute
     POSITIONS (ragged chunks use -1 for pads -> zero output rows).
+    ``token_major`` allows a result laid out (B,Sq,Hq,D).
     K2-analog decode kernel.
     """
     import math
@@ -438,7 +443,7 @@ def attention_decode(q, k_cache, v_cache, seq_lens, seq_ids=None, scale=None,
     if q.is_cuda:
         c = _require_ext("attention_decode")
         if not ring and _extend_on_mfma(q, k_cache):
-            out = _token_major_like(q)
+            out = _attention_out(q, token_major)
             if seq_ids is None:
                 seq_ids = torch.arange(B, device=q.device, dtype=torch.int32)
             c.flash_extend(out, q.contiguous(), k_cache, v_cache, positions, seq_ids=seq_ids,
@@ -467,7 +472,7 @@ def attention_decode(q, k_cache, v_cache, seq_lens, seq_ids=None, scale=None,
                     sliding_window=sliding_window, ring=ring,
                 ).view(B, Hkv, hi - lo, Sq, D))
             return torch.cat(outs, dim=2).view(B, Hq, Sq, D)
-        out = torch.empty_like(q)
+        out = _attention_out(q, False)
         if seq_ids is None:
             seq_ids = torch.arange(B, device=q.device, dtype=torch.int32)
         c.attention_decode(
@@ -521,7 +526,7 @@ def attention_decode_lse(q, k_cache, v_cache, seq_lens, seq_ids=None,
         positions = seq_lens
     if q.is_cuda:
         c = _require_ext("attention_decode")
-        out = torch.empty_like(q)
+        out = _attention_out(q, False)
         lse = torch.empty(B, Hq, Sq, dtype=torch.float32, device=q.device)
         if seq_ids is None:
             seq_ids = torch.arange(B, device=q.device, dtype=torch.int32)
@@ -647,10 +652,10 @@ def gelu_tanh_mul_fused(gate_up):
 
 
 def attention_decode_paged(q, k_cache, v_cache, seq_lens, block_table,
-                           scale=None, sliding_window: int = 0):
+                           scale=None, sliding_window: int = 0, token_major: bool = False):
     """Decode attention against a paged (num_blocks, block_size, Hkv, D)
     cache via a (B, max_blocks) block table. `seq_lens`: (B,) lengths or
-    (B,Sq) per-query positions."""
+    (B,Sq) per-query positions. ``token_major`` allows a result laid out (B,Sq,Hq,D)."""
     import math
     scale = scale if scale is not None else 1.0 / math.sqrt(q.shape[-1])
     B, Hq, Sq, D = q.shape
@@ -663,12 +668,12 @@ def attention_decode_paged(q, k_cache, v_cache, seq_lens, block_table,
     if q.is_cuda:
         c = _require_ext("attention_decode_paged")
         if _extend_on_mfma(q, k_cache):
-            out = _token_major_like(q)
+            out = _attention_out(q, token_major)
             c.flash_extend(out, q.contiguous(), k_cache, v_cache, positions,
                            block_table=block_table, scale=float(scale),
                            window=int(sliding_window))
             return out
-        out = torch.empty_like(q)
+        out = _attention_out(q, False)
         c.attention_decode_paged(
             out, q.contiguous(), k_cache, v_cache,
             positions.to(torch.int32).contiguous(),

@@ -2122,3 +2122,32 @@ def test_normed_prompt_with_a_mask(dtype, kind, monkeypatch):
     assert _rel(got[keep], want[keep]) < tol
     for a, b in zip(rows, model.kv_mgr.get_cache(0)):
         assert _rel(a, b) < tol
+
+
+@pytest.mark.parametrize("S", [1, 5])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["cached", "linear", "paged", "lse"])
+def test_attention_results_are_contiguous(S, dtype, kind):
+    """Results are contiguous whatever the queries' strides, so that they can be viewed; the layer's
+    own layout comes on request and holds the same values."""
+    torch.manual_seed(S)
+    if kind == "cached" and dtype == torch.float32:
+        pytest.skip("not a form the entry point takes")
+    dev, B, H, D, cap = _dev(), 2, 4, 64, 32
+    q = torch.randn(B, S, H, D, device=dev).to(dtype).transpose(1, 2)
+    k, v = (torch.randn(B, H, cap, D, device=dev).to(dtype) for _ in range(2))
+    pos = (7 + torch.arange(S, device=dev)).expand(B, S)
+    seq = torch.arange(B, device=dev)
+    if kind == "cached":
+        call = lambda q, **kw: ops.attention_prefill_cached(q, k, v, seq, **kw)  # noqa: E731
+    elif kind == "linear":
+        call = lambda q, **kw: ops.attention_decode(q, k, v, pos, **kw)  # noqa: E731
+    elif kind == "lse":
+        call = lambda q, **kw: ops.attention_decode_lse(q, k, v, pos)[0]  # noqa: E731
+    else:
+        pages = [t.transpose(1, 2).reshape(B * 2, 16, H, D).contiguous() for t in (k, v)]
+        table = torch.arange(B * 2, device=dev).view(B, 2)
+        call = lambda q, **kw: ops.attention_decode_paged(q, *pages, pos, table, **kw)  # noqa: E731
+    out, same, major = call(q), call(q.contiguous()), call(q, token_major=True)
+    assert out.is_contiguous() and out.view(B, -1).shape == (B, H * S * D)
+    assert torch.equal(out, same) and torch.equal(out, major)
