@@ -168,7 +168,8 @@ class AttentionBase(nn.Module):
         norms = (self.q_norm, self.k_norm)
         if (hidden.is_cuda and self.head_dim in (64, 128)
                 and all(type(n) is RMSNorm and n.weight.numel() == self.head_dim
-                        and n.weight.dtype == hidden.dtype for n in norms)
+                        and n.weight.dtype == hidden.dtype and n.weight.is_contiguous()
+                        and n.weight.data_ptr() % 16 == 0 for n in norms)
                 and norms[0].variance_epsilon == norms[1].variance_epsilon):
             return (norms[0].weight, norms[1].weight, norms[0].variance_epsilon)
         return None

@@ -2151,3 +2151,17 @@ def test_attention_results_are_contiguous(S, dtype, kind):
     out, same, major = call(q), call(q.contiguous()), call(q, token_major=True)
     assert out.is_contiguous() and out.view(B, -1).shape == (B, H * S * D)
     assert torch.equal(out, same) and torch.equal(out, major)
+
+
+def test_head_norm_weights_of_any_alignment():
+    """The fused front end refuses head-norm weights off 16 bytes; the layer sends those, and strided
+    ones, through norms of their own, as it does norms that it does not know."""
+    dev = _dev()
+    _, att = _normed_attention(torch.bfloat16, 8, 1)
+    h = torch.randn(1, 8, 256, device=dev).to(torch.bfloat16)
+    q, k, eps = att._front_norms(h)
+    assert q is att.q_norm.weight and k is att.k_norm.weight and eps == 1e-5
+    flat = torch.zeros(64 * 3, device=dev, dtype=torch.bfloat16)
+    for view in (flat[1:65], flat[::2][:64], flat[:64].float()):
+        att.q_norm.weight = torch.nn.Parameter(view, requires_grad=False)
+        assert att._front_norms(h) is None
