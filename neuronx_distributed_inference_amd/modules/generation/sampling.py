@@ -150,7 +150,7 @@ class DataParallelSampler(nn.Module):
         rank = dist.get_rank(group=mappings.ps.get_tensor_model_parallel_group())
         per = B // self.dp
         if self.inner.static_greedy:
-            local = resharded.argmax(dim=-1)
+            local = ops.row_max(resharded)[1]
         else:
             sp = sampling_params
             if sp is None:
@@ -161,7 +161,7 @@ class DataParallelSampler(nn.Module):
                 )
             sp = sp[(rank % self.dp) * per:((rank % self.dp) + 1) * per]
             k = min(self.config.global_topk, resharded.shape[-1])
-            vals, idxs = resharded.topk(k, dim=-1)
+            vals, idxs = ops.row_topk(resharded, k)
             rand = self.inner._rand(per, logits.device)
             pick = ops.topk_topp_sample(
                 vals.float(), sp[:, 0], sp[:, 1], sp[:, 2], rand, global_topk=k

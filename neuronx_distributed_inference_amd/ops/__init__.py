@@ -853,7 +853,10 @@ def row_max(x: torch.Tensor):
 
 
 def row_topk(x: torch.Tensor, k: int):
-    """(values, indices) of the last dim's k largest elements in order, x.topk(k)."""
+    """(values, indices) of the last dim's k largest elements in order, x.topk(k).
+
+    torch's topk, which serves more than ROW_TOPK_MAX and the other types, records a memset
+    into a captured graph; replays after the first have faulted, so a capture refuses it."""
     if (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32)
             and 1 <= k <= min(ROW_TOPK_MAX, x.size(-1)) and x.numel() // x.size(-1) < 65536):
         c = _require_ext("row_topk")
@@ -865,6 +868,9 @@ def row_topk(x: torch.Tensor, k: int):
                          device=x.device)
         c.row_topk(vals, idx, rows, ws, k)
         return vals, idx
+    if x.is_cuda and torch.cuda.is_current_stream_capturing():
+        raise RuntimeError(f"row_topk: k = {k} of {x.dtype} cannot be captured (at most "
+                           f"{ROW_TOPK_MAX} of 16- or 32-bit floats)")
     return x.topk(k, dim=-1)
 
 

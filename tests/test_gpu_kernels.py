@@ -2165,3 +2165,13 @@ def test_head_norm_weights_of_any_alignment():
     for view in (flat[1:65], flat[::2][:64], flat[:64].float()):
         att.q_norm.weight = torch.nn.Parameter(view, requires_grad=False)
         assert att._front_norms(h) is None
+
+
+def test_row_topk_refuses_what_a_capture_cannot_hold(monkeypatch):
+    """More than the kernel holds goes to torch's topk, but not into a graph."""
+    x = torch.randn(2, 5000, device=_dev())
+    assert torch.equal(ops.row_topk(x, 3000)[0], x.topk(3000)[0])
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    for bad in ((x, 3000), (x.double(), 2)):
+        with pytest.raises(RuntimeError, match="captured"):
+            ops.row_topk(*bad)
