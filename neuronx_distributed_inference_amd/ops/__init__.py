@@ -839,15 +839,24 @@ def moe_grouped_gemm(x_sorted: torch.Tensor, w: torch.Tensor,
 ROW_TOPK_MAX = 2048
 
 
+def _row_kernels(x: torch.Tensor) -> bool:
+    """Whether the row kernels take x: they have no backward and count elements in 31 bits."""
+    return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32)
+            and 0 < x.size(-1) < (1 << 31) - 8192 and not (x.requires_grad and torch.is_grad_enabled()))
+
+
+def _rows(x: torch.Tensor) -> torch.Tensor:
+    rows = x.reshape(-1, x.size(-1))
+    return rows if rows.stride(1) == 1 else rows.contiguous()
+
+
 def row_max(x: torch.Tensor):
     """(values, indices) of the last dim's largest elements, x.max(-1)."""
-    if x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32) and x.size(-1) > 0:
+    if _row_kernels(x):
         c = _require_ext("row_max")
-        rows = x.reshape(-1, x.size(-1))
-        rows = rows if rows.stride(1) == 1 else rows.contiguous()
         vals = torch.empty(x.shape[:-1], dtype=x.dtype, device=x.device)
         idx = torch.empty(x.shape[:-1], dtype=torch.long, device=x.device)
-        c.row_max(vals, idx, rows)
+        c.row_max(vals, idx, _rows(x))
         return vals, idx
     return x.max(dim=-1)
 
@@ -857,16 +866,11 @@ def row_topk(x: torch.Tensor, k: int):
 
     torch's topk, which serves more than ROW_TOPK_MAX and the other types, records a memset
     into a captured graph; replays after the first have faulted, so a capture refuses it."""
-    if (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32)
-            and 1 <= k <= min(ROW_TOPK_MAX, x.size(-1)) and x.numel() // x.size(-1) < 65536):
+    if _row_kernels(x) and 1 <= k <= min(ROW_TOPK_MAX, x.size(-1)):
         c = _require_ext("row_topk")
-        rows = x.reshape(-1, x.size(-1))
-        rows = rows if rows.stride(1) == 1 else rows.contiguous()
         vals = torch.empty(*x.shape[:-1], k, dtype=x.dtype, device=x.device)
         idx = torch.empty(*x.shape[:-1], k, dtype=torch.long, device=x.device)
-        ws = torch.empty(2 * rows.size(0) * k * -(-x.size(-1) // 4096), dtype=torch.long,
-                         device=x.device)
-        c.row_topk(vals, idx, rows, ws, k)
+        c.row_topk(vals, idx, _rows(x), k)
         return vals, idx
     if x.is_cuda and torch.cuda.is_current_stream_capturing():
         raise RuntimeError(f"row_topk: k = {k} of {x.dtype} cannot be captured (at most "

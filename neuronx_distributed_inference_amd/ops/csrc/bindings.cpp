@@ -92,7 +92,7 @@ void moe_routed_down(torch::Tensor out, torch::Tensor ws, torch::Tensor h, torch
                      c10::optional<torch::Tensor> s_down, torch::Tensor tiles, torch::Tensor inv,
                      c10::optional<torch::Tensor> weights, long mt);
 void row_max(torch::Tensor val, torch::Tensor idx, torch::Tensor x);
-void row_topk(torch::Tensor val, torch::Tensor idx, torch::Tensor x, torch::Tensor ws, long k);
+void row_topk(torch::Tensor val, torch::Tensor idx, torch::Tensor x, long k);
 void router_topk(torch::Tensor vals, torch::Tensor idx, torch::Tensor logits,
                  long top_k, long act_sigmoid, long pre_softmax,
                  long normalize);

@@ -2167,10 +2167,70 @@ def test_head_norm_weights_of_any_alignment():
         assert att._front_norms(h) is None
 
 
+def _topk_exact(x, k):
+    """Order of the row kernels: NaN first, then by value (-0 as 0), equal ones by index."""
+    key = torch.where(torch.isnan(x.float()), float("inf"), x.float()) + 0.0
+    o = torch.sort(key, dim=-1, descending=True, stable=True).indices
+    nan = torch.isnan(x.float()).gather(1, o)
+    return o.gather(1, torch.sort(nan.int(), dim=-1, descending=True, stable=True).indices)[:, :k]
+
+
+@pytest.mark.parametrize("n,k", [
+    (1, 1), (2, 2), (65, 64), (511, 3), (512, 512), (513, 513), (1024, 512), (1025, 1), (4096, 513),
+    (8191, 2048), (8192, 2048), (8200, 513), (20003, 512), (65536, 2048),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["random", "equal", "rising", "falling", "few", "zeros", "nan"])
+def test_row_topk_orders_and_ties(n, k, dtype, kind):
+    """Exact, at the edges of the row sizes and of k, whatever the order: rows that rise or fall, of
+    one value, of few values (more candidates than a workgroup holds), of both zeros (values keep
+    their sign), of NaN and infinities, and large elements that share a group."""
+    torch.manual_seed(n + k)
+    x = torch.randn(2, n)
+    if kind == "equal":
+        x[:] = -3.0
+    elif kind == "rising":
+        x = x.sort(-1).values
+    elif kind == "falling":
+        x = x.sort(-1, descending=True).values
+    elif kind == "few":
+        x = torch.randint(0, 3, (2, n)).float()
+        x[0, ::1024] = 5                                      # one thread's elements
+        x[1, (torch.arange(n) // 8) % 1024 == 7] = 4
+    elif kind == "zeros":
+        x = torch.where(torch.rand(2, n) < 0.5, 0.0, -0.0)
+    elif kind == "nan":
+        x[torch.rand(2, n) < 0.3] = float("nan")
+        x[torch.rand(2, n) < 0.3] = float("-inf")
+        x[torch.rand(2, n) < 0.1] = float("inf")
+    x = x.to(dtype)
+    want = _topk_exact(x, k)
+    vals, idx = ops.row_topk(x.to(_dev()), k)
+    assert torch.equal(idx.cpu(), want)
+    bits = torch.int16 if dtype == torch.bfloat16 else torch.int32
+    assert torch.equal(vals.cpu().view(bits), x.gather(1, want).view(bits))
+    vals, idx = ops.row_max(x.to(_dev()))
+    assert torch.equal(idx.cpu(), want[:, 0])
+
+
+@pytest.mark.parametrize("rows,n,k", [(70000, 16, 3), (1050000, 2, 1), (66000, 600, 5)])
+def test_row_topk_many_rows(rows, n, k):
+    """More rows than a grid dimension of 65535, and than one launch takes."""
+    torch.manual_seed(n)
+    x = torch.randn(rows, n, device=_dev()).to(torch.bfloat16)
+    want = _topk_exact(x.cpu(), k)
+    assert torch.equal(ops.row_topk(x, k)[1].cpu(), want)
+    assert torch.equal(ops.row_max(x)[1].cpu(), want[:, 0])
+
+
 def test_row_topk_refuses_what_a_capture_cannot_hold(monkeypatch):
-    """More than the kernel holds goes to torch's topk, but not into a graph."""
+    """More than the kernel holds goes to torch's topk, but not into a graph; gradients go through
+    torch's as well."""
     x = torch.randn(2, 5000, device=_dev())
     assert torch.equal(ops.row_topk(x, 3000)[0], x.topk(3000)[0])
+    y = x.clone().requires_grad_()
+    ops.row_topk(y, 2)[0].sum().backward()
+    assert float(y.grad.sum()) == 4.0
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
     for bad in ((x, 3000), (x.double(), 2)):
         with pytest.raises(RuntimeError, match="captured"):
