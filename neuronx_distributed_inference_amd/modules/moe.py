@@ -178,14 +178,31 @@ class ExpertMLPs(nn.Module):
         El = self.num_local_experts
         gates = torch.zeros(T, El, dtype=x.dtype, device=x.device)
         gates = gates.scatter(1, idx, weights.to(x.dtype))
-        gte = gates.t().unsqueeze(1)                       # (E, 1, T)
-        # weights on the left: the right operand of a 16-bit batched product is contiguous
-        xe = x.t().unsqueeze(0)
+        if x.is_cuda and x.dtype in (torch.bfloat16, torch.float16):
+            return self._forward_dense_16bit(x, gates)
+        gte = gates.t().unsqueeze(-1)                      # (E, T, 1)
         if self.scale_input:
-            xe = xe * gte                                  # Llama4: gate input
-        xe = xe.expand(El, H, T).contiguous()
-        g = torch.bmm(self.w_gate, xe)
-        u = torch.bmm(self.w_up, xe)
+            xe = x.unsqueeze(0) * gte                      # Llama4: gate input
+        else:
+            xe = x.unsqueeze(0).expand(El, T, H)
+        g = torch.bmm(xe, self.w_gate.transpose(1, 2))
+        u = torch.bmm(xe, self.w_up.transpose(1, 2))
+        y = torch.bmm(self.act_mul(g, u), self.w_down.transpose(1, 2))
+        if not self.scale_input:
+            y = y * gte
+        return y.sum(dim=0)
+
+    def _forward_dense_16bit(self, x: torch.Tensor, gates: torch.Tensor) -> torch.Tensor:
+        """The same with the weights on the left: a batched 16-bit product on the GPU needs a
+        contiguous right operand (a transposed view has faulted)."""
+        El, I, H = self.w_gate.shape
+        gte = gates.t().unsqueeze(1)                       # (E, 1, T)
+        if self.scale_input:
+            xe = (x.t().unsqueeze(0) * gte).contiguous()
+            g, u = torch.bmm(self.w_gate, xe), torch.bmm(self.w_up, xe)
+        else:                                              # one product, no copy per expert
+            g, u = ((w.reshape(El * I, H) @ x.t()).view(El, I, -1)
+                    for w in (self.w_gate, self.w_up))
         y = torch.bmm(self.w_down, self.act_mul(g, u))
         if not self.scale_input:
             y = y * gte

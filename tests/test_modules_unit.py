@@ -696,3 +696,30 @@ def test_moe_grouped_tile32_cpu_matches_dense(monkeypatch):
     want = m._forward_dense(x, w, idx)
     got = m._forward_grouped(x, w, idx)
     torch.testing.assert_close(got, want, atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_moe_dense_does_not_copy_tokens_per_expert(dtype, monkeypatch):
+    """The dense products of the CPU (and of fp32) read the tokens through a view of stride 0; what
+    the GPU needs in 16 bits, weights on the left, gives the same up to two roundings."""
+    from neuronx_distributed_inference_amd.modules.moe import ExpertMLPs
+
+    torch.manual_seed(0)
+    E, H, I, T, k = 4, 32, 48, 7, 2
+    m = ExpertMLPs(num_experts=E, hidden_size=H, intermediate_size=I, tp_degree=1, dtype=dtype)
+    for p in m.parameters():
+        torch.nn.init.normal_(p, std=0.2)
+    x = torch.randn(T, H).to(dtype)
+    w, idx = torch.softmax(torch.randn(T, E), -1).topk(k, -1)
+    lefts, bmm = [], torch.bmm
+    monkeypatch.setattr(torch, "bmm", lambda a, b: lefts.append(a) or bmm(a, b))
+    with torch.no_grad():
+        want = m._forward_dense(x, w, idx)
+        assert lefts[0].shape == (E, T, H) and lefts[0].stride(0) == 0
+        gates = torch.zeros(T, E, dtype=dtype).scatter(1, idx, w.to(dtype))
+        for scale_input in (False, True):
+            m.scale_input = scale_input
+            want = m._forward_dense(x, w, idx)
+            got = m._forward_dense_16bit(x, gates)
+            tol = 1e-6 if dtype == torch.float32 else 2.0 ** -6
+            assert (got - want).float().norm() < tol * want.float().norm()
