@@ -210,13 +210,12 @@ class ExpertMLPs(nn.Module):
 
     def _forward_grouped(self, x: torch.Tensor, weights: torch.Tensor,
                          idx: torch.Tensor) -> torch.Tensor:
-        """Grouped expert GEMM: sort assignments by expert,
-        pad each segment to 64-row tiles, one kernel launch per
-        projection for ALL experts. Static shapes + tensor-only table
-        construction -> hipGraph-capturable; no top_k/E redundant FLOPs
-        (the dense-bmm path is compute-bound at decode batch >=128).
-        Non-local assignments (EP) route to a sentinel segment whose
-        tiles the kernel skips; their contribution is masked out."""
+        """The chosen experts' products alone, no top_k/E redundant FLOPs; static
+        shapes and tables made on the device, so a captured step holds them. On the GPU the
+        routed kernels, with 16-bit and 8-bit weights; MXFP4 weights, and the CPU reference of
+        all, go through the grouped products: assignments sorted by expert, each expert's
+        padded to 64-row tiles, those of other ranks' experts (EP) in a last segment whose
+        tiles are skipped."""
         T, H = x.shape
         El = self.num_local_experts
         offset = self._local_offset()
@@ -233,33 +232,14 @@ class ExpertMLPs(nn.Module):
         flat = (idx - offset).view(-1)
         local = (flat >= 0) & (flat < El)
         flat_routed = torch.where(local, flat, torch.full_like(flat, El))
-        # fine-grained MoE (few tokens per expert): a 32-row tile halves
-        # the padded-row waste. bf16 kernel only (quantized kernels are
-        # 64-row); opt-in via NXDI_MOE_TILE32=1 while it soaks.
-        import os as _os
-
-        if fp8 or mx4:
-            I0 = self.w_gate_q.shape[1]
-        else:
-            I0 = self.w_gate.shape[1]
-        tile = 32 if (
-            not fp8 and not mx4
-            and _os.environ.get("NXDI_MOE_TILE32") != "0"
-            and T * top_k < 48 * El
-            and I0 % 128 == 0 and H % 128 == 0
-        ) else 64
         order, dest, expert_ids, gtab, Mpad = ops.moe_grouped_tables(
-            flat_routed, El + 1, top_k, tile=tile)
+            flat_routed, El + 1, top_k)
         # sentinel segment (id El) never computes
         expert_ids = torch.where(expert_ids >= El,
                                  torch.full_like(expert_ids, -1), expert_ids)
         gatew = weights.view(-1)[order]
         lmask = local[order]
 
-        if fp8 or mx4:
-            I, Hn = self.w_gate_q.shape[1], self.w_down_q.shape[1]
-        else:
-            I, Hn = self.w_gate.shape[1], self.w_down.shape[1]
         if self.scale_input:
             # input scaling is nonlinear through the GLU: keep the
             # materialized gather for this (rare) variant
@@ -282,10 +262,8 @@ class ExpertMLPs(nn.Module):
             u = ops.moe_grouped_gemm_fp8(x_in, self.w_up_q, self.w_up_s,
                                          expert_ids, x_gather=xg)
         else:
-            g = ops.moe_grouped_gemm(x_in, self.w_gate, expert_ids,
-                                     x_gather=xg, mt=tile)
-            u = ops.moe_grouped_gemm(x_in, self.w_up, expert_ids,
-                                     x_gather=xg, mt=tile)
+            g = ops.moe_grouped_gemm(x_in, self.w_gate, expert_ids, x_gather=xg)
+            u = ops.moe_grouped_gemm(x_in, self.w_up, expert_ids, x_gather=xg)
         h = self.act_mul(g, u)
         # routing-weighted combine fuses into the down epilogue (fp32
         # atomics, one rmw per element); non-local assignments are
@@ -308,7 +286,7 @@ class ExpertMLPs(nn.Module):
         else:
             ops.moe_grouped_gemm(h, self.w_down, expert_ids,
                                  combine_out=out32, combine_scale=gw_tab,
-                                 combine_gather=gtab, mt=tile)
+                                 combine_gather=gtab)
         return out32.to(x.dtype)
 
     def forward(self, x: torch.Tensor, weights: torch.Tensor, idx: torch.Tensor):

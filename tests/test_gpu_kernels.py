@@ -850,9 +850,9 @@ def test_moe_grouped_gemm_kernel():
 
 
 def test_moe_grouped_matches_dense_gpu():
-    """Full MoE layer: grouped path vs dense bmm path on GPU bf16, plus a
-    timing line at decode batch 256 (Mixtral-like shapes, TP-degree 8
-    shard sizes to fit the test box quickly)."""
+    """Full MoE layer: the chosen experts alone (routed kernels) vs the dense
+    products on GPU bf16, plus a timing line at decode batch 256 (Mixtral-like
+    shapes, TP-degree 8 shard sizes to fit the test box quickly)."""
     from neuronx_distributed_inference_amd.modules.moe import ExpertMLPs
 
     torch.manual_seed(0)
@@ -1150,7 +1150,7 @@ def test_moe_grouped_fp8_kernel_gpu():
 
 
 def test_moe_fp8_module_gpu():
-    """ExpertMLPs.quantize_fp8 end-to-end on GPU vs the bf16 dense path."""
+    """ExpertMLPs.quantize_fp8 end-to-end on GPU (routed kernels) vs the bf16 dense path."""
     from neuronx_distributed_inference_amd.modules.moe import ExpertMLPs
 
     torch.manual_seed(8)
@@ -1279,27 +1279,33 @@ def test_router_topk_fused_gpu(mode):
     torch.testing.assert_close(got_v.cpu(), want_v, atol=1e-5, rtol=1e-5)
 
 
-def test_moe_grouped_tile32_gpu(monkeypatch):
-    """mt=32 grouped kernel (fine-grained tile) vs the dense bmm path on
-    GPU at a 128-expert top-8 shape."""
-    from neuronx_distributed_inference_amd.modules.moe import ExpertMLPs
-
-    monkeypatch.setenv("NXDI_MOE_TILE32", "1")
+@pytest.mark.parametrize("bn", [128, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_moe_grouped_tile32_gpu(bn, dtype):
+    """The grouped product in 32-row tiles: gathered tokens, plain and combined by routing weights,
+    against its CPU reference in fp32. Half a unit of the result's type (the combined sums are 32-bit
+    atomics of 8 terms)."""
     torch.manual_seed(15)
     dev = _dev()
-    E, H, I, T, top_k = 32, 256, 384, 48, 8
-    m = ExpertMLPs(num_experts=E, hidden_size=H, intermediate_size=I,
-                   tp_degree=1, dtype=torch.bfloat16)
-    with torch.no_grad():
-        for p in m.parameters():
-            p.normal_(0, 0.05)
-    m = m.to(dev)
-    x = torch.randn(T, H, dtype=torch.bfloat16, device=dev) * 0.3
-    w, idx = torch.softmax(torch.randn(T, E, device=dev), -1).topk(top_k, -1)
-    want = m._forward_dense(x, w, idx)
-    got = m._forward_grouped(x, w, idx)
-    torch.testing.assert_close(got.float(), want.float(),
-                               atol=5e-2, rtol=5e-2)
+    E, N, K, T, top_k = 32, 768, 256, 48, 8
+    w = (torch.randn(E, N, K) * 0.05).to(dtype)
+    x = (torch.randn(T, K) * 0.3).to(dtype)
+    wt, idx = torch.softmax(torch.randn(T, E), -1).topk(top_k, -1)
+    flat = idx.reshape(-1).to(dev)
+    order, dest, eids, gtab, Mpad = ops.moe_grouped_tables(flat, E, top_k, tile=32)
+    got = ops.moe_grouped_gemm(x.to(dev), w.to(dev), eids, bn=bn, x_gather=gtab, mt=32)
+    want = torch.stack([x.float() @ w[e].float().t() for e in range(E)])     # (E, T, N)
+    rows = got.index_select(0, dest).cpu()
+    order = order.cpu()
+    per_row = want[flat.cpu()[order], order // top_k]
+    assert _rel(rows, per_row) < 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    scale = torch.zeros(Mpad, device=dev)
+    scale[dest] = wt.reshape(-1).to(dev)[order.to(dev)]
+    out = torch.zeros(T, N, device=dev)
+    ops.moe_grouped_gemm(x.to(dev), w.to(dev), eids, bn=bn, x_gather=gtab, combine_out=out,
+                         combine_scale=scale, combine_gather=gtab, mt=32)
+    total = (want[idx, torch.arange(T).view(T, 1)] * wt.unsqueeze(-1)).sum(1)
+    assert _rel(out, total) < 1e-5
 
 
 def _rel(a, b):
