@@ -882,6 +882,12 @@ def row_topk(x: torch.Tensor, k: int):
 MOE_WORKSPACE = 1 << 30
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """t, or a copy where it is not contiguous or starts off 16 bytes."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def moe_routed_experts(x: torch.Tensor, weights: torch.Tensor, idx: torch.Tensor, w_gate, w_up,
                        w_down, scales=None, first: int = 0, num_experts: int = 0,
                        gelu: bool = False, scale_input: bool = False) -> torch.Tensor:
@@ -891,6 +897,8 @@ def moe_routed_experts(x: torch.Tensor, weights: torch.Tensor, idx: torch.Tensor
     ``scale_input`` the weights scale the experts' inputs and the outputs are added as they are.
     GPU only; x bf16/f16 (T, H)."""
     c = _require_ext("moe_routed_experts")
+    x, w_gate, w_up, w_down = (_aligned(t) for t in (x, w_gate, w_up, w_down))
+    scales = scales and [_aligned(s) for s in scales]
     T, H = x.shape
     E, I = w_gate.shape[0], w_gate.shape[1]
     n, dev = idx.numel(), x.device
@@ -918,7 +926,7 @@ def moe_routed_experts(x: torch.Tensor, weights: torch.Tensor, idx: torch.Tensor
         xs[inv.long()] = (x.unsqueeze(1) * weights.view(T, -1, 1).to(x.dtype)).reshape(n, H)
         c.moe_routed_glu(h, xs, w_gate, w_up, s[0], s[1], tiles, None, mt, int(gelu))
     else:
-        c.moe_routed_glu(h, x.contiguous(), w_gate, w_up, s[0], s[1], tiles, gather, mt, int(gelu))
+        c.moe_routed_glu(h, x, w_gate, w_up, s[0], s[1], tiles, gather, mt, int(gelu))
     cols = min(H, max(256, MOE_WORKSPACE // (4 * rows) // 256 * 256))
     ws = torch.empty(rows * cols, dtype=torch.float32, device=dev)
     c.moe_routed_down(out, ws, h, w_down, s[2], tiles, inv, None if scale_input else weights, mt)

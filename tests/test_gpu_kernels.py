@@ -2241,3 +2241,30 @@ def test_row_topk_refuses_what_a_capture_cannot_hold(monkeypatch):
     for bad in ((x, 3000), (x.double(), 2)):
         with pytest.raises(RuntimeError, match="captured"):
             ops.row_topk(*bad)
+
+
+@pytest.mark.parametrize("f8", [False, True])
+def test_moe_routed_experts_of_any_layout(f8):
+    """Tokens, weights and scales that start off 16 bytes or are strided give what contiguous ones do,
+    bit for bit."""
+    torch.manual_seed(0)
+    dev, T, E, k, H, I = _dev(), 40, 4, 2, 128, 256
+    x = torch.randn(T, H, device=dev).to(torch.bfloat16)
+    wt, idx = torch.softmax(torch.randn(T, E, device=dev), -1).topk(k, dim=-1)
+    w = [(torch.randn(E, *s, device=dev) * 0.1).to(torch.bfloat16) for s in ((I, H), (I, H), (H, I))]
+    scales = None
+    if f8:
+        w, scales = zip(*[ops.fp8_moe_quantize(v) for v in w])
+    want = ops.moe_routed_experts(x, wt, idx, *w, scales=scales, num_experts=E)
+
+    def off(t):
+        v = torch.empty(t.numel() + 1, dtype=t.dtype, device=dev)[1:].view(t.shape)
+        return v.copy_(t)
+
+    def strided(t):
+        return torch.stack([t, t], -1)[..., 0]
+
+    for f in (off, strided):
+        got = ops.moe_routed_experts(f(x), f(wt), f(idx), *[f(v) for v in w],
+                                     scales=scales and [f(s) for s in scales], num_experts=E)
+        assert torch.equal(got, want)
