@@ -192,6 +192,10 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
 
     int qpos = a.positions ? a.positions[(long)b * a.S + token] : token;
     if (r_own >= R || (row < 0 && !a.clamp_rows)) qpos = -1;
+    // the lane's own first visible key; positions past the capacity see what is left of theirs
+    const int key_lo = a.window > 0 ? qpos - a.window + 1
+                                    : a.window < 0 ? qpos / -a.window * -a.window : 0;
+    const bool past = __any(qpos >= a.cap);
     qpos = min(qpos, a.cap - 1);
 
     // bounds of the wave's and the workgroup's valid rows
@@ -233,10 +237,9 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
     if (bmax < 0) lo = 0;
     // the wave's own first visible key, and from where on every key is inside all its windows
     const int w_lo = a.window > 0 ? max(0, wmin - a.window + 1) : (C && wmax >= 0 ? (wmin / C) * C : 0);
-    const int w_in = a.window > 0 ? wmax - a.window + 1 : (C && wmax >= 0 ? (wmax / C) * C : 0);
-
-    // the lane's own first visible key
-    const int key_lo = a.window > 0 ? qpos - a.window + 1 : (C ? (qpos / C) * C : 0);
+    const int w_in = past && a.window ? 0x7fffffff
+                     : a.window > 0   ? wmax - a.window + 1
+                                      : (C && wmax >= 0 ? (wmax / C) * C : 0);
 
     int t_lo = lo / KT, t_hi = (bmax + KT) / KT;      // tiles [t_lo, t_hi); none when bmax < 0
     if (a.nsplit > 1) {
@@ -679,8 +682,10 @@ FaArgs flash_args(const torch::Tensor& q, double scale, long window) {
     return a;
 }
 
-// Splits over the keys: two workgroups fit a CU, so fill 512 places, but leave a split
-// at least 4 tiles (256 keys) of the longest row, below which combining costs more.
+// Splits over the keys: two workgroups fit a CU, so fill 512 places, but leave a split at least 4
+// tiles (256 keys) of a row that fills the capacity, below which combining costs more. (Rows' own
+// lengths are on the device: a short row's tiles are shared by as many splits. 6 tokens over 300
+// of 32768 15 us, one workgroup a token 46; over 1000 of 32768, 8 rows, 20 and 109.)
 int flash_splits(const FaArgs& a) {
     const long tiles = ((long)a.Hq / a.Hkv * a.S + QROWS - 1) / QROWS * a.B * a.Hkv;
     const long most = std::max(1, a.cap / (4 * KT));

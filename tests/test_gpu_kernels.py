@@ -2268,3 +2268,24 @@ def test_moe_routed_experts_of_any_layout(f8):
         got = ops.moe_routed_experts(f(x), f(wt), f(idx), *[f(v) for v in w],
                                      scales=scales and [f(s) for s in scales], num_experts=E)
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("window", [0, 40, -64])
+@pytest.mark.parametrize("Sq", [1, 12])
+@pytest.mark.parametrize("paged", [False, True])
+def test_attention_positions_past_the_capacity(window, Sq, paged):
+    """Tokens whose position is past the cache see the rows that their window still has there (the
+    rounding of the result and half as much again)."""
+    torch.manual_seed(0)
+    dev, B, H, D, cap = _dev(), 2, 4, 64, 128
+    q = torch.randn(B, H, Sq, D).to(torch.bfloat16)
+    k, v = (torch.randn(B, H, cap, D).to(torch.bfloat16) for _ in range(2))
+    pos = torch.tensor([[cap - 5], [cap + 20]]) + torch.arange(Sq) * 3
+    want = ops.attention_decode(q.float(), k.float(), v.float(), pos, sliding_window=window)
+    if paged:
+        pages = [t.transpose(1, 2).reshape(B * 8, 16, H, D).contiguous().to(dev) for t in (k, v)]
+        got = ops.attention_decode_paged(q.to(dev), *pages, pos.to(dev), torch.arange(B * 8, device=dev)
+                                         .view(B, 8), sliding_window=window)
+    else:
+        got = ops.attention_decode(q.to(dev), k.to(dev), v.to(dev), pos.to(dev), sliding_window=window)
+    assert _rel(got, want) < 1.5 * 2.0 ** -9
