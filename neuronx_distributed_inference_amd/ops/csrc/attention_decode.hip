@@ -433,6 +433,7 @@ template <int NE, bool F8> struct DmRaw {
 constexpr float DM_GROWTH = 8.f;   // log2 growth of a maximum that is put off
 constexpr float DM_DEPTH = 64.f;   // and how far below the largest score P may count from (fp16)
 constexpr int DM_TILE = 32;        // keys of a wave's step
+constexpr int DM_LEAST = 128;      // keys of a split: one step of each wave
 
 template <typename T, typename CT, int D, bool PAGED>
 __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
@@ -443,8 +444,8 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
     const int* __restrict__ positions, const int* __restrict__ seq_ids,
     const int* __restrict__ block_table, const float* __restrict__ sinks,
     float* __restrict__ lse_out, const float scale, const float v_scale, const int window,
-    const int ring, const int Hkv, const int Sq, const int gq, const int Smax, const int chunk,
-    const int nsplit, const int block_size, const int max_blocks) {
+    const int ring, const int Hkv, const int Sq, const int gq, const int Smax, const int nsplit,
+    const int block_size, const int max_blocks) {
     using DT = DmTraits<T>;
     using vec8 = typename DT::vec8;
     constexpr bool F8 = sizeof(CT) == 1;
@@ -487,8 +488,13 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
         span = max(span, __shfl_xor(span, off, WAVE_SIZE));
         first = min(first, __shfl_xor(first, off, WAVE_SIZE));
     }
-    const int k_hi = __builtin_amdgcn_readfirstlane(min(min(span, Smax), (split + 1) * chunk));
-    const int k_lo = __builtin_amdgcn_readfirstlane(max(ring ? 0 : first, split * chunk));
+    // the splits share the keys that are seen (see launch_decode)
+    const int all_hi = __builtin_amdgcn_readfirstlane(min(span, Smax));
+    const int all_lo = min(__builtin_amdgcn_readfirstlane(ring ? 0 : first), all_hi);
+    const int seen = all_lo / DM_TILE * DM_TILE;
+    const int chunk = max(DM_LEAST, ((all_hi - seen + nsplit - 1) / nsplit + DM_TILE - 1) / DM_TILE * DM_TILE);
+    const int k_hi = min(all_hi, seen + (split + 1) * chunk);
+    const int k_lo = max(all_lo, seen + split * chunk);
     const int t_lo = k_lo / DM_TILE, t_hi = k_lo < k_hi ? (k_hi + DM_TILE - 1) / DM_TILE : 0;
     // position of the key in cache row l: l itself; in a ring the newest one that is l modulo
     // Smax, which is base + l up to the newest row and base + l - Smax behind it
@@ -857,16 +863,18 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
     // 1024, 87 at 2048; 128 rows of 512: 40 / 40 / 52), as rows of unequal length even out over
     // the CUs by themselves. A split keeps 128 rows, one step of each wave (1 row of 300: 7.8 us;
     // 256: 8.4), 256 in long caches where the combining pass weighs more (1 row of 8192: 11.8 us
-    // with 256, 13.5 with 128).
+    // with 256, 13.5 with 128). Their number goes by the capacity, which the host knows; what
+    // they share by the keys that a row sees, so that short rows keep them busy too. 32/8 heads
+    // of 128, shares of the capacity -> of the row: 1 row of 700 in a cache of 8192 10.1 -> 9.2 us,
+    // of 1000 (or a window of 1024) in 32768 18.9 -> 12.5, 16 rows of 700 in 8192 25.7 -> 15.0 (in
+    // pages 27.8 -> 15.9), full rows the same (16 of half to full 8192 73.3, 73.7; 64 of 2048
+    // 73.5, 73.9).
     // Lane-group kernel: >= 1024 workgroups when possible, chunks of >= 128 rows.
-    int nsplit, chunk;
+    int nsplit, chunk = 0;
     if constexpr (MFMA) {
-        const int least = Smax <= 2048 ? 128 : 256;
+        const int least = Smax <= 2048 ? DM_LEAST : 2 * DM_LEAST;
         nsplit = 512 / std::max(1, B * Hkv * nct);
         nsplit = std::max(1, std::min({nsplit, (Smax + least - 1) / least, 64}));
-        // (a cache of no rows has one split, which reads nothing and writes zeros)
-        chunk = std::max(DM_TILE, ((Smax + nsplit - 1) / nsplit + DM_TILE - 1) / DM_TILE * DM_TILE);
-        nsplit = std::max(1, (Smax + chunk - 1) / chunk);
     } else {
         nsplit = 1024 / std::max(1, B * Hkv * Sq);
         nsplit = std::max(1, std::min({nsplit, (Smax + 127) / 128, 64}));
@@ -894,7 +902,7 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
                            PG ? block_table->data_ptr<int>() : nullptr,                     \
                            sinks ? sinks->data_ptr<float>() : nullptr,                      \
                            lse_out ? lse_out->data_ptr<float>() : nullptr, scale, v_scale,  \
-                           window, ring, Hkv, Sq, gq, Smax, chunk, nsplit, block_size, max_blocks)
+                           window, ring, Hkv, Sq, gq, Smax, nsplit, block_size, max_blocks)
         if (paged) DM_GO(true);
         else DM_GO(false);
 #undef DM_GO

@@ -1400,7 +1400,7 @@ def test_attention_extend_missing_pages_and_rows():
 def test_attention_decode_mfma(D, gq, Sq, dtype, window, kind):
     """The matrix-core decode kernel at lengths around its 32-key steps and its splits (1, 31..33,
     127..129, full), one row of padding, one or two column tiles, missing pages; against the fp32
-    reference on the same rounded inputs. Probabilities are held in two 16-bit parts, so what is
+    reference on the same rounded inputs. Probabilities keep their 24 bits, so what is
     left is the rounding of the result: 2^-9 in bf16, 2^-12 in fp16 (2-norm)."""
     if (kind in ("paged", "lse") and gq > 8) or (kind == "ring" and window < 0):
         pytest.skip("not a form the entry point takes")
@@ -1455,6 +1455,45 @@ def test_attention_decode_mfma(D, gq, Sq, dtype, window, kind):
         ok = torch.isfinite(want_lse)
         assert torch.equal(ok, torch.isfinite(lse.cpu()))
         torch.testing.assert_close(lse.cpu()[ok], want_lse[ok], atol=2e-5, rtol=2e-5)
+
+
+@pytest.mark.parametrize("cap,kind", [(2048, "linear"), (8192, "linear"), (8192, "paged"),
+                                      (8192, "fp8"), (8192, "ring")])
+@pytest.mark.parametrize("window", [0, 100, 1000, -512])
+def test_attention_decode_short_rows_of_long_cache(cap, kind, window):
+    """Splits share the keys that a row sees, not the capacity: rows around the least share of a
+    split (128 keys), around shares of a whole step more, windows that begin inside a step, the
+    full row, and what lies behind a row is NaN. Tolerance: the rounding of the result, 2^-9."""
+    if kind == "ring" and window <= 0:
+        pytest.skip("not a form the entry point takes")
+    torch.manual_seed(cap + window)
+    dev, Hkv, gq, D, bs = _dev(), 1, 4, 128, 32
+    lens = torch.tensor([1, 127, 128, 129, 700, cap // 128 * 32 + 1, cap - 1, cap])
+    B = lens.numel()
+    for rows in (range(B), [4], [7]):              # one row alone is split most
+        rows = list(rows)
+        n, pos = len(rows), lens[rows].view(-1, 1) - 1
+        q = torch.randn(n, Hkv * gq, 1, D, device=dev).bfloat16()
+        kc = torch.randn(n, Hkv, cap, D, device=dev).bfloat16()
+        vc = torch.randn(n, Hkv, cap, D, device=dev).bfloat16()
+        if kind == "fp8":
+            kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+        kw = dict(sliding_window=window)
+        kr, vr = kc.float().cpu(), vc.float().cpu()
+        if kind == "ring":
+            kw["ring"] = True
+        elif kind != "fp8":
+            for i in range(n):
+                kc[i, :, int(pos[i]) + 1:] = float("nan")
+                vc[i, :, int(pos[i]) + 1:] = float("nan")
+        if kind == "paged":
+            pk, pv = (c.view(n * cap // bs, bs, Hkv, D) for c in (kc, vc))
+            bt = torch.arange(n * cap // bs, device=dev, dtype=torch.int32).view(n, -1)
+            out = ops.attention_decode_paged(q, pk, pv, pos.to(dev), bt, **kw)
+        else:
+            out = ops.attention_decode(q, kc, vc, pos.to(dev), **kw)
+        want = ops.attention_decode(q.float().cpu(), kr, vr, pos, **kw)
+        assert _rel(out, want) < 2.0 ** -9
 
 
 @pytest.mark.parametrize("S,D,Dv,H,G,per_head,dtype", [
