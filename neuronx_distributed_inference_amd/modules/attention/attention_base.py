@@ -35,6 +35,11 @@ PHASE_CTE = "context_encoding"
 PHASE_TKG = "token_generation"
 
 
+def _hooked(module: nn.Module) -> bool:
+    """Whether a hook records or replaces what goes through the module (utils/tensor_capture)."""
+    return bool(module._forward_hooks or module._forward_pre_hooks)
+
+
 class AttentionBase(nn.Module):
     def __init__(self, config, layer_idx: int = 0, rotary: Optional[RotaryEmbedding] = None):
         super().__init__()
@@ -170,7 +175,8 @@ class AttentionBase(nn.Module):
                 and all(type(n) is RMSNorm and n.weight.numel() == self.head_dim
                         and n.weight.dtype == hidden.dtype and n.weight.is_contiguous()
                         and n.weight.data_ptr() % 16 == 0 for n in norms)
-                and norms[0].variance_epsilon == norms[1].variance_epsilon):
+                and norms[0].variance_epsilon == norms[1].variance_epsilon
+                and not any(map(_hooked, (*norms, self.qkv_proj)))):
             return (norms[0].weight, norms[1].weight, norms[0].variance_epsilon)
         return None
 
@@ -211,7 +217,7 @@ class AttentionBase(nn.Module):
             and self.clip_qkv is None
             and cos is not None
             and not (paged and (not hidden.is_cuda or self.head_dim not in (64, 128)
-                                or self.kv_shard_degree > 1))
+                                or self.kv_shard_degree > 1 or _hooked(self.qkv_proj)))
             and not ((norms or paged) and self.dp_degree > 1)
             and not self.rope_interleaved
             and self.qk_norm_post_rope is None

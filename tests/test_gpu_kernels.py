@@ -2328,3 +2328,57 @@ def test_attention_positions_past_the_capacity(window, Sq, paged):
     else:
         got = ops.attention_decode(q.to(dev), k.to(dev), v.to(dev), pos.to(dev), sliding_window=window)
     assert _rel(got, want) < 1.5 * 2.0 ** -9
+
+
+@pytest.mark.parametrize("normed,paged", [(True, False), (True, True), (False, True)])
+def test_tensor_capture_of_what_the_front_end_takes_in(normed, paged):
+    """Head norms, and the projection in front of pages, still answer to hooks: a captured step
+    leaves the fused front end for the modules, and gives what it gives (the rounding of q and k
+    more, of the result and of the projection: six of half a unit). Linear caches without norms
+    have the projection's own linear layer to hook."""
+    from neuronx_distributed_inference_amd.config import EngineConfig
+    from neuronx_distributed_inference_amd.models.qwen3.modeling_qwen3 import (
+        Qwen3ForCausalLM, Qwen3InferenceConfig)
+    from neuronx_distributed_inference_amd.utils.tensor_capture import TensorCapture
+
+    torch.manual_seed(0)
+    dev, B, S = _dev(), 2, 9
+    ec = EngineConfig(batch_size=B, max_batch_size=B, seq_len=64, max_length=64,
+                      torch_dtype="bfloat16", tp_degree=1, fused_qkv=True, is_block_kv_layout=paged,
+                      pa_block_size=8, pa_num_blocks=16 if paged else None)
+    cfg = Qwen3InferenceConfig(
+        neuron_config=ec, vocab_size=64, hidden_size=256, intermediate_size=256, head_dim=64,
+        num_hidden_layers=1, num_attention_heads=4, num_key_value_heads=2,
+        max_position_embeddings=64, rms_norm_eps=1e-5, hidden_act="silu")
+    with torch.device("cuda"):
+        lm = Qwen3ForCausalLM(cfg).eval()
+    for p in lm.parameters():
+        if p.requires_grad:
+            p.data.normal_(0, 0.06)
+    att = lm.model.layers[0].self_attn
+    names = ["layers.0.self_attn.qkv_proj"]
+    if normed:
+        names += ["layers.0.self_attn.q_norm", "layers.0.self_attn.k_norm"]
+    else:
+        att.q_norm = att.k_norm = None
+    bt = torch.arange(16, device=dev).view(B, 8) if paged else None
+    seq = torch.arange(B, device=dev, dtype=torch.int32)
+
+    def step(n, at):
+        pos = (torch.arange(n, device=dev) + at).repeat(B, 1)
+        h = torch.randn(B, n, 256, device=dev, generator=torch.Generator(dev).manual_seed(at)).bfloat16()
+        if paged:
+            from neuronx_distributed_inference_amd.modules.kvcache.block_kv_cache_manager import (
+                generate_slot_mapping)
+            lm.model.kv_mgr.set_step_context(bt, generate_slot_mapping(bt, pos, 8))
+        cos, sin = lm.model.rotary.get_cos_sin(pos, device=dev)
+        return att(h, cos, sin, lm.model.kv_mgr, pos.int(),
+                   "context_encoding" if at == 0 else "token_generation", seq_ids=seq)
+
+    with torch.inference_mode():
+        plain = [step(S, 0), step(1, S)]
+        with TensorCapture(lm.model, names) as cap:
+            hooked = [step(S, 0), step(1, S)]
+    assert [len(cap.captured[n]) for n in names] == [2] * len(names)
+    for a, b in zip(hooked, plain):
+        assert _rel(a, b) < 6 * 2.0 ** -8
