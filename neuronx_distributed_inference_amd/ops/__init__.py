@@ -916,6 +916,8 @@ def moe_routed_experts(x: torch.Tensor, weights: torch.Tensor, idx: torch.Tensor
     rows = tiles_max * mt
     tabs = torch.empty(1 + 2 * tiles_max + rows + n, dtype=torch.int32, device=dev)
     tiles, gather, inv = tabs.split([1 + 2 * tiles_max, rows, n])
+    if idx.dtype not in (torch.int32, torch.int64):
+        idx = idx.long()
     c.moe_route(tiles, gather, inv, idx.contiguous(), E, first, mt)
     weights = weights.float().contiguous()
     s = scales or (None, None, None)

@@ -2382,3 +2382,15 @@ def test_tensor_capture_of_what_the_front_end_takes_in(normed, paged):
     assert [len(cap.captured[n]) for n in names] == [2] * len(names)
     for a, b in zip(hooked, plain):
         assert _rel(a, b) < 6 * 2.0 ** -8
+
+
+@pytest.mark.parametrize("kind", [torch.int32, torch.int16, torch.uint8])
+def test_moe_routed_experts_take_any_whole_number(kind):
+    """Choices in other integer types are the same choices."""
+    torch.manual_seed(0)
+    dev, T, E, k, H, I = _dev(), 40, 4, 2, 128, 256
+    x = torch.randn(T, H, device=dev).to(torch.bfloat16)
+    wt, idx = torch.softmax(torch.randn(T, E, device=dev), -1).topk(k, dim=-1)
+    w = [(torch.randn(E, *s, device=dev) * 0.1).to(torch.bfloat16) for s in ((I, H), (I, H), (H, I))]
+    want = ops.moe_routed_experts(x, wt, idx, *w, num_experts=E)
+    assert torch.equal(ops.moe_routed_experts(x, wt, idx.to(kind), *w, num_experts=E), want)
