@@ -212,23 +212,23 @@ class ExpertMLPs(nn.Module):
                          idx: torch.Tensor) -> torch.Tensor:
         """The chosen experts' products alone, no top_k/E redundant FLOPs; static
         shapes and tables made on the device, so a captured step holds them. On the GPU the
-        routed kernels, with 16-bit and 8-bit weights; MXFP4 weights, and the CPU reference of
-        all, go through the grouped products: assignments sorted by expert, each expert's
-        padded to 64-row tiles, those of other ranks' experts (EP) in a last segment whose
-        tiles are skipped."""
+        routed kernels, with 16-bit and 8-bit weights; MXFP4 weights, an ``act_mul`` that those
+        kernels do not have, and the CPU reference of all go through the grouped products:
+        assignments sorted by expert, each expert's padded to 64-row tiles, those of other
+        ranks' experts (EP) in a last segment whose tiles are skipped."""
         T, H = x.shape
         El = self.num_local_experts
         offset = self._local_offset()
         top_k = idx.shape[1]
         fp8 = getattr(self, "fp8", False)
         mx4 = getattr(self, "mx4", False)
-        if x.is_cuda and not mx4:
+        if x.is_cuda and not mx4 and self.act_mul in (ops.silu_mul, ops.gelu_tanh_mul):
             ws = [getattr(self, n + ("_q" if fp8 else "")) for n in ("w_gate", "w_up", "w_down")]
             return ops.moe_routed_experts(
                 x, weights, idx, *ws,
                 scales=(self.w_gate_s, self.w_up_s, self.w_down_s) if fp8 else None,
                 first=offset, num_experts=self.num_experts,
-                gelu=self.act_mul is not ops.silu_mul, scale_input=self.scale_input)
+                gelu=self.act_mul is ops.gelu_tanh_mul, scale_input=self.scale_input)
         flat = (idx - offset).view(-1)
         local = (flat >= 0) & (flat < El)
         flat_routed = torch.where(local, flat, torch.full_like(flat, El))

@@ -2394,3 +2394,36 @@ def test_moe_routed_experts_take_any_whole_number(kind):
     w = [(torch.randn(E, *s, device=dev) * 0.1).to(torch.bfloat16) for s in ((I, H), (I, H), (H, I))]
     want = ops.moe_routed_experts(x, wt, idx, *w, num_experts=E)
     assert torch.equal(ops.moe_routed_experts(x, wt, idx.to(kind), *w, num_experts=E), want)
+
+
+@pytest.mark.parametrize("f8", [False, True])
+def test_expert_layer_with_an_activation_of_its_own(f8):
+    """The routed kernels have SiLU and GELU; a layer whose ``act_mul`` is another one computes that
+    one. Against the layer on the CPU in fp32, from the same rounded inputs: the products, the
+    activation and the result are rounded, half a unit each, and so is the scaled result."""
+    from neuronx_distributed_inference_amd.modules.moe import ExpertMLPs
+
+    torch.manual_seed(0)
+    dev, T, E, k, H, I = _dev(), 40, 4, 2, 128, 256
+    m = ExpertMLPs(E, H, I, 1, torch.bfloat16)
+    for p in m.parameters():
+        p.data.normal_(0, 0.1)
+    if f8:
+        assert m.quantize_fp8()
+    m.act_mul = lambda g, u: torch.relu(g) * u
+    x = torch.randn(T, H).to(torch.bfloat16)
+    wt, idx = torch.softmax(torch.randn(T, E), -1).topk(k, dim=-1)
+    with torch.inference_mode():
+        got = m.to(dev)(x.to(dev), wt.to(dev), idx.to(dev))
+        ws = [getattr(m, n + "_q" if f8 else n) for n in ("w_gate", "w_up", "w_down")]
+        if f8:
+            ws = [ops.fp8_moe_dequant(w, getattr(m, n + "_s"))
+                  for w, n in zip(ws, ("w_gate", "w_up", "w_down"))]
+        g, u, d = (w.float().cpu() for w in ws)
+        want = torch.zeros(T, H)
+        for t in range(T):
+            for j in range(k):
+                e = int(idx[t, j])
+                h = torch.relu(g[e] @ x[t].float()) * (u[e] @ x[t].float())
+                want[t] += wt[t, j] * (d[e] @ h)
+    assert _rel(got, want) < 4 * 2.0 ** -9
