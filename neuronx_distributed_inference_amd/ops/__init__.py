@@ -110,6 +110,12 @@ def block_kv_cache_update(k_cache, v_cache, k_new, v_new, slot_mapping):
     ref.block_kv_cache_update(k_cache, v_cache, k_new, v_new, slot_mapping)
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """t, or a copy where it is not contiguous or starts off 16 bytes."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def attention_prefill(q, k, v, mask=None, scale=None, sinks=None, causal=True,
                       sliding_window: int = 0):
     """Flash-attention forward for context encoding.
@@ -126,7 +132,7 @@ def attention_prefill(q, k, v, mask=None, scale=None, sinks=None, causal=True,
             and q.shape[-1] in (64, 128) and q.shape[2] == k.shape[2]
         ):
             out = torch.empty_like(q)
-            c.flash_prefill(out, q.contiguous(), k.contiguous(), v.contiguous(),
+            c.flash_prefill(out, q.contiguous(), _aligned(k), _aligned(v),
                             float(scale), int(sliding_window),
                             sinks=None if sinks is None else sinks.detach())
             return out
@@ -383,12 +389,14 @@ def _attention_out(q, token_major):
     return torch.empty(B, S, H, D, dtype=q.dtype, device=q.device).transpose(1, 2)
 
 
-def _extend_on_mfma(q, k_cache):
+def _extend_on_mfma(q, k_cache, v_cache):
     """Several query tokens of a 16-bit model against a cache of the same type: the matrix-core
     kernel reads each K/V row once for all of them; the decode kernel (one workgroup a query
-    token) serves single tokens, fp32, 8-bit caches and the other head sizes."""
+    token) serves single tokens, fp32, 8-bit caches, the other head sizes and caches that start
+    off 16 bytes (the former stages 16 bytes at a time straight to LDS)."""
     return q.shape[2] > 1 and q.shape[3] in (64, 128) and q.dtype == k_cache.dtype \
-        and q.dtype in (torch.bfloat16, torch.float16)
+        and q.dtype in (torch.bfloat16, torch.float16) \
+        and (k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0
 
 
 def attention_prefill_cached(q, k_cache, v_cache, seq_ids, scale=None,
@@ -407,7 +415,7 @@ def attention_prefill_cached(q, k_cache, v_cache, seq_ids, scale=None,
     if q.is_cuda:
         c = _require_ext("attention_prefill_cached")
         out = _attention_out(q, token_major)
-        c.flash_prefill_cached(out, q.contiguous(), k_cache, v_cache,
+        c.flash_prefill_cached(out, q.contiguous(), _aligned(k_cache), _aligned(v_cache),
                                seq_ids, float(scale), int(sliding_window),
                                sinks=None if sinks is None else sinks.detach())
         return out
@@ -442,7 +450,7 @@ def attention_decode(q, k_cache, v_cache, seq_lens, seq_ids=None, scale=None,
         positions = seq_lens
     if q.is_cuda:
         c = _require_ext("attention_decode")
-        if not ring and _extend_on_mfma(q, k_cache):
+        if not ring and _extend_on_mfma(q, k_cache, v_cache):
             out = _attention_out(q, token_major)
             if seq_ids is None:
                 seq_ids = torch.arange(B, device=q.device, dtype=torch.int32)
@@ -667,7 +675,7 @@ def attention_decode_paged(q, k_cache, v_cache, seq_lens, block_table,
         positions = seq_lens
     if q.is_cuda:
         c = _require_ext("attention_decode_paged")
-        if _extend_on_mfma(q, k_cache):
+        if _extend_on_mfma(q, k_cache, v_cache):
             out = _attention_out(q, token_major)
             c.flash_extend(out, q.contiguous(), k_cache, v_cache, positions,
                            block_table=block_table, scale=float(scale),
@@ -880,12 +888,6 @@ def row_topk(x: torch.Tensor, k: int):
 
 # bytes of fp32 products that the routed down projection keeps at a time
 MOE_WORKSPACE = 1 << 30
-
-
-def _aligned(t: torch.Tensor) -> torch.Tensor:
-    """t, or a copy where it is not contiguous or starts off 16 bytes."""
-    t = t.contiguous()
-    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def moe_routed_experts(x: torch.Tensor, weights: torch.Tensor, idx: torch.Tensor, w_gate, w_up,

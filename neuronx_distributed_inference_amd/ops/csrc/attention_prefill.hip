@@ -620,6 +620,8 @@ void flash_run(torch::Tensor& out, const torch::Tensor& q, const torch::Tensor& 
     TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4 && out.dim() == 4, "bad shapes");
     TORCH_CHECK(q.is_contiguous() && k.is_contiguous() && v.is_contiguous(),
                 "contiguous tensors required");
+    TORCH_CHECK(((size_t)k.data_ptr() | (size_t)v.data_ptr()) % 16 == 0,
+                "flash attention: K/V are staged 16 bytes at a time");
     TORCH_CHECK(out.sizes() == q.sizes() && out.stride(3) == 1 && out.stride(2) % 4 == 0 &&
                 out.stride(1) % 4 == 0 && out.stride(0) % 4 == 0, "flash attention: bad output layout");
     TORCH_CHECK(k.sizes() == v.sizes() && k.size(3) == D, "flash attention: K/V shapes differ");

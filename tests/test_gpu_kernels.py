@@ -2427,3 +2427,30 @@ def test_expert_layer_with_an_activation_of_its_own(f8):
                 h = torch.relu(g[e] @ x[t].float()) * (u[e] @ x[t].float())
                 want[t] += wt[t, j] * (d[e] @ h)
     assert _rel(got, want) < 4 * 2.0 ** -9
+
+
+@pytest.mark.parametrize("kind", ["prompt", "cached", "extend", "paged"])
+def test_attention_takes_keys_and_values_off_16_bytes(kind):
+    """K and V that start off 16 bytes give what aligned ones do (by another kernel over a cache:
+    the rounding of the two results)."""
+    torch.manual_seed(0)
+    dev, B, H, S, D, cap, bs = _dev(), 2, 4, 40, 64, 64, 16
+    q = torch.randn(B, H, S, D, device=dev).to(torch.bfloat16)
+    rows = S if kind == "prompt" else cap
+    k, v = (torch.randn(B, H, rows, D, device=dev).to(torch.bfloat16) for _ in range(2))
+    pos = torch.arange(S, device=dev).expand(B, S)
+    seq = torch.arange(B, device=dev, dtype=torch.int32)
+    if kind == "paged":
+        k, v = (t.transpose(1, 2).reshape(B * cap // bs, bs, H, D).contiguous() for t in (k, v))
+    call = {
+        "prompt": lambda k, v: ops.attention_prefill(q, k, v),
+        "cached": lambda k, v: ops.attention_prefill_cached(q, k, v, seq),
+        "extend": lambda k, v: ops.attention_decode(q, k, v, pos, seq_ids=seq),
+        "paged": lambda k, v: ops.attention_decode_paged(
+            q, k, v, pos, torch.arange(B * cap // bs, device=dev).view(B, -1)),
+    }[kind]
+
+    def off(t):
+        return torch.empty(t.numel() + 1, dtype=t.dtype, device=dev)[1:].view(t.shape).copy_(t)
+
+    assert _rel(call(off(k), off(v)), call(k, v)) < 2.0 ** -8
