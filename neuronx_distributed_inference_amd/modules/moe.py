@@ -296,8 +296,8 @@ class ExpertMLPs(nn.Module):
         # The routed kernels are the GPU default at every size (opt out with
         # NXDI_MOE_GROUPED=0): they read the chosen experts' weights once,
         # the dense products all experts' and compute E/top_k times as much.
-        # 8 experts of 4096 x 14336: 250 us for a token, 529-567 for 16-191;
-        # one pass over all the weights alone takes 577.
+        # 8 experts of 4096 x 14336: 250 us for a token, 529-567 for 16-191
+        # (all the weights, 2.8 GB, at 5.0-5.3 TB/s; a large copy does 4.9).
         import os as _os
 
         if getattr(self, "fp8", False) or getattr(self, "mx4", False):

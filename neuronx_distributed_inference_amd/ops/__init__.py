@@ -391,8 +391,8 @@ def _attention_out(q, token_major):
 
 def _extend_on_mfma(q, k_cache, v_cache):
     """Several query tokens of a 16-bit model against a cache of the same type: the matrix-core
-    kernel reads each K/V row once for all of them; the decode kernel (one workgroup a query
-    token) serves single tokens, fp32, 8-bit caches, the other head sizes and caches that start
+    kernel reads each K/V row once for all of them; the decode kernel (once for 16 pairs of token
+    and head, in fp32 for each token) serves single tokens, fp32, 8-bit caches, the other head sizes and caches that start
     off 16 bytes (the former stages 16 bytes at a time straight to LDS)."""
     return q.shape[2] > 1 and q.shape[3] in (64, 128) and q.dtype == k_cache.dtype \
         and q.dtype in (torch.bfloat16, torch.float16) \

@@ -6,8 +6,9 @@
 // HBM); with many the matrix cores, and before those the LDS (128 B/clk a CU).
 //
 //   * Workgroup = 8 waves, MT rows of one expert x 256 columns. K goes in steps of 128 B of a
-//     weight row (128 deep with 8-bit weights, and then 64 rows at most) through a ring of three LDS buffers, global_load_lds throughout, one raw barrier a step and a
-//     counted vmcnt: two steps are in flight while one is computed.
+//     weight row (128 deep with 8-bit weights, and then 64 rows at most) through a ring of three
+//     LDS buffers, global_load_lds throughout, one raw barrier a step and a counted vmcnt: two
+//     steps are in flight while one is computed.
 //   * The row tiles of an expert want the same weights: the list of workgroups (8 row tiles x
 //     all column tiles, rows fastest) is cut into 8 contiguous parts, one for each XCD, so that
 //     they meet in one L2. The list covers real tiles only; the grid is sized for the worst
@@ -22,9 +23,10 @@
 //
 // The three products of a layer in us, before = moe_grouped_kernel (64 rows x 256 columns, a
 // launch each for gate, up and activation, atomics):
-//   128 experts of 2048 x 768, 8 a token:  2048 tokens 776 -> 364 (weights alone: 247);
+//   128 experts of 2048 x 768, 8 a token:  2048 tokens 776 -> 364 (weights at the 4.9 TB/s of
+//     a large copy: 247);
 //     512 tokens 379 -> 266;  8 experts of 4096 x 14336, 2 a token: 4096 tokens 6379 -> 3290
-//     (bf16 products alone 1850), 256 tokens 688 -> 604 (577), 128 tokens in 8 bits
+//     (bf16 products alone 1850), 256 tokens 688 -> 604 (577 at that rate), 128 tokens in 8 bits
 //     376 -> 309 (288).
 // Row tiles (32, 64, 128), gate + up and down with its sum: 32 rows an expert 164+102, 144+92,
 // 144+100 (64 rows 224+138, 172+118, 150+118); 128 rows 358+234, 237+185, 202+164;
