@@ -677,13 +677,14 @@ def test_moe_mx4_grouped_cpu_matches_bf16():
     assert err < 0.35, float(err)  # 4-bit weights: coarse but bounded
 
 
-def test_moe_grouped_tile32_cpu_matches_dense(monkeypatch):
-    """32-row tile path (fine-grained MoE) vs the dense path on CPU."""
+def test_moe_grouped_tile32_cpu_matches_dense():
+    """Grouped products in 32-row tiles (few tokens an expert), gathered and combined, vs the
+    layer's dense path on CPU."""
     import torch
 
+    from neuronx_distributed_inference_amd import ops
     from neuronx_distributed_inference_amd.modules.moe import ExpertMLPs
 
-    monkeypatch.setenv("NXDI_MOE_TILE32", "1")
     torch.manual_seed(14)
     E, H, I, T, top_k = 16, 128, 256, 24, 4   # 6 tokens/expert avg
     m = ExpertMLPs(num_experts=E, hidden_size=H, intermediate_size=I,
@@ -694,7 +695,14 @@ def test_moe_grouped_tile32_cpu_matches_dense(monkeypatch):
     x = torch.randn(T, H) * 0.3
     w, idx = torch.softmax(torch.randn(T, E), -1).topk(top_k, dim=-1)
     want = m._forward_dense(x, w, idx)
-    got = m._forward_grouped(x, w, idx)
+    order, dest, eids, gtab, Mpad = ops.moe_grouped_tables(idx.reshape(-1), E, top_k, tile=32)
+    assert Mpad % 32 == 0 and eids.numel() == Mpad // 32
+    g, u = (ops.moe_grouped_gemm(x, v, eids, x_gather=gtab, mt=32) for v in (m.w_gate, m.w_up))
+    scale = torch.zeros(Mpad)
+    scale[dest] = w.reshape(-1)[order]
+    got = ops.moe_grouped_gemm(ops.silu_mul(g, u), m.w_down, eids, mt=32,
+                               combine_out=torch.zeros(T, H), combine_scale=scale,
+                               combine_gather=gtab)
     torch.testing.assert_close(got, want, atol=1e-4, rtol=1e-4)
 
 
