@@ -848,9 +848,15 @@ ROW_TOPK_MAX = 2048
 
 
 def _row_kernels(x: torch.Tensor) -> bool:
-    """Whether the row kernels take x: they have no backward and count elements in 31 bits."""
+    """Whether the row kernels take x: they count elements in 31 bits."""
     return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16, torch.float32)
-            and 0 < x.size(-1) < (1 << 31) - 8192 and not (x.requires_grad and torch.is_grad_enabled()))
+            and 0 < x.size(-1) < (1 << 31) - 8192)
+
+
+def _wants_gradients(x: torch.Tensor) -> bool:
+    """The kernels have no backward: values of such an x are gathered from it. (Logits of a model
+    that is captured outside of inference mode are such.)"""
+    return x.requires_grad and torch.is_grad_enabled()
 
 
 def _rows(x: torch.Tensor) -> torch.Tensor:
@@ -865,7 +871,7 @@ def row_max(x: torch.Tensor):
         vals = torch.empty(x.shape[:-1], dtype=x.dtype, device=x.device)
         idx = torch.empty(x.shape[:-1], dtype=torch.long, device=x.device)
         c.row_max(vals, idx, _rows(x))
-        return vals, idx
+        return (x.gather(-1, idx.unsqueeze(-1)).squeeze(-1) if _wants_gradients(x) else vals), idx
     return x.max(dim=-1)
 
 
@@ -879,7 +885,7 @@ def row_topk(x: torch.Tensor, k: int):
         vals = torch.empty(*x.shape[:-1], k, dtype=x.dtype, device=x.device)
         idx = torch.empty(*x.shape[:-1], k, dtype=torch.long, device=x.device)
         c.row_topk(vals, idx, _rows(x), k)
-        return vals, idx
+        return (x.gather(-1, idx) if _wants_gradients(x) else vals), idx
     if x.is_cuda and torch.cuda.is_current_stream_capturing():
         raise RuntimeError(f"row_topk: k = {k} of {x.dtype} cannot be captured (at most "
                            f"{ROW_TOPK_MAX} of 16- or 32-bit floats)")

@@ -2269,8 +2269,8 @@ def test_row_topk_many_rows(rows, n, k):
 
 
 def test_row_topk_refuses_what_a_capture_cannot_hold(monkeypatch):
-    """More than the kernel holds goes to torch's topk, but not into a graph; gradients go through
-    torch's as well."""
+    """More than the kernel holds goes to torch's topk, but not into a graph; the kernel's
+    values pass gradients on."""
     x = torch.randn(2, 5000, device=_dev())
     assert torch.equal(ops.row_topk(x, 3000)[0], x.topk(3000)[0])
     y = x.clone().requires_grad_()
@@ -2454,3 +2454,42 @@ def test_attention_takes_keys_and_values_off_16_bytes(kind):
         return torch.empty(t.numel() + 1, dtype=t.dtype, device=dev)[1:].view(t.shape).copy_(t)
 
     assert _rel(call(off(k), off(v)), call(k, v)) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("do_sample", [False, True])
+def test_decode_captured_outside_of_inference_mode(do_sample):
+    """Loading a model captures its decode step with gradients enabled, so that the logits want them:
+    the sampling step is captured all the same. Greedy tokens are the logits' largest, and so are
+    sampled ones of one candidate."""
+    from neuronx_distributed_inference_amd.config import EngineConfig, OnDeviceSamplingConfig
+    from neuronx_distributed_inference_amd.models.llama.modeling_llama import (
+        LlamaForCausalLM, LlamaInferenceConfig)
+
+    torch.manual_seed(0)
+    dev, B = _dev(), 2
+    ec = EngineConfig(
+        batch_size=B, max_batch_size=B, seq_len=64, max_length=64, torch_dtype="bfloat16",
+        tp_degree=1, output_logits=True, on_device_sampling_config=OnDeviceSamplingConfig(
+            do_sample=do_sample, top_k=1 if not do_sample else 5))
+    cfg = LlamaInferenceConfig(
+        neuron_config=ec, vocab_size=512, hidden_size=256, intermediate_size=256,
+        num_hidden_layers=1, num_attention_heads=4, num_key_value_heads=2,
+        max_position_embeddings=64, rms_norm_eps=1e-5, rope_theta=10000.0, hidden_act="silu",
+        tie_word_embeddings=False)
+    with torch.device("cuda"):
+        lm = LlamaForCausalLM(cfg).eval()
+    for p in lm.parameters():
+        if p.requires_grad:
+            p.data.normal_(0, 0.1)
+    assert torch.is_grad_enabled()
+    lm.enable_submodels()
+    lm.warmup()
+    params = torch.tensor([[1, 1.0, 1.0]] * B, device=dev)
+    with torch.inference_mode():
+        ids = torch.randint(0, 512, (B, 8), device=dev)
+        tok = lm(input_ids=ids, sampling_params=params).tokens
+        for at in range(8, 11):
+            out = lm(input_ids=tok.view(B, 1), sampling_params=params,
+                     position_ids=torch.full((B, 1), at, device=dev))
+            tok = out.tokens.clone()
+            assert torch.equal(tok.view(-1), out.logits.view(B, -1).argmax(-1))
