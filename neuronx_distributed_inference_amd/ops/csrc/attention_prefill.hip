@@ -594,12 +594,9 @@ void flash_launch(torch::Tensor& out, const torch::Tensor& q, const torch::Tenso
     const int gq = a.Hq / a.Hkv;
     a.nqt = (int)(((long)gq * a.S + QROWS - 1) / QROWS);
     const size_t lds = 4 * KT * D * 2 + 8 * sizeof(int) + (PAGED ? 2 * (KT + 1) * sizeof(int) : 0);
-    static const bool once = [&] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_kernel<T, D, PAGED, HILO>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        return true;
-    }();
-    (void)once;
+    // a limit of the function on the device at hand, the same in every call
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_kernel<T, D, PAGED, HILO>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const long blocks = (long)a.B * a.Hkv * a.nqt * a.nsplit;
     TORCH_CHECK(blocks < (1l << 31), "flash attention: too many query rows");
     hipLaunchKernelGGL((flash_kernel<T, D, PAGED, HILO>), dim3((unsigned)blocks), dim3(256), lds, stream,
