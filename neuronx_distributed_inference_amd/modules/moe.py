@@ -210,7 +210,7 @@ class ExpertMLPs(nn.Module):
 
     def _forward_grouped(self, x: torch.Tensor, weights: torch.Tensor,
                          idx: torch.Tensor) -> torch.Tensor:
-        """The chosen experts' products alone (SURVEY K12), no top_k/E redundant FLOPs; static
+        """The chosen experts' products alone, no top_k/E redundant FLOPs; static
         shapes and tables made on the device, so a captured step holds them. On the GPU the
         routed kernels, with 16-bit and 8-bit weights; MXFP4 weights, an ``act_mul`` that those
         kernels do not have, and the CPU reference of all go through the grouped products:
