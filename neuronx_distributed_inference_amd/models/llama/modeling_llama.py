@@ -109,6 +109,10 @@ class LlamaDecoderLayer(nn.Module):
         h = self.mlp(h, sequence_parallel=sequence_parallel)
         return h, residual
 
+    def fused_parts(self):
+        """What modules/fused_layer.py runs in place of :meth:`forward`."""
+        return self.self_attn, self.mlp
+
 
 class LlamaModel(DecoderModel):
     def build_layers(self, config: InferenceConfig) -> nn.ModuleList:

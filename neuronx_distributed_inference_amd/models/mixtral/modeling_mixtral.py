@@ -45,6 +45,10 @@ class MixtralDecoderLayer(nn.Module):
         h = self.mlp(h)
         return h, residual
 
+    def fused_parts(self):
+        """What modules/fused_layer.py runs in place of :meth:`forward`."""
+        return self.self_attn, self.mlp
+
 
 class MixtralModel(DecoderModel):
     def build_layers(self, config):

@@ -29,6 +29,7 @@ from neuronx_distributed_inference_amd.modules.attention.attention_base import (
     PHASE_CTE,
     PHASE_TKG,
 )
+from neuronx_distributed_inference_amd.modules.fused_layer import fusable, run_layers
 from neuronx_distributed_inference_amd.modules.generation.sampling import (
     Sampler,
     prepare_sampling_params,
@@ -267,7 +268,17 @@ class DecoderModel(nn.Module):
         residual = None
         post_fns = getattr(self, "_layer_post_fns", None)
         h_embed = h
-        for ri, (li, layer) in enumerate(self.layer_runs()):
+        runs = self.layer_runs()
+        fused = [layer for _, layer in runs]
+        if (not sp_active and not post_fns and not getattr(self, "eagle3_capture_layers", None)
+                and type(self).before_layer_run is DecoderModel.before_layer_run
+                and fusable(fused, self.norm, h, attention_mask, phase)):
+            h = run_layers(fused, self.norm, h, cos, sin, self.kv_mgr, position_ids, phase,
+                           attention_mask, seq_ids)
+            runs, normed = (), True
+        else:
+            normed = False
+        for ri, (li, layer) in enumerate(runs):
             h = self.before_layer_run(ri, h, h_embed)
             if sp_active:
                 h, residual = layer(
@@ -291,7 +302,9 @@ class DecoderModel(nn.Module):
                 if li == cap[0]:
                     self.eagle3_hiddens = {}
                 self.eagle3_hiddens[li] = (h + residual) if residual is not None else h
-        if residual is not None:
+        if normed:
+            pass
+        elif residual is not None:
             h, _ = self.norm(h, residual)
         else:
             h = self.norm(h)

@@ -56,6 +56,10 @@ class Qwen3MoeDecoderLayer(nn.Module):
         h = self.mlp(h)
         return h, residual
 
+    def fused_parts(self):
+        """What modules/fused_layer.py runs in place of :meth:`forward`."""
+        return self.self_attn, self.mlp
+
 
 class Qwen3MoeModel(DecoderModel):
     def build_layers(self, config):

@@ -30,6 +30,7 @@ from neuronx_distributed_inference_amd.modules.attention.gqa import (
 from neuronx_distributed_inference_amd.modules.norm import RMSNorm
 from neuronx_distributed_inference_amd.modules.rope import RotaryEmbedding
 from neuronx_distributed_inference_amd.parallel import state as ps
+from neuronx_distributed_inference_amd.parallel.layers import plain_linear
 
 PHASE_CTE = "context_encoding"
 PHASE_TKG = "token_generation"
@@ -180,8 +181,15 @@ class AttentionBase(nn.Module):
             return (norms[0].weight, norms[1].weight, norms[0].variance_epsilon)
         return None
 
-    # ------------------------------------------------------------------
-    def forward(
+    def _qkv_product(self, hidden: torch.Tensor) -> torch.Tensor:
+        """Output of the fused q|k|v projection, or its parts of K, which qkv_rope_update adds up
+        (head sizes whose kernel does)."""
+        if (self.head_dim in (32, 64, 128, 256) and plain_linear(self.qkv_proj.qkv, hidden)
+                and not _hooked(self.qkv_proj)):
+            return ops.linear_parts(hidden, self.qkv_proj.qkv.weight)
+        return self.qkv_proj.qkv(hidden)
+
+    def attend_fused(
         self,
         hidden: torch.Tensor,
         cos: torch.Tensor,
@@ -193,18 +201,12 @@ class AttentionBase(nn.Module):
         seq_ids: Optional[torch.Tensor] = None,
         active_mask: Optional[torch.Tensor] = None,
         sequence_parallel: bool = False,
-    ) -> torch.Tensor:
+    ) -> Optional[torch.Tensor]:
+        """The input of the output projection (B, S, heads * head_dim), where a fused front end
+        serves this call; None where the modules one by one have to."""
         B, S, _ = hidden.shape
-        if sequence_parallel:
-            S = S * self.tp_degree  # hidden is S-sharded; attention runs full-S
         if not self.use_rope:  # NoPE layer (Llama4 global-attention layers)
             cos, sin = None, None
-        # a 4-D mask in TKG is an EXPLICIT attention mask (tree-structured
-        # speculation); 2-D masks stay padding masks
-        if (active_mask is None and attention_mask is not None
-                and attention_mask.dim() == 4 and phase == PHASE_TKG):
-            active_mask = attention_mask
-
         # Fused TKG front end (K2-analog): one GEMM -> one kernel doing
         # RoPE (and plain per-head qk-norms) + cache write, into rows or pages,
         # + q relayout. Other norms and clip_qkv need the unfused path.
@@ -223,7 +225,7 @@ class AttentionBase(nn.Module):
             and self.qk_norm_post_rope is None
             and self.q_scale_fn is None
         ):
-            y = self.qkv_proj.qkv(hidden)
+            y = self._qkv_product(hidden)
             import neuronx_distributed_inference_amd.ops as _ops
 
             if paged:
@@ -246,10 +248,10 @@ class AttentionBase(nn.Module):
                 wpos, seq_ids,
                 self.num_heads_per_rank, self.num_kv_heads_per_rank,
                 norms=norms or None, slots=kv_mgr.slot_mapping if paged else None,
+                dtype=hidden.dtype,
             )
             out = self._decode(q, kv_mgr, position_ids, seq_ids, active_mask)
-            out = out.transpose(1, 2).reshape(B, S, -1)
-            return self.o_proj(out)
+            return out.transpose(1, 2).reshape(B, S, -1)
 
         # Fused CTE front end: one GEMM -> qkv_rope_update (RoPE + cache
         # scatter + q relayout) -> flash attention reading K/V straight from
@@ -283,10 +285,11 @@ class AttentionBase(nn.Module):
             if kc.dtype == hidden.dtype:  # fp8 cache: unfused CTE path below
                 import neuronx_distributed_inference_amd.ops as _ops
 
-                y = self.qkv_proj.qkv(hidden)
+                y = self._qkv_product(hidden)
                 q = _ops.qkv_rope_update(
                     y, cos, sin, kc, vc, position_ids, seq_ids,
                     self.num_heads_per_rank, self.num_kv_heads_per_rank, norms=norms or None,
+                    dtype=hidden.dtype,
                 )
                 if norms and attention_mask is not None:
                     # by position, which counts the mask's tokens wherever they stand, with
@@ -301,8 +304,37 @@ class AttentionBase(nn.Module):
                         q, kc, vc, seq_ids, scale=self.scale, sinks=self.sinks,
                         sliding_window=self.sliding_window, token_major=True,
                     )
-                out = out.transpose(1, 2).reshape(B, S, -1)
-                return self.o_proj(out)
+                return out.transpose(1, 2).reshape(B, S, -1)
+        return None
+
+    # ------------------------------------------------------------------
+    def forward(
+        self,
+        hidden: torch.Tensor,
+        cos: torch.Tensor,
+        sin: torch.Tensor,
+        kv_mgr,
+        position_ids: torch.Tensor,
+        phase: str,
+        attention_mask: Optional[torch.Tensor] = None,
+        seq_ids: Optional[torch.Tensor] = None,
+        active_mask: Optional[torch.Tensor] = None,
+        sequence_parallel: bool = False,
+    ) -> torch.Tensor:
+        B, S, _ = hidden.shape
+        if sequence_parallel:
+            S = S * self.tp_degree  # hidden is S-sharded; attention runs full-S
+        # a 4-D mask in TKG is an EXPLICIT attention mask (tree-structured
+        # speculation); 2-D masks stay padding masks
+        if (active_mask is None and attention_mask is not None
+                and attention_mask.dim() == 4 and phase == PHASE_TKG):
+            active_mask = attention_mask
+        out = self.attend_fused(hidden, cos, sin, kv_mgr, position_ids, phase, attention_mask,
+                                seq_ids, active_mask, sequence_parallel)
+        if out is not None:
+            return self.o_proj(out)
+        if not self.use_rope:
+            cos, sin = None, None
 
         if (
             phase == PHASE_CTE and self.cp_degree > 1

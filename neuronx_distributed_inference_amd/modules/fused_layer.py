@@ -1,0 +1,83 @@
+"""Decoder layers (norm, attention, residual, norm, feed-forward, residual) in fewer launches.
+
+Between two products stands one kernel: the residual sum and the norm that follows take the parts
+of K of the output and down projections (``ops.add_norm``), rope and cache write those of q|k|v,
+and gate|up writes its activation. A step of few tokens is a chain of such launches, each waiting
+for the last. The layer's modules keep the weights; they are not called, so a layer with hooks on
+any of them, biases, 8-bit weights, adapters or tensor parallelism keeps the chain of modules.
+"""
+
+from __future__ import annotations
+
+import torch
+from torch.nn.modules import module as nn_module
+
+from neuronx_distributed_inference_amd import ops
+from neuronx_distributed_inference_amd.modules.attention.attention_base import (
+    PHASE_TKG,
+    AttentionBase,
+    _hooked,
+)
+from neuronx_distributed_inference_amd.modules.mlp import GatedMLP
+from neuronx_distributed_inference_amd.modules.norm import RMSNorm
+from neuronx_distributed_inference_amd.parallel.layers import plain_linear
+
+
+def _plain_norm(norm, h: torch.Tensor) -> bool:
+    return (type(norm) is RMSNorm and not _hooked(norm) and norm.weight.dtype == h.dtype
+            and norm.weight.is_contiguous() and norm.weight.data_ptr() % 16 == 0)
+
+
+def fusable(layers, final_norm, h: torch.Tensor, attention_mask, phase: str) -> bool:
+    """Whether :func:`run_layers` may stand for calling the layers and the final norm on h."""
+    if not (h.is_cuda and h.dtype in (torch.bfloat16, torch.float16) and h.shape[-1] % 8 == 0
+            and h.shape[-1] <= 32768 and h.numel() and h.is_contiguous()
+            and h.data_ptr() % 16 == 0):
+        return False
+    if nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks:
+        return False
+    if attention_mask is not None and attention_mask.dim() == 4 and phase == PHASE_TKG:
+        return False
+    if not _plain_norm(final_norm, h):
+        return False
+    for layer in layers:
+        ready = getattr(layer, "fused_parts", None)
+        if ready is None or _hooked(layer):
+            return False
+        attn, mlp = ready()
+        if not (isinstance(attn, AttentionBase) and type(attn).forward is AttentionBase.forward
+                and type(attn).attend_fused is AttentionBase.attend_fused
+                and not _hooked(attn) and not _hooked(attn.o_proj)
+                and plain_linear(attn.o_proj.o_proj, h)
+                and _plain_norm(layer.input_layernorm, h)
+                and _plain_norm(layer.post_attention_layernorm, h)):
+            return False
+    return True
+
+
+def _feed_forward(mlp, x: torch.Tensor) -> torch.Tensor:
+    """Output of the feed-forward, or its parts of K."""
+    if (type(mlp) is GatedMLP and not _hooked(mlp) and mlp.fused
+            and mlp.act_mul_fused is ops.silu_mul_fused
+            and plain_linear(mlp.gate_up_proj, x) and plain_linear(mlp.down_proj, x)):
+        return ops.linear_parts(ops.linear_silu_mul(x, mlp.gate_up_proj.weight),
+                                mlp.down_proj.weight)
+    return mlp(x)
+
+
+def run_layers(layers, final_norm, h: torch.Tensor, cos, sin, kv_mgr, position_ids, phase,
+               attention_mask, seq_ids) -> torch.Tensor:
+    """Normed output of the stack; h becomes the residual stream."""
+    layers = list(layers)
+    x = layers[0].input_layernorm(h)
+    for layer, after in zip(layers, layers[1:] + [None]):
+        attn, mlp = layer.fused_parts()
+        args = (x, cos, sin, kv_mgr, position_ids, phase, attention_mask, seq_ids)
+        a = attn.attend_fused(*args)
+        y = attn(*args) if a is None else ops.linear_parts(a, attn.o_proj.o_proj.weight)
+        norm = layer.post_attention_layernorm
+        x = ops.add_norm(y, h, norm.weight, norm.variance_epsilon)
+        y = _feed_forward(mlp, x)
+        norm = final_norm if after is None else after.input_layernorm
+        x = ops.add_norm(y, h, norm.weight, norm.variance_epsilon)
+    return x

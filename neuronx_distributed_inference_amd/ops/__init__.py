@@ -211,8 +211,8 @@ def lt_linear(x: torch.Tensor, weight: torch.Tensor,
 
 
 # ----------------------------------------------------------------------
-# Decode-GEMM dispatch: skinny_gemm5 (hand-written CDNA4 all-glds kernel,
-# ops/csrc/skinny_gemm5.hip) vs the autotuned hipBLASLt path, TIMED per
+# Decode-GEMM dispatch: the tiled kernel (hand-written CDNA4 all-glds kernel,
+# ops/csrc/tile_gemm.hip) vs the autotuned hipBLASLt path, TIMED per
 # exact (M, N, K, bias, dtype) shape at first sight and the winner
 # replayed (graph-safe: replay is a plain stream enqueue). Covers the
 # reference's fused decode projections.
@@ -249,6 +249,29 @@ def skinny_gemm5(x2: torch.Tensor, weight: torch.Tensor, bias=None, rs=None,
     return y
 
 
+def _sg5_candidates(M: int, N: int, K: int):
+    """(mt, splitk) variants: splitk sized so total blocks land near
+    0.5-2x the 256 CUs (guide: per-block latency ~constant in N); row
+    sub-tiles (mt < M) trade extra W traffic for >1 block/CU
+    co-residency (block-level DMA/compute overlap)."""
+    cands = []
+    mts = [0]
+    if M > 128:
+        mts.append(128)
+    if M > 64:
+        mts.append(64)
+    for mt in mts:
+        mb = 1 if mt == 0 else (M + mt - 1) // mt
+        for sk in (1, 2, 4, 8):
+            if K % (64 * sk):
+                continue
+            blocks = (N // 64) * sk * mb
+            if blocks > 560 or (sk > 1 and blocks > 520):
+                continue
+            cands.append((mt, sk))
+    return cands
+
+
 _SK5F8_WS = {}
 
 
@@ -278,31 +301,52 @@ def skinny_gemm5_fp8(x2: torch.Tensor, wq_u8: torch.Tensor,
     return y
 
 
-def _sg5_candidates(M: int, N: int, K: int):
-    """(mt, splitk) variants: splitk sized so total blocks land near
-    0.5-2x the 256 CUs (guide: per-block latency ~constant in N); row
-    sub-tiles (mt < M) trade extra W traffic for >1 block/CU
-    co-residency (block-level DMA/compute overlap)."""
-    cands = []
-    mts = [0]
-    if M > 128:
-        mts.append(128)
-    if M > 64:
-        mts.append(64)
-    for mt in mts:
-        mb = 1 if mt == 0 else (M + mt - 1) // mt
-        for sk in (1, 2, 4, 8):
-            if K % (64 * sk):
-                continue
-            blocks = (N // 64) * sk * mb
-            if blocks > 560 or (sk > 1 and blocks > 520):
-                continue
-            cands.append((mt, sk))
-    return cands
+def _tile_takes(x2: torch.Tensor, weight: torch.Tensor, glu: bool = False) -> int:
+    """Parts of K that the tiled product (csrc/tile_gemm.hip) plans for x2 @ weight^T, 0 where it
+    does not take it."""
+    if not (x2.is_cuda and x2.dtype in (torch.bfloat16, torch.float16) and x2.dtype == weight.dtype
+            and x2.is_contiguous() and weight.is_contiguous()
+            and (x2.data_ptr() | weight.data_ptr()) % 16 == 0):
+        return 0
+    c = _require_ext("tile_gemm")
+    return c.tile_gemm_splits(x2.shape[0], weight.shape[0], weight.shape[1], glu)
+
+
+def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """x @ weight^T for a kernel that adds up the parts of K itself (add_norm, qkv_rope_update):
+    (parts, *x.shape[:-1], N) in fp32 where the product is split, else (*x.shape[:-1], N)."""
+    x2 = x.reshape(-1, x.shape[-1])
+    if _tile_takes(x2, weight):
+        y = _C.tile_gemm(x2, weight, parts=True)
+        return y.view(*y.shape[:-2], *x.shape[:-1], weight.shape[0])
+    from neuronx_distributed_inference_amd.parallel.layers import _linear
+
+    return _linear(x, weight)
+
+
+def linear_silu_mul(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """silu(gate) * up of x @ [gate | up]^T."""
+    x2 = x.reshape(-1, x.shape[-1])
+    if _tile_takes(x2, weight, True):
+        return _C.tile_gemm(x2, weight, glu=True).view(*x.shape[:-1], weight.shape[0] // 2)
+    from neuronx_distributed_inference_amd.parallel.layers import _linear
+
+    return silu_mul_fused(_linear(x, weight))
+
+
+def add_norm(y: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
+             eps: float) -> torch.Tensor:
+    """RMS norm of residual + y; residual becomes the sum. y: of residual's shape, or parts of a
+    split product (linear_parts)."""
+    out = torch.empty_like(residual)
+    _require_ext("add_norm").add_norm(
+        out, residual, y.reshape(y.shape[0], -1, y.shape[-1]) if y.dim() > residual.dim() else y,
+        weight, eps)
+    return out
 
 
 def _sg5_autotune(key, x2, weight, bias) -> int:
-    """Returns 0 (= lt/library path) or the winning (mt, splitk). Timed
+    """Returns 0 (= lt/library path) or the winning number of parts of K. Timed
     over ROTATING weight clones so the stream is cache-cold like the real
     decode loop (the 256 MB L3 would otherwise hold the whole weight and
     flip the verdict); x stays hot, which is also realistic."""
@@ -334,12 +378,11 @@ def _sg5_autotune(key, x2, weight, bias) -> int:
         results[0] = _time(lambda w: lt_linear(x2, w, bias))
     except Exception:  # noqa: BLE001
         results[0] = float("inf")
-    for mt, sk in _sg5_candidates(M, N, K):
+    for sk in sorted({1, _tile_takes(x2, weight)} - {0}):
         try:
-            results[(mt, sk)] = _time(
-                lambda w, s=sk, m=mt: skinny_gemm5(x2, w, bias, splitk=s, mt=m))
+            results[sk] = _time(lambda w, s=sk: _C.tile_gemm(x2, w, bias, splits=s))
         except Exception:  # noqa: BLE001
-            results[(mt, sk)] = float("inf")
+            results[sk] = float("inf")
     del wcopies
     choice = min(results, key=results.get)
     # microbench rankings transfer to in-graph steady state with ~±20%
@@ -353,31 +396,25 @@ def _sg5_autotune(key, x2, weight, bias) -> int:
 
 
 def decode_linear(x: torch.Tensor, weight: torch.Tensor, bias=None) -> torch.Tensor:
-    """Shape-autotuned decode projection: hand-written skinny_gemm5 vs
-    hipBLASLt, winner replayed per shape. Falls through to lt_linear for
-    shapes sg5 does not serve."""
+    """Shape-autotuned decode projection: the tiled kernel (csrc/tile_gemm.hip), in one part of K
+    and in as many as it plans, vs hipBLASLt, winner replayed per shape. Falls through to
+    lt_linear for shapes that the tiled kernel does not take."""
     shape = x.shape
-    x2 = x.reshape(-1, shape[-1])
+    x2 = x.reshape(-1, shape[-1]).contiguous()
     M, K = x2.shape
     N = weight.shape[0]
-    eligible = (
-        8 <= M <= 256 and N % 64 == 0 and K % 64 == 0
-        and x.dtype in (torch.bfloat16, torch.float16)
-        and os.environ.get("NXDI_DISABLE_SG5") != "1"
-    )
-    if not eligible:
+    if not _tile_takes(x2, weight) or os.environ.get("NXDI_DISABLE_SG5") == "1" \
+            or (bias is not None and not bias.is_contiguous()):
         return lt_linear(x, weight, bias)
     key = (M, N, K, bias is not None, x.dtype)
     choice = _sg5_state["choice"].get(key)
     if choice is None:
         if torch.cuda.is_current_stream_capturing():
             return lt_linear(x, weight, bias)  # never tune inside a capture
-        choice = _sg5_autotune(key, x2.contiguous(), weight, bias)
+        choice = _sg5_autotune(key, x2, weight, bias)
     if choice == 0:
         return lt_linear(x, weight, bias)
-    mt, sk = choice
-    y = skinny_gemm5(x2.contiguous(), weight, bias, splitk=sk, mt=mt)
-    return y.view(*shape[:-1], N)
+    return _C.tile_gemm(x2, weight, bias, splits=choice).view(*shape[:-1], N)
 
 
 def _attention_out(q, token_major):
@@ -594,18 +631,20 @@ def topk_topp_sample(logits, top_k, top_p, temperature, rand, global_topk: int =
 
 
 def qkv_rope_update(qkv, cos, sin, k_cache, v_cache, positions, seq_ids, Hq, Hkv,
-                    norms=None, slots=None):
+                    norms=None, slots=None, dtype=None):
     """Fused qkv-GEMM output -> RoPE(q,k) -> cache write(k,v) -> q (B,Hq,S,D).
 
-    qkv: (B, S, (Hq+2Hkv)*D) contiguous; cos/sin (B,S,D) fp32. ``norms`` = (q weight, k weight,
+    qkv: (B, S, (Hq+2Hkv)*D) contiguous, or the parts of a split product (linear_parts); cos/sin
+    (B,S,D) fp32. ``norms`` = (q weight, k weight,
     eps) of per-head RMS norms before the rope. With ``slots`` (B*S flat slots) the caches are
-    pages (blocks, block size, Hkv, D) and positions and seq_ids are not read.
+    pages (blocks, block size, Hkv, D) and positions and seq_ids are not read. ``dtype``: of the
+    result, where qkv's is that of parts.
     """
-    B, S, _ = qkv.shape
+    B, S, _ = qkv.shape[-3:]
     D = k_cache.shape[3]
     if qkv.is_cuda:
         c = _require_ext("qkv_rope_update")
-        q_out = torch.empty(B, Hq, S, D, dtype=qkv.dtype, device=qkv.device)
+        q_out = torch.empty(B, Hq, S, D, dtype=dtype or qkv.dtype, device=qkv.device)
         if slots is not None:
             slots = seq_ids = positions = slots.to(torch.int32).contiguous()
         elif seq_ids is None:

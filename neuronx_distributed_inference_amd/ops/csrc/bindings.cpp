@@ -103,10 +103,20 @@ int lt_tune(int64_t M, int64_t N, int64_t K, bool has_bias,
             torch::Tensor sx, torch::Tensor sw, torch::Tensor sy,
             c10::optional<torch::Tensor> bias);
 void gelu_tanh_mul_fused(torch::Tensor out, torch::Tensor gate_up);
+void add_norm(torch::Tensor out, torch::Tensor residual, torch::Tensor y, torch::Tensor weight,
+              double eps);
+long tile_gemm_splits(long M, long N, long K, bool glu);
+torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
+                        long splits, bool parts, bool glu);
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("rms_norm", &rms_norm, "RMSNorm (CDNA4)");
     m.def("rms_norm_fused_add", &rms_norm_fused_add, "RMSNorm + residual add (CDNA4)");
+    m.def("add_norm", &add_norm, "residual sum and RMSNorm, of split products too (CDNA4)");
+    m.def("tile_gemm_splits", &tile_gemm_splits, "parts of K of a tiled product, 0: not taken");
+    m.def("tile_gemm", &tile_gemm, "tiled 16-bit product of up to 512 rows (CDNA4)",
+          py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("splits") = 0,
+          py::arg("parts") = false, py::arg("glu") = false);
     m.def("silu_mul", &silu_mul, "SiLU(gate)*up (CDNA4)");
     m.def("gelu_tanh_mul", &gelu_tanh_mul, "GELU-tanh(gate)*up (CDNA4)");
     m.def("rope_apply", &rope_apply, "RoPE rotate-half in place (CDNA4)");

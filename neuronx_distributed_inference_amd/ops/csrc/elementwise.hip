@@ -58,6 +58,74 @@ __global__ void rmsnorm_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// residual += y; out = RMSNorm(residual), with y in 16 bits or as `parts` planes in fp32 (the
+// parts of K of a product, tile_gemm.hip), which are added up on the way. A row's values stay in
+// registers between the sum and the norm: V times 8 a thread. A decode step waits for it twice a
+// layer, so a row of few rows takes as many threads as it has 16-byte pieces and the planes' loads
+// go out together.
+// ---------------------------------------------------------------------------
+template <typename T, bool PARTS, int V>
+__global__ __launch_bounds__(1024) void add_norm_kernel(
+    T* __restrict__ out, T* __restrict__ residual, const void* __restrict__ y,
+    const T* __restrict__ weight, const float eps, const int H, const int parts,
+    const long plane) {
+    __shared__ float red[16];
+    using VT = VecTraits<T>;
+    const long row = blockIdx.x;
+    float f[V][8];
+    float ssq = 0.f;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int i = (v * blockDim.x + threadIdx.x) * 8;
+        if (i >= H) continue;
+        const Vec8<T> r = load_vec8(residual + row * H + i);
+        if constexpr (PARTS) {
+            const float* p = (const float*)y + row * H + i;
+            Vec8<float> a = load_vec8(p);
+            int k = 1;
+            for (; k + 3 <= parts; k += 3) {
+                const Vec8<float> b = load_vec8(p + k * plane), c = load_vec8(p + (k + 1) * plane),
+                                  d = load_vec8(p + (k + 2) * plane);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) a.v[j] += b.v[j] + c.v[j] + d.v[j];
+            }
+            for (; k < parts; ++k) {
+                const Vec8<float> b = load_vec8(p + k * plane);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) a.v[j] += b.v[j];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) f[v][j] = a.v[j];
+        } else {
+            const Vec8<T> a = load_vec8((const T*)y + row * H + i);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) f[v][j] = VT::to_float(a.v[j]);
+        }
+        Vec8<T> o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            f[v][j] += VT::to_float(r.v[j]);
+            ssq += f[v][j] * f[v][j];
+            o.v[j] = VT::from_float(f[v][j]);
+            f[v][j] = VT::to_float(o.v[j]);      // what is normed is the residual as it is kept
+        }
+        store_vec8(residual + row * H + i, o);
+    }
+    ssq = block_reduce_sum(ssq, red);
+    const float inv = rsqrtf(ssq / H + eps);
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const int i = (v * blockDim.x + threadIdx.x) * 8;
+        if (i >= H) continue;
+        const Vec8<T> w = load_vec8(weight + i);
+        Vec8<T> o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o.v[j] = VT::from_float(f[v][j] * inv * VT::to_float(w.v[j]));
+        store_vec8(out + row * H + i, o);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // SiLU(gate) * up and GELU-tanh(gate) * up
 // ---------------------------------------------------------------------------
 template <typename T, bool GELU>
@@ -174,6 +242,50 @@ void rms_norm_fused_add(torch::Tensor out, torch::Tensor x, torch::Tensor residu
             (scalar_t*)residual.data_ptr(), (const scalar_t*)weight.data_ptr(),
             (float)eps, (int)rows, H);
     });
+    HIP_CHECK_KERNEL();
+}
+
+// out = RMSNorm(residual += y): y of residual's shape and type, or (parts, rows, H) in fp32
+void add_norm(torch::Tensor out, torch::Tensor residual, torch::Tensor y, torch::Tensor weight,
+              double eps) {
+    const int H = residual.size(-1);
+    const long rows = H ? residual.numel() / H : 0;
+    const bool planes = y.scalar_type() == at::ScalarType::Float &&
+                        residual.scalar_type() != at::ScalarType::Float;
+    TORCH_CHECK(H % 8 == 0 && H <= 32768, "add_norm: rows of up to 32768, a multiple of 8");
+    TORCH_CHECK(out.is_contiguous() && residual.is_contiguous() && y.is_contiguous() &&
+                weight.is_contiguous() && out.numel() == residual.numel() &&
+                weight.numel() == H && out.scalar_type() == residual.scalar_type() &&
+                weight.scalar_type() == residual.scalar_type(), "add_norm: operands");
+    TORCH_CHECK(planes ? y.dim() == 3 && y.numel() == y.size(0) * rows * H && y.size(0) > 0
+                       : y.scalar_type() == residual.scalar_type() && y.numel() == rows * H,
+                "add_norm: y");
+    TORCH_CHECK((((size_t)out.data_ptr() | (size_t)residual.data_ptr() | (size_t)y.data_ptr() |
+                  (size_t)weight.data_ptr()) & 15) == 0, "add_norm: alignment");
+    if (rows == 0) return;
+    const int parts = planes ? (int)y.size(0) : 1;
+    // many rows: 256 threads each, several rows a CU; few: one value of 16 bytes a thread
+    const int wide = (H / 8 + 63) / 64 * 64;
+    int threads = std::min(wide, rows >= 512 && H <= 8192 ? 256 : 1024);
+    const int V = (H / 8 + threads - 1) / threads;
+    auto stream = at::hip::getCurrentHIPStream();
+#define ADD_NORM(P, VV)                                                                          \
+    hipLaunchKernelGGL((add_norm_kernel<scalar_t, P, VV>), dim3((unsigned)rows), dim3(threads),  \
+                       0, stream, (scalar_t*)out.data_ptr(), (scalar_t*)residual.data_ptr(),     \
+                       y.data_ptr(), (const scalar_t*)weight.data_ptr(), (float)eps, H, parts,   \
+                       rows * H)
+#define ADD_NORM_V(P)                                                                            \
+    do {                                                                                         \
+        if (V == 1) ADD_NORM(P, 1);                                                              \
+        else if (V == 2) ADD_NORM(P, 2);                                                         \
+        else ADD_NORM(P, 4);                                                                     \
+    } while (0)
+    DISPATCH_FLOAT_TYPES(residual.scalar_type(), "add_norm", [&] {
+        if (planes) ADD_NORM_V(true);
+        else ADD_NORM_V(false);
+    });
+#undef ADD_NORM_V
+#undef ADD_NORM
     HIP_CHECK_KERNEL();
 }
 

@@ -83,6 +83,7 @@ __global__ void qkv_rope_update_kernel(
 template <typename T, typename CT, int L>
 __global__ void __launch_bounds__(256)
 qkv_rope_vec_kernel(T* __restrict__ q_out, const T* __restrict__ qkv,
+                    const float* __restrict__ qkv_parts, const int nparts,
                     const float* __restrict__ cosb, const float* __restrict__ sinb,
                     CT* __restrict__ k_cache, CT* __restrict__ v_cache,
                     const int* __restrict__ positions, const int* __restrict__ seq_ids,
@@ -97,13 +98,43 @@ qkv_rope_vec_kernel(T* __restrict__ q_out, const T* __restrict__ qkv,
     if (bs >= rows) return;                      // whole heads: `per` is a multiple of L
     const int in = (int)(item - (long)bs * per), h = in / L, i = (in % L) * 8;
     const int b = bs / S, s = bs - b * S;
-    const T* src = qkv + ((long)bs * Ht + h) * D + i;
-    const Vec8<T> a = load_vec8(src), c = load_vec8(src + half);
+    const long at0 = ((long)bs * Ht + h) * D + i;
     float x1[8], x2[8];
+    if (nparts == 0) {
+        const Vec8<T> a = load_vec8(qkv + at0), c = load_vec8(qkv + at0 + half);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        x1[j] = VT::to_float(a.v[j]);
-        x2[j] = VT::to_float(c.v[j]);
+        for (int j = 0; j < 8; ++j) {
+            x1[j] = VT::to_float(a.v[j]);
+            x2[j] = VT::to_float(c.v[j]);
+        }
+    } else {                                     // the parts of a split product
+        const long plane = (long)rows * Ht * D;
+        const float* p = qkv_parts + at0;
+        Vec8<float> a = load_vec8(p), c = load_vec8(p + half);
+        int k = 1;
+        for (; k + 2 <= nparts; k += 2) {
+            const Vec8<float> a1 = load_vec8(p + k * plane), c1 = load_vec8(p + k * plane + half);
+            const Vec8<float> a2 = load_vec8(p + (k + 1) * plane),
+                              c2 = load_vec8(p + (k + 1) * plane + half);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                a.v[j] += a1.v[j] + a2.v[j];
+                c.v[j] += c1.v[j] + c2.v[j];
+            }
+        }
+        if (k < nparts) {
+            const Vec8<float> a1 = load_vec8(p + k * plane), c1 = load_vec8(p + k * plane + half);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                a.v[j] += a1.v[j];
+                c.v[j] += c1.v[j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            x1[j] = a.v[j];
+            x2[j] = c.v[j];
+        }
     }
     if (h < Hq + Hkv) {
         const T* w = h < Hq ? qw : kw;
@@ -218,11 +249,17 @@ void qkv_rope_update(torch::Tensor q_out, torch::Tensor qkv,
                      long Hq, long Hkv, c10::optional<torch::Tensor> q_norm,
                      c10::optional<torch::Tensor> k_norm, double eps,
                      c10::optional<torch::Tensor> slots) {
-    const int B = qkv.size(0), S = qkv.size(1);
+    // qkv: (B, S, width), or its parts in fp32, (parts, B, S, width) beside a q_out of 16 bits
+    const int nparts = qkv.dim() == 4 ? (int)qkv.size(0) : 0;
+    const int B = q_out.size(0), S = q_out.size(2);
     const int D = k_cache.size(3);
     const int Bc = k_cache.size(0), Smax = k_cache.size(2);
-    TORCH_CHECK(qkv.size(2) == (Hq + 2 * Hkv) * D, "qkv width mismatch");
+    TORCH_CHECK(qkv.size(-1) == (Hq + 2 * Hkv) * D &&
+                qkv.numel() == (long)std::max(nparts, 1) * B * S * qkv.size(-1),
+                "qkv width mismatch");
     TORCH_CHECK(qkv.is_contiguous(), "qkv must be contiguous");
+    TORCH_CHECK(qkv.scalar_type() == (nparts ? at::ScalarType::Float : q_out.scalar_type()),
+                "qkv: type");
     const int ht_half = (int)(Hq + 2 * Hkv) * (D / 2);
     dim3 blocks((unsigned)(B * S), (unsigned)((ht_half + 255) / 256));
     auto stream = at::hip::getCurrentHIPStream();
@@ -233,14 +270,14 @@ void qkv_rope_update(torch::Tensor q_out, torch::Tensor qkv,
                         (q_norm ? (size_t)q_norm->data_ptr() : 0) |
                         (k_norm ? (size_t)k_norm->data_ptr() : 0);
     const bool vec = (D == 32 || D == 64 || D == 128 || D == 256) && bits % 16 == 0 && D <= cosb.size(-1);
-    TORCH_CHECK(vec || (!q_norm && !k_norm && !slots),
-                "qkv_rope_update: norms and pages need head sizes 32, 64, 128 or 256");
-    TORCH_CHECK(fp8 || k_cache.scalar_type() == qkv.scalar_type(), "cache/new dtype mismatch");
+    TORCH_CHECK(vec || (!q_norm && !k_norm && !slots && !nparts),
+                "qkv_rope_update: norms, pages and parts need head sizes 32, 64, 128 or 256");
+    TORCH_CHECK(fp8 || k_cache.scalar_type() == q_out.scalar_type(), "cache/new dtype mismatch");
     if (vec) {
         for (const auto* w : {&q_norm, &k_norm})
             if (w->has_value())
                 TORCH_CHECK((*w)->numel() == D && (*w)->is_contiguous() &&
-                            (*w)->scalar_type() == qkv.scalar_type(), "qkv_rope_update: norm");
+                            (*w)->scalar_type() == q_out.scalar_type(), "qkv_rope_update: norm");
         if (slots)
             TORCH_CHECK(slots->scalar_type() == at::ScalarType::Int && slots->is_contiguous() &&
                         slots->numel() == (long)B * S && k_cache.size(2) == Hkv, "slots");
@@ -250,7 +287,8 @@ void qkv_rope_update(torch::Tensor q_out, torch::Tensor qkv,
         const long smax = slots ? k_cache.size(0) * k_cache.size(1) : Smax;
 #define QKV_VEC(CT, LL)                                                                            \
     hipLaunchKernelGGL((qkv_rope_vec_kernel<scalar_t, CT, LL>), dim3((unsigned)nb), dim3(256), 0,  \
-        stream, (scalar_t*)q_out.data_ptr(), (const scalar_t*)qkv.data_ptr(),                      \
+        stream, (scalar_t*)q_out.data_ptr(), (const scalar_t*)(nparts ? nullptr : qkv.data_ptr()), \
+        nparts ? qkv.data_ptr<float>() : nullptr, nparts,                                          \
         cosb.data_ptr<float>(), sinb.data_ptr<float>(), (CT*)k_cache.data_ptr(),                   \
         (CT*)v_cache.data_ptr(), slots ? nullptr : positions.data_ptr<int>(),                      \
         slots ? nullptr : seq_ids.data_ptr<int>(), slots ? slots->data_ptr<int>() : nullptr,       \
@@ -262,7 +300,7 @@ void qkv_rope_update(torch::Tensor q_out, torch::Tensor qkv,
         if (D == 32) { QKV_VEC(CT, 2); } else if (D == 64) { QKV_VEC(CT, 4); }                     \
         else if (D == 128) { QKV_VEC(CT, 8); } else { QKV_VEC(CT, 16); }                           \
     } while (0)
-        DISPATCH_FT(qkv.scalar_type(), "qkv_rope_update", [&] {
+        DISPATCH_FT(q_out.scalar_type(), "qkv_rope_update", [&] {
             if (fp8) {
                 QKV_VEC_D(__hip_fp8_e4m3);
             } else {

@@ -1,0 +1,391 @@
+// y (M, N) = x (M, K) @ w (N, K)^T in 16 bits, up to 512 rows: the products of decoding and of short
+// prompts, bound by the weights' bytes, which come once, straight to LDS.
+//
+// A workgroup holds a ring of D chunks (64 of K, 128 bytes a row) of its tiles of x and w, filled
+// by global_load_lds and waited for by count, with one barrier a chunk. What fills the memory
+// pipes is the bytes on the way: 64 to 128 KB a CU. K is split so that all 256 CUs have a tile;
+// the parts stay in fp32 and the kernel that follows (residual sum and norm, rope) adds them up,
+// so that a split costs no launch. With GLU a wave has the gate and the up rows of its columns and
+// writes silu(gate) * up, which saves a launch and both in 16 bits.
+
+#include "common.h"
+#include <torch/extension.h>
+#include <ATen/hip/HIPContext.h>
+
+namespace {
+
+typedef __bf16 tg_bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 tg_f16x8 __attribute__((ext_vector_type(8)));
+typedef float tg_f32x4 __attribute__((ext_vector_type(4)));
+
+template <typename T> struct TgMfma;
+template <> struct TgMfma<__hip_bfloat16> {
+    using vec8 = tg_bf16x8;
+    static DEV_INLINE tg_f32x4 mfma(vec8 a, vec8 b, tg_f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    }
+};
+template <> struct TgMfma<__half> {
+    using vec8 = tg_f16x8;
+    static DEV_INLINE tg_f32x4 mfma(vec8 a, vec8 b, tg_f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+    }
+};
+
+template <int N> DEV_INLINE void tg_wait() {
+    asm volatile("s_waitcnt vmcnt(%c0)" ::"i"(N) : "memory");
+}
+
+// wait until at most `left` chunks of G loads are in flight
+template <int G, int MAX> DEV_INLINE void tg_wait_chunks(int left) {
+    if constexpr (MAX == 0) {
+        tg_wait<0>();
+    } else {
+        if (left >= MAX) tg_wait<G * MAX>();
+        else tg_wait_chunks<G, MAX - 1>(left);
+    }
+}
+
+template <int AUX> DEV_INLINE void tg_load(const char* src, char* dst) {
+    __builtin_amdgcn_global_load_lds(
+        (const __attribute__((address_space(1))) unsigned int*)src,
+        (__attribute__((address_space(3))) unsigned int*)dst, 16, 0, AUX);
+}
+
+constexpr int TG_BK = 64;    // K of a chunk: 128 bytes a row
+
+struct TgArgs {
+    void* y;             // (M, N), or (M, N / 2) with GLU
+    float* part;         // (splits, M, N) fp32 when splits > 1
+    const void* x;       // (M, K)
+    const void* w;       // (N, K)
+    const void* bias;    // (N,) or null
+    int M, N, K, splits, mblocks, ntiles, per_xcd, work;
+};
+
+// A workgroup of WM x WN waves makes BM x BN outputs (of one of `splits` parts of K), a wave
+// BM/WM x BN/WN of them. D chunks of x and w are in LDS or on the way there.
+template <typename T, int BM, int BN, int WM, int WN, int D, bool GLU, bool ONCE>
+__global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a) {
+    using MF = TgMfma<T>;
+    using vec8 = typename MF::vec8;
+    constexpr int NW = WM * WN;
+    constexpr int FM = BM / WM / 16, FN = BN / WN / 16;
+    constexpr int XPT = BM / 8, WPT = BN / 8;          // pieces of 8 rows, 1 KB, a wave's load
+    constexpr int XP = XPT >= NW ? XPT / NW : 1, WP = WPT / NW;
+    static_assert(WPT % NW == 0 && (XPT % NW == 0 || XPT < NW), "pieces");
+    static_assert(!GLU || FN % 2 == 0, "gate and up of a column in one wave");
+    constexpr int G = XP + WP;                         // loads of a wave and chunk
+    constexpr int CHUNK = (BM + BN) * 128;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+
+    // workgroups go round the XCDs: each gets one run of the work, row blocks of a tile of w
+    // next to each other
+    const int item = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
+    if (item >= a.work) return;
+    const int mb = item % a.mblocks;
+    const int rest = item / a.mblocks;
+    const int nt = rest % a.ntiles, slice = rest / a.ntiles;
+    const int m0 = mb * BM;
+    const int chunks = a.K / TG_BK;
+    const int c_lo = (int)((long)slice * chunks / a.splits);
+    const int n = (int)((long)(slice + 1) * chunks / a.splits) - c_lo;    // >= 1: splits <= chunks
+
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int wm = wid / WN, wn = wid % WN;
+    const int lrow = lane & 15, lslot = lane >> 4;
+
+    // where the lane's 16 bytes of each piece come from; LDS rows hold 16-byte slots in the order
+    // slot ^ (row & 7), so that 8 rows of one slot lie in different banks. Rows past the end
+    // repeat the last one.
+    const int prow = lane >> 3;
+    const unsigned kbytes = (unsigned)a.K * sizeof(T);
+    unsigned xo[XP], wo[WP];
+#pragma unroll
+    for (int i = 0; i < XP; ++i) {
+        const int r = (wid * XP + i) % XPT * 8 + prow;
+        xo[i] = (unsigned)min(r, a.M - 1 - m0) * kbytes + ((lane & 7) ^ (r & 7)) * 16;
+    }
+#pragma unroll
+    for (int i = 0; i < WP; ++i) {
+        const int r = (wid * WP + i) * 8 + prow;
+        unsigned row;
+        if constexpr (GLU) {
+            // of a wave's rows half are gate and half are up, of the same columns
+            constexpr int PW = BN / WN;
+            const int in = r % PW;
+            row = min(r / PW * (PW / 2) + in % (PW / 2), a.N / 2 - 1 - nt * (BN / 2)) +
+                  (in >= PW / 2 ? a.N / 2 : 0);
+        } else {
+            row = min(r, a.N - 1 - nt * BN);
+        }
+        wo[i] = row * kbytes + ((lane & 7) ^ (r & 7)) * 16;
+    }
+    const char* x0 = (const char*)a.x + (long)m0 * kbytes + (long)c_lo * 128;
+    const char* w0 = (const char*)a.w + (long)nt * (GLU ? BN / 2 : BN) * kbytes + (long)c_lo * 128;
+    // tiles start at different chunks and wrap round: in step they would all ask for the same
+    // 128 bytes of rows a power of two apart, which few of the memory channels hold
+    int at = ((blockIdx.x >> 3) / a.mblocks) % n;
+    auto stage = [&](int buf) {
+        char* base = smem + buf * CHUNK;
+        const char* wp = w0 + (long)at * 128;
+        const char* xp = x0 + (long)at * 128;
+#pragma unroll
+        for (int i = 0; i < WP; ++i)
+            tg_load<ONCE ? 2 : 0>(wp + wo[i], base + BM * 128 + (wid * WP + i) * 1024);
+#pragma unroll
+        for (int i = 0; i < XP; ++i)
+            tg_load<0>(xp + xo[i], base + ((wid * XP + i) % XPT) * 1024);
+        at = at + 1 == n ? 0 : at + 1;
+    };
+
+    tg_f32x4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = {0.f, 0.f, 0.f, 0.f};
+
+    int off[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        off[h] = lrow * 128 + (((h * 4 + lslot) ^ (lrow & 7)) << 4);
+    const int xoff = wm * (BM / WM) * 128, woff = BM * 128 + wn * (BN / WN) * 128;
+    vec8 xa[2][FM], wb[2][FN];
+    auto read = [&](int buf, int h) {
+        const char* base = smem + buf * CHUNK + off[h];
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+            wb[h][j] = *reinterpret_cast<const vec8*>(base + woff + j * 2048);
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+            xa[h][i] = *reinterpret_cast<const vec8*>(base + xoff + i * 2048);
+    };
+    auto mma = [&](int h) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = MF::mfma(wb[h][j], xa[h][i], acc[i][j]);
+    };
+
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+        if (i < n) stage(i);
+    tg_wait_chunks<G, D - 1>(min(D, n) - 1);
+    __builtin_amdgcn_s_barrier();
+    read(0, 0);
+    int buf = 0, t = 0;
+    // The second half of a chunk is read before the products of the first, and the first half of
+    // the next chunk before those of the second. Between them every wave has read the chunk, which
+    // its successor D chunks on then overwrites, and has its loads of the next one.
+    for (; t < n - D; ++t) {
+        const int next = buf == D - 1 ? 0 : buf + 1;
+        read(buf, 1);
+        mma(0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        tg_wait<G * (D - 2)>();
+        __builtin_amdgcn_s_barrier();
+        read(next, 0);
+        stage(buf);
+        mma(1);
+        buf = next;
+    }
+    for (; t < n; ++t) {
+        const int next = buf == D - 1 ? 0 : buf + 1;
+        read(buf, 1);
+        mma(0);
+        if (t + 1 < n) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            tg_wait_chunks<G, D - 1>(n - t - 2);
+            __builtin_amdgcn_s_barrier();
+            read(next, 0);
+        }
+        mma(1);
+        buf = next;
+    }
+
+    // w's rows stand in the products' rows: register r of acc[i][j] is column j * 16 +
+    // lane / 16 * 4 + r of row i * 16 + lane % 16
+    constexpr int FC = GLU ? FN / 2 : FN, CW = GLU ? BN / 2 : BN;
+    const int cols = GLU ? a.N / 2 : a.N;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+        const int m = m0 + wm * (BM / WM) + i * 16 + lrow;
+        if (m >= a.M) continue;
+#pragma unroll
+        for (int j = 0; j < FC; ++j) {
+            const int c = nt * CW + wn * (CW / WN) + j * 16 + lslot * 4;
+            if (c >= cols) continue;
+            tg_f32x4 v = acc[i][j];
+            if constexpr (GLU) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = v[r] / (1.f + __expf(-v[r])) * acc[i][j + FC][r];
+            } else if (a.splits > 1) {
+                *reinterpret_cast<tg_f32x4*>(a.part + ((long)slice * a.M + m) * a.N + c) = v;
+                continue;
+            } else if (a.bias) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] += VecTraits<T>::to_float(((const T*)a.bias)[c + r]);
+            }
+            __align__(8) T o[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r] = VecTraits<T>::from_float(v[r]);
+            *reinterpret_cast<int2*>((T*)a.y + (long)m * cols + c) = *reinterpret_cast<int2*>(o);
+        }
+    }
+}
+
+// y = sum of the parts (+ bias)
+template <typename T>
+__global__ __launch_bounds__(256) void tile_sum_kernel(T* __restrict__ y,
+                                                       const float* __restrict__ part,
+                                                       const T* __restrict__ bias, const long MN,
+                                                       const int N, const int splits) {
+    const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= MN) return;
+    tg_f32x4 s = *reinterpret_cast<const tg_f32x4*>(part + i);
+    for (int k = 1; k < splits; ++k) s += *reinterpret_cast<const tg_f32x4*>(part + k * MN + i);
+    __align__(8) T o[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (bias) s[r] += VecTraits<T>::to_float(bias[i % N + r]);
+        o[r] = VecTraits<T>::from_float(s[r]);
+    }
+    *reinterpret_cast<int2*>(y + i) = *reinterpret_cast<int2*>(o);
+}
+
+// The tile of a shape. A chunk of w (BN rows of 128 bytes) is what a workgroup streams, x comes
+// again and again from the L2: few rows take small tiles with a deep ring, so that a CU has 64 KB
+// and more on the way; many rows take tall ones, for fewer reads of x and w from LDS a product.
+enum TgTile { T16, T16N, T32, T32N, T64, T64N, T128, T128N, T128W, T128B, T256W };
+
+struct TgPlan {
+    TgTile tile;
+    int bm, bn, splits;
+};
+
+// What is not taken (splits == 0) goes to the library. Times of 16-bit products on weights that
+// are not in a cache, 32-bit parts left to the next kernel, here / library (or the kernels with a
+// ring of 3 chunks that were here before):
+//   rows   (6144, 4096)  (4096, 4096)  (28672, 4096)  (4096, 14336)  (57344, 8192)
+//   1       10.7 / 13.6    7.7 / 10.3    40.7 /  49.9   20.9 / 27.4   150 / 160
+//   16      11.0 / 16.2    8.1 / 13.2    39.9 /  51.7   20.7 / 26.8   151 / 164
+//   64      12.9 / 19.7   10.0 / 15.5    43.6 /  54.3   23.4 / 32.4   166 / 184
+//   128     17.8 / 21.4   14.0 / 18.9    49.0 /  60.4   30.5 / 43.2   157 / 221
+//   256     24.2 / 27.2   17.8 / 25.2    70.8 /  84.1   40.5 / 53.4   268 / 239
+//   512     34.9 / 38.2   25.5 / 29.7     123 /   105   62.1 / 89.2   442 / 375
+// so up to 256 rows, unless the tiles of more than 128 rows need a second round of the chip, and
+// up to 512 rows where the tiles of the outputs alone leave CUs idle. Parts of K fill the 256 CUs
+// once, each with 2 chunks or more.
+TgPlan tg_plan(long M, long N, long K, bool glu) {
+    TgPlan p{T16, 16, 128, 0};
+    if (M < 1 || M > 512 || N < 64 || N % (glu ? 8 : 4) || K < 256 || K % TG_BK ||
+        K * N * 2 >= (1L << 32))
+        return p;
+    // half the width where that many more tiles spare parts of K, or with GLU fill the chip
+    const bool narrow = glu ? N < 25600 : N <= 4096;
+    if (M <= 16) p = narrow ? TgPlan{T16N, 16, 64, 0} : TgPlan{T16, 16, 128, 0};
+    else if (M <= 32) p = narrow ? TgPlan{T32N, 32, 64, 0} : TgPlan{T32, 32, 128, 0};
+    else if (M <= 64) p = narrow ? TgPlan{T64N, 64, 64, 0} : TgPlan{T64, 64, 128, 0};
+    else if (M <= 128 && narrow && glu) p = {T128N, 128, 64, 0};
+    else if (M <= 128 && N * K < (60 << 20)) p = {T128, 128, 128, 0};
+    else if (M <= 128) p = {T128W, 128, 256, 0};
+    else if (N * K <= (20 << 20)) p = {T128B, 128, 128, 0};
+    else p = {T256W, 128, 256, 0};
+    const long tiles = (M + p.bm - 1) / p.bm * ((N + p.bn - 1) / p.bn);
+    if (M > 128 && tiles > 256) return p;
+    if (M > 256 && (tiles > 128 || glu)) return p;
+    p.splits = glu ? 1 : (int)std::max(1L, std::min({256 / tiles, K / 128, 16L}));
+    return p;
+}
+
+template <typename T, int BM, int BN, int WM, int WN, int D, bool GLU, bool ONCE>
+void tg_go(TgArgs& a, hipStream_t stream) {
+    a.mblocks = (a.M + BM - 1) / BM;
+    a.ntiles = (a.N + BN - 1) / BN;
+    a.work = a.mblocks * a.ntiles * a.splits;
+    a.per_xcd = (a.work + 7) / 8;
+    constexpr int LDS = D * (BM + BN) * 128;
+    auto* k = tile_gemm_kernel<T, BM, BN, WM, WN, D, GLU, ONCE>;
+    TORCH_CHECK(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    LDS) == hipSuccess, "tile_gemm: LDS");
+    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(64 * WM * WN), LDS, stream, a);
+    HIP_CHECK_KERNEL();
+}
+
+template <typename T, bool GLU>
+void tg_tile(TgArgs& a, TgTile tile, hipStream_t s) {
+    switch (tile) {
+        case T16: tg_go<T, 16, 128, 1, 4, 4, GLU, true>(a, s); break;
+        case T16N: tg_go<T, 16, 64, 1, 2, 8, GLU, true>(a, s); break;
+        case T32: tg_go<T, 32, 128, 1, 4, 4, GLU, true>(a, s); break;
+        case T32N: tg_go<T, 32, 64, 1, 2, 6, GLU, true>(a, s); break;
+        case T64: tg_go<T, 64, 128, 1, 4, 3, GLU, true>(a, s); break;
+        case T64N: tg_go<T, 64, 64, 2, 2, 5, GLU, true>(a, s); break;
+        case T128: tg_go<T, 128, 128, 2, 4, 5, GLU, true>(a, s); break;
+        case T128N: tg_go<T, 128, 64, 4, 2, 6, GLU, true>(a, s); break;
+        case T128W: tg_go<T, 128, 256, 2, 4, 3, GLU, true>(a, s); break;
+        case T128B: tg_go<T, 128, 128, 2, 4, 5, GLU, false>(a, s); break;
+        case T256W: tg_go<T, 128, 256, 2, 4, 3, GLU, false>(a, s); break;
+    }
+}
+
+}  // namespace
+
+// Parts of K that tile_gemm takes for this shape, 0: none, it is the library's.
+long tile_gemm_splits(long M, long N, long K, bool glu) { return tg_plan(M, N, K, glu).splits; }
+
+// x (M, K) @ w (N, K)^T. `splits` 0: as planned, which leaves (splits, M, N) parts in fp32 where
+// there are several (`parts`) or sums them up. `glu`: silu of the first half of the columns times
+// the second.
+torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
+                        long splits, bool parts, bool glu) {
+    TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "tile_gemm: shapes");
+    TORCH_CHECK(x.is_contiguous() && w.is_contiguous() && x.scalar_type() == w.scalar_type(),
+                "tile_gemm: contiguous operands of one type");
+    TORCH_CHECK(((size_t)x.data_ptr() | (size_t)w.data_ptr()) % 16 == 0, "tile_gemm: alignment");
+    const bool bf = x.scalar_type() == at::ScalarType::BFloat16;
+    TORCH_CHECK(bf || x.scalar_type() == at::ScalarType::Half, "tile_gemm: bf16/f16 only");
+    TgArgs a{};
+    a.M = x.size(0);
+    a.K = x.size(1);
+    a.N = w.size(0);
+    const TgPlan plan = tg_plan(a.M, a.N, a.K, glu);
+    TORCH_CHECK(plan.splits > 0, "tile_gemm: shape not taken");
+    TORCH_CHECK(splits >= 0 && splits <= a.K / TG_BK && !(glu && splits > 1), "tile_gemm: splits");
+    a.splits = splits ? splits : plan.splits;
+    TORCH_CHECK(!bias || (!parts && !glu && bias->is_contiguous() && bias->numel() == a.N &&
+                          bias->scalar_type() == x.scalar_type()), "tile_gemm: bias");
+    torch::Tensor y, part;
+    if (a.splits > 1) {
+        part = torch::empty({a.splits, a.M, a.N}, x.options().dtype(torch::kFloat32));
+        a.part = part.data_ptr<float>();
+    }
+    if (a.splits == 1 || !parts) {
+        y = torch::empty({a.M, glu ? a.N / 2 : a.N}, x.options());
+        a.y = y.data_ptr();
+    }
+    a.x = x.data_ptr();
+    a.w = w.data_ptr();
+    a.bias = bias ? bias->data_ptr() : nullptr;
+    auto stream = at::hip::getCurrentHIPStream();
+    if (bf) {
+        if (glu) tg_tile<__hip_bfloat16, true>(a, plan.tile, stream);
+        else tg_tile<__hip_bfloat16, false>(a, plan.tile, stream);
+    } else {
+        if (glu) tg_tile<__half, true>(a, plan.tile, stream);
+        else tg_tile<__half, false>(a, plan.tile, stream);
+    }
+    if (a.splits == 1) return y;
+    if (parts) return part;
+    const long MN = (long)a.M * a.N;
+    const dim3 grid((unsigned)((MN / 4 + 255) / 256));
+    if (bf)
+        hipLaunchKernelGGL((tile_sum_kernel<__hip_bfloat16>), grid, dim3(256), 0, stream,
+                           (__hip_bfloat16*)a.y, a.part, (const __hip_bfloat16*)a.bias, MN, a.N,
+                           a.splits);
+    else
+        hipLaunchKernelGGL((tile_sum_kernel<__half>), grid, dim3(256), 0, stream, (__half*)a.y,
+                           a.part, (const __half*)a.bias, MN, a.N, a.splits);
+    HIP_CHECK_KERNEL();
+    return y;
+}

@@ -216,11 +216,23 @@ def _linear(x: torch.Tensor, weight: torch.Tensor,
 
         if _ops.lt_linear_enabled():
             # decode-size batches route through the shape-autotuned
-            # skinny_gemm5-vs-hipBLASLt dispatcher (ops.decode_linear)
-            if x.numel() // x.shape[-1] <= 256:
+            # tiled-kernel-vs-hipBLASLt dispatcher (ops.decode_linear)
+            if x.numel() // x.shape[-1] <= 512:
                 return _ops.decode_linear(x, weight, bias)
             return _ops.lt_linear(x, weight, bias)
     return F.linear(x, weight, bias)
+
+
+def plain_linear(mod: nn.Module, x: torch.Tensor) -> bool:
+    """Whether calling the module on x is no more than x @ weight^T in 16 bits on the GPU, so that
+    a fused kernel may stand for it: no bias, 8-bit weight, tensor parallelism, hook or subclass."""
+    return (type(mod) in (ColumnParallelLinear, RowParallelLinear)
+            and mod.tp_degree == 1 and mod._group is None
+            and ps.get_tensor_model_parallel_size() == 1
+            and mod.bias is None and not getattr(mod, "fp8", False)
+            and not (mod._forward_hooks or mod._forward_pre_hooks)
+            and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16)
+            and mod.weight.dtype == x.dtype)
 
 
 class ColumnParallelLinear(nn.Module):

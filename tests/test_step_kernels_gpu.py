@@ -1,0 +1,187 @@
+"""GPU tests of the kernels that a model step is made of beside attention: tiled products whose
+parts of K the next kernel adds up, residual sum and norm, and the layers that run on them."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from neuronx_distributed_inference_amd import ops
+
+F64 = torch.float64
+EPS16 = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+def _product(M, N, K, dtype, seed=0):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    x = torch.randn(M, K, device="cuda", generator=g).to(dtype)
+    w = (torch.randn(N, K, device="cuda", generator=g) * 0.05).to(dtype)
+    exact = x.to(F64) @ w.to(F64).t()
+    # K sums in 32 bits: at most K roundings of 2^-24 of the largest partial sum
+    sums = K * 2.0 ** -24 * (x.to(F64).abs() @ w.to(F64).abs().t())
+    return x, w, exact, sums
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 64, 256), (1, 4100, 320), (2, 2048, 2048), (16, 6144, 512), (17, 4352, 256),
+    (32, 100, 1088), (33, 11408, 256), (48, 4092, 4096), (64, 4100, 576), (65, 132, 2048),
+    (93, 3072, 2048), (128, 4096, 256), (127, 16384, 4096), (129, 68, 320), (200, 4096, 4096),
+    (256, 6144, 4096), (257, 2048, 2048), (300, 4096, 512), (512, 4096, 256)])
+def test_tile_gemm(M, N, K, dtype):
+    x, w, exact, sums = _product(M, N, K, dtype)
+    plan = ops._tile_takes(x, w)
+    assert plan >= 1
+    for splits in {1, 2, plan, K // 64}:
+        parts = ops._C.tile_gemm(x, w, None, splits, True)
+        assert parts.dim() == (3 if splits > 1 else 2)
+        if splits > 1:
+            got, limit = parts.to(F64).sum(0), sums
+        else:
+            got, limit = parts.to(F64), sums + EPS16[dtype] * exact.abs()
+        assert ((got - exact).abs() <= limit + 1e-30).all()
+        bias = torch.linspace(-1, 1, N, device="cuda").to(dtype)
+        y = ops._C.tile_gemm(x, w, bias, splits)
+        want = exact + bias.to(F64)
+        assert y.dtype == dtype
+        assert ((y.to(F64) - want).abs() <= 2 * sums + EPS16[dtype] * want.abs() + 1e-7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 256), (7, 28672, 512), (16, 1000, 320), (32, 16384, 256),
+                                   (40, 72, 256), (64, 25608, 256), (65, 16384, 256),
+                                   (128, 28672, 256), (200, 2056, 2048), (256, 28672, 1024)])
+def test_tile_gemm_glu(M, N, K, dtype):
+    x, w, exact, sums = _product(M, N, K, dtype)
+    y = ops._C.tile_gemm(x, w, glu=True)
+    g, u = exact[:, : N // 2], exact[:, N // 2:]
+    want = torch.nn.functional.silu(g) * u
+    # the slope of silu stays below 1.1; its exp and division are good to 2^-20
+    limit = 1.1 * sums[:, : N // 2] * u.abs() + g.abs() * sums[:, N // 2:] \
+        + (EPS16[dtype] + 2.0 ** -20) * want.abs() + 1e-7
+    assert ((y.to(F64) - want).abs() <= limit).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 192), (1, 60, 256), (8, 66, 256), (8, 64, 260),
+                                   (513, 4096, 4096), (512, 28672, 4096), (129, 57344, 8192)])
+def test_tile_gemm_leaves_to_the_library(M, N, K):
+    assert ops._C.tile_gemm_splits(M, N, K, False) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,H,parts", [(1, 8, 0), (1, 2048, 1), (3, 4096, 8), (64, 8192, 5),
+                                          (5, 520, 4), (2, 32768, 2), (600, 4096, 0),
+                                          (513, 16384, 3), (700, 8192, 2)])
+def test_add_norm(rows, H, parts, dtype):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows + H)
+    shape = (parts, rows, H) if parts else (rows, H)
+    y = torch.randn(shape, device="cuda", generator=g)
+    y = y if parts else y.to(dtype)
+    res = torch.randn(rows, H, device="cuda", generator=g).to(dtype)
+    w = torch.randn(H, device="cuda", generator=g).to(dtype)
+    total = res.to(F64) + (y.to(F64).sum(0) if parts else y.to(F64))
+    out = ops.add_norm(y, res, w, 1e-5)
+    # the residual as it is kept, under the root mean square of the sum
+    want = res.to(F64) * torch.rsqrt(total.square().mean(-1, keepdim=True) + 1e-5) * w.to(F64)
+    # one rounding of each result, some of 2^-24 before it
+    assert ((res.to(F64) - total).abs() <= EPS16[dtype] * total.abs() + 1e-5).all()
+    assert ((out.to(F64) - want).abs() <= (EPS16[dtype] + 2.0 ** -16) * want.abs() + 1e-4).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("parts", [1, 2, 3, 8])
+@pytest.mark.parametrize("normed", [False, True])
+def test_qkv_rope_update_adds_parts(parts, normed, dtype):
+    B, S, Hq, Hkv, D = 3, 2, 8, 2, 64
+    g = torch.Generator(device="cuda")
+    g.manual_seed(parts)
+    y = torch.randn(parts, B, S, (Hq + 2 * Hkv) * D, device="cuda", generator=g)
+    ang = torch.randn(B, S, D // 2, device="cuda", generator=g).repeat(1, 1, 2)
+    pos = torch.randint(0, 16, (B, S), device="cuda", generator=g, dtype=torch.int32)
+    pos[:, 1] = pos[:, 0] + 1
+    ids = torch.arange(B, device="cuda", dtype=torch.int32)
+    norms = None
+    if normed:
+        norms = tuple(torch.randn(D, device="cuda", generator=g).to(dtype) for _ in range(2)) + (1e-6,)
+    caches = [torch.zeros(B, Hkv, 20, D, device="cuda", dtype=dtype) for _ in range(2)]
+    q = ops.qkv_rope_update(y, ang.cos(), ang.sin(), *caches, pos, ids, Hq, Hkv, norms=norms,
+                            dtype=dtype)
+    wide = [torch.zeros(B, Hkv, 20, D, dtype=F64) for _ in range(2)]
+    want = ops.qkv_rope_update(y.to(F64).sum(0).cpu(), ang.to(F64).cos().cpu(),
+                               ang.to(F64).sin().cpu(), *wide, pos.cpu(), ids.cpu(), Hq, Hkv,
+                               norms=norms and tuple(t.cpu().to(F64) for t in norms[:2]) + (1e-6,))
+    for a, b in zip([q] + caches, [want] + wide):
+        # rope adds two products: a rounding each of the parts' sums and the angles in 32 bits
+        assert ((a.cpu().to(F64) - b).abs() <= EPS16[dtype] * b.abs() + 1e-4).all()
+
+
+def _small_llama(dtype, layers=2, moe=False, **kw):
+    from neuronx_distributed_inference_amd.config import EngineConfig
+    from neuronx_distributed_inference_amd.models.llama.modeling_llama import (
+        LlamaForCausalLM, LlamaInferenceConfig)
+    from neuronx_distributed_inference_amd.models.mixtral.modeling_mixtral import (
+        MixtralForCausalLM, MixtralInferenceConfig)
+
+    ec = EngineConfig(batch_size=2, max_batch_size=2, seq_len=160, max_length=160,
+                      torch_dtype=dtype, tp_degree=1, output_logits=True, fused_qkv=True,
+                      fused_gate_up=True, enable_batch_bucketing=False, **kw)
+    sizes = dict(neuron_config=ec, hidden_size=512, intermediate_size=1024,
+                 num_hidden_layers=layers, num_attention_heads=8, num_key_value_heads=2,
+                 head_dim=64, vocab_size=512, max_position_embeddings=320, rms_norm_eps=1e-5,
+                 rope_theta=10000.0, hidden_act="silu", tie_word_embeddings=False)
+    if moe:
+        sizes.update(num_local_experts=4, num_experts_per_tok=4)   # no choice that rounding flips
+    with torch.device("cuda"):
+        lm = (MixtralForCausalLM(MixtralInferenceConfig(**sizes)) if moe else
+              LlamaForCausalLM(LlamaInferenceConfig(**sizes))).eval()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(0)
+    for name, p in lm.model.named_parameters():
+        if "norm" in name:
+            p.data.uniform_(0.5, 1.5, generator=g)
+        else:
+            p.data.normal_(0, 0.05, generator=g)
+    return lm
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("moe", [False, True])
+@pytest.mark.parametrize("hook", ["layer", "norm", "o_proj", "down", "final", "global"])
+def test_fused_layers_and_layers_with_hooks(hook, moe, dtype):
+    """A hook sees its module's tensors, from the chain of modules; without one the fused layers
+    give the same logits and cache."""
+    if moe and hook == "down":
+        pytest.skip("no down projection")
+    lm = _small_llama(dtype, moe=moe)
+    ids = torch.randint(0, 512, (2, 70), device="cuda")
+    step = torch.randint(0, 512, (2, 1), device="cuda")
+
+    def run():
+        lm.reset()
+        with torch.inference_mode():
+            a = lm(input_ids=ids).logits
+            b = lm(input_ids=step, position_ids=torch.full((2, 1), 70, device="cuda")).logits
+        return a.float(), b.float(), lm.model.kv_mgr.get_cache(1)[0].data.float().clone()
+
+    fused = run()
+    layer = lm.model.layers[1]
+    seen = []
+    note = lambda *a: seen.append(1)  # noqa: E731
+    if hook == "global":
+        h = torch.nn.modules.module.register_module_forward_hook(note)
+    else:
+        mod = {"layer": layer, "norm": layer.post_attention_layernorm,
+               "o_proj": layer.self_attn.o_proj, "final": lm.model.norm,
+               "down": getattr(layer.mlp, "down_proj", None)}[hook]
+        h = mod.register_forward_hook(note)
+    try:
+        plain = run()
+    finally:
+        h.remove()
+    assert len(seen) >= 2
+    # 16-bit activations of two layers, rounded at other places
+    tol = 0.03 if dtype == "bfloat16" else 0.004
+    for a, b in zip(fused, plain):
+        assert (a - b).norm() <= tol * b.norm()
