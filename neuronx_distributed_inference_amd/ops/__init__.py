@@ -12,6 +12,8 @@ always use the reference path.
 
 from __future__ import annotations
 
+import functools
+import math
 import os
 from typing import Optional, Tuple
 
@@ -935,6 +937,30 @@ def row_topk(x: torch.Tensor, k: int):
 MOE_WORKSPACE = 1 << 30
 
 
+@functools.lru_cache(maxsize=1024)
+def _moe_tile_rows(n: int, experts: int, local: int, H: int, I: int, f8: bool) -> int:
+    """Rows of a tile of the routed products, where each of ``experts`` has n / experts rows on
+    average, spread as by chance: the least steps of the chip's rounds (256 workgroups), each
+    160 + rows of a tile long (fitted to the times beside csrc/moe_routed.hip). Taller tiles read
+    weights less often."""
+    mean = n / experts
+    bk = 128 if f8 else 64
+    best = None
+    for mt in (32, 48, 64) if f8 else (32, 64, 96, 128, 160):
+        # an expert has a j-th tile where its rows exceed j * mt
+        tiles = local * sum(0.5 * math.erfc((j * mt + 0.5 - mean) / math.sqrt(2 * mean))
+                            for j in range(int(2 * mean / mt) + 8))
+        steps = 0
+        for cols, k in ((I / 128, H), (H / 256, I)):
+            wgs = max(1, round(tiles)) * math.ceil(cols)
+            # the last round may end early: its workgroups have the chip to themselves
+            steps += (math.ceil(wgs / 256) + max(1, wgs / 256)) / 2 * k / bk
+        cost = steps * (160 + mt)
+        if best is None or cost < best[0]:
+            best = cost, mt
+    return best[1]
+
+
 def moe_routed_experts(x: torch.Tensor, weights: torch.Tensor, idx: torch.Tensor, w_gate, w_up,
                        w_down, scales=None, first: int = 0, num_experts: int = 0,
                        gelu: bool = False, scale_input: bool = False) -> torch.Tensor:
@@ -952,13 +978,7 @@ def moe_routed_experts(x: torch.Tensor, weights: torch.Tensor, idx: torch.Tensor
     out = torch.empty(T, H, dtype=x.dtype, device=dev)
     if n == 0:
         return out.zero_()
-    # rows of a tile by the rows an expert has on average (measured beside the kernel: taller
-    # tiles read weights less often, lower ones leave more workgroups)
-    mean = n / max(num_experts, E)
-    if scales:
-        mt = 64 if mean > 32 else 32
-    else:
-        mt = 128 if mean >= 48 else 64 if mean >= 24 else 32
+    mt = _moe_tile_rows(n, max(num_experts, E), E, H, I, bool(scales))
     tiles_max = (n + min(n, E) * (mt - 1)) // mt
     rows = tiles_max * mt
     tabs = torch.empty(1 + 2 * tiles_max + rows + n, dtype=torch.int32, device=dev)
@@ -977,7 +997,9 @@ def moe_routed_experts(x: torch.Tensor, weights: torch.Tensor, idx: torch.Tensor
     else:
         c.moe_routed_glu(h, x, w_gate, w_up, s[0], s[1], tiles, gather, mt, int(gelu))
     cols = min(H, max(256, MOE_WORKSPACE // (4 * rows) // 256 * 256))
-    ws = torch.empty(rows * cols, dtype=torch.float32, device=dev)
+    # with few tiles the down projection's workgroups share them (csrc/moe_routed.hip)
+    few = n // mt * -(-H // 256) <= 512 and cols == H
+    ws = torch.empty(max(rows * cols, 768 * 256 * mt if few else 0), dtype=torch.float32, device=dev)
     c.moe_routed_down(out, ws, h, w_down, s[2], tiles, inv, None if scale_input else weights, mt)
     return out
 

@@ -7,8 +7,12 @@
 //
 //   * Workgroup = 8 waves, MT rows of one expert x 256 columns. K goes in steps of 128 B of a
 //     weight row (128 deep with 8-bit weights, and then 64 rows at most) through a ring of three
-//     LDS buffers, global_load_lds throughout, one raw barrier a step and a counted vmcnt: two
-//     steps are in flight while one is computed.
+//     or four LDS buffers (as many as 160 KB hold), global_load_lds throughout, one raw barrier a
+//     step and a counted vmcnt: all but one of the buffers are in flight.
+//   * A second row tile of an expert reads its weights again (from the L2 at best) and adds a
+//     round of workgroups, so the height goes by the rows an expert has by chance and not only on
+//     average: 2048 tokens x 8 of 128 experts (128 rows +- 11) take 128 tiles of 160 rows, and
+//     would take 190 of 128.
 //   * The row tiles of an expert want the same weights: the list of workgroups (8 row tiles x
 //     all column tiles, rows fastest) is cut into 8 contiguous parts, one for each XCD, so that
 //     they meet in one L2. The list covers real tiles only; the grid is sized for the worst
@@ -20,18 +24,26 @@
 //     the order of its choice: the same sum in every run. fp32 atomics into the output instead
 //     took longer than the product itself (2048 tokens x 8 experts x 2048 columns: 201 of
 //     341 us; 284 of 1831 us for 4096 tokens x 2 x 4096).
+//   * Down projections of few tiles (8 experts x 16 column tiles leave half of the CUs without
+//     one) are shared out by steps: 256 workgroups take equal runs of the list's steps, across
+//     tiles, their loads running on into the next tile, and leave a part for each tile they
+//     touch; the kernel that adds up the choices adds the parts as well. 8 experts of 14336 x
+//     4096 in 8 bits, 32 rows each: 122 -> 89 us (5.3 TB/s). Runs of whole tiles for all
+//     products (a workgroup a CU) gained nothing where there are many: 360 and 353 us at 2048
+//     tokens of 128 experts, 3206 and 3307 for 4096 tokens of 8.
 //
-// The three products of a layer in us, before = moe_grouped_kernel (64 rows x 256 columns, a
-// launch each for gate, up and activation, atomics):
-//   128 experts of 2048 x 768, 8 a token:  2048 tokens 776 -> 364 (weights at the 4.9 TB/s of
-//     a large copy: 247);
-//     512 tokens 379 -> 266;  8 experts of 4096 x 14336, 2 a token: 4096 tokens 6379 -> 3290
-//     (bf16 products alone 1850), 256 tokens 688 -> 604 (577 at that rate), 128 tokens in 8 bits
-//     376 -> 309 (288).
-// Row tiles (32, 64, 128), gate + up and down with its sum: 32 rows an expert 164+102, 144+92,
-// 144+100 (64 rows 224+138, 172+118, 150+118); 128 rows 358+234, 237+185, 202+164;
-// 8 experts in 8 bits, 32 rows: 198+117, 185+143 (32 fills more of the chip); 128 rows 474+280,
-//   380+267 (128 rows x 128 columns: 440+258).
+// The layer's products with their table and sum in us, before (tiles of 32, 64 and 128 rows, a
+// ring of three, no shares, all tiles in step) -> now:
+//   128 experts of 2048 x 768, 8 a token:  64 tokens 228 -> 228, 512 255 -> 257, 1024 300 -> 290,
+//     2048 410 -> 357, 3000 487 -> 487, 4096 610 -> 562
+//   8 experts of 4096 x 14336, 2 a token:  16 tokens 558 -> 500, 128 586 -> 496, 256 630 -> 517,
+//     1024 1115 -> 951, 4096 3186 -> 3149;  in 8 bits 16 tokens 305 -> 270, 128 320 -> 289,
+//     200 349 -> 312, 256 400 -> 400
+// Row tiles there (rows an expert on average: times of tiles of 32, 64, 96, 128, 160 rows):
+//   128 experts  32: 283 257 261 264 270;  64: 376 318 290 295 296;  128: 578 445 414 405 357;
+//     188: 751 563 512 487 551;  256: 1015 730 647 601 562
+//   8 experts in 8 bits (32, 48, 64 rows)  4: 270 275 275;  32: 332 289 295;  40: 369 294 304;
+//     50: 386 407 312;  64: 513 421 404
 
 #include "common.h"
 #include <torch/extension.h>
@@ -91,106 +103,175 @@ DEV_INLINE float mr_act(float g, int gelu) {
 
 template <bool F8, int MT>
 struct MrTile {
-    static_assert(!F8 || MT < 128, "the ring would not fit");
     static constexpr int BN = 256;
     static constexpr int BK = F8 ? 128 : 64;          // 128 B of a weight row
     static constexpr int XH = BK / 64;                // 128 B images of x a step
-    static constexpr int WM = MT == 128 ? 2 : 1;      // waves along the rows
+    static constexpr int WM = MT >= 96 ? 2 : 1;       // waves along the rows
     static constexpr int WN = 8 / WM;
     static constexpr int MI = MT / WM / 16;
     static constexpr int NI = BN / WN / 16;
     static constexpr int XB = XH * MT * 128;
     static constexpr int STEP = XB + BN * 128;        // bytes of a ring buffer
+    static constexpr int D = STEP * 4 <= 163840 ? 4 : 3;
+    static_assert(STEP * D <= 163840, "the ring does not fit");
 };
+
+typedef const __attribute__((address_space(4))) int* mr_table;     // read by scalar loads
+constexpr int MR_WGS = 256;          // workgroups of a launch at most: one a CU
+constexpr int MR_GRP = 8;            // row tiles of a group
+
+// Where a launch's workgroups stop inside tiles, and not only at their ends (see the top): tiles
+// that fill the last round of the chip badly, with 8 steps or more for every workgroup.
+DEV_INLINE bool mr_shares(const int total, const int nk) {
+    const int rounds = (total + MR_WGS - 1) / MR_WGS;
+    return rounds <= 2 && total * 100 < rounds * MR_WGS * 85 && total * nk >= MR_WGS * 8;
+}
 
 template <typename T, bool F8, bool GLU, int MT>
 __global__ void __launch_bounds__(512, 2)
 moe_routed_kernel(void* __restrict__ y, const T* __restrict__ x, const char* __restrict__ w0,
                   const char* __restrict__ w1, const float* __restrict__ s0,
-                  const float* __restrict__ s1, const int* __restrict__ tiles,
-                  const int* __restrict__ gather, const int N, const int K, const int col0,
-                  const int ncols, const int ntn, const int gelu) {
+                  const float* __restrict__ s1, const int* __restrict__ tiles_,
+                  const int* __restrict__ gather_, const int N, const int K, const int col0,
+                  const int ncols, const int ntn, const int gelu, const int can_share) {
     using MF = MrMfma<T>;
     using vec8 = typename MF::vec8;
     using C = MrTile<F8, MT>;
-    constexpr int MI = C::MI, NI = C::NI, XH = C::XH;
+    constexpr int MI = C::MI, NI = C::NI, XH = C::XH, D = C::D;
     constexpr int BNO = GLU ? C::BN / 2 : C::BN;      // output columns of a workgroup
     constexpr int WP = C::BN / 64;                    // 1 KB pieces of W a wave stages
-    constexpr int XP = XH * MT / 8;                   // pieces of x in all
-    constexpr int XW = (XP + 7) / 8;                  // and of a wave that has any
+    constexpr int XP = XH * MT / 8;                   // pieces of x in all: a wave takes every 8th
+    constexpr int XW = (XP + 7) / 8;
     constexpr int ES = F8 ? 1 : 2;
-    constexpr int GRP = 8;                            // row tiles of a group
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
-    // workgroup -> tile of the list, contiguous parts for the XCDs
-    const int nreal = tiles[0], total = nreal * ntn, per = (total + 7) >> 3;
-    const int slot_wg = blockIdx.x >> 3, li = (blockIdx.x & 7) * per + slot_wg;
-    if (slot_wg >= per || li >= total) return;        // uniform over the workgroup
-    const int grp = li / (GRP * ntn), rows_grp = min(GRP, nreal - grp * GRP);
-    const int in = li - grp * GRP * ntn, rt = grp * GRP + in % rows_grp;
-    const int n0 = (in / rows_grp) * BNO;             // first column, of the slab
-    const int e = tiles[1 + 2 * rt], rows = tiles[2 + 2 * rt];
-    const long m0 = (long)rt * MT;
+    mr_table tiles = (mr_table)(size_t)tiles_, gather = (mr_table)(size_t)gather_;
+    const int nreal = tiles[0], total = nreal * ntn, nk = K / C::BK;
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    // the workgroup's part of the list: a tile, or `left` steps from step k0 of tile li0 on
+    const bool share = !GLU && can_share && mr_shares(total, nk);
+    const int per = (total + 7) >> 3, wg = xcd * (MR_WGS / 8) + slot;
+    int li0 = xcd * per + slot, k0 = 0, left = nk;
+    const int end = share ? total : min(total, (xcd + 1) * per);
+    if (share) {
+        if (slot >= MR_WGS / 8) return;
+        const long all = (long)total * nk;
+        const int from = (int)(wg * all / MR_WGS);
+        left = (int)((wg + 1) * all / MR_WGS) - from;
+        li0 = from / nk;
+        k0 = from - li0 * nk;
+    }
+    if (li0 >= end || left == 0) return;              // uniform over the workgroup
 
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm0 = (wid / C::WN) * (MI * 16), wn = wid % C::WN;
+    const int wm = wid / C::WN, wn = wid % C::WN;     // fragments wm, wm + WM, ... of the rows
     const int lrow = lane & 15, ls = lane >> 4, prow = lane >> 3;
     const int pslot = (lane & 7) ^ prow;              // source side of the XOR swizzle
     const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
 
-    const bool x_wave = XP >= 8 || wid < XP;
+    // tile of the list -> row tile, first column (of the slab)
+    auto place = [&](int li, int& rt, int& n0) {
+        const int grp = li / (MR_GRP * ntn), rows_grp = min(MR_GRP, nreal - grp * MR_GRP);
+        const int in = li - grp * MR_GRP * ntn;
+        rt = grp * MR_GRP + in % rows_grp;
+        n0 = (in / rows_grp) * BNO;
+    };
+
+    // ---- loads: a cursor that runs ahead of the products, into the next tile too ----
+    int s_li = li0, s_k = k0, s_left = left;
     const char* xsrc[XW];
-    unsigned xdst[XW];
-#pragma unroll
-    for (int i = 0; i < XW; ++i) {
-        const int piece = (x_wave ? wid * XW : 0) + i, img = piece / (MT / 8);
-        const int r = (piece % (MT / 8)) * 8 + prow;
-        const long src = gather ? (r < rows ? gather[m0 + r] : 0) : m0 + r;
-        xsrc[i] = reinterpret_cast<const char*>(x + src * K) + img * 128 + pslot * 16;
-        xdst[i] = lds0 + piece * 1024;
-    }
     const char* wsrc[WP];
-    unsigned wdst[WP];
+    auto sources = [&]() {
+        int rt, n0;
+        place(s_li, rt, n0);
+        const int e = tiles[1 + 2 * rt], rows = tiles[2 + 2 * rt];
+        const int m0 = rt * MT;
+        // Whole tiles start at different steps and wrap round: in step they would all ask for the
+        // same 128 bytes of rows a power of two apart, which few of the memory channels hold
+        // (8 experts in 16 bits, 32 rows each: 516 -> 501 us; 2048 tokens of 128: 0.87 -> 0.85 of
+        // the time before; in 8 bits the same). Row tiles of the same weights keep together.
+        if (!share) s_k = (e * ntn + n0 / BNO) % nk;
 #pragma unroll
-    for (int i = 0; i < WP; ++i) {
-        const int piece = wid * WP + i, r = piece * 8 + prow;
-        const bool up = GLU && r >= C::BN / 2;
-        const int n = min(col0 + n0 + (up ? r - C::BN / 2 : r), N - 1);
-        wsrc[i] = (up ? w1 : w0) + ((long)e * N + n) * K * ES + pslot * 16;
-        wdst[i] = lds0 + C::XB + piece * 1024;
-    }
-    auto stage = [&](int t, unsigned buf) {
-        if (x_wave) {
+        for (int i = 0; i < XW; ++i) {
+            const int piece = min(wid + 8 * i, XP - 1), img = piece / (MT / 8);
+            const int r0 = (piece % (MT / 8)) * 8;
+            long src = m0 + r0 + prow;
+            if (GLU && gather) {                      // rows past the end repeat the first token
+                int id = 0;
 #pragma unroll
-            for (int i = 0; i < XW; ++i) mr_load_lds(xsrc[i] + t * (C::BK * 2), xdst[i] + buf);
+                for (int q = 0; q < 8; ++q) {
+                    const int g = gather[m0 + r0 + q];
+                    id = prow == q ? g : id;
+                }
+                src = r0 + prow < rows ? id : 0;
+            }
+            xsrc[i] = reinterpret_cast<const char*>(x + src * K) + img * 128 + pslot * 16;
         }
 #pragma unroll
-        for (int i = 0; i < WP; ++i) mr_load_lds(wsrc[i] + t * 128, wdst[i] + buf);
+        for (int i = 0; i < WP; ++i) {
+            const int r = (wid * WP + i) * 8 + prow;
+            const bool up = GLU && r >= C::BN / 2;
+            const int n = min(col0 + n0 + (up ? r - C::BN / 2 : r), N - 1);
+            wsrc[i] = (up ? w1 : w0) + ((long)e * N + n) * K * ES + pslot * 16;
+        }
+    };
+    const bool more = wid < XP % 8;                   // this wave loads a piece of x more
+    auto stage = [&](unsigned buf) {
+        const unsigned xd = lds0 + buf + wid * 1024, wd = lds0 + buf + C::XB + wid * (WP * 1024);
+#pragma unroll
+        for (int i = 0; i < XP / 8; ++i) mr_load_lds(xsrc[i] + s_k * (C::BK * 2), xd + i * 8192);
+        if (XP % 8 && more) mr_load_lds(xsrc[XW - 1] + s_k * (C::BK * 2), xd + (XW - 1) * 8192);
+#pragma unroll
+        for (int i = 0; i < WP; ++i) mr_load_lds(wsrc[i] + s_k * 128, wd + i * 1024);
+        --s_left;
+        if (++s_k == nk) {
+            s_k = 0;
+            if (share) {
+                ++s_li;
+                if (s_left > 0) sources();
+            }
+        }
+    };
+    // wait until at most n steps of this wave's loads are in flight
+    auto wait_steps = [&](int n) {
+        constexpr int L0 = WP + XP / 8, L1 = L0 + 1;
+        if (D > 3 && n >= 2) {
+            if (XP % 8 && more) mr_vm_wait<2 * L1>();
+            else mr_vm_wait<2 * L0>();
+        } else if (n >= 1) {
+            if (XP % 8 && more) mr_vm_wait<L1>();
+            else mr_vm_wait<L0>();
+        } else {
+            mr_vm_wait<0>();
+        }
     };
 
     mr_f32x4 acc[MI][NI];
+    auto clear = [&]() {
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] = {0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < NI; ++j) acc[i][j] = {0.f, 0.f, 0.f, 0.f};
+    };
     // row of W's image that fragment j of this wave starts at: with GLU the first half of the
     // fragments are gate columns, the second the same up columns
     auto wrow = [&](int j) {
         constexpr int NH = NI / 2;
         return GLU ? (j / NH) * (C::BN / 2) + (wn * NH + j % NH) * 16 : (wn * NI + j) * 16;
     };
-    auto compute = [&](unsigned buf) {
-        const char* xb = smem + buf + (wm0 + lrow) * 128;
+    auto compute = [&](unsigned buf, auto frags) {
+        constexpr int MF_ = decltype(frags)::value;
+        const char* xb = smem + buf + (wm * 16 + lrow) * 128;
         const char* wb = smem + buf + C::XB + lrow * 128;
 #pragma unroll
         for (int kq = 0; kq < C::BK / 32; ++kq) {
-            vec8 a[MI], b[NI];
+            vec8 a[MF_], b[NI];
             const int sx = ((kq & 1) * 4 + ls) ^ (lrow & 7);
 #pragma unroll
-            for (int i = 0; i < MI; ++i)
-                a[i] = *reinterpret_cast<const vec8*>(xb + (kq >> 1) * (MT * 128) + i * 2048 +
-                                                      sx * 16);
+            for (int i = 0; i < MF_; ++i)
+                a[i] = *reinterpret_cast<const vec8*>(xb + (kq >> 1) * (MT * 128) +
+                                                      i * (C::WM * 2048) + sx * 16);
 #pragma unroll
             for (int j = 0; j < NI; ++j) {
                 if constexpr (F8) {
@@ -206,85 +287,145 @@ moe_routed_kernel(void* __restrict__ y, const T* __restrict__ x, const char* __r
                 }
             }
 #pragma unroll
-            for (int i = 0; i < MI; ++i)
+            for (int i = 0; i < MF_; ++i)
 #pragma unroll
                 for (int j = 0; j < NI; ++j) acc[i][j] = MF::mfma(b[j], a[i], acc[i][j]);
+            // (all halves' fragments at once would not fit the registers)
+            if constexpr (MI * NI > 16) __builtin_amdgcn_sched_barrier(0);
         }
     };
 
-    const int nk = K / C::BK;
-    const bool active = wm0 < rows;                   // a wave without rows only stages
-    stage(0, 0);
-    if (nk > 1) stage(1, C::STEP);
-    unsigned cur = 0, nxt = 2 * C::STEP;
-    for (int t = 0; t < nk; ++t) {
-        if (t + 1 < nk) {
-            if (XP >= 8 || !x_wave) mr_vm_wait<WP + (XP >= 8 ? XW : 0)>();
-            else mr_vm_wait<WP + XW>();
-        } else {
-            mr_vm_wait<0>();
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        // the buffer computed in the turn before is free
-        if (t + 2 < nk) stage(t + 2, nxt);
-        if (active) compute(cur);
-        cur = cur == 2 * C::STEP ? 0 : cur + C::STEP;
-        nxt = nxt == 2 * C::STEP ? 0 : nxt + C::STEP;
+    // ---- products: the cursor of the tile at hand ----
+    int li = li0, k = k0, rt, n0, rows;
+    auto enter = [&]() {
+        place(li, rt, n0);
+        rows = tiles[2 + 2 * rt];
+        clear();
+    };
+    enter();
+    sources();
+    int staged = 0;
+    unsigned cur = 0, nxt = 0;
+    for (; staged < D - 1 && s_left > 0; ++staged) {
+        stage(nxt);
+        nxt += C::STEP;
     }
-    if (!active) return;
+    for (;;) {
+        const int steps = min(nk - k, left);
+        // a loop of its own for the tiles where a wave has rows in half of its fragments at most:
+        // with both in one loop the accumulators are copied at every step
+        auto run = [&](auto frags) {
+            for (int i = 0; i < steps; ++i) {
+                // `staged` steps are on the way or there, the oldest is the one at hand
+                wait_steps(staged - 1);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                // the buffer computed in the turn before is free
+                if (s_left > 0) {
+                    stage(nxt);
+                    nxt = nxt == (D - 1) * C::STEP ? 0 : nxt + C::STEP;
+                } else {
+                    --staged;
+                }
+                compute(cur, frags);
+                cur = cur == (D - 1) * C::STEP ? 0 : cur + C::STEP;
+            }
+        };
+        constexpr int HALF = (MI + 1) / 2;
+        if (rows > (HALF * C::WM + wm) * 16) run(std::integral_constant<int, MI>{});
+        else run(std::integral_constant<int, HALF>{});
+        left -= steps;
 
-    constexpr int NO = GLU ? NI / 2 : NI;
+        // ---- the tile, or this workgroup's share of it, is done ----
+        constexpr int NO = GLU ? NI / 2 : NI;
+        const long m0 = share ? (long)(wg + li) * MT : (long)rt * MT;
+        const int pitch = share ? C::BN : ncols;
+        const int e = tiles[1 + 2 * rt];
+        int row = wm * 16 + lrow;
+        asm volatile("" : "+v"(row));     // not hoisted: addresses would not fit the registers
 #pragma unroll
-    for (int j = 0; j < NO; ++j) {
-        const int c = n0 + (wn * NO + j) * 16 + ls * 4;      // column of the slab
-        if (c >= ncols) continue;
-        mr_f32x4 sg = {1.f, 1.f, 1.f, 1.f}, su = sg;
-        if constexpr (F8) {
-            sg = *reinterpret_cast<const mr_f32x4*>(s0 + (long)e * N + col0 + c);
-            if (GLU) su = *reinterpret_cast<const mr_f32x4*>(s1 + (long)e * N + col0 + c);
-        }
+        for (int j = 0; j < NO; ++j) {
+            const int ct = (wn * NO + j) * 16 + ls * 4, c = n0 + ct;     // column of the slab
+            if (c >= ncols) continue;
+            mr_f32x4 sg = {1.f, 1.f, 1.f, 1.f}, su = sg;
+            if constexpr (F8) {
+                sg = *reinterpret_cast<const mr_f32x4*>(s0 + (long)e * N + col0 + c);
+                if (GLU) su = *reinterpret_cast<const mr_f32x4*>(s1 + (long)e * N + col0 + c);
+            }
 #pragma unroll
-        for (int i = 0; i < MI; ++i) {
-            const int m = wm0 + i * 16 + lrow;
-            if (m >= rows) continue;
-            mr_f32x4 v = acc[i][j] * sg;
-            if constexpr (GLU) {
-                const mr_f32x4 u = acc[i][j + NO] * su;
-                T o[4];
+            for (int i = 0; i < MI; ++i) {
+                const int m = i * (C::WM * 16) + row;
+                if (m >= rows) continue;
+                mr_f32x4 v = acc[i][j] * sg;
+                if constexpr (GLU) {
+                    const mr_f32x4 u = acc[i][j + NO] * su;
+                    T o[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    o[r] = VecTraits<T>::from_float(mr_act(v[r], gelu) * u[r]);
-                *reinterpret_cast<uint2*>(reinterpret_cast<T*>(y) + (m0 + m) * ncols + c) =
-                    *reinterpret_cast<const uint2*>(o);
-            } else {
-                *reinterpret_cast<mr_f32x4*>(reinterpret_cast<float*>(y) + (m0 + m) * ncols + c) = v;
+                    for (int r = 0; r < 4; ++r)
+                        o[r] = VecTraits<T>::from_float(mr_act(v[r], gelu) * u[r]);
+                    *reinterpret_cast<uint2*>(reinterpret_cast<T*>(y) + (m0 + m) * ncols + c) =
+                        *reinterpret_cast<const uint2*>(o);
+                } else {
+                    *reinterpret_cast<mr_f32x4*>(reinterpret_cast<float*>(y) + (m0 + m) * pitch +
+                                                 (share ? ct : c)) = v;
+                }
             }
         }
+        if (GLU || left == 0) break;
+        // the scales' loads end here, for the compiler too: it would wait for them, and with them
+        // for all loads in flight, at every step
+        if constexpr (F8) __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0)
+        k = 0;
+        ++li;
+        enter();
     }
 }
 
-// out[t, col0 + c] = sum over the token's choices of weight * y[row of the choice, c]
+// out[t, col0 + c] = sum over the token's choices of weight * y[row of the choice, c]. Where the
+// products' workgroups stop inside tiles (share_tile: rows of one), workgroup w's share of tile li
+// is a tile of 256 columns at w + li, and a row is the sum of its tile's shares in their order.
 template <typename T, int TOPK>
 __global__ void __launch_bounds__(256)
 moe_routed_sum_kernel(T* __restrict__ out, const float* __restrict__ y,
                       const int* __restrict__ inv, const float* __restrict__ weights,
-                      const int ntok, const int topk, const int N, const int col0,
-                      const int ncols) {
+                      const int* __restrict__ tiles, const int ntok, const int topk, const int N,
+                      const int col0, const int ncols, const int ntn, const int nk,
+                      const int share_tile) {
     const int per = ncols / 8;
     const long id = (long)blockIdx.x * 256 + threadIdx.x;
     if (id >= (long)ntok * per) return;
     const int t = (int)(id / per), c = (int)(id % per) * 8;
     const int k = TOPK ? TOPK : topk;
+    const int nreal = tiles[0], total = nreal * ntn;
+    const bool share = share_tile && mr_shares(total, nk);
     float v[8] = {};
 #pragma unroll
     for (int j = 0; j < k; ++j) {
         const int row = inv[(long)t * k + j];
         const float wt = weights ? weights[(long)t * k + j] : 1.f;
         const float* p = y + (long)max(row, 0) * ncols + c;
+        long step = 0;
+        int n = 1;
+        if (share) {
+            const int rt = max(row, 0) / share_tile, grp = rt / MR_GRP;
+            const int rows_grp = min(MR_GRP, nreal - grp * MR_GRP);
+            const int li = grp * MR_GRP * ntn + (c >> 8) * rows_grp + rt % MR_GRP;
+            const long all = (long)total * nk, s0 = (long)li * nk;
+            const int w0 = (int)(((s0 + 1) * MR_WGS - 1) / all);
+            n = (int)(((s0 + nk) * MR_WGS - 1) / all) - w0 + 1;
+            step = (long)share_tile * 256;
+            p = y + (w0 + li) * step + (max(row, 0) % share_tile) * 256 + (c & 255);
+        }
         float4 a = *reinterpret_cast<const float4*>(p);
         float4 b = *reinterpret_cast<const float4*>(p + 4);
+        for (int i = 1; i < n; ++i) {
+            p += step;
+            const float4 a1 = *reinterpret_cast<const float4*>(p);
+            const float4 b1 = *reinterpret_cast<const float4*>(p + 4);
+            a.x += a1.x; a.y += a1.y; a.z += a1.z; a.w += a1.w;
+            b.x += b1.x; b.y += b1.y; b.z += b1.z; b.w += b1.w;
+        }
         if (row < 0) a = b = float4{0.f, 0.f, 0.f, 0.f};     // another rank's expert
         v[0] += a.x * wt; v[1] += a.y * wt; v[2] += a.z * wt; v[3] += a.w * wt;
         v[4] += b.x * wt; v[5] += b.y * wt; v[6] += b.z * wt; v[7] += b.w * wt;
@@ -297,73 +438,95 @@ moe_routed_sum_kernel(T* __restrict__ out, const float* __restrict__ y,
 
 // The table: tiles[0] = number of row tiles, then (expert, rows) of each; gather = token of a
 // tile row (padding rows stay unwritten: readers go by `rows`); inv = tile row of a choice, or
-// -1 where the expert is not one of the El from `first`. One workgroup: counts and ranks by LDS
-// atomics, the scan over experts a wave's. (Rows within an expert may come in any order: each
-// is multiplied by itself, and the sum goes by `inv`.) 16384 choices of 128 experts: 63 us with
-// a scan by one thread and a search per tile, before the 10 launches it also replaces.
+// -1 where the expert is not one of the El from `first`. Rows of an expert stand in the order of
+// their choices, so that a row's tile, and the shares that its sum is made of, are the same in
+// every run. A workgroup an expert: all of them count all choices (LDS atomics), which spares a
+// launch and a wait between counts and rows, and each ranks its own by ballots, its 16 waves a
+// run of the choices each. 16384 choices of 128 experts: 20 us by one workgroup (rows in any
+// order), 17 now.
 template <typename I>
 __global__ void __launch_bounds__(1024)
 moe_route_kernel(int* __restrict__ tiles, int* __restrict__ gather, int* __restrict__ inv,
                  const I* __restrict__ idx, const int n, const int El, const long first,
                  const int topk, const int mt) {
-    extern __shared__ int rsm[];
-    int *count = rsm, *next = rsm + El;
+    extern __shared__ int count[];                    // [El]
+    __shared__ int s_mine[16], s_before[16], s_all[16];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, own = blockIdx.x;
     for (int e = threadIdx.x; e < El; e += 1024) count[e] = 0;
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += 1024) {
-        const long e = (long)idx[i] - first;
+    const int run = ((n + 15) / 16 + 63) / 64 * 64, lo = wid * run, hi = min(n, lo + run);
+    int mine = 0;
+#pragma unroll 4
+    for (int i = lo + lane; i - lane < hi; i += 64) {
+        const long e = i < hi ? (long)idx[i] - first : -1;
         if (e >= 0 && e < El) atomicAdd(&count[e], 1);
+        mine += __popcll(__ballot(e == own));
     }
+    if (lane == 0) s_mine[wid] = mine;
     __syncthreads();
-    if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        int carry = 0;
-        for (int base = 0; base < El; base += 64) {
-            const int e = base + lane, c = e < El ? count[e] : 0, nt = (c + mt - 1) / mt;
-            int s = nt;
+    int before = 0, all = 0;                          // tiles of the experts before, of all
+    for (int e = threadIdx.x; e < El; e += 1024) {
+        const int nt = (count[e] + mt - 1) / mt;
+        all += nt;
+        before += e < own ? nt : 0;
+    }
 #pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const int up = __shfl_up(s, off, 64);
-                if (lane >= off) s += up;
-            }
-            const int start = carry + s - nt;
-            if (e < El) next[e] = start * mt;
-            for (int j = 0; j < nt; ++j) {
-                tiles[1 + 2 * (start + j)] = e;
-                tiles[2 + 2 * (start + j)] = min(mt, c - j * mt);
-            }
-            carry += __shfl(s, 63, 64);
-        }
-        if (lane == 0) tiles[0] = carry;
+    for (int off = 32; off > 0; off >>= 1) {
+        before += __shfl_xor(before, off, 64);
+        all += __shfl_xor(all, off, 64);
+    }
+    if (lane == 0) {
+        s_before[wid] = before;
+        s_all[wid] = all;
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += 1024) {
-        const long e = (long)idx[i] - first;
-        int row = -1;
-        if (e >= 0 && e < El) {
-            row = atomicAdd(&next[e], 1);
-            gather[row] = i / topk;
+    int start = 0, row = 0;
+    all = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        start += s_before[w];
+        all += s_all[w];
+        row += w < wid ? s_mine[w] : 0;
+    }
+    const int c = count[own];
+    for (int j = threadIdx.x; j * mt < c; j += 1024) {
+        tiles[1 + 2 * (start + j)] = own;
+        tiles[2 + 2 * (start + j)] = min(mt, c - j * mt);
+    }
+    if (own == 0 && threadIdx.x == 0) tiles[0] = all;
+    row += start * mt;
+#pragma unroll 4
+    for (int i = lo + lane; i - lane < hi; i += 64) {
+        const long e = i < hi ? (long)idx[i] - first : -1;
+        const unsigned long long m = __ballot(e == own);
+        if (e == own) {
+            const int at = row + __popcll(m & ((1ull << lane) - 1));
+            gather[at] = i / topk;
+            inv[i] = at;
+        } else if (own == 0 && i < hi && (e < 0 || e >= El)) {
+            inv[i] = -1;
         }
-        inv[i] = row;
+        row += __popcll(m);
     }
 }
 
 template <typename T, bool F8, bool GLU, int MT>
 void mr_launch(void* y, const torch::Tensor& x, const torch::Tensor& w0, const torch::Tensor& w1,
                const float* s0, const float* s1, const torch::Tensor& tiles, const int* gather,
-               int max_tiles, int col0, int ncols, int gelu, hipStream_t st) {
+               int max_tiles, int col0, int ncols, int gelu, int share, hipStream_t st) {
     using C = MrTile<F8, MT>;
-    constexpr int LDS = 3 * C::STEP, BNO = GLU ? C::BN / 2 : C::BN;
+    constexpr int LDS = C::D * C::STEP, BNO = GLU ? C::BN / 2 : C::BN;
     // a limit of the function, the same in every call
     (void)hipFuncSetAttribute((const void*)moe_routed_kernel<T, F8, GLU, MT>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     const int ntn = (ncols + BNO - 1) / BNO;
-    const long grid = ((long)max_tiles * ntn + 7) / 8 * 8;
-    TORCH_CHECK(grid < (1L << 31), "moe_routed: too many tiles");
+    TORCH_CHECK((long)max_tiles * ntn < (1L << 30), "moe_routed: too many tiles");
+    // a workgroup a tile; shares need all MR_WGS, whatever the table turns out to hold
+    const long grid = std::max(share ? (long)MR_WGS : 0, ((long)max_tiles * ntn + 7) / 8 * 8);
     hipLaunchKernelGGL((moe_routed_kernel<T, F8, GLU, MT>), dim3((unsigned)grid), dim3(512), LDS, st, y,
                        (const T*)x.data_ptr(), (const char*)w0.data_ptr(),
                        (const char*)w1.data_ptr(), s0, s1, tiles.data_ptr<int>(), gather,
-                       (int)w0.size(1), (int)w0.size(2), col0, ncols, ntn, gelu);
+                       (int)w0.size(1), (int)w0.size(2), col0, ncols, ntn, gelu, share);
     HIP_CHECK_KERNEL();
 }
 
@@ -371,17 +534,20 @@ template <bool GLU>
 void mr_dispatch(void* y, const torch::Tensor& x, const torch::Tensor& w0,
                  const torch::Tensor& w1, const float* s0, const float* s1,
                  const torch::Tensor& tiles, const int* gather, int mt, int col0, int ncols,
-                 int gelu) {
+                 int gelu, int share) {
     const int max_tiles = (int)((tiles.numel() - 1) / 2);
     auto st = at::hip::getCurrentHIPStream();
     const bool f8 = s0 != nullptr, bf = x.scalar_type() == at::ScalarType::BFloat16;
 #define MR(TT, FF, MM) mr_launch<TT, FF, GLU, MM>(y, x, w0, w1, s0, s1, tiles, gather, max_tiles, \
-                                                  col0, ncols, gelu, st)
+                                                  col0, ncols, gelu, share, st)
 #define MR_M(TT)                                                                                  \
     do {                                                                                          \
         if (f8 && mt == 64) MR(TT, true, 64);                                                     \
+        else if (f8 && mt == 48) MR(TT, true, 48);                                                \
         else if (f8) MR(TT, true, 32);                                                            \
+        else if (mt == 160) MR(TT, false, 160);                                                   \
         else if (mt == 128) MR(TT, false, 128);                                                   \
+        else if (mt == 96) MR(TT, false, 96);                                                     \
         else if (mt == 64) MR(TT, false, 64);                                                     \
         else MR(TT, false, 32);                                                                   \
     } while (0)
@@ -393,8 +559,9 @@ void mr_dispatch(void* y, const torch::Tensor& x, const torch::Tensor& w0,
 
 void mr_check(const torch::Tensor& x, const torch::Tensor& w, const c10::optional<torch::Tensor>& s,
               const torch::Tensor& tiles, long mt) {
-    TORCH_CHECK(mt == 32 || mt == 64 || (mt == 128 && !s.has_value()),
-                "moe_routed: mt must be 32, 64 or, with 16-bit weights, 128");
+    TORCH_CHECK(mt == 32 || mt == 64 || (s.has_value() ? mt == 48
+                                                       : mt == 96 || mt == 128 || mt == 160),
+                "moe_routed: mt must be 32, 64, with 8-bit weights 48, with 16-bit 96, 128, 160");
     TORCH_CHECK(x.dim() == 2 && w.dim() == 3 && x.size(1) == w.size(2), "moe_routed: shapes");
     TORCH_CHECK(x.is_contiguous() && w.is_contiguous() && tiles.is_contiguous(),
                 "moe_routed: contiguous tensors required");
@@ -428,8 +595,8 @@ void moe_route(torch::Tensor tiles, torch::Tensor gather, torch::Tensor inv, tor
                 gather.scalar_type() == at::ScalarType::Int &&
                 inv.scalar_type() == at::ScalarType::Int, "moe_route: int32 tables");
     auto st = at::hip::getCurrentHIPStream();
-    const int lds = 2 * (int)num_local * 4;
-#define MR_ROUTE(I) hipLaunchKernelGGL(moe_route_kernel<I>, dim3(1), dim3(1024), lds, st,         \
+    const int lds = (int)num_local * 4;
+#define MR_ROUTE(I) hipLaunchKernelGGL(moe_route_kernel<I>, dim3((unsigned)num_local), dim3(1024), lds, st,         \
         tiles.data_ptr<int>(), gather.data_ptr<int>(), inv.data_ptr<int>(), idx.data_ptr<I>(),    \
         (int)n, (int)num_local, first, (int)idx.size(1), (int)mt)
     TORCH_CHECK(idx.scalar_type() == at::ScalarType::Long ||
@@ -459,7 +626,7 @@ void moe_routed_glu(torch::Tensor h, torch::Tensor x, torch::Tensor w_gate, torc
     mr_dispatch<true>(h.data_ptr(), x, w_gate, w_up, s_gate ? s_gate->data_ptr<float>() : nullptr,
                       s_up ? s_up->data_ptr<float>() : nullptr, tiles,
                       gather ? gather->data_ptr<int>() : nullptr, (int)mt, 0,
-                      (int)w_gate.size(1), (int)gelu);
+                      (int)w_gate.size(1), (int)gelu, 0);
 }
 
 // `ws` holds the products of as many columns at a time as it has room for
@@ -481,16 +648,20 @@ void moe_routed_down(torch::Tensor out, torch::Tensor ws, torch::Tensor h, torch
                 (room > 0 || ws.numel() >= rows * N), "moe_routed_down: workspace");
     const long slab = ws.numel() >= rows * N ? N : room;
     const int topk = (int)(inv.numel() / T);
+    const int nk = (int)(w_down.size(2) / (s_down.has_value() ? 128 : 64));
+    // shares: of at most 2 * MR_WGS tiles, and so fewer than 3 * MR_WGS of them
+    const bool share = slab == N && ws.numel() >= 3L * MR_WGS * mt * 256;
     auto st = at::hip::getCurrentHIPStream();
     for (long c = 0; c < N; c += slab) {
         const int nc = (int)std::min(slab, N - c);
         mr_dispatch<false>(ws.data_ptr(), h, w_down, w_down,
                            s_down ? s_down->data_ptr<float>() : nullptr, nullptr, tiles, nullptr,
-                           (int)mt, (int)c, nc, 0);
+                           (int)mt, (int)c, nc, 0, share);
         const long blocks = (T * (nc / 8) + 255) / 256;
 #define MR_SUM(TT, KK) hipLaunchKernelGGL((moe_routed_sum_kernel<TT, KK>), dim3((unsigned)blocks),  \
         dim3(256), 0, st, (TT*)out.data_ptr(), ws.data_ptr<float>(), inv.data_ptr<int>(),          \
-        weights ? weights->data_ptr<float>() : nullptr, (int)T, topk, (int)N, (int)c, nc)
+        weights ? weights->data_ptr<float>() : nullptr, tiles.data_ptr<int>(), (int)T, topk,       \
+        (int)N, (int)c, nc, (nc + 255) / 256, nk, share ? (int)mt : 0)
 #define MR_SUMK(TT)                                                                                \
     do {                                                                                           \
         if (topk == 8) {                                                                           \

@@ -185,3 +185,40 @@ def test_fused_layers_and_layers_with_hooks(hook, moe, dtype):
     tol = 0.03 if dtype == "bfloat16" else 0.004
     for a, b in zip(fused, plain):
         assert (a - b).norm() <= tol * b.norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("mt,f8,T,E,k,H,I", [
+    # tiles filled to the last row, by half and by one; experts without rows
+    (96, False, 200, 4, 2, 320, 192), (160, False, 330, 4, 2, 256, 128), (128, False, 70, 4, 2, 64, 64),
+    (160, False, 81, 4, 4, 1088, 64), (48, True, 99, 4, 2, 384, 256), (64, True, 33, 8, 1, 256, 128),
+    # shares of tiles: fewer tiles than workgroups, between one and two rounds of them
+    (32, False, 40, 8, 2, 4096, 2048), (96, False, 300, 8, 2, 4096, 1088), (48, True, 128, 8, 2, 4096, 3584),
+    (64, False, 130, 16, 2, 4608, 512), (160, False, 7, 3, 3, 8192, 1344)])
+def test_moe_routed_tile_heights_and_shares(mt, f8, T, E, k, H, I, dtype, monkeypatch):
+    """As test_moe_routed_experts, for tiles of one height and with the down projection shared out
+    or not (a workspace too small for shares): rounded activations and results, 32-bit sums."""
+    monkeypatch.setattr(ops, "_moe_tile_rows", lambda *a: mt)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(mt + T)
+    x = torch.randn(T, H, device="cuda", generator=g).to(dtype)
+    logits = torch.randn(T, E, device="cuda", generator=g)
+    logits[:, 0] += 3.0                                      # one expert of many rows
+    wt, idx = torch.softmax(logits, -1).topk(k, dim=-1)
+    w = [(torch.randn(E, *s, device="cuda", generator=g) * 0.05).to(dtype)
+         for s in ((I, H), (I, H), (H, I))]
+    scales, ref = None, [v.to(F64) for v in w]
+    if f8:
+        w, scales = zip(*[ops.fp8_moe_quantize(v) for v in w])
+        ref = [ops.fp8_moe_dequant(v, s).to(F64) for v, s in zip(w, scales)]
+    want = torch.zeros(T, H, dtype=F64, device="cuda")
+    for e in range(E):
+        t, j = (idx == e).nonzero(as_tuple=True)
+        xe = x[t].to(F64)
+        h = torch.nn.functional.silu(xe @ ref[0][e].t()) * (xe @ ref[1][e].t())
+        want.index_add_(0, t, (h @ ref[2][e].t()) * wt[t, j].to(F64).unsqueeze(1))
+    for room in (1 << 30, 4 * H * mt):
+        monkeypatch.setattr(ops, "MOE_WORKSPACE", room)
+        got = ops.moe_routed_experts(x, wt, idx, *w, scales=scales, num_experts=E)
+        assert (got.to(F64) - want).norm() < EPS16[dtype] * want.norm()
+        assert torch.equal(got, ops.moe_routed_experts(x, wt, idx, *w, scales=scales, num_experts=E))
