@@ -25,6 +25,7 @@ from typing import Dict, List, Optional
 import torch
 import torch.nn as nn
 
+from neuronx_distributed_inference_amd import ops
 from neuronx_distributed_inference_amd.models.model_base import DecoderModel
 from neuronx_distributed_inference_amd.modules.attention.attention_base import PHASE_CTE
 from neuronx_distributed_inference_amd.ops import seqmix
@@ -105,6 +106,10 @@ class HybridDecoderModel(DecoderModel):
             if self.kv_mgr.num_blocks < self.kv_mgr.state.num_slots * M:
                 raise RuntimeError(
                     "the page pool is smaller than slots x max_length: pass a block_table")
+            if ops._index(seq_ids) and seq_ids.numel() == B <= 65535:
+                block_table = torch.empty(B, M, dtype=torch.int32, device=seq_ids.device)
+                ops._require_ext("linear_table").linear_table(block_table, seq_ids)
+                return block_table
             sid = seq_ids.long().view(B, 1)
             block_table = torch.where(
                 sid >= 0,

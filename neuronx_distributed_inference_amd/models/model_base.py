@@ -24,10 +24,12 @@ from typing import Dict, List, Optional
 import torch
 import torch.nn as nn
 
+from neuronx_distributed_inference_amd import ops
 from neuronx_distributed_inference_amd.config import InferenceConfig
 from neuronx_distributed_inference_amd.modules.attention.attention_base import (
     PHASE_CTE,
     PHASE_TKG,
+    _hooked,
 )
 from neuronx_distributed_inference_amd.modules.fused_layer import fusable, run_layers
 from neuronx_distributed_inference_amd.modules.generation.sampling import (
@@ -208,6 +210,34 @@ class DecoderModel(nn.Module):
     def _phase(input_ids: torch.Tensor, position_ids: torch.Tensor) -> str:
         return PHASE_CTE if input_ids.shape[-1] > 1 else PHASE_TKG
 
+    def _fused_start(self, layers, input_ids, position_ids, seq_ids, attention_mask, phase):
+        """What ops.step_start makes of the step's tokens, where nothing but the plain modules
+        would come before the first layer's attention and the layers run fused; else None."""
+        emb, rot = self.embed_tokens, self.rotary
+        mm = getattr(self, "multimodal_ctx", None)
+        if (mm and phase == PHASE_CTE) or getattr(self, "_cos_sin_fn", None) is not None:
+            return None
+        if (type(self).embed is not DecoderModel.embed
+                or type(self).prepare_hidden is not DecoderModel.prepare_hidden
+                or type(emb) is not ParallelEmbedding or _hooked(emb) or emb.shard_along_embedding
+                or mappings.ps.get_tensor_model_parallel_size() != 1
+                or type(rot) is not RotaryEmbedding or "get_cos_sin" in vars(rot)):
+            return None
+        table = emb.weight
+        if not (table.is_cuda and input_ids.is_cuda):
+            return None
+        rot.ensure_table(1, position_ids.device)
+        if not (rot._cached_len == rot._cos_cached.shape[0]
+                and ops.step_start_takes(input_ids, position_ids, seq_ids, table,
+                                         rot._cos_cached)):
+            return None
+        like = table.new_empty(*input_ids.shape, table.shape[1])
+        if not fusable(layers, self.norm, like, attention_mask, phase):
+            return None
+        norm = layers[0].input_layernorm
+        return ops.step_start(input_ids, position_ids, seq_ids, table, rot._cos_cached,
+                              rot._sin_cached, norm.weight, norm.variance_epsilon)
+
     # -- the graph body -------------------------------------------------
     def forward(
         self,
@@ -238,13 +268,24 @@ class DecoderModel(nn.Module):
             self.ec.sequence_parallel_enabled
             and phase == PHASE_CTE and tp > 1 and S % tp == 0 and S >= tp
         )
-        h = self.embed_tokens(input_ids, sequence_parallel=sp_active) \
-            if sp_active else self.embed(input_ids)
+        post_fns = getattr(self, "_layer_post_fns", None)
+        runs = self.layer_runs()
+        fused = [layer for _, layer in runs]
+        may_fuse = (not sp_active and not post_fns
+                    and not getattr(self, "eagle3_capture_layers", None)
+                    and type(self).before_layer_run is DecoderModel.before_layer_run)
+        start = self._fused_start(fused, input_ids, position_ids, seq_ids, attention_mask,
+                                  phase) if may_fuse else None
+        if start is not None:
+            h = None
+        else:
+            h = self.embed_tokens(input_ids, sequence_parallel=sp_active) \
+                if sp_active else self.embed(input_ids)
         # multimodal splice (llava/pixtral pattern): projected vision
         # features replace the image-placeholder token embeddings. The mask
         # derives from input_ids, so bucket padding is handled for free.
         mm = getattr(self, "multimodal_ctx", None)
-        if mm and phase == PHASE_CTE and not sp_active:
+        if mm and phase == PHASE_CTE and not sp_active and start is None:
             # one splice per modality: [(placeholder_token_id, features), ...]
             # (single image/videos: qwen2-vl passes both in one prefill)
             splices = mm.get("splices")
@@ -254,27 +295,26 @@ class DecoderModel(nn.Module):
                 mask = (input_ids == tok).unsqueeze(-1)
                 h = h.masked_scatter(mask, feats.to(h.dtype).reshape(-1, h.shape[-1]))
         # models with non-1D rope (qwen2-vl m-rope) install a custom hook
-        if self.rotary is None and getattr(self, "_cos_sin_fn", None) is None:
+        if start is not None:
+            h, x, cos, sin, position_ids, seq_ids = start
+        elif self.rotary is None and getattr(self, "_cos_sin_fn", None) is None:
             cos = sin = None                 # position-free / bias-based models
         else:
             cos_sin_fn = getattr(self, "_cos_sin_fn", None) or self.rotary.get_cos_sin
             cos, sin = cos_sin_fn(position_ids, device=h.device)
-        h = self.prepare_hidden(h)
-        # int32 once here: the KV/attention kernels take int32 and a per-layer
-        # .to() would launch 4 conversion kernels per layer per step
-        position_ids = position_ids.to(torch.int32)
-        if seq_ids is not None:
-            seq_ids = seq_ids.to(torch.int32)
+        if start is None:
+            x = None
+            h = self.prepare_hidden(h)
+            # int32 once here: the KV/attention kernels take int32 and a per-layer
+            # .to() would launch 4 conversion kernels per layer per step
+            position_ids = position_ids.to(torch.int32)
+            if seq_ids is not None:
+                seq_ids = seq_ids.to(torch.int32)
         residual = None
-        post_fns = getattr(self, "_layer_post_fns", None)
         h_embed = h
-        runs = self.layer_runs()
-        fused = [layer for _, layer in runs]
-        if (not sp_active and not post_fns and not getattr(self, "eagle3_capture_layers", None)
-                and type(self).before_layer_run is DecoderModel.before_layer_run
-                and fusable(fused, self.norm, h, attention_mask, phase)):
+        if start is not None or (may_fuse and fusable(fused, self.norm, h, attention_mask, phase)):
             h = run_layers(fused, self.norm, h, cos, sin, self.kv_mgr, position_ids, phase,
-                           attention_mask, seq_ids)
+                           attention_mask, seq_ids, x)
             runs, normed = (), True
         else:
             normed = False

@@ -30,7 +30,7 @@ def _plain_norm(norm, h: torch.Tensor) -> bool:
 
 def fusable(layers, final_norm, h: torch.Tensor, attention_mask, phase: str) -> bool:
     """Whether :func:`run_layers` may stand for calling the layers and the final norm on h."""
-    if not (h.is_cuda and h.dtype in (torch.bfloat16, torch.float16) and h.shape[-1] % 8 == 0
+    if not (layers and h.is_cuda and h.dtype in (torch.bfloat16, torch.float16) and h.shape[-1] % 8 == 0
             and h.shape[-1] <= 32768 and h.numel() and h.is_contiguous()
             and h.data_ptr() % 16 == 0):
         return False
@@ -66,10 +66,12 @@ def _feed_forward(mlp, x: torch.Tensor) -> torch.Tensor:
 
 
 def run_layers(layers, final_norm, h: torch.Tensor, cos, sin, kv_mgr, position_ids, phase,
-               attention_mask, seq_ids) -> torch.Tensor:
-    """Normed output of the stack; h becomes the residual stream."""
+               attention_mask, seq_ids, x=None) -> torch.Tensor:
+    """Normed output of the stack; h becomes the residual stream. x: the first layer's normed
+    input, where that is there already."""
     layers = list(layers)
-    x = layers[0].input_layernorm(h)
+    if x is None:
+        x = layers[0].input_layernorm(h)
     for layer, after in zip(layers, layers[1:] + [None]):
         attn, mlp = layer.fused_parts()
         args = (x, cos, sin, kv_mgr, position_ids, phase, attention_mask, seq_ids)

@@ -182,6 +182,10 @@ def generate_slot_mapping(block_table: torch.Tensor, positions: torch.Tensor,
     `block_kv_cache_manager.py:376-430`): positions (B,S) + per-sequence
     block table (B, max_blocks) -> flat slots (B*S,). Negative positions
     (padding) map to slot -1 (dropped by the scatter kernel)."""
+    if (block_table.shape[1] > 0 and positions.dim() == 2
+            and block_table.shape[0] >= positions.shape[0]
+            and ops._index(block_table, positions)):
+        return ops.slot_mapping(block_table, positions, block_size)
     valid = positions >= 0
     pos = positions.clamp(min=0)
     blk = (pos // block_size).clamp(max=block_table.shape[1] - 1)

@@ -336,6 +336,61 @@ def linear_silu_mul(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return silu_mul_fused(_linear(x, weight))
 
 
+def _index(*tensors) -> bool:
+    """Whether all are contiguous int32 or int64 tensors of the current device."""
+    return all(t.is_cuda and t.dtype in (torch.int64, torch.int32) and t.is_contiguous()
+               and t.device.index == torch.cuda.current_device() for t in tensors)
+
+
+def step_start(ids, positions, seq_ids, table, cos_table, sin_table, weight, eps: float):
+    """(embedding rows, their RMS norm, cos, sin, int32 positions, int32 rows of the cache) of a
+    step's tokens: (B, S) int64 ids and positions, rope tables (rows, D) in fp32. GPU only; see
+    step_start_takes."""
+    c = _require_ext("step_start")
+    new = lambda *shape, dtype: torch.empty(*ids.shape, *shape, dtype=dtype, device=ids.device)  # noqa: E731
+    h, x = (new(table.shape[1], dtype=table.dtype) for _ in range(2))
+    cos, sin = (new(cos_table.shape[1], dtype=torch.float32) for _ in range(2))
+    pos32 = new(dtype=torch.int32)
+    sid32 = None if seq_ids is None else torch.empty_like(seq_ids, dtype=torch.int32)
+    c.step_start(h, x, cos, sin, pos32, sid32, ids, positions, seq_ids, table, cos_table, sin_table,
+                 weight, eps)
+    return h, x, cos, sin, pos32, sid32
+
+
+def step_start_takes(ids, positions, seq_ids, table, cos_table) -> bool:
+    """Whether step_start serves these; the norm's weight is the caller's to look at."""
+    return (ids.dim() == 2 and ids.dtype == torch.int64 and positions.dtype == torch.int64
+            and positions.shape == ids.shape and _index(ids, positions) and ids.numel() > 0
+            and (seq_ids is None or (_index(seq_ids) and seq_ids.dim() == 1
+                                     and seq_ids.numel() <= ids.numel()))
+            and table.device == ids.device and table.is_contiguous()
+            and table.dtype in (torch.bfloat16, torch.float16) and table.shape[1] % 8 == 0
+            and table.shape[1] <= 32768 and table.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled() and table.requires_grad)
+            and cos_table.device == ids.device and cos_table.shape[1] % 4 == 0)
+
+
+def slot_mapping(block_table, positions, block_size: int):
+    """Flat cache slots (B*S,) of (B, S) positions under (B, pages) tables, -1 for none."""
+    slots = torch.empty(positions.numel(), dtype=torch.int64, device=positions.device)
+    _require_ext("slot_mapping").slot_mapping(slots, block_table, positions, block_size)
+    return slots
+
+
+def copy_many(dst, src) -> None:
+    """dst[i].copy_(src[i]), in one launch for those that are alike and of the current device."""
+    here = torch.cuda.current_device()
+    pairs = []
+    for d, s in zip(dst, src):
+        if (s.is_cuda and s.device == d.device and d.device.index == here and s.dtype == d.dtype
+                and s.shape == d.shape and s.is_contiguous() and d.is_contiguous()):
+            pairs.append((d, s))
+        else:
+            d.copy_(s, non_blocking=True)
+    if pairs:
+        _require_ext("copy_many").copy_many(*map(list, zip(*pairs)))
+
+
 def add_norm(y: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
              eps: float) -> torch.Tensor:
     """RMS norm of residual + y; residual becomes the sum. y: of residual's shape, or parts of a

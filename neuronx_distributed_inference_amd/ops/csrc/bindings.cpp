@@ -109,10 +109,27 @@ long tile_gemm_splits(long M, long N, long K, bool glu);
 torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
                         long splits, bool parts, bool glu);
 
+void step_start(torch::Tensor h, torch::Tensor x, torch::Tensor cos, torch::Tensor sin,
+                torch::Tensor pos32, c10::optional<torch::Tensor> sid32, torch::Tensor ids,
+                torch::Tensor positions, c10::optional<torch::Tensor> seq_ids, torch::Tensor table,
+                torch::Tensor cos_table, torch::Tensor sin_table, torch::Tensor weight,
+                double eps);
+void slot_mapping(torch::Tensor slots, torch::Tensor table, torch::Tensor positions,
+                  long block_size);
+void step_layout(torch::Tensor pos32, torch::Tensor sid32, torch::Tensor nvalid,
+                 torch::Tensor positions, torch::Tensor seq_ids);
+void linear_table(torch::Tensor table, torch::Tensor seq_ids);
+void copy_many(std::vector<torch::Tensor> dst, std::vector<torch::Tensor> src);
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("rms_norm", &rms_norm, "RMSNorm (CDNA4)");
     m.def("rms_norm_fused_add", &rms_norm_fused_add, "RMSNorm + residual add (CDNA4)");
     m.def("add_norm", &add_norm, "residual sum and RMSNorm, of split products too (CDNA4)");
+    m.def("step_start", &step_start, "embedding rows, first norm, rope rows, int32 positions");
+    m.def("slot_mapping", &slot_mapping, "flat cache slots of positions");
+    m.def("step_layout", &step_layout, "int32 positions and rows, valid positions of a row");
+    m.def("linear_table", &linear_table, "page table of rows that own their pages");
+    m.def("copy_many", &copy_many, "several copies in one launch");
     m.def("tile_gemm_splits", &tile_gemm_splits, "parts of K of a tiled product, 0: not taken");
     m.def("tile_gemm", &tile_gemm, "tiled 16-bit product of up to 512 rows (CDNA4)",
           py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("splits") = 0,

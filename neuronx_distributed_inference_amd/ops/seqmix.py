@@ -151,9 +151,19 @@ class StepLayout:
     int32 positions (B,S), state slots (B,), valid-token counts (B,)."""
 
     def __init__(self, positions: torch.Tensor, seq_ids: torch.Tensor):
-        self.positions = _i32(positions)
-        self.seq_ids = _i32(seq_ids)
-        self.nvalid = (self.positions >= 0).sum(-1).to(torch.int32)
+        from neuronx_distributed_inference_amd import ops
+
+        if (ops._index(positions, seq_ids) and positions.dim() == 2 and seq_ids.dim() == 1
+                and seq_ids.numel() == positions.shape[0]):
+            self.positions, self.seq_ids = (torch.empty_like(t, dtype=torch.int32)
+                                            for t in (positions, seq_ids))
+            self.nvalid = torch.empty_like(self.seq_ids)
+            ops._require_ext("step_layout").step_layout(self.positions, self.seq_ids, self.nvalid,
+                                                        positions, seq_ids)
+        else:
+            self.positions = _i32(positions)
+            self.seq_ids = _i32(seq_ids)
+            self.nvalid = (self.positions >= 0).sum(-1).to(torch.int32)
         self._i32 = {}
         # the residual stream in the GEMM input dtype, handed from one
         # sublayer's residual kernel to the next sublayer (None: not yet made)

@@ -26,6 +26,8 @@ from typing import Callable, Dict, List, Optional, Tuple
 
 import torch
 
+from neuronx_distributed_inference_amd import ops
+
 logger = logging.getLogger("nxdi_amd")
 
 
@@ -56,9 +58,10 @@ class GraphRunner:
         self.pool = self.graph.pool()
 
     def __call__(self, *inputs):
-        for s, x in zip(self.static_inputs, inputs):
-            if isinstance(s, torch.Tensor) and x is not None:
-                s.copy_(x, non_blocking=True)
+        pairs = [(s, x) for s, x in zip(self.static_inputs, inputs)
+                 if isinstance(s, torch.Tensor) and x is not None]
+        if pairs:
+            ops.copy_many(*zip(*pairs))
         self.graph.replay()
         return self.static_outputs
 

@@ -222,3 +222,67 @@ def test_moe_routed_tile_heights_and_shares(mt, f8, T, E, k, H, I, dtype, monkey
         got = ops.moe_routed_experts(x, wt, idx, *w, scales=scales, num_experts=E)
         assert (got.to(F64) - want).norm() < EPS16[dtype] * want.norm()
         assert torch.equal(got, ops.moe_routed_experts(x, wt, idx, *w, scales=scales, num_experts=E))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,S,H,D,seq", [(1, 1, 8, 4, None), (3, 5, 2048, 64, torch.int64), (64, 1, 4096, 128, torch.int32),
+                                         (1, 600, 8192, 128, torch.int64), (2, 2, 32768, 256, None)])
+def test_step_start(B, S, H, D, seq, dtype):
+    """Rows and rope tables to the bit, the norm within the rounding of its result."""
+    V, L = 50, 40
+    table = torch.randn(V, H, device="cuda").to(dtype)
+    cos, sin = torch.randn(2, L, D, device="cuda")
+    w = torch.randn(H, device="cuda").to(dtype)
+    ids = torch.randint(0, V, (B, S), device="cuda")
+    pos = torch.randint(-3, L + 9, (B, S), device="cuda")
+    sid = None if seq is None else torch.randint(-1, 9, (B,), device="cuda").to(seq)
+    assert ops.step_start_takes(ids, pos, sid, table, cos)
+    h, x, c, s, p32, s32 = ops.step_start(ids, pos, sid, table, cos, sin, w, 1e-5)
+    assert torch.equal(h, table[ids]) and torch.equal(p32, pos.int())
+    at = pos.clamp(0, L - 1)
+    assert torch.equal(c, cos[at]) and torch.equal(s, sin[at])
+    assert (s32 is None) if sid is None else torch.equal(s32, sid.int())
+    r = h.to(F64)
+    want = r * torch.rsqrt(r.square().mean(-1, keepdim=True) + 1e-5) * w.to(F64)
+    assert ((x.to(F64) - want).abs() <= (EPS16[dtype] + 1e-5) * want.abs() + 1e-7).all()
+    for bad in (ids.int(), ids.t() if B > 1 and S > 1 else ids.cpu(), ids[:, :0]):
+        assert not ops.step_start_takes(bad, pos, sid, table, cos)
+
+
+@pytest.mark.parametrize("tdt", [torch.int64, torch.int32])
+@pytest.mark.parametrize("pdt", [torch.int64, torch.int32])
+def test_slots_layouts_and_tables(tdt, pdt):
+    """The index kernels against the same index arithmetic on the CPU, to the bit."""
+    from neuronx_distributed_inference_amd.models.hybrid_base import HybridDecoderModel
+    from neuronx_distributed_inference_amd.modules.kvcache.block_kv_cache_manager import (
+        generate_slot_mapping)
+    from neuronx_distributed_inference_amd.ops.seqmix import StepLayout
+
+    for B, S, M, bs in ((1, 1, 1, 1), (3, 300, 5, 7), (65, 2, 9, 64)):
+        table = torch.randint(-1, 1000, (B + 1, M)).to(tdt)
+        pos = torch.randint(-4, M * bs + 9, (B, S)).to(pdt)
+        got = generate_slot_mapping(table.cuda(), pos.cuda(), bs)
+        assert got.dtype == torch.int64
+        assert torch.equal(got.cpu(), generate_slot_mapping(table, pos, bs))
+        seq = torch.randint(-1, 7, (B,)).to(tdt)
+        a, b = StepLayout(pos.cuda(), seq.cuda()), StepLayout(pos, seq)
+        for n in ("positions", "seq_ids", "nvalid"):
+            assert getattr(a, n).dtype == torch.int32
+            assert torch.equal(getattr(a, n).cpu(), getattr(b, n)), n
+        model = type("M", (), {"max_blocks_per_seq": M * 300})()
+        model.kv_mgr = type("K", (), {"num_blocks": 10 ** 6, "state": type("S", (), {"num_slots": 8})})()
+        tables = [HybridDecoderModel.begin_step(model, pos.to(d), seq.to(d), None) for d in ("cuda", "cpu")]
+        assert torch.equal(tables[0].cpu().long(), tables[1])
+
+
+def test_copy_many():
+    g = torch.Generator(device="cuda").manual_seed(0)
+    src = [torch.randint(0, 255, (n,), device="cuda", generator=g, dtype=torch.uint8)
+           for n in (0, 1, 15, 16, 4097, 70001, 3, 5, 31, 64)]
+    src += [src[4][1:], src[5][::2], torch.randn(3, 5), torch.randn(2, 3, device="cuda").t(),
+            torch.arange(9, device="cuda")]
+    dst = [torch.zeros(t.shape, dtype=t.dtype, device="cuda") for t in src[:-1]]
+    dst.append(torch.zeros(9, device="cuda"))            # another type
+    ops.copy_many(dst, src)
+    for d, s in zip(dst, src):
+        assert torch.equal(d, s.to(d.device, d.dtype))
