@@ -1018,6 +1018,346 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, long qstride, const bf16* __r
     }
 }
 
+// ------------------------------ paged attention of whole rows, heads of 64 and 128
+// The same scores and options for bf16 portions whose keys and values are equally wide. Bound by
+// the vector units (a logarithm and an exponential a score), so everything else is kept off them
+// and off the L2:
+//   * 128 query rows a workgroup (tokens x heads of the group), 32 a wave. Scores are made
+//     transposed (mfma 32x32x16), so that a lane owns one row and its maximum, sum and bias are
+//     plain registers; P stays in registers as the B operand of O^T = V^T P^T, in two 16-bit
+//     parts as above.
+//   * Tiles of 64 keys go straight to LDS (global_load_lds) in two buffers, whole rows, the next
+//     while one is computed, the pages looked up a tile before that. V is transposed by
+//     ds_read_b64_tr on its way to the registers: the kernel above fetches each V row 16 bytes at
+//     a time from 64 rows at once, eight times what the tile holds from the L2.
+//   * The union of the rows' keys starts at the first that any of them sees, as above; tiles that
+//     all rows see whole take no mask.
+//   * The accumulator is rescaled only when a maximum grew by more than 2^8.
+// 4031 tokens, 16 heads of 128 on 4 KV heads, window of 1024, log-distance bias, gate:
+// 251 us with the kernel above, WF_US now.
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+#define WF_ROWS 128
+#define WF_KT 64
+#define WF_GROWTH 8.f
+#define LOG2E 1.4426950408889634f
+
+// 16 bytes a lane to the 1 KB of LDS at the wave-uniform `dst`; written out, as the compiler would
+// wait for all of them before each transposing LDS read
+DEV void wf_load_lds(const void* src, unsigned dst) {
+    const unsigned at = __builtin_amdgcn_readfirstlane(dst);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 :: "s"(at), "v"(src) : "memory", "m0");
+}
+
+DEV float wf_half_swap(float x) {
+    const unsigned u = __builtin_bit_cast(unsigned, x);
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return __builtin_bit_cast(float, (threadIdx.x & 32) ? r[0] : r[1]);
+}
+
+struct WfArgs {
+    const bf16* q;
+    const bf16* kc;
+    const bf16* vc;
+    const int* pos;
+    const int* seq;
+    const int* btab;
+    const float* r1;
+    const float* r2;
+    const bf16* gate;
+    const float* sink;
+    bf16* out;
+    long qstride, gstride, ktok, khead, vtok, vhead;
+    int max_blocks, H, G, B, bsz, page_shift, S, window, keep, qt_every, ghead, cmask, nqt;
+    float scale, cap, qt_coef;
+};
+
+template <int D>
+__global__ void __launch_bounds__(256, 2) window_flash_kernel(const WfArgs a) {
+    constexpr int ROWB = D * 2, SLOTS = ROWB / 16, RPI = 64 / SLOTS, NLD = WF_KT / 4 / RPI;
+    constexpr int TILE_B = WF_KT * ROWB, NKS = D / 16, NDB = D / 32;
+    extern __shared__ __attribute__((aligned(16))) char wf_smem[];
+    int* s_bounds = reinterpret_cast<int*>(wf_smem + 4 * TILE_B);
+
+    // KV heads go round the 8 XCDs, so that one L2 serves a head's keys; the last rows start first
+    const int NH = a.B * a.G;
+    int hg, qt;
+    {
+        const int id = blockIdx.x;
+        if ((NH & 7) == 0) {
+            const int per = NH >> 3, t = id >> 3;
+            hg = (id & 7) + 8 * (t % per);
+            qt = t / per;
+        } else {
+            hg = id % NH;
+            qt = id / NH;
+        }
+        qt = a.nqt - 1 - qt;
+    }
+    const int b = hg / a.G, g = hg % a.G, rep = a.H / a.G, R = rep * a.S;
+    if (a.seq[b] < 0) return;
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = lane >> 5;
+    const int r_own = qt * WF_ROWS + wid * 32 + (lane & 31), rr = min(r_own, R - 1);
+    const int token = rr / rep, head = g * rep + rr % rep;
+    const int qpos = r_own < R ? a.pos[(long)b * a.S + token] : -1;
+
+    int wmin = qpos < 0 ? 0x7fffffff : qpos, wmax = qpos;
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1) {
+        wmin = min(wmin, __shfl_xor(wmin, off, WAVE));
+        wmax = max(wmax, __shfl_xor(wmax, off, WAVE));
+    }
+    if (lane == 0) {
+        s_bounds[wid * 2] = wmin;
+        s_bounds[wid * 2 + 1] = wmax;
+    }
+    bf16x8_t qf[NKS];
+    {
+        const bf16* qp = a.q + ((long)b * a.S + token) * a.qstride + (long)head * D + half * 8;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks)
+            qf[ks] = *reinterpret_cast<const bf16x8_t*>(qp + ks * 16);
+    }
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) asm volatile("" : "+v"(qf[ks]));
+    float a1 = a.r1 ? a.r1[head] : 0.f, a2 = a.r2 ? a.r2[head] : 0.f;
+    // landed before the first tile is on its way: no wait for them inside the loop
+    asm volatile("" : "+v"(a1), "+v"(a2));
+    const float temp = (a.qt_every > 0 && qpos >= 0)
+        ? 1.f + a.qt_coef * logf((float)((qpos + 1) / a.qt_every) + 1.f) : 1.f;
+    const float c = a.scale * temp * LOG2E;              // scores in log2 units
+    const float a1l = a.r2 ? a1 : a1 * LOG2E;            // of log2(1 + a2 dist), or of dist
+    __syncthreads();
+    int bmin = s_bounds[0], bmax = s_bounds[1];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+        bmin = min(bmin, s_bounds[w * 2]);
+        bmax = max(bmax, s_bounds[w * 2 + 1]);
+    }
+    bmin = __builtin_amdgcn_readfirstlane(bmin);
+    bmax = __builtin_amdgcn_readfirstlane(bmax);
+    wmin = __builtin_amdgcn_readfirstlane(wmin);
+    wmax = __builtin_amdgcn_readfirstlane(wmax);
+    if (bmax < 0) return;                                // uniform over the workgroup
+    auto first_of = [&](int p) {                         // first key of a position's window
+        return max(max(0, p - a.window + 1), a.cmask > 0 ? p / a.cmask * a.cmask : 0);
+    };
+    const int lo = first_of(bmin), nfirst = min(a.keep, lo), shift = lo - nfirst;
+    const int n = nfirst + (bmax - lo + 1), tiles = (n + WF_KT - 1) / WF_KT;
+    // the wave's own first key, and the first from which on all its windows hold every key
+    const int w_lo = wmax < 0 ? 0 : first_of(wmin), w_in = wmax < 0 ? 0 : first_of(wmax);
+    const int key_lo = qpos < 0 ? 0 : first_of(qpos);
+    const int clo = qpos >= 0 && a.cmask > 0 ? qpos / a.cmask * a.cmask : 0;
+
+    const int st_row = wid * (WF_KT / 4) + lane / SLOTS, st_p = lane % SLOTS;
+    auto swz_k = [](int r) { return D == 128 ? (r & 15) : ((r >> 1) & 7); };
+    auto swz_v = [](int r) { return D == 128 ? ((r & 3) << 2) : (((r >> 1) & 1) << 2); };
+    const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)wf_smem;
+    const int* bt = a.btab + (long)b * a.max_blocks;
+    const bf16* kbase = a.kc + (long)g * a.khead;
+    const bf16* vbase = a.vc + (long)g * a.vhead;
+    int blk[NLD], rem[NLD];                              // page and row in it, a tile ahead
+    auto load_blocks = [&](int t) {
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) {
+            const int m = min(t * WF_KT + st_row + i * RPI, n - 1);
+            const int j = m < nfirst ? m : m + shift;
+            const int page = a.page_shift >= 0 ? j >> a.page_shift : j / a.bsz;
+            blk[i] = bt[page];
+            rem[i] = j - page * a.bsz;
+        }
+    };
+    auto stage = [&](int buf) {
+        const unsigned kd = lds0 + buf * 2 * TILE_B + wid * (TILE_B / 4), vd = kd + TILE_B;
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) {
+            const int r = st_row + i * RPI;
+            const long slot = (long)max(blk[i], 0) * a.bsz + rem[i];
+            wf_load_lds(kbase + slot * a.ktok + (st_p ^ swz_k(r)) * 8, kd + i * 1024);
+            wf_load_lds(vbase + slot * a.vtok + (st_p ^ swz_v(r)) * 8, vd + i * 1024);
+        }
+    };
+
+    f32x16_t o[NDB];
+#pragma unroll
+    for (int i = 0; i < NDB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+    float m = -INFINITY, l = 0.f;
+    const int ka_row = lane & 31, vi = lane & 15, va_row = half * 4 + (vi >> 2);
+    const int va_d = ((lane >> 4) & 1) * 16 + (vi & 3) * 4;
+
+    load_blocks(0);
+    stage(0);
+    if (tiles > 1) load_blocks(1);
+    for (int t = 0; t < tiles; ++t) {
+        const int buf = t & 1;
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (t + 1 < tiles) {
+            stage(buf ^ 1);
+            if (t + 2 < tiles) load_blocks(t + 2);
+        }
+        const int base = t * WF_KT, k0 = base + shift;   // k0: the tile's first key, if base >= nfirst
+        const bool plain = base >= nfirst;               // consecutive keys
+        if (wmax < 0 || (plain && (k0 > wmax || (k0 + WF_KT <= w_lo && k0 >= a.keep)))) continue;
+        const char* kb = wf_smem + buf * 2 * TILE_B;
+        const char* vb = kb + TILE_B;
+        f32x16_t s[2];
+#pragma unroll
+        for (int nn = 0; nn < 2; ++nn) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[nn][r] = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) {
+                const int r = nn * 32 + ka_row;
+                const bf16x8_t ka = *reinterpret_cast<const bf16x8_t*>(
+                    kb + r * ROWB + (((ks * 2 + half) ^ swz_k(r)) << 4));
+                s[nn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka, qf[ks], s[nn], 0, 0, 0);
+            }
+        }
+        // lane's key r of block nn: nn * 32 + 8 * (r >> 2) + 4 * half + (r & 3)
+        if (plain) {
+            const float d0 = (float)(qpos - k0 - 4 * half);
+            if (a.r1 && a.r2) {
+                const float b0 = fmaf(a2, d0, 1.f);
+#pragma unroll
+                for (int nn = 0; nn < 2; ++nn)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const float y = fmaf(-a2, (float)(nn * 32 + 8 * (r >> 2) + (r & 3)), b0);
+                        s[nn][r] = fmaf(s[nn][r], c, -a1l * __builtin_amdgcn_logf(y));
+                    }
+            } else if (a.r1) {
+#pragma unroll
+                for (int nn = 0; nn < 2; ++nn)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        s[nn][r] = fmaf(s[nn][r], c,
+                                        -a1l * (d0 - (float)(nn * 32 + 8 * (r >> 2) + (r & 3))));
+            } else {
+#pragma unroll
+                for (int nn = 0; nn < 2; ++nn)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) s[nn][r] *= c;
+            }
+        } else {
+#pragma unroll
+            for (int nn = 0; nn < 2; ++nn)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int mm = base + nn * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+                    const float dist = (float)(qpos - (mm < nfirst ? mm : mm + shift));
+                    float x = s[nn][r] * c;
+                    if (a.r1) x -= a1l * (a.r2 ? __builtin_amdgcn_logf(fmaf(a2, dist, 1.f)) : dist);
+                    s[nn][r] = x;
+                }
+        }
+        if (a.cap > 0.f) {
+#pragma unroll
+            for (int nn = 0; nn < 2; ++nn)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    s[nn][r] = a.cap * LOG2E * fast_tanh_(s[nn][r] / (LOG2E * a.cap));
+        }
+        if (!plain || base + WF_KT > n || k0 + WF_KT - 1 > wmin || k0 < w_in) {
+#pragma unroll
+            for (int nn = 0; nn < 2; ++nn)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int mm = base + nn * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+                    const int j = mm < nfirst ? mm : mm + shift;
+                    const bool ok = (mm < n) & (j <= qpos) &
+                                    ((j >= key_lo) | ((j < a.keep) & (j >= clo)));
+                    s[nn][r] = ok ? s[nn][r] : -INFINITY;
+                }
+        }
+        float mx = s[0][0];
+#pragma unroll
+        for (int nn = 0; nn < 2; ++nn)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[nn][r]);
+        mx = fmaxf(mx, wf_half_swap(mx));
+        if (__any(mx > m + WF_GROWTH || (m == -INFINITY && mx > m))) {
+            const float mn = fmaxf(m, mx), f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+            m = mn;
+            l *= f;
+#pragma unroll
+            for (int i = 0; i < NDB; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[i][r] *= f;
+        }
+        const float mu = m == -INFINITY ? 0.f : m;       // (0: a row that has seen no key yet)
+#pragma unroll
+        for (int nn = 0; nn < 2; ++nn)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float e = __builtin_amdgcn_exp2f(s[nn][r] - mu);
+                l += e;
+                s[nn][r] = e;
+            }
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            bf16x8_t ph, pl;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float e = s[kt >> 1][(kt & 1) * 8 + j];
+                ph[j] = (__bf16)e;
+                pl[j] = (__bf16)(e - (float)ph[j]);
+            }
+#pragma unroll
+            for (int db = 0; db < NDB; ++db) {
+                bf16x8_t va;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int r = kt * 16 + j * 8 + va_row, d = db * 32 + va_d;
+                    const char* at = vb + r * ROWB + (((d >> 3) ^ swz_v(r)) << 4) + (d & 7) * 2;
+                    const bf16x4_t y = __builtin_bit_cast(bf16x4_t,
+                        __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                            (__attribute__((address_space(3))) s16x4_t*)at));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) va[j * 4 + e] = y[e];
+                }
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, ph, o[db], 0, 0, 0);
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pl, o[db], 0, 0, 0);
+            }
+        }
+    }
+    // ---- a lane's row: 4 channels from 32 * db + 8 * (r >> 2) + 4 * half on ----
+    l += wf_half_swap(l);
+    if (qpos < 0) return;
+    float inv = l > 0.f ? 1.f / l : 0.f;
+    if (a.sink) {                                        // one more term in the denominator
+        const float sk = a.sink[head] * LOG2E, mf = fmaxf(m, sk);
+        const float f = m > -INFINITY ? __builtin_amdgcn_exp2f(m - mf) : 0.f;
+        inv = f / (l * f + __builtin_amdgcn_exp2f(sk - mf));
+    }
+    const long tok = (long)b * a.S + token;
+    bf16* op = a.out + (tok * a.H + head) * (long)D;
+    if (a.gate && a.ghead) inv *= sigmoidf_(__bfloat162float(a.gate[tok * a.gstride + head]));
+    const bf16* gp = a.gate && !a.ghead ? a.gate + tok * a.gstride + (long)head * D : nullptr;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+            const int d = db * 32 + 8 * q4 + 4 * half;
+            bf16x4_t y, gt;
+            if (gp) gt = *reinterpret_cast<const bf16x4_t*>(gp + d);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v = o[db][q4 * 4 + e] * inv;
+                if (gp) v *= sigmoidf_((float)gt[e]);
+                y[e] = (__bf16)v;
+            }
+            *reinterpret_cast<bf16x4_t*>(op + d) = y;
+        }
+}
+
 // ------------------------------------ latent-cache decode, matrix cores
 // Single-token steps of multi-query layers whose values are the first Dv
 // channels of the (one) key row per token — the absorbed form of latent
@@ -4869,6 +5209,28 @@ int nx_paged_attn(const void* q, long qstride, const void* kc, long ktok, long k
         const bool steps_ok = S > 1 || (wide && rp >= 8);
         if (io_bf16 && out_bf16 && steps_ok && rep_ok && dk_ok && k_al && v_al &&
             (qstride % 8) == 0 && ((uintptr_t)q % 16) == 0) {
+            // heads as wide as their values: whole rows of K and V (window_flash_kernel)
+            if (S > 1 && Dk == Dv && (Dk == 64 || Dk == 128) && (long)B * G <= 65535 &&
+                (!gate || ghead || ((gstride % 4) == 0 && ((uintptr_t)gate % 8) == 0)) &&
+                ((uintptr_t)out % 8) == 0) {
+                WfArgs f{};
+                f.q = (const bf16*)q; f.kc = (const bf16*)kc; f.vc = (const bf16*)vc;
+                f.pos = pos; f.seq = seq; f.btab = btab; f.r1 = r1; f.r2 = r2;
+                f.gate = (const bf16*)gate; f.sink = sink; f.out = (bf16*)out;
+                f.qstride = qstride; f.gstride = gstride;
+                f.ktok = ktok; f.khead = khead; f.vtok = vtok; f.vhead = vhead;
+                f.max_blocks = max_blocks; f.H = H; f.G = G; f.B = B; f.bsz = bsz; f.S = S;
+                f.page_shift = (bsz & (bsz - 1)) == 0 ? __builtin_ctz(bsz) : -1;
+                f.window = window; f.keep = keep; f.qt_every = qt_every; f.ghead = ghead;
+                f.cmask = cmask; f.scale = scale; f.cap = cap; f.qt_coef = qt_coef;
+                f.nqt = ((long)rp * S + WF_ROWS - 1) / WF_ROWS;
+                const int lds = 4 * WF_KT * Dk * 2 + 64;
+                auto* k = Dk == 128 ? window_flash_kernel<128> : window_flash_kernel<64>;
+                if (hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        lds) != hipSuccess) return -5;
+                k<<<dim3((unsigned)((long)f.nqt * B * G)), dim3(256), lds, st>>>(f);
+                return (int)hipGetLastError();
+            }
             const int QTm = MA_ROWS / rp;
             const int nsplit = wide ? (Dv + 127) / 128 : 1;
             dim3 gm((S + QTm - 1) / QTm, G * nsplit, B), bm(256);

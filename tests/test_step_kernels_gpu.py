@@ -286,3 +286,66 @@ def test_copy_many():
     ops.copy_many(dst, src)
     for d, s in zip(dst, src):
         assert torch.equal(d, s.to(d.device, d.dtype))
+
+
+WINDOWED = [
+    # S, H, G, D, page, start, options
+    (2, 4, 4, 64, 16, 0, {}),
+    (33, 12, 4, 128, 24, 200, dict(window=70, keep_first=3, r=True, gate="full")),
+    (127, 4, 1, 64, 64, 5, dict(window=64, keep_first=80, r=True)),
+    (128, 8, 8, 128, 16, 0, dict(chunk=48, sink=True, gate="head")),
+    (300, 16, 4, 128, 64, 0, dict(window=100, keep_first=4, r=True, gate="full")),
+    (65, 16, 1, 64, 24, 611, dict(window=1, slopes=True, q_temp=(0.3, 64))),
+    (130, 6, 2, 128, 16, 70, dict(window=130, keep_first=64, chunk=90, softcap=20.0, r=True)),
+    (64, 2, 2, 64, 64, 1000, dict(softcap=5.0, sink=True, slopes=True)),
+    (3, 64, 1, 128, 16, 333, dict(keep_first=9, window=32, sink=True, gate="head"))]
+
+
+def _windowed(S, H, G, D, page, start, opts, seed=0):
+    """Arguments of seqmix.paged_attention for rows of unequal length, the last tokens padding."""
+    g = torch.Generator().manual_seed(seed + S + D)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    B, opts = 3, dict(opts)
+    pos = torch.stack([start + 17 * b + torch.arange(S) for b in range(B)])
+    for b in range(1, B):
+        if S > b:
+            pos[b, S - b:] = -1
+    nb = (start + 17 * B + S) // page + 1
+    table = torch.randperm(B * nb, generator=g).view(B, nb).int()
+    kc, vc = (rnd(B * nb, page, G, D).bfloat16() for _ in range(2))
+    q = rnd(B, S, H * D + 8).bfloat16()[..., : H * D]
+    if opts.pop("r", False):
+        opts.update(r1=torch.rand(H, generator=g), r2=torch.rand(H, generator=g) * 0.3)
+    if opts.pop("slopes", False):
+        opts["slopes"] = torch.rand(H, generator=g) * 0.05
+    if opts.pop("sink", False):
+        opts["sink"] = rnd(H)
+    gate = opts.pop("gate", None)
+    if gate:
+        opts.update(gate=rnd(B, S, H * D if gate == "full" else H).bfloat16(),
+                    gate_per_head=gate == "head")
+    return q, kc, vc, pos, table, D ** -0.5, H, opts
+
+
+def _windowed_error(args):
+    from neuronx_distributed_inference_amd.ops import ref, seqmix
+
+    q, kc, vc, pos, table, scale, H, opts = args
+    want = ref.paged_attention(q.reshape(*q.shape[:2], H, -1), kc, vc, pos, table, scale, **opts)
+    cu = lambda t: t.cuda() if torch.is_tensor(t) else t  # noqa: E731
+    rows = torch.empty(*q.shape[:2], q.shape[2] + 8, dtype=q.dtype, device="cuda")
+    rows[..., : q.shape[2]] = q.cuda()
+    step = seqmix.StepLayout(pos.cuda(), torch.arange(q.shape[0], device="cuda"))
+    got = seqmix.paged_attention(rows[..., : q.shape[2]], kc.cuda(), vc.cuda(), step, table.cuda(), scale, H,
+                                 **{k: cu(v) for k, v in opts.items()})
+    ok = pos >= 0
+    got, want = got.cpu().to(F64)[ok], want.to(F64)[ok]
+    return ((got - want).norm() / want.norm()).item()
+
+
+@pytest.mark.parametrize("S,H,G,D,page,start,opts", WINDOWED)
+def test_windowed_attention_of_portions(S, H, G, D, page, start, opts):
+    """Rows that end inside tiles, windows, kept keys and blocks that begin and end inside them,
+    every option, against the plain reference: the result's rounding (2^-9) and as much for P's
+    16 bits and the hardware logarithm."""
+    assert _windowed_error(_windowed(S, H, G, D, page, start, opts)) < 2.0 ** -8
