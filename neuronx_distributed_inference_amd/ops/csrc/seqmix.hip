@@ -1034,7 +1034,7 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, long qstride, const bf16* __r
 //     all rows see whole take no mask.
 //   * The accumulator is rescaled only when a maximum grew by more than 2^8.
 // 4031 tokens, 16 heads of 128 on 4 KV heads, window of 1024, log-distance bias, gate:
-// 251 us with the kernel above, WF_US now.
+// 251 us with the kernel above, 93 now.
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
@@ -1356,6 +1356,288 @@ __global__ void __launch_bounds__(256, 2) window_flash_kernel(const WfArgs a) {
             }
             *reinterpret_cast<bf16x4_t*>(op + d) = y;
         }
+}
+
+// Single tokens, heads of 64 and 128: the same scores and options in bf16. Bound by the keys' and
+// values' bytes; a workgroup has one token's heads of a KV head (16 at most) and its 8 waves take
+// tiles of 32 keys in turn, straight to registers, the next tile in flight while one is computed
+// and the pages looked up a tile before that. Scores are K Q^T (mfma 16x16x32), so that P sits in
+// the registers as the operand of P V; it enters in three 16-bit parts, which add up to its 24
+// bits. The waves meet once, in LDS. 48 rows, 16 heads of 128 on 4 KV heads, 350 to 700 keys,
+// log-distance bias, gate: 41 us by multiply-adds (window_attn_kernel), 22 now.
+struct WdBuf {
+    uint4 k[2][4];
+    uint4 v[8];
+};
+#define WD_WAVES 8
+#define WD_KT 32
+
+template <int D>
+__global__ void __launch_bounds__(WD_WAVES * WAVE) window_decode_kernel(const WfArgs a) {
+    constexpr int NKS = D / 32, DV = D / 16;
+    const int rep = a.H / a.G, nct = (rep + 15) >> 4;
+    const int b = blockIdx.y, g = blockIdx.x / nct, c0 = blockIdx.x % nct * 16;
+    const int nc = min(16, rep - c0);
+    const int i = a.pos[b];
+    if (a.seq[b] < 0 || i < 0) return;                   // uniform over the workgroup
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = lane & 15, q4 = lane >> 4;
+    const int head = g * rep + c0 + min(n, nc - 1);
+    bf16x8_t qf[NKS];
+    {
+        const bf16* qp = a.q + (long)b * a.qstride + (long)head * D + q4 * 8;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks)
+            qf[ks] = *reinterpret_cast<const bf16x8_t*>(qp + ks * 32);
+    }
+    const float a1 = a.r1 ? a.r1[head] : 0.f, a2 = a.r2 ? a.r2[head] : 0.f;
+    const float a1l = a.r2 ? a1 : a1 * LOG2E;            // of log2(1 + a2 dist), or of dist
+    const float temp = a.qt_every > 0
+        ? 1.f + a.qt_coef * logf((float)((i + 1) / a.qt_every) + 1.f) : 1.f;
+    const float c = a.scale * temp * LOG2E;
+    const int lo = max(max(0, i - a.window + 1), a.cmask > 0 ? i / a.cmask * a.cmask : 0);
+    // as above the first `keep` keys come first; those before the token's block are not seen
+    const int nfirst = min(a.keep, lo);
+    const int clo = a.cmask > 0 ? i / a.cmask * a.cmask : 0;
+    const int shift = lo - nfirst, nk = nfirst + (i - lo + 1);
+    const int tiles = (nk + WD_KT - 1) / WD_KT;
+    const int* bt = a.btab + (long)b * a.max_blocks;
+    const bf16* kbase = a.kc + (long)g * a.khead;
+    const bf16* vbase = a.vc + (long)g * a.vhead + n * DV;
+
+    // lanes 0..31 look up the cache slot of a key of the tile each
+    auto look_up = [&](int t, int& rem) {
+        const int m = min(t * WD_KT + (lane & 31), nk - 1), j = m < nfirst ? m : m + shift;
+        const int page = a.page_shift >= 0 ? j >> a.page_shift : j / a.bsz;
+        rem = j - page * a.bsz;
+        return bt[page];
+    };
+    auto load = [&](WdBuf& u, int page, int rem) {
+        const int slot = max(page, 0) * a.bsz + rem;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            const bf16* p = kbase + (long)__shfl(slot, kb * 16 + n, WAVE) * a.ktok + q4 * 8;
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) u.k[kb][ks] = *reinterpret_cast<const uint4*>(p + ks * 32);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int kk = (j >> 2) * 16 + q4 * 4 + (j & 3);
+            const bf16* p = vbase + (long)__shfl(slot, kk, WAVE) * a.vtok;
+            if constexpr (DV == 8) u.v[j] = *reinterpret_cast<const uint4*>(p);
+            else {
+                const uint2 w = *reinterpret_cast<const uint2*>(p);
+                u.v[j].x = w.x;
+                u.v[j].y = w.y;
+            }
+        }
+    };
+    f32x4_t o[DV];
+#pragma unroll
+    for (int d = 0; d < DV; ++d) o[d] = {0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;                        // of column n; l: of this lane's keys
+
+    // scores in log2 units of key `mm` of the union
+    auto biased = [&](float s, int mm, float sc, float b1, float b2) {
+        const int j = mm < nfirst ? mm : mm + shift;
+        const float dist = (float)(i - j);
+        float x = s * sc;
+        if (a.r1) x -= b1 * (a.r2 ? __builtin_amdgcn_logf(fmaf(b2, dist, 1.f)) : dist);
+        if (a.cap > 0.f) x = a.cap * LOG2E * fast_tanh_(x / (LOG2E * a.cap));
+        return (mm < nk) & (j >= clo) ? x : -INFINITY;
+    };
+    auto step = [&](WdBuf& u, int t) {
+        f32x4_t s[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            s[kb] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks)
+                s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    __builtin_bit_cast(bf16x8_t, u.k[kb][ks]), qf[ks], s[kb], 0, 0, 0);
+        }
+        float x[8], mx = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            x[j] = biased(s[j >> 2][j & 3], t * WD_KT + (j >> 2) * 16 + q4 * 4 + (j & 3), c, a1l, a2);
+            mx = fmaxf(mx, x[j]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+        if (__any(mx > m + WF_GROWTH || (m == -INFINITY && mx > m))) {
+            const float mn = fmaxf(m, mx), f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+            m = mn;
+            l *= f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float fr = __shfl(f, q4 * 4 + r, WAVE);
+#pragma unroll
+                for (int d = 0; d < DV; ++d) o[d][r] *= fr;
+            }
+        }
+        const float mu = m == -INFINITY ? 0.f : m;
+        bf16x8_t p[3];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            float e = __builtin_amdgcn_exp2f(x[j] - mu);
+            l += e;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                p[k][j] = (__bf16)e;
+                e -= (float)p[k][j];
+            }
+        }
+        // V: pairs of channels of 8 keys -> for each channel, pairs of keys
+#pragma unroll
+        for (int d = 0; d < DV; ++d) {
+            unsigned w[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const unsigned* v0 = reinterpret_cast<const unsigned*>(&u.v[2 * e]);
+                const unsigned* v1 = reinterpret_cast<const unsigned*>(&u.v[2 * e + 1]);
+                w[e] = __builtin_amdgcn_perm(v1[d >> 1], v0[d >> 1],
+                                             (d & 1) ? 0x07060302u : 0x05040100u);
+            }
+            const bf16x8_t vb = __builtin_bit_cast(bf16x8_t, make_uint4(w[0], w[1], w[2], w[3]));
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p[k], vb, o[d], 0, 0, 0);
+        }
+    };
+    if (wid < tiles) {
+        WdBuf u0, u1;
+        int t = wid, r0, r1;
+        int p0 = look_up(t, r0), p1 = look_up(t + WD_WAVES, r1);
+        load(u0, p0, r0);
+        for (;;) {
+            // past the end the loads repeat the last key: no branch between them and their use
+            p0 = look_up(t + 2 * WD_WAVES, r0);
+            load(u1, p1, r1);
+            step(u0, t);
+            t += WD_WAVES;
+            if (t >= tiles) break;
+            p1 = look_up(t + 2 * WD_WAVES, r1);
+            load(u0, p0, r0);
+            step(u1, t);
+            t += WD_WAVES;
+            if (t >= tiles) break;
+        }
+    }
+    l += __shfl_xor(l, 16, WAVE);
+    l += __shfl_xor(l, 32, WAVE);
+
+    // ---- the waves meet ----
+    extern __shared__ __attribute__((aligned(16))) float wd_lds[];
+    float* ml = wd_lds;                                  // [waves][16][2]
+    float* ol = wd_lds + WD_WAVES * 32;                  // [waves][nc][D]
+    if (q4 == 0) {
+        ml[(wid * 16 + n) * 2] = m;
+        ml[(wid * 16 + n) * 2 + 1] = l;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (q4 * 4 + r >= nc) continue;
+        float* p = ol + (wid * nc + q4 * 4 + r) * D + n * DV;
+#pragma unroll
+        for (int d = 0; d < DV; d += 4)
+            *reinterpret_cast<float4*>(p + d) = float4{o[d][r], o[d + 1][r], o[d + 2][r], o[d + 3][r]};
+    }
+    __syncthreads();
+    // a column is D / 4 lanes of one wave
+    for (int base = wid * 64; base < nc * (D / 4); base += WD_WAVES * 64) {
+        const bool in = base + lane < nc * (D / 4);
+        const int idx = in ? base + lane : base, cl = idx / (D / 4), d = idx % (D / 4) * 4;
+        const int hh = g * rep + c0 + cl;
+        float ms = -INFINITY, ls = 0.f;
+#pragma unroll
+        for (int w = 0; w < WD_WAVES; ++w) ms = fmaxf(ms, ml[(w * 16 + cl) * 2]);
+        float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < WD_WAVES; ++w) {
+            const float lw = ml[(w * 16 + cl) * 2 + 1];
+            if (lw == 0.f) continue;                     // no key seen
+            const float f = ms == -INFINITY ? 1.f
+                                            : __builtin_amdgcn_exp2f(ml[(w * 16 + cl) * 2] - ms);
+            ls += f * lw;
+            const float4 y = *reinterpret_cast<const float4*>(ol + (w * nc + cl) * D + d);
+            acc[0] += f * y.x;
+            acc[1] += f * y.y;
+            acc[2] += f * y.z;
+            acc[3] += f * y.w;
+        }
+        // Values that are not finite: a part of P of 0 or below times one is no value. Columns
+        // whose sums are finite under values that are not are done again by multiply-adds, where
+        // a key that is not seen is not read.
+        const bool lost = !((acc[0] + acc[1]) * 0.f + (acc[2] + acc[3]) * 0.f == 0.f) && ls == ls;
+        unsigned long long bad = __ballot(lost);
+        while (bad) {
+            const int cb = (base + __ffsll(bad) - 1) / (D / 4), hb = g * rep + c0 + cb;
+            const bf16* qp = a.q + (long)b * a.qstride + (long)hb * D;
+            const float b1 = a.r1 ? a.r1[hb] * (a.r2 ? 1.f : LOG2E) : 0.f, b2 = a.r2 ? a.r2[hb] : 0.f;
+            float mr = -INFINITY, lr = 0.f, y[D / 64];
+#pragma unroll
+            for (int e = 0; e < D / 64; ++e) y[e] = 0.f;
+#pragma unroll 1
+            for (int k0 = 0; k0 < nk; k0 += 64) {
+                const int mm = min(k0 + lane, nk - 1), j = mm < nfirst ? mm : mm + shift;
+                const int page = bt[j / a.bsz];
+                const long slot = (long)max(page, 0) * a.bsz + j % a.bsz;
+                float s = 0.f;
+#pragma unroll 1
+                for (int e = 0; e < D; ++e)
+                    s += __bfloat162float(qp[e]) * __bfloat162float(kbase[slot * a.ktok + e]);
+                s = biased(s, k0 + lane, c, b1, b2);
+                const float mn = fmaxf(mr, wave_max(s));
+                const float f = mr == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mr - mn);
+                const float p = s == -INFINITY ? 0.f
+                                               : __builtin_amdgcn_exp2f(s - (mn == -INFINITY ? 0.f : mn));
+                mr = mn;
+                lr = lr * f + wave_sum(p);
+#pragma unroll
+                for (int e = 0; e < D / 64; ++e) y[e] *= f;
+#pragma unroll 1
+                for (int k = 0; k < min(64, nk - k0); ++k) {
+                    const float pk = __shfl(p, k, WAVE);
+                    const long sk = ((long)__shfl((int)(slot >> 32), k, WAVE) << 32) |
+                                    (unsigned)__shfl((int)slot, k, WAVE);
+                    if (pk == 0.f) continue;
+#pragma unroll
+                    for (int e = 0; e < D / 64; ++e)
+                        y[e] += pk * __bfloat162float(
+                            a.vc[(long)g * a.vhead + sk * a.vtok + lane * (D / 64) + e]);
+                }
+            }
+            float z[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z[e] = __shfl(y[e % (D / 64)], (d + e) / (D / 64), WAVE);
+            if (cl == cb) {
+                ms = mr;
+                ls = lr;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] = z[e];
+            }
+            bad &= ~__ballot(cl == cb);
+        }
+        if (!in) continue;
+        float inv = ls > 0.f ? 1.f / ls : ls == ls ? 0.f : ls;
+        if (a.sink) {                                    // one more term in the denominator
+            const float sk = a.sink[hh] * LOG2E, mf = fmaxf(ms, sk);
+            const float f = ms > -INFINITY ? __builtin_amdgcn_exp2f(ms - mf) : 0.f;
+            inv = f / (ls * f + __builtin_amdgcn_exp2f(sk - mf));
+        }
+        if (a.gate && a.ghead) inv *= sigmoidf_(__bfloat162float(a.gate[(long)b * a.gstride + hh]));
+        bf16x4_t y;
+        if (a.gate && !a.ghead) {
+            const bf16x4_t gt = *reinterpret_cast<const bf16x4_t*>(
+                a.gate + (long)b * a.gstride + (long)hh * D + d);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = (__bf16)(acc[e] * inv * sigmoidf_((float)gt[e]));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = (__bf16)(acc[e] * inv);
+        }
+        *reinterpret_cast<bf16x4_t*>(a.out + ((long)b * a.H + hh) * D + d) = y;
+    }
 }
 
 // ------------------------------------ latent-cache decode, matrix cores
@@ -5207,30 +5489,36 @@ int nx_paged_attn(const void* q, long qstride, const void* kc, long ktok, long k
         const bool wide = dkp > 192 || dvp > 128;
         const bool dk_ok = dkp <= 640;
         const bool steps_ok = S > 1 || (wide && rp >= 8);
+        // heads as wide as their values: whole rows of K and V
+        if (io_bf16 && out_bf16 && Dk == Dv && (Dk == 64 || Dk == 128) && B <= 65535 &&
+            (S == 1 || rep_ok) && k_al && v_al && (qstride % 8) == 0 && ((uintptr_t)q % 16) == 0 &&
+            (!gate || ghead || ((gstride % 4) == 0 && ((uintptr_t)gate % 8) == 0)) &&
+            ((uintptr_t)out % 8) == 0) {
+            WfArgs f{};
+            f.q = (const bf16*)q; f.kc = (const bf16*)kc; f.vc = (const bf16*)vc;
+            f.pos = pos; f.seq = seq; f.btab = btab; f.r1 = r1; f.r2 = r2;
+            f.gate = (const bf16*)gate; f.sink = sink; f.out = (bf16*)out;
+            f.qstride = qstride; f.gstride = gstride;
+            f.ktok = ktok; f.khead = khead; f.vtok = vtok; f.vhead = vhead;
+            f.max_blocks = max_blocks; f.H = H; f.G = G; f.B = B; f.bsz = bsz; f.S = S;
+            f.page_shift = (bsz & (bsz - 1)) == 0 ? __builtin_ctz(bsz) : -1;
+            f.window = window; f.keep = keep; f.qt_every = qt_every; f.ghead = ghead;
+            f.cmask = cmask; f.scale = scale; f.cap = cap; f.qt_coef = qt_coef;
+            f.nqt = (int)(((long)rp * S + WF_ROWS - 1) / WF_ROWS);
+            const int nc = rp < 16 ? rp : 16;
+            const int lds = S == 1 ? (WD_WAVES * 32 + WD_WAVES * nc * Dk) * 4
+                                   : 4 * WF_KT * Dk * 2 + 64;
+            auto* k = S == 1 ? (Dk == 128 ? window_decode_kernel<128> : window_decode_kernel<64>)
+                             : (Dk == 128 ? window_flash_kernel<128> : window_flash_kernel<64>);
+            const dim3 grid = S == 1 ? dim3((unsigned)(G * ((rp + 15) / 16)), (unsigned)B)
+                                     : dim3((unsigned)((long)f.nqt * B * G));
+            if (hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    lds) != hipSuccess) return -5;
+            k<<<grid, dim3(S == 1 ? WD_WAVES * WAVE : 256), lds, st>>>(f);
+            return (int)hipGetLastError();
+        }
         if (io_bf16 && out_bf16 && steps_ok && rep_ok && dk_ok && k_al && v_al &&
             (qstride % 8) == 0 && ((uintptr_t)q % 16) == 0) {
-            // heads as wide as their values: whole rows of K and V (window_flash_kernel)
-            if (S > 1 && Dk == Dv && (Dk == 64 || Dk == 128) && (long)B * G <= 65535 &&
-                (!gate || ghead || ((gstride % 4) == 0 && ((uintptr_t)gate % 8) == 0)) &&
-                ((uintptr_t)out % 8) == 0) {
-                WfArgs f{};
-                f.q = (const bf16*)q; f.kc = (const bf16*)kc; f.vc = (const bf16*)vc;
-                f.pos = pos; f.seq = seq; f.btab = btab; f.r1 = r1; f.r2 = r2;
-                f.gate = (const bf16*)gate; f.sink = sink; f.out = (bf16*)out;
-                f.qstride = qstride; f.gstride = gstride;
-                f.ktok = ktok; f.khead = khead; f.vtok = vtok; f.vhead = vhead;
-                f.max_blocks = max_blocks; f.H = H; f.G = G; f.B = B; f.bsz = bsz; f.S = S;
-                f.page_shift = (bsz & (bsz - 1)) == 0 ? __builtin_ctz(bsz) : -1;
-                f.window = window; f.keep = keep; f.qt_every = qt_every; f.ghead = ghead;
-                f.cmask = cmask; f.scale = scale; f.cap = cap; f.qt_coef = qt_coef;
-                f.nqt = ((long)rp * S + WF_ROWS - 1) / WF_ROWS;
-                const int lds = 4 * WF_KT * Dk * 2 + 64;
-                auto* k = Dk == 128 ? window_flash_kernel<128> : window_flash_kernel<64>;
-                if (hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        lds) != hipSuccess) return -5;
-                k<<<dim3((unsigned)((long)f.nqt * B * G)), dim3(256), lds, st>>>(f);
-                return (int)hipGetLastError();
-            }
             const int QTm = MA_ROWS / rp;
             const int nsplit = wide ? (Dv + 127) / 128 : 1;
             dim3 gm((S + QTm - 1) / QTm, G * nsplit, B), bm(256);

@@ -349,3 +349,42 @@ def test_windowed_attention_of_portions(S, H, G, D, page, start, opts):
     every option, against the plain reference: the result's rounding (2^-9) and as much for P's
     16 bits and the hardware logarithm."""
     assert _windowed_error(_windowed(S, H, G, D, page, start, opts)) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("H,G,D,page,start,opts", [
+    (4, 4, 64, 16, 0, {}), (12, 4, 128, 24, 200, dict(window=70, keep_first=3, r=True, gate="full")),
+    (16, 4, 128, 64, 700, dict(window=1024, keep_first=4, r=True, gate="full")),
+    (17, 1, 64, 64, 255, dict(window=256, keep_first=300, sink=True, gate="head")),
+    (40, 2, 128, 16, 95, dict(chunk=48, keep_first=60, softcap=20.0)),
+    (16, 1, 64, 24, 2211, dict(slopes=True, q_temp=(0.3, 64))), (3, 1, 128, 16, 31, dict(window=1, r=True))])
+def test_windowed_attention_of_single_tokens(H, G, D, page, start, opts):
+    """One key to several rounds of the waves, more heads than a tile has columns, every option:
+    the result's rounding (2^-9) and as much for the hardware logarithm and exponential."""
+    q, kc, vc, pos, table, scale, H, o = _windowed(3, H, G, D, page, start, opts)
+    for s in range(3):
+        one = lambda t: t[:, s:s + 1] if torch.is_tensor(t) and t.dim() == 3 and t.shape[1] == 3 else t  # noqa: E731
+        args = (q[:, s:s + 1], kc, vc, pos[:, s:s + 1], table, scale, H, {k: one(v) for k, v in o.items()})
+        assert _windowed_error(args) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_windowed_attention_of_single_tokens_values_not_finite(D, bad):
+    """A value that is not finite reaches the rows that see its key, as such, and no others."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    H, G, page, n = 6, 2, 16, 300
+    q, kc, vc, _, table, scale, H, o = _windowed(2, H, G, D, page, n, dict(window=100, keep_first=2))
+    pos = torch.tensor([[n], [n + 3], [n + 9]])
+    clean = vc.clone()
+    for b, key in ((0, n - 50), (1, n - 96), (2, 1), (2, 50)):     # seen; seen; kept; not seen
+        vc[table[b, key // page], key % page, 0, 5] = bad
+    step = seqmix.StepLayout(pos.cuda(), torch.arange(3, device="cuda"))
+    run = lambda v: seqmix.paged_attention(q[:, :1].contiguous().cuda(), kc.cuda(), v.cuda(), step,  # noqa: E731
+                                           table.cuda(), scale, H, **o).cpu().float().view(3, H, D)
+    got, want = run(vc), run(clean)
+    hit = torch.zeros(3, H, D, dtype=torch.bool)
+    hit[:, :H // G, 5] = True
+    assert torch.equal(torch.isfinite(got), ~hit)
+    assert (torch.isnan(got[hit]) if bad != bad else got[hit] == bad).all()
+    assert (got[~hit] - want[~hit]).abs().max() < 2.0 ** -7 * want.abs().max()
