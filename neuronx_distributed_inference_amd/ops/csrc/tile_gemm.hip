@@ -64,19 +64,22 @@ struct TgArgs {
 };
 
 // A workgroup of WM x WN waves makes BM x BN outputs (of one of `splits` parts of K), a wave
-// BM/WM x BN/WN of them. D chunks of x and w are in LDS or on the way there.
-template <typename T, int BM, int BN, int WM, int WN, int D, bool GLU, bool ONCE>
+// BM/WM x BN/WN of them. D chunks of w and DX of x are in LDS or on the way there. Where they
+// differ, half of the waves load w and half x: a wave's loads are waited for in their order, and
+// one that has both would wait for w as early as for x, which is near (L2).
+template <typename T, int BM, int BN, int WM, int WN, int D, int DX, bool GLU, bool ONCE>
 __global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a) {
     using MF = TgMfma<T>;
     using vec8 = typename MF::vec8;
     constexpr int NW = WM * WN;
     constexpr int FM = BM / WM / 16, FN = BN / WN / 16;
     constexpr int XPT = BM / 8, WPT = BN / 8;          // pieces of 8 rows, 1 KB, a wave's load
-    constexpr int XP = XPT >= NW ? XPT / NW : 1, WP = WPT / NW;
-    static_assert(WPT % NW == 0 && (XPT % NW == 0 || XPT < NW), "pieces");
+    constexpr bool APART = DX != D;
+    constexpr int LW = APART ? NW / 2 : NW;            // waves that load w (and x)
+    constexpr int XP = XPT >= LW ? XPT / LW : 1, WP = WPT / LW;
+    static_assert(WPT % LW == 0 && (XPT % LW == 0 || XPT < LW), "pieces");
     static_assert(!GLU || FN % 2 == 0, "gate and up of a column in one wave");
-    constexpr int G = XP + WP;                         // loads of a wave and chunk
-    constexpr int CHUNK = (BM + BN) * 128;
+    constexpr int XB = BM * 128, WB = BN * 128, W0 = DX * XB;    // bytes of a chunk; w's ring
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     // workgroups go round the XCDs: each gets one run of the work, row blocks of a tile of w
@@ -91,7 +94,10 @@ __global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a)
     const int c_lo = (int)((long)slice * chunks / a.splits);
     const int n = (int)((long)(slice + 1) * chunks / a.splits) - c_lo;    // >= 1: splits <= chunks
 
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lw = wid % LW;
+    const bool has_w = !APART || wid < LW, has_x = !APART || wid >= LW;
+    const int depth = has_w ? D : DX;
     const int wm = wid / WN, wn = wid % WN;
     const int lrow = lane & 15, lslot = lane >> 4;
 
@@ -103,12 +109,12 @@ __global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a)
     unsigned xo[XP], wo[WP];
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
-        const int r = (wid * XP + i) % XPT * 8 + prow;
+        const int r = (lw * XP + i) % XPT * 8 + prow;
         xo[i] = (unsigned)min(r, a.M - 1 - m0) * kbytes + ((lane & 7) ^ (r & 7)) * 16;
     }
 #pragma unroll
     for (int i = 0; i < WP; ++i) {
-        const int r = (wid * WP + i) * 8 + prow;
+        const int r = (lw * WP + i) * 8 + prow;
         unsigned row;
         if constexpr (GLU) {
             // of a wave's rows half are gate and half are up, of the same columns
@@ -126,17 +132,34 @@ __global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a)
     // tiles start at different chunks and wrap round: in step they would all ask for the same
     // 128 bytes of rows a power of two apart, which few of the memory channels hold
     int at = ((blockIdx.x >> 3) / a.mblocks) % n;
-    auto stage = [&](int buf) {
-        char* base = smem + buf * CHUNK;
-        const char* wp = w0 + (long)at * 128;
-        const char* xp = x0 + (long)at * 128;
+    int to = 0;                                        // buffer of the next chunk loaded
+    auto stage = [&]() {
+        if (has_w) {
+            char* base = smem + W0 + to * WB;
+            const char* wp = w0 + (long)at * 128;
 #pragma unroll
-        for (int i = 0; i < WP; ++i)
-            tg_load<ONCE ? 2 : 0>(wp + wo[i], base + BM * 128 + (wid * WP + i) * 1024);
+            for (int i = 0; i < WP; ++i)
+                tg_load<ONCE ? 2 : 0>(wp + wo[i], base + (lw * WP + i) * 1024);
+        }
+        if (has_x) {
+            char* base = smem + to * XB;
+            const char* xp = x0 + (long)at * 128;
 #pragma unroll
-        for (int i = 0; i < XP; ++i)
-            tg_load<0>(xp + xo[i], base + ((wid * XP + i) % XPT) * 1024);
+            for (int i = 0; i < XP; ++i) tg_load<0>(xp + xo[i], base + ((lw * XP + i) % XPT) * 1024);
+        }
         at = at + 1 == n ? 0 : at + 1;
+        to = to + 1 == depth ? 0 : to + 1;
+    };
+    // until at most `left` chunks of the wave's loads are in flight; ALL: as many as a full ring has
+    auto wait = [&](int left) {
+        if (!APART) tg_wait_chunks<XP + WP, D - 1>(left);
+        else if (has_w) tg_wait_chunks<WP, D - 1>(left);
+        else tg_wait_chunks<XP, DX - 1>(left);
+    };
+    auto wait_full = [&]() {
+        if (!APART) tg_wait<(XP + WP) * (D - 2)>();
+        else if (has_w) tg_wait<WP * (D - 2)>();
+        else tg_wait<XP * (DX - 2)>();
     };
 
     tg_f32x4 acc[FM][FN];
@@ -149,16 +172,15 @@ __global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a)
 #pragma unroll
     for (int h = 0; h < 2; ++h)
         off[h] = lrow * 128 + (((h * 4 + lslot) ^ (lrow & 7)) << 4);
-    const int xoff = wm * (BM / WM) * 128, woff = BM * 128 + wn * (BN / WN) * 128;
+    const int xoff = wm * (BM / WM) * 128, woff = W0 + wn * (BN / WN) * 128;
     vec8 xa[2][FM], wb[2][FN];
-    auto read = [&](int buf, int h) {
-        const char* base = smem + buf * CHUNK + off[h];
+    auto read = [&](int bx, int bw, int h) {
+        const char* xs = smem + bx * XB + xoff + off[h];
+        const char* ws = smem + bw * WB + woff + off[h];
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
-            wb[h][j] = *reinterpret_cast<const vec8*>(base + woff + j * 2048);
+        for (int j = 0; j < FN; ++j) wb[h][j] = *reinterpret_cast<const vec8*>(ws + j * 2048);
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
-            xa[h][i] = *reinterpret_cast<const vec8*>(base + xoff + i * 2048);
+        for (int i = 0; i < FM; ++i) xa[h][i] = *reinterpret_cast<const vec8*>(xs + i * 2048);
     };
     auto mma = [&](int h) {
 #pragma unroll
@@ -169,38 +191,41 @@ __global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a)
 
 #pragma unroll
     for (int i = 0; i < D; ++i)
-        if (i < n) stage(i);
-    tg_wait_chunks<G, D - 1>(min(D, n) - 1);
+        if (i < n && (i < DX || has_w)) stage();
+    wait(min(depth, n) - 1);
     __builtin_amdgcn_s_barrier();
-    read(0, 0);
-    int buf = 0, t = 0;
+    read(0, 0, 0);
+    int bx = 0, bw = 0, t = 0;
     // The second half of a chunk is read before the products of the first, and the first half of
     // the next chunk before those of the second. Between them every wave has read the chunk, which
-    // its successor D chunks on then overwrites, and has its loads of the next one.
+    // its successor a ring on then overwrites, and has its loads of the next one.
     for (; t < n - D; ++t) {
-        const int next = buf == D - 1 ? 0 : buf + 1;
-        read(buf, 1);
+        const int nx = bx == DX - 1 ? 0 : bx + 1, nw = bw == D - 1 ? 0 : bw + 1;
+        read(bx, bw, 1);
         mma(0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        tg_wait<G * (D - 2)>();
+        wait_full();
         __builtin_amdgcn_s_barrier();
-        read(next, 0);
-        stage(buf);
+        read(nx, nw, 0);
+        stage();
         mma(1);
-        buf = next;
+        bx = nx;
+        bw = nw;
     }
     for (; t < n; ++t) {
-        const int next = buf == D - 1 ? 0 : buf + 1;
-        read(buf, 1);
+        const int nx = bx == DX - 1 ? 0 : bx + 1, nw = bw == D - 1 ? 0 : bw + 1;
+        read(bx, bw, 1);
         mma(0);
         if (t + 1 < n) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            tg_wait_chunks<G, D - 1>(n - t - 2);
+            wait(min(depth - 2, n - t - 2));
             __builtin_amdgcn_s_barrier();
-            read(next, 0);
+            read(nx, nw, 0);
+            if (APART && !has_w && t + DX < n) stage();
         }
         mma(1);
-        buf = next;
+        bx = nx;
+        bw = nw;
     }
 
     // w's rows stand in the products' rows: register r of acc[i][j] is column j * 16 +
@@ -256,7 +281,7 @@ __global__ __launch_bounds__(256) void tile_sum_kernel(T* __restrict__ y,
 // The tile of a shape. A chunk of w (BN rows of 128 bytes) is what a workgroup streams, x comes
 // again and again from the L2: few rows take small tiles with a deep ring, so that a CU has 64 KB
 // and more on the way; many rows take tall ones, for fewer reads of x and w from LDS a product.
-enum TgTile { T16, T16N, T32, T32N, T64, T64N, T128, T128N, T128W, T128B, T256W };
+enum TgTile { T16, T16N, T32, T32N, T64, T64N, T128, T128N, T128W, T128B, T192, T256W };
 
 struct TgPlan {
     TgTile tile;
@@ -270,12 +295,19 @@ struct TgPlan {
 //   1       10.7 / 13.6    7.7 / 10.3    40.7 /  49.9   20.9 / 27.4   150 / 160
 //   16      11.0 / 16.2    8.1 / 13.2    39.9 /  51.7   20.7 / 26.8   151 / 164
 //   64      12.9 / 19.7   10.0 / 15.5    43.6 /  54.3   23.4 / 32.4   166 / 184
-//   128     17.8 / 21.4   14.0 / 18.9    49.0 /  60.4   30.5 / 43.2   157 / 221
-//   256     24.2 / 27.2   17.8 / 25.2    70.8 /  84.1   40.5 / 53.4   268 / 239
+//   128     17.0 / 21.4   14.0 / 18.9    50.5 /  60.4   29.8 / 43.2   154 / 221
+//   192     21.7 / 26.2   17.1 / 20.3    62.1 /  79     35.3 / 66.9   224 / 232
+//   256     24.2 / 27.2   17.8 / 25.2    75.2 /  84.1   43.5 / 53.4   268 / 239
 //   512     34.9 / 38.2   25.5 / 29.7     123 /   105   62.1 / 89.2   442 / 375
 // so up to 256 rows, unless the tiles of more than 128 rows need a second round of the chip, and
 // up to 512 rows where the tiles of the outputs alone leave CUs idle. Parts of K fill the 256 CUs
 // once, each with 2 chunks or more.
+// From 128 rows on what bounds them is what a CU takes in, x and w together: 40 to 43 GB/s in every
+// tile tried (chunks of x laid out in a row changed nothing, deeper rings of either no more), so a
+// tile of 192 rows, which reads w once for them, and x apart from w in time: 129 to 192 rows
+// 71.8 -> 62.9, 39.7 -> 35.0, 23.1 -> 20.8 (160 rows of the third, fourth and first shape; 256 rows
+// in one tile 74.2, 42.6, 24.5: no better than two of 128). Gate|up of few columns takes tiles of
+// 128 also where 256 would leave half of the CUs idle: 128 rows of the third shape 72.0 -> 50.5.
 TgPlan tg_plan(long M, long N, long K, bool glu) {
     TgPlan p{T16, 16, 128, 0};
     if (M < 1 || M > 512 || N < 64 || N % (glu ? 8 : 4) || K < 256 || K % TG_BK ||
@@ -287,9 +319,10 @@ TgPlan tg_plan(long M, long N, long K, bool glu) {
     else if (M <= 32) p = narrow ? TgPlan{T32N, 32, 64, 0} : TgPlan{T32, 32, 128, 0};
     else if (M <= 64) p = narrow ? TgPlan{T64N, 64, 64, 0} : TgPlan{T64, 64, 128, 0};
     else if (M <= 128 && narrow && glu) p = {T128N, 128, 64, 0};
-    else if (M <= 128 && N * K < (60 << 20)) p = {T128, 128, 128, 0};
+    else if (M <= 128 && (glu ? N < 49152 : N * K < (60 << 20))) p = {T128, 128, 128, 0};
     else if (M <= 128) p = {T128W, 128, 256, 0};
     else if (N * K <= (20 << 20)) p = {T128B, 128, 128, 0};
+    else if (M <= 192) p = {T192, 192, 128, 0};
     else p = {T256W, 128, 256, 0};
     const long tiles = (M + p.bm - 1) / p.bm * ((N + p.bn - 1) / p.bn);
     if (M > 128 && tiles > 256) return p;
@@ -298,14 +331,15 @@ TgPlan tg_plan(long M, long N, long K, bool glu) {
     return p;
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int D, bool GLU, bool ONCE>
+template <typename T, int BM, int BN, int WM, int WN, int D, bool GLU, bool ONCE, int DX = D>
 void tg_go(TgArgs& a, hipStream_t stream) {
     a.mblocks = (a.M + BM - 1) / BM;
     a.ntiles = (a.N + BN - 1) / BN;
     a.work = a.mblocks * a.ntiles * a.splits;
     a.per_xcd = (a.work + 7) / 8;
-    constexpr int LDS = D * (BM + BN) * 128;
-    auto* k = tile_gemm_kernel<T, BM, BN, WM, WN, D, GLU, ONCE>;
+    constexpr int LDS = (DX * BM + D * BN) * 128;
+    static_assert(LDS <= 163840, "the rings do not fit");
+    auto* k = tile_gemm_kernel<T, BM, BN, WM, WN, D, DX, GLU, ONCE>;
     TORCH_CHECK(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     LDS) == hipSuccess, "tile_gemm: LDS");
     hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(64 * WM * WN), LDS, stream, a);
@@ -325,6 +359,7 @@ void tg_tile(TgArgs& a, TgTile tile, hipStream_t s) {
         case T128N: tg_go<T, 128, 64, 4, 2, 6, GLU, true>(a, s); break;
         case T128W: tg_go<T, 128, 256, 2, 4, 3, GLU, true>(a, s); break;
         case T128B: tg_go<T, 128, 128, 2, 4, 5, GLU, false>(a, s); break;
+        case T192: tg_go<T, 192, 128, 4, 2, 5, GLU, true, 3>(a, s); break;
         case T256W: tg_go<T, 128, 256, 2, 4, 3, GLU, false>(a, s); break;
     }
 }

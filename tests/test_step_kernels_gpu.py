@@ -388,3 +388,26 @@ def test_windowed_attention_of_single_tokens_values_not_finite(D, bad):
     assert torch.equal(torch.isfinite(got), ~hit)
     assert (torch.isnan(got[hit]) if bad != bad else got[hit] == bad).all()
     assert (got[~hit] - want[~hit]).abs().max() < 2.0 ** -7 * want.abs().max()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,glu", [
+    (129, 5124, 4160, False), (160, 21000, 1024, False), (191, 32764, 704, False), (192, 6144, 4096, False),
+    (193, 32768, 704, False), (129, 28680, 768, True), (192, 21000, 1024, True), (65, 28672, 256, True),
+    (128, 49152, 256, True), (128, 49144, 320, True)])
+def test_tile_gemm_rings_of_their_own(M, N, K, glu, dtype):
+    """Tiles of 192 rows, whose halves of the waves load x and w through rings of unequal length:
+    fewer chunks than either ring, as many, more; and the other tiles at the border."""
+    x, w, exact, sums = _product(M, N, K, dtype)
+    if glu:
+        g, u = exact.chunk(2, dim=1)
+        want = torch.nn.functional.silu(g) * u
+        gs, us = sums.chunk(2, dim=1)
+        limit = 1.1 * gs * u.abs() + us * g.abs() + (EPS16[dtype] + 2.0 ** -18) * want.abs() + 1e-6
+        got = ops._C.tile_gemm(x, w, glu=True).to(F64)
+        assert ((got - want).abs() <= limit).all()
+        return
+    for splits in {1, 2, ops._tile_takes(x, w), K // 64}:
+        parts = ops._C.tile_gemm(x, w, None, splits, True).to(F64)
+        got, limit = (parts.sum(0), sums) if splits > 1 else (parts, sums + EPS16[dtype] * exact.abs())
+        assert ((got - exact).abs() <= limit + 1e-30).all()
