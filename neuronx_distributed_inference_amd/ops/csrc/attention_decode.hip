@@ -357,7 +357,7 @@ __global__ __launch_bounds__(256) void decode_attn_pass1(
 //   * The accumulator is rescaled only when a maximum grew by more than 2^8.
 // Measured in a captured graph (MI355X, bf16, 32/8 heads of 128, lengths half to full, before ->
 // now, stream rate): 64 rows of 2048 131 -> 76 us (5.3 TB/s); 16 of 8192 136 -> 73; 128 of 512
-// 68 -> 40; 256 of 168 57 -> 35; 1 of 300 18.2 -> 7.8; 1 of 8192 55 -> 12; 13 rows of 8000, 64/8
+// 68 -> 40; 256 of 168 57 -> 28; 1 of 300 18.2 -> 7.8; 1 of 8192 55 -> 12; 13 rows of 8000, 64/8
 // heads 271 -> 72 us, e4m3 279 -> 48 us. Error against 64 bits, bf16: 1.66e-3 (the rounding of
 // the result), before 1.66e-3 to 3.5e-3 (the scaled query was rounded too).
 typedef __bf16 dm_bf16x8 __attribute__((ext_vector_type(8)));
@@ -435,7 +435,7 @@ constexpr float DM_DEPTH = 64.f;   // and how far below the largest score P may 
 constexpr int DM_TILE = 32;        // keys of a wave's step
 constexpr int DM_LEAST = 128;      // keys of a split: one step of each wave
 
-template <typename T, typename CT, int D, bool PAGED>
+template <typename T, typename CT, int D, bool PAGED, int WPR>
 __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
     T* __restrict__ out,               // (B, Hq, Sq, D), written when nsplit == 1
     float* __restrict__ o_part,        // (B, Hq, Sq, nsplit, D)
@@ -445,7 +445,7 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
     const int* __restrict__ block_table, const float* __restrict__ sinks,
     float* __restrict__ lse_out, const float scale, const float v_scale, const int window,
     const int ring, const int Hkv, const int Sq, const int gq, const int Smax, const int nsplit,
-    const int block_size, const int max_blocks) {
+    const int block_size, const int max_blocks, const int B) {
     using DT = DmTraits<T>;
     using vec8 = typename DT::vec8;
     constexpr bool F8 = sizeof(CT) == 1;
@@ -455,19 +455,32 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
     constexpr int DV = D / 16;             // channels a lane holds of a V row
     constexpr int ES = sizeof(CT);
 
-    const int split = blockIdx.x;
     const int ncol = gq * Sq;
     const int nct = (ncol + 15) >> 4;
-    const int hkv = blockIdx.y / nct;
-    const int c0 = (blockIdx.y % nct) * 16;
-    const int nc = min(16, ncol - c0);
-    const int b = blockIdx.z;
-    const int Hq = Hkv * gq;
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: so are the loops
     const int n = lane & 15, g = lane >> 4;
+    // a set of columns is WPR waves' work (see launch_decode); the last ones may have none
+    const int sub = wid % WPR, slot0 = wid - sub;
+    int split, y, b;
+    bool idle = false;
+    if constexpr (WPR == 4) {
+        split = blockIdx.x;
+        y = blockIdx.y;
+        b = blockIdx.z;
+    } else {                                   // (no splits)
+        const long set = (long)blockIdx.x * (4 / WPR) + wid / WPR;
+        idle = set >= (long)B * Hkv * nct;
+        split = 0;
+        b = idle ? B - 1 : (int)(set / (Hkv * nct));
+        y = idle ? 0 : (int)(set % (Hkv * nct));
+    }
+    const int hkv = y / nct;
+    const int c0 = (y % nct) * 16;
+    const int nc = min(16, ncol - c0), ncw = min(16, ncol);    // ncw: columns of a wave's LDS
+    const int Hq = Hkv * gq;
 
-    const int row = PAGED ? 0 : seq_ids[b];
+    const int row = idle ? -1 : PAGED ? 0 : seq_ids[b];
     const int col = min(c0 + n, ncol - 1);
     const int sq = col / gq;
     const int head = hkv * gq + col % gq;
@@ -644,22 +657,22 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
         }
     };
 
-    if (t_lo + wid < t_hi) {
+    if (t_lo + sub < t_hi) {
         Buf u0, u1;
-        int t = t_lo + wid;
-        int blk = page_load(t), next = page_load(t + 4);
+        int t = t_lo + sub;
+        int blk = page_load(t), next = page_load(t + WPR);
         load(u0, t, blk);
         for (;;) {
             // past the end the loads repeat the last key: no branch between them and their use
-            blk = page_load(t + 8);
-            load(u1, t + 4, next);
+            blk = page_load(t + 2 * WPR);
+            load(u1, t + WPR, next);
             step(u0, t);
-            t += 4;
+            t += WPR;
             if (t >= t_hi) break;
-            next = page_load(t + 8);
-            load(u0, t + 4, blk);
+            next = page_load(t + 2 * WPR);
+            load(u0, t + WPR, blk);
             step(u1, t);
-            t += 4;
+            t += WPR;
             if (t >= t_hi) break;
         }
     }
@@ -667,10 +680,10 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
     l += __shfl_xor(l, 32, WAVE_SIZE);
     m -= LIFT;
 
-    // ---- the four waves meet ----
+    // ---- the waves of a set meet ----
     extern __shared__ __attribute__((aligned(16))) float dm_lds[];
-    float* o_lds = dm_lds;                     // [4][nc][D]
-    float* ml_lds = dm_lds + 4 * nc * D;       // [4][16][2]
+    float* o_lds = dm_lds;                     // [4][ncw][D]
+    float* ml_lds = dm_lds + 4 * ncw * D;      // [4][16][2]
     if (g == 0) {
         ml_lds[(wid * 16 + n) * 2] = m;
         ml_lds[(wid * 16 + n) * 2 + 1] = l;
@@ -678,7 +691,7 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         if (g * 4 + r >= nc) continue;
-        float* p = o_lds + (wid * nc + g * 4 + r) * D + n * DV;
+        float* p = o_lds + (wid * ncw + g * 4 + r) * D + n * DV;
 #pragma unroll
         for (int i = 0; i < DV; i += 4)
             *reinterpret_cast<float4*>(p + i) =
@@ -686,7 +699,8 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
     }
     __syncthreads();
     // (whole waves, for the rows that are done again: a column is 32 or 16 lanes of one)
-    for (int base = wid * 64; base < nc * (D / 4); base += 256) {
+    if (idle) return;
+    for (int base = sub * 64; base < nc * (D / 4); base += WPR * 64) {
         const bool in = base + lane < nc * (D / 4);
         const int idx = in ? base + lane : base;
         const int cl = idx / (D / 4), d = idx % (D / 4) * 4;
@@ -694,16 +708,16 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
         const int hh = hkv * gq + cc % gq;
         float ms = -INFINITY, ls = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) ms = fmaxf(ms, ml_lds[(w * 16 + cl) * 2]);
+        for (int w = slot0; w < slot0 + WPR; ++w) ms = fmaxf(ms, ml_lds[(w * 16 + cl) * 2]);
         float4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
+        for (int w = slot0; w < slot0 + WPR; ++w) {
             const float lw = ml_lds[(w * 16 + cl) * 2 + 1];
             if (lw == 0.f) continue;       // no key seen
             // (no maximum, but a sum: it is NaN, as of a query that is, and stays)
             const float f = ms == -INFINITY ? 1.f : exp2f(ml_lds[(w * 16 + cl) * 2] - ms);
             ls += f * lw;
-            const float4 y = *reinterpret_cast<const float4*>(o_lds + (w * nc + cl) * D + d);
+            const float4 y = *reinterpret_cast<const float4*>(o_lds + (w * ncw + cl) * D + d);
             acc.x += f * y.x;
             acc.y += f * y.y;
             acc.z += f * y.z;
@@ -892,9 +906,21 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
         if (B == 0 || Sq == 0) return;
         const int nc = std::min(16, gq * Sq);
         const size_t lds = (4 * nc * D + 4 * 16 * 2) * sizeof(float);
-        dim3 grid(nsplit, Hkv * nct, B);
-#define DM_GO(PG)                                                                           \
-        hipLaunchKernelGGL((decode_mfma_kernel<T, CT, D, PG>), grid, dim3(256), lds, stream, \
+        const long sets = (long)B * Hkv * nct;
+        // Waves of a set of columns (of one row's KV head). Where rows are short a workgroup is
+        // gone after a step or two of its waves, and what it waits for on the way (positions,
+        // pages, the first keys, the other waves) is most of its time: a wave a set takes more
+        // steps, and all sets are there at once. 32/8 heads of 128, half to full caches, 4 waves
+        // and 1: 256 rows of 168 34.1, 28.2 us (e4m3, 64/8 heads 32.7, 23.0), 200 of 100 24.3,
+        // 20.2, 128 of 168 21.0, 18.1, 100 of 300 25.7, 23.5, but 64 of 300 15.5, 20.4, 256 of 500
+        // 76, 81, 160 of 700 64, 81, 128 of 512 in e4m3 27.8, 29.0. (2 waves lie between, within
+        // 1 us of the better.)
+        const int span = window ? std::min(Smax, std::abs(window) + Sq + DM_TILE) : Smax;
+        const bool alone = nsplit == 1 && span <= 384 && sets >= 768;
+        TORCH_CHECK(sets < (1L << 31), "attention_decode: too many rows");
+        const dim3 grid = alone ? dim3((unsigned)((sets + 3) / 4)) : dim3(nsplit, Hkv * nct, B);
+#define DM_GO(PG, W)                                                                        \
+        hipLaunchKernelGGL((decode_mfma_kernel<T, CT, D, PG, W>), grid, dim3(256), lds, stream, \
                            (T*)out.data_ptr(), o_part.data_ptr<float>(),                    \
                            ml_part.data_ptr<float>(), (const T*)q.data_ptr(),               \
                            (const CT*)k_cache.data_ptr(), (const CT*)v_cache.data_ptr(),    \
@@ -902,9 +928,14 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
                            PG ? block_table->data_ptr<int>() : nullptr,                     \
                            sinks ? sinks->data_ptr<float>() : nullptr,                      \
                            lse_out ? lse_out->data_ptr<float>() : nullptr, scale, v_scale,  \
-                           window, ring, Hkv, Sq, gq, Smax, nsplit, block_size, max_blocks)
-        if (paged) DM_GO(true);
-        else DM_GO(false);
+                           window, ring, Hkv, Sq, gq, Smax, nsplit, block_size, max_blocks, B)
+        if (paged) {
+            if (alone) DM_GO(true, 1);
+            else DM_GO(true, 4);
+        } else {
+            if (alone) DM_GO(false, 1);
+            else DM_GO(false, 4);
+        }
 #undef DM_GO
         HIP_CHECK_KERNEL();
         if (nsplit == 1) return;

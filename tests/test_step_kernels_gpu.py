@@ -411,3 +411,33 @@ def test_tile_gemm_rings_of_their_own(M, N, K, glu, dtype):
         parts = ops._C.tile_gemm(x, w, None, splits, True).to(F64)
         got, limit = (parts.sum(0), sums) if splits > 1 else (parts, sums + EPS16[dtype] * exact.abs())
         assert ((got - exact).abs() <= limit + 1e-30).all()
+
+
+@pytest.mark.parametrize("kind", ["linear", "ring", "paged", "fp8", "window"])
+@pytest.mark.parametrize("B,Hkv,gq,Sq,D", [(171, 3, 4, 1, 128), (65, 8, 1, 3, 64), (193, 8, 8, 1, 64),
+                                           (257, 7, 5, 4, 128), (64, 8, 4, 1, 128)])
+def test_decode_attention_of_many_short_rows(kind, B, Hkv, gq, Sq, D):
+    """A wave a row (the last workgroup's may have none) against the same rows in small
+    batches, which four waves or splits of the keys serve: both round the result once (2^-9)."""
+    g = torch.Generator(device="cuda").manual_seed(B)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()  # noqa: E731
+    cap, Hq = 96 if kind != "window" else 700, Hkv * gq
+    q = rnd(B, Hq, Sq, D)
+    pos = torch.randint(0, 2 * cap if kind == "ring" else cap - Sq, (B, 1), device="cuda", generator=g) \
+        + torch.arange(Sq, device="cuda")
+    if kind == "paged":
+        k, v = rnd(B * 6, 16, Hkv, D), rnd(B * 6, 16, Hkv, D)
+        table = torch.randperm(B * 6, device="cuda", generator=g).view(B, 6).int()
+        table[3, 2:] = -1
+        run = lambda a, b: ops.attention_decode_paged(q[a:b], k, v, pos[a:b], table[a:b])  # noqa: E731
+    else:
+        k, v = rnd(B, Hkv, cap, D), rnd(B, Hkv, cap, D)
+        if kind == "fp8":
+            k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+        rows = torch.randperm(B, device="cuda", generator=g).int()
+        kw = {"ring": dict(sliding_window=cap, ring=True), "window": dict(sliding_window=40)}.get(kind, {})
+        run = lambda a, b: ops.attention_decode(q[a:b], k, v, pos[a:b], rows[a:b], **kw)  # noqa: E731
+    got = run(0, B)
+    want = torch.cat([run(a, min(a + 20, B)) for a in range(0, B, 20)])
+    err = (got.to(F64) - want.to(F64)).norm(dim=-1) / want.to(F64).norm(dim=-1).clamp(min=1e-3)
+    assert torch.isfinite(got).all() and err.max() < 2.0 ** -7 and err.mean() < 2.0 ** -8
