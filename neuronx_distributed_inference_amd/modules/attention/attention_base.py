@@ -189,6 +189,38 @@ class AttentionBase(nn.Module):
             return ops.linear_parts(hidden, self.qkv_proj.qkv.weight)
         return self.qkv_proj.qkv(hidden)
 
+    def prompt_front(self, hidden: torch.Tensor, cos, kv_mgr, phase: str, seq_ids,
+                     sequence_parallel: bool = False):
+        """Cache rows (keys, values) that the fused front end of whole prompts (see attend_fused)
+        writes and reads, None where it does not serve the call."""
+        if phase != PHASE_CTE or not self.qkv_proj.fused:
+            return None
+        norms = self._front_norms(hidden)
+        if not (
+            norms is not None
+            and self.clip_qkv is None
+            and cos is not None
+            and seq_ids is not None
+            and not self.rope_interleaved
+            and self.qk_norm_post_rope is None
+            and self.q_scale_fn is None
+            and not sequence_parallel
+            and self.cp_degree == 1
+            and self.dp_degree == 1
+            and not getattr(kv_mgr, "is_paged", False)
+            and self.kv_shard_degree == 1
+            and not (getattr(kv_mgr, "ring_layers", None)
+                     and kv_mgr.is_ring(self.layer_idx))
+            and (not hidden.is_cuda or self.head_dim in (64, 128))
+            and not (norms and hidden.dtype == torch.float32)
+        ):
+            return None
+        kc, vc = kv_mgr.get_cache(self.layer_idx)
+        kc = kc.data if hasattr(kc, "data") else kc
+        vc = vc.data if hasattr(vc, "data") else vc
+        # fp8 cache: unfused CTE path
+        return (kc, vc) if kc.dtype == hidden.dtype else None
+
     def attend_fused(
         self,
         hidden: torch.Tensor,
@@ -259,52 +291,31 @@ class AttentionBase(nn.Module):
         # kernels per layer vs the unfused path. Right-padded batches are
         # handled without a mask: pad positions (-1) were skipped by the
         # scatter, so causal-by-row-index only ever sees the real prefix.
-        if (
-            phase == PHASE_CTE
-            and self.qkv_proj.fused
-            and norms is not None
-            and self.clip_qkv is None
-            and cos is not None
-            and seq_ids is not None
-            and not self.rope_interleaved
-            and self.qk_norm_post_rope is None
-            and self.q_scale_fn is None
-            and not sequence_parallel
-            and self.cp_degree == 1
-            and self.dp_degree == 1
-            and not getattr(kv_mgr, "is_paged", False)
-            and self.kv_shard_degree == 1
-            and not (getattr(kv_mgr, "ring_layers", None)
-                     and kv_mgr.is_ring(self.layer_idx))
-            and (not hidden.is_cuda or self.head_dim in (64, 128))
-            and not (norms and hidden.dtype == torch.float32)
-        ):
-            kc, vc = kv_mgr.get_cache(self.layer_idx)
-            kc = kc.data if hasattr(kc, "data") else kc
-            vc = vc.data if hasattr(vc, "data") else vc
-            if kc.dtype == hidden.dtype:  # fp8 cache: unfused CTE path below
-                import neuronx_distributed_inference_amd.ops as _ops
+        rows = self.prompt_front(hidden, cos, kv_mgr, phase, seq_ids, sequence_parallel)
+        if rows is not None:
+            kc, vc = rows
+            import neuronx_distributed_inference_amd.ops as _ops
 
-                y = self._qkv_product(hidden)
-                q = _ops.qkv_rope_update(
-                    y, cos, sin, kc, vc, position_ids, seq_ids,
-                    self.num_heads_per_rank, self.num_kv_heads_per_rank, norms=norms or None,
-                    dtype=hidden.dtype,
+            y = self._qkv_product(hidden)
+            q = _ops.qkv_rope_update(
+                y, cos, sin, kc, vc, position_ids, seq_ids,
+                self.num_heads_per_rank, self.num_kv_heads_per_rank, norms=norms or None,
+                dtype=hidden.dtype,
+            )
+            if norms and attention_mask is not None:
+                # by position, which counts the mask's tokens wherever they stand, with
+                # probabilities in 32 bits as on the masked path
+                out = _ops.attention_decode(
+                    q, kc, vc, position_ids, seq_ids=seq_ids, scale=self.scale,
+                    sinks=self.sinks, sliding_window=self.sliding_window,
+                    token_major=True,
                 )
-                if norms and attention_mask is not None:
-                    # by position, which counts the mask's tokens wherever they stand, with
-                    # probabilities in 32 bits as on the masked path
-                    out = _ops.attention_decode(
-                        q, kc, vc, position_ids, seq_ids=seq_ids, scale=self.scale,
-                        sinks=self.sinks, sliding_window=self.sliding_window,
-                        token_major=True,
-                    )
-                else:
-                    out = _ops.attention_prefill_cached(
-                        q, kc, vc, seq_ids, scale=self.scale, sinks=self.sinks,
-                        sliding_window=self.sliding_window, token_major=True,
-                    )
-                return out.transpose(1, 2).reshape(B, S, -1)
+            else:
+                out = _ops.attention_prefill_cached(
+                    q, kc, vc, seq_ids, scale=self.scale, sinks=self.sinks,
+                    sliding_window=self.sliding_window, token_major=True,
+                )
+            return out.transpose(1, 2).reshape(B, S, -1)
         return None
 
     # ------------------------------------------------------------------

@@ -14,6 +14,7 @@ from torch.nn.modules import module as nn_module
 
 from neuronx_distributed_inference_amd import ops
 from neuronx_distributed_inference_amd.modules.attention.attention_base import (
+    PHASE_CTE,
     PHASE_TKG,
     AttentionBase,
     _hooked,
@@ -55,14 +56,43 @@ def fusable(layers, final_norm, h: torch.Tensor, attention_mask, phase: str) -> 
     return True
 
 
+def _plain_mlp(mlp, x: torch.Tensor) -> bool:
+    return (type(mlp) is GatedMLP and not _hooked(mlp) and mlp.fused
+            and mlp.act_mul_fused is ops.silu_mul_fused
+            and plain_linear(mlp.gate_up_proj, x) and plain_linear(mlp.down_proj, x))
+
+
 def _feed_forward(mlp, x: torch.Tensor) -> torch.Tensor:
     """Output of the feed-forward, or its parts of K."""
-    if (type(mlp) is GatedMLP and not _hooked(mlp) and mlp.fused
-            and mlp.act_mul_fused is ops.silu_mul_fused
-            and plain_linear(mlp.gate_up_proj, x) and plain_linear(mlp.down_proj, x)):
+    if _plain_mlp(mlp, x):
         return ops.linear_parts(ops.linear_silu_mul(x, mlp.gate_up_proj.weight),
                                 mlp.down_proj.weight)
     return mlp(x)
+
+
+PROMPT_ROWS = 512       # csrc/tile_gemm.hip takes no more
+
+
+def _short_prompt(layers, final_norm, h, x, cos, sin, kv_mgr, position_ids, seq_ids):
+    """What :func:`run_layers` gives for a short whole prompt of dense layers without q/k norms,
+    its launches made by one native call (csrc/prompt_layers.cpp); None where that does not serve."""
+    if h.numel() > PROMPT_ROWS * h.shape[-1] or not (cos.is_contiguous() and sin.is_contiguous()):
+        return None
+    weights, sizes, numbers = [], [], []
+    for layer, after in zip(layers, layers[1:] + [None]):
+        attn, mlp = layer.fused_parts()
+        qkv = attn.qkv_proj
+        rows = attn.prompt_front(x, cos, kv_mgr, PHASE_CTE, seq_ids)
+        if (rows is None or not attn.use_rope or attn.sinks is not None or attn._front_norms(x)
+                or _hooked(qkv) or not plain_linear(qkv.qkv, x) or not _plain_mlp(mlp, x)):
+            return None
+        norm, following = layer.post_attention_layernorm, after.input_layernorm if after else final_norm
+        weights += [qkv.qkv.weight, attn.o_proj.o_proj.weight, norm.weight, mlp.gate_up_proj.weight,
+                    mlp.down_proj.weight, following.weight, *rows]
+        sizes += [attn.num_heads_per_rank, attn.num_kv_heads_per_rank, int(attn.sliding_window)]
+        numbers += [norm.variance_epsilon, following.variance_epsilon, float(attn.scale)]
+    return ops._require_ext("prompt_layers").prompt_layers(
+        h, x, cos, sin, position_ids, seq_ids, weights, sizes, numbers)
 
 
 def run_layers(layers, final_norm, h: torch.Tensor, cos, sin, kv_mgr, position_ids, phase,
@@ -72,6 +102,12 @@ def run_layers(layers, final_norm, h: torch.Tensor, cos, sin, kv_mgr, position_i
     layers = list(layers)
     if x is None:
         x = layers[0].input_layernorm(h)
+    if (phase == PHASE_CTE and cos is not None and seq_ids is not None
+            and position_ids.dtype == seq_ids.dtype == torch.int32
+            and position_ids.is_contiguous() and seq_ids.is_contiguous()):
+        y = _short_prompt(layers, final_norm, h, x, cos, sin, kv_mgr, position_ids, seq_ids)
+        if y is not None:
+            return y
     for layer, after in zip(layers, layers[1:] + [None]):
         attn, mlp = layer.fused_parts()
         args = (x, cos, sin, kv_mgr, position_ids, phase, attention_mask, seq_ids)

@@ -120,11 +120,18 @@ void step_layout(torch::Tensor pos32, torch::Tensor sid32, torch::Tensor nvalid,
                  torch::Tensor positions, torch::Tensor seq_ids);
 void linear_table(torch::Tensor table, torch::Tensor seq_ids);
 void copy_many(std::vector<torch::Tensor> dst, std::vector<torch::Tensor> src);
+c10::optional<torch::Tensor> prompt_layers(torch::Tensor h, torch::Tensor x, torch::Tensor cos,
+                                           torch::Tensor sin, torch::Tensor positions,
+                                           torch::Tensor seq_ids,
+                                           const std::vector<torch::Tensor>& weights,
+                                           const std::vector<long>& sizes,
+                                           const std::vector<double>& numbers);
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("rms_norm", &rms_norm, "RMSNorm (CDNA4)");
     m.def("rms_norm_fused_add", &rms_norm_fused_add, "RMSNorm + residual add (CDNA4)");
     m.def("add_norm", &add_norm, "residual sum and RMSNorm, of split products too (CDNA4)");
+    m.def("prompt_layers", &prompt_layers, "the launches of plain layers over a short prompt");
     m.def("step_start", &step_start, "embedding rows, first norm, rope rows, int32 positions");
     m.def("slot_mapping", &slot_mapping, "flat cache slots of positions");
     m.def("step_layout", &step_layout, "int32 positions and rows, valid positions of a row");

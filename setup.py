@@ -37,6 +37,7 @@ sources = [
     os.path.join(CSRC, "moe_routed.hip"),
     os.path.join(CSRC, "router_topk.hip"),
     os.path.join(CSRC, "row_topk.hip"),
+    os.path.join(CSRC, "prompt_layers.cpp"),
     os.path.join(CSRC, "lt_gemm.cpp"),
 ]
 

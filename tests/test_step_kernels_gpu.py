@@ -441,3 +441,40 @@ def test_decode_attention_of_many_short_rows(kind, B, Hkv, gq, Sq, D):
     want = torch.cat([run(a, min(a + 20, B)) for a in range(0, B, 20)])
     err = (got.to(F64) - want.to(F64)).norm(dim=-1) / want.to(F64).norm(dim=-1).clamp(min=1e-3)
     assert torch.isfinite(got).all() and err.max() < 2.0 ** -7 and err.mean() < 2.0 ** -8
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("B,S,ragged", [(1, 2, False), (1, 159, False), (2, 70, True), (2, 100, False),
+                                        (2, 101, False)])
+def test_short_prompts_by_one_native_call(B, S, ragged, dtype, monkeypatch):
+    """The native call makes the launches that the layers make one by one: logits and cache to the
+    bit, also for more rows than it takes, an off-cut weight and another row of the cache."""
+    from neuronx_distributed_inference_amd.modules import fused_layer
+
+    lm = _small_llama(dtype)
+    ids = torch.randint(0, 512, (B, S), device="cuda")
+    mask = torch.ones(B, S, dtype=torch.long, device="cuda")
+    if ragged:
+        mask[1, S // 3:] = 0
+    seq = torch.arange(B, device="cuda").flip(0)
+    calls = []
+    native = fused_layer._short_prompt
+
+    def run(rows):
+        monkeypatch.setattr(fused_layer, "PROMPT_ROWS", rows)
+        monkeypatch.setattr(fused_layer, "_short_prompt",
+                            lambda *a: calls.append(native(*a)) or calls[-1])
+        lm.reset()
+        with torch.inference_mode():
+            out = lm(input_ids=ids, attention_mask=mask, seq_ids=seq).logits.clone()
+        return [out] + [t.data.clone() for i in range(2) for t in lm.model.kv_mgr.get_cache(i)]
+
+    a, b = run(200), run(0)
+    assert (calls[0] is not None) == (B * S <= 200) and calls[1] is None
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
+    w = lm.model.layers[1].mlp.down_proj.weight
+    off = torch.empty(w.numel() + 1, dtype=w.dtype, device="cuda")[1:].view_as(w).copy_(w.data)
+    monkeypatch.setattr(w, "data", off)
+    c = run(200)
+    assert calls[2] is None
+    assert all((x.float() - y.float()).norm() <= 0.03 * y.float().norm() for x, y in zip(c, a))
