@@ -257,7 +257,12 @@ class DecoderModel(nn.Module):
                 generate_slot_mapping,
             )
 
-            slots = generate_slot_mapping(block_table, position_ids, self.kv_mgr.block_size)
+            # the GPU kernels take int32: once a step and not once a layer
+            slots = generate_slot_mapping(
+                block_table, position_ids, self.kv_mgr.block_size,
+                torch.int32 if position_ids.is_cuda else torch.int64)
+            if block_table.is_cuda:
+                block_table = block_table.to(torch.int32).contiguous()
             self.kv_mgr.set_step_context(block_table, slots)
         from neuronx_distributed_inference_amd.parallel import state as _ps
 

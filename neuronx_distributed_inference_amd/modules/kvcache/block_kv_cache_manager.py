@@ -177,7 +177,7 @@ class RecurrentStateManager(nn.Module):
 
 
 def generate_slot_mapping(block_table: torch.Tensor, positions: torch.Tensor,
-                          block_size: int) -> torch.Tensor:
+                          block_size: int, dtype=torch.int64) -> torch.Tensor:
     """In-graph slot-mapping computation (ref
     `block_kv_cache_manager.py:376-430`): positions (B,S) + per-sequence
     block table (B, max_blocks) -> flat slots (B*S,). Negative positions
@@ -185,7 +185,7 @@ def generate_slot_mapping(block_table: torch.Tensor, positions: torch.Tensor,
     if (block_table.shape[1] > 0 and positions.dim() == 2
             and block_table.shape[0] >= positions.shape[0]
             and ops._index(block_table, positions)):
-        return ops.slot_mapping(block_table, positions, block_size)
+        return ops.slot_mapping(block_table, positions, block_size, dtype)
     valid = positions >= 0
     pos = positions.clamp(min=0)
     blk = (pos // block_size).clamp(max=block_table.shape[1] - 1)
@@ -193,4 +193,4 @@ def generate_slot_mapping(block_table: torch.Tensor, positions: torch.Tensor,
     blocks = torch.gather(block_table.long(), 1, blk.long())
     slots = blocks * block_size + off
     slots = torch.where(valid & (blocks >= 0), slots, torch.full_like(slots, -1))
-    return slots.flatten()
+    return slots.flatten().to(dtype)

@@ -370,9 +370,9 @@ def step_start_takes(ids, positions, seq_ids, table, cos_table) -> bool:
             and cos_table.device == ids.device and cos_table.shape[1] % 4 == 0)
 
 
-def slot_mapping(block_table, positions, block_size: int):
+def slot_mapping(block_table, positions, block_size: int, dtype=torch.int64):
     """Flat cache slots (B*S,) of (B, S) positions under (B, pages) tables, -1 for none."""
-    slots = torch.empty(positions.numel(), dtype=torch.int64, device=positions.device)
+    slots = torch.empty(positions.numel(), dtype=dtype, device=positions.device)
     _require_ext("slot_mapping").slot_mapping(slots, block_table, positions, block_size)
     return slots
 

@@ -73,15 +73,15 @@ __global__ __launch_bounds__(1024) void step_start_kernel(
 // Flat cache slots of positions: page of the sequence's table * block size + offset, -1 for
 // padding (negative positions) and missing pages; positions past the table count into its last
 // page, as offsets do.
-template <typename TT, typename P>
+template <typename O, typename TT, typename P>
 __global__ __launch_bounds__(256) void slot_mapping_kernel(
-    long* __restrict__ slots, const TT* __restrict__ table, const P* __restrict__ positions,
+    O* __restrict__ slots, const TT* __restrict__ table, const P* __restrict__ positions,
     const long n, const int S, const long cols, const long block_size) {
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     const long p = positions[i], pos = max(p, 0l);
     const long page = table[i / S * cols + min(pos / block_size, cols - 1)];
-    slots[i] = p >= 0 && page >= 0 ? page * block_size + pos % block_size : -1;
+    slots[i] = (O)(p >= 0 && page >= 0 ? page * block_size + pos % block_size : -1);
 }
 
 // int32 positions and cache rows, and the number of valid positions of a row. One workgroup a row.
@@ -216,20 +216,27 @@ void slot_mapping(torch::Tensor slots, torch::Tensor table, torch::Tensor positi
                   long block_size) {
     TORCH_CHECK(whole(table) && whole(positions) && table.dim() == 2 && positions.dim() == 2 &&
                 table.size(0) >= positions.size(0) && table.size(1) > 0 && block_size > 0 &&
-                on(slots, at::kLong) && slots.numel() == positions.numel(), "slot_mapping");
+                whole(slots) && slots.numel() == positions.numel(), "slot_mapping");
     const long n = positions.numel();
     if (n == 0) return;
     auto stream = at::hip::getCurrentHIPStream();
     const bool t64 = table.scalar_type() == at::kLong, p64 = positions.scalar_type() == at::kLong;
-#define SLOTS(TT, P)                                                                               \
-    hipLaunchKernelGGL((slot_mapping_kernel<TT, P>), dim3((unsigned)((n + 255) / 256)), dim3(256), \
-                       0, stream, slots.data_ptr<long>(), table.data_ptr<TT>(),                    \
+    const bool o64 = slots.scalar_type() == at::kLong;
+#define SLOTS(O, TT, P)                                                                            \
+    hipLaunchKernelGGL((slot_mapping_kernel<O, TT, P>), dim3((unsigned)((n + 255) / 256)),         \
+                       dim3(256), 0, stream, slots.data_ptr<O>(), table.data_ptr<TT>(),            \
                        positions.data_ptr<P>(), n, (int)positions.size(1), table.size(1),          \
                        block_size)
-    if (t64 && p64) SLOTS(long, long);
-    else if (t64) SLOTS(long, int);
-    else if (p64) SLOTS(int, long);
-    else SLOTS(int, int);
+#define SLOTS_O(TT, P)                                                                             \
+    do {                                                                                           \
+        if (o64) SLOTS(long, TT, P);                                                               \
+        else SLOTS(int, TT, P);                                                                    \
+    } while (0)
+    if (t64 && p64) SLOTS_O(long, long);
+    else if (t64) SLOTS_O(long, int);
+    else if (p64) SLOTS_O(int, long);
+    else SLOTS_O(int, int);
+#undef SLOTS_O
 #undef SLOTS
     HIP_CHECK_KERNEL();
 }

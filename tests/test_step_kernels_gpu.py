@@ -261,9 +261,10 @@ def test_slots_layouts_and_tables(tdt, pdt):
     for B, S, M, bs in ((1, 1, 1, 1), (3, 300, 5, 7), (65, 2, 9, 64)):
         table = torch.randint(-1, 1000, (B + 1, M)).to(tdt)
         pos = torch.randint(-4, M * bs + 9, (B, S)).to(pdt)
-        got = generate_slot_mapping(table.cuda(), pos.cuda(), bs)
-        assert got.dtype == torch.int64
-        assert torch.equal(got.cpu(), generate_slot_mapping(table, pos, bs))
+        for out in (torch.int64, torch.int32):
+            got = generate_slot_mapping(table.cuda(), pos.cuda(), bs, out)
+            assert got.dtype == out
+            assert torch.equal(got.cpu(), generate_slot_mapping(table, pos, bs, out))
         seq = torch.randint(-1, 7, (B,)).to(tdt)
         a, b = StepLayout(pos.cuda(), seq.cuda()), StepLayout(pos, seq)
         for n in ("positions", "seq_ids", "nvalid"):
