@@ -226,13 +226,17 @@ def _linear(x: torch.Tensor, weight: torch.Tensor,
 def plain_linear(mod: nn.Module, x: torch.Tensor) -> bool:
     """Whether calling the module on x is no more than x @ weight^T in 16 bits on the GPU, so that
     a fused kernel may stand for it: no bias, 8-bit weight, tensor parallelism, hook or subclass."""
-    return (type(mod) in (ColumnParallelLinear, RowParallelLinear)
-            and mod.tp_degree == 1 and mod._group is None
+    if type(mod) not in (ColumnParallelLinear, RowParallelLinear):
+        return False
+    # (asked for every product of a step: the dicts themselves, not the search through them)
+    own, params = mod.__dict__, mod._parameters
+    weight = params.get("weight")
+    return (own["tp_degree"] == 1 and own["_group"] is None
             and ps.get_tensor_model_parallel_size() == 1
-            and mod.bias is None and not getattr(mod, "fp8", False)
+            and params.get("bias") is None and own.get("bias") is None and not own.get("fp8", False)
             and not (mod._forward_hooks or mod._forward_pre_hooks)
             and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16)
-            and mod.weight.dtype == x.dtype)
+            and weight is not None and weight.dtype == x.dtype)
 
 
 class ColumnParallelLinear(nn.Module):

@@ -479,3 +479,25 @@ def test_short_prompts_by_one_native_call(B, S, ragged, dtype, monkeypatch):
     c = run(200)
     assert calls[2] is None
     assert all((x.float() - y.float()).norm() <= 0.03 * y.float().norm() for x, y in zip(c, a))
+
+
+@pytest.mark.parametrize("E", [1, 8, 63, 64, 65, 128, 200, 257, 512, 513, 1000])
+@pytest.mark.parametrize("kind", ["normal", "ties", "masked"])
+def test_router_topk_of_any_width(E, kind):
+    """Choices and their order against torch's stable sort, ties by the lowest index; masked logits
+    (-inf, the type's lowest) are not chosen while others are left."""
+    k = min(8, E)
+    x = torch.randn(333, E, device="cuda")
+    if kind == "ties":
+        x = torch.randint(0, 3, (333, E), device="cuda").float()
+    if kind == "masked":
+        x[:, k:] = torch.where(torch.rand(333, E - k, device="cuda") < 0.5, x[:, k:],
+                               torch.finfo(torch.float32).min)
+        x[:, E - 1 if E > k else 0] = -float("inf") if E > k else x[:, 0]
+    vals = torch.empty(333, k, device="cuda")
+    idx = torch.empty(333, k, dtype=torch.long, device="cuda")
+    ops._C.router_topk(vals, idx, x, k, 0, 0, 0)
+    top, order = x.sort(dim=-1, descending=True, stable=True)
+    assert torch.equal(idx, order[:, :k])
+    want = torch.softmax(top[:, :k].double(), -1)
+    assert ((vals - want).abs() < 1e-6).all()
