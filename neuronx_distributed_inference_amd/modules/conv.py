@@ -42,6 +42,9 @@ class CausalShortConv(nn.Module):
         """x (B,S,C). Reads the carried tail, then advances it by this
         step's inputs (two launches: every token of the step must have read
         the old tail before it is overwritten)."""
+        if x.is_cuda and x.shape[1] == 1 and self.taps > 1:
+            return seqmix.short_conv_step(x, self.weight, tail, step, self.activation,
+                                          self.residual, out_dtype, bias=self.bias)
         y = seqmix.short_conv(x, self.weight, tail, step, self.activation,
                               self.residual, out_dtype, bias=self.bias)
         if self.taps > 1:

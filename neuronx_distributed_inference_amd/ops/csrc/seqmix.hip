@@ -267,6 +267,36 @@ __global__ void short_conv_commit_kernel(const TIn* __restrict__ x, long xs,
     }
 }
 
+// Single tokens: conv and new tail in one pass, a thread a (row, channel), whose tail no other
+// reads. Bound by launches: 48 rows, conv and commit apart and now, 744 -> 715 us for a step with two
+// convolutions a layer (4 layers).
+template <typename TIn, typename TOut>
+__global__ void short_conv_step_kernel(const TIn* __restrict__ x, long xs,
+                                       const float* __restrict__ w, float* __restrict__ tail,
+                                       const int* __restrict__ pos, const int* __restrict__ seq,
+                                       TOut* __restrict__ y, int B, int C, int taps, int act_silu,
+                                       int residual, const float* __restrict__ bias) {
+    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= (long)B * C) return;
+    const int c = idx % C, b = idx / C, R = taps - 1;
+    const int p = pos[b], slot = seq[b];
+    if (p < 0 || slot < 0) { stf<TOut>(y + idx, 0.f); return; }
+    const float cur = ldf<TIn>(x + (long)b * xs + c);
+    const float* wr = w + (long)c * taps;
+    float* tr = tail + (long)slot * R * C + c;
+    float acc = bias ? bias[c] : 0.f;
+    for (int j = 0; j < R; ++j) {
+        const float v = p - R + j < 0 ? 0.f : tr[(long)j * C];
+        acc += wr[j] * v;
+        if (j > 0) tr[(long)(j - 1) * C] = v;
+    }
+    acc += wr[R] * cur;
+    if (R > 0) tr[(long)(R - 1) * C] = cur;
+    if (act_silu) acc = acc * sigmoidf_(acc);
+    if (residual) acc += cur;
+    stf<TOut>(y + idx, acc);
+}
+
 // ------------------------------------------------------------ paged KV write
 template <typename T>
 __global__ void paged_kv_write_kernel(T* __restrict__ kc, T* __restrict__ vc,
@@ -5393,6 +5423,23 @@ int nx_short_conv(const void* x, long xs, int x_bf16, const float* w, const floa
     else if (y_bf16) SC(float, bf16);
     else SC(float, float);
 #undef SC
+    return (int)hipGetLastError();
+}
+
+int nx_short_conv_step(const void* x, long xs, int x_bf16, const float* w, float* tail,
+                       const int* pos, const int* seq, void* y, int y_bf16, int B, int C, int taps,
+                       int act_silu, int residual, const float* bias, hipStream_t st) {
+    const long total = (long)B * C;
+    if (total <= 0) return 0;
+    if (taps < 1) return -1;
+    dim3 grid((unsigned)((total + 255) / 256)), block(256);
+#define SCS(TI, TO) short_conv_step_kernel<TI, TO><<<grid, block, 0, st>>>( \
+        (const TI*)x, xs, w, tail, pos, seq, (TO*)y, B, C, taps, act_silu, residual, bias)
+    if (x_bf16 && y_bf16) SCS(bf16, bf16);
+    else if (x_bf16) SCS(bf16, float);
+    else if (y_bf16) SCS(float, bf16);
+    else SCS(float, float);
+#undef SCS
     return (int)hipGetLastError();
 }
 

@@ -247,6 +247,20 @@ def short_conv(x, w, tail, step: StepLayout, activation: str = "none",
                           activation, residual, out_dtype, bias)
 
 
+def short_conv_step(x, w, tail, step: StepLayout, activation: str = "none",
+                    residual: bool = False, out_dtype=torch.float32, bias=None):
+    """short_conv and short_conv_commit of single tokens (S = 1), in one launch. GPU only."""
+    lib = _load()
+    B, S, C = x.shape
+    assert S == 1 and tail.dtype == torch.float32 and tail.is_contiguous()
+    y = torch.empty(B, S, C, dtype=out_dtype, device=x.device)
+    _check(lib.nx_short_conv_step(
+        _p(x), ctypes.c_long(_rows_view(x)), _is_bf16(x), _p(_f32(w)), _p(tail), _p(step.positions),
+        _p(step.seq_ids), _p(y), _is_bf16(y), B, C, w.shape[1], int(activation == "silu"),
+        int(residual), _p(None if bias is None else _f32(bias)), _stream()), "short_conv_step")
+    return y
+
+
 def short_conv_commit(x, tail, step: StepLayout):
     if x.is_cuda:
         lib = _load()

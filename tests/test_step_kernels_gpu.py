@@ -501,3 +501,27 @@ def test_router_topk_of_any_width(E, kind):
     assert torch.equal(idx, order[:, :k])
     want = torch.softmax(top[:, :k].double(), -1)
     assert ((vals - want).abs() < 1e-6).all()
+
+
+@pytest.mark.parametrize("xd,yd", [(torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16),
+                                   (torch.float32, torch.float32)])
+@pytest.mark.parametrize("taps,silu,residual,bias", [(2, False, True, False), (4, True, False, True), (7, False, False, False)])
+def test_short_conv_of_single_tokens(taps, silu, residual, bias, xd, yd):
+    """Conv and tail in one launch against the two: the same sums in the same order, to the bit;
+    first tokens, padding rows and rows of other sequences among them."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    B, C = 9, 333
+    x = torch.randn(B, 1, C + 7, device="cuda").to(xd)[..., 3:3 + C]
+    w, tail = torch.randn(C, taps, device="cuda"), torch.randn(12, taps - 1, C, device="cuda")
+    pos = torch.tensor([[0], [1], [2], [3], [50], [-1], [9], [2], [6]], device="cuda")
+    seq = torch.tensor([3, 0, 11, 5, 4, 6, -1, 8, 9], device="cuda")
+    step = seqmix.StepLayout(pos, seq)
+    kw = dict(activation="silu" if silu else "none", residual=residual, out_dtype=yd,
+              bias=torch.randn(C, device="cuda") if bias else None)
+    t0 = tail.clone()
+    want = seqmix.short_conv(x, w, t0, step, **kw)
+    seqmix.short_conv_commit(x, t0, step)
+    t1 = tail.clone()
+    got = seqmix.short_conv_step(x, w, t1, step, **kw)
+    assert torch.equal(got, want) and torch.equal(t0, t1)
