@@ -30,6 +30,7 @@ from neuronx_distributed_inference_amd.modules.attention.attention_base import (
     PHASE_CTE,
     PHASE_TKG,
     _hooked,
+    coarse_rows,
 )
 from neuronx_distributed_inference_amd.modules.fused_layer import fusable, run_layers
 from neuronx_distributed_inference_amd.modules.generation.sampling import (
@@ -278,7 +279,8 @@ class DecoderModel(nn.Module):
         fused = [layer for _, layer in runs]
         may_fuse = (not sp_active and not post_fns
                     and not getattr(self, "eagle3_capture_layers", None)
-                    and type(self).before_layer_run is DecoderModel.before_layer_run)
+                    and type(self).before_layer_run is DecoderModel.before_layer_run
+                    and not coarse_rows(self.dtype, getattr(self.kv_mgr, "dtype", self.dtype)))
         start = self._fused_start(fused, input_ids, position_ids, seq_ids, attention_mask,
                                   phase) if may_fuse else None
         if start is not None:

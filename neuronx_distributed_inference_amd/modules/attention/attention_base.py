@@ -41,6 +41,14 @@ def _hooked(module: nn.Module) -> bool:
     return bool(module._forward_hooks or module._forward_pre_hooks)
 
 
+def coarse_rows(dtype: torch.dtype, cache_dtype: torch.dtype) -> bool:
+    """Whether cache rows are far coarser than the activations they come from (fp16 onto 8 bits).
+    There a rounding left out on the way moves some elements by a whole step of 2^-4, 100 times
+    what it spares, and a decoded token's row would differ from the row that a prompt, whose path
+    rounds after every module, leaves for the same token: such models keep the modules' roundings."""
+    return dtype == torch.float16 and cache_dtype.itemsize == 1
+
+
 class AttentionBase(nn.Module):
     def __init__(self, config, layer_idx: int = 0, rotary: Optional[RotaryEmbedding] = None):
         super().__init__()
@@ -181,10 +189,12 @@ class AttentionBase(nn.Module):
             return (norms[0].weight, norms[1].weight, norms[0].variance_epsilon)
         return None
 
-    def _qkv_product(self, hidden: torch.Tensor) -> torch.Tensor:
+    def _qkv_product(self, hidden: torch.Tensor, cache_dtype: torch.dtype) -> torch.Tensor:
         """Output of the fused q|k|v projection, or its parts of K, which qkv_rope_update adds up
-        (head sizes whose kernel does)."""
+        (head sizes whose kernel does). Rows of fp16 models that are kept in 8 bits are rounded to
+        16 first, see coarse_rows."""
         if (self.head_dim in (32, 64, 128, 256) and plain_linear(self.qkv_proj.qkv, hidden)
+                and not coarse_rows(hidden.dtype, cache_dtype)
                 and not _hooked(self.qkv_proj)):
             return ops.linear_parts(hidden, self.qkv_proj.qkv.weight)
         return self.qkv_proj.qkv(hidden)
@@ -257,13 +267,13 @@ class AttentionBase(nn.Module):
             and self.qk_norm_post_rope is None
             and self.q_scale_fn is None
         ):
-            y = self._qkv_product(hidden)
             import neuronx_distributed_inference_amd.ops as _ops
 
             if paged:
                 kc, vc = kv_mgr.k_caches[self.layer_idx], kv_mgr.v_caches[self.layer_idx]
             else:
                 kc, vc = kv_mgr.get_cache(self.layer_idx)
+            y = self._qkv_product(hidden, kc.dtype)
             wpos = position_ids
             if self.kv_shard_degree > 1:
                 from neuronx_distributed_inference_amd.modules.attention import (
@@ -296,7 +306,7 @@ class AttentionBase(nn.Module):
             kc, vc = rows
             import neuronx_distributed_inference_amd.ops as _ops
 
-            y = self._qkv_product(hidden)
+            y = self._qkv_product(hidden, kc.dtype)
             q = _ops.qkv_rope_update(
                 y, cos, sin, kc, vc, position_ids, seq_ids,
                 self.num_heads_per_rank, self.num_kv_heads_per_rank, norms=norms or None,

@@ -141,7 +141,7 @@ def _small_llama(dtype, layers=2, moe=False, **kw):
     for name, p in lm.model.named_parameters():
         if "norm" in name:
             p.data.uniform_(0.5, 1.5, generator=g)
-        else:
+        elif p.element_size() > 1:                           # (8 bits: a cache)
             p.data.normal_(0, 0.05, generator=g)
     return lm
 
@@ -525,3 +525,25 @@ def test_short_conv_of_single_tokens(taps, silu, residual, bias, xd, yd):
     t1 = tail.clone()
     got = seqmix.short_conv_step(x, w, t1, step, **kw)
     assert torch.equal(got, want) and torch.equal(t0, t1)
+
+
+def test_rows_of_8_bits_keep_the_roundings_on_the_way():
+    """fp16 onto an 8-bit cache: a decoded token leaves the row that the modules one by one leave."""
+    lm = _small_llama("float16", kv_cache_quant=True)
+    ids = torch.randint(0, 512, (2, 40), device="cuda")
+    step = torch.randint(0, 512, (2, 1), device="cuda")
+
+    def run():
+        lm.reset()
+        with torch.inference_mode():
+            lm(input_ids=ids)
+            lm(input_ids=step, position_ids=torch.full((2, 1), 40, device="cuda"))
+        return [t.data[:, :, 40].float() for i in range(2) for t in lm.model.kv_mgr.get_cache(i)]
+
+    got = run()
+    note = [m.register_forward_hook(lambda *a: None) for m in lm.model.modules()]
+    want = run()
+    for h in note:
+        h.remove()
+    for a, b in zip(got, want):
+        assert (a != b).float().mean().item() <= 0.002
