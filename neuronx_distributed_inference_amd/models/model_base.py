@@ -220,6 +220,7 @@ class DecoderModel(nn.Module):
             return None
         if (type(self).embed is not DecoderModel.embed
                 or type(self).prepare_hidden is not DecoderModel.prepare_hidden
+                or "embed" in vars(self) or "prepare_hidden" in vars(self)
                 or type(emb) is not ParallelEmbedding or _hooked(emb) or emb.shard_along_embedding
                 or mappings.ps.get_tensor_model_parallel_size() != 1
                 or type(rot) is not RotaryEmbedding or "get_cos_sin" in vars(rot)):
@@ -280,6 +281,7 @@ class DecoderModel(nn.Module):
         may_fuse = (not sp_active and not post_fns
                     and not getattr(self, "eagle3_capture_layers", None)
                     and type(self).before_layer_run is DecoderModel.before_layer_run
+                    and "before_layer_run" not in vars(self)
                     and not coarse_rows(self.dtype, getattr(self.kv_mgr, "dtype", self.dtype)))
         start = self._fused_start(fused, input_ids, position_ids, seq_ids, attention_mask,
                                   phase) if may_fuse else None

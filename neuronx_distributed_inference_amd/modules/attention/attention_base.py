@@ -37,8 +37,9 @@ PHASE_TKG = "token_generation"
 
 
 def _hooked(module: nn.Module) -> bool:
-    """Whether a hook records or replaces what goes through the module (utils/tensor_capture)."""
-    return bool(module._forward_hooks or module._forward_pre_hooks)
+    """Whether a hook records or replaces what goes through the module (utils/tensor_capture), or
+    the instance has a forward of its own."""
+    return bool(module._forward_hooks or module._forward_pre_hooks) or "forward" in module.__dict__
 
 
 def coarse_rows(dtype: torch.dtype, cache_dtype: torch.dtype) -> bool:

@@ -3,8 +3,9 @@
 Between two products stands one kernel: the residual sum and the norm that follows take the parts
 of K of the output and down projections (``ops.add_norm``), rope and cache write those of q|k|v,
 and gate|up writes its activation. A step of few tokens is a chain of such launches, each waiting
-for the last. The layer's modules keep the weights; they are not called, so a layer with hooks on
-any of them, biases, 8-bit weights, adapters or tensor parallelism keeps the chain of modules.
+for the last. The layer's modules keep the weights; they are not called, so a layer with hooks or a
+forward of its own on any of them, biases, 8-bit weights, adapters or tensor parallelism keeps the
+chain of modules.
 """
 
 from __future__ import annotations
@@ -19,6 +20,7 @@ from neuronx_distributed_inference_amd.modules.attention.attention_base import (
     AttentionBase,
     _hooked,
 )
+from neuronx_distributed_inference_amd.modules.attention.gqa import GroupQueryAttentionO
 from neuronx_distributed_inference_amd.modules.mlp import GatedMLP
 from neuronx_distributed_inference_amd.modules.norm import RMSNorm
 from neuronx_distributed_inference_amd.parallel.layers import plain_linear
@@ -27,6 +29,13 @@ from neuronx_distributed_inference_amd.parallel.layers import plain_linear
 def _plain_norm(norm, h: torch.Tensor) -> bool:
     return (type(norm) is RMSNorm and not _hooked(norm) and norm.weight.dtype == h.dtype
             and norm.weight.is_contiguous() and norm.weight.data_ptr() % 16 == 0)
+
+
+def _as_written(layer) -> bool:
+    """Whether the layer's forward is the one that its fused_parts stands for: a subclass with a
+    forward of its own inherits fused_parts all the same."""
+    owner = next((c for c in type(layer).__mro__ if "fused_parts" in vars(c)), None)
+    return owner is not None and type(layer).forward is owner.forward and not _hooked(layer)
 
 
 def fusable(layers, final_norm, h: torch.Tensor, attention_mask, phase: str) -> bool:
@@ -42,13 +51,13 @@ def fusable(layers, final_norm, h: torch.Tensor, attention_mask, phase: str) -> 
     if not _plain_norm(final_norm, h):
         return False
     for layer in layers:
-        ready = getattr(layer, "fused_parts", None)
-        if ready is None or _hooked(layer):
+        if not _as_written(layer):
             return False
-        attn, mlp = ready()
+        attn, _ = layer.fused_parts()
         if not (isinstance(attn, AttentionBase) and type(attn).forward is AttentionBase.forward
                 and type(attn).attend_fused is AttentionBase.attend_fused
-                and not _hooked(attn) and not _hooked(attn.o_proj)
+                and not _hooked(attn)
+                and type(attn.o_proj) is GroupQueryAttentionO and not _hooked(attn.o_proj)
                 and plain_linear(attn.o_proj.o_proj, h)
                 and _plain_norm(layer.input_layernorm, h)
                 and _plain_norm(layer.post_attention_layernorm, h)):

@@ -547,3 +547,54 @@ def test_rows_of_8_bits_keep_the_roundings_on_the_way():
         h.remove()
     for a, b in zip(got, want):
         assert (a != b).float().mean().item() <= 0.002
+
+
+@pytest.mark.parametrize("moe", [False, True])
+@pytest.mark.parametrize("what", ["layer class", "o_proj class", "layer", "self_attn", "norm", "o_proj",
+                                  "o_proj.o_proj", "qkv", "mlp", "down", "final", "embed_tokens",
+                                  "embed", "prepare_hidden", "before_layer_run"])
+def test_a_forward_of_its_own_is_called(what, moe, monkeypatch):
+    """A module whose forward is not the one that the fused layers stand for (a subclass's, or set
+    on the instance) is called, in the prompt and in the step after it, and its result counts."""
+    if moe and what == "down":
+        pytest.skip("no down projection")
+    lm = _small_llama("bfloat16", moe=moe)
+    model, layer = lm.model, lm.model.layers[1]
+    attn, seen = layer.self_attn, []
+
+    def halved(forward):
+        def run(*a, **kw):
+            seen.append(1)
+            y = forward(*a, **kw)
+            return (y[0] * 0.5, *y[1:]) if isinstance(y, tuple) else y * 0.5
+        return run
+
+    def run():
+        lm.reset()
+        with torch.inference_mode():
+            a = lm(input_ids=ids, position_ids=pos).logits
+            b = lm(input_ids=step, position_ids=torch.full((2, 1), 70, device="cuda")).logits
+        return torch.cat([a, b], dim=1).float()
+
+    ids, step = torch.randint(0, 512, (2, 70), device="cuda"), torch.randint(0, 512, (2, 1), device="cuda")
+    pos = torch.arange(70, device="cuda").repeat(2, 1)
+    start, starts = ops.step_start, []
+    monkeypatch.setattr(ops, "step_start", lambda *a: starts.append(1) or start(*a))
+    plain = run()
+    assert len(starts) == 2                      # nothing here keeps the start kernel away
+    if what.endswith(" class"):
+        mod = layer if what == "layer class" else attn.o_proj
+        base = type(mod)
+        mod.__class__ = type("Own", (base,), {"forward": halved(base.forward)})
+    elif what in ("embed", "prepare_hidden", "before_layer_run"):
+        setattr(model, what, halved(getattr(model, what)))
+    else:
+        mod = {"layer": layer, "self_attn": attn, "norm": layer.post_attention_layernorm,
+               "o_proj": attn.o_proj, "o_proj.o_proj": attn.o_proj.o_proj,
+               "qkv": attn.qkv_proj.qkv, "mlp": layer.mlp,
+               "down": getattr(layer.mlp, "down_proj", None), "final": model.norm,
+               "embed_tokens": model.embed_tokens}[what]
+        mod.forward = halved(mod.forward)
+    own = run()
+    assert len(seen) >= 2
+    assert (own - plain).norm() > 0.05 * plain.norm()
