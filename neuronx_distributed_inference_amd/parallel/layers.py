@@ -23,6 +23,7 @@ import os
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules import module as nn_module
 
 from neuronx_distributed_inference_amd.parallel import mappings, state as ps
 
@@ -225,8 +226,8 @@ def _linear(x: torch.Tensor, weight: torch.Tensor,
 
 def plain_linear(mod: nn.Module, x: torch.Tensor) -> bool:
     """Whether calling the module on x is no more than x @ weight^T in 16 bits on the GPU, so that
-    a fused kernel may stand for it: no bias, 8-bit weight, tensor parallelism, hook, subclass or
-    forward of its own."""
+    a fused kernel may stand for it: no bias, 8-bit weight, tensor parallelism, hook (of its
+    own or of all modules), subclass or forward of its own."""
     if type(mod) not in (ColumnParallelLinear, RowParallelLinear):
         return False
     # (asked for every product of a step: the dicts themselves, not the search through them)
@@ -235,7 +236,8 @@ def plain_linear(mod: nn.Module, x: torch.Tensor) -> bool:
     return (own["tp_degree"] == 1 and own["_group"] is None
             and ps.get_tensor_model_parallel_size() == 1
             and params.get("bias") is None and own.get("bias") is None and not own.get("fp8", False)
-            and not (mod._forward_hooks or mod._forward_pre_hooks or "forward" in own)
+            and not (mod._forward_hooks or mod._forward_pre_hooks or "forward" in own
+                     or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks)
             and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16)
             and weight is not None and weight.dtype == x.dtype)
 

@@ -598,3 +598,18 @@ def test_a_forward_of_its_own_is_called(what, moe, monkeypatch):
     own = run()
     assert len(seen) >= 2
     assert (own - plain).norm() > 0.05 * plain.norm()
+
+
+def test_hooks_of_all_modules_see_the_qkv_projection():
+    lm = _small_llama("bfloat16")
+    ids = torch.randint(0, 512, (2, 70), device="cuda")
+    seen = []
+    h = torch.nn.modules.module.register_module_forward_hook(lambda m, *a: seen.append(m))
+    try:
+        with torch.inference_mode():
+            lm(input_ids=ids)
+            lm(input_ids=ids[:, :1], position_ids=torch.full((2, 1), 70, device="cuda"))
+    finally:
+        h.remove()
+    for layer in lm.model.layers:
+        assert sum(m is layer.self_attn.qkv_proj.qkv for m in seen) == 2
