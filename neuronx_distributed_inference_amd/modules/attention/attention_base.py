@@ -190,13 +190,12 @@ class AttentionBase(nn.Module):
             return (norms[0].weight, norms[1].weight, norms[0].variance_epsilon)
         return None
 
-    def _qkv_product(self, hidden: torch.Tensor, cache_dtype: torch.dtype) -> torch.Tensor:
-        """Output of the fused q|k|v projection, or its parts of K, which qkv_rope_update adds up
-        (head sizes whose kernel does). Rows of fp16 models that are kept in 8 bits are rounded to
-        16 first, see coarse_rows."""
-        if (self.head_dim in (32, 64, 128, 256) and plain_linear(self.qkv_proj.qkv, hidden)
-                and not coarse_rows(hidden.dtype, cache_dtype)
-                and not _hooked(self.qkv_proj)):
+    def _qkv_product(self, hidden: torch.Tensor, cos, sin, kc, vc) -> torch.Tensor:
+        """Output of the fused q|k|v projection, or its parts of K, where qkv_rope_update adds them
+        up. Rows of fp16 models that are kept in 8 bits are rounded to 16 first, see coarse_rows."""
+        if (plain_linear(self.qkv_proj.qkv, hidden) and not _hooked(self.qkv_proj)
+                and not coarse_rows(hidden.dtype, kc.dtype)
+                and ops.rope_takes_parts(cos, sin, kc, vc)):
             return ops.linear_parts(hidden, self.qkv_proj.qkv.weight)
         return self.qkv_proj.qkv(hidden)
 
@@ -274,7 +273,7 @@ class AttentionBase(nn.Module):
                 kc, vc = kv_mgr.k_caches[self.layer_idx], kv_mgr.v_caches[self.layer_idx]
             else:
                 kc, vc = kv_mgr.get_cache(self.layer_idx)
-            y = self._qkv_product(hidden, kc.dtype)
+            y = self._qkv_product(hidden, cos, sin, kc, vc)
             wpos = position_ids
             if self.kv_shard_degree > 1:
                 from neuronx_distributed_inference_amd.modules.attention import (
@@ -307,7 +306,7 @@ class AttentionBase(nn.Module):
             kc, vc = rows
             import neuronx_distributed_inference_amd.ops as _ops
 
-            y = self._qkv_product(hidden, kc.dtype)
+            y = self._qkv_product(hidden, cos, sin, kc, vc)
             q = _ops.qkv_rope_update(
                 y, cos, sin, kc, vc, position_ids, seq_ids,
                 self.num_heads_per_rank, self.num_kv_heads_per_rank, norms=norms or None,

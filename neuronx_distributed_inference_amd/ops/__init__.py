@@ -687,6 +687,14 @@ def topk_topp_sample(logits, top_k, top_p, temperature, rand, global_topk: int =
     return ref.topk_topp_sample(logits, top_k, top_p, temperature, rand, global_topk)
 
 
+def rope_takes_parts(cos, sin, k_cache, v_cache) -> bool:
+    """Whether qkv_rope_update adds up the parts of a split product here: its kernel of 16-byte
+    pieces does, for heads of these sizes and rows that start on 16 bytes."""
+    D = k_cache.shape[3]
+    return D in (32, 64, 128, 256) and D <= cos.shape[-1] and not any(
+        t.data_ptr() % 16 for t in (k_cache, v_cache, cos, sin))
+
+
 def qkv_rope_update(qkv, cos, sin, k_cache, v_cache, positions, seq_ids, Hq, Hkv,
                     norms=None, slots=None, dtype=None):
     """Fused qkv-GEMM output -> RoPE(q,k) -> cache write(k,v) -> q (B,Hq,S,D).

@@ -23,7 +23,7 @@ void flash_prefill_cached(torch::Tensor out, torch::Tensor q, torch::Tensor k_ca
 // that, key and value cache rows; sizes: 3 a layer, query heads, KV heads, window; numbers: 3 a
 // layer, the norms' eps and the scale. h (B, S, H), the residual stream, is updated; x is its
 // norm. The normed output, or nothing, with nothing done, where a product is not the tiled
-// kernel's.
+// kernel's or rope does not take its parts.
 c10::optional<torch::Tensor> prompt_layers(torch::Tensor h, torch::Tensor x, torch::Tensor cos,
                                            torch::Tensor sin, torch::Tensor positions,
                                            torch::Tensor seq_ids,
@@ -48,8 +48,9 @@ c10::optional<torch::Tensor> prompt_layers(torch::Tensor h, torch::Tensor x, tor
                 (size_t)w[j].data_ptr() % 16)
                 return c10::nullopt;
         if (w[0].size(0) != (Hq + 2 * Hkv) * D || w[0].size(1) != H || w[1].size(0) != H ||
-            w[1].size(1) != Hq * D || w[3].size(1) != H || w[4].size(0) != H ||
-            2 * w[4].size(1) != w[3].size(0) || (size_t)x.data_ptr() % 16 ||
+            w[1].size(1) != Hq * D || cos.size(-1) < D ||
+            ((size_t)cos.data_ptr() | (size_t)sin.data_ptr()) % 16 || w[3].size(1) != H ||
+            w[4].size(0) != H || 2 * w[4].size(1) != w[3].size(0) || (size_t)x.data_ptr() % 16 ||
             !tile_gemm_splits(rows, w[0].size(0), H, false) ||
             !tile_gemm_splits(rows, H, Hq * D, false) ||
             !tile_gemm_splits(rows, w[3].size(0), H, true) ||
