@@ -393,12 +393,11 @@ def copy_many(dst, src) -> None:
 
 def add_norm(y: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
              eps: float) -> torch.Tensor:
-    """RMS norm of residual + y; residual becomes the sum. y: of residual's shape, or parts of a
-    split product (linear_parts)."""
+    """RMS norm of residual + y; residual becomes the sum. y: of residual's shape and any layout
+    (what a module of the program's own hands out), or parts of a split product (linear_parts)."""
     out = torch.empty_like(residual)
-    _require_ext("add_norm").add_norm(
-        out, residual, y.reshape(y.shape[0], -1, y.shape[-1]) if y.dim() > residual.dim() else y,
-        weight, eps)
+    y = y.reshape(y.shape[0], -1, y.shape[-1]) if y.dim() > residual.dim() else _aligned(y)
+    _require_ext("add_norm").add_norm(out, residual, y, weight, eps)
     return out
 
 

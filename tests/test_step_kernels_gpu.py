@@ -646,3 +646,39 @@ def test_rows_that_start_off_16_bytes(dtype):
     for got in (rope, cache):
         for a, b in zip(got, want):
             assert (a - b).norm() <= tol * b.norm()
+
+
+@pytest.mark.parametrize("how", ["rows apart", "transposed", "off 16 bytes"])
+def test_feed_forward_results_of_any_layout(how):
+    """A feed-forward of the program's own may hand out rows apart, transposed or off 16 bytes."""
+    lm = _small_llama("bfloat16")
+    ids = torch.randint(0, 512, (2, 70), device="cuda")
+
+    class Own(torch.nn.Module):
+        def __init__(self, mlp):
+            super().__init__()
+            self.mlp = mlp
+
+        def forward(self, x, sequence_parallel=False):
+            y = self.mlp(x)
+            B, S, H = y.shape
+            if how == "rows apart":
+                z = y.new_empty(B, S, 2 * H)[..., :H]
+            elif how == "transposed":
+                z = y.new_empty(H, S, B).permute(2, 1, 0)
+            else:
+                z = y.new_empty(y.numel() + 1)[1:].view(B, S, H)
+            return z.copy_(y)
+
+    def run():
+        lm.reset()
+        with torch.inference_mode():
+            a = lm(input_ids=ids).logits
+            b = lm(input_ids=ids[:, :1], position_ids=torch.full((2, 1), 70, device="cuda")).logits
+        return a.float(), b.float()
+
+    want = run()
+    for layer in lm.model.layers:
+        layer.mlp = Own(layer.mlp)
+    for a, b in zip(run(), want):
+        assert (a - b).norm() <= 0.03 * b.norm()
