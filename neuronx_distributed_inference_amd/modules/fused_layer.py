@@ -85,7 +85,8 @@ PROMPT_ROWS = 512       # csrc/tile_gemm.hip takes no more
 def _short_prompt(layers, final_norm, h, x, cos, sin, kv_mgr, position_ids, seq_ids):
     """What :func:`run_layers` gives for a short whole prompt of dense layers without q/k norms,
     its launches made by one native call (csrc/prompt_layers.cpp); None where that does not serve."""
-    if h.numel() > PROMPT_ROWS * h.shape[-1] or not (cos.is_contiguous() and sin.is_contiguous()):
+    if h.numel() > PROMPT_ROWS * h.shape[-1] or not (cos.is_contiguous() and sin.is_contiguous()
+                                                     and ops.tiles_enabled()):
         return None
     weights, sizes, numbers = [], [], []
     for layer, after in zip(layers, layers[1:] + [None]):

@@ -303,10 +303,16 @@ def skinny_gemm5_fp8(x2: torch.Tensor, wq_u8: torch.Tensor,
     return y
 
 
+def tiles_enabled() -> bool:
+    """Whether 16-bit products may take the tiled kernel: not under NXDI_DISABLE_SG5=1, which leaves
+    them to hipBLASLt, nor where lt_linear_enabled leaves them to torch."""
+    return os.environ.get("NXDI_DISABLE_SG5") != "1" and lt_linear_enabled()
+
+
 def _tile_takes(x2: torch.Tensor, weight: torch.Tensor, glu: bool = False) -> int:
     """Parts of K that the tiled product (csrc/tile_gemm.hip) plans for x2 @ weight^T, 0 where it
     does not take it."""
-    if not (x2.is_cuda and x2.dtype in (torch.bfloat16, torch.float16) and x2.dtype == weight.dtype
+    if not (tiles_enabled() and x2.is_cuda and x2.dtype in (torch.bfloat16, torch.float16) and x2.dtype == weight.dtype
             and x2.is_contiguous() and weight.is_contiguous()
             and (x2.data_ptr() | weight.data_ptr()) % 16 == 0):
         return 0
@@ -459,8 +465,7 @@ def decode_linear(x: torch.Tensor, weight: torch.Tensor, bias=None) -> torch.Ten
     x2 = x.reshape(-1, shape[-1]).contiguous()
     M, K = x2.shape
     N = weight.shape[0]
-    if not _tile_takes(x2, weight) or os.environ.get("NXDI_DISABLE_SG5") == "1" \
-            or (bias is not None and not bias.is_contiguous()):
+    if not _tile_takes(x2, weight) or (bias is not None and not bias.is_contiguous()):
         return lt_linear(x, weight, bias)
     key = (M, N, K, bias is not None, x.dtype)
     choice = _sg5_state["choice"].get(key)

@@ -682,3 +682,29 @@ def test_feed_forward_results_of_any_layout(how):
         layer.mlp = Own(layer.mlp)
     for a, b in zip(run(), want):
         assert (a - b).norm() <= 0.03 * b.norm()
+
+
+@pytest.mark.parametrize("switch", ["NXDI_DISABLE_SG5", "NXDI_DISABLE_HIPBLASLT"])
+@pytest.mark.parametrize("moe", [False, True])
+def test_switches_of_the_products_hold_in_fused_layers(switch, moe, monkeypatch):
+    """Neither the tiled product nor the native prompt, which is made of it, under either switch."""
+    lm = _small_llama("bfloat16", moe=moe)
+    ids = torch.randint(0, 512, (2, 70), device="cuda")
+
+    def run():
+        lm.reset()
+        with torch.inference_mode():
+            a = lm(input_ids=ids).logits
+            b = lm(input_ids=ids[:, :1], position_ids=torch.full((2, 1), 70, device="cuda")).logits
+        return a.float(), b.float()
+
+    want = run()
+    calls = []
+    for name in ("tile_gemm", "prompt_layers"):
+        monkeypatch.setattr(ops._C, name, lambda *a, _n=name, **kw: calls.append(_n))
+    monkeypatch.setitem(ops._lt_state, "enabled", None)
+    monkeypatch.setenv(switch, "1")
+    got = run()
+    assert not calls
+    for a, b in zip(got, want):
+        assert (a - b).norm() <= 0.03 * b.norm()
