@@ -1255,12 +1255,13 @@ __global__ void __launch_bounds__(256, 2) window_flash_kernel(const WfArgs a) {
         if (plain) {
             const float d0 = (float)(qpos - k0 - 4 * half);
             if (a.r1 && a.r2) {
-                const float b0 = fmaf(a2, d0, 1.f);
+                // (of the whole distance, which is exact: 1 + a2 * d0 less a2 * a key's place in
+                // the tile would cancel at the near keys)
 #pragma unroll
                 for (int nn = 0; nn < 2; ++nn)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        const float y = fmaf(-a2, (float)(nn * 32 + 8 * (r >> 2) + (r & 3)), b0);
+                        const float y = fmaf(a2, d0 - (float)(nn * 32 + 8 * (r >> 2) + (r & 3)), 1.f);
                         s[nn][r] = fmaf(s[nn][r], c, -a1l * __builtin_amdgcn_logf(y));
                     }
             } else if (a.r1) {

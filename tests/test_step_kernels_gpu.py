@@ -708,3 +708,14 @@ def test_switches_of_the_products_hold_in_fused_layers(switch, moe, monkeypatch)
     assert not calls
     for a, b in zip(got, want):
         assert (a - b).norm() <= 0.03 * b.norm()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("S", [70, 300])
+def test_windowed_attention_under_steep_distances(S, D):
+    """Portions under r2 of 1e5 and more: 1 + r2 * distance is one multiply-add of the whole distance. Made
+    from a tile's first distance less a key's place in it, its sum cancels at the near keys, and
+    what is lost is 59 * r2 of 2^-24: of a key's own 1, an eighth and more."""
+    args = list(_windowed(S, 8, 2, D, 16, 40, dict(window=200)))
+    args[-1] = dict(window=200, r1=torch.linspace(0.1, 0.4, 8), r2=torch.linspace(1e5, 2e5, 8))
+    assert _windowed_error(tuple(args)) < 2.0 ** -8
