@@ -343,9 +343,11 @@ def linear_silu_mul(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 
 def _index(*tensors) -> bool:
-    """Whether all are contiguous int32 or int64 tensors of the current device."""
-    return all(t.is_cuda and t.dtype in (torch.int64, torch.int32) and t.is_contiguous()
-               and t.device.index == torch.cuda.current_device() for t in tensors)
+    """Whether all are contiguous int32 or int64 tensors of the current device, and the kernels over
+    such are there (models of the sequence-mixing library alone load no other)."""
+    return _C is not None and all(
+        t.is_cuda and t.dtype in (torch.int64, torch.int32) and t.is_contiguous()
+        and t.device.index == torch.cuda.current_device() for t in tensors)
 
 
 def step_start(ids, positions, seq_ids, table, cos_table, sin_table, weight, eps: float):
@@ -384,17 +386,19 @@ def slot_mapping(block_table, positions, block_size: int, dtype=torch.int64):
 
 
 def copy_many(dst, src) -> None:
-    """dst[i].copy_(src[i]), in one launch for those that are alike and of the current device."""
+    """dst[i].copy_(src[i]), in one launch for those that are alike and of the current device (where
+    the kernel is there, see _index)."""
     here = torch.cuda.current_device()
     pairs = []
     for d, s in zip(dst, src):
-        if (s.is_cuda and s.device == d.device and d.device.index == here and s.dtype == d.dtype
-                and s.shape == d.shape and s.is_contiguous() and d.is_contiguous()):
+        if (_C is not None and s.is_cuda and s.device == d.device and d.device.index == here
+                and s.dtype == d.dtype and s.shape == d.shape
+                and s.is_contiguous() and d.is_contiguous()):
             pairs.append((d, s))
         else:
             d.copy_(s, non_blocking=True)
     if pairs:
-        _require_ext("copy_many").copy_many(*map(list, zip(*pairs)))
+        _C.copy_many(*map(list, zip(*pairs)))
 
 
 def add_norm(y: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,

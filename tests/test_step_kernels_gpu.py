@@ -719,3 +719,31 @@ def test_windowed_attention_under_steep_distances(S, D):
     args = list(_windowed(S, 8, 2, D, 16, 40, dict(window=200)))
     args[-1] = dict(window=200, r1=torch.linspace(0.1, 0.4, 8), r2=torch.linspace(1e5, 2e5, 8))
     assert _windowed_error(tuple(args)) < 2.0 ** -8
+
+
+def test_sequence_mixing_models_without_the_other_library(monkeypatch):
+    """Step layouts, slots, page tables and the inputs of captured steps of models that load the
+    sequence-mixing library only."""
+    from neuronx_distributed_inference_amd.models.hybrid_base import HybridDecoderModel
+    from neuronx_distributed_inference_amd.modules.kvcache.block_kv_cache_manager import (
+        generate_slot_mapping)
+    from neuronx_distributed_inference_amd.ops.seqmix import StepLayout
+    from neuronx_distributed_inference_amd.runtime.graph_engine import GraphRunner
+
+    monkeypatch.setattr(ops, "_C", None)
+    pos, seq = torch.randint(-2, 90, (3, 5)), torch.tensor([2, -1, 0])
+    table = torch.randint(-1, 40, (3, 6))
+    model = type("M", (), {"max_blocks_per_seq": 7})()
+    model.kv_mgr = type("K", (), {"num_blocks": 10 ** 6, "state": type("S", (), {"num_slots": 8})})()
+
+    def run(dev):
+        a = StepLayout(pos.to(dev), seq.to(dev))
+        return [a.positions, a.seq_ids, a.nvalid,
+                generate_slot_mapping(table.to(dev), pos.to(dev), 16, torch.int32),
+                HybridDecoderModel.begin_step(model, pos.to(dev), seq.to(dev), None).long()]
+
+    for a, b in zip(run("cuda"), run("cpu")):
+        assert a.dtype == b.dtype and torch.equal(a.cpu(), b)
+    step = GraphRunner(lambda x, y: x * 2 + y, (torch.zeros(4, device="cuda"), torch.zeros(4, device="cuda")))
+    x, y = torch.arange(4.0, device="cuda"), torch.ones(4, device="cuda")
+    assert torch.equal(step(x, y), x * 2 + y)
