@@ -1068,9 +1068,12 @@ def moe_routed_experts(x: torch.Tensor, weights: torch.Tensor, idx: torch.Tensor
     else:
         c.moe_routed_glu(h, x, w_gate, w_up, s[0], s[1], tiles, gather, mt, int(gelu))
     cols = min(H, max(256, MOE_WORKSPACE // (4 * rows) // 256 * 256))
-    # with few tiles the down projection's workgroups share them (csrc/moe_routed.hip)
-    few = n // mt * -(-H // 256) <= 512 and cols == H
-    ws = torch.empty(max(rows * cols, 768 * 256 * mt if few else 0), dtype=torch.float32, device=dev)
+    # up to 512 tiles may be shared out to the down projection's 256 workgroups, with a part for each
+    # tile that a workgroup touches (csrc/moe_routed.hip): fewer than workgroups and tiles together
+    wide = -(-H // 256)
+    few = n // mt * wide <= 512 and cols == H
+    shares = 256 + min(512, tiles_max * wide) if few else 0
+    ws = torch.empty(max(rows * cols, shares * 256 * mt), dtype=torch.float32, device=dev)
     c.moe_routed_down(out, ws, h, w_down, s[2], tiles, inv, None if scale_input else weights, mt)
     return out
 

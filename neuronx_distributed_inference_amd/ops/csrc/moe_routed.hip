@@ -661,8 +661,10 @@ void moe_routed_down(torch::Tensor out, torch::Tensor ws, torch::Tensor h, torch
     const long slab = ws.numel() >= rows * N ? N : room;
     const int topk = (int)(inv.numel() / T);
     const int nk = (int)(w_down.size(2) / (s_down.has_value() ? 128 : 64));
-    // shares: of at most 2 * MR_WGS tiles, and so fewer than 3 * MR_WGS of them
-    const bool share = slab == N && ws.numel() >= 3L * MR_WGS * mt * 256;
+    // shares: of at most 2 * MR_WGS tiles (mr_shares); workgroup w's of tile li stands at w + li,
+    // so that there are fewer than tiles and workgroups together
+    const long most = std::min(2L * MR_WGS, (tiles.numel() - 1) / 2 * ((N + 255) / 256));
+    const bool share = slab == N && ws.numel() >= (MR_WGS + most) * mt * 256;
     auto st = at::hip::getCurrentHIPStream();
     for (long c = 0; c < N; c += slab) {
         const int nc = (int)std::min(slab, N - c);

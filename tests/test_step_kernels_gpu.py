@@ -747,3 +747,28 @@ def test_sequence_mixing_models_without_the_other_library(monkeypatch):
     step = GraphRunner(lambda x, y: x * 2 + y, (torch.zeros(4, device="cuda"), torch.zeros(4, device="cuda")))
     x, y = torch.arange(4.0, device="cuda"), torch.ones(4, device="cuda")
     assert torch.equal(step(x, y), x * 2 + y)
+
+
+@pytest.mark.parametrize("T,E,k,H,I,f8", [(1, 8, 2, 4096, 1024, False), (1, 8, 2, 4096, 1024, True),
+                                          (24, 64, 8, 2048, 512, False), (300, 8, 2, 4096, 1088, False)])
+def test_moe_routed_room_for_shares_by_the_tiles(T, E, k, H, I, f8):
+    """The down projection's shares take a place for each workgroup and each tile there can be, as
+    long as those are few, and no more than that."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(T, H, device="cuda", generator=g).bfloat16()
+    wt, idx = torch.softmax(torch.randn(T, E, device="cuda", generator=g), -1).topk(k, dim=-1)
+    w = [(torch.randn(E, *s, device="cuda", generator=g) * 0.05).bfloat16() for s in ((I, H), (I, H), (H, I))]
+    scales = None
+    if f8:
+        w, scales = zip(*[ops.fp8_moe_quantize(v) for v in w])
+    mt = ops._moe_tile_rows(T * k, E, E, H, I, f8)
+    tiles = (T * k + min(T * k, E) * (mt - 1)) // mt
+    products = max(tiles * mt * H, (256 + min(512, tiles * -(-H // 256))) * mt * 256) * 4
+    rest = tiles * mt * I * 2 + T * H * 2 + (1 + 2 * tiles + tiles * mt + T * k) * 4
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    ops.moe_routed_experts(x, wt, idx, *w, scales=scales, num_experts=E)
+    # the allocator leaves up to 1 MB of a block with each of the large tensors (products, h, out)
+    assert torch.cuda.max_memory_allocated() - before <= products + rest + (3 << 20)
