@@ -15,6 +15,7 @@ from __future__ import annotations
 import functools
 import math
 import os
+import time
 from typing import Optional, Tuple
 
 import torch
@@ -412,44 +413,58 @@ def add_norm(y: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
 
 
 def _sg5_autotune(key, x2, weight, bias) -> int:
-    """Returns 0 (= lt/library path) or the winning number of parts of K. Timed
-    over ROTATING weight clones so the stream is cache-cold like the real
-    decode loop (the 256 MB L3 would otherwise hold the whole weight and
-    flip the verdict); x stays hot, which is also realistic."""
-    M, N, K = key[0], key[1], key[2]
+    """Returns 0 (= lt/library path) or the number of parts of K that the tiled
+    kernel plans. Timed over ROTATING weight clones so the stream is cache-cold
+    like the real decode loop (the 256 MB L3 would otherwise hold the whole
+    weight and flip the verdict); x stays hot, which is also realistic. Costs
+    2 to 6 ms a shape beside the 25 to 80 ms of the library's own search. (One
+    part where several are planned was no faster in any shape measured: 1024 to
+    28672 columns, K of 2048 to 14336, 1 to 512 rows.)"""
     n_iter = 12
     # rotate enough copies that successive calls miss L3 (256 MB)
     wbytes = weight.numel() * weight.element_size()
     ncopy = max(2, min(8, int(320e6 // max(wbytes, 1)) + 1))
     try:
         wcopies = [weight] + [weight.clone() for _ in range(ncopy - 1)]
+        busy = torch.empty(1 << 27, dtype=torch.uint8, device=weight.device)
     except torch.cuda.OutOfMemoryError:  # pragma: no cover
-        wcopies = [weight]
+        wcopies, busy = [weight], weight.new_empty(1 << 20)
     results = {}
     torch.cuda.synchronize()
 
     def _time(fn):
+        """GPU time of a call. The calls wait behind a fill that lasts until all are queued: one
+        after the other, products of 10 us would be timed by what the host takes to launch them,
+        which captured steps do not wait for."""
         fn(wcopies[0])  # warm (triggers lt's own tune / LDS attr set)
         torch.cuda.synchronize()
-        t0 = torch.cuda.Event(enable_timing=True)
-        t1 = torch.cuda.Event(enable_timing=True)
-        t0.record()
-        for i in range(n_iter):
-            fn(wcopies[i % len(wcopies)])
-        t1.record()
-        torch.cuda.synchronize()
-        return t0.elapsed_time(t1) / n_iter
+        t = [torch.cuda.Event(enable_timing=True) for _ in range(3)]
+        fills = 32                                       # some 25 us each
+        while True:
+            begin = time.perf_counter()
+            t[0].record()
+            for _ in range(fills):
+                busy.zero_()
+            t[1].record()
+            for i in range(n_iter):
+                fn(wcopies[i % len(wcopies)])
+            t[2].record()
+            host = (time.perf_counter() - begin) * 1e3
+            torch.cuda.synchronize()
+            if t[0].elapsed_time(t[1]) >= host or fills >= 256:
+                return t[1].elapsed_time(t[2]) / n_iter
+            fills *= 4
 
     try:
         results[0] = _time(lambda w: lt_linear(x2, w, bias))
     except Exception:  # noqa: BLE001
         results[0] = float("inf")
-    for sk in sorted({1, _tile_takes(x2, weight)} - {0}):
-        try:
-            results[sk] = _time(lambda w, s=sk: _C.tile_gemm(x2, w, bias, splits=s))
-        except Exception:  # noqa: BLE001
-            results[sk] = float("inf")
-    del wcopies
+    sk = _tile_takes(x2, weight)
+    try:
+        results[sk] = _time(lambda w: _C.tile_gemm(x2, w, bias, splits=sk))
+    except Exception:  # noqa: BLE001
+        results[sk] = float("inf")
+    del wcopies, busy
     choice = min(results, key=results.get)
     # microbench rankings transfer to in-graph steady state with ~±20%
     # error (DVFS + cache state differ): ship the hand-written kernel
@@ -462,8 +477,7 @@ def _sg5_autotune(key, x2, weight, bias) -> int:
 
 
 def decode_linear(x: torch.Tensor, weight: torch.Tensor, bias=None) -> torch.Tensor:
-    """Shape-autotuned decode projection: the tiled kernel (csrc/tile_gemm.hip), in one part of K
-    and in as many as it plans, vs hipBLASLt, winner replayed per shape. Falls through to
+    """Shape-autotuned decode projection: the tiled kernel (csrc/tile_gemm.hip) vs hipBLASLt, winner replayed per shape. Falls through to
     lt_linear for shapes that the tiled kernel does not take."""
     shape = x.shape
     x2 = x.reshape(-1, shape[-1]).contiguous()

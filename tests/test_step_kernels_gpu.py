@@ -772,3 +772,30 @@ def test_moe_routed_room_for_shares_by_the_tiles(T, E, k, H, I, f8):
     ops.moe_routed_experts(x, wt, idx, *w, scales=scales, num_experts=E)
     # the allocator leaves up to 1 MB of a block with each of the large tensors (products, h, out)
     assert torch.cuda.max_memory_allocated() - before <= products + rest + (3 << 20)
+
+
+def test_products_are_chosen_by_the_gpus_time(monkeypatch):
+    """A library call that the host takes 50 us to launch and the GPU 8 to run stays the choice
+    beside a kernel that takes the GPU 25 us or more and is launched at once: captured steps wait
+    for the GPU only."""
+    import time
+
+    M, N, K = 48, 2048, 2048
+    x, w, _, _ = _product(M, N, K, torch.bfloat16)
+    lt, tiled = ops.lt_linear, ops._C.tile_gemm
+
+    def slow_launch(*a):
+        until = time.perf_counter() + 50e-6
+        while time.perf_counter() < until:
+            pass
+        return lt(*a)
+
+    def slow_kernel(*a, **kw):
+        for _ in range(3):
+            y = tiled(*a, **kw)
+        return y
+
+    monkeypatch.setattr(ops, "lt_linear", slow_launch)
+    monkeypatch.setattr(ops._C, "tile_gemm", slow_kernel)
+    monkeypatch.setitem(ops._sg5_state, "choice", {})
+    assert ops._sg5_autotune((M, N, K, False, x.dtype), x, w, None) == 0
