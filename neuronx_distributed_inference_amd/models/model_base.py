@@ -49,6 +49,9 @@ from neuronx_distributed_inference_amd.parallel.layers import (
 
 logger = logging.getLogger("nxdi_amd")
 
+# what ops.step_start does in their place: replaced ones are called
+_LOOKUP, _ROPE = ParallelEmbedding.forward, RotaryEmbedding.get_cos_sin
+
 
 @dataclass
 class ModelOutput:
@@ -194,6 +197,12 @@ class DecoderModel(nn.Module):
                          h_embed: torch.Tensor) -> torch.Tensor:
         return h
 
+    _plain = dict(embed=embed, prepare_hidden=prepare_hidden, before_layer_run=before_layer_run)
+
+    def _own(self, name: str) -> bool:
+        """Whether a subclass, or a program, has put another method in place of the one above."""
+        return getattr(type(self), name) is not DecoderModel._plain[name] or name in vars(self)
+
     def finalize_logits(self, logits: torch.Tensor) -> torch.Tensor:
         """Post-lm_head transform (e.g. a tanh soft cap)."""
         return logits
@@ -218,12 +227,12 @@ class DecoderModel(nn.Module):
         mm = getattr(self, "multimodal_ctx", None)
         if (mm and phase == PHASE_CTE) or getattr(self, "_cos_sin_fn", None) is not None:
             return None
-        if (type(self).embed is not DecoderModel.embed
-                or type(self).prepare_hidden is not DecoderModel.prepare_hidden
-                or "embed" in vars(self) or "prepare_hidden" in vars(self)
-                or type(emb) is not ParallelEmbedding or _hooked(emb) or emb.shard_along_embedding
+        if (self._own("embed") or self._own("prepare_hidden")
+                or type(emb) is not ParallelEmbedding or ParallelEmbedding.forward is not _LOOKUP
+                or _hooked(emb) or emb.shard_along_embedding
                 or mappings.ps.get_tensor_model_parallel_size() != 1
-                or type(rot) is not RotaryEmbedding or "get_cos_sin" in vars(rot)):
+                or type(rot) is not RotaryEmbedding or RotaryEmbedding.get_cos_sin is not _ROPE
+                or "get_cos_sin" in vars(rot)):
             return None
         table = emb.weight
         if not (table.is_cuda and input_ids.is_cuda):
@@ -280,8 +289,7 @@ class DecoderModel(nn.Module):
         fused = [layer for _, layer in runs]
         may_fuse = (not sp_active and not post_fns
                     and not getattr(self, "eagle3_capture_layers", None)
-                    and type(self).before_layer_run is DecoderModel.before_layer_run
-                    and "before_layer_run" not in vars(self)
+                    and not self._own("before_layer_run")
                     and not coarse_rows(self.dtype, getattr(self.kv_mgr, "dtype", self.dtype)))
         start = self._fused_start(fused, input_ids, position_ids, seq_ids, attention_mask,
                                   phase) if may_fuse else None

@@ -56,8 +56,9 @@ class Qwen3MoeDecoderLayer(nn.Module):
         h = self.mlp(h)
         return h, residual
 
+    fused_forward = forward        # what modules/fused_layer.py stands for, of these parts
+
     def fused_parts(self):
-        """What modules/fused_layer.py runs in place of :meth:`forward`."""
         return self.self_attn, self.mlp
 
 

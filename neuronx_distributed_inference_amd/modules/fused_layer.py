@@ -26,16 +26,17 @@ from neuronx_distributed_inference_amd.modules.norm import RMSNorm
 from neuronx_distributed_inference_amd.parallel.layers import plain_linear
 
 
+# what the loop does in their place, by heart: a class whose forward was replaced is not plain
+_FORWARDS = {c: c.forward for c in (AttentionBase, GroupQueryAttentionO, GatedMLP, RMSNorm)}
+
+
+def _plain(module, cls) -> bool:
+    return type(module) is cls and cls.forward is _FORWARDS[cls] and not _hooked(module)
+
+
 def _plain_norm(norm, h: torch.Tensor) -> bool:
-    return (type(norm) is RMSNorm and not _hooked(norm) and norm.weight.dtype == h.dtype
+    return (_plain(norm, RMSNorm) and norm.weight.dtype == h.dtype
             and norm.weight.is_contiguous() and norm.weight.data_ptr() % 16 == 0)
-
-
-def _as_written(layer) -> bool:
-    """Whether the layer's forward is the one that its fused_parts stands for: a subclass with a
-    forward of its own inherits fused_parts all the same."""
-    owner = next((c for c in type(layer).__mro__ if "fused_parts" in vars(c)), None)
-    return owner is not None and type(layer).forward is owner.forward and not _hooked(layer)
 
 
 def fusable(layers, final_norm, h: torch.Tensor, attention_mask, phase: str) -> bool:
@@ -51,13 +52,14 @@ def fusable(layers, final_norm, h: torch.Tensor, attention_mask, phase: str) -> 
     if not _plain_norm(final_norm, h):
         return False
     for layer in layers:
-        if not _as_written(layer):
+        # (a subclass with a forward of its own inherits fused_parts all the same)
+        if getattr(type(layer), "fused_forward", None) is not type(layer).forward or _hooked(layer):
             return False
         attn, _ = layer.fused_parts()
-        if not (isinstance(attn, AttentionBase) and type(attn).forward is AttentionBase.forward
+        if not (isinstance(attn, AttentionBase)
+                and type(attn).forward is _FORWARDS[AttentionBase]
                 and type(attn).attend_fused is AttentionBase.attend_fused
-                and not _hooked(attn)
-                and type(attn.o_proj) is GroupQueryAttentionO and not _hooked(attn.o_proj)
+                and not _hooked(attn) and _plain(attn.o_proj, GroupQueryAttentionO)
                 and plain_linear(attn.o_proj.o_proj, h)
                 and _plain_norm(layer.input_layernorm, h)
                 and _plain_norm(layer.post_attention_layernorm, h)):
@@ -66,7 +68,7 @@ def fusable(layers, final_norm, h: torch.Tensor, attention_mask, phase: str) -> 
 
 
 def _plain_mlp(mlp, x: torch.Tensor) -> bool:
-    return (type(mlp) is GatedMLP and not _hooked(mlp) and mlp.fused
+    return (_plain(mlp, GatedMLP) and mlp.fused
             and mlp.act_mul_fused is ops.silu_mul_fused
             and plain_linear(mlp.gate_up_proj, x) and plain_linear(mlp.down_proj, x))
 

@@ -228,7 +228,7 @@ def plain_linear(mod: nn.Module, x: torch.Tensor) -> bool:
     """Whether calling the module on x is no more than x @ weight^T in 16 bits on the GPU, so that
     a fused kernel may stand for it: no bias, 8-bit weight, tensor parallelism, hook (of its
     own or of all modules), subclass or forward of its own."""
-    if type(mod) not in (ColumnParallelLinear, RowParallelLinear):
+    if _FORWARDS.get(type(mod)) is not type(mod).forward:
         return False
     # (asked for every product of a step: the dicts themselves, not the search through them)
     own, params = mod.__dict__, mod._parameters
@@ -373,6 +373,10 @@ class RowParallelLinear(nn.Module):
         if self.bias is not None:
             y = y + self.bias
         return y
+
+
+# as written: a class whose forward was replaced is not plain
+_FORWARDS = {c: c.forward for c in (ColumnParallelLinear, RowParallelLinear)}
 
 
 class ParallelEmbedding(nn.Module):

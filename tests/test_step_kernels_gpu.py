@@ -550,12 +550,13 @@ def test_rows_of_8_bits_keep_the_roundings_on_the_way():
 
 
 @pytest.mark.parametrize("moe", [False, True])
-@pytest.mark.parametrize("what", ["layer class", "o_proj class", "layer", "self_attn", "norm", "o_proj",
+@pytest.mark.parametrize("what", ["layer class", "o_proj class", "layers' class", "norms' class",
+                                  "linears' class", "o_projs' class", "attentions' class", "layer", "self_attn", "norm", "o_proj",
                                   "o_proj.o_proj", "qkv", "mlp", "down", "final", "embed_tokens",
                                   "embed", "prepare_hidden", "before_layer_run"])
 def test_a_forward_of_its_own_is_called(what, moe, monkeypatch):
-    """A module whose forward is not the one that the fused layers stand for (a subclass's, or set
-    on the instance) is called, in the prompt and in the step after it, and its result counts."""
+    """A module whose forward is not the one that the fused layers stand for (a subclass's, set on
+    the instance or put in its class's place) is called, in the prompt and in the step after it, and its result counts."""
     if moe and what == "down":
         pytest.skip("no down projection")
     lm = _small_llama("bfloat16", moe=moe)
@@ -582,7 +583,11 @@ def test_a_forward_of_its_own_is_called(what, moe, monkeypatch):
     monkeypatch.setattr(ops, "step_start", lambda *a: starts.append(1) or start(*a))
     plain = run()
     assert len(starts) == 2                      # nothing here keeps the start kernel away
-    if what.endswith(" class"):
+    if what.endswith("s' class"):
+        mod = {"layers'": layer, "norms'": model.norm, "linears'": attn.o_proj.o_proj,
+               "o_projs'": attn.o_proj, "attentions'": attn}[what[:-6]]
+        monkeypatch.setattr(type(mod), "forward", halved(type(mod).forward))
+    elif what.endswith(" class"):
         mod = layer if what == "layer class" else attn.o_proj
         base = type(mod)
         mod.__class__ = type("Own", (base,), {"forward": halved(base.forward)})
