@@ -415,11 +415,14 @@ def test_tile_gemm_rings_of_their_own(M, N, K, glu, dtype):
 
 
 @pytest.mark.parametrize("kind", ["linear", "ring", "paged", "fp8", "window"])
-@pytest.mark.parametrize("B,Hkv,gq,Sq,D", [(171, 3, 4, 1, 128), (65, 8, 1, 3, 64), (193, 8, 8, 1, 64),
-                                           (257, 7, 5, 4, 128), (64, 8, 4, 1, 128)])
+@pytest.mark.parametrize("B,Hkv,gq,Sq,D", [(257, 3, 4, 1, 128), (97, 8, 1, 3, 64), (193, 8, 8, 1, 64),
+                                           (257, 7, 5, 4, 128), (259, 3, 1, 3, 64), (64, 8, 4, 1, 128)])
 def test_decode_attention_of_many_short_rows(kind, B, Hkv, gq, Sq, D):
     """A wave a row (the last workgroup's may have none) against the same rows in small
-    batches, which four waves or splits of the keys serve: both round the result once (2^-9)."""
+    batches, which four waves or splits of the keys serve: both round the result once (2^-9). A
+    wave a row from 768 sets of columns on; the last shape has fewer."""
+    sets = B * Hkv * -(-gq * Sq // 16)
+    assert (sets >= 768) == (B != 64) and 20 * Hkv * -(-gq * Sq // 16) < 768
     g = torch.Generator(device="cuda").manual_seed(B)
     rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()  # noqa: E731
     cap, Hq = 96 if kind != "window" else 700, Hkv * gq
@@ -804,3 +807,68 @@ def test_products_are_chosen_by_the_gpus_time(monkeypatch):
     monkeypatch.setattr(ops._C, "tile_gemm", slow_kernel)
     monkeypatch.setitem(ops._sg5_state, "choice", {})
     assert ops._sg5_autotune((M, N, K, False, x.dtype), x, w, None) == 0
+
+
+def _small_of(kind, dtype):
+    """A two-layer model of the kinds that run_layers serves beside _small_llama's, random weights."""
+    import importlib
+
+    from neuronx_distributed_inference_amd.config import EngineConfig
+
+    family, cls = {"llama": ("llama", "Llama"), "qwen2": ("qwen2", "Qwen2"), "qwen3": ("qwen3", "Qwen3"),
+                   "qwen3moe": ("qwen3_moe", "Qwen3Moe")}[kind.split()[0]]
+    mod = importlib.import_module(f"neuronx_distributed_inference_amd.models.{family}.modeling_{family}")
+    paged = dict(is_block_kv_layout=True, pa_block_size=16, pa_num_blocks=24) if "paged" in kind else {}
+    ec = EngineConfig(batch_size=2, max_batch_size=2, seq_len=160, max_length=160, torch_dtype=dtype,
+                      tp_degree=1, output_logits=True, fused_qkv=True, fused_gate_up=True,
+                      enable_batch_bucketing=False, **paged)
+    sizes = dict(neuron_config=ec, hidden_size=512, intermediate_size=1024, num_hidden_layers=2,
+                 num_attention_heads=8, num_key_value_heads=2, head_dim=64, vocab_size=512,
+                 max_position_embeddings=320, rms_norm_eps=1e-5, rope_theta=10000.0, hidden_act="silu",
+                 tie_word_embeddings=False)
+    if family == "qwen3_moe":                     # all experts: no choice that rounding flips
+        sizes.update(num_experts=4, num_experts_per_tok=4, moe_intermediate_size=512)
+    with torch.device("cuda"):
+        lm = getattr(mod, cls + "ForCausalLM")(getattr(mod, cls + "InferenceConfig")(**sizes)).eval()
+    g = torch.Generator(device="cuda").manual_seed(0)
+    for name, p in lm.model.named_parameters():
+        p.data.uniform_(0.5, 1.5, generator=g) if "norm" in name else p.data.normal_(0, 0.05, generator=g)
+    assert any("bias" in n for n, _ in lm.model.named_parameters()) == (family == "qwen2")
+    return lm
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("kind", ["qwen2", "qwen3", "qwen3moe", "llama paged", "qwen2 paged", "qwen3 paged",
+                                  "qwen3moe paged"])
+def test_fused_layers_of_other_kinds(kind, dtype, monkeypatch):
+    """q/k norms, q|k|v biases and pages (a first portion, a second onto its pages, a step): the
+    fused layers against the chain of modules."""
+    from neuronx_distributed_inference_amd.models import model_base
+
+    lm = _small_of(kind, dtype)
+    ids = torch.randint(0, 512, (2, 71), device="cuda")
+    pos = torch.arange(71, device="cuda").repeat(2, 1)
+    table = torch.randperm(24, device="cuda")[:20].view(2, 10)
+    calls, run_layers = [], model_base.run_layers
+    monkeypatch.setattr(model_base, "run_layers", lambda *a: calls.append(1) or run_layers(*a))
+
+    def run():
+        lm.reset()
+        cuts, out = ([(0, 40), (40, 70), (70, 71)] if "paged" in kind else [(0, 70), (70, 71)]), []
+        with torch.inference_mode():
+            for a, b in cuts:
+                kw = dict(block_table=table, phase="token_generation") if "paged" in kind else {}
+                out.append(lm(input_ids=ids[:, a:b].contiguous(), position_ids=pos[:, a:b].contiguous(),
+                              **kw).logits.float())
+        return out + [t.data.float().clone() for i in range(2) for t in lm.model.kv_mgr.get_cache(i)]
+
+    fused = run()
+    assert len(calls) == len(fused) - 4
+    hook = lm.model.norm.register_forward_hook(lambda *a: None)
+    plain = run()
+    hook.remove()
+    assert len(calls) == len(fused) - 4
+    # 16-bit activations of two layers, rounded at other places
+    tol = 0.03 if dtype == "bfloat16" else 0.004
+    for a, b in zip(fused, plain):
+        assert b.norm() > 0 and (a - b).norm() <= tol * b.norm()
