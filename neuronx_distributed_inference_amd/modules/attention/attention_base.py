@@ -193,7 +193,8 @@ class AttentionBase(nn.Module):
     def _qkv_product(self, hidden: torch.Tensor, cos, sin, kc, vc) -> torch.Tensor:
         """Output of the fused q|k|v projection, or its parts of K, where qkv_rope_update adds them
         up. Rows of fp16 models that are kept in 8 bits are rounded to 16 first, see coarse_rows."""
-        if (plain_linear(self.qkv_proj.qkv, hidden) and not _hooked(self.qkv_proj)
+        if (hidden.shape[0] * hidden.shape[1] <= ops.TILE_ROWS
+                and plain_linear(self.qkv_proj.qkv, hidden) and not _hooked(self.qkv_proj)
                 and not coarse_rows(hidden.dtype, kc.dtype)
                 and ops.rope_takes_parts(cos, sin, kc, vc)):
             return ops.linear_parts(hidden, self.qkv_proj.qkv.weight)

@@ -35,8 +35,9 @@ def _plain(module, cls) -> bool:
 
 
 def _plain_norm(norm, h: torch.Tensor) -> bool:
-    return (_plain(norm, RMSNorm) and norm.weight.dtype == h.dtype
-            and norm.weight.is_contiguous() and norm.weight.data_ptr() % 16 == 0)
+    weight = norm._parameters.get("weight")
+    return (_plain(norm, RMSNorm) and weight is not None and weight.dtype == h.dtype
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
 
 
 def fusable(layers, final_norm, h: torch.Tensor, attention_mask, phase: str) -> bool:
@@ -81,7 +82,7 @@ def _feed_forward(mlp, x: torch.Tensor) -> torch.Tensor:
     return mlp(x)
 
 
-PROMPT_ROWS = 512       # csrc/tile_gemm.hip takes no more
+PROMPT_ROWS = ops.TILE_ROWS
 
 
 def _short_prompt(layers, final_norm, h, x, cos, sin, kv_mgr, position_ids, seq_ids):

@@ -304,6 +304,9 @@ def skinny_gemm5_fp8(x2: torch.Tensor, wq_u8: torch.Tensor,
     return y
 
 
+TILE_ROWS = 512         # csrc/tile_gemm.hip takes no more
+
+
 def tiles_enabled() -> bool:
     """Whether 16-bit products may take the tiled kernel: not under NXDI_DISABLE_SG5=1, which leaves
     them to hipBLASLt, nor where lt_linear_enabled leaves them to torch."""
@@ -313,9 +316,10 @@ def tiles_enabled() -> bool:
 def _tile_takes(x2: torch.Tensor, weight: torch.Tensor, glu: bool = False) -> int:
     """Parts of K that the tiled product (csrc/tile_gemm.hip) plans for x2 @ weight^T, 0 where it
     does not take it."""
-    if not (tiles_enabled() and x2.is_cuda and x2.dtype in (torch.bfloat16, torch.float16) and x2.dtype == weight.dtype
+    if not (x2.shape[0] <= TILE_ROWS and x2.is_cuda and x2.dtype == weight.dtype
+            and x2.dtype in (torch.bfloat16, torch.float16)
             and x2.is_contiguous() and weight.is_contiguous()
-            and (x2.data_ptr() | weight.data_ptr()) % 16 == 0):
+            and (x2.data_ptr() | weight.data_ptr()) % 16 == 0 and tiles_enabled()):
         return 0
     c = _require_ext("tile_gemm")
     return c.tile_gemm_splits(x2.shape[0], weight.shape[0], weight.shape[1], glu)
