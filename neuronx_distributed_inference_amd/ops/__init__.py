@@ -234,7 +234,8 @@ def _sg5_workspace(rows: int, N: int, splitk: int, device) -> torch.Tensor:
 def skinny_gemm5(x2: torch.Tensor, weight: torch.Tensor, bias=None, rs=None,
                  splitk: int = 1, mode: int = 0, mt: int = 0) -> torch.Tensor:
     """y = x2 @ weight^T (+bias), optionally scaled per-row by fp32 rs
-    (the rmsnorm fold: y[m] = rs[m] * (x[m] @ W^T)). GPU only.
+    (the rmsnorm fold: y[m] = rs[m] * (x[m] @ W^T)). GPU only. An op of
+    its own: decode_linear takes csrc/tile_gemm.hip.
 
     `mt`: row-block tile (0 = one block over all rows; 64/128 split M
     across blocks for >1 block/CU co-residency)."""
@@ -253,7 +254,7 @@ def skinny_gemm5(x2: torch.Tensor, weight: torch.Tensor, bias=None, rs=None,
 
 
 def _sg5_candidates(M: int, N: int, K: int):
-    """(mt, splitk) variants: splitk sized so total blocks land near
+    """(mt, splitk) variants of skinny_gemm5: splitk sized so total blocks land near
     0.5-2x the 256 CUs (guide: per-block latency ~constant in N); row
     sub-tiles (mt < M) trade extra W traffic for >1 block/CU
     co-residency (block-level DMA/compute overlap)."""
