@@ -910,13 +910,21 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
         // Waves of a set of columns (of one row's KV head). Where rows are short a workgroup is
         // gone after a step or two of its waves, and what it waits for on the way (positions,
         // pages, the first keys, the other waves) is most of its time: a wave a set takes more
-        // steps, and all sets are there at once. 32/8 heads of 128, half to full caches, 4 waves
-        // and 1: 256 rows of 168 34.1, 28.2 us (e4m3, 64/8 heads 32.7, 23.0), 200 of 100 24.3,
-        // 20.2, 128 of 168 21.0, 18.1, 100 of 300 25.7, 23.5, but 64 of 300 15.5, 20.4, 256 of 500
-        // 76, 81, 160 of 700 64, 81, 128 of 512 in e4m3 27.8, 29.0. (2 waves lie between, within
-        // 1 us of the better.)
+        // steps, and all sets are there at once. Longer rows are bound by their bytes, for which 4
+        // waves have more on the way; in 8 bits a row of many has half as many bytes, and a row of
+        // few wants all the waves there are. 4 waves' time over one's, half to full caches of
+        // 64, 128, 200, 256, 384 keys (8 KV heads of 4 query heads; 1 and 8 are like it):
+        //   sets           768                      1536                     4096
+        //   128, 16 bits   1.21 1.17 1.15 1.08 1.04  1.31 1.09 1.00 0.94 0.88  1.67 1.26 1.24 0.97 0.92
+        //   128, e4m3      1.23 1.09 1.12 0.96 0.98  1.42 1.22 1.10 1.02 0.97  1.89 1.59 1.43 1.28 1.20
+        //   64, 16 bits    0.94 0.93 0.90 0.92 0.91  1.15 1.10 0.99 0.95 0.87  1.58 1.33 1.18 1.02 1.00
+        //   64, e4m3       0.89 0.85 0.80 0.75 0.71  1.17 1.06 0.96 0.96 0.88  1.66 1.37 1.27 1.13 1.11
+        // (1024 sets: 64 in 16 bits 1.26 1.22 1.15, e4m3 0.94 0.92 0.86; 2048: e4m3 1.16 and 1.01
+        // at 384.) 256 rows of 168, heads of 128: 37.4 -> 30.7 us.
         const int span = window ? std::min(Smax, std::abs(window) + Sq + DM_TILE) : Smax;
-        const bool alone = nsplit == 1 && span <= 384 && sets >= 768;
+        const bool f8 = sizeof(CT) == 1;
+        const bool alone = nsplit == 1 && sets >= (D == 128 ? 768 : f8 ? 2048 : 1024) &&
+                           span <= (f8 && sets >= 2048 ? 384 : 200);
         TORCH_CHECK(sets < (1L << 31), "attention_decode: too many rows");
         const dim3 grid = alone ? dim3((unsigned)((sets + 3) / 4)) : dim3(nsplit, Hkv * nct, B);
 #define DM_GO(PG, W)                                                                        \
