@@ -920,11 +920,13 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
         //   64, 16 bits    0.94 0.93 0.90 0.92 0.91  1.15 1.10 0.99 0.95 0.87  1.58 1.33 1.18 1.02 1.00
         //   64, e4m3       0.89 0.85 0.80 0.75 0.71  1.17 1.06 0.96 0.96 0.88  1.66 1.37 1.27 1.13 1.11
         // (1024 sets: 64 in 16 bits 1.26 1.22 1.15, e4m3 0.94 0.92 0.86; 2048: e4m3 1.16 and 1.01
-        // at 384.) 256 rows of 168, heads of 128: 37.4 -> 30.7 us.
+        // at 384.) In 16 bits the line is at 7 tiles: 224 keys 1.15 0.97 1.05, heads of 64 0.94
+        // 1.01 1.11; 248 1.06 0.95 1.03 and 0.91 0.95 1.02. 256 rows of 168, heads of 128: 37.4 ->
+        // 30.7 us.
         const int span = window ? std::min(Smax, std::abs(window) + Sq + DM_TILE) : Smax;
         const bool f8 = sizeof(CT) == 1;
         const bool alone = nsplit == 1 && sets >= (D == 128 ? 768 : f8 ? 2048 : 1024) &&
-                           span <= (f8 && sets >= 2048 ? 384 : 200);
+                           span <= DM_TILE * (f8 && sets >= 2048 ? 12 : 7);
         TORCH_CHECK(sets < (1L << 31), "attention_decode: too many rows");
         const dim3 grid = alone ? dim3((unsigned)((sets + 3) / 4)) : dim3(nsplit, Hkv * nct, B);
 #define DM_GO(PG, W)                                                                        \
