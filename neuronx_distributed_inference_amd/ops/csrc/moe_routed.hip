@@ -400,35 +400,43 @@ moe_routed_sum_kernel(T* __restrict__ out, const float* __restrict__ y,
     const int nreal = tiles[0], total = nreal * ntn;
     const bool share = share_tile && mr_shares(total, nk);
     float v[8] = {};
+    auto add = [&](int row, float wt, float4 a, float4 b) {
+        if (row < 0) a = b = float4{0.f, 0.f, 0.f, 0.f};     // another rank's expert
+        v[0] += a.x * wt; v[1] += a.y * wt; v[2] += a.z * wt; v[3] += a.w * wt;
+        v[4] += b.x * wt; v[5] += b.y * wt; v[6] += b.z * wt; v[7] += b.w * wt;
+    };
+    if (!share) {                      // (a loop of its own: all choices' loads go out together)
 #pragma unroll
-    for (int j = 0; j < k; ++j) {
-        const int row = inv[(long)t * k + j];
-        const float wt = weights ? weights[(long)t * k + j] : 1.f;
-        const float* p = y + (long)max(row, 0) * ncols + c;
-        long step = 0;
-        int n = 1;
-        if (share) {
+        for (int j = 0; j < k; ++j) {
+            const int row = inv[(long)t * k + j];
+            const float wt = weights ? weights[(long)t * k + j] : 1.f;
+            const float* p = y + (long)max(row, 0) * ncols + c;
+            add(row, wt, *reinterpret_cast<const float4*>(p), *reinterpret_cast<const float4*>(p + 4));
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < k; ++j) {
+            const int row = inv[(long)t * k + j];
+            const float wt = weights ? weights[(long)t * k + j] : 1.f;
             const int rt = max(row, 0) / share_tile, grp = rt / MR_GRP;
             const int rows_grp = min(MR_GRP, nreal - grp * MR_GRP);
             const int li = grp * MR_GRP * ntn + (c >> 8) * rows_grp + rt % MR_GRP;
             const long all = (long)total * nk, s0 = (long)li * nk;
             const int w0 = (int)(((s0 + 1) * MR_WGS - 1) / all);
-            n = (int)(((s0 + nk) * MR_WGS - 1) / all) - w0 + 1;
-            step = (long)share_tile * 256;
-            p = y + (w0 + li) * step + (max(row, 0) % share_tile) * 256 + (c & 255);
+            const int n = (int)(((s0 + nk) * MR_WGS - 1) / all) - w0 + 1;
+            const long step = (long)share_tile * 256;
+            const float* p = y + (w0 + li) * step + (max(row, 0) % share_tile) * 256 + (c & 255);
+            float4 a = *reinterpret_cast<const float4*>(p);
+            float4 b = *reinterpret_cast<const float4*>(p + 4);
+            for (int i = 1; i < n; ++i) {
+                p += step;
+                const float4 a1 = *reinterpret_cast<const float4*>(p);
+                const float4 b1 = *reinterpret_cast<const float4*>(p + 4);
+                a.x += a1.x; a.y += a1.y; a.z += a1.z; a.w += a1.w;
+                b.x += b1.x; b.y += b1.y; b.z += b1.z; b.w += b1.w;
+            }
+            add(row, wt, a, b);
         }
-        float4 a = *reinterpret_cast<const float4*>(p);
-        float4 b = *reinterpret_cast<const float4*>(p + 4);
-        for (int i = 1; i < n; ++i) {
-            p += step;
-            const float4 a1 = *reinterpret_cast<const float4*>(p);
-            const float4 b1 = *reinterpret_cast<const float4*>(p + 4);
-            a.x += a1.x; a.y += a1.y; a.z += a1.z; a.w += a1.w;
-            b.x += b1.x; b.y += b1.y; b.z += b1.z; b.w += b1.w;
-        }
-        if (row < 0) a = b = float4{0.f, 0.f, 0.f, 0.f};     // another rank's expert
-        v[0] += a.x * wt; v[1] += a.y * wt; v[2] += a.z * wt; v[3] += a.w * wt;
-        v[4] += b.x * wt; v[5] += b.y * wt; v[6] += b.z * wt; v[7] += b.w * wt;
     }
     Vec8<T> o;
 #pragma unroll
