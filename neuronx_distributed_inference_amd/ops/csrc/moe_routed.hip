@@ -444,85 +444,91 @@ moe_routed_sum_kernel(T* __restrict__ out, const float* __restrict__ y,
     store_vec8(out + (long)t * N + col0 + c, o);
 }
 
-// The table: tiles[0] = number of row tiles, then (expert, rows) of each; gather = token of a
-// tile row (padding rows stay unwritten: readers go by `rows`); inv = tile row of a choice, or
-// -1 where the expert is not one of the El from `first`. Rows of an expert stand in the order of
-// their choices, so that a row's tile, and the shares that its sum is made of, are the same in
-// every run. A workgroup an expert: all of them count all choices (LDS atomics), which spares a
+DEV_INLINE int mr_wave_sum(int x) {    // of a wave's values, in every lane, by DPP
+#define MR_STEP(CTRL, ROWS) x += __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false)
+    MR_STEP(0x111, 0xf);               // row_shr 1, 2, 4, 8
+    MR_STEP(0x112, 0xf);
+    MR_STEP(0x114, 0xf);
+    MR_STEP(0x118, 0xf);
+    MR_STEP(0x142, 0xa);               // row_bcast 15, 31
+    MR_STEP(0x143, 0xc);
+#undef MR_STEP
+    return __builtin_amdgcn_readlane(x, 63);
+}
+
+// The table: tiles[0] = number of row tiles, then (expert, rows) of each; gather =
+// token of a tile row (padding rows stay unwritten: readers go by `rows`); inv = tile row of a
+// choice, or -1 where the expert is not one of the El from `first`. Rows of an expert stand in the
+// order of their choices, so that a row's tile, and the shares that its sum is made of, are the
+// same in every run. A workgroup an expert: all of them count all choices (LDS atomics), which spares a
 // launch and a wait between counts and rows, and each ranks its own by ballots, its 16 waves a
 // run of the choices each. 16384 choices of 128 experts: 20 us by one workgroup (rows in any
-// order), 12 now.
+// order), 11 now. Few choices wait for one load after the other: 4 waves, and what the first pass
+// read stays in registers (2 and 128 choices of 8 experts 4.3 and 4.6 -> 3.4 and 3.7 us).
 template <typename I>
 __global__ void __launch_bounds__(1024)
 moe_route_kernel(int* __restrict__ tiles, int* __restrict__ gather, int* __restrict__ inv,
                  const I* __restrict__ idx, const int n, const int El, const long first,
                  const int topk, const int mt) {
     extern __shared__ int count[];                    // [El]
-    __shared__ int s_mine[16], s_before[16], s_all[16];
+    __shared__ int s_mine[16];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, own = blockIdx.x;
-    for (int e = threadIdx.x; e < El; e += 1024) count[e] = 0;
-    __syncthreads();
-    const int run = ((n + 15) / 16 + 63) / 64 * 64, lo = wid * run, hi = min(n, lo + run);
-    int mine = 0;
+    const int nw = blockDim.x >> 6;
+    for (int e = threadIdx.x; e < El; e += blockDim.x) count[e] = 0;
+    const int run = ((n + nw - 1) / nw + 63) / 64 * 64, lo = wid * run, hi = min(n, lo + run);
+    int mine = 0, e[8];                               // -1: not one of the El, -2: past the end
     // eight loads at a time: what the kernel waits for
-    for (int i0 = lo; i0 < hi; i0 += 512) {
-        long e[8];
+    auto load = [&](int i0) {
+        long v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) e[u] = (long)idx[min(i0 + u * 64 + lane, n - 1)] - first;
+        for (int u = 0; u < 8; ++u) v[u] = (long)idx[min(i0 + u * 64 + lane, n - 1)] - first;
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            e[u] = i0 + u * 64 + lane >= hi ? -2 : v[u] >= 0 && v[u] < El ? (int)v[u] : -1;
+    };
+    if (lo < hi) load(lo);
+    __syncthreads();
+    for (int i0 = lo; i0 < hi; i0 += 512) {
+        if (i0 != lo) load(i0);
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            if (i0 + u * 64 + lane >= hi) e[u] = -1;
-            if (e[u] >= 0 && e[u] < El) atomicAdd(&count[e[u]], 1);
+            if (e[u] >= 0) atomicAdd(&count[e[u]], 1);
             mine += __popcll(__ballot(e[u] == own));
         }
     }
     if (lane == 0) s_mine[wid] = mine;
     __syncthreads();
     int before = 0, all = 0;                          // tiles of the experts before, of all
-    for (int e = threadIdx.x; e < El; e += 1024) {
-        const int nt = (count[e] + mt - 1) / mt;
+    for (int x = lane; x < El; x += 64) {             // (each wave by itself)
+        const int nt = (count[x] + mt - 1) / mt;
         all += nt;
-        before += e < own ? nt : 0;
+        before += x < own ? nt : 0;
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        before += __shfl_xor(before, off, 64);
-        all += __shfl_xor(all, off, 64);
-    }
-    if (lane == 0) {
-        s_before[wid] = before;
-        s_all[wid] = all;
-    }
-    __syncthreads();
-    int start = 0, row = 0;
-    all = 0;
-#pragma unroll
-    for (int w = 0; w < 16; ++w) {
-        start += s_before[w];
-        all += s_all[w];
-        row += w < wid ? s_mine[w] : 0;
-    }
+    const int start = mr_wave_sum(before);
+    int row = 0;
+    for (int w = 0; w < wid; ++w) row += s_mine[w];
     const int c = count[own];
-    for (int j = threadIdx.x; j * mt < c; j += 1024) {
+    for (int j = threadIdx.x; j * mt < c; j += blockDim.x) {
         tiles[1 + 2 * (start + j)] = own;
         tiles[2 + 2 * (start + j)] = min(mt, c - j * mt);
     }
-    if (own == 0 && threadIdx.x == 0) tiles[0] = all;
+    if (own == 0 && wid == 0) {
+        all = mr_wave_sum(all);
+        if (lane == 0) tiles[0] = all;
+    }
     row += start * mt;
     for (int i0 = lo; i0 < hi; i0 += 512) {
-        long e[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) e[u] = (long)idx[min(i0 + u * 64 + lane, n - 1)] - first;
+        if (run > 512) load(i0);
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const int i = i0 + u * 64 + lane;
-            const bool in = i < hi, is = in && e[u] == own;
+            const bool is = e[u] == own;
             const unsigned long long m = __ballot(is);
             if (is) {
                 const int at = row + __popcll(m & ((1ull << lane) - 1));
                 gather[at] = i / topk;
                 inv[i] = at;
-            } else if (own == 0 && in && (e[u] < 0 || e[u] >= El)) {
+            } else if (own == 0 && e[u] == -1) {
                 inv[i] = -1;
             }
             row += __popcll(m);
@@ -616,7 +622,9 @@ void moe_route(torch::Tensor tiles, torch::Tensor gather, torch::Tensor inv, tor
                 inv.scalar_type() == at::ScalarType::Int, "moe_route: int32 tables");
     auto st = at::hip::getCurrentHIPStream();
     const int lds = (int)num_local * 4;
-#define MR_ROUTE(I) hipLaunchKernelGGL(moe_route_kernel<I>, dim3((unsigned)num_local), dim3(1024), lds, st,         \
+    // runs of 512 choices are read once (see the kernel): 4 waves for up to four of them
+    const int threads = n <= 2048 ? 256 : 1024;
+#define MR_ROUTE(I) hipLaunchKernelGGL(moe_route_kernel<I>, dim3((unsigned)num_local), dim3(threads), lds, st,      \
         tiles.data_ptr<int>(), gather.data_ptr<int>(), inv.data_ptr<int>(), idx.data_ptr<I>(),    \
         (int)n, (int)num_local, first, (int)idx.size(1), (int)mt)
     TORCH_CHECK(idx.scalar_type() == at::ScalarType::Long ||

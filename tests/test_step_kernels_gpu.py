@@ -874,3 +874,34 @@ def test_fused_layers_of_other_kinds(kind, dtype, monkeypatch):
     tol = 0.03 if dtype == "bfloat16" else 0.004
     for a, b in zip(fused, plain):
         assert b.norm() > 0 and (a - b).norm() <= tol * b.norm()
+
+
+@pytest.mark.parametrize("itype", [torch.int64, torch.int32])
+@pytest.mark.parametrize("n_tok,E,k,first,El", [(1, 8, 2, 0, 8), (3, 4, 1, 2, 2), (64, 8, 8, 0, 8), (255, 130, 8, 1, 65),
+                                                (256, 9, 8, 0, 9), (257, 64, 8, 0, 64), (1024, 8, 8, 3, 4),
+                                                (1025, 300, 8, 0, 300), (5000, 8, 2, 0, 8)])
+def test_moe_route_of_any_number_of_choices(n_tok, E, k, first, El, itype):
+    """The table of rows against the same made on the CPU, to the bit: runs of choices that a wave
+    reads once (up to 512 each of 4, then of 16 waves) and longer ones, other ranks' experts."""
+    mt = 32
+    idx = torch.randint(0, E, (n_tok, k), generator=torch.Generator().manual_seed(n_tok)).to(itype)
+    n = idx.numel()
+    most = (n + min(n, El) * (mt - 1)) // mt
+    tiles, gather, inv = (torch.full((s,), -7, dtype=torch.int32, device="cuda")
+                          for s in (1 + 2 * most, most * mt, n))
+    ops._C.moe_route(tiles, gather, inv, idx.cuda(), El, first, mt)
+    want_t, want_g, want_i = [], {}, [-1] * n
+    flat = [int(e) - first for e in idx.flatten()]
+    by = [[i for i, e in enumerate(flat) if e == x] for x in range(El)]
+    for e, rows in enumerate(by):
+        for a in range(0, len(rows), mt):
+            for j, i in enumerate(rows[a:a + mt]):
+                want_i[i] = len(want_t) * mt + j
+                want_g[want_i[i]] = i // k
+            want_t.append((e, len(rows[a:a + mt])))
+    t = tiles.tolist()
+    assert t[0] == len(want_t)
+    assert list(zip(t[1::2], t[2::2]))[:len(want_t)] == want_t
+    assert inv.tolist() == want_i
+    got = gather.tolist()
+    assert all(got[r] == tok for r, tok in want_g.items())
