@@ -122,9 +122,17 @@ constexpr int MR_GRP = 8;            // row tiles of a group
 
 // Where a launch's workgroups stop inside tiles, and not only at their ends (see the top): tiles
 // that fill the last round of the chip badly, with 8 steps or more for every workgroup.
-DEV_INLINE bool mr_shares(const int total, const int nk) {
+// Shares of one expert's row tiles read its weights at different times, whole tiles together, so
+// that up to half of a round gains however its rows lie (8 experts of 8192 x 2048 in 8 bits, 400
+// tokens, 16 tiles 170 -> 147 us), and more than that only where few experts have a second tile
+// (`crowded`) and the shares are long: 8 of 14336 x 4096 in 16 bits, 128 rows each 639 -> 561, 10
+// tiles 606 -> 594, but 13 tiles 666 -> 709, 11 of 96 rows 637 -> 649; 4 of 8192 x 4096, 12 tiles
+// 294 -> 368; 64 of 1408 x 2048, 4 tokens (16 steps a workgroup) 82.5 -> 86.7.
+constexpr int MR_CROWDED = 1 << 30;  // in tiles[0]: an eighth more row tiles than experts with rows
+DEV_INLINE bool mr_shares(const int total, const int nk, const bool crowded) {
     const int rounds = (total + MR_WGS - 1) / MR_WGS;
-    return rounds <= 2 && total * 100 < rounds * MR_WGS * 85 && total * nk >= MR_WGS * 8;
+    if (rounds > 2 || total * 100 >= rounds * MR_WGS * 85 || total * nk < MR_WGS * 8) return false;
+    return total <= MR_WGS / 2 || (!crowded && total * nk >= MR_WGS * 16);
 }
 
 template <typename T, bool F8, bool GLU, int MT>
@@ -146,10 +154,11 @@ moe_routed_kernel(void* __restrict__ y, const T* __restrict__ x, const char* __r
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     mr_table tiles = (mr_table)(size_t)tiles_, gather = (mr_table)(size_t)gather_;
-    const int nreal = tiles[0], total = nreal * ntn, nk = K / C::BK;
+    const int head = tiles[0], nreal = head & (MR_CROWDED - 1);
+    const int total = nreal * ntn, nk = K / C::BK;
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     // the workgroup's part of the list: a tile, or `left` steps from step k0 of tile li0 on
-    const bool share = !GLU && can_share && mr_shares(total, nk);
+    const bool share = !GLU && can_share && mr_shares(total, nk, head & MR_CROWDED);
     const int per = (total + 7) >> 3, wg = xcd * (MR_WGS / 8) + slot;
     int li0 = xcd * per + slot, k0 = 0, left = nk;
     const int end = share ? total : min(total, (xcd + 1) * per);
@@ -397,8 +406,8 @@ moe_routed_sum_kernel(T* __restrict__ out, const float* __restrict__ y,
     if (id >= (long)ntok * per) return;
     const int t = (int)(id / per), c = (int)(id % per) * 8;
     const int k = TOPK ? TOPK : topk;
-    const int nreal = tiles[0], total = nreal * ntn;
-    const bool share = share_tile && mr_shares(total, nk);
+    const int head = tiles[0], nreal = head & (MR_CROWDED - 1), total = nreal * ntn;
+    const bool share = share_tile && mr_shares(total, nk, head & MR_CROWDED);
     float v[8] = {};
     auto add = [&](int row, float wt, float4 a, float4 b) {
         if (row < 0) a = b = float4{0.f, 0.f, 0.f, 0.f};     // another rank's expert
@@ -456,7 +465,7 @@ DEV_INLINE int mr_wave_sum(int x) {    // of a wave's values, in every lane, by 
     return __builtin_amdgcn_readlane(x, 63);
 }
 
-// The table: tiles[0] = number of row tiles, then (expert, rows) of each; gather =
+// The table: tiles[0] = number of row tiles (and MR_CROWDED), then (expert, rows) of each; gather =
 // token of a tile row (padding rows stay unwritten: readers go by `rows`); inv = tile row of a
 // choice, or -1 where the expert is not one of the El from `first`. Rows of an expert stand in the
 // order of their choices, so that a row's tile, and the shares that its sum is made of, are the
@@ -498,11 +507,12 @@ moe_route_kernel(int* __restrict__ tiles, int* __restrict__ gather, int* __restr
     }
     if (lane == 0) s_mine[wid] = mine;
     __syncthreads();
-    int before = 0, all = 0;                          // tiles of the experts before, of all
+    int before = 0, all = 0, used = 0;                // tiles of the experts before, of all; experts
     for (int x = lane; x < El; x += 64) {             // (each wave by itself)
         const int nt = (count[x] + mt - 1) / mt;
         all += nt;
         before += x < own ? nt : 0;
+        used += nt > 0;
     }
     const int start = mr_wave_sum(before);
     int row = 0;
@@ -514,7 +524,8 @@ moe_route_kernel(int* __restrict__ tiles, int* __restrict__ gather, int* __restr
     }
     if (own == 0 && wid == 0) {
         all = mr_wave_sum(all);
-        if (lane == 0) tiles[0] = all;
+        used = mr_wave_sum(used);
+        if (lane == 0) tiles[0] = all | ((long)all * 8 >= (long)used * 9 ? MR_CROWDED : 0);
     }
     row += start * mt;
     for (int i0 = lo; i0 < hi; i0 += 512) {

@@ -876,6 +876,40 @@ def test_fused_layers_of_other_kinds(kind, dtype, monkeypatch):
         assert b.norm() > 0 and (a - b).norm() <= tol * b.norm()
 
 
+@pytest.mark.parametrize("mt,f8,rows,E,H,I,shared", [
+    (32, False, 60, 4, 4096, 2048, True),      # second tiles, but 128 tiles: half a round
+    (32, False, 70, 4, 4096, 2048, False),     # 192 of them
+    (64, False, 50, 16, 2560, 2048, True),     # 160, a row tile an expert
+    (48, True, 40, 24, 4096, 1536, True),      # 384 in two rounds, 18 steps a workgroup
+    (48, True, 40, 24, 4096, 1280, False)])    # 15 steps
+def test_moe_routed_shares_by_tiles_of_an_expert(mt, f8, rows, E, H, I, shared, monkeypatch):
+    """On both sides of the rule for shares (mr_shares): even choices, sums against 64 bits."""
+    ntn, nk, tiles = -(-H // 256), I // (128 if f8 else 64), E * -(-rows // mt)
+    total = tiles * ntn
+    assert total * 100 < -(-total // 256) * 256 * 85 and total * nk >= 2048
+    assert shared == (total <= 128 or (total * nk >= 4096 and tiles * 8 < E * 9))
+    monkeypatch.setattr(ops, "_moe_tile_rows", lambda *a: mt)
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    T, k = rows * E // 2, 2
+    x = torch.randn(T, H, device="cuda", generator=g).bfloat16()
+    idx = torch.stack([torch.arange(T, device="cuda") % E, (torch.arange(T, device="cuda") + 1) % E], 1)
+    wt = torch.rand(T, k, device="cuda", generator=g) + 0.1
+    w = [(torch.randn(E, *s, device="cuda", generator=g) * 0.05).bfloat16() for s in ((I, H), (I, H), (H, I))]
+    scales, ref = None, [v.to(F64) for v in w]
+    if f8:
+        w, scales = zip(*[ops.fp8_moe_quantize(v) for v in w])
+        ref = [ops.fp8_moe_dequant(v, s).to(F64) for v, s in zip(w, scales)]
+    want = torch.zeros(T, H, dtype=F64, device="cuda")
+    for e in range(E):
+        t, j = (idx == e).nonzero(as_tuple=True)
+        xe = x[t].to(F64)
+        h = torch.nn.functional.silu(xe @ ref[0][e].t()) * (xe @ ref[1][e].t())
+        want.index_add_(0, t, (h @ ref[2][e].t()) * wt[t, j].to(F64).unsqueeze(1))
+    got = ops.moe_routed_experts(x, wt, idx, *w, scales=scales, num_experts=E)
+    assert (got.to(F64) - want).norm() < EPS16[torch.bfloat16] * want.norm()
+    assert torch.equal(got, ops.moe_routed_experts(x, wt, idx, *w, scales=scales, num_experts=E))
+
+
 @pytest.mark.parametrize("itype", [torch.int64, torch.int32])
 @pytest.mark.parametrize("n_tok,E,k,first,El", [(1, 8, 2, 0, 8), (3, 4, 1, 2, 2), (64, 8, 8, 0, 8), (255, 130, 8, 1, 65),
                                                 (256, 9, 8, 0, 9), (257, 64, 8, 0, 64), (1024, 8, 8, 3, 4),
@@ -899,8 +933,10 @@ def test_moe_route_of_any_number_of_choices(n_tok, E, k, first, El, itype):
                 want_i[i] = len(want_t) * mt + j
                 want_g[want_i[i]] = i // k
             want_t.append((e, len(rows[a:a + mt])))
+    used = sum(bool(r) for r in by)
+    crowded = len(want_t) * 8 >= used * 9
     t = tiles.tolist()
-    assert t[0] == len(want_t)
+    assert t[0] == len(want_t) + (1 << 30) * crowded
     assert list(zip(t[1::2], t[2::2]))[:len(want_t)] == want_t
     assert inv.tolist() == want_i
     got = gather.tolist()
