@@ -32,7 +32,12 @@ from neuronx_distributed_inference_amd.modules.attention.attention_base import (
     _hooked,
     coarse_rows,
 )
-from neuronx_distributed_inference_amd.modules.fused_layer import fusable, run_layers
+from neuronx_distributed_inference_amd.modules.fused_layer import (
+    fusable,
+    packed_layers,
+    prompt_operands,
+    run_layers,
+)
 from neuronx_distributed_inference_amd.modules.generation.sampling import (
     Sampler,
     prepare_sampling_params,
@@ -220,34 +225,76 @@ class DecoderModel(nn.Module):
     def _phase(input_ids: torch.Tensor, position_ids: torch.Tensor) -> str:
         return PHASE_CTE if input_ids.shape[-1] > 1 else PHASE_TKG
 
-    def _fused_start(self, layers, input_ids, position_ids, seq_ids, attention_mask, phase):
-        """What ops.step_start makes of the step's tokens, where nothing but the plain modules
-        would come before the first layer's attention and the layers run fused; else None."""
+    def _starts_fused(self, layers, input_ids, position_ids, seq_ids, attention_mask, phase):
+        """Whether ops.step_start makes what comes before the first layer's attention: nothing but
+        the plain modules would, and the layers run fused."""
         emb, rot = self.embed_tokens, self.rotary
         mm = getattr(self, "multimodal_ctx", None)
         if (mm and phase == PHASE_CTE) or getattr(self, "_cos_sin_fn", None) is not None:
-            return None
+            return False
         if (self._own("embed") or self._own("prepare_hidden")
                 or type(emb) is not ParallelEmbedding or ParallelEmbedding.forward is not _LOOKUP
                 or _hooked(emb) or emb.shard_along_embedding
                 or mappings.ps.get_tensor_model_parallel_size() != 1
                 or type(rot) is not RotaryEmbedding or RotaryEmbedding.get_cos_sin is not _ROPE
                 or "get_cos_sin" in vars(rot)):
-            return None
+            return False
         table = emb.weight
         if not (table.is_cuda and input_ids.is_cuda):
-            return None
+            return False
         rot.ensure_table(1, position_ids.device)
         if not (rot._cached_len == rot._cos_cached.shape[0]
                 and ops.step_start_takes(input_ids, position_ids, seq_ids, table,
                                          rot._cos_cached)):
-            return None
+            return False
         like = table.new_empty(*input_ids.shape, table.shape[1])
-        if not fusable(layers, self.norm, like, attention_mask, phase):
+        return fusable(layers, self.norm, like, attention_mask, phase)
+
+    def _fused_start(self, layers, input_ids, position_ids, seq_ids, attention_mask, phase):
+        """What ops.step_start makes of the step's tokens, see _starts_fused; else None."""
+        if not self._starts_fused(layers, input_ids, position_ids, seq_ids, attention_mask, phase):
             return None
-        norm = layers[0].input_layernorm
-        return ops.step_start(input_ids, position_ids, seq_ids, table, rot._cos_cached,
-                              rot._sin_cached, norm.weight, norm.variance_epsilon)
+        rot, norm = self.rotary, layers[0].input_layernorm
+        return ops.step_start(input_ids, position_ids, seq_ids, self.embed_tokens.weight,
+                              rot._cos_cached, rot._sin_cached, norm.weight, norm.variance_epsilon)
+
+    def _may_fuse(self) -> bool:
+        return (not getattr(self, "_layer_post_fns", None)
+                and not getattr(self, "eagle3_capture_layers", None)
+                and not self._own("before_layer_run")
+                and not coarse_rows(self.dtype, getattr(self.kv_mgr, "dtype", self.dtype)))
+
+    def packed_prompts(self, input_ids, position_ids, seq_ids, sampling_params, lengths,
+                       padded: int):
+        """forward of whole prompts, rows of (B, S) ids, without work on their padding; None, with
+        nothing done, where there is none or the layers do not run packed. lengths: ops.PromptLengths
+        of the rows, None: no padding in them. padded: rows of the batch in its bucket."""
+        B, S = input_ids.shape
+        if (type(self).forward is not _FORWARD or type(self).begin_step is not DecoderModel.begin_step
+                or "begin_step" in vars(self) or _hooked(self) or not 0 < B <= ops.PACKED_PROMPTS
+                or getattr(self.kv_mgr, "is_paged", False) or getattr(self, "eagle_capture_hidden", False)
+                or (lengths is None and B * S == padded)
+                or not self._may_fuse() or seq_ids is None or seq_ids.numel() != B):
+            return None
+        layers = [layer for _, layer in self.layer_runs()]
+        if not self._starts_fused(layers, input_ids, position_ids, seq_ids, None, PHASE_CTE):
+            return None
+        rot, norm, table = self.rotary, layers[0].input_layernorm, self.embed_tokens.weight
+        like = table.new_empty(*input_ids.shape, table.shape[1])
+        operands = prompt_operands(layers, self.norm, like, like, rot._cos_cached, self.kv_mgr,
+                                    seq_ids)
+        if operands is None:
+            return None
+        lengths = [S] * B if lengths is None else lengths.get()
+        if lengths is None or sum(lengths) == padded:
+            return None
+        start = ops.step_start_packed(input_ids, position_ids, seq_ids, table, rot._cos_cached,
+                                      rot._sin_cached, norm.weight, norm.variance_epsilon, lengths)
+        h = packed_layers(operands, start, lengths)
+        if h is None:
+            return None
+        # a prompt's last row stands before the next one's first
+        return self._outputs(h.index_select(0, start[6][1:] - 1), sampling_params, False)
 
     # -- the graph body -------------------------------------------------
     def forward(
@@ -287,10 +334,7 @@ class DecoderModel(nn.Module):
         post_fns = getattr(self, "_layer_post_fns", None)
         runs = self.layer_runs()
         fused = [layer for _, layer in runs]
-        may_fuse = (not sp_active and not post_fns
-                    and not getattr(self, "eagle3_capture_layers", None)
-                    and not self._own("before_layer_run")
-                    and not coarse_rows(self.dtype, getattr(self.kv_mgr, "dtype", self.dtype)))
+        may_fuse = not sp_active and self._may_fuse()
         start = self._fused_start(fused, input_ids, position_ids, seq_ids, attention_mask,
                                   phase) if may_fuse else None
         if start is not None:
@@ -400,13 +444,17 @@ class DecoderModel(nn.Module):
         else:
             h_last = h[:, -1:, :]
 
-        # kept for medusa/eagle heads (graph-safe: a static tensor each capture)
-        self.last_hidden = h_last
         # EAGLE draft prefill needs the FULL prompt hidden states (ref
         # EAGLE CTE, model_base.py:1931-2093); opt-in to avoid keeping
         # (B, S, H) alive on every CTE
         if getattr(self, "eagle_capture_hidden", False):
             self.full_hidden = h
+        return self._outputs(h_last, sampling_params, is_speculation)
+
+    def _outputs(self, h_last: torch.Tensor, sampling_params, is_speculation: bool):
+        """Tokens and logits of the rows (B, 1|S, H) that go into the head."""
+        # kept for medusa/eagle heads (graph-safe: a static tensor each capture)
+        self.last_hidden = h_last
         logits_shard = self.finalize_logits(self.lm_head(h_last))  # (B, 1|S, V/tp)
 
         # rejection-sampling speculation reads the per-position top-Kg
@@ -441,6 +489,9 @@ class DecoderModel(nn.Module):
 
     def reset_cache(self):
         self.kv_mgr.reset()
+
+
+_FORWARD = DecoderModel.forward
 
 
 class CausalLMBase(nn.Module):
@@ -579,8 +630,11 @@ class CausalLMBase(nn.Module):
                 self._default_sampling_params = cached
             sampling_params = cached
         # drop an all-ones padding mask on the host so the device path never
-        # syncs per layer
-        if attention_mask is not None and S > 1 and bool(attention_mask.all()):
+        # syncs per layer (the wrapper of whole prompts does, as late as it can)
+        late = not self.kv_cache_populated and phase is None and block_table is None \
+            and not getattr(self.ec, "windowed_context_encoding_size", 0) \
+            and getattr(self.context_encoding_model, "drops_full_masks", False)
+        if attention_mask is not None and S > 1 and not late and bool(attention_mask.all()):
             attention_mask = None
         if seq_ids is None:
             seq_ids = torch.arange(B, device=input_ids.device)

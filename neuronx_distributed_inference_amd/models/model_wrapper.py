@@ -21,6 +21,7 @@ from typing import List, Optional
 
 import torch
 
+from neuronx_distributed_inference_amd import ops
 from neuronx_distributed_inference_amd.modules import autobucketing as ab
 from neuronx_distributed_inference_amd.modules.attention.attention_base import (
     PHASE_CTE,
@@ -47,6 +48,8 @@ def pad_dim(t: Optional[torch.Tensor], dim: int, target: int, value) -> Optional
 
 
 class ModelWrapper:
+    drops_full_masks = True     # a prompt's mask of ones is none
+
     def __init__(
         self,
         config,
@@ -163,6 +166,18 @@ class ModelWrapper:
             bucket = ab.get_target_bucket(
                 S, self.buckets,
                 strategy=getattr(self.ec, "bucket_strategy", "first_fit"))
+            # padding (of the rows, to the bucket and of the batch) is left out where the layers
+            # can do without it
+            if S > 1:
+                lengths = None if attention_mask is None else \
+                    ops.PromptLengths(attention_mask, position_ids)
+                pack = getattr(self.model, "packed_prompts", None)
+                out = pack(input_ids, position_ids, seq_ids, sampling_params, lengths,
+                           max(B, self.batch_size) * bucket) if pack else None
+                if out is not None:
+                    return out
+                if lengths is not None and lengths.all():
+                    attention_mask = None
             input_ids = pad_dim(input_ids, 1, bucket, 0)
             attention_mask = pad_dim(attention_mask, 1, bucket, 0)
             position_ids = pad_dim(position_ids, 1, bucket, -1)

@@ -85,11 +85,9 @@ def _feed_forward(mlp, x: torch.Tensor) -> torch.Tensor:
 PROMPT_ROWS = ops.TILE_ROWS
 
 
-def _short_prompt(layers, final_norm, h, x, cos, sin, kv_mgr, position_ids, seq_ids):
-    """What :func:`run_layers` gives for a short whole prompt of dense layers without q/k norms,
-    its launches made by one native call (csrc/prompt_layers.cpp); None where that does not serve."""
-    if h.numel() > PROMPT_ROWS * h.shape[-1] or not (cos.is_contiguous() and sin.is_contiguous()
-                                                     and ops.tiles_enabled()):
+def prompt_operands(layers, final_norm, h, x, cos, kv_mgr, seq_ids):
+    """What csrc/prompt_layers.cpp takes of dense layers without q/k norms, None for others."""
+    if not ops.tiles_enabled():
         return None
     weights, sizes, numbers = [], [], []
     for layer, after in zip(layers, layers[1:] + [None]):
@@ -104,8 +102,29 @@ def _short_prompt(layers, final_norm, h, x, cos, sin, kv_mgr, position_ids, seq_
                     mlp.down_proj.weight, following.weight, *rows]
         sizes += [attn.num_heads_per_rank, attn.num_kv_heads_per_rank, int(attn.sliding_window)]
         numbers += [norm.variance_epsilon, following.variance_epsilon, float(attn.scale)]
+    return weights, sizes, numbers
+
+
+def _short_prompt(layers, final_norm, h, x, cos, sin, kv_mgr, position_ids, seq_ids):
+    """What :func:`run_layers` gives for a short whole prompt of dense layers without q/k norms,
+    its launches made by one native call (csrc/prompt_layers.cpp); None where that does not serve."""
+    if h.numel() > PROMPT_ROWS * h.shape[-1] or not (cos.is_contiguous() and sin.is_contiguous()):
+        return None
+    operands = prompt_operands(layers, final_norm, h, x, cos, kv_mgr, seq_ids)
+    if operands is None:
+        return None
     return ops._require_ext("prompt_layers").prompt_layers(
-        h, x, cos, sin, position_ids, seq_ids, weights, sizes, numbers)
+        h, x, cos, sin, position_ids, seq_ids, *operands)
+
+
+def packed_layers(operands, start, lengths):
+    """Normed output (rows, 1, H) of the layers over prompts without their padding: `start` of
+    ops.step_start_packed, operands of :func:`prompt_operands`. None, with nothing done, where that
+    does not serve."""
+    h, x, cos, sin, position_ids, rows, starts, prompts = start
+    return ops._require_ext("prompt_layers").prompt_layers(
+        h, x, cos, sin, position_ids, rows, *operands, starts=starts, prompt_sid=prompts,
+        longest=max(lengths))
 
 
 def run_layers(layers, final_norm, h: torch.Tensor, cos, sin, kv_mgr, position_ids, phase,

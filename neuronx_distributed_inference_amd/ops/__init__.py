@@ -384,6 +384,59 @@ def step_start_takes(ids, positions, seq_ids, table, cos_table) -> bool:
             and cos_table.device == ids.device and cos_table.shape[1] % 4 == 0)
 
 
+PACKED_PROMPTS = 256    # csrc/step_start.hip takes no more
+
+
+class PromptLengths:
+    """Tokens of each row of a (B, S) padding mask. Counting begins at once; the host goes on until
+    it asks for them."""
+
+    def __init__(self, mask, positions):
+        self._got = None
+        self.mask = mask
+        self._takes = (
+            mask.dim() == 2 and mask.shape == positions.shape and mask.is_cuda
+            and mask.is_contiguous() and mask.dtype in (torch.int64, torch.int32, torch.bool)
+            and mask.numel() and mask.device == positions.device and _index(positions))
+        if self._takes:
+            rows = torch.empty(mask.shape[0], 2, dtype=torch.int32, device=mask.device)
+            _C.prompt_lengths(rows, mask, positions)
+            self._host = torch.empty(rows.shape, dtype=torch.int32, pin_memory=True)
+            self._host.copy_(rows, non_blocking=True)
+            self._event = torch.cuda.Event()
+            self._event.record()
+
+    def get(self):
+        """A list, where every row's tokens stand at its front and the positions behind them are
+        negative; else None."""
+        if self._takes and self._got is None:
+            self._event.synchronize()
+            rows = self._host.tolist()
+            self._got = all(n > 0 and ok for n, ok in rows) and [n for n, _ in rows]
+        return self._got or None
+
+    def all(self) -> bool:
+        """Whether there is no padding."""
+        lengths = self.get()
+        return min(lengths) == self.mask.shape[1] if lengths else bool(self.mask.all())
+
+
+def step_start_packed(ids, positions, seq_ids, table, cos_table, sin_table, weight, eps: float,
+                      lengths):
+    """step_start of the first lengths[b] tokens of each row b of (B, S) ids, one after the other:
+    (h, x, cos, sin, positions, cache rows) with as many rows, (B + 1,) first rows of the prompts,
+    (B,) their cache rows. For operands that step_start takes, B of up to PACKED_PROMPTS."""
+    n, B = sum(lengths), len(lengths)
+    new = lambda *shape, dtype=torch.int32: torch.empty(*shape, dtype=dtype, device=ids.device)  # noqa: E731
+    h, x = (new(n, 1, table.shape[1], dtype=table.dtype) for _ in range(2))
+    cos, sin = (new(n, 1, cos_table.shape[1], dtype=torch.float32) for _ in range(2))
+    pos32, sid32, starts, prompts = new(n, 1), new(n), new(B + 1), new(B)
+    _require_ext("step_start_packed").step_start_packed(
+        h, x, cos, sin, pos32, sid32, starts, prompts, ids, positions, seq_ids, table, cos_table,
+        sin_table, weight, eps, lengths)
+    return h, x, cos, sin, pos32, sid32, starts, prompts
+
+
 def slot_mapping(block_table, positions, block_size: int, dtype=torch.int64):
     """Flat cache slots (B*S,) of (B, S) positions under (B, pages) tables, -1 for none."""
     slots = torch.empty(positions.numel(), dtype=dtype, device=positions.device)

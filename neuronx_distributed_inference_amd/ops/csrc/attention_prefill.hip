@@ -127,6 +127,7 @@ struct FaArgs {
     const int* positions;    // (B, S) position of each query (-1: padding), or null: token index
     const int* seq_ids;      // (B,) cache row, or null: batch row
     const int* block_table;  // (B, max_blocks), paged caches
+    const int* starts;       // (B + 1,) packed prompts: first row of each in q and out (rows, Hq, D), or null
     const float* sinks;      // (Hq,) or null
     float* o_part;           // (nsplit, B, Hq, S, D), nsplit > 1
     float* ml_part;          // (nsplit, B, Hq, S, 2)
@@ -179,7 +180,10 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
     const int split = rest % a.nsplit;
     const int b = hg / a.Hkv, hkv = hg % a.Hkv;
     const int gq = a.Hq / a.Hkv;
-    const int R = gq * a.S;
+    // packed: S is the longest prompt's; the workgroups past a shorter one have nothing to do
+    const int row0 = a.starts ? a.starts[b] : 0;
+    const int R = gq * (a.starts ? a.starts[b + 1] - row0 : a.S);
+    if (qt * QROWS >= R) return;
 
     const int lane = threadIdx.x & 63;
     const int wid = threadIdx.x >> 6;
@@ -212,7 +216,8 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
     // Q as the B operand: column = the lane's row, 8 channels at half*8 of each k-step
     vec8 qf[NKS];
     {
-        const T* qp = q + (((long)b * a.Hq + head) * a.S + token) * D + half * 8;
+        const T* qp = q + (a.starts ? ((long)(row0 + token) * a.Hq + head)
+                                    : ((long)b * a.Hq + head) * a.S + token) * D + half * 8;
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) qf[ks] = *reinterpret_cast<const vec8*>(qp + ks * 16);
     }
@@ -543,7 +548,7 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
         l = l * f + exp2f(sk - mt);
     }
     const float inv = l > 0.f ? f / l : 0.f;
-    T* po = out + b * a.ob + head * a.oh + token * a.os;
+    T* po = out + (a.starts ? row0 * a.os : b * a.ob) + head * a.oh + token * a.os;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
@@ -639,7 +644,7 @@ void flash_run(torch::Tensor& out, const torch::Tensor& q, const torch::Tensor& 
     }
     a.ob = out.stride(0);
     a.oh = out.stride(1);
-    a.os = out.stride(2);
+    a.os = out.stride(a.starts ? 0 : 2);
     torch::Tensor o_part, ml_part;
     if (a.nsplit > 1) {
         auto opts = torch::TensorOptions().dtype(torch::kFloat32).device(q.device());
@@ -718,6 +723,28 @@ void flash_prefill_cached(torch::Tensor out, torch::Tensor q,
     a.clamp_rows = 1;   // rows of -1 are batch padding: read row 0, the host drops the result
     TORCH_CHECK(sid.numel() == a.B, "seq_ids must be (B,)");
     flash_run(out, q, k_cache, v_cache, a, sinks_opt);
+}
+
+// The same for prompts one after the other without padding: q and out (rows, Hq, 1, D), prompt b
+// from row starts[b] to starts[b + 1], the longest of `longest` tokens.
+void flash_prefill_packed(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
+                          torch::Tensor v_cache, torch::Tensor seq_ids, torch::Tensor starts,
+                          long longest, double scale, long window) {
+    FaArgs a = flash_args(q, scale, window);
+    TORCH_CHECK(a.S == 1 && longest > 0 && starts.scalar_type() == at::kInt &&
+                starts.is_contiguous() && seq_ids.scalar_type() == at::kInt &&
+                seq_ids.is_contiguous() && starts.numel() == seq_ids.numel() + 1 &&
+                starts.is_cuda() && seq_ids.is_cuda(), "flash_prefill_packed: prompts");
+    a.B = seq_ids.numel();
+    a.S = (int)longest;
+    a.Hkv = k_cache.size(1);
+    a.Smax = k_cache.size(2);
+    a.cap = std::min(a.S, a.Smax);
+    a.seq_ids = seq_ids.data_ptr<int>();
+    a.starts = starts.data_ptr<int>();
+    a.clamp_rows = 1;
+    c10::optional<torch::Tensor> none;
+    flash_run(out, q, k_cache, v_cache, a, none);
 }
 
 // Several query tokens a sequence against the cache, each attending the rows up to its own

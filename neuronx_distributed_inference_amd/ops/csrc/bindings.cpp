@@ -98,7 +98,17 @@ void router_topk(torch::Tensor vals, torch::Tensor idx, torch::Tensor logits,
                  long normalize);
 bool lt_available();
 void lt_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias);
+               c10::optional<torch::Tensor> bias, bool timed);
+void flash_prefill_packed(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
+                          torch::Tensor v_cache, torch::Tensor seq_ids, torch::Tensor starts,
+                          long longest, double scale, long window);
+void step_start_packed(torch::Tensor h, torch::Tensor x, torch::Tensor cos, torch::Tensor sin,
+                       torch::Tensor pos32, torch::Tensor sid32, torch::Tensor starts,
+                       torch::Tensor prompt_sid, torch::Tensor ids, torch::Tensor positions,
+                       torch::Tensor seq_ids, torch::Tensor table, torch::Tensor cos_table,
+                       torch::Tensor sin_table, torch::Tensor weight, double eps,
+                       const std::vector<long>& lengths);
+void prompt_lengths(torch::Tensor out, torch::Tensor mask, torch::Tensor positions);
 int lt_tune(int64_t M, int64_t N, int64_t K, bool has_bias,
             torch::Tensor sx, torch::Tensor sw, torch::Tensor sy,
             c10::optional<torch::Tensor> bias);
@@ -125,13 +135,23 @@ c10::optional<torch::Tensor> prompt_layers(torch::Tensor h, torch::Tensor x, tor
                                            torch::Tensor seq_ids,
                                            const std::vector<torch::Tensor>& weights,
                                            const std::vector<long>& sizes,
-                                           const std::vector<double>& numbers);
+                                           const std::vector<double>& numbers,
+                                           c10::optional<torch::Tensor> starts,
+                                           c10::optional<torch::Tensor> prompt_sid, long longest);
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("rms_norm", &rms_norm, "RMSNorm (CDNA4)");
     m.def("rms_norm_fused_add", &rms_norm_fused_add, "RMSNorm + residual add (CDNA4)");
     m.def("add_norm", &add_norm, "residual sum and RMSNorm, of split products too (CDNA4)");
-    m.def("prompt_layers", &prompt_layers, "the launches of plain layers over a short prompt");
+    m.def("prompt_layers", &prompt_layers, "the launches of plain layers over prompts",
+          py::arg("h"), py::arg("x"), py::arg("cos"), py::arg("sin"), py::arg("positions"),
+          py::arg("seq_ids"), py::arg("weights"), py::arg("sizes"), py::arg("numbers"),
+          py::arg("starts") = py::none(), py::arg("prompt_sid") = py::none(),
+          py::arg("longest") = 0);
+    m.def("step_start_packed", &step_start_packed, "step_start of prompts without their padding");
+    m.def("prompt_lengths", &prompt_lengths, "tokens of right-padded prompts");
+    m.def("flash_prefill_packed", &flash_prefill_packed,
+          "MFMA causal flash prefill of prompts one after the other (CDNA4)");
     m.def("step_start", &step_start, "embedding rows, first norm, rope rows, int32 positions");
     m.def("slot_mapping", &slot_mapping, "flat cache slots of positions");
     m.def("step_layout", &step_layout, "int32 positions and rows, valid positions of a row");
@@ -238,7 +258,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("normalize"));
     m.def("lt_available", &lt_available, "hipblaslt usable on this device");
     m.def("lt_linear", &lt_linear, "autotuned hipBLASLt linear (graph-safe)",
-          py::arg("y"), py::arg("x"), py::arg("w"), py::arg("bias") = py::none());
+          py::arg("y"), py::arg("x"), py::arg("w"), py::arg("bias") = py::none(),
+          py::arg("timed") = true);
     m.def("lt_tune", &lt_tune, "pre-tune one GEMM shape",
           py::arg("M"), py::arg("N"), py::arg("K"), py::arg("has_bias"),
           py::arg("sx"), py::arg("sw"), py::arg("sy"), py::arg("bias") = py::none());

@@ -41,6 +41,7 @@
 namespace {
 
 constexpr size_t kWorkspaceBytes = 64ull << 20;
+constexpr size_t kMaxFirst = 4096;   // choices kept without timing: a few for each number of rows seen
 
 struct LtCtx {
     hipblasLtHandle_t handle{nullptr};
@@ -50,6 +51,10 @@ struct LtCtx {
     std::map<std::tuple<int64_t, int64_t, int64_t, int, int>,
              hipblasLtMatmulAlgo_t>
         algos;
+    // same key -> the library's own first choice
+    std::map<std::tuple<int64_t, int64_t, int64_t, int, int>,
+             hipblasLtMatmulAlgo_t>
+        first;
     bool disabled{false};
 };
 
@@ -126,6 +131,21 @@ std::tuple<int64_t, int64_t, int64_t, int, int> make_key(
     return {M, N, K, has_bias ? 1 : 0, (int)dt};
 }
 
+// The library's candidates for a product, its first choice first.
+int ask(const Descs& ds, int most, std::vector<hipblasLtMatmulHeuristicResult_t>& results) {
+    hipblasLtMatmulPreference_t pref;
+    LT_CHECK(hipblasLtMatmulPreferenceCreate(&pref));
+    size_t ws = kWorkspaceBytes;
+    LT_CHECK(hipblasLtMatmulPreferenceSetAttribute(
+        pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &ws, sizeof(ws)));
+    results.resize(most);
+    int found = 0;
+    const hipblasStatus_t st = hipblasLtMatmulAlgoGetHeuristic(
+        ctx().handle, ds.op, ds.a, ds.b, ds.d, ds.d, pref, most, results.data(), &found);
+    hipblasLtMatmulPreferenceDestroy(pref);
+    return st == HIPBLAS_STATUS_SUCCESS ? found : 0;
+}
+
 // Timed tune: try the heuristic candidates, keep the fastest. Returns the
 // number of candidates that ran, or -1 if none work (caller falls back).
 int tune_shape(int64_t M, int64_t N, int64_t K, bool has_bias,
@@ -134,19 +154,9 @@ int tune_shape(int64_t M, int64_t N, int64_t K, bool has_bias,
     Descs ds;
     build_descs(ds, M, N, K, dt, has_bias ? bias : nullptr);
 
-    hipblasLtMatmulPreference_t pref;
-    LT_CHECK(hipblasLtMatmulPreferenceCreate(&pref));
-    size_t ws = kWorkspaceBytes;
-    LT_CHECK(hipblasLtMatmulPreferenceSetAttribute(
-        pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &ws, sizeof(ws)));
-    constexpr int kMaxAlgos = 48;
-    std::vector<hipblasLtMatmulHeuristicResult_t> results(kMaxAlgos);
-    int found = 0;
-    hipblasStatus_t st = hipblasLtMatmulAlgoGetHeuristic(
-        ctx().handle, ds.op, ds.a, ds.b, ds.d, ds.d, pref, kMaxAlgos,
-        results.data(), &found);
-    hipblasLtMatmulPreferenceDestroy(pref);
-    if (st != HIPBLAS_STATUS_SUCCESS || found == 0) return -1;
+    std::vector<hipblasLtMatmulHeuristicResult_t> results;
+    const int found = ask(ds, 48, results);
+    if (found == 0) return -1;
 
     hipEvent_t t0, t1;
     HIP_CHECK(hipEventCreate(&t0));
@@ -209,8 +219,11 @@ bool lt_available() {
 // y(M,N) = x(M,K) @ w(N,K)^T [+ bias(N)]; tunes on first sight of a shape
 // (loud error if that happens inside hipGraph capture — warmup must cover
 // every bucket shape first).
+// `timed` false: the library's own first choice for the shape instead of the timed one. Prompts
+// without their padding have another number of rows each time: a search takes 25 to 80 ms, the
+// question 0.1.
 void lt_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias_opt) {
+               c10::optional<torch::Tensor> bias_opt, bool timed) {
     auto& c = ctx();
     TORCH_CHECK(!c.disabled, "hipblaslt unavailable");
     TORCH_CHECK(x.is_contiguous() && w.is_contiguous() && y.is_contiguous());
@@ -223,12 +236,26 @@ void lt_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
 
     hipblasLtMatmulAlgo_t algo;
     bool hit = false;
+    const auto key = make_key(M, N, K, has_bias, dt);
     {
         std::lock_guard<std::mutex> lock(c.mu);
-        auto it = c.algos.find(make_key(M, N, K, has_bias, dt));
+        auto it = c.algos.find(key);
         if (it != c.algos.end()) { algo = it->second; hit = true; }
+        if (!hit && !timed) {
+            it = c.first.find(key);
+            if (it != c.first.end()) { algo = it->second; hit = true; }
+        }
     }
-    if (!hit) {
+    Descs ds;
+    build_descs(ds, M, N, K, dt, has_bias ? bias : nullptr);
+    if (!hit && !timed) {
+        std::vector<hipblasLtMatmulHeuristicResult_t> results;
+        TORCH_CHECK(ask(ds, 1, results) > 0, "lt_linear: no hipblaslt algo for ", M, "x", N, "x", K);
+        algo = results[0].algo;
+        std::lock_guard<std::mutex> lock(c.mu);
+        if (c.first.size() >= kMaxFirst) c.first.clear();
+        c.first[key] = algo;
+    } else if (!hit) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         hipStreamIsCapturing(stream, &cap);
         TORCH_CHECK(cap == hipStreamCaptureStatusNone,
@@ -239,10 +266,8 @@ void lt_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
         TORCH_CHECK(ran > 0, "lt_linear: no hipblaslt algo for ",
                     M, "x", N, "x", K);
         std::lock_guard<std::mutex> lock(c.mu);
-        algo = c.algos[make_key(M, N, K, has_bias, dt)];
+        algo = c.algos[key];
     }
-    Descs ds;
-    build_descs(ds, M, N, K, dt, has_bias ? bias : nullptr);
     enqueue(ds, &algo, w.data_ptr(), x.data_ptr(), y.data_ptr(), stream);
 }
 
