@@ -44,6 +44,8 @@ class LayerRun:
         # context encoding = every row starts its sequence in this step;
         # mixers may take a whole-prompt path then
         kv_mgr.step.fresh = phase == PHASE_CTE
+        if kv_mgr.step.fused:
+            return self.layer.step_once(h, residual, kv_mgr, self.run_idx)
         return self.layer(h, kv_mgr, self.run_idx), None
 
 

@@ -35,9 +35,13 @@ from typing import Dict, List
 import torch
 import torch.nn as nn
 
+from torch.nn.modules import module as nn_module
+
+from neuronx_distributed_inference_amd import ops
 from neuronx_distributed_inference_amd.config import InferenceConfig
 from neuronx_distributed_inference_amd.models.hybrid_base import HybridDecoderModel
 from neuronx_distributed_inference_amd.models.model_base import CausalLMBase
+from neuronx_distributed_inference_amd.modules.attention.attention_base import _hooked
 from neuronx_distributed_inference_amd.modules.attention.distance_bias import (
     DistanceBiasWindowAttention,
 )
@@ -49,6 +53,7 @@ from neuronx_distributed_inference_amd.ops import seqmix
 from neuronx_distributed_inference_amd.parallel.layers import (
     ColumnParallelLinear,
     RowParallelLinear,
+    plain_linear,
 )
 
 
@@ -175,6 +180,40 @@ class NabelixParallelMixer(nn.Module):
         right = self.right(rqkv, rb, rag, kv_mgr.state, f"run{run_idx}", step)
         return self.left_o(left), self.right_o(right)
 
+    def step_products(self):
+        """(rows of the weight, K) of the products of a step in fewer launches, whether no kernel
+        adds up their parts."""
+        return [(self.in_proj.weight, True), (self.right.ag2.weight, True),
+                (self.left_o.weight, False)]
+
+    def step_once(self, h, kv_mgr, run_idx: int, step):
+        """forward of single tokens (B, 1, width), its two outputs as parts of K."""
+        left, right = self.left, self.right
+        y = ops._C.tile_gemm(h.view(-1, h.shape[-1]), self.in_proj.weight)
+        lq, lk, lv, lg, rqkv, rb, rag = torch.split(y, self.splits, dim=-1)
+        kc, vc = (t.data for t in kv_mgr.get_cache(run_idx))
+        q, gate = lq.unsqueeze(1), lg.unsqueeze(1)
+        new = (lk, lv, kv_mgr.slot_mapping)
+        if not seqmix.new_rows_taken(q, lk, lv, gate, kc, vc):
+            seqmix.paged_kv_write(kc, vc, *new, step)
+            new = None
+        o = seqmix.window_bias_attention(
+            q, kc, vc, step, kv_mgr.block_table, left.r1, left.r2, left.scale, left.window,
+            left.keep_first, left.num_heads, gate=gate, out_dtype=q.dtype, new_rows=new)
+        if (rag.data_ptr() | 2 * rag.stride(0)) % 16:
+            rag = rag.clone(memory_format=torch.contiguous_format)
+        ag = ops._C.tile_gemm(rag, right.ag2.weight)
+        a, gate = torch.split(ag, [right.decay_width, right.num_heads * right.vdim], dim=-1)
+        states = kv_mgr.state
+        m = seqmix.gated_delta_conv(
+            rqkv, right.conv.weight, states.get(f"run{run_idx}.conv"), rb, a, right.dt_bias,
+            right.A_log, gate, right.norm_weight, right.eps, states.get(f"run{run_idx}.mem"), step,
+            right.dim, right.vdim, right.gate_act)
+        parts = ops._C.tile_gemm_pair(o.view(-1, o.shape[-1]), self.left_o.weight, m,
+                                      self.right_o.weight)
+        n = parts.shape[0] // 2
+        return (parts[:n], self.left_scale), (parts[n:], self.right_scale)
+
 
 class NabelixLayer(nn.Module):
     def __init__(self, config: NabelixInferenceConfig, layer_idx: int):
@@ -214,6 +253,62 @@ class NabelixLayer(nn.Module):
             seqmix.residual_add(x, self.mlp(n))
         return x
 
+    def steps_once(self, rows: int) -> bool:
+        """Whether :meth:`step_once` may stand for calling the layer on that many single tokens:
+        plain modules without hooks or a forward of their own, of sizes that its kernels take."""
+        m, mlp = self.mixer, self.mlp
+        right = m.right
+        own = [self, self.norm1, self.canon, m, m.left, right, right.conv]
+        own += [self.norm2, mlp] if mlp is not None else []
+        if any(_FORWARDS.get(type(t)) is not type(t).forward or _hooked(t) for t in own):
+            return False
+        like = m.in_proj.weight[:0]
+        linears = [m.in_proj, m.left_o, m.right_o]
+        linears += [right.ag2] if right.ag2 is not None else []
+        linears += [mlp.gate_up_proj, mlp.down_proj] if mlp is not None and mlp.fused else []
+        weights = [t.weight for t in linears if t is not None]
+        if not (like.is_cuda and like.dtype == self.out_dtype == torch.bfloat16
+                and right.ag2 is not None and right.num_heads == right.num_kv_heads
+                and right.dim in (64, 128) and right.vdim <= 128
+                and (mlp is None or (mlp.fused and mlp.act_mul_fused is seqmix.gelu_tanh_mul_fused))
+                and all(plain_linear(t, like) for t in linears)
+                and all(w.is_contiguous() and w.data_ptr() % 16 == 0 for w in weights)
+                and m.left_o.weight.shape == m.right_o.weight.shape
+                and all(t.bias is None and 2 <= t.taps <= 4 for t in (self.canon, right.conv))
+                and self.canon.residual and self.canon.activation == "none"
+                and right.conv.activation == "silu" and not right.conv.residual
+                and self.norm1.bias is None and like.shape[1] % 8 == 0 and like.shape[1] <= 8192):
+            return False
+        products = m.step_products()
+        takes = ops._C.tile_gemm_splits
+        if mlp is not None:
+            products = products + [(mlp.down_proj.weight, False)]
+            if not takes(rows, *mlp.gate_up_proj.weight.shape, 2) or self.norm2.bias is not None:
+                return False
+        return all(takes(rows, *w.shape, 0, whole) for w, whole in products)
+
+    def step_once(self, x, pending, kv_mgr, run_idx: int):
+        """:meth:`forward` of single tokens in 9 launches for 20. Between two products stands one
+        kernel, which takes in the parts of K of the one before; ``pending`` are such parts that the
+        stream x still lacks, for the kernel that comes first here or, of the result, next."""
+        step = kv_mgr.step
+        h = seqmix.stream_step(x, pending or (), self.norm1.weight, self.norm1.eps, step,
+                               self.canon.weight, kv_mgr.state.get(f"run{run_idx}.canon"))
+        pending = self.mixer.step_once(h, kv_mgr, run_idx, step)
+        if self.mlp is None:
+            return x, pending
+        n = seqmix.stream_step(x, pending, self.norm2.weight, self.norm2.eps, step)
+        n = n.view(-1, n.shape[-1])
+        act = ops._C.tile_gemm(n, self.mlp.gate_up_proj.weight, glu=2)
+        down = self.mlp.down_proj.weight
+        parts = max(2, ops._C.tile_gemm_splits(n.shape[0], *down.shape))
+        return x, ((ops._C.tile_gemm(act, down, splits=parts, parts=True), 1.0),)
+
+
+# what step_once does in their place, by heart: a class whose forward was replaced is not plain
+_FORWARDS = {c: c.forward for c in (NabelixLayer, NabelixParallelMixer, DistanceBiasWindowAttention,
+                                    GatedDeltaRule, CausalShortConv, LayerNorm, GatedMLP)}
+
 
 class _FinalNorm(LayerNorm):
     def __init__(self, width, eps, out_dtype):
@@ -221,7 +316,12 @@ class _FinalNorm(LayerNorm):
         self.out_dtype = out_dtype
 
     def forward(self, x, residual=None):
+        if residual is not None:       # what the stream still lacks, see NabelixLayer.step_once
+            return seqmix.stream_step(x, residual, self.weight, self.eps, None), None
         return seqmix.layer_norm(x, self.weight, self.eps, self.out_dtype)
+
+
+_FINAL = _FinalNorm.forward
 
 
 class NabelixModel(HybridDecoderModel):
@@ -234,6 +334,24 @@ class NabelixModel(HybridDecoderModel):
     def run_order(self, config):
         self._pass_starts = set(config.pass_starts())
         return config.run_order()
+
+    def begin_step(self, position_ids, seq_ids, block_table):
+        block_table = super().begin_step(position_ids, seq_ids, block_table)
+        self.kv_mgr.step.fused = self._steps_once(position_ids)
+        return block_table
+
+    def _steps_once(self, positions) -> bool:
+        rows = positions.shape[0]
+        return (positions.is_cuda and positions.shape[1] == 1 and ops.extension_available()
+                and ops.tiles_enabled() and rows <= ops.TILE_ROWS
+                and not (nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks)
+                and not getattr(self, "_layer_post_fns", None)
+                and not getattr(self, "eagle3_capture_layers", None)
+                and type(self.norm) is _FinalNorm and _FinalNorm.forward is _FINAL
+                and not _hooked(self.norm) and self.norm.bias is None
+                and self.norm.out_dtype == torch.bfloat16
+                and positions.device.index == torch.cuda.current_device()
+                and all(layer.steps_once(rows) for layer in self.layers))
 
     def before_layer_run(self, run_idx, h, h_embed):
         if run_idx == 0:

@@ -314,16 +314,17 @@ def tiles_enabled() -> bool:
     return os.environ.get("NXDI_DISABLE_SG5") != "1" and lt_linear_enabled()
 
 
-def _tile_takes(x2: torch.Tensor, weight: torch.Tensor, glu: bool = False) -> int:
+def _tile_takes(x2: torch.Tensor, weight: torch.Tensor, glu: bool = False,
+                whole: bool = False) -> int:
     """Parts of K that the tiled product (csrc/tile_gemm.hip) plans for x2 @ weight^T, 0 where it
-    does not take it."""
+    does not take it. whole: no kernel follows that adds up parts."""
     if not (x2.shape[0] <= TILE_ROWS and x2.is_cuda and x2.dtype == weight.dtype
             and x2.dtype in (torch.bfloat16, torch.float16)
             and x2.is_contiguous() and weight.is_contiguous()
             and (x2.data_ptr() | weight.data_ptr()) % 16 == 0 and tiles_enabled()):
         return 0
     c = _require_ext("tile_gemm")
-    return c.tile_gemm_splits(x2.shape[0], weight.shape[0], weight.shape[1], glu)
+    return c.tile_gemm_splits(x2.shape[0], weight.shape[0], weight.shape[1], glu, whole)
 
 
 def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -517,7 +518,7 @@ def _sg5_autotune(key, x2, weight, bias) -> int:
         results[0] = _time(lambda w: lt_linear(x2, w, bias))
     except Exception:  # noqa: BLE001
         results[0] = float("inf")
-    sk = _tile_takes(x2, weight)
+    sk = _tile_takes(x2, weight, whole=True)
     try:
         results[sk] = _time(lambda w: _C.tile_gemm(x2, w, bias, splits=sk))
     except Exception:  # noqa: BLE001
@@ -541,16 +542,16 @@ def decode_linear(x: torch.Tensor, weight: torch.Tensor, bias=None) -> torch.Ten
     x2 = x.reshape(-1, shape[-1]).contiguous()
     M, K = x2.shape
     N = weight.shape[0]
-    if not _tile_takes(x2, weight) or (bias is not None and not bias.is_contiguous()):
-        return lt_linear(x, weight, bias)
+    if not _tile_takes(x2, weight, whole=True) or (bias is not None and not bias.is_contiguous()):
+        return lt_linear(x2, weight, bias).view(*shape[:-1], N)
     key = (M, N, K, bias is not None, x.dtype)
     choice = _sg5_state["choice"].get(key)
     if choice is None:
         if torch.cuda.is_current_stream_capturing():
-            return lt_linear(x, weight, bias)  # never tune inside a capture
+            return lt_linear(x2, weight, bias).view(*shape[:-1], N)  # never tune inside a capture
         choice = _sg5_autotune(key, x2, weight, bias)
     if choice == 0:
-        return lt_linear(x, weight, bias)
+        return lt_linear(x2, weight, bias).view(*shape[:-1], N)
     return _C.tile_gemm(x2, weight, bias, splits=choice).view(*shape[:-1], N)
 
 

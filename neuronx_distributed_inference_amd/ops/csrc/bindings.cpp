@@ -115,9 +115,10 @@ int lt_tune(int64_t M, int64_t N, int64_t K, bool has_bias,
 void gelu_tanh_mul_fused(torch::Tensor out, torch::Tensor gate_up);
 void add_norm(torch::Tensor out, torch::Tensor residual, torch::Tensor y, torch::Tensor weight,
               double eps);
-long tile_gemm_splits(long M, long N, long K, bool glu);
+torch::Tensor tile_gemm_pair(torch::Tensor x, torch::Tensor w, torch::Tensor x2, torch::Tensor w2);
+long tile_gemm_splits(long M, long N, long K, long glu, bool whole);
 torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
-                        long splits, bool parts, bool glu);
+                        long splits, bool parts, long glu);
 
 void step_start(torch::Tensor h, torch::Tensor x, torch::Tensor cos, torch::Tensor sin,
                 torch::Tensor pos32, c10::optional<torch::Tensor> sid32, torch::Tensor ids,
@@ -157,10 +158,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("step_layout", &step_layout, "int32 positions and rows, valid positions of a row");
     m.def("linear_table", &linear_table, "page table of rows that own their pages");
     m.def("copy_many", &copy_many, "several copies in one launch");
-    m.def("tile_gemm_splits", &tile_gemm_splits, "parts of K of a tiled product, 0: not taken");
+    m.def("tile_gemm_splits", &tile_gemm_splits, "parts of K of a tiled product, 0: not taken",
+          py::arg("M"), py::arg("N"), py::arg("K"), py::arg("glu") = 0, py::arg("whole") = false);
+    m.def("tile_gemm_pair", &tile_gemm_pair, "parts of K of two tiled products of one shape");
     m.def("tile_gemm", &tile_gemm, "tiled 16-bit product of up to 512 rows (CDNA4)",
           py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("splits") = 0,
-          py::arg("parts") = false, py::arg("glu") = false);
+          py::arg("parts") = false, py::arg("glu") = 0);
     m.def("silu_mul", &silu_mul, "SiLU(gate)*up (CDNA4)");
     m.def("gelu_tanh_mul", &gelu_tanh_mul, "GELU-tanh(gate)*up (CDNA4)");
     m.def("rope_apply", &rope_apply, "RoPE rotate-half in place (CDNA4)");

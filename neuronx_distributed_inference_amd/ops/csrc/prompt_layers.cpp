@@ -5,9 +5,9 @@
 #include <torch/extension.h>
 #include <vector>
 
-long tile_gemm_splits(long M, long N, long K, bool glu);
+long tile_gemm_splits(long M, long N, long K, long glu, bool whole);
 torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
-                        long splits, bool parts, bool glu);
+                        long splits, bool parts, long glu);
 void add_norm(torch::Tensor out, torch::Tensor residual, torch::Tensor y, torch::Tensor weight,
               double eps);
 void qkv_rope_update(torch::Tensor q_out, torch::Tensor qkv, torch::Tensor cosb, torch::Tensor sinb,
@@ -31,7 +31,7 @@ namespace {
 // take it
 torch::Tensor product(const torch::Tensor& x, const torch::Tensor& w, bool glu) {
     const long rows = x.size(0), N = w.size(0);
-    if (tile_gemm_splits(rows, N, x.size(1), glu))
+    if (tile_gemm_splits(rows, N, x.size(1), glu, glu))
         return tile_gemm(x, w, c10::nullopt, 0, !glu, glu);
     torch::Tensor y = torch::empty({rows, N}, x.options());
     try {
@@ -86,10 +86,10 @@ c10::optional<torch::Tensor> prompt_layers(torch::Tensor h, torch::Tensor x, tor
             w[4].size(0) != H || 2 * w[4].size(1) != w[3].size(0) || w[4].size(1) % 8 ||
             (size_t)x.data_ptr() % 16)
             return c10::nullopt;
-        if (!starts && (!tile_gemm_splits(rows, w[0].size(0), H, false) ||
-                        !tile_gemm_splits(rows, H, Hq * D, false) ||
-                        !tile_gemm_splits(rows, w[3].size(0), H, true) ||
-                        !tile_gemm_splits(rows, H, w[4].size(1), false)))
+        if (!starts && (!tile_gemm_splits(rows, w[0].size(0), H, false, false) ||
+                        !tile_gemm_splits(rows, H, Hq * D, false, false) ||
+                        !tile_gemm_splits(rows, w[3].size(0), H, true, true) ||
+                        !tile_gemm_splits(rows, H, w[4].size(1), false, false)))
             return c10::nullopt;
     }
     torch::Tensor xs = x.view({rows, H});

@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 #include <stdint.h>
+#include <type_traits>
 
 #define WAVE 64
 #define DEV __device__ __forceinline__
@@ -295,6 +296,127 @@ __global__ void short_conv_step_kernel(const TIn* __restrict__ x, long xs,
     if (act_silu) acc = acc * sigmoidf_(acc);
     if (residual) acc += cur;
     stf<TOut>(y + idx, acc);
+}
+
+// What stands between two products of a decoder layer whose residual stream is fp32, a row of
+// single tokens a workgroup: x += sa * a + sb * b (each the sum of the parts of K of a product, in
+// fp32), LayerNorm, and with TAPS the short convolution over time that is added to the norm, with its
+// new tail; out in bf16. Bound by launches: 48 rows of 2048 took 21 us in four (sum of parts,
+// residual, norm, convolution), 6 here.
+DEV uint16_t f2bf_rne(float f);
+struct StreamArgs {
+    float* x;                    // (rows, C)
+    const float* a;              // (na, rows, C)
+    const float* b;              // (nb, rows, C)
+    const float* w;              // norm
+    const float* cw;             // (C, TAPS)
+    float* tail;                 // (slots, TAPS - 1, C)
+    const int* pos;
+    const int* seq;
+    bf16* out;
+    float sa, sb, eps;
+    int na, nb, C;
+    long rows;
+};
+
+template <int V, int TAPS>
+__global__ void __launch_bounds__(LN_THREADS) stream_step_kernel(const StreamArgs s) {
+    __shared__ float red[LN_THREADS / WAVE];
+    constexpr int R = TAPS > 1 ? TAPS - 1 : 1;
+    const long row = blockIdx.x, plane = s.rows * s.C;
+    constexpr bool EARLY = V <= 2;               // taps' weights in registers before the sums
+    float v[V][8], t[V][R][8], cw[V][8 * (TAPS > 1 ? TAPS : 1)], sum = 0.f;
+    auto taps = [&](int k, int c) {
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) load8<float>(s.cw + (long)c * TAPS + j * 8, cw[k] + j * 8);
+    };
+    const int p = TAPS ? s.pos[row] : 0, slot = TAPS ? s.seq[row] : 0;
+    const bool live = !TAPS || (p >= 0 && slot >= 0);
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        const int c = (k * LN_THREADS + threadIdx.x) * 8;
+        if (c >= s.C) continue;
+        load8<float>(s.x + row * s.C + c, v[k]);
+        if constexpr (TAPS > 1) {
+            // on their way before the sums
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if (live) load8<float>(s.tail + ((long)slot * R + r) * s.C + c, t[k][r]);
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (!live || p - R + r < 0) t[k][r][e] = 0.f;
+            }
+            if constexpr (EARLY) taps(k, c);
+        }
+        float y[8];
+#pragma unroll 1
+        for (int j = 0; j < 2; ++j) {
+            const float* part = j ? s.b : s.a;
+            const int n = j ? s.nb : s.na;
+            if (n == 0) continue;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[e] = 0.f;
+            for (int i = 0; i < n; i += 4) {
+                float q[4][8];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    load8<float>(part + min(i + u, n - 1) * plane + row * s.C + c, q[u]);
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) y[e] += i + u < n ? q[u][e] : 0.f;
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[k][e] += (j ? s.sb : s.sa) * y[e];
+        }
+        if (s.na | s.nb) st8<float>(s.x + row * s.C + c, v[k]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum += v[k][e];
+    }
+    const float mean = block_sum(sum, red) / s.C;
+    float sq = 0.f;
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        const int c = (k * LN_THREADS + threadIdx.x) * 8;
+        if (c >= s.C) continue;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float d = v[k][e] - mean;
+            sq += d * d;
+        }
+    }
+    const float inv = 1.f / sqrtf(block_sum(sq, red) / s.C + s.eps);
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        const int c = (k * LN_THREADS + threadIdx.x) * 8;
+        if (c >= s.C) continue;
+        float w[8], o[8];
+        load8<float>(s.w + c, w);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (v[k][e] - mean) * inv * w[e];
+        if constexpr (TAPS > 1) {
+            if (live) {
+                float* tr = s.tail + (long)slot * R * s.C + c;
+#pragma unroll
+                for (int r = 0; r + 1 < R; ++r) st8<float>(tr + (long)r * s.C, t[k][r + 1]);
+                st8<float>(tr + (long)(R - 1) * s.C, o);
+            }
+            if constexpr (!EARLY) taps(k, c);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                float acc = 0.f;
+#pragma unroll
+                for (int r = 0; r < R; ++r) acc += cw[k][e * TAPS + r] * t[k][r][e];
+                acc += cw[k][e * TAPS + R] * o[e];
+                o[e] = live ? o[e] + acc : 0.f;
+            }
+        }
+        uint32_t pk[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            pk[e] = (uint32_t)f2bf_rne(o[2 * e]) | ((uint32_t)f2bf_rne(o[2 * e + 1]) << 16);
+        *reinterpret_cast<uint4*>(s.out + row * s.C + c) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+    }
 }
 
 // ------------------------------------------------------------ paged KV write
@@ -1103,6 +1225,13 @@ struct WfArgs {
     long qstride, gstride, ktok, khead, vtok, vhead;
     int max_blocks, H, G, B, bsz, page_shift, S, window, keep, qt_every, ghead, cmask, nqt;
     float scale, cap, qt_coef;
+    // single tokens whose key and value the kernel puts into the cache as well, or null
+    const bf16* kn;
+    const bf16* vn;
+    const int* slots;
+    bf16* kw;
+    bf16* vw;
+    long knstride, vnstride, nslots;
 };
 
 template <int D>
@@ -1395,7 +1524,9 @@ __global__ void __launch_bounds__(256, 2) window_flash_kernel(const WfArgs a) {
 // and the pages looked up a tile before that. Scores are K Q^T (mfma 16x16x32), so that P sits in
 // the registers as the operand of P V; it enters in three 16-bit parts, which add up to its 24
 // bits. The waves meet once, in LDS. 48 rows, 16 heads of 128 on 4 KV heads, 350 to 700 keys,
-// log-distance bias, gate: 41 us by multiply-adds (window_attn_kernel), 22 now.
+// log-distance bias, gate: 41 us by multiply-adds (window_attn_kernel), 22 now. With kn and vn the
+// token's own key and value come from there and go into the cache on the way, where a launch of its
+// own took 4.8 us.
 struct WdBuf {
     uint4 k[2][4];
     uint4 v[8];
@@ -1435,26 +1566,46 @@ __global__ void __launch_bounds__(WD_WAVES * WAVE) window_decode_kernel(const Wf
     const int* bt = a.btab + (long)b * a.max_blocks;
     const bf16* kbase = a.kc + (long)g * a.khead;
     const bf16* vbase = a.vc + (long)g * a.vhead + n * DV;
+    const bf16* kown = a.kn ? a.kn + (long)b * a.knstride + (long)g * D : nullptr;
+    const bf16* vown = a.kn ? a.vn + (long)b * a.vnstride + (long)g * D : nullptr;
+    if (kown && c0 == 0 && wid == WD_WAVES - 1 && lane < D / 4) {
+        const long s = a.slots[b];
+        const int e = lane % (D / 8) * 8;
+        if (s >= 0 && s < a.nslots) {
+            if (lane < D / 8)
+                *reinterpret_cast<uint4*>(a.kw + s * a.ktok + (long)g * a.khead + e) =
+                    *reinterpret_cast<const uint4*>(kown + e);
+            else
+                *reinterpret_cast<uint4*>(a.vw + s * a.vtok + (long)g * a.vhead + e) =
+                    *reinterpret_cast<const uint4*>(vown + e);
+        }
+    }
 
     // lanes 0..31 look up the cache slot of a key of the tile each
     auto look_up = [&](int t, int& rem) {
         const int m = min(t * WD_KT + (lane & 31), nk - 1), j = m < nfirst ? m : m + shift;
         const int page = a.page_shift >= 0 ? j >> a.page_shift : j / a.bsz;
         rem = j - page * a.bsz;
+        if (kown && m == nk - 1) {                       // the token's own
+            rem = -1;
+            return 0;
+        }
         return bt[page];
     };
     auto load = [&](WdBuf& u, int page, int rem) {
-        const int slot = max(page, 0) * a.bsz + rem;
+        const int slot = max(page, 0) * a.bsz + rem;     // -1: the token's own
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
-            const bf16* p = kbase + (long)__shfl(slot, kb * 16 + n, WAVE) * a.ktok + q4 * 8;
+            const int sl = __shfl(slot, kb * 16 + n, WAVE);
+            const bf16* p = (sl < 0 ? kown : kbase + (long)sl * a.ktok) + q4 * 8;
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks) u.k[kb][ks] = *reinterpret_cast<const uint4*>(p + ks * 32);
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int kk = (j >> 2) * 16 + q4 * 4 + (j & 3);
-            const bf16* p = vbase + (long)__shfl(slot, kk, WAVE) * a.vtok;
+            const int sl = __shfl(slot, kk, WAVE);
+            const bf16* p = sl < 0 ? vown + n * DV : vbase + (long)sl * a.vtok;
             if constexpr (DV == 8) u.v[j] = *reinterpret_cast<const uint4*>(p);
             else {
                 const uint2 w = *reinterpret_cast<const uint2*>(p);
@@ -1558,6 +1709,8 @@ __global__ void __launch_bounds__(WD_WAVES * WAVE) window_decode_kernel(const Wf
     l += __shfl_xor(l, 32, WAVE);
 
     // ---- the waves meet ----
+    // the row that was written may be read again below
+    if (kown && wid == WD_WAVES - 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     extern __shared__ __attribute__((aligned(16))) float wd_lds[];
     float* ml = wd_lds;                                  // [waves][16][2]
     float* ol = wd_lds + WD_WAVES * 32;                  // [waves][nc][D]
@@ -2569,9 +2722,13 @@ __global__ void gated_rmsnorm_kernel(const float* __restrict__ o, const T* __res
 // 16 lanes for themselves, 8 key channels a lane, four value channels a wave at a time), so the
 // small chains of the preparation hide behind it; the norm over the value channels goes through
 // LDS. 48 rows of 16 heads of 128 x 128 (101 MB): 26 us; the three kernels above took 56.
-template <typename T, int D>
+// With TAPS the short convolution and silu of q, k and v come first, of the raw projections (in T)
+// and the carried tail, a channel a thread, where every head has a q and k of its own: q, k and v are
+// neither written nor read in 32 bits. The same 48 rows, 4 taps: 5.4 + 26.6 us apart, 30.0 so.
+template <typename T, int D, int TAPS>
 __global__ void __launch_bounds__(512)
-delta_step_kernel(const float* __restrict__ qkv, long cstride, const T* __restrict__ beta,
+delta_step_kernel(const std::conditional_t<(TAPS > 0), T, float>* __restrict__ qkv, long cstride,
+                  const float* __restrict__ cw, float* __restrict__ tail, const T* __restrict__ beta,
                   long bstride, const T* __restrict__ a, long astride,
                   const float* __restrict__ dt_bias, const float* __restrict__ a_log,
                   const T* __restrict__ gate, long gstride, const float* __restrict__ norm_w,
@@ -2580,6 +2737,7 @@ delta_step_kernel(const float* __restrict__ qkv, long cstride, const T* __restri
                   int per_head, int gate_silu) {
     constexpr int F = D / 64, NI = 4;            // float4s of a lane in a state row; rows of a lane
     __shared__ float os[32 * NI];
+    __shared__ __attribute__((aligned(16))) float cs[TAPS > 0 ? 2 * D + 128 : 4];   // q, k, v
     const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
     const int slot = seq[b], p = pos[b];
     T* op = out + ((long)b * H + h) * Dv;
@@ -2590,26 +2748,42 @@ delta_step_kernel(const float* __restrict__ qkv, long cstride, const T* __restri
     const int lane = tid & 63, part = lane & 15, row0 = (tid >> 6) * 4 + (lane >> 4);
     const int g = h / (H / G);
     float* st = state + ((long)slot * H + h) * Dv * D + part * 4;
-    const float* vp = qkv + (long)b * cstride + 2L * G * D + (long)h * Dv;
     float4 s[NI][F];
     float v[NI];
+    // convolution: a channel a thread, its loads out before the state's
+    constexpr int R = TAPS > 1 ? TAPS - 1 : 1;
+    const int C = 2 * G * D + H * Dv;
+    float ct[R], cwv[R + 1], ccur;
+    float* ctail = nullptr;
+    if constexpr (TAPS > 0) {
+        const int i = min(tid, 2 * D + Dv - 1);
+        const int c = i < D ? g * D + i : i < 2 * D ? G * D + g * D + i - D : 2 * G * D + h * Dv + i - 2 * D;
+        ctail = tail + (long)slot * R * C + c;
+#pragma unroll
+        for (int r = 0; r <= R; ++r) cwv[r] = cw[(long)c * TAPS + r];
+#pragma unroll
+        for (int r = 0; r < R; ++r) ct[r] = ctail[(long)r * C];
+        ccur = ldf<T>(qkv + (long)b * cstride + c);
+    }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int r = min(row0 + 32 * i, Dv - 1);
 #pragma unroll
         for (int f = 0; f < F; ++f)
             s[i][f] = *reinterpret_cast<const float4*>(st + (long)r * D + f * 64);
-        v[i] = vp[r];
+        if constexpr (TAPS == 0) v[i] = qkv[(long)b * cstride + 2L * G * D + (long)h * Dv + r];
     }
     float4 q[F], k[F], dec[F];
-    const float* qp = qkv + (long)b * cstride + (long)g * D + part * 4;
     const T* ap = a + (long)b * astride + (per_head ? h : (long)h * D + part * 4);
     const float* bp = dt_bias + (per_head ? h : h * D + part * 4);
     float av[4 * F], bv[4 * F];
 #pragma unroll
     for (int f = 0; f < F; ++f) {
-        q[f] = *reinterpret_cast<const float4*>(qp + f * 64);
-        k[f] = *reinterpret_cast<const float4*>(qp + (long)G * D + f * 64);
+        if constexpr (TAPS == 0) {
+            const float* qp = qkv + (long)b * cstride + (long)g * D + part * 4;
+            q[f] = *reinterpret_cast<const float4*>(qp + f * 64);
+            k[f] = *reinterpret_cast<const float4*>(qp + (long)G * D + f * 64);
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             av[4 * f + e] = ldf<T>(ap + (per_head ? 0 : f * 64 + e));
@@ -2619,6 +2793,31 @@ delta_step_kernel(const float* __restrict__ qkv, long cstride, const T* __restri
     const float bt = sigmoidf_(ldf<T>(beta + (long)b * bstride + h));
     const float neg_rate = -expf(a_log[h]);
     asm volatile("" ::: "memory");               // all of the above in flight
+    if constexpr (TAPS > 0) {
+        if (tid < 2 * D + Dv) {
+            float acc = 0.f;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if (p - R + r < 0) ct[r] = 0.f;
+                acc += cwv[r] * ct[r];
+                if (r > 0) ctail[(long)(r - 1) * C] = ct[r];
+            }
+            ctail[(long)(R - 1) * C] = ccur;
+            acc += cwv[R] * ccur;
+            cs[tid] = acc * sigmoidf_(acc);
+        }
+        // (the state's loads stay in flight over it)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            q[f] = *reinterpret_cast<const float4*>(cs + part * 4 + f * 64);
+            k[f] = *reinterpret_cast<const float4*>(cs + D + part * 4 + f * 64);
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i) v[i] = cs[2 * D + min(row0 + 32 * i, Dv - 1)];
+    }
     float sq = 0.f, sk = 0.f, qk = 0.f;
 #pragma unroll
     for (int f = 0; f < F; ++f) {
@@ -5478,8 +5677,12 @@ int nx_paged_attn(const void* q, long qstride, const void* kc, long ktok, long k
                   const float* sink, const void* gate, long gstride, void* out, int io_bf16,
                   int out_bf16, int B, int S, int H, int G, int Dk, int Dv, int bsz,
                   float scale, int window, int keep, float cap, float qt_coef, int qt_every,
-                  float* ws, int nks, int ghead, int cmask, hipStream_t st) {
+                  float* ws, int nks, int ghead, int cmask, const void* kn, long knstride,
+                  const void* vn, long vnstride, const int* slots, long nslots, hipStream_t st) {
     if ((long)B * S <= 0) return 0;
+    if (kn && !(S == 1 && (knstride % 8) == 0 && (vnstride % 8) == 0 &&
+                (((uintptr_t)kn | (uintptr_t)vn) % 16) == 0 && vc != kc && khead == Dk &&
+                vhead == Dv)) return -8;
     if (Dv > WAVE * 8 || H % G != 0 || Dk <= 0 || Dv <= 0) return -1;
     if (!io_bf16 && out_bf16) return -2;
     if (r2 != nullptr && r1 == nullptr) return -4;
@@ -5553,6 +5756,8 @@ int nx_paged_attn(const void* q, long qstride, const void* kc, long ktok, long k
             f.window = window; f.keep = keep; f.qt_every = qt_every; f.ghead = ghead;
             f.cmask = cmask; f.scale = scale; f.cap = cap; f.qt_coef = qt_coef;
             f.nqt = (int)(((long)rp * S + WF_ROWS - 1) / WF_ROWS);
+            f.kn = (const bf16*)kn; f.vn = (const bf16*)vn; f.slots = slots; f.nslots = nslots;
+            f.kw = (bf16*)kc; f.vw = (bf16*)vc; f.knstride = knstride; f.vnstride = vnstride;
             const int nc = rp < 16 ? rp : 16;
             const int lds = S == 1 ? (WD_WAVES * 32 + WD_WAVES * nc * Dk) * 4
                                    : 4 * WF_KT * Dk * 2 + 64;
@@ -5565,6 +5770,7 @@ int nx_paged_attn(const void* q, long qstride, const void* kc, long ktok, long k
             k<<<grid, dim3(S == 1 ? WD_WAVES * WAVE : 256), lds, st>>>(f);
             return (int)hipGetLastError();
         }
+        if (kn) return -8;                                // only the kernel above takes new rows
         if (io_bf16 && out_bf16 && steps_ok && rep_ok && dk_ok && k_al && v_al &&
             (qstride % 8) == 0 && ((uintptr_t)q % 16) == 0) {
             const int QTm = MA_ROWS / rp;
@@ -5654,8 +5860,8 @@ int nx_gated_delta(const float* qkv, long cstride, const void* beta, long bstrid
         if (S != 1 || (D != 64 && D != 128) || Dv > 128 || cstride % 4 || H % G || B > 65535)
             return -1;
         dim3 gs(H, B), bs(512);
-#define DST(TT, DD) delta_step_kernel<TT, DD><<<gs, bs, 0, st>>>( \
-        qkv, cstride, (const TT*)beta, bstride, (const TT*)a, astride, dt_bias, a_log, \
+#define DST(TT, DD) delta_step_kernel<TT, DD, 0><<<gs, bs, 0, st>>>( \
+        qkv, cstride, nullptr, nullptr, (const TT*)beta, bstride, (const TT*)a, astride, dt_bias, a_log, \
         (const TT*)gate, gstride, norm_w, eps, state, pos, seq, (TT*)out, H, G, Dv, per_head, \
         gate_silu)
         if (in_bf16) { if (D == 64) DST(bf16, 64); else DST(bf16, 128); }
@@ -5721,6 +5927,51 @@ int nx_gated_delta(const float* qkv, long cstride, const void* beta, long bstrid
     else gated_rmsnorm_kernel<float><<<g2, b2, 0, st>>>(
         obuf, (const float*)gate, gstride, norm_w, eps, pos, seq, (float*)out, ntok, S, H, Dv,
         gate_silu);
+    return (int)hipGetLastError();
+}
+
+// One token a row, of the raw bf16 projections: convolution, recurrence and norm.
+int nx_gated_delta_conv(const void* qkv, long cstride, const float* cw, float* tail, int taps,
+                        const void* beta, long bstride, const void* a, long astride,
+                        const void* gate, long gstride, const float* dt_bias, const float* a_log,
+                        const float* norm_w, float eps, float* state, const int* pos,
+                        const int* seq, void* out, int B, int H, int D, int Dv, int per_head,
+                        int gate_silu, hipStream_t st) {
+    if (B <= 0) return 0;
+    if ((D != 64 && D != 128) || Dv > 128 || B > 65535 || taps < 2 || taps > 4) return -1;
+    dim3 gs(H, B), bs(512);
+#define DSC(DD, TP) delta_step_kernel<bf16, DD, TP><<<gs, bs, 0, st>>>( \
+    (const bf16*)qkv, cstride, cw, tail, (const bf16*)beta, bstride, (const bf16*)a, astride, \
+    dt_bias, a_log, (const bf16*)gate, gstride, norm_w, eps, state, pos, seq, (bf16*)out, H, H, Dv, \
+    per_head, gate_silu)
+#define DSCT(DD) do { if (taps == 2) DSC(DD, 2); else if (taps == 3) DSC(DD, 3); else DSC(DD, 4); } while (0)
+    if (D == 64) DSCT(64);
+    else DSCT(128);
+#undef DSCT
+#undef DSC
+    return (int)hipGetLastError();
+}
+
+// taps 0: no convolution. -1: not a shape or alignment that it takes
+int nx_stream_step(float* x, const float* a, int na, float sa, const float* b, int nb, float sb,
+                   const float* w, float eps, const float* cw, float* tail, int taps,
+                   const int* pos, const int* seq, void* out, long rows, int C, hipStream_t st) {
+    if (rows <= 0) return 0;
+    if (C <= 0 || C % 8 || C > LN_THREADS * 8 * 4 || taps < 0 || taps == 1 || taps > 4 ||
+        rows > 0x7fffffff || na < 0 || nb < 0 ||
+        (((uintptr_t)x | (uintptr_t)a | (uintptr_t)b | (uintptr_t)w | (uintptr_t)tail |
+          (uintptr_t)cw | (uintptr_t)out) % 16)) return -1;
+    StreamArgs s{x, a, b, w, cw, tail, pos, seq, (bf16*)out, sa, sb, eps, na, nb, C, rows};
+    const dim3 grid((unsigned)rows), block(LN_THREADS);
+#define STT(V) do { \
+    if (taps == 0) stream_step_kernel<V, 0><<<grid, block, 0, st>>>(s); \
+    else if (taps == 2) stream_step_kernel<V, 2><<<grid, block, 0, st>>>(s); \
+    else if (taps == 3) stream_step_kernel<V, 3><<<grid, block, 0, st>>>(s); \
+    else stream_step_kernel<V, 4><<<grid, block, 0, st>>>(s); } while (0)
+    if (C <= LN_THREADS * 8) STT(1);
+    else if (C <= LN_THREADS * 16) STT(2);
+    else STT(4);
+#undef STT
     return (int)hipGetLastError();
 }
 

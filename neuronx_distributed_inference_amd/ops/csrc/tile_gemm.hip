@@ -6,7 +6,8 @@
 // pipes is the bytes on the way: 64 to 128 KB a CU. K is split so that all 256 CUs have a tile;
 // the parts stay in fp32 and the kernel that follows (residual sum and norm, rope) adds them up,
 // so that a split costs no launch. With GLU a wave has the gate and the up rows of its columns and
-// writes silu(gate) * up, which saves a launch and both in 16 bits.
+// writes silu(gate) (or gelu) * up, which saves a launch and both in 16 bits. Two products whose
+// sum the next kernel wants (a mixer's two output projections) go in one launch.
 
 #include "common.h"
 #include <torch/extension.h>
@@ -59,15 +60,28 @@ struct TgArgs {
     float* part;         // (splits, M, N) fp32 when splits > 1
     const void* x;       // (M, K)
     const void* w;       // (N, K)
+    const void* x2;      // a second product of the same sizes, parts after the first's, or null
+    const void* w2;
     const void* bias;    // (N,) or null
     int M, N, K, splits, mblocks, ntiles, per_xcd, work;
+    unsigned xbytes, xbytes2;    // from a row of x to the next
 };
+
+// none; silu and the tanh form of gelu of the gate
+enum TgGlu { PLAIN, SILU, GELU };
+
+template <int GLU> DEV_INLINE float tg_act(float z) {
+    if constexpr (GLU == GELU)
+        return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+    return z / (1.f + __expf(-z));
+}
+
 
 // A workgroup of WM x WN waves makes BM x BN outputs (of one of `splits` parts of K), a wave
 // BM/WM x BN/WN of them. D chunks of w and DX of x are in LDS or on the way there. Where they
 // differ, half of the waves load w and half x: a wave's loads are waited for in their order, and
 // one that has both would wait for w as early as for x, which is near (L2).
-template <typename T, int BM, int BN, int WM, int WN, int D, int DX, bool GLU, bool ONCE>
+template <typename T, int BM, int BN, int WM, int WN, int D, int DX, int GLU, bool ONCE>
 __global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a) {
     using MF = TgMfma<T>;
     using vec8 = typename MF::vec8;
@@ -91,8 +105,10 @@ __global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a)
     const int nt = rest % a.ntiles, slice = rest / a.ntiles;
     const int m0 = mb * BM;
     const int chunks = a.K / TG_BK;
-    const int c_lo = (int)((long)slice * chunks / a.splits);
-    const int n = (int)((long)(slice + 1) * chunks / a.splits) - c_lo;    // >= 1: splits <= chunks
+    const bool second = slice >= a.splits;
+    const int part = second ? slice - a.splits : slice;
+    const int c_lo = (int)((long)part * chunks / a.splits);
+    const int n = (int)((long)(part + 1) * chunks / a.splits) - c_lo;     // >= 1: splits <= chunks
 
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lw = wid % LW;
@@ -105,12 +121,12 @@ __global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a)
     // slot ^ (row & 7), so that 8 rows of one slot lie in different banks. Rows past the end
     // repeat the last one.
     const int prow = lane >> 3;
-    const unsigned kbytes = (unsigned)a.K * sizeof(T);
+    const unsigned kbytes = (unsigned)a.K * sizeof(T), xbytes = second ? a.xbytes2 : a.xbytes;
     unsigned xo[XP], wo[WP];
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
         const int r = (lw * XP + i) % XPT * 8 + prow;
-        xo[i] = (unsigned)min(r, a.M - 1 - m0) * kbytes + ((lane & 7) ^ (r & 7)) * 16;
+        xo[i] = (unsigned)min(r, a.M - 1 - m0) * xbytes + ((lane & 7) ^ (r & 7)) * 16;
     }
 #pragma unroll
     for (int i = 0; i < WP; ++i) {
@@ -127,8 +143,8 @@ __global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a)
         }
         wo[i] = row * kbytes + ((lane & 7) ^ (r & 7)) * 16;
     }
-    const char* x0 = (const char*)a.x + (long)m0 * kbytes + (long)c_lo * 128;
-    const char* w0 = (const char*)a.w + (long)nt * (GLU ? BN / 2 : BN) * kbytes + (long)c_lo * 128;
+    const char* x0 = (const char*)(second ? a.x2 : a.x) + (long)m0 * xbytes + (long)c_lo * 128;
+    const char* w0 = (const char*)(second ? a.w2 : a.w) + (long)nt * (GLU ? BN / 2 : BN) * kbytes + (long)c_lo * 128;
     // tiles start at different chunks and wrap round: in step they would all ask for the same
     // 128 bytes of rows a power of two apart, which few of the memory channels hold
     int at = ((blockIdx.x >> 3) / a.mblocks) % n;
@@ -243,8 +259,8 @@ __global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a)
             tg_f32x4 v = acc[i][j];
             if constexpr (GLU) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = v[r] / (1.f + __expf(-v[r])) * acc[i][j + FC][r];
-            } else if (a.splits > 1) {
+                for (int r = 0; r < 4; ++r) v[r] = tg_act<GLU>(v[r]) * acc[i][j + FC][r];
+            } else if (a.part) {
                 *reinterpret_cast<tg_f32x4*>(a.part + ((long)slice * a.M + m) * a.N + c) = v;
                 continue;
             } else if (a.bias) {
@@ -308,13 +324,18 @@ struct TgPlan {
 // 71.8 -> 62.9, 39.7 -> 35.0, 23.1 -> 20.8 (160 rows of the third, fourth and first shape; 256 rows
 // in one tile 74.2, 42.6, 24.5: no better than two of 128). Gate|up of few columns takes tiles of
 // 128 also where 256 would leave half of the CUs idle: 128 rows of the third shape 72.0 -> 50.5.
-TgPlan tg_plan(long M, long N, long K, bool glu) {
+// `whole`: no kernel follows that would add up parts. Then up to 64 rows take tiles of half the width
+// where these fill most of the chip undivided, also where those of the full width in two parts are
+// a little faster by themselves: the sum is a launch of its own, some 3 us. 48 rows, undivided /
+// two parts without their sum / library: (11408, 2048) 14.3 / 13.4 / 17.6 us, (16384, 2048)
+// 15.5 / 16.6 / 19.1, (12288, 4096) 23.6 / 22.5 / 25.2; 100 rows of the last 33.0 / 27.2 / 32.4.
+TgPlan tg_plan(long M, long N, long K, bool glu, bool whole) {
     TgPlan p{T16, 16, 128, 0};
-    if (M < 1 || M > 512 || N < 64 || N % (glu ? 8 : 4) || K < 256 || K % TG_BK ||
+    if (M < 1 || M > 512 || N < 64 || N % (glu ? 8 : 4) || K < (whole && !glu ? 128 : 256) || K % TG_BK ||
         K * N * 2 >= (1L << 32))
         return p;
     // half the width where that many more tiles spare parts of K, or with GLU fill the chip
-    const bool narrow = glu ? N < 25600 : N <= 4096;
+    const bool narrow = glu ? N < 25600 : N <= 4096 || (whole && M <= 64 && N > 8192 && N <= 16384);
     if (M <= 16) p = narrow ? TgPlan{T16N, 16, 64, 0} : TgPlan{T16, 16, 128, 0};
     else if (M <= 32) p = narrow ? TgPlan{T32N, 32, 64, 0} : TgPlan{T32, 32, 128, 0};
     else if (M <= 64) p = narrow ? TgPlan{T64N, 64, 64, 0} : TgPlan{T64, 64, 128, 0};
@@ -331,11 +352,11 @@ TgPlan tg_plan(long M, long N, long K, bool glu) {
     return p;
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int D, bool GLU, bool ONCE, int DX = D>
+template <typename T, int BM, int BN, int WM, int WN, int D, int GLU, bool ONCE, int DX = D>
 void tg_go(TgArgs& a, hipStream_t stream) {
     a.mblocks = (a.M + BM - 1) / BM;
     a.ntiles = (a.N + BN - 1) / BN;
-    a.work = a.mblocks * a.ntiles * a.splits;
+    a.work = a.mblocks * a.ntiles * a.splits * (a.w2 ? 2 : 1);
     a.per_xcd = (a.work + 7) / 8;
     constexpr int LDS = (DX * BM + D * BN) * 128;
     static_assert(LDS <= 163840, "the rings do not fit");
@@ -346,7 +367,7 @@ void tg_go(TgArgs& a, hipStream_t stream) {
     HIP_CHECK_KERNEL();
 }
 
-template <typename T, bool GLU>
+template <typename T, int GLU>
 void tg_tile(TgArgs& a, TgTile tile, hipStream_t s) {
     switch (tile) {
         case T16: tg_go<T, 16, 128, 1, 4, 4, GLU, true>(a, s); break;
@@ -367,24 +388,56 @@ void tg_tile(TgArgs& a, TgTile tile, hipStream_t s) {
 }  // namespace
 
 // Parts of K that tile_gemm takes for this shape, 0: none, it is the library's.
-long tile_gemm_splits(long M, long N, long K, bool glu) { return tg_plan(M, N, K, glu).splits; }
+long tile_gemm_splits(long M, long N, long K, long glu, bool whole) {
+    return tg_plan(M, N, K, glu != PLAIN, whole).splits;
+}
+
+namespace {
+
+// rows of x may lie further apart than they are long (columns of a wider tensor)
+void tg_operands(const torch::Tensor& x, const torch::Tensor& w) {
+    TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "tile_gemm: shapes");
+    TORCH_CHECK(x.stride(1) == 1 && (x.size(0) < 2 || (x.stride(0) >= x.size(1) &&
+                x.stride(0) % 8 == 0 && x.stride(0) < (1L << 20))) && w.is_contiguous() &&
+                x.scalar_type() == w.scalar_type(), "tile_gemm: rows of one type");
+    TORCH_CHECK(((size_t)x.data_ptr() | (size_t)w.data_ptr()) % 16 == 0, "tile_gemm: alignment");
+    TORCH_CHECK(x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf,
+                "tile_gemm: bf16/f16 only");
+}
+
+unsigned tg_row_bytes(const torch::Tensor& x) {
+    return (unsigned)(x.size(0) < 2 ? x.size(1) : x.stride(0)) * 2;
+}
+
+void tg_launch(TgArgs& a, TgTile tile, bool bf, long glu) {
+    auto stream = at::hip::getCurrentHIPStream();
+    if (bf) {
+        if (glu == SILU) tg_tile<__hip_bfloat16, SILU>(a, tile, stream);
+        else if (glu == GELU) tg_tile<__hip_bfloat16, GELU>(a, tile, stream);
+        else tg_tile<__hip_bfloat16, PLAIN>(a, tile, stream);
+    } else {
+        TORCH_CHECK(glu != GELU, "tile_gemm: gelu in bf16 only");
+        if (glu == SILU) tg_tile<__half, SILU>(a, tile, stream);
+        else tg_tile<__half, PLAIN>(a, tile, stream);
+    }
+}
+
+}  // namespace
 
 // x (M, K) @ w (N, K)^T. `splits` 0: as planned, which leaves (splits, M, N) parts in fp32 where
-// there are several (`parts`) or sums them up. `glu`: silu of the first half of the columns times
-// the second.
+// there are several (`parts`) or sums them up. `glu`: silu (1) or gelu (2) of the first half of the
+// columns times the second.
 torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
-                        long splits, bool parts, bool glu) {
-    TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "tile_gemm: shapes");
-    TORCH_CHECK(x.is_contiguous() && w.is_contiguous() && x.scalar_type() == w.scalar_type(),
-                "tile_gemm: contiguous operands of one type");
-    TORCH_CHECK(((size_t)x.data_ptr() | (size_t)w.data_ptr()) % 16 == 0, "tile_gemm: alignment");
+                        long splits, bool parts, long glu) {
+    tg_operands(x, w);
+    TORCH_CHECK(glu >= PLAIN && glu <= GELU, "tile_gemm: glu");
     const bool bf = x.scalar_type() == at::ScalarType::BFloat16;
-    TORCH_CHECK(bf || x.scalar_type() == at::ScalarType::Half, "tile_gemm: bf16/f16 only");
     TgArgs a{};
     a.M = x.size(0);
     a.K = x.size(1);
     a.N = w.size(0);
-    const TgPlan plan = tg_plan(a.M, a.N, a.K, glu);
+    a.xbytes = tg_row_bytes(x);
+    const TgPlan plan = tg_plan(a.M, a.N, a.K, glu, !parts);
     TORCH_CHECK(plan.splits > 0, "tile_gemm: shape not taken");
     TORCH_CHECK(splits >= 0 && splits <= a.K / TG_BK && !(glu && splits > 1), "tile_gemm: splits");
     a.splits = splits ? splits : plan.splits;
@@ -403,13 +456,7 @@ torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::T
     a.w = w.data_ptr();
     a.bias = bias ? bias->data_ptr() : nullptr;
     auto stream = at::hip::getCurrentHIPStream();
-    if (bf) {
-        if (glu) tg_tile<__hip_bfloat16, true>(a, plan.tile, stream);
-        else tg_tile<__hip_bfloat16, false>(a, plan.tile, stream);
-    } else {
-        if (glu) tg_tile<__half, true>(a, plan.tile, stream);
-        else tg_tile<__half, false>(a, plan.tile, stream);
-    }
+    tg_launch(a, plan.tile, bf, glu);
     if (a.splits == 1) return y;
     if (parts) return part;
     const long MN = (long)a.M * a.N;
@@ -423,4 +470,29 @@ torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::T
                            a.part, (const __half*)a.bias, MN, a.N, a.splits);
     HIP_CHECK_KERNEL();
     return y;
+}
+
+// Parts of K of x @ w^T and then of x2 @ w2^T, products of one shape: (2 n, M, N) in fp32.
+torch::Tensor tile_gemm_pair(torch::Tensor x, torch::Tensor w, torch::Tensor x2, torch::Tensor w2) {
+    tg_operands(x, w);
+    tg_operands(x2, w2);
+    TORCH_CHECK(x.sizes() == x2.sizes() && w.sizes() == w2.sizes() &&
+                x.scalar_type() == x2.scalar_type(), "tile_gemm_pair: shapes");
+    TgArgs a{};
+    a.M = x.size(0);
+    a.K = x.size(1);
+    a.N = w.size(0);
+    const TgPlan plan = tg_plan(a.M, a.N, a.K, false, false);
+    TORCH_CHECK(plan.splits > 0, "tile_gemm_pair: shape not taken");
+    a.splits = std::max(1, plan.splits / 2);
+    torch::Tensor part = torch::empty({2 * a.splits, a.M, a.N}, x.options().dtype(torch::kFloat32));
+    a.part = part.data_ptr<float>();
+    a.x = x.data_ptr();
+    a.w = w.data_ptr();
+    a.x2 = x2.data_ptr();
+    a.w2 = w2.data_ptr();
+    a.xbytes = tg_row_bytes(x);
+    a.xbytes2 = tg_row_bytes(x2);
+    tg_launch(a, plan.tile, x.scalar_type() == at::kBFloat16, PLAIN);
+    return part;
 }

@@ -173,6 +173,8 @@ class StepLayout:
         # dense rows of latent layers whose cache a later layer reads (whole
         # prompts only), by the owner's cache index
         self.latent_rows = {}
+        # whether the layers of the step run in fewer launches, see models/nabelix
+        self.fused = False
         # the step's token ids and the (vocab, layers * dim) table that layers
         # read them from, for models that use ids past the embedding
         self.tokens = None
@@ -306,7 +308,7 @@ def paged_attention(q, k_cache, v_cache, step: StepLayout, block_table, scale: f
                     num_heads: int, window: Optional[int] = None, keep_first: int = 0,
                     r1=None, r2=None, gate=None, softcap: float = 0.0, sink=None,
                     q_temp=None, out_dtype=None, gate_per_head: bool = False,
-                    chunk: int = 0, slopes=None):
+                    chunk: int = 0, slopes=None, new_rows=None):
     """q (B,S,H*Dk) (row-strided view allowed) against the paged cache ->
     (B,S,H*Dv). Options (see ref.paged_attention): sliding ``window`` with
     ``keep_first`` always-visible tokens (None = plain causal), ``chunk`` > 0
@@ -315,7 +317,9 @@ def paged_attention(q, k_cache, v_cache, step: StepLayout, block_table, scale: f
     score cap, per-head softmax ``sink``, query
     temperature ``q_temp`` = (coef, every), sigmoid output ``gate``
     ((B,S,H*Dv), or (B,S,H) with ``gate_per_head``).
-    ``v_cache`` may be ``k_cache[..., :Dv]`` (values inside the key rows)."""
+    ``v_cache`` may be ``k_cache[..., :Dv]`` (values inside the key rows).
+    ``new_rows`` = (k, v, slot mapping) of single tokens: their keys (B, G*Dk) and values, which
+    stand for those in the cache and are written there, where new_rows_taken says so."""
     B, S = q.shape[0], q.shape[1]
     H = num_heads
     G, Dk = k_cache.shape[2], k_cache.shape[3]
@@ -361,7 +365,8 @@ def paged_attention(q, k_cache, v_cache, step: StepLayout, block_table, scale: f
             k_cache.shape[1], ctypes.c_float(scale),
             int(window) if window is not None else 0x7fffffff, int(keep_first),
             ctypes.c_float(softcap or 0.0), ctypes.c_float(coef), every,
-            _p(ws), nks, int(bool(gate_per_head)), int(chunk or 0), _stream()),
+            _p(ws), nks, int(bool(gate_per_head)), int(chunk or 0),
+            *_new_rows(new_rows, step, k_cache), _stream()),
             "paged_attention")
         return out
     return ref.paged_attention(
@@ -371,13 +376,33 @@ def paged_attention(q, k_cache, v_cache, step: StepLayout, block_table, scale: f
         gate_per_head=gate_per_head, chunk=int(chunk or 0), slopes=slopes)
 
 
+def _new_rows(rows, step, k_cache):
+    if rows is None:
+        return _p(None), ctypes.c_long(0), _p(None), ctypes.c_long(0), _p(None), ctypes.c_long(0)
+    k, v, slots = rows
+    assert k.stride(-1) == v.stride(-1) == 1 and k.dtype == v.dtype == k_cache.dtype
+    return (_p(k), ctypes.c_long(k.stride(0)), _p(v), ctypes.c_long(v.stride(0)), _p(step.i32(slots)),
+            ctypes.c_long(k_cache.shape[0] * k_cache.shape[1]))
+
+
+def new_rows_taken(q, k, v, gate, k_cache, v_cache) -> bool:
+    """Whether paged_attention of single tokens takes new_rows: bf16 heads of 64 or 128, as wide as
+    their values, everything on 16 bytes."""
+    D = k_cache.shape[3]
+    return (q.dtype == torch.bfloat16 and D in (64, 128) and v_cache.shape[3] == D
+            and q.shape[0] <= 65535 and q.shape[1] == 1
+            and k_cache.is_contiguous() and v_cache.is_contiguous()
+            and k_cache.data_ptr() != v_cache.data_ptr()
+            and not any(t.data_ptr() % 16 or t.stride(0) % 8 for t in (q, k, v, gate, k_cache, v_cache)))
+
+
 def window_bias_attention(q, k_cache, v_cache, step: StepLayout, block_table,
                           r1, r2, scale: float, window: int, keep_first: int,
-                          num_heads: int, gate=None, out_dtype=None):
+                          num_heads: int, gate=None, out_dtype=None, new_rows=None):
     """Sliding window + kept first tokens with a log-distance penalty."""
     return paged_attention(q, k_cache, v_cache, step, block_table, scale, num_heads,
                            window=window, keep_first=keep_first, r1=r1, r2=r2,
-                           gate=gate, out_dtype=out_dtype)
+                           gate=gate, out_dtype=out_dtype, new_rows=new_rows)
 
 
 # Portions of at least this many tokens run in chunks; shorter ones token by token. At 32 tokens
@@ -434,6 +459,48 @@ def gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps: float,
     return ref.gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps,
                                 state, step.positions, step.seq_ids, kv_heads,
                                 dim, vdim, out_dtype, gate_act)
+
+
+def gated_delta_conv(qkv, conv_w, tail, beta, a, dt_bias, a_log, gate, norm_w, eps: float, state,
+                     step: StepLayout, dim: int, vdim: int, gate_act: str = "sigmoid"):
+    """Short convolution with silu of the raw projections and gated_delta_rule, of single tokens
+    (B, width) in bf16 with a q and k for every head, in one launch; tail and state advance. GPU only."""
+    B, H = beta.shape
+    per_head = a.shape[-1] == H and dim != 1
+    assert a.shape[-1] == (H if per_head else H * dim) == dt_bias.numel()
+    assert qkv.shape[-1] == 2 * H * dim + H * vdim == conv_w.shape[0] and state.dtype == torch.float32
+    assert tail.dtype == torch.float32 and tail.is_contiguous() and state.is_contiguous()
+    assert qkv.dtype == beta.dtype == a.dtype == gate.dtype == torch.bfloat16
+    assert state.data_ptr() % 16 == 0 and all(t.stride(-1) == 1 for t in (qkv, beta, a, gate))
+    out = torch.empty(B, H * vdim, dtype=qkv.dtype, device=qkv.device)
+    long = ctypes.c_long
+    _check(_load().nx_gated_delta_conv(
+        _p(qkv), long(qkv.stride(0)), _p(_f32(conv_w)), _p(tail), conv_w.shape[1],
+        _p(beta), long(beta.stride(0)), _p(a), long(a.stride(0)), _p(gate), long(gate.stride(0)),
+        _p(_f32(dt_bias)), _p(_f32(a_log)), _p(_f32(norm_w)), ctypes.c_float(eps), _p(state),
+        _p(step.positions), _p(step.seq_ids), _p(out), B, H, dim, vdim, int(per_head),
+        int(gate_act == "silu"), _stream()), "gated_delta_conv")
+    return out
+
+
+def stream_step(x, pending, norm_w, eps: float, step: StepLayout, conv_w=None, tail=None):
+    """Residual sum, LayerNorm and, with conv_w, the short convolution that is added to it, of single
+    tokens in one launch, in bf16. x (B, 1, C) is the fp32 stream, which takes in the sum of
+    ``pending``: ((parts, B, C) in fp32, scale) pairs, two at the most; tail advances. GPU only."""
+    C = x.shape[-1]
+    rows = x.numel() // C
+    assert x.dtype == torch.float32 and x.is_contiguous() and len(pending) <= 2
+    for parts, _ in pending:
+        assert parts.dtype == torch.float32 and parts.is_contiguous() and parts.shape[1:] == (rows, C)
+    (a, sa), (b, sb) = (list(pending) + [(None, 0.0)] * 2)[:2]
+    taps = 0 if conv_w is None else conv_w.shape[1]
+    out = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device)
+    _check(_load().nx_stream_step(
+        _p(x), _p(a), 0 if a is None else a.shape[0], ctypes.c_float(sa), _p(b),
+        0 if b is None else b.shape[0], ctypes.c_float(sb), _p(_f32(norm_w)), ctypes.c_float(eps),
+        _p(None if conv_w is None else _f32(conv_w)), _p(tail), taps,
+        _p(step.positions if taps else None), _p(step.seq_ids if taps else None), _p(out), ctypes.c_long(rows), C, _stream()), "stream_step")
+    return out
 
 
 HEAD_PRODUCT_MAX_TOKENS = 256

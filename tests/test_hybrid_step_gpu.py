@@ -1,0 +1,226 @@
+"""Single tokens of the hybrid decoder in fewer launches, against its modules one by one."""
+
+import copy
+import sys
+
+import pytest
+import torch
+
+from neuronx_distributed_inference_amd import ops
+from neuronx_distributed_inference_amd.config import EngineConfig
+from neuronx_distributed_inference_amd.models.nabelix.modeling_nabelix import (
+    NabelixForCausalLM,
+    NabelixInferenceConfig,
+)
+from neuronx_distributed_inference_amd.ops import seqmix
+
+sys.path.insert(0, __file__.rsplit("/", 1)[0])
+from test_nabelix import layer_cfg, left_cfg, make_weights, model_cfg, right_cfg  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+F64 = torch.float64
+BF = torch.bfloat16
+
+
+def _model(slots, taps=4, conv=4, width=512, dim=128, loop=None, ff=768, layers=2, heads=4):
+    layer = layer_cfg(left_cfg(heads, 2, dim, dim, size=24, keep=3, scale=dim ** -0.5),
+                      right_cfg(heads, heads, dim, dim, conv=conv, decay_rank=64, gate_rank=64), ff=ff)
+    cfg = model_cfg([layer] * layers, width=width, vocab=96, taps=taps,
+                    loop=loop or {"start": 0, "stop": 0, "times": 1})
+    # a feed-forward every other layer where there is none in one
+    if ff and layers > 1:
+        cfg["layers"] = [copy.deepcopy(layer) for _ in range(layers)]
+        cfg["layers"][0]["mlp"] = None
+    ec = EngineConfig(batch_size=slots, max_batch_size=slots, kv_cache_batch_size=slots,
+                      seq_len=64, max_length=64, torch_dtype="bfloat16", tp_degree=1,
+                      is_block_kv_layout=True, pa_block_size=16, pa_num_blocks=4 * slots,
+                      enable_hip_graphs=False)
+    config = NabelixInferenceConfig(neuron_config=ec, **copy.deepcopy(cfg))
+    lm = NabelixForCausalLM(config)
+    sd = NabelixForCausalLM.convert_hf_to_native_state_dict(make_weights(cfg), config)
+    lm.model.load_state_dict(sd, strict=False)
+    return lm.cuda().eval()
+
+
+def _everything(lm):
+    mgr = lm.model.kv_mgr
+    out = {n: t for n, t in mgr.named_buffers()}
+    runs = len(lm.model.layer_runs())
+    for i in range(runs):
+        out.update({"k%d" % i: mgr.get_cache(i)[0].data, "v%d" % i: mgr.get_cache(i)[1].data})
+        for n in ("canon", "conv", "mem"):
+            out["%s%d" % (n, i)] = mgr.state.get("run%d.%s" % (i, n))
+    return {n: t.detach() for n, t in out.items()}
+
+
+def _steps(lm, B, pads=()):
+    """Three steps from a state and cache of noise; logits and all that the steps leave behind."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    with torch.inference_mode():
+        for n, t in _everything(lm).items():
+            if t.is_floating_point():
+                t.copy_(torch.empty(t.shape, device="cuda").normal_(0, 0.3, generator=g))
+        pos = torch.randint(2, 60, (B, 1), generator=g, device="cuda")
+        pos[0] = 0                                             # a sequence's first token
+        seq = torch.arange(B, device="cuda")
+        for b in pads:
+            seq[b] = pos[b] = -1
+        logits = []
+        for i in range(3):
+            ids = torch.randint(0, 96, (B, 1), generator=g, device="cuda")
+            logits.append(lm.model(ids, None, torch.where(pos < 0, pos, pos + i), seq)[1])
+        return torch.stack(logits), {n: t.clone() for n, t in _everything(lm).items()}
+
+
+@pytest.mark.parametrize("B,kw", [
+    (1, {}), (2, dict(taps=2, conv=3)), (16, dict(taps=3, conv=2, dim=64)), (17, dict(width=2112)),
+    (33, dict(loop={"start": 0, "stop": 2, "times": 2})), (65, dict(width=4160, ff=256)),
+    (130, dict(ff=0))])
+def test_steps_in_fewer_launches(B, kw):
+    lm = _model(B, **kw)
+    pads = (1, B - 1) if B > 4 else ()
+    # the modules' sums of two products and their activations are rounded to 16 bits on the way
+    took = []
+    inner = lm.model._steps_once
+    lm.model._steps_once = lambda p: took.append(inner(p)) or took[-1]
+    got, after = _steps(lm, B, pads)
+    assert took == [True] * 3
+    lm.model._steps_once = lambda p: False
+    want, before = _steps(lm, B, pads)
+    live = [b for b in range(B) if b not in pads]
+    assert (got[:, live] - want[:, live]).norm() <= 0.03 * want[:, live].norm()
+    for n, t in before.items():
+        if t.is_floating_point():
+            assert (after[n].float() - t.float()).norm() <= 0.03 * t.float().norm() + 1e-6, n
+            # what no row owns stays as it was
+            assert after[n].shape == t.shape
+
+
+def test_hooks_keep_the_modules():
+    lm = _model(2)
+    for module in (lm.model.layers[0], lm.model.layers[1].mlp, lm.model.layers[0].mixer.right.conv,
+                   lm.model.layers[1].mixer.in_proj, lm.model.norm):
+        seen = []
+        hook = module.register_forward_hook(lambda *a: seen.append(1))
+        _steps(lm, 2)
+        assert seen and not lm.model.kv_mgr.step.fused
+        hook.remove()
+    _steps(lm, 2)
+    assert lm.model.kv_mgr.step.fused
+
+
+@pytest.mark.parametrize("C", [8, 2048, 2056, 4104, 8192])
+@pytest.mark.parametrize("taps", [0, 2, 3, 4])
+@pytest.mark.parametrize("na,nb", [(0, 0), (1, 0), (4, 5), (16, 3)])
+def test_stream_step(C, taps, na, nb):
+    B = 5
+    g = torch.Generator(device="cuda").manual_seed(C + taps)
+    rnd = lambda *s: torch.empty(*s, device="cuda").normal_(0, 1, generator=g)  # noqa: E731
+    x, w = rnd(B, 1, C), rnd(C)
+    pend = [(rnd(n, B, C), sc) for n, sc in ((na, 0.7), (nb, -1.3)) if n]
+    step = seqmix.StepLayout(torch.tensor([[0], [1], [2], [-1], [9]], device="cuda"),
+                             torch.tensor([2, 0, 5, 3, -1], device="cuda"))
+    cw, tail = (rnd(C, taps), rnd(6, taps - 1, C)) if taps else (None, None)
+    xw = x.to(F64) + sum((sc * p.to(F64).sum(0).view(B, 1, C) for p, sc in pend), torch.zeros((), device="cuda"))
+    hn = torch.nn.functional.layer_norm(xw, (C,), w.to(F64), None, 1e-5)
+    want = hn
+    if taps:
+        want, want_tail = hn.clone(), tail.clone()
+        for b, (p, s) in enumerate([(0, 2), (1, 0), (2, 5), (-1, 3), (9, -1)]):
+            if p < 0 or s < 0:
+                want[b] = 0
+                continue
+            t = tail[s].to(F64)
+            t[:max(0, taps - 1 - p)] = 0
+            cols = torch.cat([t, hn[b]])
+            want[b, 0] += (cols * cw.to(F64).t()).sum(0)
+            want_tail[s] = cols[1:].float()
+    got = seqmix.stream_step(x, pend, w, 1e-5, step, cw, tail)
+    assert got.dtype == BF and got.shape == x.shape
+    # 2^-8: a rounding to bf16; sums of up to 20 values of 32 bits, a norm and 5 products
+    size = 4 * (xw.abs().amax() + 30)
+    assert (x.to(F64) - xw).abs().amax() <= 2.0 ** -22 * size
+    assert ((got.to(F64) - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -19 * size).all()
+    if taps:
+        assert (tail.to(F64) - want_tail).abs().amax() <= 2.0 ** -19 * size
+
+
+@pytest.mark.parametrize("B,H,D,Dv,taps,per_head", [(1, 1, 128, 128, 4, False), (3, 4, 64, 72, 2, False),
+                                                    (7, 2, 128, 16, 3, True), (5, 3, 64, 128, 4, True)])
+def test_delta_step_with_its_convolution(B, H, D, Dv, taps, per_head):
+    g = torch.Generator(device="cuda").manual_seed(B)
+    rnd = lambda *s: torch.empty(*s, device="cuda").normal_(0, 1, generator=g)  # noqa: E731
+    C = 2 * H * D + H * Dv
+    wide = rnd(B, C + 32).to(BF)
+    qkv, beta, a, gate = wide[:, 8:8 + C], rnd(B, H).to(BF), rnd(B, H if per_head else H * D).to(BF), \
+        rnd(B, H * Dv).to(BF)
+    cw, tail, state = rnd(C, taps), rnd(B + 2, taps - 1, C), 0.1 * rnd(B + 2, H, Dv, D)
+    bias, a_log, nw = rnd(a.shape[1]), rnd(H), rnd(Dv)
+    pos = torch.arange(B, device="cuda").view(B, 1) - int(B > 3)
+    step = seqmix.StepLayout(pos, torch.arange(B, device="cuda").flip(0) + 1)
+    t2, s2 = tail.clone(), state.clone()
+    got = seqmix.gated_delta_conv(qkv, cw, tail, beta, a, bias, a_log, gate, nw, 1e-5, state, step, D, Dv)
+    c = seqmix.short_conv_step(qkv.unsqueeze(1), cw, t2, step, "silu", False, torch.float32)
+    want = seqmix.gated_delta_rule(c, beta.unsqueeze(1), a.unsqueeze(1), bias, a_log, gate.unsqueeze(1), nw,
+                                   1e-5, s2, step, H, D, Dv, out_dtype=BF)
+    # the same sums in the same order
+    assert torch.equal(got, want[:, 0]) and torch.equal(tail, t2) and torch.equal(state, s2)
+
+
+@pytest.mark.parametrize("B,H,G,D,page,bad", [(1, 2, 2, 128, 16, False), (9, 8, 2, 64, 64, False),
+                                              (5, 40, 1, 128, 7, False), (4, 4, 4, 128, 32, True)])
+def test_window_attention_writes_its_rows(B, H, G, D, page, bad):
+    g = torch.Generator(device="cuda").manual_seed(D)
+    rnd = lambda *s: torch.empty(*s, device="cuda").normal_(0, 1, generator=g).to(BF)  # noqa: E731
+    pages = 8 * B
+    kc, vc = rnd(pages, page, G, D), rnd(pages, page, G, D)
+    q, k, v, gate = rnd(B, 1, H * D), rnd(B, G * D), rnd(B, G * D), rnd(B, 1, H * D)
+    if bad:
+        v[0, 3] = float("inf")
+        v[1, 5] = float("nan")
+    pos = torch.randint(0, 8 * page, (B, 1), generator=g, device="cuda")
+    pos[0] = 0
+    seq = torch.arange(B, device="cuda")
+    if B > 6:
+        seq[3] = pos[3] = -1
+    step = seqmix.StepLayout(pos, seq)
+    table = torch.randperm(pages, generator=g, device="cuda").view(B, 8).int()
+    slots = torch.where(pos < 0, -1, table.gather(1, pos.clamp(min=0) // page) * page + pos % page).view(-1)
+    r1, r2 = torch.rand(H, device="cuda"), torch.rand(H, device="cuda")
+    call = lambda kc, vc, **kw: seqmix.window_bias_attention(  # noqa: E731
+        q, kc, vc, step, table, r1, r2, D ** -0.5, 33, 2, H, gate=gate, **kw)
+    k1, v1 = kc.clone(), vc.clone()
+    assert seqmix.new_rows_taken(q, k, v, gate, kc, vc)
+    got = call(k1, v1, new_rows=(k, v, slots))
+    seqmix.paged_kv_write(kc, vc, k, v, slots, step)
+    want = call(kc, vc)
+    live = seq >= 0
+    for x, y in ((got[live], want[live]), (k1, kc), (v1, vc)):
+        assert torch.equal(x.view(torch.int16), y.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 64, 128), (17, 4096, 128), (48, 11408, 2048), (64, 1000, 256),
+                                   (100, 16384, 512), (129, 2048, 256)])
+def test_products_of_whole_results(M, N, K):
+    """Rows that lie apart, gelu, and two products in one launch."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    rnd = lambda *s: torch.empty(*s, device="cuda").normal_(0, 1, generator=g).to(BF)  # noqa: E731
+    x, w, x2, w2 = rnd(M, K + 24)[:, 16:16 + K], rnd(N, K), rnd(M, K), rnd(N, K)
+    d = lambda t: t.to(F64)  # noqa: E731
+    e1, e2 = d(x) @ d(w).t(), d(x2) @ d(w2).t()
+    s1, s2 = (K * 2.0 ** -24 * (d(a).abs() @ d(b).abs().t()) for a, b in ((x, w), (x2, w2)))
+    assert ops._C.tile_gemm_splits(M, N, K, 0, True) >= 1
+    y = ops._C.tile_gemm(x, w)
+    assert ((d(y) - e1).abs() <= s1 + 2.0 ** -8 * e1.abs() + 1e-30).all()
+    if K >= 256:
+        parts = d(ops._C.tile_gemm_pair(x, w, x2, w2))
+        n = parts.shape[0] // 2
+        assert ((parts[:n].sum(0) - e1).abs() <= s1 + 1e-30).all()
+        assert ((parts[n:].sum(0) - e2).abs() <= s2 + 1e-30).all()
+        gate, up = e1[:, : N // 2], e1[:, N // 2:]
+        want = torch.nn.functional.gelu(gate, approximate="tanh") * up
+        y = ops._C.tile_gemm(x, w, glu=2)
+        # the slope of gelu stays below 1.13; tanh of 32 bits beside one: 2^-22 of the gate
+        limit = 1.13 * s1[:, : N // 2] * up.abs() + gate.abs() * s1[:, N // 2:] \
+            + 2.0 ** -8 * want.abs() + 2.0 ** -21 * (gate * up).abs() + 1e-6
+        assert ((d(y) - want).abs() <= limit).all()
