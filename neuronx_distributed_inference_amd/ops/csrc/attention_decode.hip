@@ -337,10 +337,10 @@ __global__ __launch_bounds__(256) void decode_attn_pass1(
 // time through the matrix pipe and the vector units are left with one exponential a score:
 //   * S^T = K Q^T on 16x16x32 tiles: the rows are keys, the columns up to 16 (query token,
 //     head of the group) pairs, so every K row is used by all of them. The A operand is 16
-//     contiguous bytes of a key row: it comes straight from memory, without LDS.
+//     contiguous bytes of a key row.
 //   * O = P V: the C layout of S^T gives a lane 4 consecutive keys of its column in each of
 //     the two 16-key tiles, which is the A operand of P for the same 32 keys in another
-//     order. V rows are loaded in that order, 16 bytes of channels a lane (a whole row for
+//     order. V rows are read in that order, 16 bytes of channels a lane (a whole row for
 //     16 lanes), and turned in registers: one byte permutation makes a B operand word. Which
 //     channels a column of the product stands for is free, so nothing else moves.
 //   * P enters as three 16-bit parts that add up to its 24 bits. (Two parts: 64 rows of 2048 73.1
@@ -351,14 +351,22 @@ __global__ __launch_bounds__(256) void decode_attn_pass1(
 //     most: far from overflow, and what lies deeper is less than a 32-bit sum keeps. One key
 //     whose values are 10^-4 of the others' ahead of 60000 at e^-19, fp16, error 2-norm: 1.9e-4
 //     (two parts and one reference 4.2e-3, 32-bit multiply-adds of scaled queries 5.1e-4).
-//   * Loads of the next 32 keys are in flight while these are computed (two register
-//     buffers, 16 KB a wave); waves of a workgroup take 32-key tiles in turn and meet in LDS
-//     once at the end.
+//   * The next 32 keys are on their way while these are computed: straight to LDS (STAGED), into
+//     a place of the wave's own, so that no wave waits for another, and from there to the
+//     registers just before they are computed. What a CU holds in flight is some 140 lines of
+//     128 bytes, and a load that asks for 64 bytes of each of 16 rows (K as the matrix operand
+//     wants it; 32 bytes in 8 bits) takes a line for half of one: staged, every load is of whole
+//     lines, and past the caches. (Streaming alone, 64 rows of 1024 to 2048 keys: 71.6 us as
+//     operands, 61.5 as whole lines, not cached.) Caches that start off 16 bytes go straight to
+//     two register buffers, as all did. Waves of a workgroup take 32-key tiles in turn and meet in
+//     LDS once at the end.
 //   * The accumulator is rescaled only when a maximum grew by more than 2^8.
 // Measured in a captured graph (MI355X, bf16, 32/8 heads of 128, lengths half to full, before ->
 // now, stream rate): 64 rows of 2048 131 -> 76 us (5.3 TB/s); 16 of 8192 136 -> 73; 128 of 512
 // 68 -> 40; 256 of 168 57 -> 28; 1 of 300 18.2 -> 7.8; 1 of 8192 55 -> 12; 13 rows of 8000, 64/8
-// heads 271 -> 72 us, e4m3 279 -> 48 us. Error against 64 bits, bf16: 1.66e-3 (the rounding of
+// heads 271 -> 72 us, e4m3 279 -> 48 us. Straight to registers -> staged: 64 rows of 2048 75.5 ->
+// 66.5 us (6.1 TB/s), in pages 88 -> 78.5; 256 of 168 36.0 -> 31.8; 13 of 8000, e4m3, 44.7 -> 35.1;
+// 100 of 1200, heads of 64, 41.0 -> 36.6; 1 row the same. Error against 64 bits, bf16: 1.66e-3 (the rounding of
 // the result), before 1.66e-3 to 3.5e-3 (the scaled query was rounded too).
 typedef __bf16 dm_bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 dm_f16x8 __attribute__((ext_vector_type(8)));
@@ -430,12 +438,18 @@ template <int NE, bool F8> struct DmRaw {
     }
 };
 
+// 16 bytes a lane to the 1 KB of LDS at dst; past the caches, which a step's keys would only sweep
+DEV_INLINE void dm_load_lds(const char* src, char* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) unsigned int*)src,
+                                     (__attribute__((address_space(3))) unsigned int*)dst, 16, 0, 2);
+}
+
 constexpr float DM_GROWTH = 8.f;   // log2 growth of a maximum that is put off
 constexpr float DM_DEPTH = 64.f;   // and how far below the largest score P may count from (fp16)
 constexpr int DM_TILE = 32;        // keys of a wave's step
 constexpr int DM_LEAST = 128;      // keys of a split: one step of each wave
 
-template <typename T, typename CT, int D, bool PAGED, int WPR>
+template <typename T, typename CT, int D, bool PAGED, int WPR, bool STAGED>
 __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
     T* __restrict__ out,               // (B, Hq, Sq, D), written when nsplit == 1
     float* __restrict__ o_part,        // (B, Hq, Sq, nsplit, D)
@@ -537,6 +551,53 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
         DmRaw<8, F8> k[2][NKS];
         DmRaw<DV, F8> v[8];
         unsigned bad;              // bit j: key j of the lane has no page
+    };
+    // STAGED: the wave's tile in LDS, K then V, 16-byte pieces of a row in the order piece ^ turn(row)
+    extern __shared__ __attribute__((aligned(16))) float dm_lds[];
+    constexpr int ROWB = D * ES, PPR = ROWB / 16, RPI = 64 / PPR, TILE_B = DM_TILE * ROWB;
+    char* const tile = reinterpret_cast<char*>(dm_lds) + wid * 2 * TILE_B;
+    auto turn = [](int r) { return PPR == 4 ? (r >> 1) & 3 : r & (PPR - 1); };
+    auto stage = [&](int t, int blk) -> unsigned {
+        unsigned bad = 0;
+        int prow = 0;                  // cache row of the lane's key, -1: no page
+        if constexpr (PAGED) prow = blk < 0 ? -1 : blk * block_size + page_key(t) % block_size;
+#pragma unroll
+        for (int i = 0; i < DM_TILE / RPI; ++i) {
+            const int r = i * RPI + lane / PPR;
+            const int at = ((lane % PPR) ^ turn(r)) * 16;
+            const char *kp, *vp;
+            if constexpr (PAGED) {
+                const long off = ((long)max(__shfl(prow, r, WAVE_SIZE), 0) * Hkv + hkv) * ROWB + at;
+                kp = kbase + off;
+                vp = vbase + off;
+            } else {
+                const unsigned off = (unsigned)(min(t * DM_TILE + r, last) * ROWB) + at;
+                kp = kbase + off;
+                vp = vbase + off;
+            }
+            dm_load_lds(kp, tile + i * 1024);
+            dm_load_lds(vp, tile + TILE_B + i * 1024);
+        }
+        if constexpr (PAGED) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                bad |= ((unsigned)__shfl(prow, (j >> 2) * 16 + g * 4 + (j & 3), WAVE_SIZE) >> 31) << j;
+        }
+        return bad;
+    };
+    auto fetch = [&](Buf& u) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) {
+                const int r = kb * 16 + n, at = (ks * 32 + g * 8) * ES;
+                u.k[kb][ks].load(tile + r * ROWB + (((at >> 4) ^ turn(r)) << 4) + (at & 15));
+            }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int r = (j >> 2) * 16 + g * 4 + (j & 3), at = n * DV * ES;
+            u.v[j].load(tile + TILE_B + r * ROWB + (((at >> 4) ^ turn(r)) << 4) + (at & 15));
+        }
     };
     auto load = [&](Buf& u, int t, int blk) {
         u.bad = 0;
@@ -657,7 +718,29 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
         }
     };
 
-    if (t_lo + sub < t_hi) {
+    if constexpr (STAGED) {
+        if (t_lo + sub < t_hi) {
+            int t = t_lo + sub;
+            unsigned bad = stage(t, page_load(t));
+            int blk = page_load(t + WPR);
+            for (;; t += WPR) {
+                Buf u;
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                fetch(u);
+                u.bad = bad;
+                if (t + WPR >= t_hi) {
+                    step(u, t);
+                    break;
+                }
+                // into registers before the next tile lands in their place
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                bad = stage(t + WPR, blk);
+                blk = page_load(t + 2 * WPR);
+                step(u, t);
+            }
+        }
+        __syncthreads();                       // the tiles' place is the waves' meeting place
+    } else if (t_lo + sub < t_hi) {
         Buf u0, u1;
         int t = t_lo + sub;
         int blk = page_load(t), next = page_load(t + WPR);
@@ -681,7 +764,6 @@ __global__ __launch_bounds__(256, 2) void decode_mfma_kernel(
     m -= LIFT;
 
     // ---- the waves of a set meet ----
-    extern __shared__ __attribute__((aligned(16))) float dm_lds[];
     float* o_lds = dm_lds;                     // [4][ncw][D]
     float* ml_lds = dm_lds + 4 * ncw * D;      // [4][16][2]
     if (g == 0) {
@@ -873,8 +955,8 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
     constexpr bool MFMA = !std::is_same<T, float>::value && (D == 64 || D == 128);
     const int nct = (gq * Sq + 15) / 16;
     // Splits over the keys. Matrix-core kernel: two workgroups fit a CU, so 512 fill the chip;
-    // more only add partial sums to write and combine (64 rows of 2048: 76 us at 512, 84 at
-    // 1024, 87 at 2048; 128 rows of 512: 40 / 40 / 52), as rows of unequal length even out over
+    // more only add partial sums to write and combine (64 rows of 2048: 68 us at 512, 72 at
+    // 1024, 73 at 2048; 13 rows of 8000 of 8 heads in 8 bits 36 / 38 / 44), as rows of unequal length even out over
     // the CUs by themselves. A split keeps 128 rows, one step of each wave (1 row of 300: 7.8 us;
     // 256: 8.4), 256 in long caches where the combining pass weighs more (1 row of 8192: 11.8 us
     // with 256, 13.5 with 128). Their number goes by the capacity, which the host knows; what
@@ -905,7 +987,9 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
     if constexpr (MFMA) {
         if (B == 0 || Sq == 0) return;
         const int nc = std::min(16, gq * Sq);
-        const size_t lds = (4 * nc * D + 4 * 16 * 2) * sizeof(float);
+        const bool staged = ((size_t)k_cache.data_ptr() | (size_t)v_cache.data_ptr()) % 16 == 0;
+        const size_t lds = std::max((4 * nc * D + 4 * 16 * 2) * sizeof(float),
+                                    staged ? 4 * 2 * DM_TILE * D * sizeof(CT) : 0);
         const long sets = (long)B * Hkv * nct;
         // Waves of a set of columns (of one row's KV head). Where rows are short a workgroup is
         // gone after a step or two of its waves, and what it waits for on the way (positions,
@@ -930,7 +1014,12 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
         TORCH_CHECK(sets < (1L << 31), "attention_decode: too many rows");
         const dim3 grid = alone ? dim3((unsigned)((sets + 3) / 4)) : dim3(nsplit, Hkv * nct, B);
 #define DM_GO(PG, W)                                                                        \
-        hipLaunchKernelGGL((decode_mfma_kernel<T, CT, D, PG, W>), grid, dim3(256), lds, stream, \
+        do {                                                                                \
+            if (staged) DM_RUN(PG, W, true);                                                \
+            else DM_RUN(PG, W, false);                                                      \
+        } while (0)
+#define DM_RUN(PG, W, ST)                                                                   \
+        hipLaunchKernelGGL((decode_mfma_kernel<T, CT, D, PG, W, ST>), grid, dim3(256), lds, stream, \
                            (T*)out.data_ptr(), o_part.data_ptr<float>(),                    \
                            ml_part.data_ptr<float>(), (const T*)q.data_ptr(),               \
                            (const CT*)k_cache.data_ptr(), (const CT*)v_cache.data_ptr(),    \
@@ -947,6 +1036,7 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
             else DM_GO(false, 4);
         }
 #undef DM_GO
+#undef DM_RUN
         HIP_CHECK_KERNEL();
         if (nsplit == 1) return;
     } else if (paged) {

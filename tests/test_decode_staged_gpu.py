@@ -1,0 +1,60 @@
+"""Decode attention over keys and values that go through LDS, against caches that start off 16 bytes,
+which go straight to registers: the same sums in the same order."""
+
+import pytest
+import torch
+
+from neuronx_distributed_inference_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _off(t):
+    """A copy that starts 8 bytes behind 16."""
+    n = 8 // t.element_size()
+    flat = torch.empty(t.numel() + 2 * n, dtype=t.dtype, device=t.device)
+    at = n if flat.data_ptr() % 16 == 0 else 0
+    copy = flat[at:at + t.numel()].view(t.shape)
+    copy.copy_(t)
+    assert copy.data_ptr() % 16 == 8
+    return copy
+
+
+# a wave's step is 32 keys, a workgroup's 128, splits keep 128 or 256; 768 sets go a wave a set
+@pytest.mark.parametrize("B,Hkv,gq,cap", [(1, 1, 1, 1), (2, 2, 4, 31), (3, 2, 8, 32), (2, 8, 1, 33), (1, 2, 16, 129),
+                                          (5, 3, 4, 257), (1, 8, 4, 4097), (64, 8, 2, 700), (97, 8, 4, 200)])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype,f8", [(torch.bfloat16, False), (torch.float16, False), (torch.bfloat16, True)])
+@pytest.mark.parametrize("window", [0, 40])
+def test_staged_as_straight(B, Hkv, gq, cap, D, dtype, f8, window):
+    g = torch.Generator(device="cuda").manual_seed(cap)
+    rnd = lambda *s: torch.empty(*s, device="cuda").normal_(0, 1, generator=g).to(dtype)  # noqa: E731
+    q, k, v = rnd(B, Hkv * gq, 1, D), rnd(B, Hkv, cap, D), rnd(B, Hkv, cap, D)
+    if f8:
+        k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+    else:
+        v[0, 0, cap // 2, 3] = float("nan")
+    pos = torch.randint(0, cap, (B, 1), generator=g, device="cuda")
+    pos[-1] = cap - 1
+    if B > 2:
+        pos[1] = -1
+    call = lambda k, v: ops.attention_decode(q, k, v, pos, sliding_window=window)  # noqa: E731
+    a, b = call(k, v), call(_off(k), _off(v))
+    assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("B,Hkv,gq,pages,size", [(1, 2, 4, 1, 16), (3, 2, 8, 5, 7), (2, 8, 4, 33, 64), (100, 8, 1, 4, 32)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_staged_pages_as_straight(B, Hkv, gq, pages, size, D):
+    g = torch.Generator(device="cuda").manual_seed(pages)
+    rnd = lambda *s: torch.empty(*s, device="cuda").normal_(0, 1, generator=g).to(torch.bfloat16)  # noqa: E731
+    n = B * pages + 1
+    q, k, v = rnd(B, Hkv * gq, 1, D), rnd(n, size, Hkv, D), rnd(n, size, Hkv, D)
+    v[0] = float("nan")                                # what stands in for a missing page
+    table = (torch.randperm(n - 1, generator=g, device="cuda") + 1).view(B, pages).int()
+    if pages > 2:
+        table[0, 1] = -1
+    pos = torch.randint(0, pages * size, (B, 1), generator=g, device="cuda")
+    call = lambda k, v: ops.attention_decode_paged(q, k, v, pos, table)  # noqa: E731
+    a, b = call(k, v), call(_off(k), _off(v))
+    assert a.isfinite().all() and torch.equal(a.view(torch.int16), b.view(torch.int16))
