@@ -1520,11 +1520,13 @@ __global__ void __launch_bounds__(256, 2) window_flash_kernel(const WfArgs a) {
 
 // Single tokens, heads of 64 and 128: the same scores and options in bf16. Bound by the keys' and
 // values' bytes; a workgroup has one token's heads of a KV head (16 at most) and its 8 waves take
-// tiles of 32 keys in turn, straight to registers, the next tile in flight while one is computed
-// and the pages looked up a tile before that. Scores are K Q^T (mfma 16x16x32), so that P sits in
+// tiles of 32 keys in turn, straight to registers or (STAGED) each to a place of its own in LDS in
+// loads of whole lines (as operands a load takes 64 bytes of each of 16 rows, and it is lines of 128
+// that a CU can have so many of in flight), the next tile on its way while one is computed and the
+// pages looked up a tile before that (OWN: see kn). Scores are K Q^T (mfma 16x16x32), so that P sits in
 // the registers as the operand of P V; it enters in three 16-bit parts, which add up to its 24
 // bits. The waves meet once, in LDS. 48 rows, 16 heads of 128 on 4 KV heads, 350 to 700 keys,
-// log-distance bias, gate: 41 us by multiply-adds (window_attn_kernel), 22 now. With kn and vn the
+// log-distance bias, gate: 41 us by multiply-adds (window_attn_kernel), 19 straight, 17 staged. With kn and vn the
 // token's own key and value come from there and go into the cache on the way, where a launch of its
 // own took 4.8 us.
 struct WdBuf {
@@ -1534,7 +1536,12 @@ struct WdBuf {
 #define WD_WAVES 8
 #define WD_KT 32
 
-template <int D>
+DEV void wd_load_lds(const bf16* src, char* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) unsigned int*)src,
+                                     (__attribute__((address_space(3))) unsigned int*)dst, 16, 0, 2);
+}
+
+template <int D, bool STAGED, bool OWN>
 __global__ void __launch_bounds__(WD_WAVES * WAVE) window_decode_kernel(const WfArgs a) {
     constexpr int NKS = D / 32, DV = D / 16;
     const int rep = a.H / a.G, nct = (rep + 15) >> 4;
@@ -1565,10 +1572,10 @@ __global__ void __launch_bounds__(WD_WAVES * WAVE) window_decode_kernel(const Wf
     const int tiles = (nk + WD_KT - 1) / WD_KT;
     const int* bt = a.btab + (long)b * a.max_blocks;
     const bf16* kbase = a.kc + (long)g * a.khead;
-    const bf16* vbase = a.vc + (long)g * a.vhead + n * DV;
-    const bf16* kown = a.kn ? a.kn + (long)b * a.knstride + (long)g * D : nullptr;
-    const bf16* vown = a.kn ? a.vn + (long)b * a.vnstride + (long)g * D : nullptr;
-    if (kown && c0 == 0 && wid == WD_WAVES - 1 && lane < D / 4) {
+    const bf16* vbase = a.vc + (long)g * a.vhead;
+    const bf16* kown = OWN ? a.kn + (long)b * a.knstride + (long)g * D : nullptr;
+    const bf16* vown = OWN ? a.vn + (long)b * a.vnstride + (long)g * D : nullptr;
+    if (OWN && c0 == 0 && wid == WD_WAVES - 1 && lane < D / 4) {
         const long s = a.slots[b];
         const int e = lane % (D / 8) * 8;
         if (s >= 0 && s < a.nslots) {
@@ -1586,26 +1593,57 @@ __global__ void __launch_bounds__(WD_WAVES * WAVE) window_decode_kernel(const Wf
         const int m = min(t * WD_KT + (lane & 31), nk - 1), j = m < nfirst ? m : m + shift;
         const int page = a.page_shift >= 0 ? j >> a.page_shift : j / a.bsz;
         rem = j - page * a.bsz;
-        if (kown && m == nk - 1) {                       // the token's own
+        if (OWN && m == nk - 1) {                       // the token's own
             rem = -1;
             return 0;
         }
         return bt[page];
     };
-    auto load = [&](WdBuf& u, int page, int rem) {
+    // the wave's tile in LDS, K then V, 16-byte pieces of a row in the order piece ^ row
+    constexpr int ROWB = D * 2, PPR = ROWB / 16, RPI = 64 / PPR, TILE_B = WD_KT * ROWB;
+    extern __shared__ __attribute__((aligned(16))) float wd_lds[];
+    char* const tile = reinterpret_cast<char*>(wd_lds) + wid * 2 * TILE_B;
+    auto stage = [&](int page, int rem) {
         const int slot = max(page, 0) * a.bsz + rem;     // -1: the token's own
+#pragma unroll
+        for (int j = 0; j < WD_KT / RPI; ++j) {
+            const int r = j * RPI + lane / PPR, sl = __shfl(slot, r, WAVE);
+            const int at = ((lane % PPR) ^ (r & (PPR - 1))) * 8;
+            wd_load_lds((OWN && sl < 0 ? kown : kbase + (long)sl * a.ktok) + at, tile + j * 1024);
+            wd_load_lds((OWN && sl < 0 ? vown : vbase + (long)sl * a.vtok) + at, tile + TILE_B + j * 1024);
+        }
+    };
+    auto load = [&](WdBuf& u, int page, int rem) {
+        const int slot = max(page, 0) * a.bsz + rem;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
             const int sl = __shfl(slot, kb * 16 + n, WAVE);
-            const bf16* p = (sl < 0 ? kown : kbase + (long)sl * a.ktok) + q4 * 8;
+            const bf16* p = (OWN && sl < 0 ? kown : kbase + (long)sl * a.ktok) + q4 * 8;
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks) u.k[kb][ks] = *reinterpret_cast<const uint4*>(p + ks * 32);
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const int kk = (j >> 2) * 16 + q4 * 4 + (j & 3);
-            const int sl = __shfl(slot, kk, WAVE);
-            const bf16* p = sl < 0 ? vown + n * DV : vbase + (long)sl * a.vtok;
+            const int sl = __shfl(slot, (j >> 2) * 16 + q4 * 4 + (j & 3), WAVE);
+            const bf16* p = (OWN && sl < 0 ? vown : vbase + (long)sl * a.vtok) + n * DV;
+            if constexpr (DV == 8) u.v[j] = *reinterpret_cast<const uint4*>(p);
+            else {
+                const uint2 w = *reinterpret_cast<const uint2*>(p);
+                u.v[j].x = w.x;
+                u.v[j].y = w.y;
+            }
+        }
+    };
+    auto fetch = [&](WdBuf& u) {
+        auto piece = [&](int r, int at) { return r * ROWB + (((at >> 4) ^ (r & (PPR - 1))) << 4) + (at & 15); };
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks)
+                u.k[kb][ks] = *reinterpret_cast<const uint4*>(tile + piece(kb * 16 + n, ks * 64 + q4 * 16));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const char* p = tile + TILE_B + piece((j >> 2) * 16 + q4 * 4 + (j & 3), n * DV * 2);
             if constexpr (DV == 8) u.v[j] = *reinterpret_cast<const uint4*>(p);
             else {
                 const uint2 w = *reinterpret_cast<const uint2*>(p);
@@ -1686,7 +1724,28 @@ __global__ void __launch_bounds__(WD_WAVES * WAVE) window_decode_kernel(const Wf
                 o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p[k], vb, o[d], 0, 0, 0);
         }
     };
-    if (wid < tiles) {
+    if constexpr (STAGED) {
+        if (wid < tiles) {
+            int rem, page = look_up(wid, rem);
+            stage(page, rem);
+            page = look_up(wid + WD_WAVES, rem);
+            for (int t = wid;; t += WD_WAVES) {
+                WdBuf u;
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                fetch(u);
+                if (t + WD_WAVES >= tiles) {
+                    step(u, t);
+                    break;
+                }
+                // in registers before the next tile lands in their place
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                stage(page, rem);
+                page = look_up(t + 2 * WD_WAVES, rem);
+                step(u, t);
+            }
+        }
+        __syncthreads();                                 // the tiles' place is the waves' meeting place
+    } else if (wid < tiles) {
         WdBuf u0, u1;
         int t = wid, r0, r1;
         int p0 = look_up(t, r0), p1 = look_up(t + WD_WAVES, r1);
@@ -1710,8 +1769,7 @@ __global__ void __launch_bounds__(WD_WAVES * WAVE) window_decode_kernel(const Wf
 
     // ---- the waves meet ----
     // the row that was written may be read again below
-    if (kown && wid == WD_WAVES - 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    extern __shared__ __attribute__((aligned(16))) float wd_lds[];
+    if (OWN && wid == WD_WAVES - 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     float* ml = wd_lds;                                  // [waves][16][2]
     float* ol = wd_lds + WD_WAVES * 32;                  // [waves][nc][D]
     if (q4 == 0) {
@@ -5759,10 +5817,22 @@ int nx_paged_attn(const void* q, long qstride, const void* kc, long ktok, long k
             f.kn = (const bf16*)kn; f.vn = (const bf16*)vn; f.slots = slots; f.nslots = nslots;
             f.kw = (bf16*)kc; f.vw = (bf16*)vc; f.knstride = knstride; f.vnstride = vnstride;
             const int nc = rp < 16 ? rp : 16;
-            const int lds = S == 1 ? (WD_WAVES * 32 + WD_WAVES * nc * Dk) * 4
-                                   : 4 * WF_KT * Dk * 2 + 64;
-            auto* k = S == 1 ? (Dk == 128 ? window_decode_kernel<128> : window_decode_kernel<64>)
+            // Through LDS where the keys' bytes bound it: many rows of 4 steps of a wave and more.
+            // Few rows, or short ones, wait a little longer for their first keys that way. 16 heads of
+            // 128 on 4 KV heads, half to full caches of 384 / 768 / 1472 keys, straight -> staged:
+            // 16 rows 9.6 -> 10.4, 14.7 -> 15.0, 21.4 -> 19.6 us; 32 10.0 -> 11.1, 17.7 -> 16.0,
+            // 23.7 -> 22.0; 48 10.9 -> 11.6, 19.0 -> 17.1, 26.5 -> 24.5; 100 rows of 1000, 8 heads of 64,
+            // 50.6 -> 42.3.
+            const long seen = (long)max_blocks * bsz, span = (long)window + keep;
+            const bool staged = (long)B * G * ((rp + 15) / 16) >= 96 && (seen < span ? seen : span) >= 512;
+#define WDK(DD) (staged ? (kn ? window_decode_kernel<DD, true, true> : window_decode_kernel<DD, true, false>) \
+                        : (kn ? window_decode_kernel<DD, false, true> : window_decode_kernel<DD, false, false>))
+            auto* k = S == 1 ? (Dk == 128 ? WDK(128) : WDK(64))
                              : (Dk == 128 ? window_flash_kernel<128> : window_flash_kernel<64>);
+            const int meet = (WD_WAVES * 32 + WD_WAVES * nc * Dk) * 4, tile = WD_WAVES * 2 * WD_KT * Dk * 2;
+            const int lds = S == 1 ? (staged && tile > meet ? tile : meet)
+                                   : 4 * WF_KT * Dk * 2 + 64;
+#undef WDK
             const dim3 grid = S == 1 ? dim3((unsigned)(G * ((rp + 15) / 16)), (unsigned)B)
                                      : dim3((unsigned)((long)f.nqt * B * G));
             if (hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -167,9 +167,10 @@ def test_delta_step_with_its_convolution(B, H, D, Dv, taps, per_head):
     assert torch.equal(got, want[:, 0]) and torch.equal(tail, t2) and torch.equal(state, s2)
 
 
-@pytest.mark.parametrize("B,H,G,D,page,bad", [(1, 2, 2, 128, 16, False), (9, 8, 2, 64, 64, False),
-                                              (5, 40, 1, 128, 7, False), (4, 4, 4, 128, 32, True)])
-def test_window_attention_writes_its_rows(B, H, G, D, page, bad):
+@pytest.mark.parametrize("B,H,G,D,page,bad,window", [
+    (1, 2, 2, 128, 16, False, 33), (9, 8, 2, 64, 64, False, 33), (5, 40, 1, 128, 7, False, 33),
+    (4, 4, 4, 128, 32, True, 33), (33, 16, 4, 128, 64, True, 700), (25, 8, 4, 64, 80, True, 510)])
+def test_window_attention_writes_its_rows(B, H, G, D, page, bad, window):
     g = torch.Generator(device="cuda").manual_seed(D)
     rnd = lambda *s: torch.empty(*s, device="cuda").normal_(0, 1, generator=g).to(BF)  # noqa: E731
     pages = 8 * B
@@ -188,7 +189,7 @@ def test_window_attention_writes_its_rows(B, H, G, D, page, bad):
     slots = torch.where(pos < 0, -1, table.gather(1, pos.clamp(min=0) // page) * page + pos % page).view(-1)
     r1, r2 = torch.rand(H, device="cuda"), torch.rand(H, device="cuda")
     call = lambda kc, vc, **kw: seqmix.window_bias_attention(  # noqa: E731
-        q, kc, vc, step, table, r1, r2, D ** -0.5, 33, 2, H, gate=gate, **kw)
+        q, kc, vc, step, table, r1, r2, D ** -0.5, window, 2, H, gate=gate, **kw)
     k1, v1 = kc.clone(), vc.clone()
     assert seqmix.new_rows_taken(q, k, v, gate, kc, vc)
     got = call(k1, v1, new_rows=(k, v, slots))
@@ -197,6 +198,30 @@ def test_window_attention_writes_its_rows(B, H, G, D, page, bad):
     live = seq >= 0
     for x, y in ((got[live], want[live]), (k1, kc), (v1, vc)):
         assert torch.equal(x.view(torch.int16), y.view(torch.int16))
+
+
+@pytest.mark.parametrize("B,H,G,D,page,pages,window", [
+    (96, 4, 1, 128, 16, 32, 512), (24, 64, 4, 64, 64, 9, 10 ** 6), (13, 160, 8, 128, 100, 20, 700)])
+def test_many_rows_through_lds_as_few_without(B, H, G, D, page, pages, window):
+    """Many long rows at once take another way to the registers than two at a time do."""
+    g = torch.Generator(device="cuda").manual_seed(D)
+    rnd = lambda *s: torch.empty(*s, device="cuda").normal_(0, 1, generator=g).to(BF)  # noqa: E731
+    kc, vc = rnd(B * pages, page, G, D), rnd(B * pages, page, G, D)
+    vc[5, 3] = float("inf")
+    q, r1, r2 = rnd(B, 1, H * D), torch.rand(H, device="cuda"), torch.rand(H, device="cuda")
+    pos = torch.randint(0, pages * page, (B, 1), generator=g, device="cuda")
+    pos[0] = pages * page - 1
+    table = torch.randperm(B * pages, generator=g, device="cuda").view(B, pages).int()
+    table[1, 1] = -1
+
+    def call(rows):
+        step = seqmix.StepLayout(pos[rows].contiguous(), torch.arange(pos[rows].shape[0], device="cuda"))
+        return seqmix.window_bias_attention(q[rows], kc, vc, step, table[rows].contiguous(), r1, r2,
+                                            D ** -0.5, window, 3, H)
+
+    got = call(slice(0, B))
+    want = torch.cat([call(slice(i, i + 1)) for i in range(B)])
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 64, 128), (17, 4096, 128), (48, 11408, 2048), (64, 1000, 256),
