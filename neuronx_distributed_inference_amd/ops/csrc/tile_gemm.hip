@@ -297,7 +297,7 @@ __global__ __launch_bounds__(256) void tile_sum_kernel(T* __restrict__ y,
 // The tile of a shape. A chunk of w (BN rows of 128 bytes) is what a workgroup streams, x comes
 // again and again from the L2: few rows take small tiles with a deep ring, so that a CU has 64 KB
 // and more on the way; many rows take tall ones, for fewer reads of x and w from LDS a product.
-enum TgTile { T16, T16N, T32, T32N, T64, T64N, T128, T128N, T128W, T128B, T192, T256W };
+enum TgTile { T16, T16N, T32, T32N, T64, T64N, T128, T128N, T128W, T128B, T192, T256, T256W };
 
 struct TgPlan {
     TgTile tile;
@@ -313,7 +313,7 @@ struct TgPlan {
 //   64      12.9 / 19.7   10.0 / 15.5    43.6 /  54.3   23.4 / 32.4   166 / 184
 //   128     17.0 / 21.4   14.0 / 18.9    50.5 /  60.4   29.8 / 43.2   154 / 221
 //   192     21.7 / 26.2   17.1 / 20.3    62.1 /  79     35.3 / 66.9   224 / 232
-//   256     24.2 / 27.2   17.8 / 25.2    75.2 /  84.1   43.5 / 53.4   268 / 239
+//   256     22.5 / 27.2   17.8 / 25.2    64.7 /  84.1   37.9 / 53.4   268 / 239
 //   512     34.9 / 38.2   25.5 / 29.7     123 /   105   62.1 / 89.2   442 / 375
 // so up to 256 rows, unless the tiles of more than 128 rows need a second round of the chip, and
 // up to 512 rows where the tiles of the outputs alone leave CUs idle. Parts of K fill the 256 CUs
@@ -321,8 +321,11 @@ struct TgPlan {
 // From 128 rows on what bounds them is what a CU takes in, x and w together: 40 to 43 GB/s in every
 // tile tried (chunks of x laid out in a row changed nothing, deeper rings of either no more), so a
 // tile of 192 rows, which reads w once for them, and x apart from w in time: 129 to 192 rows
-// 71.8 -> 62.9, 39.7 -> 35.0, 23.1 -> 20.8 (160 rows of the third, fourth and first shape; 256 rows
-// in one tile 74.2, 42.6, 24.5: no better than two of 128). Gate|up of few columns takes tiles of
+// 71.8 -> 62.9, 39.7 -> 35.0, 23.1 -> 20.8 (160 rows of the third, fourth and first shape). 193 to 256
+// rows in one tile as well, its w apart from the cache as nothing else reads it (tiles of 128 x 256 read
+// w twice): 256 rows of the third shape 69.5 -> 64.7, (32000, 4096) 76 -> 70, (8192, 28672) 139 -> 134,
+// (10240, 8192) 51.3 -> 50.0; more than 256 rows would fill a second tile in part only: 300 rows of
+// the first shape 33.9 with it, 28.4 without. Gate|up of few columns takes tiles of
 // 128 also where 256 would leave half of the CUs idle: 128 rows of the third shape 72.0 -> 50.5.
 // `whole`: no kernel follows that would add up parts. Then up to 64 rows take tiles of half the width
 // where these fill most of the chip undivided, also where those of the full width in two parts are
@@ -344,6 +347,7 @@ TgPlan tg_plan(long M, long N, long K, bool glu, bool whole) {
     else if (M <= 128) p = {T128W, 128, 256, 0};
     else if (N * K <= (20 << 20)) p = {T128B, 128, 128, 0};
     else if (M <= 192) p = {T192, 192, 128, 0};
+    else if (M <= 256) p = {T256, 256, 128, 0};
     else p = {T256W, 128, 256, 0};
     const long tiles = (M + p.bm - 1) / p.bm * ((N + p.bn - 1) / p.bn);
     if (M > 128 && tiles > 256) return p;
@@ -381,6 +385,7 @@ void tg_tile(TgArgs& a, TgTile tile, hipStream_t s) {
         case T128W: tg_go<T, 128, 256, 2, 4, 3, GLU, true>(a, s); break;
         case T128B: tg_go<T, 128, 128, 2, 4, 5, GLU, false>(a, s); break;
         case T192: tg_go<T, 192, 128, 4, 2, 5, GLU, true, 3>(a, s); break;
+        case T256: tg_go<T, 256, 128, 4, 2, 3, GLU, true>(a, s); break;
         case T256W: tg_go<T, 128, 256, 2, 4, 3, GLU, false>(a, s); break;
     }
 }

@@ -63,6 +63,14 @@ def test_tile_gemm_glu(M, N, K, dtype):
     assert ((y.to(F64) - want).abs() <= limit).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(193, 20616, 1088), (224, 6152, 4096), (255, 31000, 768)])
+def test_tile_gemm_256_rows(M, N, K):
+    """The tile of 256 rows: rows and columns short of it, a ring that ends in each of its slots."""
+    assert N * K > 20 << 20
+    test_tile_gemm(M, N, K, torch.bfloat16)
+    test_tile_gemm_glu(M, N, K, torch.float16)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 4096, 192), (1, 60, 256), (8, 66, 256), (8, 64, 260),
                                    (513, 4096, 4096), (512, 28672, 4096), (129, 57344, 8192)])
 def test_tile_gemm_leaves_to_the_library(M, N, K):
