@@ -13,6 +13,11 @@
 //     round of workgroups, so the height goes by the rows an expert has by chance and not only on
 //     average: 2048 tokens x 8 of 128 experts (128 rows +- 11) take 128 tiles of 160 rows, and
 //     would take 190 of 128.
+//   * An expert's weights that no other row tile wants come past the caches: at 2048 tokens of 128
+//     experts 347 -> 317 us, 64 tokens 221 -> 198; 128 tokens of 8 experts in 16 bits 515 -> 467, in
+//     8 bits 281 -> 264. Where another wants them they are shared in the L2 (1024 tokens of 8 experts
+//     with all past it 935 -> 980). The tallest tiles of more choices than one holds for each expert are
+//     bound by the matrix cores, and there the question itself costs 1 to 2 %: a kernel without it.
 //   * The row tiles of an expert want the same weights: the list of workgroups (8 row tiles x
 //     all column tiles, rows fastest) is cut into 8 contiguous parts, one for each XCD, so that
 //     they meet in one L2. The list covers real tiles only; the grid is sized for the worst
@@ -88,6 +93,23 @@ DEV_INLINE void mr_load_lds(const char* src, unsigned dst) {
                  :: "s"(at), "v"(src) : "memory", "m0");
 }
 
+// The same, past the caches where `once` (the same for the wave). The branch is hidden from the
+// compiler, which would double the tallest tiles' registers for it: 317 -> 362 us at 2048 tokens of 128
+// experts.
+DEV_INLINE void mr_load_lds_once(const char* src, unsigned dst, int once) {
+    const unsigned at = __builtin_amdgcn_readfirstlane(dst);
+    once = __builtin_amdgcn_readfirstlane(once);
+    asm volatile("s_mov_b32 m0, %0\n\t"
+                 "s_cmp_lg_u32 %2, 0\n\t"
+                 "s_cbranch_scc1 1f\n\t"
+                 "global_load_lds_dwordx4 %1, off\n\t"
+                 "s_branch 2f\n"
+                 "1:\n\t"
+                 "global_load_lds_dwordx4 %1, off nt\n"
+                 "2:"
+                 :: "s"(at), "v"(src), "s"(once) : "memory", "m0", "scc");
+}
+
 template <int N>
 DEV_INLINE void mr_vm_wait() {
     asm volatile("s_waitcnt vmcnt(%c0)" ::"i"(N) : "memory");
@@ -135,7 +157,7 @@ DEV_INLINE bool mr_shares(const int total, const int nk, const bool crowded) {
     return total <= MR_WGS / 2 || (!crowded && total * nk >= MR_WGS * 16);
 }
 
-template <typename T, bool F8, bool GLU, int MT>
+template <typename T, bool F8, bool GLU, int MT, bool ONCE>
 __global__ void __launch_bounds__(512, 2)
 moe_routed_kernel(void* __restrict__ y, const T* __restrict__ x, const char* __restrict__ w0,
                   const char* __restrict__ w1, const float* __restrict__ s0,
@@ -191,11 +213,17 @@ moe_routed_kernel(void* __restrict__ y, const T* __restrict__ x, const char* __r
     int s_li = li0, s_k = k0, s_left = left;
     const char* xsrc[XW];
     const char* wsrc[WP];
+    int once = 0;                                     // no other row tile has these weights
     auto sources = [&]() {
         int rt, n0;
         place(s_li, rt, n0);
         const int e = tiles[1 + 2 * rt], rows = tiles[2 + 2 * rt];
         const int m0 = rt * MT;
+        if constexpr (ONCE) {                         // (without branches, as in mr_load_lds_once)
+            const int before = max(rt - 1, 0), after = min(rt + 1, nreal - 1);
+            once = !((int)(before != rt) & (int)(tiles[1 + 2 * before] == e) |
+                     (int)(after != rt) & (int)(tiles[1 + 2 * after] == e));
+        }
         // Whole tiles start at different steps and wrap round: in step they would all ask for the
         // same 128 bytes of rows a power of two apart, which few of the memory channels hold
         // (8 experts in 16 bits, 32 rows each: 516 -> 501 us; 2048 tokens of 128: 0.87 -> 0.85 of
@@ -232,7 +260,10 @@ moe_routed_kernel(void* __restrict__ y, const T* __restrict__ x, const char* __r
         for (int i = 0; i < XP / 8; ++i) mr_load_lds(xsrc[i] + s_k * (C::BK * 2), xd + i * 8192);
         if (XP % 8 && more) mr_load_lds(xsrc[XW - 1] + s_k * (C::BK * 2), xd + (XW - 1) * 8192);
 #pragma unroll
-        for (int i = 0; i < WP; ++i) mr_load_lds(wsrc[i] + s_k * 128, wd + i * 1024);
+        for (int i = 0; i < WP; ++i) {
+            if constexpr (ONCE) mr_load_lds_once(wsrc[i] + s_k * 128, wd + i * 1024, once);
+            else mr_load_lds(wsrc[i] + s_k * 128, wd + i * 1024);
+        }
         --s_left;
         if (++s_k == nk) {
             s_k = 0;
@@ -547,21 +578,21 @@ moe_route_kernel(int* __restrict__ tiles, int* __restrict__ gather, int* __restr
     }
 }
 
-template <typename T, bool F8, bool GLU, int MT>
+template <typename T, bool F8, bool GLU, int MT, bool ONCE = true>
 void mr_launch(void* y, const torch::Tensor& x, const torch::Tensor& w0, const torch::Tensor& w1,
                const float* s0, const float* s1, const torch::Tensor& tiles, const int* gather,
                int max_tiles, int col0, int ncols, int gelu, int share, hipStream_t st) {
     using C = MrTile<F8, MT>;
     constexpr int LDS = C::D * C::STEP, BNO = GLU ? C::BN / 2 : C::BN;
     // a limit of the function, the same in every call
-    (void)hipFuncSetAttribute((const void*)moe_routed_kernel<T, F8, GLU, MT>,
+    (void)hipFuncSetAttribute((const void*)moe_routed_kernel<T, F8, GLU, MT, ONCE>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     const int ntn = (ncols + BNO - 1) / BNO;
     TORCH_CHECK((long)max_tiles * ntn < (1L << 30), "moe_routed: too many tiles");
     // a workgroup a tile; shares need all MR_WGS, whatever the table turns out to hold
     const long grid = std::max(share ? (long)MR_WGS : 0, ((long)max_tiles * ntn + 7) / 8 * 8);
-    hipLaunchKernelGGL((moe_routed_kernel<T, F8, GLU, MT>), dim3((unsigned)grid), dim3(512), LDS, st, y,
-                       (const T*)x.data_ptr(), (const char*)w0.data_ptr(),
+    hipLaunchKernelGGL((moe_routed_kernel<T, F8, GLU, MT, ONCE>), dim3((unsigned)grid), dim3(512),
+                       LDS, st, y, (const T*)x.data_ptr(), (const char*)w0.data_ptr(),
                        (const char*)w1.data_ptr(), s0, s1, tiles.data_ptr<int>(), gather,
                        (int)w0.size(1), (int)w0.size(2), col0, ncols, ntn, gelu, share);
     HIP_CHECK_KERNEL();
@@ -575,13 +606,16 @@ void mr_dispatch(void* y, const torch::Tensor& x, const torch::Tensor& w0,
     const int max_tiles = (int)((tiles.numel() - 1) / 2);
     auto st = at::hip::getCurrentHIPStream();
     const bool f8 = s0 != nullptr, bf = x.scalar_type() == at::ScalarType::BFloat16;
-#define MR(TT, FF, MM) mr_launch<TT, FF, GLU, MM>(y, x, w0, w1, s0, s1, tiles, gather, max_tiles, \
-                                                  col0, ncols, gelu, share, st)
+    // more choices than a tile holds for each expert: hardly one has its weights to itself
+    const bool many = max_tiles > 2 * w0.size(0);
+#define MR(TT, FF, ...) mr_launch<TT, FF, GLU, __VA_ARGS__>(y, x, w0, w1, s0, s1, tiles, gather,  \
+                                                            max_tiles, col0, ncols, gelu, share, st)
 #define MR_M(TT)                                                                                  \
     do {                                                                                          \
         if (f8 && mt == 64) MR(TT, true, 64);                                                     \
         else if (f8 && mt == 48) MR(TT, true, 48);                                                \
         else if (f8) MR(TT, true, 32);                                                            \
+        else if (mt == 160 && many) MR(TT, false, 160, false);                                    \
         else if (mt == 160) MR(TT, false, 160);                                                   \
         else if (mt == 128) MR(TT, false, 128);                                                   \
         else if (mt == 96) MR(TT, false, 96);                                                     \
