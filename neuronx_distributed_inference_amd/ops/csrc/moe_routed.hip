@@ -13,6 +13,11 @@
 //     round of workgroups, so the height goes by the rows an expert has by chance and not only on
 //     average: 2048 tokens x 8 of 128 experts (128 rows +- 11) take 128 tiles of 160 rows, and
 //     would take 190 of 128.
+//   * The last round of workgroups, where it would fill half of the chip or less, takes its tiles in
+//     halves of 128 columns, in rings of their own: a token of 8 of 128 experts (48 tiles)
+//     42 -> 31 us with its table and sum, 128 tokens of 8 experts in 16 bits (3 1/2 rounds) 467 ->
+//     453, 512 in 8 bits 630 -> 592. More than half of the chip's tiles stay whole: their halves would be
+//     a round more.
 //   * An expert's weights that no other row tile wants come past the caches: at 2048 tokens of 128
 //     experts 347 -> 317 us, 64 tokens 221 -> 198; 128 tokens of 8 experts in 16 bits 515 -> 467, in
 //     8 bits 281 -> 264. Where another wants them they are shared in the L2 (1024 tokens of 8 experts
@@ -37,14 +42,14 @@
 //     products (a workgroup a CU) gained nothing where there are many: 360 and 353 us at 2048
 //     tokens of 128 experts, 3206 and 3307 for 4096 tokens of 8.
 //
-// The layer's products with their table and sum in us, before (tiles of 32, 64 and 128 rows, a
-// ring of three, no shares, all tiles in step) -> now:
-//   128 experts of 2048 x 768, 8 a token:  64 tokens 228 -> 228, 512 255 -> 257, 1024 300 -> 290,
-//     2048 410 -> 357, 3000 487 -> 487, 4096 610 -> 562
-//   8 experts of 4096 x 14336, 2 a token:  16 tokens 558 -> 500, 128 586 -> 496, 256 630 -> 517,
-//     1024 1115 -> 951, 4096 3186 -> 3149;  in 8 bits 16 tokens 305 -> 270, 128 320 -> 289,
-//     200 349 -> 312, 256 400 -> 400
-// Row tiles there (rows an expert on average: times of tiles of 32, 64, 96, 128, 160 rows):
+// The layer's products with their table and sum in us, tiles of 32, 64 and 128 rows in a ring of
+// three, all in step and through the caches -> now:
+//   128 experts of 2048 x 768, 8 a token:  64 tokens 228 -> 199, 1024 300 -> 255, 2048 410 -> 313,
+//     3000 487 -> 459, 4096 610 -> 521
+//   8 experts of 4096 x 14336, 2 a token:  16 tokens 558 -> 434, 128 586 -> 453, 256 630 -> 475,
+//     1024 1115 -> 917, 2048 1700;  in 8 bits 16 tokens 305 -> 226, 128 320 -> 262, 200 349 -> 279,
+//     256 400 -> 378
+// Row tiles there, before the last two of these (rows an expert on average: times of tiles of 32, 64, 96, 128, 160 rows):
 //   128 experts  32: 283 257 261 264 270;  64: 376 318 290 295 296;  128: 578 445 414 405 357;
 //     188: 751 563 512 487 551;  256: 1015 730 647 601 562
 //   8 experts in 8 bits (32, 48, 64 rows)  4: 270 275 275;  32: 332 289 295;  40: 369 294 304;
@@ -123,14 +128,15 @@ DEV_INLINE float mr_act(float g, int gelu) {
     return g / (1.f + __expf(-g));
 }
 
-template <bool F8, int MT>
+// HALF: a tile of half the columns
+template <bool F8, int MT, bool HALF>
 struct MrTile {
-    static constexpr int BN = 256;
+    static constexpr int BN = HALF ? 128 : 256;
     static constexpr int BK = F8 ? 128 : 64;          // 128 B of a weight row
     static constexpr int XH = BK / 64;                // 128 B images of x a step
-    static constexpr int WM = MT >= 96 ? 2 : 1;       // waves along the rows
+    static constexpr int WM = HALF || MT >= 96 ? 2 : 1;       // waves along the rows
     static constexpr int WN = 8 / WM;
-    static constexpr int MI = MT / WM / 16;
+    static constexpr int MI = (MT / 16 + WM - 1) / WM;
     static constexpr int NI = BN / WN / 16;
     static constexpr int XB = XH * MT * 128;
     static constexpr int STEP = XB + BN * 128;        // bytes of a ring buffer
@@ -157,42 +163,39 @@ DEV_INLINE bool mr_shares(const int total, const int nk, const bool crowded) {
     return total <= MR_WGS / 2 || (!crowded && total * nk >= MR_WGS * 16);
 }
 
-template <typename T, bool F8, bool GLU, int MT, bool ONCE>
-__global__ void __launch_bounds__(512, 2)
-moe_routed_kernel(void* __restrict__ y, const T* __restrict__ x, const char* __restrict__ w0,
-                  const char* __restrict__ w1, const float* __restrict__ s0,
-                  const float* __restrict__ s1, const int* __restrict__ tiles_,
-                  const int* __restrict__ gather_, const int N, const int K, const int col0,
-                  const int ncols, const int ntn, const int gelu, const int can_share) {
+struct MrArgs {
+    void* y;
+    const void* x;
+    const char *w0, *w1;
+    const float *s0, *s1;
+    const int *tiles, *gather;
+    int N, K, col0, ncols, ntn, gelu;
+};
+
+// A tile of the list (of its columns, the half `side`), or with `share` workgroup wg's `left` steps
+// from step k0 of tile li0 on.
+template <typename T, bool F8, bool GLU, int MT, bool ONCE, bool HALF>
+DEV_INLINE void mr_work(const MrArgs& a_, const int nreal, const bool share, const int wg, const int li0,
+                        const int k0, int left, const int side) {
     using MF = MrMfma<T>;
     using vec8 = typename MF::vec8;
-    using C = MrTile<F8, MT>;
+    using C = MrTile<F8, MT, HALF>;
     constexpr int MI = C::MI, NI = C::NI, XH = C::XH, D = C::D;
-    constexpr int BNO = GLU ? C::BN / 2 : C::BN;      // output columns of a workgroup
+    constexpr int BNO = (GLU ? 128 : 256);            // output columns of a tile
     constexpr int WP = C::BN / 64;                    // 1 KB pieces of W a wave stages
     constexpr int XP = XH * MT / 8;                   // pieces of x in all: a wave takes every 8th
     constexpr int XW = (XP + 7) / 8;
     constexpr int ES = F8 ? 1 : 2;
     extern __shared__ __attribute__((aligned(16))) char smem[];
-
-    mr_table tiles = (mr_table)(size_t)tiles_, gather = (mr_table)(size_t)gather_;
-    const int head = tiles[0], nreal = head & (MR_CROWDED - 1);
-    const int total = nreal * ntn, nk = K / C::BK;
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    // the workgroup's part of the list: a tile, or `left` steps from step k0 of tile li0 on
-    const bool share = !GLU && can_share && mr_shares(total, nk, head & MR_CROWDED);
-    const int per = (total + 7) >> 3, wg = xcd * (MR_WGS / 8) + slot;
-    int li0 = xcd * per + slot, k0 = 0, left = nk;
-    const int end = share ? total : min(total, (xcd + 1) * per);
-    if (share) {
-        if (slot >= MR_WGS / 8) return;
-        const long all = (long)total * nk;
-        const int from = (int)(wg * all / MR_WGS);
-        left = (int)((wg + 1) * all / MR_WGS) - from;
-        li0 = from / nk;
-        k0 = from - li0 * nk;
-    }
-    if (li0 >= end || left == 0) return;              // uniform over the workgroup
+    void* __restrict__ const y = a_.y;
+    const T* __restrict__ const x = (const T*)a_.x;
+    const char* __restrict__ const w0 = a_.w0;
+    const char* __restrict__ const w1 = a_.w1;
+    const float* __restrict__ const s0 = a_.s0;
+    const float* __restrict__ const s1 = a_.s1;
+    const int N = a_.N, K = a_.K, col0 = a_.col0, ncols = a_.ncols, ntn = a_.ntn, gelu = a_.gelu;
+    mr_table tiles = (mr_table)(size_t)a_.tiles, gather = (mr_table)(size_t)a_.gather;
+    const int nk = K / C::BK;
 
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -206,7 +209,7 @@ moe_routed_kernel(void* __restrict__ y, const T* __restrict__ x, const char* __r
         const int grp = li / (MR_GRP * ntn), rows_grp = min(MR_GRP, nreal - grp * MR_GRP);
         const int in = li - grp * MR_GRP * ntn;
         rt = grp * MR_GRP + in % rows_grp;
-        n0 = (in / rows_grp) * BNO;
+        n0 = (in / rows_grp) * BNO + (HALF ? side * (BNO / 2) : 0);
     };
 
     // ---- loads: a cursor that runs ahead of the products, into the next tile too ----
@@ -372,9 +375,9 @@ moe_routed_kernel(void* __restrict__ y, const T* __restrict__ x, const char* __r
                 cur = cur == (D - 1) * C::STEP ? 0 : cur + C::STEP;
             }
         };
-        constexpr int HALF = (MI + 1) / 2;
-        if (rows > (HALF * C::WM + wm) * 16) run(std::integral_constant<int, MI>{});
-        else run(std::integral_constant<int, HALF>{});
+        constexpr int FEW = (MI + 1) / 2;
+        if (rows > (FEW * C::WM + wm) * 16) run(std::integral_constant<int, MI>{});
+        else run(std::integral_constant<int, FEW>{});
         left -= steps;
 
         // ---- the tile, or this workgroup's share of it, is done ----
@@ -419,6 +422,34 @@ moe_routed_kernel(void* __restrict__ y, const T* __restrict__ x, const char* __r
         k = 0;
         ++li;
         enter();
+    }
+}
+
+template <typename T, bool F8, bool GLU, int MT, bool ONCE>
+__global__ void __launch_bounds__(512, 2)
+moe_routed_kernel(const MrArgs a, const int can_share) {
+    const int head = ((mr_table)(size_t)a.tiles)[0], nreal = head & (MR_CROWDED - 1);
+    const int total = nreal * a.ntn, nk = a.K / MrTile<F8, MT, false>::BK;
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    // the workgroup's part of the list; every exit is uniform over the workgroup
+    if (!GLU && can_share && mr_shares(total, nk, head & MR_CROWDED)) {
+        if (slot >= MR_WGS / 8) return;
+        const int wg = xcd * (MR_WGS / 8) + slot;
+        const long all = (long)total * nk;
+        const int from = (int)(wg * all / MR_WGS), left = (int)((wg + 1) * all / MR_WGS) - from;
+        if (left)
+            mr_work<T, F8, GLU, MT, ONCE, false>(a, nreal, true, wg, from / nk, from % nk, left, 0);
+        return;
+    }
+    const int rest = total % MR_WGS, halved = rest <= MR_WGS / 2 ? rest : 0, whole = total - halved;
+    const int per = (whole + 7) >> 3, per_half = (2 * halved + 7) >> 3;
+    if (slot < per) {
+        const int li = xcd * per + slot;
+        if (li < whole) mr_work<T, F8, GLU, MT, ONCE, false>(a, nreal, false, 0, li, 0, nk, 0);
+    } else if (slot < per + per_half) {
+        const int h = xcd * per_half + slot - per;
+        if (h < 2 * halved)
+            mr_work<T, F8, GLU, MT, ONCE, true>(a, nreal, false, 0, whole + (h >> 1), 0, nk, h & 1);
     }
 }
 
@@ -582,19 +613,23 @@ template <typename T, bool F8, bool GLU, int MT, bool ONCE = true>
 void mr_launch(void* y, const torch::Tensor& x, const torch::Tensor& w0, const torch::Tensor& w1,
                const float* s0, const float* s1, const torch::Tensor& tiles, const int* gather,
                int max_tiles, int col0, int ncols, int gelu, int share, hipStream_t st) {
-    using C = MrTile<F8, MT>;
-    constexpr int LDS = C::D * C::STEP, BNO = GLU ? C::BN / 2 : C::BN;
+    using C = MrTile<F8, MT, false>;
+    using H = MrTile<F8, MT, true>;
+    constexpr int LDS = std::max(C::D * C::STEP, H::D * H::STEP), BNO = GLU ? C::BN / 2 : C::BN;
     // a limit of the function, the same in every call
     (void)hipFuncSetAttribute((const void*)moe_routed_kernel<T, F8, GLU, MT, ONCE>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     const int ntn = (ncols + BNO - 1) / BNO;
     TORCH_CHECK((long)max_tiles * ntn < (1L << 30), "moe_routed: too many tiles");
-    // a workgroup a tile; shares need all MR_WGS, whatever the table turns out to hold
-    const long grid = std::max(share ? (long)MR_WGS : 0, ((long)max_tiles * ntn + 7) / 8 * 8);
+    // a workgroup a tile, up to half of MR_WGS more for those in halves, and what rounding eighths up
+    // takes; shares need all MR_WGS, whatever the table turns out to hold
+    const long units = (long)max_tiles * ntn + std::min((long)max_tiles * ntn, MR_WGS / 2L) + 14;
+    const long grid = std::max(share ? (long)MR_WGS : 0, (units + 7) / 8 * 8);
+    const MrArgs a{y, x.data_ptr(), (const char*)w0.data_ptr(), (const char*)w1.data_ptr(), s0, s1,
+                   tiles.data_ptr<int>(), gather, (int)w0.size(1), (int)w0.size(2), col0, ncols, ntn,
+                   gelu};
     hipLaunchKernelGGL((moe_routed_kernel<T, F8, GLU, MT, ONCE>), dim3((unsigned)grid), dim3(512),
-                       LDS, st, y, (const T*)x.data_ptr(), (const char*)w0.data_ptr(),
-                       (const char*)w1.data_ptr(), s0, s1, tiles.data_ptr<int>(), gather,
-                       (int)w0.size(1), (int)w0.size(2), col0, ncols, ntn, gelu, share);
+                       LDS, st, a, share);
     HIP_CHECK_KERNEL();
 }
 

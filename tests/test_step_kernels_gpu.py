@@ -232,6 +232,20 @@ def test_moe_routed_tile_heights_and_shares(mt, f8, T, E, k, H, I, dtype, monkey
         assert torch.equal(got, ops.moe_routed_experts(x, wt, idx, *w, scales=scales, num_experts=E))
 
 
+@pytest.mark.parametrize("mt,f8,T,H,I", [
+    # 8 row tiles, two an expert, times 32 (whole tiles only), 33, 48 and 49 (too many for halves) tiles
+    # of columns, the last one's second half without any where I is 64 past a tile
+    (32, False, 33, 128, 4096), (32, False, 63, 128, 4160), (64, False, 65, 64, 6144),
+    (64, False, 127, 64, 6208), (48, True, 49, 128, 4224), (32, True, 64, 256, 6272),
+    # 4 row tiles: weights that one tile has to itself; 12 of the tallest
+    (128, False, 100, 64, 8256), (96, False, 81, 64, 12288), (160, False, 330, 64, 2816),
+    # the down projection's tiles in halves too
+    (32, False, 20, 16448, 64), (48, True, 33, 16640, 128), (160, False, 150, 16512, 64)])
+def test_moe_routed_last_round(mt, f8, T, H, I, monkeypatch):
+    """All of 4 experts for each token: lists of tiles that end in whole tiles and in halves."""
+    test_moe_routed_tile_heights_and_shares(mt, f8, T, 4, 4, H, I, torch.bfloat16, monkeypatch)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,S,H,D,seq", [(1, 1, 8, 4, None), (3, 5, 2048, 64, torch.int64), (64, 1, 4096, 128, torch.int32),
                                          (1, 600, 8192, 128, torch.int64), (2, 2, 32768, 256, None)])
