@@ -247,10 +247,11 @@ class NabelixLayer(nn.Module):
         h = self.canon(hn, kv_mgr.state.get(f"run{run_idx}.canon"), step,
                        out_dtype=self.out_dtype)
         left, right = self.mixer(h, kv_mgr, run_idx, step)
-        seqmix.residual_add(x, left, self.mixer.left_scale, right, self.mixer.right_scale)
-        if self.mlp is not None:
-            n = seqmix.layer_norm(x, self.norm2.weight, self.norm2.eps, self.out_dtype)
-            seqmix.residual_add(x, self.mlp(n))
+        scaled = left, self.mixer.left_scale, right, self.mixer.right_scale
+        if self.mlp is None:
+            return seqmix.residual_add(x, *scaled)
+        n = seqmix.residual_layer_norm(x, *scaled, self.norm2.weight, self.norm2.eps, self.out_dtype)
+        seqmix.residual_add(x, self.mlp(n))
         return x
 
     def steps_once(self, rows: int) -> bool:

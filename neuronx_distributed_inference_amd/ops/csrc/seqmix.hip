@@ -66,6 +66,21 @@ template <> DEV void load8<float>(const float* p, float* v) {
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
     v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
 }
+template <typename T> DEV void store8(T* p, const float* v);
+template <> DEV void store8<float>(float* p, const float* v) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+}
+typedef float two_f32 __attribute__((ext_vector_type(2)));
+typedef __bf16 two_bf16 __attribute__((ext_vector_type(2)));
+template <> DEV void store8<bf16>(bf16* p, const float* v) {
+    uint32_t pk[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)                           // v_cvt_pk_bf16_f32: a NaN stays one
+        pk[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(
+            (two_f32){v[2 * e], v[2 * e + 1]}, two_bf16));
+    *reinterpret_cast<uint4*>(p) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+}
 
 
 // ---------------------------------------------------------------- LayerNorm
@@ -298,12 +313,13 @@ __global__ void short_conv_step_kernel(const TIn* __restrict__ x, long xs,
     stf<TOut>(y + idx, acc);
 }
 
+DEV uint16_t f2bf_rne(float f);
+
 // What stands between two products of a decoder layer whose residual stream is fp32, a row of
 // single tokens a workgroup: x += sa * a + sb * b (each the sum of the parts of K of a product, in
 // fp32), LayerNorm, and with TAPS the short convolution over time that is added to the norm, with its
 // new tail; out in bf16. Bound by launches: 48 rows of 2048 took 21 us in four (sum of parts,
 // residual, norm, convolution), 6 here.
-DEV uint16_t f2bf_rne(float f);
 struct StreamArgs {
     float* x;                    // (rows, C)
     const float* a;              // (na, rows, C)
@@ -2745,8 +2761,42 @@ delta_chunk_scan_kernel(const float* __restrict__ ws, float* __restrict__ state,
     for (int i = 0; i < NB; ++i) *reinterpret_cast<dc_f32x4*>(st + i * 16) = s[i];
 }
 
-// per-head RMS norm over the value channels, shared weight, sigmoid gate:
-// one wave per (token, head); pad tokens produce zeros
+// per-head RMS norm over the value channels, shared weight, sigmoid gate: pad tokens produce zeros.
+// LPR lanes a (token, head), 8 channels each: bound by memory, 4031 tokens of 16 heads of 128
+// 35.6 -> 16.3 us. Other widths: a wave a row below
+template <typename T, int LPR>
+__global__ void gated_rmsnorm_vec_kernel(const float* __restrict__ o, const T* __restrict__ gate,
+                                         long gstride, const float* __restrict__ w, float eps,
+                                         const int* __restrict__ pos, const int* __restrict__ seq,
+                                         T* __restrict__ out, long ntok, int S, int H,
+                                         int gate_silu) {
+    constexpr int Dv = LPR * 8;
+    const long id = (long)blockIdx.x * blockDim.x + threadIdx.x, row = id / LPR;
+    const int c = (int)(id % LPR) * 8;
+    if (row >= ntok * H) return;                         // all of a row's lanes
+    const long tok = row / H;
+    const int h = (int)(row % H);
+    T* op = out + row * Dv + c;
+    float v[8] = {};
+    if (pos[tok] < 0 || seq[tok / S] < 0) {
+        store8<T>(op, v);
+        return;
+    }
+    float g[8], wv[8], ss = 0.f;
+    load8<float>(o + row * Dv + c, v);
+    load8<T>(gate + tok * gstride + (long)h * Dv + c, g);
+    load8<float>(w + c, wv);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+#pragma unroll
+    for (int m = LPR / 2; m > 0; m >>= 1) ss += __shfl_xor(ss, m, LPR);
+    const float inv = 1.f / sqrtf(ss / Dv + eps);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        v[e] = v[e] * inv * wv[e] * (gate_silu ? g[e] * sigmoidf_(g[e]) : sigmoidf_(g[e]));
+    store8<T>(op, v);
+}
+
 template <typename T>
 __global__ void gated_rmsnorm_kernel(const float* __restrict__ o, const T* __restrict__ gate,
                                      long gstride, const float* __restrict__ w, float eps,
@@ -2941,15 +2991,32 @@ __global__ void softcap_kernel(const T* __restrict__ in, float* __restrict__ out
         out[i] = cap * tanhf(ldf<T>(in + i) / cap);
 }
 
-// x += sa*a (+ sb*b), fp32 residual stream
-template <typename T>
+// x += sa*a (+ sb*b), fp32 residual stream; VEC: 8 elements a thread (4031 rows of 2048, one summand
+// in 16 bits, 16.6 -> 16.0 us, 5.2 TB/s)
+template <typename T, bool VEC>
 __global__ void residual_add_kernel(float* __restrict__ x, const T* __restrict__ a, float sa,
                                     const T* __restrict__ b, float sb, long n) {
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (long)gridDim.x * blockDim.x) {
-        float v = x[i] + sa * ldf<T>(a + i);
-        if (b) v += sb * ldf<T>(b + i);
-        x[i] = v;
+    const long step = (long)gridDim.x * blockDim.x, first = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if constexpr (VEC) {
+        for (long i = first * 8; i < n; i += step * 8) {
+            float v[8], y[8];
+            load8<float>(x + i, v);
+            load8<T>(a + i, y);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] += sa * y[e];
+            if (b) {
+                load8<T>(b + i, y);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] += sb * y[e];
+            }
+            store8<float>(x + i, v);
+        }
+    } else {
+        for (long i = first; i < n; i += step) {
+            float v = x[i] + sa * ldf<T>(a + i);
+            if (b) v += sb * ldf<T>(b + i);
+            x[i] = v;
+        }
     }
 }
 
@@ -3006,19 +3073,6 @@ __global__ void gelu_mul_vec_kernel(const T* __restrict__ gu, T* __restrict__ ou
 // variants move 8 channels per thread with 16-byte accesses (widths that are
 // multiples of 8 on 16-byte aligned rows); the second pass re-reads the row
 // from cache, so any width works.
-template <typename T> DEV void store8(T* p, const float* v);
-template <> DEV void store8<float>(float* p, const float* v) {
-    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-    *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
-}
-template <> DEV void store8<bf16>(bf16* p, const float* v) {
-    uint32_t pk[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-        pk[e] = (uint32_t)f2bf_rne(v[2 * e]) | ((uint32_t)f2bf_rne(v[2 * e + 1]) << 16);
-    *reinterpret_cast<uint4*>(p) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-}
-
 // 4 consecutive elements as floats, one 8- or 16-byte access
 template <typename T> DEV void load4(const T* p, float* v);
 template <> DEV void load4<bf16>(const bf16* p, float* v) {
@@ -3257,6 +3311,62 @@ add_layer_norm_kernel(float* __restrict__ stream, const TY* __restrict__ y, floa
         const float v = (xr[c] - mean) * inv * w[c] + bias[c];
         xr[c] = v;
         if (copy) stf<TC>(copy + row * C + c, v);
+    }
+}
+
+// ----------------------------------------- LayerNorm with the residual step before it
+// x[row] += sa * a[row] (+ sb * b[row]) where there is an a; out = layer_norm(x[row]) * w (+ bias).
+// Bound by memory: a row stays in registers from the sum on, so each operand is read and each
+// result written once, in 16-byte pieces. 4031 rows of 2048, us: norm of the fp32 stream to 16 and
+// 32 bits 17.4 and 19.0 -> 10.7 and 14.5 (layer_norm_kernel, which takes any width and alignment), two
+// summands in 16 bits and norm 24.4 + 16.8 -> 21.5 (5.4 TB/s).
+template <typename T, typename TOut, int NV, bool ADD>
+__global__ void __launch_bounds__(LN_THREADS)
+layer_norm_vec_kernel(float* __restrict__ x, const T* __restrict__ a, float sa,
+                      const T* __restrict__ b, float sb, const float* __restrict__ w,
+                      const float* __restrict__ bias, TOut* __restrict__ out, int C, float eps) {
+    __shared__ float red[LN_THREADS / WAVE];
+    const long row = blockIdx.x;
+    float* xr = x + row * C;
+    float v[NV][8], s = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = (j * LN_THREADS + threadIdx.x) * 8;
+        if (c >= C) continue;
+        load8<float>(xr + c, v[j]);
+        if constexpr (ADD) {
+            float y[8];
+            load8<T>(a + row * C + c, y);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[j][e] += sa * y[e];
+            if (b) {
+                load8<T>(b + row * C + c, y);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[j][e] += sb * y[e];
+            }
+            store8<float>(xr + c, v[j]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += v[j][e];
+    }
+    const float mean = block_sum(s, red) / C;
+    float q = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+        if ((j * LN_THREADS + threadIdx.x) * 8 < C)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { v[j][e] -= mean; q += v[j][e] * v[j][e]; }
+    const float inv = 1.f / sqrtf(block_sum(q, red) / C + eps);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = (j * LN_THREADS + threadIdx.x) * 8;
+        if (c >= C) continue;
+        float wv[8], bv[8] = {};
+        load8<float>(w + c, wv);
+        if (bias) load8<float>(bias + c, bv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[j][e] = v[j][e] * inv * wv[e] + bv[e];
+        store8<TOut>(out + row * C + c, v[j]);
     }
 }
 
@@ -5609,13 +5719,44 @@ static inline int grid_for(long total, int block, int cap = 8192) {
 
 extern "C" {
 
-int nx_layer_norm(const float* x, const float* w, const float* bias, void* out, int out_bf16,
-                  long rows, int C, float eps, hipStream_t st) {
+int nx_residual_add(float* x, const void* a, float sa, const void* b, float sb, int is_bf16,
+                    long n, hipStream_t st);
+
+// x += sa * a (+ sb * b) where there is an a, of 16 bits or of 32; out = layer_norm(x) * w (+ bias)
+int nx_layer_norm(float* x, const void* a, float sa, const void* b, float sb, int a_bf16,
+                  const float* w, const float* bias, void* out, int out_bf16, long rows, int C,
+                  float eps, hipStream_t st) {
     if (rows <= 0) return 0;
+    if (C <= 0) return -1;
     dim3 grid((unsigned)rows), block(LN_THREADS);
-    if (out_bf16)
-        layer_norm_kernel<bf16><<<grid, block, 0, st>>>(x, w, bias, (bf16*)out, rows, C, eps);
-    else layer_norm_kernel<float><<<grid, block, 0, st>>>(x, w, bias, (float*)out, rows, C, eps);
+    const bool vec = C % 8 == 0 && C <= LN_THREADS * 8 * 4 &&
+                     (((uintptr_t)x | (uintptr_t)a | (uintptr_t)b | (uintptr_t)w | (uintptr_t)bias |
+                       (uintptr_t)out) % 16) == 0;
+    if (!vec) {
+        if (a) {
+            const int rc = nx_residual_add(x, a, sa, b, sb, a_bf16, rows * C, st);
+            if (rc) return rc;
+        }
+        if (out_bf16)
+            layer_norm_kernel<bf16><<<grid, block, 0, st>>>(x, w, bias, (bf16*)out, rows, C, eps);
+        else layer_norm_kernel<float><<<grid, block, 0, st>>>(x, w, bias, (float*)out, rows, C, eps);
+        return (int)hipGetLastError();
+    }
+#define LN(T, TO, NV, ADD) layer_norm_vec_kernel<T, TO, NV, ADD><<<grid, block, 0, st>>>( \
+            x, (const T*)a, sa, (const T*)b, sb, w, bias, (TO*)out, C, eps)
+#define LNV(T, TO, ADD) do { \
+        if (C <= LN_THREADS * 8) LN(T, TO, 1, ADD); \
+        else if (C <= LN_THREADS * 16) LN(T, TO, 2, ADD); \
+        else LN(T, TO, 4, ADD); } while (0)
+#define LNA(TO) do { \
+        if (!a) LNV(float, TO, false); \
+        else if (a_bf16) LNV(bf16, TO, true); \
+        else LNV(float, TO, true); } while (0)
+    if (out_bf16) LNA(bf16);
+    else LNA(float);
+#undef LNA
+#undef LNV
+#undef LN
     return (int)hipGetLastError();
 }
 
@@ -5991,6 +6132,24 @@ int nx_gated_delta(const float* qkv, long cstride, const void* beta, long bstrid
     }
     const long waves = ntok * H;
     dim3 g2((unsigned)((waves + 3) / 4)), b2(4 * WAVE);
+    const bool wide = gstride % 8 == 0 && (((uintptr_t)obuf | (uintptr_t)gate | (uintptr_t)norm_w |
+                                            (uintptr_t)out) % 16) == 0;
+#define GN(T, LPR) gated_rmsnorm_vec_kernel<T, LPR><<<dim3((unsigned)((waves * LPR + 255) / 256)),   \
+        dim3(256), 0, st>>>(obuf, (const T*)gate, gstride, norm_w, eps, pos, seq, (T*)out, ntok, S, H, \
+                            gate_silu)
+#define GNT(T)                                                                                     \
+    do {                                                                                           \
+        if (Dv == 64) GN(T, 8);                                                                    \
+        else if (Dv == 128) GN(T, 16);                                                             \
+        else GN(T, 32);                                                                            \
+        return (int)hipGetLastError();                                                             \
+    } while (0)
+    if (wide && (Dv == 64 || Dv == 128 || Dv == 256)) {
+        if (in_bf16) GNT(bf16);
+        else GNT(float);
+    }
+#undef GNT
+#undef GN
     if (in_bf16) gated_rmsnorm_kernel<bf16><<<g2, b2, 0, st>>>(
         obuf, (const bf16*)gate, gstride, norm_w, eps, pos, seq, (bf16*)out, ntok, S, H, Dv,
         gate_silu);
@@ -6056,11 +6215,15 @@ int nx_softcap(const void* in, int in_bf16, float* out, long n, float cap, hipSt
 int nx_residual_add(float* x, const void* a, float sa, const void* b, float sb, int is_bf16,
                     long n, hipStream_t st) {
     if (n <= 0) return 0;
-    dim3 grid(grid_for(n, 256)), block(256);
-    if (is_bf16) residual_add_kernel<bf16><<<grid, block, 0, st>>>(
-        x, (const bf16*)a, sa, (const bf16*)b, sb, n);
-    else residual_add_kernel<float><<<grid, block, 0, st>>>(
-        x, (const float*)a, sa, (const float*)b, sb, n);
+    const bool vec = n % 8 == 0 && (((uintptr_t)x | (uintptr_t)a | (uintptr_t)b) % 16) == 0;
+    dim3 grid(grid_for(vec ? n / 8 : n, 256)), block(256);
+#define RA(T, VEC) residual_add_kernel<T, VEC><<<grid, block, 0, st>>>( \
+            x, (const T*)a, sa, (const T*)b, sb, n)
+    if (is_bf16 && vec) RA(bf16, true);
+    else if (is_bf16) RA(bf16, false);
+    else if (vec) RA(float, true);
+    else RA(float, false);
+#undef RA
     return (int)hipGetLastError();
 }
 

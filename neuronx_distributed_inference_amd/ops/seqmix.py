@@ -198,12 +198,33 @@ def layer_norm(x, weight, eps: float, out_dtype: torch.dtype, bias=None):
         x = _f32(x)
         out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
         C = x.shape[-1]
-        _check(lib.nx_layer_norm(_p(x), _p(_f32(weight)),
+        _check(lib.nx_layer_norm(_p(x), None, ctypes.c_float(0), None, ctypes.c_float(0), 0,
+                                 _p(_f32(weight)),
                                  _p(None if bias is None else _f32(bias)), _p(out), _is_bf16(out),
                                  ctypes.c_long(x.numel() // C), C,
                                  ctypes.c_float(eps), _stream()), "layer_norm")
         return out
     return ref.layer_norm(x, weight, eps, out_dtype, bias)
+
+
+def residual_layer_norm(x, a, sa: float, b, sb: float, weight, eps: float,
+                        out_dtype: torch.dtype, bias=None):
+    """residual_add, then layer_norm of the stream, in one kernel."""
+    if x.is_cuda and a.dtype == (a if b is None else b).dtype and a.numel() == x.numel():
+        lib = _load()
+        assert x.dtype == torch.float32 and x.is_contiguous()
+        a = a.contiguous()
+        b = None if b is None else b.contiguous()
+        assert b is None or b.numel() == x.numel()
+        out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
+        C = x.shape[-1]
+        _check(lib.nx_layer_norm(_p(x), _p(a), ctypes.c_float(sa), _p(b), ctypes.c_float(sb),
+                                 _is_bf16(a), _p(_f32(weight)),
+                                 _p(None if bias is None else _f32(bias)), _p(out), _is_bf16(out),
+                                 ctypes.c_long(x.numel() // C), C,
+                                 ctypes.c_float(eps), _stream()), "residual_layer_norm")
+        return out
+    return layer_norm(residual_add(x, a, sa, b, sb), weight, eps, out_dtype, bias)
 
 
 def add_layer_norm(stream, y, alpha: float, weight, bias, eps: float, copy_dtype=None):

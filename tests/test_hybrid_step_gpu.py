@@ -249,3 +249,66 @@ def test_products_of_whole_results(M, N, K):
         limit = 1.13 * s1[:, : N // 2] * up.abs() + gate.abs() * s1[:, N // 2:] \
             + 2.0 ** -8 * want.abs() + 2.0 ** -21 * (gate * up).abs() + 1e-6
         assert ((d(y) - want).abs() <= limit).all()
+
+
+@pytest.mark.parametrize("out", [BF, torch.float32])
+@pytest.mark.parametrize("rows,C,summand", [(1, 8, None), (3, 2040, BF), (5, 2048, torch.float32),
+                                            (2, 2056, BF), (7, 4104, BF), (2, 8192, torch.float32),
+                                            (2, 8200, BF), (3, 37, BF)])
+def test_sum_and_norm(rows, C, summand, out):
+    """LayerNorm of a stream, alone and after its residual step: every count of pieces a thread
+    holds, widths and addresses that go without pieces, infinities and NaN as they were."""
+    g = torch.Generator(device="cuda").manual_seed(C)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    for offset in (0, 1):
+        x = rnd(rows * C + 1)[offset:offset + rows * C].view(rows, C)
+        w, bias = rnd(C), rnd(C)
+        a, b = (None, None) if summand is None else (rnd(rows, C).to(summand) for _ in range(2))
+        for second in (False, True) if summand else (False,):
+            want = x.to(F64)
+            got_x = x.clone() if not offset else torch.cat([x.new_zeros(1), x.flatten()])[1:].view(rows, C)
+            if summand:
+                want = want + 1.25 * a.to(F64) + (0.5 * b.to(F64) if second else 0)
+                got = seqmix.residual_layer_norm(got_x, a, 1.25, b if second else None, 0.5, w, 1e-5,
+                                                 out, bias)
+                alone = seqmix.residual_add(x.clone(), a, 1.25, b if second else None, 0.5)
+                assert (got_x - want).abs().max() <= 4 * 2.0 ** -24 * want.abs().max() + 1e-7
+                assert (alone - want).abs().max() <= 4 * 2.0 ** -24 * want.abs().max() + 1e-7
+            else:
+                got = seqmix.layer_norm(got_x, w, 1e-5, out, bias)
+                assert torch.equal(got_x, x)
+            want = torch.nn.functional.layer_norm(want, (C,), w.to(F64), bias.to(F64), 1e-5)
+            # rounding of the result, and 32-bit statistics of at most C / 256 terms in a chain
+            tol = (2.0 ** -8 if out is BF else 0) + 2.0 ** -18
+            assert ((got.to(F64) - want).abs() <= tol * (want.abs() + 1)).all()
+    x = rnd(2, 64)
+    x[0, 3], x[1, 5] = float("nan"), float("inf")
+    assert seqmix.layer_norm(x, rnd(64), 1e-5, out).isnan().all()
+
+
+@pytest.mark.parametrize("dtype", [BF, torch.float32])
+@pytest.mark.parametrize("Dv", [64, 96, 128, 256])
+def test_gated_norm_in_pieces(Dv, dtype):
+    """Heads in 16-byte pieces against the same from a weight that lies across them; padded rows
+    are zeros."""
+    B, S, H, D = 3, 5, 3, 64
+    g = torch.Generator(device="cuda").manual_seed(Dv)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    qkv = rnd(B, S, H * (2 * D + Dv))
+    beta, a, gate = (rnd(B, S, n).to(dtype) for n in (H, H, H * Dv))
+    weight = rnd(Dv + 1)
+    weight[:Dv] = weight[1:].clone()
+    pos = torch.arange(S, device="cuda").repeat(B, 1)
+    pos[1, 3:] = -1
+    step = seqmix.StepLayout(pos, torch.tensor([0, 1, -1], device="cuda"))
+    for act in ("sigmoid", "silu"):
+        res = []
+        for nw in (weight[:Dv].clone(), torch.cat([weight[:1], weight[:Dv]])[1:]):
+            state = torch.zeros(2, H, Dv, D, device="cuda")
+            res.append(seqmix.gated_delta_rule(qkv, beta, a, torch.zeros(H, device="cuda"),
+                                               torch.zeros(H, device="cuda"), gate, nw, 1e-5, state,
+                                               step, H, D, Dv, dtype, act))
+        assert res[1].abs().max() > 0.1 and not res[0][2].any() and not res[0][1, 3:].any()
+        # the same value but for the order of a head's squares: one rounding of the result
+        tol = 2.0 ** -8 if dtype is BF else 2.0 ** -20
+        assert ((res[0] - res[1]).abs() <= tol * res[1].abs()).all()
