@@ -430,8 +430,12 @@ def window_bias_attention(q, k_cache, v_cache, step: StepLayout, block_table,
 # of 16 heads of 128 the two are even (31 and 33 us for one row, 36 and 38 for 4, 78 and 77 for
 # 16); at 128 tokens the chunks take 57 us for the scan's 81 (4 rows) and 163 for 227 (16 rows).
 DELTA_CHUNK_MIN_TOKENS = 64
-# bytes of chunk operands kept between the two chunk kernels (they stay in the last-level cache)
-DELTA_CHUNK_WORKSPACE = 128 << 20
+# Bytes of chunk operands kept between the two chunk kernels, at most. More tokens go in spans, which
+# are not worth their ends even where a span's operands stay in the last-level cache: the chain
+# fills the chip badly, and starts and stops with each. With 128, 256, 512 MB, 1 and 2 GB, us: one row of
+# 4031 tokens of 16 heads of 128 369, 347, 347, 346, 347, of 60000 5100, 5058, 4953, 4952, 4957;
+# 13 of 1000 884, 822, 779, 779, 778; 64 of 200 of 32 heads 4350, 2618, 1898, 1650, 1651.
+DELTA_CHUNK_WORKSPACE = 1 << 30
 
 
 def gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps: float,
