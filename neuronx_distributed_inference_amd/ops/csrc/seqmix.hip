@@ -2829,7 +2829,10 @@ __global__ void gated_rmsnorm_kernel(const float* __restrict__ o, const T* __res
 // state of the head (D <= 128, Dv <= 128) on the way before they prepare q, k and the decays (each
 // 16 lanes for themselves, 8 key channels a lane, four value channels a wave at a time), so the
 // small chains of the preparation hide behind it; the norm over the value channels goes through
-// LDS. 48 rows of 16 heads of 128 x 128 (101 MB): 26 us; the three kernels above took 56.
+// LDS. 48 rows of 16 heads of 128 x 128 (101 MB): 26 us; the three kernels above took 56. The state
+// passes the caches by, which nothing reads before the next token and which others' weights want: 100
+// rows of 16 heads 51.4 -> 47.6, of 32 91.7 -> 83.3, 48 of 32 47 -> 43; in a model of four such
+// layers (48 rows) 493 -> 469 a step.
 // With TAPS the short convolution and silu of q, k and v come first, of the raw projections (in T)
 // and the carried tail, a channel a thread, where every head has a q and k of its own: q, k and v are
 // neither written nor read in 32 bits. The same 48 rows, 4 taps: 5.4 + 26.6 us apart, 30.0 so.
@@ -2878,7 +2881,8 @@ delta_step_kernel(const std::conditional_t<(TAPS > 0), T, float>* __restrict__ q
         const int r = min(row0 + 32 * i, Dv - 1);
 #pragma unroll
         for (int f = 0; f < F; ++f)
-            s[i][f] = *reinterpret_cast<const float4*>(st + (long)r * D + f * 64);
+            s[i][f] = __builtin_bit_cast(float4, __builtin_nontemporal_load(
+                reinterpret_cast<const dc_f32x4*>(st + (long)r * D + f * 64)));
         if constexpr (TAPS == 0) v[i] = qkv[(long)b * cstride + 2L * G * D + (long)h * Dv + r];
     }
     float4 q[F], k[F], dec[F];
@@ -2967,7 +2971,8 @@ delta_step_kernel(const std::conditional_t<(TAPS > 0), T, float>* __restrict__ q
             for (int f = 0; f < F; ++f) {
                 float4 x = s[i][f];
                 x.x += k[f].x * u; x.y += k[f].y * u; x.z += k[f].z * u; x.w += k[f].w * u;
-                *reinterpret_cast<float4*>(st + (long)r * D + f * 64) = x;
+                __builtin_nontemporal_store(__builtin_bit_cast(dc_f32x4, x),
+                    reinterpret_cast<dc_f32x4*>(st + (long)r * D + f * 64));
             }
             if (part == 0) os[r] = oq + u * qk;
         }
