@@ -297,7 +297,7 @@ __global__ __launch_bounds__(256) void tile_sum_kernel(T* __restrict__ y,
 // The tile of a shape. A chunk of w (BN rows of 128 bytes) is what a workgroup streams, x comes
 // again and again from the L2: few rows take small tiles with a deep ring, so that a CU has 64 KB
 // and more on the way; many rows take tall ones, for fewer reads of x and w from LDS a product.
-enum TgTile { T16, T16N, T32, T32N, T64, T64N, T128, T128N, T128W, T128B, T192, T256, T256W };
+enum TgTile { T16, T16N, T32, T32N, T64, T64N, T64W, T128, T128N, T128W, T128B, T192, T256, T256W };
 
 struct TgPlan {
     TgTile tile;
@@ -327,6 +327,9 @@ struct TgPlan {
 // (10240, 8192) 51.3 -> 50.0; more than 256 rows would fill a second tile in part only: 300 rows of
 // the first shape 33.9 with it, 28.4 without. Gate|up of few columns takes tiles of
 // 128 also where 256 would leave half of the CUs idle: 128 rows of the third shape 72.0 -> 50.5.
+// 33 to 64 rows of x are a third of what a tile of 128 columns takes in: tiles of 256 where these fill
+// the chip's rounds. 64 rows, 128 / 256 columns: (128256, 4096) 177 / 170 us, (57344, 8192) 148 / 138,
+// (65536, 2048) 46.1 / 43.5; in 2.3 rounds (151936, 2048) 116 / 120, in half of one (28672, 4096) 42 / 64.
 // `whole`: no kernel follows that would add up parts. Then up to 64 rows take tiles of half the width
 // where these fill most of the chip undivided, also where those of the full width in two parts are
 // a little faster by themselves: the sum is a launch of its own, some 3 us. 48 rows, undivided /
@@ -339,8 +342,11 @@ TgPlan tg_plan(long M, long N, long K, bool glu, bool whole) {
         return p;
     // half the width where that many more tiles spare parts of K, or with GLU fill the chip
     const bool narrow = glu ? N < 25600 : N <= 4096 || (whole && M <= 64 && N > 8192 && N <= 16384);
+    const long wides = (N + 255) / 256, rounds = (wides + 255) / 256;
+    const bool wide = wides >= 192 && wides * 100 >= rounds * 256 * 85;
     if (M <= 16) p = narrow ? TgPlan{T16N, 16, 64, 0} : TgPlan{T16, 16, 128, 0};
     else if (M <= 32) p = narrow ? TgPlan{T32N, 32, 64, 0} : TgPlan{T32, 32, 128, 0};
+    else if (M <= 64 && wide) p = {T64W, 64, 256, 0};
     else if (M <= 64) p = narrow ? TgPlan{T64N, 64, 64, 0} : TgPlan{T64, 64, 128, 0};
     else if (M <= 128 && narrow && glu) p = {T128N, 128, 64, 0};
     else if (M <= 128 && (glu ? N < 49152 : N * K < (60 << 20))) p = {T128, 128, 128, 0};
@@ -380,6 +386,7 @@ void tg_tile(TgArgs& a, TgTile tile, hipStream_t s) {
         case T32N: tg_go<T, 32, 64, 1, 2, 6, GLU, true>(a, s); break;
         case T64: tg_go<T, 64, 128, 1, 4, 3, GLU, true>(a, s); break;
         case T64N: tg_go<T, 64, 64, 2, 2, 5, GLU, true>(a, s); break;
+        case T64W: tg_go<T, 64, 256, 1, 8, 3, GLU, true>(a, s); break;
         case T128: tg_go<T, 128, 128, 2, 4, 5, GLU, true>(a, s); break;
         case T128N: tg_go<T, 128, 64, 4, 2, 6, GLU, true>(a, s); break;
         case T128W: tg_go<T, 128, 256, 2, 4, 3, GLU, true>(a, s); break;

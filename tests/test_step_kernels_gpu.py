@@ -63,6 +63,13 @@ def test_tile_gemm_glu(M, N, K, dtype):
     assert ((y.to(F64) - want).abs() <= limit).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 48904, 320), (64, 49160, 256), (47, 65528, 576)])
+def test_tile_gemm_wide(M, N, K):
+    """Tiles of 64 rows and 256 columns: rows and columns short of them, fewer chunks than the ring."""
+    test_tile_gemm(M, N, K, torch.bfloat16)
+    test_tile_gemm_glu(M, N, K, torch.float16)
+
+
 @pytest.mark.parametrize("M,N,K", [(193, 20616, 1088), (224, 6152, 4096), (255, 31000, 768)])
 def test_tile_gemm_256_rows(M, N, K):
     """The tile of 256 rows: rows and columns short of it, a ring that ends in each of its slots."""
