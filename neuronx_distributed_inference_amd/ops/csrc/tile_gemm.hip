@@ -335,6 +335,10 @@ struct TgPlan {
 // a little faster by themselves: the sum is a launch of its own, some 3 us. 48 rows, undivided /
 // two parts without their sum / library: (11408, 2048) 14.3 / 13.4 / 17.6 us, (16384, 2048)
 // 15.5 / 16.6 / 19.1, (12288, 4096) 23.6 / 22.5 / 25.2; 100 rows of the last 33.0 / 27.2 / 32.4.
+// From there to 128 rows tiles of 128 columns, for 256 in twice as many parts, where K is short and
+// they or their parts take 180 CUs: 128 rows (32000, 4096) 59.0 -> 52.3 us, (32000, 2048) 38.9 -> 29.1,
+// (24576, 4096) 51.0 -> 46.8, (16384, 4096) 39.8 -> 36.9; on 157 CUs (20000, 4096) 42.9 -> 44.5, and
+// (32000, 8192) 94.1 -> 95.2.
 TgPlan tg_plan(long M, long N, long K, bool glu, bool whole) {
     TgPlan p{T16, 16, 128, 0};
     if (M < 1 || M > 512 || N < 64 || N % (glu ? 8 : 4) || K < (whole && !glu ? 128 : 256) || K % TG_BK ||
@@ -343,13 +347,15 @@ TgPlan tg_plan(long M, long N, long K, bool glu, bool whole) {
     // half the width where that many more tiles spare parts of K, or with GLU fill the chip
     const bool narrow = glu ? N < 25600 : N <= 4096 || (whole && M <= 64 && N > 8192 && N <= 16384);
     const long wides = (N + 255) / 256, rounds = (wides + 255) / 256;
+    const long tiles128 = (N + 127) / 128;
+    const bool filled = whole && K <= 4096 && tiles128 <= 256 && tiles128 * (256 / tiles128) >= 180;
     const bool wide = wides >= 192 && wides * 100 >= rounds * 256 * 85;
     if (M <= 16) p = narrow ? TgPlan{T16N, 16, 64, 0} : TgPlan{T16, 16, 128, 0};
     else if (M <= 32) p = narrow ? TgPlan{T32N, 32, 64, 0} : TgPlan{T32, 32, 128, 0};
     else if (M <= 64 && wide) p = {T64W, 64, 256, 0};
     else if (M <= 64) p = narrow ? TgPlan{T64N, 64, 64, 0} : TgPlan{T64, 64, 128, 0};
     else if (M <= 128 && narrow && glu) p = {T128N, 128, 64, 0};
-    else if (M <= 128 && (glu ? N < 49152 : N * K < (60 << 20))) p = {T128, 128, 128, 0};
+    else if (M <= 128 && (glu ? N < 49152 : N * K < (60 << 20) || filled)) p = {T128, 128, 128, 0};
     else if (M <= 128) p = {T128W, 128, 256, 0};
     else if (N * K <= (20 << 20)) p = {T128B, 128, 128, 0};
     else if (M <= 192) p = {T192, 192, 128, 0};

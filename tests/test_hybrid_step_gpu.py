@@ -251,6 +251,14 @@ def test_products_of_whole_results(M, N, K):
         assert ((d(y) - want).abs() <= limit).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 32760, 320), (100, 22920, 2048), (128, 16376, 4096),
+                                   (127, 23044, 128)])
+def test_whole_products_of_full_chips(M, N, K):
+    """Tiles of 128 columns where they, or two parts of them, take 180 CUs and more, and just less."""
+    test_products_of_whole_results(M, N // 8 * 8, K)
+
+
+
 @pytest.mark.parametrize("out", [BF, torch.float32])
 @pytest.mark.parametrize("rows,C,summand", [(1, 8, None), (3, 2040, BF), (5, 2048, torch.float32),
                                             (2, 2056, BF), (7, 4104, BF), (2, 8192, torch.float32),
