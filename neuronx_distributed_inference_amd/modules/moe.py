@@ -43,16 +43,16 @@ class MoERouter(nn.Module):
         self.act = act  # "softmax" | "sigmoid" (Llama4: sigmoid of top-k logits)
 
     def forward(self, x: torch.Tensor):
-        logits = F.linear(x.float(), self.weight.float())  # (T, E)
-        if (logits.is_cuda and ops.extension_available()
+        if (x.is_cuda and ops.extension_available()
                 and self.top_k <= 8 and self.num_experts >= self.top_k):
             # fused top-k + activation + normalize: one launch vs the
             # ~6-kernel torch chain (launch-bound at decode sizes)
             sig = self.act == "sigmoid"
-            return ops.router_topk(
-                logits, self.top_k, sig,
+            return ops.router_choice(
+                x, self.weight, self.top_k, sig,
                 (not sig) and self.pre_softmax,
                 (not sig) and self.normalize)
+        logits = F.linear(x.float(), self.weight.float())  # (T, E)
         if self.act == "sigmoid":
             vals, idx = logits.topk(self.top_k, dim=-1)
             return torch.sigmoid(vals), idx

@@ -895,6 +895,24 @@ def attention_decode_paged(q, k_cache, v_cache, seq_lens, block_table,
 # segment. All table construction is tensor ops with STATIC shapes, so
 # the whole MoE layer is hipGraph-capturable.
 
+def router_choice(x: torch.Tensor, weight: torch.Tensor, top_k: int, act_sigmoid: bool,
+                  pre_softmax: bool, normalize: bool):
+    """router_topk of x @ weight^T in 32 bits, (T, K) rows in 16 or 32; in one launch for up to 8
+    experts, or 16 and fewer than 512 rows (csrc/router_topk.hip). GPU only."""
+    if (x.dim() == 2 and 0 < x.shape[1] and x.shape[1] % 8 == 0 and weight.dtype == torch.float32
+            and top_k <= weight.shape[0] <= (8 if x.shape[0] >= 512 else 16)
+            and x.dtype in (torch.bfloat16, torch.float16, torch.float32)
+            and x.is_contiguous() and weight.is_contiguous()
+            and (x.data_ptr() | weight.data_ptr()) % 16 == 0):
+        vals = torch.empty(x.shape[0], top_k, dtype=torch.float32, device=x.device)
+        idx = torch.empty(x.shape[0], top_k, dtype=torch.long, device=x.device)
+        _require_ext("router_few").router_few(vals, idx, x, weight, top_k, int(act_sigmoid),
+                                              int(pre_softmax), int(normalize))
+        return vals, idx
+    logits = torch.nn.functional.linear(x.float(), weight.float())
+    return router_topk(logits, top_k, act_sigmoid, pre_softmax, normalize)
+
+
 def router_topk(logits: torch.Tensor, top_k: int, act_sigmoid: bool,
                 pre_softmax: bool, normalize: bool):
     """Fused MoE router selection: top-k + activation + normalization in

@@ -93,6 +93,8 @@ void moe_routed_down(torch::Tensor out, torch::Tensor ws, torch::Tensor h, torch
                      c10::optional<torch::Tensor> weights, long mt);
 void row_max(torch::Tensor val, torch::Tensor idx, torch::Tensor x);
 void row_topk(torch::Tensor val, torch::Tensor idx, torch::Tensor x, long k);
+void router_few(torch::Tensor vals, torch::Tensor idx, torch::Tensor x, torch::Tensor w, long top_k,
+                long act_sigmoid, long pre_softmax, long normalize);
 void router_topk(torch::Tensor vals, torch::Tensor idx, torch::Tensor logits,
                  long top_k, long act_sigmoid, long pre_softmax,
                  long normalize);
@@ -254,6 +256,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("combine_out") = py::none(),
           py::arg("combine_scale") = py::none(),
           py::arg("combine_gather") = py::none());
+    m.def("router_few", &router_few, "MoE router of up to 16 experts: product and choice");
     m.def("router_topk", &router_topk,
           "fused MoE router top-k + activation + normalize (CDNA4)",
           py::arg("vals"), py::arg("idx"), py::arg("logits"),

@@ -970,3 +970,32 @@ def test_moe_route_of_any_number_of_choices(n_tok, E, k, first, El, itype):
     assert inv.tolist() == want_i
     got = gather.tolist()
     assert all(got[r] == tok for r, tok in want_g.items())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,E,k,K", [(1, 1, 1, 8), (3, 8, 2, 4096), (7, 3, 3, 4104), (200, 9, 8, 1000),
+                                     (511, 16, 4, 320), (512, 9, 2, 64), (1023, 5, 2, 512),
+                                     (1030, 8, 8, 520), (5, 8, 2, 36)])
+def test_router_of_few_experts(T, E, k, K, dtype):
+    """Product and choice in one launch against the same in 64 bits: the chosen are the largest but
+    for sums that lie within the rounding of 32 bits, their weights those of the chosen sums."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(T, K, device="cuda", generator=g).to(dtype)
+    w = torch.randn(E, K, device="cuda", generator=g) * 0.1
+    exact = x.to(F64) @ w.to(F64).t()
+    slack = K * 2.0 ** -24 * (x.to(F64).abs() @ w.to(F64).abs().t()).max()
+    for sigmoid, pre, norm in ((False, False, True), (False, True, False), (True, False, False)):
+        vals, idx = ops.router_choice(x, w, k, sigmoid, pre, norm)
+        assert vals.shape == idx.shape == (T, k) and vals.dtype == torch.float32
+        assert (idx.sort(-1).values.diff() > 0).all() and 0 <= idx.min() and idx.max() < E
+        chosen = exact.gather(1, idx)
+        assert (chosen >= exact.topk(k, -1).values - 2 * slack).all()
+        want = chosen.sigmoid() if sigmoid else \
+            (exact.softmax(-1).gather(1, idx) if pre else chosen.softmax(-1))
+        # exp of 32 bits, of sums that are off by the slack
+        assert ((vals - want).abs() <= want * (4 * slack + 2.0 ** -18)).all()
+    # a row that is not a number chooses as the rows of logits do
+    x[0] = float("nan")
+    got = ops.router_choice(x, w, k, False, False, True)
+    ref = ops.router_topk(torch.nn.functional.linear(x.float(), w), k, False, False, True)
+    assert torch.equal(got[1][:1], ref[1][:1])
