@@ -244,9 +244,11 @@ class AttentionBase(nn.Module):
         seq_ids: Optional[torch.Tensor] = None,
         active_mask: Optional[torch.Tensor] = None,
         sequence_parallel: bool = False,
+        output: Optional[torch.Tensor] = None,
     ) -> Optional[torch.Tensor]:
         """The input of the output projection (B, S, heads * head_dim), where a fused front end
-        serves this call; None where the modules one by one have to."""
+        serves this call; None where the modules one by one have to. With ``output``, that
+        projection's weight, its product as ops.linear_parts has it."""
         B, S, _ = hidden.shape
         if not self.use_rope:  # NoPE layer (Llama4 global-attention layers)
             cos, sin = None, None
@@ -293,8 +295,13 @@ class AttentionBase(nn.Module):
                 norms=norms or None, slots=kv_mgr.slot_mapping if paged else None,
                 dtype=hidden.dtype,
             )
+            if output is not None and B * S == 1 and active_mask is None:
+                y = self._decode_product(q, kv_mgr, position_ids, seq_ids, output)
+                if y is not None:
+                    return y
             out = self._decode(q, kv_mgr, position_ids, seq_ids, active_mask)
-            return out.transpose(1, 2).reshape(B, S, -1)
+            out = out.transpose(1, 2).reshape(B, S, -1)
+            return out if output is None else ops.linear_parts(out, output)
 
         # Fused CTE front end: one GEMM -> qkv_rope_update (RoPE + cache
         # scatter + q relayout) -> flash attention reading K/V straight from
@@ -326,7 +333,8 @@ class AttentionBase(nn.Module):
                     q, kc, vc, seq_ids, scale=self.scale, sinks=self.sinks,
                     sliding_window=self.sliding_window, token_major=True,
                 )
-            return out.transpose(1, 2).reshape(B, S, -1)
+            out = out.transpose(1, 2).reshape(B, S, -1)
+            return out if output is None else ops.linear_parts(out, output)
         return None
 
     # ------------------------------------------------------------------
@@ -561,6 +569,18 @@ class AttentionBase(nn.Module):
             sliding_window=self.sliding_window,
         )
 
+    def _decode_product(self, q, kv_mgr, position_ids, seq_ids, weight) -> Optional[torch.Tensor]:
+        """_decode of one token of one row and the output projection in one call, None where that
+        does not serve: its plain case."""
+        if (type(self)._decode is not _DECODE or "_decode" in self.__dict__
+                or getattr(kv_mgr, "is_paged", False) or self.kv_shard_degree > 1
+                or self.sinks is not None
+                or (getattr(kv_mgr, "ring_layers", None) and kv_mgr.is_ring(self.layer_idx))):
+            return None
+        kc, vc = kv_mgr.get_cache(self.layer_idx)
+        return ops.attention_decode_product(q, kc, vc, position_ids, seq_ids, float(self.scale),
+                                            int(self.sliding_window), weight)
+
     def _decode(self, q, kv_mgr, position_ids, seq_ids, active_mask) -> torch.Tensor:
         k_cache, v_cache = kv_mgr.get_cache(self.layer_idx)
         if active_mask is not None and active_mask.dim() == 4:
@@ -602,3 +622,7 @@ class AttentionBase(nn.Module):
             q, k_cache, v_cache, position_ids, seq_ids=seq_ids, scale=self.scale,
             sinks=self.sinks, sliding_window=self.sliding_window, ring=ring, token_major=True,
         )
+
+
+# what _decode_product stands for: a replaced method is called
+_DECODE = AttentionBase._decode

@@ -143,8 +143,9 @@ def run_layers(layers, final_norm, h: torch.Tensor, cos, sin, kv_mgr, position_i
     for layer, after in zip(layers, layers[1:] + [None]):
         attn, mlp = layer.fused_parts()
         args = (x, cos, sin, kv_mgr, position_ids, phase, attention_mask, seq_ids)
-        a = attn.attend_fused(*args)
-        y = attn(*args) if a is None else ops.linear_parts(a, attn.o_proj.o_proj.weight)
+        y = attn.attend_fused(*args, output=attn.o_proj.o_proj.weight)
+        if y is None:
+            y = attn(*args)
         norm = layer.post_attention_layernorm
         x = ops.add_norm(y, h, norm.weight, norm.variance_epsilon)
         y = _feed_forward(mlp, x)

@@ -564,6 +564,25 @@ def _attention_out(q, token_major):
     return torch.empty(B, S, H, D, dtype=q.dtype, device=q.device).transpose(1, 2)
 
 
+def attention_decode_product(q, k_cache, v_cache, positions, seq_ids, scale: float, window: int,
+                             weight):
+    """attention_decode of one token of one row, q (1, Hq, 1, D), and its product with weight
+    (N, Hq * D), as linear_parts has it; None where that does not serve."""
+    D = q.shape[3]
+    if not (q.is_cuda and D in (64, 128) and q.dtype in (torch.bfloat16, torch.float16)
+            and isinstance(k_cache, torch.Tensor) and k_cache.dtype == v_cache.dtype
+            and k_cache.dtype in (q.dtype, torch.float8_e4m3fn)
+            and q.is_contiguous() and k_cache.is_contiguous() and v_cache.is_contiguous()
+            and positions.numel() == 1 and weight.shape[1] == q.shape[1] * D
+            and _tile_takes(q.view(1, -1), weight)):
+        return None
+    if seq_ids is None:
+        seq_ids = torch.zeros(1, device=q.device, dtype=torch.int32)
+    y = _C.attention_decode_product(q, k_cache, v_cache, positions.to(torch.int32).contiguous(),
+                                    seq_ids.to(torch.int32).contiguous(), scale, window, weight)
+    return y.view(*y.shape[:-2], 1, 1, weight.shape[0])
+
+
 def _extend_on_mfma(q, k_cache, v_cache):
     """Several query tokens of a 16-bit model against a cache of the same type: the matrix-core
     kernel reads each K/V row once for all of them; the decode kernel (once for 16 pairs of token

@@ -936,6 +936,13 @@ __global__ __launch_bounds__(256) void decode_attn_pass2(
 }
 
 // ---------------------------------------------------------------------------
+// the shares of a decode row's keys, where the caller adds them up
+struct DecodeShares {
+    torch::Tensor o, ml;         // (B, Hq, Sq, n, D) and (B, Hq, Sq, n, 2) in fp32
+    int n = 1;                   // 1: none, the result is there
+    long most = 0;               // that the caller takes
+};
+
 template <typename T, typename CT, int D, int GQ>
 static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
                           const torch::Tensor& k_cache, const torch::Tensor& v_cache,
@@ -945,7 +952,7 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
                           int block_size = 0, float v_scale = 1.0f,
                           const torch::Tensor* sinks = nullptr,
                           torch::Tensor* lse_out = nullptr,
-                          int ring = 0) {
+                          int ring = 0, DecodeShares* shares = nullptr) {
     const int B = q.size(0), Hq = q.size(1), Sq = q.size(2);
     const bool paged = block_table != nullptr;
     const int Hkv = paged ? k_cache.size(2) : k_cache.size(1);
@@ -1039,6 +1046,12 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
 #undef DM_RUN
         HIP_CHECK_KERNEL();
         if (nsplit == 1) return;
+        if (shares && nsplit <= shares->most) {
+            shares->o = o_part;
+            shares->ml = ml_part;
+            shares->n = nsplit;
+            return;
+        }
     } else if (paged) {
         hipLaunchKernelGGL((decode_attn_pass1<T, CT, D, GQ, true>), grid1, dim3(256), 0, stream,
                            o_part.data_ptr<float>(), ml_part.data_ptr<float>(),
@@ -1076,7 +1089,8 @@ static void dispatch_gq(torch::Tensor& out, const torch::Tensor& q,
                         float scale, int window, int gq,
                         const torch::Tensor* bt = nullptr, int bs = 0,
                         float v_scale = 1.0f, const torch::Tensor* sinks = nullptr,
-                        torch::Tensor* lse_out = nullptr, int ring = 0) {
+                        torch::Tensor* lse_out = nullptr, int ring = 0,
+                        DecodeShares* shares = nullptr) {
     const bool fp8 = k_cache.scalar_type() == at::ScalarType::Float8_e4m3fn;
     if constexpr (!std::is_same<T, float>::value && (D == 64 || D == 128)) {
         // the matrix-core kernel takes heads in columns: any ratio
@@ -1084,10 +1098,11 @@ static void dispatch_gq(torch::Tensor& out, const torch::Tensor& q,
                     "GQA ratio > 8 not supported yet (got ", gq, ")");
         if (fp8)
             launch_decode<T, __hip_fp8_e4m3, D, 1>(out, q, k_cache, v_cache, seq_lens, seq_ids, scale,
-                                                   window, gq, bt, bs, v_scale, sinks, lse_out, ring);
+                                                   window, gq, bt, bs, v_scale, sinks, lse_out, ring,
+                                                   shares);
         else
             launch_decode<T, T, D, 1>(out, q, k_cache, v_cache, seq_lens, seq_ids, scale, window, gq,
-                                      bt, bs, v_scale, sinks, lse_out, ring);
+                                      bt, bs, v_scale, sinks, lse_out, ring, shares);
         return;
     }
 #define GQ_CASE(CT)                                                                     \
@@ -1226,4 +1241,48 @@ void attention_decode(torch::Tensor out, torch::Tensor q,
         TORCH_CHECK(false, "attention_decode: unsupported dtype");
     }
 #undef CASE_T
+}
+
+torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
+                        long splits, bool parts, long glu);
+long tile_gemm_splits(long M, long N, long K, long glu, bool whole);
+torch::Tensor shares_gemm(const torch::Tensor& o, const torch::Tensor& ml, long n, const torch::Tensor& w);
+
+// Values of all shares that a workgroup of the product adds up, at most: 256 workgroups read theirs from
+// the L2 where the kernel before would read each once. Both kernels / one, us: 6 shares of 256 (32 heads
+// of 64, context 700) 11.8 / 10.0, 6 of 1024 (32 heads of 128) 16.6 / 15.6, 16 of 256 14.1 / 13.6, but 32
+// of 1024 (context 8000) 22.1 / 23.5 and 36.4 / 42.1 (64 heads).
+constexpr long DECODE_SHARES = 8192;
+
+// attention_decode of one token of one row (16 bits, heads of 64 or 128) and the product with w
+// (N, Hq * D): as tile_gemm leaves it, its parts of K or the result.
+torch::Tensor attention_decode_product(torch::Tensor q, torch::Tensor k_cache, torch::Tensor v_cache,
+                                       torch::Tensor positions, torch::Tensor seq_ids, double scale,
+                                       long window, torch::Tensor w) {
+    TORCH_CHECK(q.dim() == 4 && k_cache.dim() == 4 && q.size(0) == 1 && q.size(2) == 1 &&
+                positions.numel() == 1, "attention_decode_product: one token of one row");
+    const int D = q.size(3), Hq = q.size(1), Hkv = k_cache.size(1);
+    TORCH_CHECK((D == 64 || D == 128) && Hq % Hkv == 0 && w.dim() == 2 && w.size(1) == (long)Hq * D &&
+                w.scalar_type() == q.scalar_type(), "attention_decode_product: shapes and types");
+    TORCH_CHECK(q.is_contiguous() && k_cache.is_contiguous() && v_cache.is_contiguous(),
+                "contiguous tensors required");
+    torch::Tensor out = torch::empty_like(q);
+    const long splits = tile_gemm_splits(1, w.size(0), w.size(1), 0, false);
+    TORCH_CHECK(splits > 0, "attention_decode_product: product not taken");
+    DecodeShares shares;
+    shares.most = DECODE_SHARES / ((w.size(1) / 64 + splits - 1) / splits * 64);
+#define ADP(T, DD)                                                                                 \
+    dispatch_gq<T, DD>(out, q, k_cache, v_cache, positions, seq_ids, (float)scale, (int)window,    \
+                       Hq / Hkv, nullptr, 0, 1.0f, nullptr, nullptr, 0, &shares)
+    if (q.scalar_type() == at::ScalarType::BFloat16) {
+        if (D == 128) ADP(__hip_bfloat16, 128);
+        else ADP(__hip_bfloat16, 64);
+    } else {
+        TORCH_CHECK(q.scalar_type() == at::ScalarType::Half, "attention_decode_product: 16 bits");
+        if (D == 128) ADP(__half, 128);
+        else ADP(__half, 64);
+    }
+#undef ADP
+    if (shares.n > 1) return shares_gemm(shares.o, shares.ml, shares.n, w);
+    return tile_gemm(out.view({1, (long)Hq * D}), w, c10::nullopt, 0, true, 0);
 }

@@ -117,6 +117,9 @@ int lt_tune(int64_t M, int64_t N, int64_t K, bool has_bias,
 void gelu_tanh_mul_fused(torch::Tensor out, torch::Tensor gate_up);
 void add_norm(torch::Tensor out, torch::Tensor residual, torch::Tensor y, torch::Tensor weight,
               double eps);
+torch::Tensor attention_decode_product(torch::Tensor q, torch::Tensor k_cache, torch::Tensor v_cache,
+                                       torch::Tensor positions, torch::Tensor seq_ids, double scale,
+                                       long window, torch::Tensor w);
 torch::Tensor tile_gemm_pair(torch::Tensor x, torch::Tensor w, torch::Tensor x2, torch::Tensor w2);
 long tile_gemm_splits(long M, long N, long K, long glu, bool whole);
 torch::Tensor tile_gemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
@@ -162,6 +165,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("copy_many", &copy_many, "several copies in one launch");
     m.def("tile_gemm_splits", &tile_gemm_splits, "parts of K of a tiled product, 0: not taken",
           py::arg("M"), py::arg("N"), py::arg("K"), py::arg("glu") = 0, py::arg("whole") = false);
+    m.def("attention_decode_product", &attention_decode_product,
+          "decode attention of one token and the output product");
     m.def("tile_gemm_pair", &tile_gemm_pair, "parts of K of two tiled products of one shape");
     m.def("tile_gemm", &tile_gemm, "tiled 16-bit product of up to 512 rows (CDNA4)",
           py::arg("x"), py::arg("w"), py::arg("bias") = py::none(), py::arg("splits") = 0,

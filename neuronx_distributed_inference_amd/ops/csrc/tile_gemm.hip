@@ -275,6 +275,142 @@ __global__ __launch_bounds__(64 * WM * WN) void tile_gemm_kernel(const TgArgs a)
     }
 }
 
+// tile_gemm_kernel for one row of attention's output that is still in shares of its keys (n of each
+// head's D values, with their maxima and sums): 4 waves add up the chunk of K that the workgroup
+// has, which is little, while the others have their first D chunks of w on the way. A wave reads
+// back from LDS what it loaded itself, so these wait for the sum, once, and never for each other.
+// Bound by latency, hence one launch for two: 2048 x 2048 behind 6 shares of 32 heads of 64, attention
+// included, 11.8 -> 10.0 us (see DECODE_SHARES for where the line lies).
+template <typename T, int BN, int WN, int D>
+__global__ __launch_bounds__(64 * (WN + 4)) void shares_gemm_kernel(const TgArgs a,
+                                                                    const float* __restrict__ o,
+                                                                    const float* __restrict__ ml,
+                                                                    const int shares, const int HD) {
+    using MF = TgMfma<T>;
+    using VT = VecTraits<T>;
+    using vec8 = typename MF::vec8;
+    constexpr int FN = BN / WN / 16, WP = BN / 8 / WN, WB = BN * 128;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    T* const xs = reinterpret_cast<T*>(smem + D * WB);       // of the workgroup's part of K
+
+    const int item = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
+    if (item >= a.work) return;
+    const int nt = item % a.ntiles, slice = item / a.ntiles;
+    const int chunks = a.K / TG_BK;
+    const int c_lo = (int)((long)slice * chunks / a.splits);
+    const int n = (int)((long)(slice + 1) * chunks / a.splits) - c_lo;
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+    if (wid >= WN) {
+        constexpr int U = 8;                                 // shares whose loads go out together
+        for (int i = (threadIdx.x - WN * 64) * 4; i < n * TG_BK; i += 1024) {
+            const int k = c_lo * TG_BK + i, head = k / HD;
+            const float* op = o + (long)head * shares * HD + k % HD;
+            const float* mp = ml + (long)head * shares * 2;
+            float m = -1e30f, l = 0.f;
+            tg_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            for (int s0 = 0; s0 < shares; s0 += U) {
+                tg_f32x4 v[U];
+                float2 p[U];
+                float mn = m;
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int s = min(s0 + u, shares - 1);
+                    p[u] = *reinterpret_cast<const float2*>(mp + s * 2);
+                    v[u] = *reinterpret_cast<const tg_f32x4*>(op + (long)s * HD);
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) mn = fmaxf(mn, p[u].x);
+                const float f = __expf(m - mn);
+                m = mn;
+                l *= f;
+                acc *= f;
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (s0 + u < shares) {
+                        const float e = __expf(p[u].x - m);
+                        l += p[u].y * e;
+                        acc += v[u] * e;
+                    }
+            }
+            const float inv = l > 0.f ? 1.f / l : 0.f;
+            __align__(8) T r[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) r[j] = VT::from_float(acc[j] * inv);
+            *reinterpret_cast<int2*>(xs + i) = *reinterpret_cast<int2*>(r);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        return;
+    }
+
+    const int lrow = lane & 15, lslot = lane >> 4, prow = lane >> 3;
+    const unsigned kbytes = (unsigned)a.K * sizeof(T);
+    unsigned wo[WP];
+#pragma unroll
+    for (int i = 0; i < WP; ++i) {
+        const int q = (wid * WP + i) * 8 + prow;
+        wo[i] = min(q, a.N - 1 - nt * BN) * kbytes + ((lane & 7) ^ (q & 7)) * 16;
+    }
+    const char* w0 = (const char*)a.w + (long)nt * BN * kbytes + (long)c_lo * 128;
+    const int first = (blockIdx.x >> 3) % n;                 // as in tile_gemm_kernel
+    int at = first, to = 0;
+    auto stage = [&]() {
+        char* base = smem + to * WB + wid * (WP * 1024);
+        const char* wp = w0 + (long)at * 128;
+#pragma unroll
+        for (int i = 0; i < WP; ++i) tg_load<2>(wp + wo[i], base + i * 1024);
+        at = at + 1 == n ? 0 : at + 1;
+        to = to + 1 == D ? 0 : to + 1;
+    };
+    tg_f32x4 acc[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[j] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+        if (i < n) stage();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int bw = 0, c = first;
+    for (int t = 0; t < n; ++t) {
+        tg_wait_chunks<WP, D - 1>(n - 1 - t);
+        vec8 xa[2], wb[2][FN];
+        const char* wp = smem + bw * WB + wid * (WP * 1024) + lrow * 128;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            xa[h] = *reinterpret_cast<const vec8*>(xs + c * TG_BK + h * 32 + lslot * 8);
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                wb[h][j] = *reinterpret_cast<const vec8*>(
+                    wp + j * 2048 + (((h * 4 + lslot) ^ (lrow & 7)) << 4));
+        }
+        if (t + D < n) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            stage();
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[j] = MF::mfma(wb[h][j], xa[h], acc[j]);
+        c = c + 1 == n ? 0 : c + 1;
+        bw = bw + 1 == D ? 0 : bw + 1;
+    }
+    if (lrow) return;                                        // (16 times the same row)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+        const int col = nt * BN + wid * (BN / WN) + j * 16 + lslot * 4;
+        if (col >= a.N) continue;
+        if (a.part) {
+            *reinterpret_cast<tg_f32x4*>(a.part + (long)slice * a.N + col) = acc[j];
+            continue;
+        }
+        __align__(8) T r[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) r[q] = VT::from_float(acc[j][q]);
+        *reinterpret_cast<int2*>((T*)a.y + col) = *reinterpret_cast<int2*>(r);
+    }
+}
+
 // y = sum of the parts (+ bias)
 template <typename T>
 __global__ __launch_bounds__(256) void tile_sum_kernel(T* __restrict__ y,
@@ -513,4 +649,60 @@ torch::Tensor tile_gemm_pair(torch::Tensor x, torch::Tensor w, torch::Tensor x2,
     a.xbytes2 = tg_row_bytes(x2);
     tg_launch(a, plan.tile, x.scalar_type() == at::kBFloat16, PLAIN);
     return part;
+}
+
+namespace {
+
+template <typename T, int BN, int WN, int D>
+void tg_shares_go(TgArgs& a, const float* o, const float* ml, int shares, int HD, hipStream_t stream) {
+    a.mblocks = 1;
+    a.ntiles = (a.N + BN - 1) / BN;
+    a.work = a.ntiles * a.splits;
+    a.per_xcd = (a.work + 7) / 8;
+    const int longest = (a.K / TG_BK + a.splits - 1) / a.splits, lds = D * BN * 128 + longest * 128;
+    TORCH_CHECK(lds <= 163840, "shares_gemm: K");
+    auto* k = shares_gemm_kernel<T, BN, WN, D>;
+    // (a limit of the function, the same in every call)
+    TORCH_CHECK(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    163840) == hipSuccess, "shares_gemm: LDS");
+    hipLaunchKernelGGL(k, dim3(a.per_xcd * 8), dim3(64 * (WN + 4)), lds, stream, a, o, ml, shares, HD);
+    HIP_CHECK_KERNEL();
+}
+
+}  // namespace
+
+// o (heads, n, D) and ml (heads, n, 2): attention's shares of one row. Their sum @ w^T, with its
+// parts of K as tile_gemm leaves them.
+torch::Tensor shares_gemm(const torch::Tensor& o, const torch::Tensor& ml, long n, const torch::Tensor& w) {
+    TgArgs a{};
+    a.M = 1;
+    a.K = w.size(1);
+    a.N = w.size(0);
+    const long heads = ml.numel() / (2 * n);
+    const int HD = (int)(a.K / heads);
+    TORCH_CHECK(o.numel() == n * a.K && heads * HD == a.K && HD % 4 == 0, "shares_gemm: shares");
+    TORCH_CHECK(w.is_contiguous() && (size_t)w.data_ptr() % 16 == 0, "shares_gemm: weight");
+    const TgPlan plan = tg_plan(1, a.N, a.K, false, false);
+    TORCH_CHECK(plan.splits > 0, "shares_gemm: shape not taken");
+    a.splits = plan.splits;
+    torch::Tensor y;
+    if (a.splits > 1) {
+        y = torch::empty({a.splits, 1, a.N}, o.options());
+        a.part = y.data_ptr<float>();
+    } else {
+        y = torch::empty({1, a.N}, w.options());
+        a.y = y.data_ptr();
+    }
+    a.w = w.data_ptr();
+    auto s = at::hip::getCurrentHIPStream();
+    const float *op = o.data_ptr<float>(), *mp = ml.data_ptr<float>();
+    const bool narrow = plan.tile == T16N;
+    if (w.scalar_type() == at::kBFloat16) {
+        if (narrow) tg_shares_go<__hip_bfloat16, 64, 2, 8>(a, op, mp, (int)n, HD, s);
+        else tg_shares_go<__hip_bfloat16, 128, 4, 4>(a, op, mp, (int)n, HD, s);
+    } else {
+        if (narrow) tg_shares_go<__half, 64, 2, 8>(a, op, mp, (int)n, HD, s);
+        else tg_shares_go<__half, 128, 4, 4>(a, op, mp, (int)n, HD, s);
+    }
+    return y;
 }

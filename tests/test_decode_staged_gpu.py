@@ -58,3 +58,34 @@ def test_staged_pages_as_straight(B, Hkv, gq, pages, size, D):
     call = lambda k, v: ops.attention_decode_paged(q, k, v, pos, table)  # noqa: E731
     a, b = call(k, v), call(_off(k), _off(v))
     assert a.isfinite().all() and torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hq,Hkv,D,N,L,pos,f8", [
+    (32, 8, 64, 2048, 1024, 700, False), (32, 8, 128, 4096, 1024, 1023, False), (8, 8, 64, 516, 512, 0, False),
+    (4, 1, 64, 64, 2048, 900, True), (16, 2, 128, 2048, 4096, 4000, True), (64, 8, 128, 8192, 8192, 8000, False),
+    (9, 3, 128, 1000, 300, 200, False), (8, 2, 64, 20000, 1500, 1400, False), (4, 4, 64, 100, 4096, 17, False)])
+def test_decode_and_its_product(Hq, Hkv, D, N, L, pos, f8, dtype):
+    """One token's attention and output product in one call: the same to the bit as one after the
+    other, with shares added up by the product, by a kernel of their own, and with none."""
+    g = torch.Generator(device="cuda").manual_seed(L + N)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)  # noqa: E731
+    q, w = rnd(1, Hq, 1, D), rnd(N, Hq * D) * 0.05
+    kc, vc = (rnd(3, Hkv, L, D) for _ in range(2))
+    if f8:
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    p = torch.tensor([[pos]], device="cuda", dtype=torch.int32)
+    sid = torch.tensor([2], device="cuda", dtype=torch.int32)
+    for window in (0, 130):
+        y = ops.attention_decode_product(q, kc, vc, p, sid, D ** -0.5, window, w)
+        o = ops.attention_decode(q, kc, vc, p, seq_ids=sid, scale=D ** -0.5, sliding_window=window)
+        want = ops.linear_parts(o.transpose(1, 2).reshape(1, 1, Hq * D), w)
+        assert y.shape == want.shape and y.dtype == want.dtype
+        # shares are added up eight at a time, of which 32 bits show the order
+        both = [t.float().sum(0) if t.dim() == 4 else t.float() for t in (y, want)]
+        slack = 2.0 ** -8 * (o.flatten().float().abs() @ w.float().abs().t())
+        assert ((both[0] - both[1]).abs().view(-1) <= slack).all()
+    vc[2, :, min(pos, 5)] = float("nan")
+    y = ops.attention_decode_product(q, kc, vc, p, sid, D ** -0.5, 0, w)
+    assert y.float().isnan().any()
+    assert ops.attention_decode_product(q.float(), kc, vc, p, sid, 1.0, 0, w) is None
