@@ -49,11 +49,11 @@
 //   8 experts of 4096 x 14336, 2 a token:  16 tokens 558 -> 434, 128 586 -> 453, 256 630 -> 475,
 //     1024 1115 -> 917, 2048 1700;  in 8 bits 16 tokens 305 -> 226, 128 320 -> 262, 200 349 -> 279,
 //     256 400 -> 378
-// Row tiles there, before the last two of these (rows an expert on average: times of tiles of 32, 64, 96, 128, 160 rows):
-//   128 experts  32: 283 257 261 264 270;  64: 376 318 290 295 296;  128: 578 445 414 405 357;
-//     188: 751 563 512 487 551;  256: 1015 730 647 601 562
-//   8 experts in 8 bits (32, 48, 64 rows)  4: 270 275 275;  32: 332 289 295;  40: 369 294 304;
-//     50: 386 407 312;  64: 513 421 404
+// Row tiles there (rows an expert on average: times of tiles of 32, 64, 96, 128, 160 rows):
+//   128 experts  32: 261 228 232 238 245;  64: 359 297 252 263 264;  128: 565 425 400 380 322;
+//     188: 741 544 485 476 509;  256: 990 693 587 575 532
+//   8 experts in 8 bits (32, 48, 64 rows)  4: 241 242 240;  32: 295 261 268;  40: 339 288 285;
+//     50: 362 369 284;  64: 462 398 388
 
 #include "common.h"
 #include <torch/extension.h>
