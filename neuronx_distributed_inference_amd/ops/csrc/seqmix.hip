@@ -1784,8 +1784,6 @@ __global__ void __launch_bounds__(WD_WAVES * WAVE) window_decode_kernel(const Wf
     l += __shfl_xor(l, 32, WAVE);
 
     // ---- the waves meet ----
-    // the row that was written may be read again below
-    if (OWN && wid == WD_WAVES - 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     float* ml = wd_lds;                                  // [waves][16][2]
     float* ol = wd_lds + WD_WAVES * 32;                  // [waves][nc][D]
     if (q4 == 0) {
@@ -1840,10 +1838,11 @@ __global__ void __launch_bounds__(WD_WAVES * WAVE) window_decode_kernel(const Wf
                 const int mm = min(k0 + lane, nk - 1), j = mm < nfirst ? mm : mm + shift;
                 const int page = bt[j / a.bsz];
                 const long slot = (long)max(page, 0) * a.bsz + j % a.bsz;
+                // (the token's own row is in the cache by the hand of one workgroup of several)
+                const bf16* kp = OWN && mm == nk - 1 ? kown : kbase + slot * a.ktok;
                 float s = 0.f;
 #pragma unroll 1
-                for (int e = 0; e < D; ++e)
-                    s += __bfloat162float(qp[e]) * __bfloat162float(kbase[slot * a.ktok + e]);
+                for (int e = 0; e < D; ++e) s += __bfloat162float(qp[e]) * __bfloat162float(kp[e]);
                 s = biased(s, k0 + lane, c, b1, b2);
                 const float mn = fmaxf(mr, wave_max(s));
                 const float f = mr == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mr - mn);
@@ -1859,10 +1858,10 @@ __global__ void __launch_bounds__(WD_WAVES * WAVE) window_decode_kernel(const Wf
                     const long sk = ((long)__shfl((int)(slot >> 32), k, WAVE) << 32) |
                                     (unsigned)__shfl((int)slot, k, WAVE);
                     if (pk == 0.f) continue;
+                    const bf16* vp = OWN && k0 + k == nk - 1 ? vown : vbase + sk * a.vtok;
 #pragma unroll
                     for (int e = 0; e < D / 64; ++e)
-                        y[e] += pk * __bfloat162float(
-                            a.vc[(long)g * a.vhead + sk * a.vtok + lane * (D / 64) + e]);
+                        y[e] += pk * __bfloat162float(vp[lane * (D / 64) + e]);
                 }
             }
             float z[4];

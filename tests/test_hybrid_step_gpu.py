@@ -169,18 +169,26 @@ def test_delta_step_with_its_convolution(B, H, D, Dv, taps, per_head):
 
 @pytest.mark.parametrize("B,H,G,D,page,bad,window", [
     (1, 2, 2, 128, 16, False, 33), (9, 8, 2, 64, 64, False, 33), (5, 40, 1, 128, 7, False, 33),
-    (4, 4, 4, 128, 32, True, 33), (33, 16, 4, 128, 64, True, 700), (25, 8, 4, 64, 80, True, 510)])
-def test_window_attention_writes_its_rows(B, H, G, D, page, bad, window):
+    (4, 4, 4, 128, 32, True, 33), (33, 16, 4, 128, 64, True, 700), (25, 8, 4, 64, 80, True, 510),
+    # several workgroups a KV head, of which one writes the row that all of them see
+    (4, 34, 2, 64, 16, True, 33), (5, 40, 1, 128, 7, True, 33), (34, 40, 1, 64, 80, True, 600)])
+@pytest.mark.parametrize("writes", [True, False])
+def test_window_attention_writes_its_rows(B, H, G, D, page, bad, window, writes):
+    """Against the rows written by a launch of their own. A row without a place in the cache, or
+    whose page is missing, counts with its own key and value all the same."""
     g = torch.Generator(device="cuda").manual_seed(D)
     rnd = lambda *s: torch.empty(*s, device="cuda").normal_(0, 1, generator=g).to(BF)  # noqa: E731
     pages = 8 * B
     kc, vc = rnd(pages, page, G, D), rnd(pages, page, G, D)
     q, k, v, gate = rnd(B, 1, H * D), rnd(B, G * D), rnd(B, G * D), rnd(B, 1, H * D)
+    pos = torch.randint(0, 8 * page, (B, 1), generator=g, device="cuda")
+    pos[0] = 0
+    if B > 2:
+        pos[2] = 3 * page                              # the first of its page
     if bad:
         v[0, 3] = float("inf")
         v[1, 5] = float("nan")
-    pos = torch.randint(0, 8 * page, (B, 1), generator=g, device="cuda")
-    pos[0] = 0
+        v[2, 1] = float("-inf")
     seq = torch.arange(B, device="cuda")
     if B > 6:
         seq[3] = pos[3] = -1
@@ -188,15 +196,23 @@ def test_window_attention_writes_its_rows(B, H, G, D, page, bad, window):
     table = torch.randperm(pages, generator=g, device="cuda").view(B, 8).int()
     slots = torch.where(pos < 0, -1, table.gather(1, pos.clamp(min=0) // page) * page + pos % page).view(-1)
     r1, r2 = torch.rand(H, device="cuda"), torch.rand(H, device="cuda")
-    call = lambda kc, vc, **kw: seqmix.window_bias_attention(  # noqa: E731
+    call = lambda kc, vc, table, **kw: seqmix.window_bias_attention(  # noqa: E731
         q, kc, vc, step, table, r1, r2, D ** -0.5, window, 2, H, gate=gate, **kw)
     k1, v1 = kc.clone(), vc.clone()
     assert seqmix.new_rows_taken(q, k, v, gate, kc, vc)
-    got = call(k1, v1, new_rows=(k, v, slots))
+    if writes:
+        got, after = call(k1, v1, table, new_rows=(k, v, slots)), (k1, v1)
+    else:
+        gone = table.clone()
+        if B > 2:
+            gone[2, 3] = -1
+        before = k1.clone(), v1.clone()
+        got, after = call(k1, v1, gone, new_rows=(k, v, torch.full_like(slots, -1))), None
+        assert all(torch.equal(x.view(torch.int16), y.view(torch.int16)) for x, y in zip((k1, v1), before))
     seqmix.paged_kv_write(kc, vc, k, v, slots, step)
-    want = call(kc, vc)
+    want = call(kc, vc, table)
     live = seq >= 0
-    for x, y in ((got[live], want[live]), (k1, kc), (v1, vc)):
+    for x, y in ((got[live], want[live]), *zip(after or (), (kc, vc))):
         assert torch.equal(x.view(torch.int16), y.view(torch.int16))
 
 
