@@ -268,12 +268,15 @@ class NabelixLayer(nn.Module):
         linears += [right.ag2] if right.ag2 is not None else []
         linears += [mlp.gate_up_proj, mlp.down_proj] if mlp is not None and mlp.fused else []
         weights = [t.weight for t in linears if t is not None]
+        small = [self.norm1.weight, self.canon.weight]       # in 16-byte pieces too
+        small += [self.norm2.weight] if mlp is not None else []
         if not (like.is_cuda and like.dtype == self.out_dtype == torch.bfloat16
                 and right.ag2 is not None and right.num_heads == right.num_kv_heads
                 and right.dim in (64, 128) and right.vdim <= 128
                 and (mlp is None or (mlp.fused and mlp.act_mul_fused is seqmix.gelu_tanh_mul_fused))
                 and all(plain_linear(t, like) for t in linears)
                 and all(w.is_contiguous() and w.data_ptr() % 16 == 0 for w in weights)
+                and all(w.data_ptr() % 16 == 0 for w in small)
                 and m.left_o.weight.shape == m.right_o.weight.shape
                 and all(t.bias is None and 2 <= t.taps <= 4 for t in (self.canon, right.conv))
                 and self.canon.residual and self.canon.activation == "none"
@@ -350,6 +353,7 @@ class NabelixModel(HybridDecoderModel):
                 and not getattr(self, "eagle3_capture_layers", None)
                 and type(self.norm) is _FinalNorm and _FinalNorm.forward is _FINAL
                 and not _hooked(self.norm) and self.norm.bias is None
+                and self.norm.weight.data_ptr() % 16 == 0
                 and self.norm.out_dtype == torch.bfloat16
                 and positions.device.index == torch.cuda.current_device()
                 and all(layer.steps_once(rows) for layer in self.layers))
