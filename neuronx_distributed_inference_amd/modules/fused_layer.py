@@ -28,6 +28,7 @@ from neuronx_distributed_inference_amd.parallel.layers import plain_linear
 
 # what the loop does in their place, by heart: a class whose forward was replaced is not plain
 _FORWARDS = {c: c.forward for c in (AttentionBase, GroupQueryAttentionO, GatedMLP, RMSNorm)}
+_ATTEND = AttentionBase.attend_fused
 
 
 def _plain(module, cls) -> bool:
@@ -38,6 +39,11 @@ def _plain_norm(norm, h: torch.Tensor) -> bool:
     weight = norm._parameters.get("weight")
     return (_plain(norm, RMSNorm) and weight is not None and weight.dtype == h.dtype
             and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
+
+
+def _own_attend(attn) -> bool:
+    """Whether a program has put an attend_fused of its own in place, which knows no `output`."""
+    return type(attn).attend_fused is not _ATTEND or "attend_fused" in attn.__dict__
 
 
 def fusable(layers, final_norm, h: torch.Tensor, attention_mask, phase: str) -> bool:
@@ -92,6 +98,8 @@ def prompt_operands(layers, final_norm, h, x, cos, kv_mgr, seq_ids):
     weights, sizes, numbers = [], [], []
     for layer, after in zip(layers, layers[1:] + [None]):
         attn, mlp = layer.fused_parts()
+        if _own_attend(attn):
+            return None
         qkv = attn.qkv_proj
         rows = attn.prompt_front(x, cos, kv_mgr, PHASE_CTE, seq_ids)
         if (rows is None or not attn.use_rope or attn.sinks is not None or attn._front_norms(x)
@@ -143,7 +151,11 @@ def run_layers(layers, final_norm, h: torch.Tensor, cos, sin, kv_mgr, position_i
     for layer, after in zip(layers, layers[1:] + [None]):
         attn, mlp = layer.fused_parts()
         args = (x, cos, sin, kv_mgr, position_ids, phase, attention_mask, seq_ids)
-        y = attn.attend_fused(*args, output=attn.o_proj.o_proj.weight)
+        if _own_attend(attn):
+            y = attn.attend_fused(*args)
+            y = y if y is None else ops.linear_parts(y, attn.o_proj.o_proj.weight)
+        else:
+            y = attn.attend_fused(*args, output=attn.o_proj.o_proj.weight)
         if y is None:
             y = attn(*args)
         norm = layer.post_attention_layernorm

@@ -639,6 +639,45 @@ def test_a_forward_of_its_own_is_called(what, moe, monkeypatch):
     assert (own - plain).norm() > 0.05 * plain.norm()
 
 
+@pytest.mark.parametrize("of_class", [False, True])
+@pytest.mark.parametrize("rows", [1, 2])
+def test_an_attend_fused_of_its_own_is_called(of_class, rows, monkeypatch):
+    """With the arguments that it always had, in short and in ragged prompts and in steps."""
+    lm = _small_llama("bfloat16")
+    lm.enable_submodels()
+    attn = lm.model.layers[1].self_attn
+    ids = torch.randint(0, 512, (rows, 70), device="cuda")
+    mask = torch.ones_like(ids)
+    mask[-1, 60:] = 0
+
+    def run():
+        lm.reset()
+        with torch.inference_mode():
+            a = lm(input_ids=ids, attention_mask=mask).logits
+            lm.reset()
+            b = lm(input_ids=ids).logits
+            c = lm(input_ids=ids[:, :1], position_ids=torch.full((rows, 1), 70, device="cuda")).logits
+        return torch.stack([a, b, c]).float()
+
+    plain, seen = run(), []
+    inner = type(attn).attend_fused
+
+    def own(self, hidden, cos, sin, kv_mgr, position_ids, phase, attention_mask=None, seq_ids=None,
+            active_mask=None, sequence_parallel=False):
+        seen.append(phase)
+        return inner(self, hidden, cos, sin, kv_mgr, position_ids, phase, attention_mask, seq_ids,
+                     active_mask, sequence_parallel) * 0.5
+
+    if of_class:
+        base = next(c for c in type(attn).__mro__ if "attend_fused" in vars(c))
+        monkeypatch.setattr(base, "attend_fused", own)
+    else:
+        attn.attend_fused = own.__get__(attn)
+    got = run()
+    assert len(seen) == (6 if of_class else 3)
+    assert ((got - plain).flatten(1).norm(dim=1) > 0.02 * plain.flatten(1).norm(dim=1)).all()
+
+
 def test_hooks_of_all_modules_see_the_qkv_projection():
     lm = _small_llama("bfloat16")
     ids = torch.randint(0, 512, (2, 70), device="cuda")
