@@ -167,8 +167,8 @@ class ModelWrapper:
                 S, self.buckets,
                 strategy=getattr(self.ec, "bucket_strategy", "first_fit"))
             # padding (of the rows, to the bucket and of the batch) is left out where the layers
-            # can do without it
-            if S > 1:
+            # can do without it; a captured call has no lengths of its own
+            if S > 1 and not (input_ids.is_cuda and torch.cuda.is_current_stream_capturing()):
                 lengths = None if attention_mask is None else \
                     ops.PromptLengths(attention_mask, position_ids)
                 pack = getattr(self.model, "packed_prompts", None)

@@ -116,3 +116,34 @@ def test_left_padding_keeps_the_mask():
     inner = lm.model.packed_prompts
     lm.model.packed_prompts = lambda *a: took.append(inner(*a))
     assert _run(lm, ids, pos, mask)[0].isfinite().all() and took == [None]
+
+
+@pytest.mark.parametrize("masked", [True, False])
+def test_captured_prompts_keep_the_padding(masked):
+    """A captured call serves every later batch of its shape, by the mask that it is given then."""
+    lm = _model(4, 101)
+    ids, pos, mask = _batch([20, 33, 70], 70)
+    sid, sampling = torch.arange(3, device="cuda"), torch.ones(3, 3, device="cuda")
+    args = (ids, mask if masked else None, pos, sid, sampling)
+    lm.model.packed_prompts = lambda *a: None
+    side = torch.cuda.Stream()
+    with torch.inference_mode():
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            lm.context_encoding_model(*args)
+        torch.cuda.current_stream().wait_stream(side)
+        del lm.model.packed_prompts
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            tokens, logits = lm.context_encoding_model(*args)
+        for lengths in ([20, 33, 70], [70, 1, 5], [2, 69, 64]):
+            new = _batch(lengths if masked else [70] * 3, 70)
+            ids.copy_(new[0].flip(0))
+            pos.copy_(new[1])
+            mask.copy_(new[2])
+            lm.model.packed_prompts = lambda *a: None
+            want = lm.context_encoding_model(*args)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(tokens, want[0]) and torch.equal(logits, want[1])
