@@ -436,6 +436,23 @@ DELTA_CHUNK_MIN_TOKENS = 64
 # 4031 tokens of 16 heads of 128 369, 347, 347, 346, 347, of 60000 5100, 5058, 4953, 4952, 4957;
 # 13 of 1000 884, 822, 779, 779, 778; 64 of 200 of 32 heads 4350, 2618, 1898, 1650, 1651.
 DELTA_CHUNK_WORKSPACE = 1 << 30
+# and where there is no room for that, or a capture's pool would hold it for good
+DELTA_CHUNK_LEAST = 128 << 20
+
+
+def _delta_workspace(chunks: int, floats: int, device) -> torch.Tensor:
+    """Room for the operands of up to that many chunks, of so many floats each, and of one at least."""
+    def room(limit):
+        return torch.empty(max(1, min(chunks, limit // (4 * floats))) * floats, dtype=torch.float32,
+                           device=device)
+
+    least = min(DELTA_CHUNK_LEAST, DELTA_CHUNK_WORKSPACE)
+    if not torch.cuda.is_current_stream_capturing():
+        try:
+            return room(DELTA_CHUNK_WORKSPACE)
+        except torch.cuda.OutOfMemoryError:
+            pass
+    return room(least)
 
 
 def gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps: float,
@@ -466,8 +483,7 @@ def gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps: float,
         if one:
             pass                                   # one launch, nothing in between
         elif wide and S >= DELTA_CHUNK_MIN_TOKENS and vdim % 16 == 0:
-            span = max(1, min(-(-S // 16), DELTA_CHUNK_WORKSPACE // (4 * B * H * unit)))
-            ws = torch.empty(span * B * H * unit, dtype=torch.float32, device=qkv.device)
+            ws = _delta_workspace(-(-S // 16), B * H * unit, qkv.device)
         else:
             prep = torch.empty(B, S, PS, dtype=torch.float32, device=qkv.device)
         _check(lib.nx_gated_delta(

@@ -357,3 +357,38 @@ def test_gated_norm_in_pieces(Dv, dtype):
         # the same value but for the order of a head's squares: one rounding of the result
         tol = 2.0 ** -8 if dtype is BF else 2.0 ** -20
         assert ((res[0] - res[1]).abs() <= tol * res[1].abs()).all()
+
+
+def test_delta_rule_where_memory_is_short(monkeypatch):
+    """Operands of fewer chunks at a time where there is no room for all, and in a capture: the same
+    to the bit."""
+    B, S, H, D = 16, 400, 16, 128                      # 220 MB of operands
+    g = torch.Generator(device="cuda").manual_seed(0)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    qkv, beta, a, gate = rnd(B, S, 3 * H * D), rnd(B, S, H), rnd(B, S, H), rnd(B, S, H * D)
+    bias, rate, w, first = rnd(H), rnd(H), rnd(D), rnd(B, H, D, D)
+    step = seqmix.StepLayout(torch.arange(S, device="cuda").repeat(B, 1), torch.arange(B, device="cuda"))
+    sizes, room = [], seqmix._delta_workspace
+    monkeypatch.setattr(seqmix, "_delta_workspace", lambda *x: sizes.append(room(*x)) or sizes[-1])
+
+    def run():
+        state = first.clone()
+        out = seqmix.gated_delta_rule(qkv, beta, a, bias, rate, gate, w, 1e-5, state, step, H, D, D)
+        return out.cpu(), state.cpu(), sizes.pop().numel() * 4
+
+    want = run()
+    empty = torch.empty
+
+    def short(*shape, **kw):
+        if torch.Size(shape).numel() > 200 << 18:
+            raise torch.cuda.OutOfMemoryError
+        return empty(*shape, **kw)
+
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", short)
+        got = run()
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    captured = run()
+    assert want[2] > 200 << 20 and got[2] == captured[2] <= 128 << 20
+    for other in (got, captured):
+        assert torch.equal(other[0], want[0]) and torch.equal(other[1], want[1])
