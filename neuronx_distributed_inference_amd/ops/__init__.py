@@ -921,7 +921,7 @@ def router_choice(x: torch.Tensor, weight: torch.Tensor, top_k: int, act_sigmoid
     if (x.dim() == 2 and 0 < x.shape[1] and x.shape[1] % 8 == 0 and weight.dtype == torch.float32
             and top_k <= weight.shape[0] <= (8 if x.shape[0] >= 512 else 16)
             and x.dtype in (torch.bfloat16, torch.float16, torch.float32)
-            and x.is_contiguous() and weight.is_contiguous()
+            and x.is_contiguous() and weight.is_contiguous() and weight.device == x.device
             and (x.data_ptr() | weight.data_ptr()) % 16 == 0):
         vals = torch.empty(x.shape[0], top_k, dtype=torch.float32, device=x.device)
         idx = torch.empty(x.shape[0], top_k, dtype=torch.long, device=x.device)

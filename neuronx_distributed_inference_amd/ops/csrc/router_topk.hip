@@ -220,6 +220,8 @@ void router_few(torch::Tensor vals, torch::Tensor idx, torch::Tensor x, torch::T
                 x.size(1) > 0, "router_few: shapes");
     const int rows = x.size(0), E = w.size(0), K = x.size(1);
     TORCH_CHECK(E >= top_k && E <= 16 && top_k >= 1 && top_k <= KMAX, "router_few: up to 16 experts");
+    TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.device() == w.device() && vals.device() == x.device() &&
+                idx.device() == x.device(), "router_few: tensors of one GPU");
     TORCH_CHECK(x.is_contiguous() && w.is_contiguous() && w.scalar_type() == at::ScalarType::Float &&
                 ((size_t)x.data_ptr() | (size_t)w.data_ptr()) % 16 == 0, "router_few: layout");
     TORCH_CHECK(vals.numel() == rows * top_k && idx.numel() == rows * top_k && vals.is_contiguous() &&

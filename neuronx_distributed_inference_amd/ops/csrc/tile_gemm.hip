@@ -551,6 +551,7 @@ namespace {
 // rows of x may lie further apart than they are long (columns of a wider tensor)
 void tg_operands(const torch::Tensor& x, const torch::Tensor& w) {
     TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1), "tile_gemm: shapes");
+    TORCH_CHECK(x.is_cuda() && w.device() == x.device(), "tile_gemm: operands of one GPU");
     TORCH_CHECK(x.stride(1) == 1 && (x.size(0) < 2 || (x.stride(0) >= x.size(1) &&
                 x.stride(0) % 8 == 0 && x.stride(0) < (1L << 20))) && w.is_contiguous() &&
                 x.scalar_type() == w.scalar_type(), "tile_gemm: rows of one type");
@@ -681,7 +682,8 @@ torch::Tensor shares_gemm(const torch::Tensor& o, const torch::Tensor& ml, long 
     const long heads = ml.numel() / (2 * n);
     const int HD = (int)(a.K / heads);
     TORCH_CHECK(o.numel() == n * a.K && heads * HD == a.K && HD % 4 == 0, "shares_gemm: shares");
-    TORCH_CHECK(w.is_contiguous() && (size_t)w.data_ptr() % 16 == 0, "shares_gemm: weight");
+    TORCH_CHECK(w.is_contiguous() && (size_t)w.data_ptr() % 16 == 0 && w.device() == o.device(),
+                "shares_gemm: weight");
     const TgPlan plan = tg_plan(1, a.N, a.K, false, false);
     TORCH_CHECK(plan.splits > 0, "shares_gemm: shape not taken");
     a.splits = plan.splits;

@@ -1038,3 +1038,17 @@ def test_router_of_few_experts(T, E, k, K, dtype):
     got = ops.router_choice(x, w, k, False, False, True)
     ref = ops.router_topk(torch.nn.functional.linear(x.float(), w), k, False, False, True)
     assert torch.equal(got[1][:1], ref[1][:1])
+
+
+def test_weights_in_host_memory_are_refused():
+    x, w = torch.zeros(2, 512, device="cuda"), torch.zeros(8, 512)
+    with pytest.raises(RuntimeError):
+        ops.router_choice(x, w, 2, False, False, True)
+    x, w = x.bfloat16(), torch.zeros(256, 512, dtype=torch.bfloat16)
+    for call in (lambda: ops.linear_parts(x, w), lambda: ops.linear_silu_mul(x, w)):
+        with pytest.raises(RuntimeError):
+            call()
+    q, cache = x[:1].view(1, 8, 1, 64), torch.zeros(1, 2, 600, 64, dtype=torch.bfloat16, device="cuda")
+    pos = torch.tensor([[500]], device="cuda")
+    with pytest.raises(RuntimeError):
+        ops.attention_decode_product(q, cache, cache, pos, None, 1.0, 0, w)
