@@ -99,7 +99,7 @@ void router_topk(torch::Tensor vals, torch::Tensor idx, torch::Tensor logits,
                  long top_k, long act_sigmoid, long pre_softmax,
                  long normalize);
 bool lt_available();
-void lt_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
+bool lt_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias, bool timed);
 void flash_prefill_packed(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
                           torch::Tensor v_cache, torch::Tensor seq_ids, torch::Tensor starts,

@@ -118,12 +118,12 @@ void build_descs(Descs& ds, int64_t M, int64_t N, int64_t K, hipDataType dt,
     LT_CHECK(hipblasLtMatrixLayoutCreate(&ds.d, dt, N, M, N));
 }
 
-void enqueue(const Descs& ds, const hipblasLtMatmulAlgo_t* algo,
-             const void* w, const void* x, void* y, hipStream_t stream) {
+hipblasStatus_t enqueue(const Descs& ds, const hipblasLtMatmulAlgo_t* algo,
+                        const void* w, const void* x, void* y, hipStream_t stream) {
     float alpha = 1.0f, beta = 0.0f;
-    LT_CHECK(hipblasLtMatmul(ctx().handle, ds.op, &alpha, w, ds.a, x, ds.b,
-                             &beta, y, ds.d, y, ds.d, algo, ctx().workspace,
-                             kWorkspaceBytes, stream));
+    return hipblasLtMatmul(ctx().handle, ds.op, &alpha, w, ds.a, x, ds.b,
+                           &beta, y, ds.d, y, ds.d, algo, ctx().workspace,
+                           kWorkspaceBytes, stream);
 }
 
 std::tuple<int64_t, int64_t, int64_t, int, int> make_key(
@@ -221,8 +221,9 @@ bool lt_available() {
 // every bucket shape first).
 // `timed` false: the library's own first choice for the shape instead of the timed one. Prompts
 // without their padding have another number of rows each time: a search takes 25 to 80 ms, the
-// question 0.1.
-void lt_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
+// question 0.1. What does not run is passed over for the library's next; false, with nothing done,
+// where it has none that does. A choice is kept once it has run.
+bool lt_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias_opt, bool timed) {
     auto& c = ctx();
     TORCH_CHECK(!c.disabled, "hipblaslt unavailable");
@@ -248,13 +249,20 @@ void lt_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
     }
     Descs ds;
     build_descs(ds, M, N, K, dt, has_bias ? bias : nullptr);
+    auto run = [&]() { return enqueue(ds, &algo, w.data_ptr(), x.data_ptr(), y.data_ptr(), stream); };
     if (!hit && !timed) {
         std::vector<hipblasLtMatmulHeuristicResult_t> results;
-        TORCH_CHECK(ask(ds, 1, results) > 0, "lt_linear: no hipblaslt algo for ", M, "x", N, "x", K);
-        algo = results[0].algo;
+        int found = ask(ds, 1, results);
+        for (int at = 0;; ++at) {
+            if (at == 1) found = ask(ds, 16, results);       // the first of them is known to fail
+            if (at >= found) return false;
+            algo = results[at].algo;
+            if (results[at].state == HIPBLAS_STATUS_SUCCESS && run() == HIPBLAS_STATUS_SUCCESS) break;
+        }
         std::lock_guard<std::mutex> lock(c.mu);
         if (c.first.size() >= kMaxFirst) c.first.clear();
         c.first[key] = algo;
+        return true;
     } else if (!hit) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         hipStreamIsCapturing(stream, &cap);
@@ -268,7 +276,8 @@ void lt_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w,
         std::lock_guard<std::mutex> lock(c.mu);
         algo = c.algos[key];
     }
-    enqueue(ds, &algo, w.data_ptr(), x.data_ptr(), y.data_ptr(), stream);
+    LT_CHECK(run());
+    return true;
 }
 
 // Pre-tune one shape with scratch tensors (called from python warmup).

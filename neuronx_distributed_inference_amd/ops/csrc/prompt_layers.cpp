@@ -15,7 +15,7 @@ void qkv_rope_update(torch::Tensor q_out, torch::Tensor qkv, torch::Tensor cosb,
                      torch::Tensor seq_ids, long Hq, long Hkv, c10::optional<torch::Tensor> q_norm,
                      c10::optional<torch::Tensor> k_norm, double eps,
                      c10::optional<torch::Tensor> slots);
-void lt_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
+bool lt_linear(torch::Tensor y, torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias,
                bool timed);
 void silu_mul_fused(torch::Tensor out, torch::Tensor gate_up);
 void flash_prefill_packed(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
@@ -34,11 +34,7 @@ torch::Tensor product(const torch::Tensor& x, const torch::Tensor& w, bool glu) 
     if (tile_gemm_splits(rows, N, x.size(1), glu, glu))
         return tile_gemm(x, w, c10::nullopt, 0, !glu, glu);
     torch::Tensor y = torch::empty({rows, N}, x.options());
-    try {
-        lt_linear(y, x, w, c10::nullopt, false);
-    } catch (const c10::Error&) {                // a shape that it has no algorithm for
-        y = at::linear(x, w);
-    }
+    if (!lt_linear(y, x, w, c10::nullopt, false)) y = at::linear(x, w);   // no algorithm for the shape
     if (!glu) return y;
     torch::Tensor o = torch::empty({rows, N / 2}, x.options());
     silu_mul_fused(o, y);

@@ -147,3 +147,19 @@ def test_captured_prompts_keep_the_padding(masked):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(tokens, want[0]) and torch.equal(logits, want[1])
+
+
+def test_products_by_the_librarys_first_choice():
+    """What packed prompts take: asked for once a shape, errors of the operands stay errors."""
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x = torch.randn(700, 320, device="cuda", generator=g).bfloat16()
+    w = torch.randn(96, 320, device="cuda", generator=g).bfloat16()
+    want = x.double() @ w.double().t()
+    slack = 2.0 ** -8 * want.abs() + 320 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    for _ in range(3):
+        y = torch.empty(700, 96, dtype=torch.bfloat16, device="cuda")
+        assert ops._C.lt_linear(y, x, w, None, False) is True
+        assert ((y.double() - want).abs() <= slack).all()
+    for bad in (w[:, :319].contiguous(), w.t()):
+        with pytest.raises(RuntimeError):
+            ops._C.lt_linear(y, x, bad, None, False)
