@@ -566,14 +566,14 @@ def _attention_out(q, token_major):
 
 def attention_decode_product(q, k_cache, v_cache, positions, seq_ids, scale: float, window: int,
                              weight):
-    """attention_decode of one token of one row, q (1, Hq, 1, D), and its product with weight
-    (N, Hq * D), as linear_parts has it; None where that does not serve."""
+    """attention_decode of one token of one row, q (1, Hq, 1, D) at positions (1, 1), and its product
+    with weight (N, Hq * D), as linear_parts has it; None where that does not serve."""
     D = q.shape[3]
     if not (q.is_cuda and D in (64, 128) and q.dtype in (torch.bfloat16, torch.float16)
             and isinstance(k_cache, torch.Tensor) and k_cache.dtype == v_cache.dtype
             and k_cache.dtype in (q.dtype, torch.float8_e4m3fn)
             and q.is_contiguous() and k_cache.is_contiguous() and v_cache.is_contiguous()
-            and positions.numel() == 1 and weight.shape[1] == q.shape[1] * D
+            and positions.dim() == 2 and positions.numel() == 1 and weight.shape[1] == q.shape[1] * D
             and _tile_takes(q.view(1, -1), weight)):
         return None
     if seq_ids is None:

@@ -89,3 +89,5 @@ def test_decode_and_its_product(Hq, Hkv, D, N, L, pos, f8, dtype):
     y = ops.attention_decode_product(q, kc, vc, p, sid, D ** -0.5, 0, w)
     assert y.float().isnan().any()
     assert ops.attention_decode_product(q.float(), kc, vc, p, sid, 1.0, 0, w) is None
+    # (1,) is a length and not a position
+    assert ops.attention_decode_product(q, kc, vc, p.view(1), sid, 1.0, 0, w) is None
