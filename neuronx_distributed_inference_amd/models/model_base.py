@@ -33,6 +33,7 @@ from neuronx_distributed_inference_amd.modules.attention.attention_base import (
     coarse_rows,
 )
 from neuronx_distributed_inference_amd.modules.fused_layer import (
+    dense_layer,
     fusable,
     packed_layers,
     prompt_operands,
@@ -247,8 +248,7 @@ class DecoderModel(nn.Module):
                 and ops.step_start_takes(input_ids, position_ids, seq_ids, table,
                                          rot._cos_cached)):
             return False
-        like = table.new_empty(*input_ids.shape, table.shape[1])
-        return fusable(layers, self.norm, like, attention_mask, phase)
+        return fusable(layers, self.norm, table[:1], attention_mask, phase)
 
     def _fused_start(self, layers, input_ids, position_ids, seq_ids, attention_mask, phase):
         """What ops.step_start makes of the step's tokens, see _starts_fused; else None."""
@@ -277,12 +277,12 @@ class DecoderModel(nn.Module):
                 or not self._may_fuse() or seq_ids is None or seq_ids.numel() != B):
             return None
         layers = [layer for _, layer in self.layer_runs()]
-        if not self._starts_fused(layers, input_ids, position_ids, seq_ids, None, PHASE_CTE):
+        # (one layer that is of another kind spares the questions, which forward asks again)
+        if not (layers and dense_layer(layers[0]) and self._starts_fused(
+                layers, input_ids, position_ids, seq_ids, None, PHASE_CTE)):
             return None
         rot, norm, table = self.rotary, layers[0].input_layernorm, self.embed_tokens.weight
-        like = table.new_empty(*input_ids.shape, table.shape[1])
-        operands = prompt_operands(layers, self.norm, like, like, rot._cos_cached, self.kv_mgr,
-                                    seq_ids)
+        operands = prompt_operands(layers, self.norm, table[:1], rot._cos_cached, self.kv_mgr, seq_ids)
         if operands is None:
             return None
         lengths = [S] * B if lengths is None else lengths.get()

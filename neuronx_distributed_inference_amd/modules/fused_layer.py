@@ -91,7 +91,16 @@ def _feed_forward(mlp, x: torch.Tensor) -> torch.Tensor:
 PROMPT_ROWS = ops.TILE_ROWS
 
 
-def prompt_operands(layers, final_norm, h, x, cos, kv_mgr, seq_ids):
+def dense_layer(layer) -> bool:
+    """Whether the layer's modules are of the kinds that :func:`prompt_operands` takes."""
+    if getattr(type(layer), "fused_forward", None) is not type(layer).forward:
+        return False
+    attn, mlp = layer.fused_parts()
+    return (isinstance(attn, AttentionBase) and attn.q_norm is None and attn.k_norm is None
+            and type(mlp) is GatedMLP)
+
+
+def prompt_operands(layers, final_norm, x, cos, kv_mgr, seq_ids):
     """What csrc/prompt_layers.cpp takes of dense layers without q/k norms, None for others."""
     if not ops.tiles_enabled():
         return None
@@ -118,7 +127,7 @@ def _short_prompt(layers, final_norm, h, x, cos, sin, kv_mgr, position_ids, seq_
     its launches made by one native call (csrc/prompt_layers.cpp); None where that does not serve."""
     if h.numel() > PROMPT_ROWS * h.shape[-1] or not (cos.is_contiguous() and sin.is_contiguous()):
         return None
-    operands = prompt_operands(layers, final_norm, h, x, cos, kv_mgr, seq_ids)
+    operands = prompt_operands(layers, final_norm, x, cos, kv_mgr, seq_ids)
     if operands is None:
         return None
     return ops._require_ext("prompt_layers").prompt_layers(

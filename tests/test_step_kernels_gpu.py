@@ -1052,3 +1052,18 @@ def test_weights_in_host_memory_are_refused():
     pos = torch.tensor([[500]], device="cuda")
     with pytest.raises(RuntimeError):
         ops.attention_decode_product(q, cache, cache, pos, None, 1.0, 0, w)
+
+
+@pytest.mark.parametrize("moe", [False, True])
+def test_layers_are_asked_once_a_prompt(moe, monkeypatch):
+    """Whether they run fused, also where they do not run without the prompt's padding."""
+    from neuronx_distributed_inference_amd.models import model_base
+
+    lm = _small_llama("bfloat16", moe=moe)
+    lm.enable_submodels()
+    ids = torch.randint(0, 512, (2, 70), device="cuda")
+    asked, inner = [], model_base.fusable
+    monkeypatch.setattr(model_base, "fusable", lambda *a: asked.append(inner(*a)) or asked[-1])
+    with torch.inference_mode():
+        lm(input_ids=ids, position_ids=torch.arange(70, device="cuda").repeat(2, 1))
+    assert asked == [True]
