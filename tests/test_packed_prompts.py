@@ -49,12 +49,12 @@ def _batch(lengths, S):
     return ids.cuda(), pos.cuda(), mask.cuda()
 
 
-def _run(lm, ids, pos, mask):
+def _run(lm, ids, pos, mask, seq_ids=None):
     B = ids.shape[0]
     lm.reset()
     with torch.inference_mode():
         out = lm(input_ids=ids, attention_mask=mask, position_ids=pos,
-                 seq_ids=torch.arange(B, device="cuda"))
+                 seq_ids=torch.arange(B, device="cuda") if seq_ids is None else seq_ids)
     kv = [t.data.clone() for i in range(2) for t in lm.model.kv_mgr.get_cache(i)]
     return out.logits.float(), out.tokens, kv
 
@@ -81,6 +81,43 @@ def test_packed_prompts(lengths, S, capacity, window, dtype):
     for a, b in zip(got[2], want[2]):
         assert (a.float() - b.float()).norm() <= tol * b.float().norm()
         assert ((a == 0).all(-1) == (b == 0).all(-1)).all()       # the same rows are written
+
+
+@pytest.mark.parametrize("lengths,S,seq_ids,batch", [
+    ([93], 93, [2], 4), ([31, 1, 70], 70, [4, 0, 2], 5), ([64, 33], 64, [1, 0], 2), ([300, 350, 9], 350, [6, 1, 3], 8)])
+@pytest.mark.parametrize("kind", [torch.int64, torch.int32])
+@pytest.mark.parametrize("masked", [True, False])
+def test_packed_prompts_of_other_cache_rows(lengths, S, seq_ids, batch, kind, masked):
+    """A batch smaller than the model's, in cache rows that are not the prompts' own numbers."""
+    lm = _model(batch, S + 7)
+    if not masked:
+        lengths = [S] * len(lengths)
+    ids, pos, mask = _batch(lengths, S)
+    seq = torch.tensor(seq_ids, device="cuda", dtype=kind)
+    noise = torch.Generator(device="cuda").manual_seed(3)
+    caches = [t.data for i in range(2) for t in lm.model.kv_mgr.get_cache(i)]
+    lm.reset = lambda: [c.normal_(0, 1, generator=noise.manual_seed(3)) for c in caches]
+    lm.kv_cache_populated = False
+    took = []
+    inner = lm.model.packed_prompts
+    lm.model.packed_prompts = lambda *a: took.append(inner(*a)) or took[-1]
+    got = _run(lm, ids, pos, mask if masked else None, seq)
+    assert took[0] is not None
+    lm.kv_cache_populated = False
+    lm.model.packed_prompts = lambda *a: None
+    want = _run(lm, ids, pos, mask if masked else None, seq)
+    assert got[0].shape == want[0].shape and (got[0] - want[0]).norm() <= 0.03 * want[0].norm()
+    lm.reset()
+    for a, b, before in zip(got[2], want[2], caches):
+        own = torch.zeros(a.shape[0], a.shape[2], dtype=torch.bool)
+        for row, n in zip(seq_ids, lengths):
+            own[row, :n] = True
+        own = own.cuda()
+        a, b, before = (t.transpose(1, 2) for t in (a, b, before))
+        assert torch.equal(a[~own], before[~own])
+        a, b = a[own].float().flatten(1), b[own].float().flatten(1)
+        assert ((a - b).norm(dim=1) <= 0.03 * b.norm(dim=1)).all()
+        assert (a != before[own].float().flatten(1)).any(dim=1).all()
 
 
 @pytest.mark.parametrize("kind", [torch.int64, torch.int32, torch.bool])
