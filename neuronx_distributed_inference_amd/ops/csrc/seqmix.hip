@@ -5962,12 +5962,13 @@ int nx_paged_attn(const void* q, long qstride, const void* kc, long ktok, long k
             f.kn = (const bf16*)kn; f.vn = (const bf16*)vn; f.slots = slots; f.nslots = nslots;
             f.kw = (bf16*)kc; f.vw = (bf16*)vc; f.knstride = knstride; f.vnstride = vnstride;
             const int nc = rp < 16 ? rp : 16;
-            // Through LDS where the keys' bytes bound it: many rows of 4 steps of a wave and more.
-            // Few rows, or short ones, wait a little longer for their first keys that way. 16 heads of
-            // 128 on 4 KV heads, half to full caches of 384 / 768 / 1472 keys, straight -> staged:
-            // 16 rows 9.6 -> 10.4, 14.7 -> 15.0, 21.4 -> 19.6 us; 32 10.0 -> 11.1, 17.7 -> 16.0,
-            // 23.7 -> 22.0; 48 10.9 -> 11.6, 19.0 -> 17.1, 26.5 -> 24.5; 100 rows of 1000, 8 heads of 64,
-            // 50.6 -> 42.3.
+            // Through LDS where the keys' bytes bound it: many rows of a cache of 4 steps of a wave and
+            // more. The host knows the cache and not the rows, and rows that are short in it lose
+            // nothing. 16 heads of 128 on 4 KV heads, half to full caches of 384 / 768 / 1472 keys,
+            // straight -> staged, us: 16 rows 10.2 -> 10.1, 14.9 -> 14.5, 21.9 -> 21.9; 32 10.5 -> 10.7,
+            // 15.6 -> 15.9, 28.3 -> 25.1; 48 11.8 -> 11.9, 19.3 -> 17.6, 30.8 -> 27.8. 48 rows of 16 to 64 /
+            // 64 to 200 / 192 to 384 keys in a cache of 4096 6.1 -> 6.2, 9.6 -> 8.7, 13.4 -> 11.9; 100 rows
+            // of 1000, 8 heads of 64, 50 -> 39.6.
             const long seen = (long)max_blocks * bsz, span = (long)window + keep;
             const bool staged = (long)B * G * ((rp + 15) / 16) >= 96 && (seen < span ? seen : span) >= 512;
 #define WDK(DD) (staged ? (kn ? window_decode_kernel<DD, true, true> : window_decode_kernel<DD, true, false>) \

@@ -485,7 +485,7 @@ TgPlan tg_plan(long M, long N, long K, bool glu, bool whole) {
     const long wides = (N + 255) / 256, rounds = (wides + 255) / 256;
     const long tiles128 = (N + 127) / 128;
     const bool filled = whole && K <= 4096 && tiles128 <= 256 && tiles128 * (256 / tiles128) >= 180;
-    const bool wide = wides >= 192 && wides * 100 >= rounds * 256 * 85;
+    const bool wide = wides * 100 >= rounds * 256 * 85;
     if (M <= 16) p = narrow ? TgPlan{T16N, 16, 64, 0} : TgPlan{T16, 16, 128, 0};
     else if (M <= 32) p = narrow ? TgPlan{T32N, 32, 64, 0} : TgPlan{T32, 32, 128, 0};
     else if (M <= 64 && wide) p = {T64W, 64, 256, 0};
