@@ -248,7 +248,8 @@ class DecoderModel(nn.Module):
                 and ops.step_start_takes(input_ids, position_ids, seq_ids, table,
                                          rot._cos_cached)):
             return False
-        return fusable(layers, self.norm, table[:1], attention_mask, phase)
+        # (of the hidden states it looks at type, width and place)
+        return fusable(layers, self.norm, table, attention_mask, phase)
 
     def _fused_start(self, layers, input_ids, position_ids, seq_ids, attention_mask, phase):
         """What ops.step_start makes of the step's tokens, see _starts_fused; else None."""
@@ -282,7 +283,7 @@ class DecoderModel(nn.Module):
                 layers, input_ids, position_ids, seq_ids, None, PHASE_CTE)):
             return None
         rot, norm, table = self.rotary, layers[0].input_layernorm, self.embed_tokens.weight
-        operands = prompt_operands(layers, self.norm, table[:1], rot._cos_cached, self.kv_mgr, seq_ids)
+        operands = prompt_operands(layers, self.norm, table, rot._cos_cached, self.kv_mgr, seq_ids)
         if operands is None:
             return None
         lengths = [S] * B if lengths is None else lengths.get()

@@ -107,11 +107,11 @@ def prompt_operands(layers, final_norm, x, cos, kv_mgr, seq_ids):
     weights, sizes, numbers = [], [], []
     for layer, after in zip(layers, layers[1:] + [None]):
         attn, mlp = layer.fused_parts()
-        if _own_attend(attn):
+        if _own_attend(attn) or attn.q_norm is not None or attn.k_norm is not None:
             return None
         qkv = attn.qkv_proj
         rows = attn.prompt_front(x, cos, kv_mgr, PHASE_CTE, seq_ids)
-        if (rows is None or not attn.use_rope or attn.sinks is not None or attn._front_norms(x)
+        if (rows is None or not attn.use_rope or attn.sinks is not None
                 or _hooked(qkv) or not plain_linear(qkv.qkv, x) or not _plain_mlp(mlp, x)):
             return None
         norm, following = layer.post_attention_layernorm, after.input_layernorm if after else final_norm
