@@ -29,6 +29,14 @@
 //     16 B are XOR-swizzled on the source side so that neither the row reads of K nor the
 //     transposing reads of V meet in a bank.
 //
+//   * Over pages that hold whole tiles (a multiple of 64 rows) a tile is one page number and one
+//     address, kept in scalar registers; a tile without a page is left out. Page numbers, divisions
+//     and marks for each key row took as many vector instructions as the exponentials: 512 tokens
+//     over 3500 in pages of 64 90 -> 74 us, 64 tokens 24 -> 18. Other page sizes keep the row form.
+//   * Over a cache a wave has priority while it multiplies with V: its SIMD's other wave then
+//     computes exponentials beside it (74.6 -> 72.4 us; 200 tokens over 2000, heads of 64, 29.6 ->
+//     27.7). Prompts from an empty cache gain at 8192 tokens what they lose at 2048 (2 %): without.
+//
 // Rows with few tiles to share (short chunks over a long cache) are split over the keys as
 // well: fp32 partial sums per split and a small combining kernel.
 //
@@ -38,8 +46,8 @@
 //                                     matrix pipe, the rest exponentials it does not hide)
 //   prompt of 2048, head size 128/64  179 -> 54 us / 145 -> 39 us
 //   prompt of 512 / 128               40 -> 16 us / 16 -> 9 us
-//   512 tokens over 4000, linear/paged 1574 -> 81 us / 1749 -> 98 us
-//   64 tokens over 4000, linear       237 -> 34 us
+//   512 tokens over 4000, linear/paged 1574 -> 72 us / 1749 -> 72 us (pages of 16 or 32: 87)
+//   64 tokens over 4000, linear       237 -> 34 us, in pages 24 -> 18
 //   32 rows of 6 tokens over 2000     351 -> 50 us (a verification step)
 //   1 row of 2 tokens over 2000       28 -> 18 us
 // No size was found at which several tokens are better off one by one. Error against 64 bits
@@ -138,13 +146,17 @@ struct FaArgs {
     int nsplit, nqt, clamp_rows;      // clamp_rows: a negative seq_id reads row 0 (else: no keys)
 };
 
-template <typename T, int D, bool PAGED, bool HILO>
+// where the keys are: a row of a linear cache, pages, or pages that hold whole tiles
+enum FaKeys { ROWS, PAGES, TILE_PAGES };
+
+template <typename T, int D, int KEYS, bool HILO>
 __global__ __launch_bounds__(256, 2) void flash_kernel(
     T* __restrict__ out, const T* __restrict__ q, const T* __restrict__ k,
     const T* __restrict__ v, const FaArgs a) {
     using FT = FaTraits<T>;
     using vec8 = typename FT::vec8;
     using vec4 = typename FT::vec4;
+    constexpr bool PAGED = KEYS == PAGES;  // a page number for each key row
     constexpr int ROWB = D * 2;            // bytes of a key row
     constexpr int SLOTS = ROWB / 16;       // 16-byte slots of a row: 16 or 8
     constexpr int RPI = 64 / SLOTS;        // rows that one wave-wide load stages: 4 or 8
@@ -260,12 +272,16 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
     // ---- staging: this lane's rows and source slots ----
     const int st_row = wid * (KT / 4) + lane / SLOTS;  // + i * RPI
     const int st_p = lane % SLOTS;
-    const long lin = PAGED ? 0 : ((long)max(row, 0) * a.Hkv + hkv) * (long)a.Smax * D;
+    const long lin = KEYS != ROWS ? 0 : ((long)max(row, 0) * a.Hkv + hkv) * (long)a.Smax * D;
     auto swz_k = [](int r) { return D == 128 ? (r & 15) : ((r >> 1) & 7); };
     auto swz_v = [](int r) { return D == 128 ? ((r & 3) << 2) : (((r >> 1) & 1) << 2); };
     const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
     int blk[NLD];                                      // paged: the next tile's page numbers
+    // of whole tiles: the pages of the tile at hand, of the one on its way and of the one after
+    const int* pages = KEYS == TILE_PAGES ? a.block_table + (long)b * a.max_blocks : nullptr;
+    int page = 0, page_now = 0, page_next = 0;
     auto load_blocks = [&](int t) {
+        if constexpr (KEYS == TILE_PAGES) page_next = pages[t * KT / a.block_size];
         if constexpr (PAGED) {
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
@@ -277,12 +293,17 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
     auto stage = [&](int t, int buf) {
         const unsigned kd = lds0 + buf * 2 * TILE_B + wid * (TILE_B / 4);
         const unsigned vd = kd + TILE_B;
+        long first = 0;                                // of the tile's keys in its page
+        if constexpr (KEYS == TILE_PAGES)
+            first = ((long)max(page_next, 0) * a.block_size + t * KT % a.block_size) * a.Hkv + hkv;
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
             const int r = st_row + i * RPI;
             const int key = min(t * KT + r, bmax);
             long off;
-            if constexpr (PAGED)
+            if constexpr (KEYS == TILE_PAGES)
+                off = (first + (long)(key - t * KT) * a.Hkv) * D;
+            else if constexpr (PAGED)
                 off = (((long)max(blk[i], 0) * a.block_size + key % a.block_size) * a.Hkv + hkv) * D;
             else
                 off = lin + (long)key * D;
@@ -324,6 +345,7 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
     }
     if (t_lo < t_hi) {
         load_blocks(t_lo);
+        page_now = page_next;
         stage(t_lo, 0);
         if (t_lo + 1 < t_hi) load_blocks(t_lo + 1);
     }
@@ -343,12 +365,15 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
         }
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
+        page = page_now;
         if (t + 1 < t_hi) {
+            page_now = page_next;
             stage(t + 1, buf ^ 1);
             if (t + 2 < t_hi) load_blocks(t + 2);
         }
         const int k0 = t * KT;
         if (k0 > wmax || k0 + KT <= w_lo) continue;     // nothing here for this wave
+        if (KEYS == TILE_PAGES && page < 0) continue;   // nor keys that anyone sees
         const char* kb = smem + buf * 2 * TILE_B;
         const char* vb = kb + TILE_B;
 
@@ -425,6 +450,9 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
                 l += e;
                 s[n][r] = e;
             }
+        // (this wave before the other of its SIMD: that one's exponentials are to run beside these
+        // products, and not both waves' products in turns)
+        if constexpr (HILO) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
             vec8 p[NP];
@@ -465,6 +493,7 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
             __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
         }
         __builtin_amdgcn_sched_group_barrier(0x008, 4 * NP, 1);
+        if constexpr (HILO) __builtin_amdgcn_s_setprio(0);
     }
 
     // ---- epilogue: rows of 4 channels from 8*(r>>2) + 4*half ----
@@ -488,7 +517,7 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
             attend_row<D>(q + at * D, k, v, max(__shfl(key_lo, own, WAVE_SIZE), t_lo * KT),
                           min(__shfl(qpos, own, WAVE_SIZE) + 1, t_hi * KT), c0,
                           [&](int key) -> long {
-                if constexpr (PAGED) {
+                if constexpr (KEYS != ROWS) {
                     const int p = a.block_table[(long)b * a.max_blocks + key / a.block_size];
                     return p < 0 ? -1 : (((long)p * a.block_size + key % a.block_size) * a.Hkv + hkv) * D;
                 }
@@ -593,18 +622,18 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(T* __restrict__ out,
     for (int j = 0; j < PER; ++j) po[j] = VecTraits<T>::from_float(acc[j] * inv);
 }
 
-template <typename T, int D, bool PAGED, bool HILO>
+template <typename T, int D, int KEYS, bool HILO>
 void flash_launch(torch::Tensor& out, const torch::Tensor& q, const torch::Tensor& k,
                   const torch::Tensor& v, FaArgs& a, hipStream_t stream) {
     const int gq = a.Hq / a.Hkv;
     a.nqt = (int)(((long)gq * a.S + QROWS - 1) / QROWS);
-    const size_t lds = 4 * KT * D * 2 + 8 * sizeof(int) + (PAGED ? 2 * (KT + 1) * sizeof(int) : 0);
+    const size_t lds = 4 * KT * D * 2 + 8 * sizeof(int) + (KEYS == PAGES ? 2 * (KT + 1) * sizeof(int) : 0);
     // a limit of the function on the device at hand, the same in every call
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_kernel<T, D, PAGED, HILO>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_kernel<T, D, KEYS, HILO>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const long blocks = (long)a.B * a.Hkv * a.nqt * a.nsplit;
     TORCH_CHECK(blocks < (1l << 31), "flash attention: too many query rows");
-    hipLaunchKernelGGL((flash_kernel<T, D, PAGED, HILO>), dim3((unsigned)blocks), dim3(256), lds, stream,
+    hipLaunchKernelGGL((flash_kernel<T, D, KEYS, HILO>), dim3((unsigned)blocks), dim3(256), lds, stream,
                        (T*)out.data_ptr(), (const T*)q.data_ptr(), (const T*)k.data_ptr(),
                        (const T*)v.data_ptr(), a);
     HIP_CHECK_KERNEL();
@@ -655,13 +684,14 @@ void flash_run(torch::Tensor& out, const torch::Tensor& q, const torch::Tensor& 
         a.ml_part = ml_part.data_ptr<float>();
     }
     auto stream = at::hip::getCurrentHIPStream();
-    const bool paged = a.block_table != nullptr;
+    const bool paged = a.block_table != nullptr, tiles = paged && a.block_size % KT == 0;
     const bool extend = a.positions != nullptr;
 #define FA_D(T, D)                                                                        \
     do {                                                                                  \
-        if (paged) flash_launch<T, D, true, true>(out, q, k, v, a, stream);               \
-        else if (extend) flash_launch<T, D, false, true>(out, q, k, v, a, stream);        \
-        else flash_launch<T, D, false, false>(out, q, k, v, a, stream);                   \
+        if (tiles) flash_launch<T, D, TILE_PAGES, true>(out, q, k, v, a, stream);         \
+        else if (paged) flash_launch<T, D, PAGES, true>(out, q, k, v, a, stream);         \
+        else if (extend) flash_launch<T, D, ROWS, true>(out, q, k, v, a, stream);         \
+        else flash_launch<T, D, ROWS, false>(out, q, k, v, a, stream);                    \
     } while (0)
 #define FA_GO(T)                                                                          \
     do {                                                                                  \
