@@ -2364,64 +2364,129 @@ gated_delta_kernel(const float* __restrict__ qkv, long cstride, const float* __r
     }
 }
 
-// ---- the same recurrence in chunks of 16 tokens, matrix cores in 32 bits
+// ---- the same recurrence in blocks of 64 tokens, matrix cores in 32 bits
 // Portions of several tokens: the scan above is a chain of two lane reductions a token (0.32 us,
-// 128 of 256 CUs for one prompt of 16 heads). With Gam_t the product of the decays from the chunk's
-// start to t, Gam_{s,t} that from after s to t, and S0 the state at the start, the chunk is
+// 128 of 256 CUs for one prompt of 16 heads). With Gam_t the product of the decays from the block's
+// start to t, Gam_{s,t} that from after s to t, and S0 the state at the start, the block is
 //   (I + L) U = beta (V - (Gam k) S0),  L_ts = beta_t k_t' diag(Gam_{s,t}) k_s   (s < t)
 //   O = (Gam q) S0 + P U,               P_ts = q_t' diag(Gam_{s,t}) k_s          (s <= t)
-//   S = diag(Gam_16) S0 + sum_s (Gam_{s,16} k_s) u_s'
+//   S = diag(Gam_64) S0 + sum_s (Gam_{s,64} k_s) u_s'
 // All but U, O and S is independent of the state:
-// (1) delta_chunk_kernel, a workgroup per (chunk, head): unit q and k, decays, the products
+// (1) delta_block_kernel, a workgroup of 16 waves per (block, head): unit q and k, decays, the products
 //     (running ones, never a quotient or an exponential of a difference: strong decays go to
-//     zero as they do in the scan), L, P, and W = (I+L)^-1 beta Gam k, U0 = (I+L)^-1 beta V by
-//     forward substitution, a thread per column. It reads the projections itself: no prep pass.
-// (2) delta_chunk_scan_kernel, a workgroup per (row, head, 16 value channels): the chain over
-//     chunks, U = U0 - W S0 and so on, three products of 16x16 and D on 16x16x4 fp32 matrix
+//     zero as they do in the scan), P, and W = (I+L)^-1 beta Gam k, U0 = (I+L)^-1 beta V. L and P in
+//     three steps: 4 tokens among themselves on the vector units, 4 with 4 of the same 16 (12 products
+//     of 4 x 4 in one 4x4x1 matrix instruction) and 16 with 16, with the decays from a group's start
+//     on the one side, to a group's end on the other and of whole groups between them. The inverse by
+//     forward substitution within 16 tokens, a thread a column, and from 16 to 16 by products of what
+//     that leaves: X_i = Y_i - sum_j M_ij X_j, M_ij = (I+L_ii)^-1 L_ij from Y as L_ij from k.
+// (2) delta_block_scan_kernel, a workgroup per (row, head, 16 value channels): the chain over
+//     blocks, U = U0 - W S0 and S, products of 16x16 and D on 16x16x4 fp32 matrix
 //     instructions (the scan's precision; 16-bit parts would need six products). Waves split the
 //     D rows of the state, which stay in registers: the C layout of its update is the B layout
-//     of the next product when the key channels of A are taken in the same order. One LDS
-//     exchange and one barrier a chunk. A fifth wave reads the outputs out, off the chain; a
-//     sixth pulls the operands into L2 eight chunks ahead, the others into registers three ahead.
-// The head is the fastest grid index of (2): the 8 workgroups that read a head's W, q, k share an
-// XCD's L2. Chunks go through a workspace of bounded size, a span of tokens at a time.
-// 4000 tokens of 16 heads of 128: (1) 121 us, bound by its 16 rounds of lane sums and the
-// substitution; (2) 224 us, the chain (0.9 us a chunk; 294 without the sixth wave, 204 with
-// operands that are always hot). Prep pass and scan took 1397 us. fp32 error against 64 bits
-// 3.1e-7 (scan 3.0e-7).
-#define DC_T 16
-#define DC_AHEAD 8     // chunks
+//     of the next product when the key channels of A are taken in the same order. What a block
+//     costs beside its 64 instructions of 32 cycles a wave is the exchange of the waves' sums, in two
+//     halves, each behind products of the other; 16 tokens at a time had it four times as often.
+//     Four waves more only load: the operands (68 KB a block, which a CU takes in no faster than in
+//     1060 cycles) stood in the way of the products in the waves that multiply.
+// (3) delta_block_out_kernel, a workgroup per (block, head): O of the state that the chain left at each
+//     block's start and of U, with the head norm and gate. On the chain it took the state waves'
+//     matrix cores for a third of their time, on half of the CUs.
+// The head is the fastest grid index of (2): the 8 workgroups that read a head's W and k share an
+// XCD's L2. Blocks go through a workspace of bounded size, a span of tokens at a time.
+// 4000 tokens of 16 heads of 128, us: (1) 100, its phases one after the other in 16 waves of a CU; (2)
+// 117, 3600 cycles a block of which the matrix cores have 2050; (3) 59, 173 MB and 17 us of products. In
+// blocks of 16 tokens with the read-out on the chain 125 + 228, and 16 the norm. 64 tokens 37 (29), 256
+// 47 (43), 512 55 (62), 16 rows of 100 113 (140): a few tokens' wait is longer now. Error against 64 bits
+// 4.2e-7 (3.5e-7, the scan 3.0e-7).
+#define DB_T 64
 typedef float dc_f32x4 __attribute__((ext_vector_type(4)));
 
-// floats of one (chunk, head): W 16D | Gam q 16D | (Gam k)' D16 | U0' Dv16 | P 256 | Gam_16 D
-__host__ DEV long dc_unit(int D, int Dv) { return 49L * D + 16L * Dv + 256; }
+
+// floats of one (block, head): -W 64D | Gam q 64D | (Gam k)' 64D | U' 4 x Dv16 | P 10 x 256 | Gam_64 D |
+// the state at its start. W, q, k, P and the state are in pieces of 16 x 16 as a wave holds them: a
+// lane's 4 values of operand A's row lane % 16 (of the state: column), places lane / 16 * 4 on
+__host__ DEV long db_unit(int D, int Dv) { return 193L * D + 64L * Dv + 2560 + (long)D * Dv; }
+
+template <int D> constexpr int db_lds() {        // bytes of delta_block_kernel's LDS
+    return (3 * DB_T * (D + 4) + DB_T * 132 + 21 * D + 4 * 16 * 20 + 4 * 256 + 6 * 16 * 20 + DB_T) * 4;
+}
+
+// e^x, and log(1 + e^x) as max(x, 0) + 2 atanh(z / (2 + z)) with z = e^-|x|, to one or two units of
+// the last place: the decays' error is that of expf and log1pf (3.0e-7 over rates of 1 to 16)
+// in a fifth of their instructions
+DEV float exp_near(float x) {
+    if (!(fabsf(x) < 80.f)) return expf(x);
+    const float y = x * 1.44269502f, r = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269502f, -y));
+    const float e = __builtin_amdgcn_exp2f(y);
+    return fmaf(e, r * 0.693147182f, e);
+}
+DEV float softplus_near(float x) {
+    const float z = exp_near(-fabsf(x)), d = 2.f + z;
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(fmaf(-d, r, 1.f), r, r);
+    const float w = z * r, v = w * w;
+    float p = 1.f / 15.f;
+    p = fmaf(p, v, 1.f / 13.f);
+    p = fmaf(p, v, 1.f / 11.f);
+    p = fmaf(p, v, 1.f / 9.f);
+    p = fmaf(p, v, 1.f / 7.f);
+    p = fmaf(p, v, 1.f / 5.f);
+    p = fmaf(p, v, 1.f / 3.f);
+    const float l = fmaf(p * v, w, w);
+    return fmaxf(x, 0.f) + (l + l);
+}
+
+// 16 values of every lane -> their sums over the wave: lane l has that of value l % 4 + l / 16 * 4 of
+// those with l % 16 < 4
+DEV float wave_sums16(float (&v)[16], int lane) {
+    float x[8], y[4];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v[m]),
+                                                        __builtin_bit_cast(unsigned, v[m + 8]), false, false);
+        x[m] = __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+    }
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, x[m]),
+                                                        __builtin_bit_cast(unsigned, x[m + 4]), false, false);
+        y[m] = part_sum<16>(__builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]));
+    }
+    const int m = lane & 3;
+    return m == 0 ? y[0] : m == 1 ? y[1] : m == 2 ? y[2] : y[3];
+}
+
+template <typename T, int N> struct __attribute__((packed)) DbRow { T v[N]; };      // of any alignment
 
 template <typename T, int D>
-__global__ void __launch_bounds__(256)
-delta_chunk_kernel(const float* __restrict__ qkv, long cstride, const T* __restrict__ beta,
+__global__ void __launch_bounds__(1024)
+delta_block_kernel(const float* __restrict__ qkv, long cstride, const T* __restrict__ beta,
                    long bstride, const T* __restrict__ a, long astride,
                    const float* __restrict__ dt_bias, const float* __restrict__ a_log,
                    const int* __restrict__ seq, const int* __restrict__ nvalid,
-                   float* __restrict__ ws, int t_base, int nchunk, int S, int H, int G, int Dv,
+                   float* __restrict__ ws, int t_base, int nblk, int S, int H, int G, int Dv,
                    int per_head) {
     constexpr int PC = D / 16;                   // channels of a thread
-    constexpr int KS = DC_T + 1, LS = DC_T + 4;   // rows of L in whole float4s
-    __shared__ __attribute__((aligned(16))) float qs[DC_T * D], ks[DC_T * D], ds[DC_T * D];
-    __shared__ float gam[DC_T * D], kh[D * KS], Ps[DC_T * KS], bs[DC_T];
-    __shared__ __attribute__((aligned(16))) float Ls[DC_T * LS];
-    const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-    const int n = nvalid[b], t0 = t_base + chunk * DC_T;
+    constexpr int RS = D + 4, VS = 132;          // rows apart: 16 of them in different banks
+    extern __shared__ __attribute__((aligned(16))) float db_smem[];
+    float *qs = db_smem, *ks = qs + DB_T * RS, *ds = ks + DB_T * RS, *vs = ds + DB_T * RS;
+    float *g4 = vs + DB_T * VS, *one = g4 + 16 * D, *gb = one + D;      // decays of 4 tokens, 1, of 16
+    float *Ls = gb + 4 * D, *Ps = Ls + 4 * 320, *Ms = Ps + 4 * 256, *bs = Ms + 6 * 320;
+    const int blk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    const int n = nvalid[b], t0 = t_base + blk * DB_T;
     if (seq[b] < 0 || t0 >= n) return;           // uniform over the workgroup
     const int tid = threadIdx.x, tk = tid >> 4, ln = tid & 15, c0 = ln * PC;
-    const int g = h / (H / G);
-    const bool valid = t0 + tk < n;
-    const long row = (long)b * S + min(t0 + tk, n - 1);   // padding repeats the last row: no
-                                                          // branch around a load
+    const int sub = tid >> 8;                    // of 16 tokens: 256 threads each
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r16 = lane & 15, q4 = lane >> 4;
     {
-        float qv[PC], kv[PC], av[PC], bv[PC], sq = 0.f, sk = 0.f;
-        const float* qp = qkv + row * cstride + (long)g * D + c0;
-        const T* ap = a + row * astride + (per_head ? h : (long)h * D + c0);
-        const float* bp = dt_bias + (per_head ? h : h * D + c0);
+        const bool valid = t0 + tk < n;
+        const long row = (long)b * S + min(t0 + tk, n - 1);  // padding repeats the last row: no
+                                                             // branch around a load
+        float qv[PC], kv[PC], av[PC], sq = 0.f, sk = 0.f;
+        DbRow<T, PC> ra;
+        DbRow<float, PC> rb;
+        const float* qp = qkv + row * cstride + (long)(h / (H / G)) * D + c0;
 #pragma unroll
         for (int i = 0; i < PC; i += 4) {
             const float4 x = *reinterpret_cast<const float4*>(qp + i);
@@ -2429,10 +2494,12 @@ delta_chunk_kernel(const float* __restrict__ qkv, long cstride, const T* __restr
             qv[i] = x.x; qv[i + 1] = x.y; qv[i + 2] = x.z; qv[i + 3] = x.w;
             kv[i] = y.x; kv[i + 1] = y.y; kv[i + 2] = y.z; kv[i + 3] = y.w;
         }
-#pragma unroll
-        for (int i = 0; i < PC; ++i) {
-            av[i] = ldf<T>(ap + (per_head ? 0 : i));
-            bv[i] = bp[per_head ? 0 : i];
+        if (per_head) {
+            ra.v[0] = a[row * astride + h];
+            rb.v[0] = dt_bias[h];
+        } else {
+            ra = *reinterpret_cast<const DbRow<T, PC>*>(a + row * astride + (long)h * D + c0);
+            rb = *reinterpret_cast<const DbRow<float, PC>*>(dt_bias + h * D + c0);
         }
         const float braw = ldf<T>(beta + row * bstride + h);
         asm volatile("" ::: "memory");
@@ -2446,15 +2513,20 @@ delta_chunk_kernel(const float* __restrict__ qkv, long cstride, const T* __restr
         const float iq = 1.f / sqrtf(part_sum<16>(sq) + 1e-6f) * (1.f / sqrtf((float)D));
         const float ik = 1.f / sqrtf(part_sum<16>(sk) + 1e-6f);
         const float neg_rate = -expf(a_log[h]);
-        float dec = expf(neg_rate * softplusf_(av[0] + bv[0]));
+        if (per_head) {
+            const float dec = exp_near(neg_rate * softplus_near(ldf<T>(&ra.v[0]) + rb.v[0]));
 #pragma unroll
-        for (int i = 0; i < PC; ++i) {
-            if (i > 0 && !per_head) dec = expf(neg_rate * softplusf_(av[i] + bv[i]));
-            av[i] = valid ? dec : 1.f;           // padding: decay 1, q = k = beta = 0
+            for (int i = 0; i < PC; ++i) av[i] = valid ? dec : 1.f;
+        } else {
+#pragma unroll
+            for (int i = 0; i < PC; ++i) {
+                const float dec = exp_near(neg_rate * softplus_near(ldf<T>(&ra.v[i]) + rb.v[i]));
+                av[i] = valid ? dec : 1.f;       // padding: decay 1, q = k = beta = 0
+            }
         }
 #pragma unroll
         for (int i = 0; i < PC; i += 4) {
-            const int at = tk * D + c0 + i;
+            const int at = tk * RS + c0 + i;
             *reinterpret_cast<float4*>(qs + at) =
                 float4{qv[i] * iq, qv[i + 1] * iq, qv[i + 2] * iq, qv[i + 3] * iq};
             *reinterpret_cast<float4*>(ks + at) =
@@ -2462,302 +2534,590 @@ delta_chunk_kernel(const float* __restrict__ qkv, long cstride, const T* __restr
             *reinterpret_cast<float4*>(ds + at) = float4{av[i], av[i + 1], av[i + 2], av[i + 3]};
         }
         if (ln == 0) bs[tk] = valid ? sigmoidf_(braw) : 0.f;
-        Ls[tk * LS + ln] = 0.f;
-        Ps[tk * KS + ln] = 0.f;
+        Ls[sub * 320 + (tk & 15) * 20 + ln] = 0.f;
+        Ps[sub * 256 + (tk & 15) * 16 + ln] = 0.f;
+        if (tid < D) one[tid] = 1.f;
     }
     __syncthreads();
-    if (tid < D) {
-        float p = 1.f;
+    // values of 128 channels from v0 on, a quarter of a row's 32 pieces a thread and turn
+    float4 vr[2];
+    auto load_values = [&](int v0) {
 #pragma unroll
-        for (int t = 0; t < DC_T; ++t) {
-            p *= ds[t * D + tid];
-            gam[t * D + tid] = p;
+        for (int i = 0; i < 2; ++i) {
+            const int t = t0 + (tid >> 5) + i * 32, c = v0 + (tid & 31) * 4;
+            vr[i] = *reinterpret_cast<const float4*>(qkv + ((long)b * S + min(t, n - 1)) * cstride +
+                                                     2L * G * D + (long)h * Dv + min(c, Dv - 4));
+            if (t >= n) vr[i] = float4{0.f, 0.f, 0.f, 0.f};
         }
+    };
+    auto store_values = [&]() {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            *reinterpret_cast<float4*>(vs + ((tid >> 5) + i * 32) * VS + (tid & 31) * 4) = vr[i];
+    };
+    {
+        // a wave has 4 tokens: their products among each other, decays to each from the first on and
+        // from each to the last
+        constexpr int CPL = D / 64;
+        const int at = wid * 4 * RS + lane * CPL;
+        float k4[4][CPL], v[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = 0.f;
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+            float kt[4], qt[4], dt[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                kt[t] = ks[at + t * RS + c];
+                qt[t] = qs[at + t * RS + c];
+                dt[t] = ds[at + t * RS + c];
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                float w = kt[s];
+                v[s * (s + 3) / 2] += qt[s] * w;
+#pragma unroll
+                for (int t = s + 1; t < 4; ++t) {
+                    w *= dt[t];
+                    v[t * (t + 1) / 2 + s] += qt[t] * w;
+                    v[10 + t * (t - 1) / 2 + s] += kt[t] * w;
+                }
+                k4[s][c] = w;
+            }
+            float p = 1.f;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                p *= dt[t];
+                ks[at + t * RS + c] = kt[t] * p;
+                qs[at + t * RS + c] = qt[t] * p;
+                ds[at + t * RS + c] = k4[t][c];
+            }
+            g4[wid * D + lane * CPL + c] = p;
+        }
+        const float sum = wave_sums16(v, lane);
+        const int e = r16 + q4 * 4, a4 = (wid & 3) * 4;
+        if (r16 < 4) {
+            if (e < 10) {
+                const int t = e < 1 ? 0 : e < 3 ? 1 : e < 6 ? 2 : 3;
+                Ps[sub * 256 + (a4 + t) * 16 + a4 + e - t * (t + 1) / 2] = sum;
+            } else {
+                const int t = e < 11 ? 1 : e < 13 ? 2 : 3;
+                Ls[sub * 320 + (a4 + t) * 20 + a4 + e - 10 - t * (t - 1) / 2] = sum;
+            }
+        }
+    }
+    __syncthreads();
+    load_values(0);                              // on their way meanwhile
+    // 4 tokens with earlier 4 of the same 16: a wave has the 6 pairs of two 16s (12 products of 4 x 4 at
+    // once), k and q, and an eighth of the channels
+    const int pr = lane >> 2, pp = pr % 6, pa = pp < 1 ? 1 : pp < 3 ? 2 : 3, pb = pp - pa * (pa - 1) / 2;
+    {
+        const int sb = (wid >> 3) * 2 + (pr >= 6 && pr < 12), d0 = (wid & 7) * (D / 8);
+        const int ra = (sb * 16 + pa * 4 + (lane & 3)) * RS + d0;
+        const float* B = ds + (sb * 16 + pb * 4 + (lane & 3)) * RS + d0;
+        const float* s1 = (pa - pb > 1 ? g4 + (sb * 4 + pb + 1) * D : one) + d0;
+        const float* s2 = (pa - pb > 2 ? g4 + (sb * 4 + pb + 2) * D : one) + d0;
+        dc_f32x4 ck = {0.f, 0.f, 0.f, 0.f}, cq = ck;
+#pragma unroll
+        for (int d = 0; d < D / 8; d += 4) {
+            const dc_f32x4 x = *reinterpret_cast<const dc_f32x4*>(ks + ra + d);
+            const dc_f32x4 z = *reinterpret_cast<const dc_f32x4*>(qs + ra + d);
+            dc_f32x4 y = *reinterpret_cast<const dc_f32x4*>(B + d);
+            y *= *reinterpret_cast<const dc_f32x4*>(s1 + d);
+            y *= *reinterpret_cast<const dc_f32x4*>(s2 + d);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                ck = __builtin_amdgcn_mfma_f32_4x4x1f32(x[r], y[r], ck, 0, 0, 0);
+                cq = __builtin_amdgcn_mfma_f32_4x4x1f32(z[r], y[r], cq, 0, 0, 0);
+            }
+        }
+        *reinterpret_cast<dc_f32x4*>(vs + (wid * 64 + lane) * 4) = ck;
+        *reinterpret_cast<dc_f32x4*>(vs + 4096 + (wid * 64 + lane) * 4) = cq;
+    }
+    __syncthreads();
+    if (tid >= 4 * D) {
+        if (tid < 4 * D + 256 && pr < 12) {      // k and q of two 16s each: a wave
+            const int what = (tid - 4 * D) >> 6, sb = (what & 1) * 2 + (pr >= 6);
+            dc_f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                c += *reinterpret_cast<const dc_f32x4*>(vs + (what >> 1) * 4096 + (((what & 1) * 8 + i) * 64 + lane) * 4);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (what < 2) Ls[sb * 320 + (pa * 4 + r) * 20 + pb * 4 + (lane & 3)] = c[r];
+                else Ps[sb * 256 + (pa * 4 + r) * 16 + pb * 4 + (lane & 3)] = c[r];
+            }
+        }
+    } else {
+        // decays from the start of the 16 to each token and from each to their end
+        const int i = tid / D, d = tid % D;
+        float p = g4[i * 4 * D + d];
+#pragma unroll
+        for (int a4 = 1; a4 < 4; ++a4) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                ks[(i * 16 + a4 * 4 + t) * RS + d] *= p;
+                qs[(i * 16 + a4 * 4 + t) * RS + d] *= p;
+            }
+            p *= g4[(i * 4 + a4) * D + d];
+        }
+        gb[i * D + d] = p;
+        p = 1.f;
+#pragma unroll
+        for (int a4 = 2; a4 >= 0; --a4) {
+            p *= g4[(i * 4 + a4 + 1) * D + d];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) ds[(i * 16 + a4 * 4 + t) * RS + d] *= p;
+        }
+    }
+    __syncthreads();
+    store_values();
+
+    float* o = ws + (((long)b * nblk + blk) * H + h) * db_unit(D, Dv);
+    float *oq = o + 64L * D, *ok = o + 128L * D, *ou = o + 192L * D, *op = ou + 64L * Dv, *og = op + 2560;
+    for (int v0 = 0; v0 < Dv; v0 += 128) {
+        const int vn = min(128, Dv - v0), wn = v0 ? 0 : D;
+        if (v0) {
+            load_values(v0);
+            __syncthreads();
+            store_values();
+        }
+        __syncthreads();
+        // Y_i = (I + L_ii)^-1 beta (Gam k | V)_i, a thread a column
+        const int c = tid & 255;
+        if (c < wn + vn) {
+            const float *L = Ls + sub * 320, *bt = bs + sub * 16;
+            const int step = c < wn ? RS : VS;
+            float* const col = c < wn ? ks + sub * 16 * RS + c : vs + sub * 16 * VS + c - wn;
+            float x[16];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) x[t] = col[t * step];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) {
+                float v = x[t];
+#pragma unroll
+                for (int s = 0; s < t; s += 4) {
+                    const float4 l4 = *reinterpret_cast<const float4*>(L + t * 20 + s);
+                    v -= l4.x * x[s];
+                    if (s + 1 < t) v -= l4.y * x[s + 1];
+                    if (s + 2 < t) v -= l4.z * x[s + 2];
+                    if (s + 3 < t) v -= l4.w * x[s + 3];
+                }
+                x[t] = bt[t] * v;
+            }
+#pragma unroll
+            for (int t = 0; t < 16; ++t) col[t * step] = x[t];
+        }
+        __syncthreads();
+        if (!v0) {
+            if (wid < 12) {
+                // of 16 tokens i with earlier 16 j: M_ij = (I + L_ii)^-1 L_ij = Y_i diag(Gam_{j,i}) k_j',
+                // Y that of Gam k, and P_ij
+                const int pair = wid % 6, i = pair < 1 ? 1 : pair < 3 ? 2 : 3, j = pair - i * (i - 1) / 2;
+                const float* A = (wid < 6 ? ks : qs) + (i * 16 + r16) * RS + q4 * 4;
+                const float* B = ds + (j * 16 + r16) * RS + q4 * 4;
+                dc_f32x4 c[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+                for (int kk = 0; kk < D / 16; ++kk) {
+                    dc_f32x4 x = *reinterpret_cast<const dc_f32x4*>(A + kk * 16);
+                    const dc_f32x4 y = *reinterpret_cast<const dc_f32x4*>(B + kk * 16);
+                    for (int m = j + 1; m < i; ++m)
+                        x *= *reinterpret_cast<const dc_f32x4*>(gb + m * D + kk * 16 + q4 * 4);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        c[r & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[r], y[r], c[r & 1], 0, 0, 0);
+                }
+                c[0] += c[1];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = q4 * 4 + r;
+                    if (wid < 6) Ms[pair * 320 + t * 20 + r16] = c[0][r];
+                    else op[(i * (i + 1) / 2 + j) * 256 + (t + (r16 >> 2) * 16) * 4 + (r16 & 3)] = c[0][r];
+                }
+            }
+            __syncthreads();
+        }
+        // X_i = Y_i - sum over j < i of M_ij X_j; a wave has 16 columns of all four
+        const bool isw = wid < wn / 16;
+        const int tile = isw ? wid : wid - wn / 16;
+        if (isw || tile < vn / 16) {
+            const float* y = isw ? ks + tile * 16 + r16 : vs + tile * 16 + r16;
+            const int ys = isw ? RS : VS;
+            dc_f32x4 X[4];
+            float gg = 1.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) X[i][r] = y[(i * 16 + q4 * 4 + r) * ys];
+                if (isw && i > 0) {
+                    gg *= gb[(i - 1) * D + tile * 16 + r16];
+                    X[i] *= gg;
+                }
+#pragma unroll
+                for (int j = 0; j < i; ++j) {
+                    const dc_f32x4 m = -*reinterpret_cast<const dc_f32x4*>(
+                        Ms + (i * (i - 1) / 2 + j) * 320 + r16 * 20 + q4 * 4);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        X[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[r], X[j][r], X[i], 0, 0, 0);
+                }
+                if (isw) {                       // (out in whole lines, below)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) ks[(i * 16 + q4 * 4 + r) * RS + tile * 16 + r16] = -X[i][r];
+                } else {
+                    *reinterpret_cast<dc_f32x4*>(ou + (long)i * Dv * 16 + (v0 + tile * 16 + r16) * 16 + q4 * 4) = X[i];
+                }
+            }
+        }
+    }
+    for (int at = tid; at < DB_T * D / 4; at += 1024) {      // q from the block's start
+        const int piece = at >> 6, i = piece / (D / 16), t = i * 16 + r16, d = piece % (D / 16) * 16 + q4 * 4;
+        dc_f32x4 x = *reinterpret_cast<const dc_f32x4*>(qs + t * RS + d);
+        for (int m = 0; m < i; ++m) x *= *reinterpret_cast<const dc_f32x4*>(gb + m * D + d);
+        *reinterpret_cast<dc_f32x4*>(oq + at * 4) = x;
+    }
+    for (int at = tid; at < DB_T * D / 4; at += 1024) {      // k to its end, 4 tokens a thread
+        const int piece = at >> 6, i = piece / (D / 16), d = piece % (D / 16) * 16 + r16;
+        float f = 1.f;
+        for (int m = i + 1; m < 4; ++m) f *= gb[m * D + d];
+        dc_f32x4 x;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = ds[(i * 16 + q4 * 4 + r) * RS + d] * f;
+        *reinterpret_cast<dc_f32x4*>(ok + at * 4) = x;
+    }
+    __syncthreads();
+    for (int at = tid; at < DB_T * D / 4; at += 1024) {
+        const int piece = at >> 6, t = piece / (D / 16) * 16 + r16, d = piece % (D / 16) * 16 + q4 * 4;
+        *reinterpret_cast<dc_f32x4*>(o + at * 4) = *reinterpret_cast<const dc_f32x4*>(ks + t * RS + d);
     }
     {
-        const int s = tk;                        // 16 lanes carry Gam_{s,t} k_s over t
-        float w[PC];
-#pragma unroll
-        for (int i = 0; i < PC; ++i) w[i] = ks[s * D + c0 + i];
-        for (int t = (tid >> 6) * 4; t < DC_T; ++t) {
-            float al = 0.f, ap = 0.f;
-#pragma unroll
-            for (int i = 0; i < PC; ++i) {
-                if (t > s) w[i] *= ds[t * D + c0 + i];
-                al += ks[t * D + c0 + i] * w[i];
-                ap += qs[t * D + c0 + i] * w[i];
-            }
-            al = part_sum<16>(al);
-            ap = part_sum<16>(ap);
-            if (ln == 0 && t >= s) {
-                Ps[t * KS + s] = ap;
-                if (t > s) Ls[t * LS + s] = al;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < PC; ++i) kh[(c0 + i) * KS + s] = w[i];
+        const int t = (tid >> 4) & 15, c = tid & 15;
+        op[(sub * (sub + 1) / 2 + sub) * 256 + (t + (c >> 2) * 16) * 4 + (c & 3)] = Ps[tid];
     }
-    __syncthreads();
-    float* o = ws + (((long)b * nchunk + chunk) * H + h) * dc_unit(D, Dv);
-    for (int col = tid; col < D + Dv; col += 256) {
-        const float* vp = qkv + ((long)b * S + t0) * cstride + 2L * G * D + (long)h * Dv + (col - D);
-        float x[DC_T];
-        if (col < D) {
-#pragma unroll
-            for (int t = 0; t < DC_T; ++t) x[t] = ks[t * D + col] * gam[t * D + col];
-        } else {
-#pragma unroll
-            for (int t = 0; t < DC_T; ++t) x[t] = vp[(long)min(t, n - 1 - t0) * cstride];
-#pragma unroll
-            for (int t = 0; t < DC_T; ++t) x[t] = t0 + t < n ? x[t] : 0.f;
-        }
-#pragma unroll
-        for (int t = 0; t < DC_T; ++t) {
-            float v = x[t];
-#pragma unroll
-            for (int s = 0; s < t; s += 4) {
-                const float4 L = *reinterpret_cast<const float4*>(&Ls[t * LS + s]);
-                v -= L.x * x[s];
-                if (s + 1 < t) v -= L.y * x[s + 1];
-                if (s + 2 < t) v -= L.z * x[s + 2];
-                if (s + 3 < t) v -= L.w * x[s + 3];
-            }
-            x[t] = bs[t] * v;
-        }
-        if (col < D) {
-#pragma unroll
-            for (int t = 0; t < DC_T; ++t) o[t * D + col] = x[t];
-        } else {
-            float* u = o + 48L * D + (long)(col - D) * DC_T;
-#pragma unroll
-            for (int t = 0; t < DC_T; t += 4)
-                *reinterpret_cast<float4*>(u + t) = float4{x[t], x[t + 1], x[t + 2], x[t + 3]};
-        }
-    }
-    for (int i = tid; i < DC_T * D; i += 256) {
-        o[16 * D + i] = qs[i] * gam[i];
-        o[32 * D + i] = kh[(i >> 4) * KS + (i & 15)];
-    }
-    o[48L * D + 16L * Dv + tid] = Ps[tk * KS + ln];
-    if (tid < D) o[48L * D + 16L * Dv + 256 + tid] = gam[(DC_T - 1) * D + tid];
+    if (tid < D) og[tid] = gb[tid] * gb[D + tid] * gb[2 * D + tid] * gb[3 * D + tid];
 }
 
 template <int D>
-__global__ void __launch_bounds__(6 * WAVE)
-delta_chunk_scan_kernel(const float* __restrict__ ws, float* __restrict__ state,
+__global__ void __launch_bounds__(512)
+delta_block_scan_kernel(float* __restrict__ ws, float* __restrict__ state,
                         const int* __restrict__ pos, const int* __restrict__ seq,
-                        const int* __restrict__ nvalid, float* __restrict__ obuf, int t_base,
-                        int nchunk, int S, int H, int Dv) {
-    constexpr int NB = D / 64;                   // 16-row blocks of the state a wave holds
-    __shared__ dc_f32x4 exu[2][4][WAVE], exo[2][4][WAVE];   // parity, wave, lane
-    __shared__ dc_f32x4 scratch[WAVE];
+                        const int* __restrict__ nvalid, int t_base, int nblk, int S, int H, int Dv) {
+    constexpr int NB = D / 64;                   // 16-row pieces of the state a wave holds
+    constexpr int WB = DB_T * D * 4 + 4096, KB = DB_T * D * 4;       // bytes of W and U0, of K
+    constexpr int NW = WB / 4096, NK = KB / 4096;                    // loads of a loading wave
+    extern __shared__ __attribute__((aligned(16))) char ds_smem[];
+    // [2][W | U0] [2][K] [16 tokens][wave][lane]
+    dc_f32x4* const ex = reinterpret_cast<dc_f32x4*>(ds_smem + 2 * WB + 2 * KB);
     const int h = blockIdx.x, col0 = blockIdx.y * 16, b = blockIdx.z;
     const int slot = seq[b], n = nvalid[b];
     if (slot < 0 || n <= t_base) return;         // uniform over the workgroup
-    const int nch = min(nchunk, (n - t_base + DC_T - 1) / DC_T);
+    const int nb = min(nblk, (n - t_base + DB_T - 1) / DB_T);
     const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const long unit = dc_unit(D, Dv);
-    const char* base = reinterpret_cast<const char*>(ws + ((long)b * nchunk * H + h) * unit);
-    const long hop = (long)H * unit * 4;         // bytes from chunk to chunk
-    const unsigned au = (48 * D + (col0 + r16) * 16 + g * 4) * 4;
-    const unsigned ap = (48 * D + 16 * Dv + r16 * 16 + g * 4) * 4;
+    const long unit = db_unit(D, Dv);
+    float* const base = ws + ((long)b * nblk * H + h) * unit;
+    const long hop = (long)H * unit;
     auto barrier = [] {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
-
-    if (wid == 5) {
-        // the runner ahead: pulls this workgroup's share of the chunk after next few into L2, so
-        // that the 3 chunks that fit the registers cover what is left of the way. The loads go
-        // to a scratch kilobyte of LDS and nothing waits for them until the end.
-        const unsigned lds = __builtin_amdgcn_readfirstlane(
-            (unsigned)(size_t)(__attribute__((address_space(3))) char*)scratch);
-        for (int c = 0; c <= nch; ++c) {
-            const char* o = base + min(c + DC_AHEAD, nch - 1) * hop;
-            for (int at = blockIdx.y * 1024; at < (int)unit * 4; at += gridDim.y * 1024) {
-                const char* from = o + min(at + lane * 16, (int)unit * 4 - 16);
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                             :: "s"(lds), "v"(from) : "memory", "m0");
-            }
-            __builtin_amdgcn_s_barrier();
+    // Barriers A (the sums' halves 0 and 1 are there) and B (2 and 3) of each block. W of block c is
+    // read before A(c), K between A(c) and the next turn.
+    if (wid >= 4) {
+        const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)ds_smem;
+        const int p0 = wid - 4;
+        auto get = [&](const char* from, unsigned to) {
+            const unsigned at = __builtin_amdgcn_readfirstlane(to);
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                         :: "s"(at), "v"(from + lane * 16) : "memory", "m0");
+        };
+        auto get_w = [&](int c) {
+            const char* o = reinterpret_cast<const char*>(base + min(c, nb - 1) * hop);
+            const unsigned to = lds0 + (c & 1) * WB;
+#pragma unroll
+            for (int i = 0; i < NW - 1; ++i) get(o + (i * 4 + p0) * 1024, to + (i * 4 + p0) * 1024);
+            // (past the last block: what its update overwrites, not used)
+            get(o + (192L * D + (long)p0 * Dv * 16 + col0 * 16) * 4, to + KB + p0 * 1024);
+        };
+        auto get_k = [&](int c) {
+            const char* o = reinterpret_cast<const char*>(base + min(c, nb - 1) * hop) + 128 * D * 4;
+            const unsigned to = lds0 + 2 * WB + (c & 1) * KB;
+#pragma unroll
+            for (int i = 0; i < NK; ++i) get(o + (i * 4 + p0) * 1024, to + (i * 4 + p0) * 1024);
+        };
+        get_w(0);
+        get_k(0);
+        get_w(1);
+        asm volatile("s_waitcnt vmcnt(%c0)" ::"i"(NW + NK) : "memory");
+        __builtin_amdgcn_s_barrier();            // W of the first
+        for (int c = 0; c < nb; ++c) {
+            asm volatile("s_waitcnt vmcnt(%c0)" ::"i"(NW) : "memory");
+            __builtin_amdgcn_s_barrier();        // A: K of this block is there, W of it is read
+            get_k(c + 1);
+            asm volatile("s_waitcnt vmcnt(%c0)" ::"i"(NK) : "memory");
+            __builtin_amdgcn_s_barrier();        // B: W of the next is there
+            get_w(c + 2);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         return;
     }
-    if (wid == 4) {
-        // the read-out: after barrier c, U of chunk c from exu and O of chunk c - 1 (whose exo
-        // the state waves completed before that barrier) to memory
-        struct Ops {
-            dc_f32x4 u0, p;
-        };
-        auto load = [&](Ops& x, int c) {
-            const char* o = base + min(c, nch - 1) * hop;
-            x.u0 = *reinterpret_cast<const dc_f32x4*>(o + au);
-            x.p = *reinterpret_cast<const dc_f32x4*>(o + ap);
-            asm volatile("" ::: "memory");       // in flight from here on
-            __builtin_amdgcn_sched_barrier(0);
-        };
-        dc_f32x4 uu = {0.f, 0.f, 0.f, 0.f};
-        float* op = obuf + (((long)b * S + t_base + g * 4) * H + h) * Dv + col0 + r16;
-        auto sums = [&](const Ops& cur, int c) {
-            dc_f32x4 u = cur.u0;
-#pragma unroll
-            for (int w = 0; w < 4; ++w) u -= exu[c & 1][w][lane];
-            return u;
-        };
-        auto read_out = [&](const Ops& prev, int c) {
-            dc_f32x4 oo = exo[c & 1][0][lane];
-#pragma unroll
-            for (int w = 1; w < 4; ++w) oo += exo[c & 1][w][lane];
-            if (__any(!((uu[0] + uu[1]) * 0.f + (uu[2] + uu[3]) * 0.f == 0.f))) {
-                // a token whose update is not finite: P is 0 for the tokens before it, but
-                // 0 * NaN is not. Row by row, over the tokens that each one sees
-                for (int w = 0; w < 4; ++w)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float us = __shfl(uu[e], r16 + 16 * w, WAVE);
-                        // (an infinite update makes infinities of both signs in the state)
-                        const float later = us + us * 0.f;
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const float ps = __shfl(prev.p[e], g * 4 + r + 16 * w, WAVE);
-                            const int over = g * 4 + r - (w * 4 + e);
-                            if (over >= 0) oo[r] += ps * (over ? later : us);
-                        }
-                    }
-                return oo;
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                oo = __builtin_amdgcn_mfma_f32_16x16x4f32(prev.p[r], uu[r], oo, 0, 0, 0);
-            return oo;
-        };
-        // chunks before the last are whole: their stores are unconditional, or the compiler
-        // cannot count them and waits for the stores of the turn before
-        auto step = [&](const Ops& cur, const Ops& prev, int c) {
-            barrier();
-            const dc_f32x4 un = sums(cur, c), oo = read_out(prev, c - 1);
-            float* o = op + (long)(c - 1) * DC_T * H * Dv;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o[(long)r * H * Dv] = oo[r];
-            uu = un;
-        };
-        auto last = [&](const Ops& prev) {
-            barrier();
-            const dc_f32x4 oo = read_out(prev, nch - 1);
-            const int left = n - t_base - (nch - 1) * DC_T - g * 4;
-            float* o = op + (long)(nch - 1) * DC_T * H * Dv;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (r < left) o[(long)r * H * Dv] = oo[r];
-        };
-        Ops x0, x1, x2, x3;
-        load(x0, 0);
-        load(x1, 1);
-        load(x2, 2);
-        barrier();
-        uu = sums(x0, 0);
-        for (int c = 1;;) {
-            if (c >= nch) { last(x0); break; }
-            load(x3, c + 2);
-            step(x1, x0, c);
-            if (++c >= nch) { last(x1); break; }
-            load(x0, c + 2);
-            step(x2, x1, c);
-            if (++c >= nch) { last(x2); break; }
-            load(x1, c + 2);
-            step(x3, x2, c);
-            if (++c >= nch) { last(x3); break; }
-            load(x2, c + 2);
-            step(x0, x3, c);
-            ++c;
-        }
-        return;
-    }
-
-    // state waves: NB blocks of 16 rows each, C layout
     float* st = state + (((long)slot * H + h) * Dv + col0 + r16) * D + wid * (NB * 16) + g * 4;
     const bool carry = t_base > 0 || pos[(long)b * S] > 0;
-    dc_f32x4 s[NB];
+    dc_f32x4 s[NB], w[4][NB], k[4][NB], gm[NB], gn[NB], u0;
 #pragma unroll
     for (int i = 0; i < NB; ++i)
         s[i] = carry ? *reinterpret_cast<const dc_f32x4*>(st + i * 16) : dc_f32x4{0.f, 0.f, 0.f, 0.f};
-    struct Ops {
-        dc_f32x4 w[NB], q[NB], k[NB], gm[NB], u0;
-    };
-    const unsigned aw = (r16 * D + wid * NB * 16 + g * 4) * 4;
-    const unsigned ak = (32 * D + (wid * NB * 16 + r16) * 16 + g * 4) * 4;
-    const unsigned ag = (48 * D + 16 * Dv + 256 + wid * NB * 16 + g * 4) * 4;
-    auto load = [&](Ops& x, int c) {
-        const char* o = base + min(c, nch - 1) * hop;
+    const int ag = 192 * D + 64 * Dv + 2560 + wid * NB * 16 + g * 4;
+    const int au = 192 * D + wid * Dv * 16 + (col0 + r16) * 16 + g * 4;
+    const int as = 193 * D + 64 * Dv + 2560 + (wid * NB * (Dv / 16) + blockIdx.y) * 256 + lane * 4;
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    unsigned own[4];                             // all ones for the wave's own 16 tokens
 #pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            x.w[i] = *reinterpret_cast<const dc_f32x4*>(o + aw + i * 64);
-            x.q[i] = *reinterpret_cast<const dc_f32x4*>(o + aw + 16 * D * 4 + i * 64);
-            x.k[i] = *reinterpret_cast<const dc_f32x4*>(o + ak + i * 1024);
-            x.gm[i] = *reinterpret_cast<const dc_f32x4*>(o + ag + i * 64);
-        }
-        x.u0 = *reinterpret_cast<const dc_f32x4*>(o + au);
-        asm volatile("" ::: "memory");           // in flight from here on
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    auto step = [&](const Ops& x, int c) {
-        const int par = c & 1;
-        dc_f32x4 u[NB], o[NB], v[4];
-#pragma unroll
-        for (int i = 0; i < NB; ++i) u[i] = o[i] = dc_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int i = 0; i < NB; ++i)
-                u[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w[i][r], s[i][r], u[i], 0, 0, 0);
-#pragma unroll
-        for (int i = 1; i < NB; ++i) u[0] += u[i];
-        exu[par][wid][lane] = u[0];
-        barrier();
-#pragma unroll
-        for (int w = 0; w < 4; ++w) v[w] = exu[par][w][lane];
-        // while the sums arrive
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int i = 0; i < NB; ++i)
-                o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][r], s[i][r], o[i], 0, 0, 0);
-        const dc_f32x4 uu = x.u0 - ((v[0] + v[1]) + (v[2] + v[3]));
-#pragma unroll
-        for (int i = 0; i < NB; ++i) s[i] *= x.gm[i];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int i = 0; i < NB; ++i)
-                s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i][r], uu[r], s[i], 0, 0, 0);
-#pragma unroll
-        for (int i = 1; i < NB; ++i) o[0] += o[i];
-        exo[par][wid][lane] = o[0];
-    };
-    Ops x0, x1, x2, x3;
-    load(x0, 0);
-    load(x1, 1);
-    load(x2, 2);
-    for (int c = 0;;) {
-        load(x3, c + 3);
-        step(x0, c);
-        if (++c >= nch) break;
-        load(x0, c + 3);
-        step(x1, c);
-        if (++c >= nch) break;
-        load(x1, c + 3);
-        step(x2, c);
-        if (++c >= nch) break;
-        load(x2, c + 3);
-        step(x3, c);
-        if (++c >= nch) break;
+    for (int t = 0; t < 4; ++t) {
+        own[t] = t == wid ? ~0u : 0u;
+        asm volatile("" : "+v"(own[t]));         // (a mask, not a branch)
     }
-    barrier();                                   // the read-out's last turn
+    auto read_w = [&](int c) {
+        const char* p = ds_smem + (c & 1) * WB + lane * 16;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+                w[t][i] = *reinterpret_cast<const dc_f32x4*>(p + (t * (D / 16) + wid * NB + i) * 1024);
+        u0 = *reinterpret_cast<const dc_f32x4*>(ds_smem + (c & 1) * WB + KB + wid * 1024 + r16 * 64 + g * 16);
+    };
+    auto read_k = [&](int c, int t) {
+        const char* p = ds_smem + 2 * WB + (c & 1) * KB + lane * 16;
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+            k[t][i] = *reinterpret_cast<const dc_f32x4*>(p + (t * (D / 16) + wid * NB + i) * 1024);
+    };
+    auto decays = [&](dc_f32x4 (&x)[NB], int c) {
+        const float* o = base + min(c, nb - 1) * hop + ag;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) x[i] = *reinterpret_cast<const dc_f32x4*>(o + i * 16);
+    };
+    decays(gm, 0);
+    barrier();
+    read_w(0);
+    for (int c = 0; c < nb; ++c) {
+        float* o = base + c * hop;
+        dc_f32x4 u[4], v[2][4];
+        // this wave's rows of U0 - W S: of 16 tokens and the next, their products in turns
+        auto ahead = [&](int t) {
+            u[t] = __builtin_bit_cast(dc_f32x4, __builtin_bit_cast(u32x4, u0) & own[t]);
+            u[t + 1] = __builtin_bit_cast(dc_f32x4, __builtin_bit_cast(u32x4, u0) & own[t + 1]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    u[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][i][r], s[i][r], u[t], 0, 0, 0);
+                    u[t + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t + 1][i][r], s[i][r], u[t + 1], 0, 0, 0);
+                }
+        };
+        auto sums = [&](int t) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+                for (int x = 0; x < 4; ++x) v[e][x] = ex[((t + e) * 4 + x) * 64 + lane];
+        };
+        auto add = [&](int t) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) u[t + e] = (v[e][0] + v[e][1]) + (v[e][2] + v[e][3]);
+        };
+        auto update = [&](int t) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int i = 0; i < NB; ++i)
+                    s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[t][i][r], u[t][r], s[i], 0, 0, 0);
+        };
+        ahead(0);
+        // while the products run
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+            *reinterpret_cast<dc_f32x4*>(o + as + i * (Dv / 16) * 256) = s[i];
+        decays(gn, c + 1);
+        ahead(2);
+        ex[(0 * 4 + wid) * 64 + lane] = u[0];
+        ex[(1 * 4 + wid) * 64 + lane] = u[1];
+        barrier();
+        sums(0);
+        read_k(c, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        ex[(2 * 4 + wid) * 64 + lane] = u[2];
+        ex[(3 * 4 + wid) * 64 + lane] = u[3];
+        read_k(c, 1);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) s[i] *= gm[i];
+        add(0);
+        update(0);
+        barrier();
+        sums(2);
+        __builtin_amdgcn_sched_barrier(0);
+        update(1);
+        read_k(c, 2);
+        read_k(c, 3);
+        add(2);
+        __builtin_amdgcn_sched_barrier(0);
+        read_w(c + 1);
+        update(2);
+        update(3);
+        __builtin_amdgcn_sched_barrier(0);
+        const u32x4 mine = (__builtin_bit_cast(u32x4, u[0]) & own[0]) | (__builtin_bit_cast(u32x4, u[1]) & own[1]) |
+                           (__builtin_bit_cast(u32x4, u[2]) & own[2]) | (__builtin_bit_cast(u32x4, u[3]) & own[3]);
+        *reinterpret_cast<u32x4*>(o + au) = mine;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) gm[i] = gn[i];
+    }
 #pragma unroll
     for (int i = 0; i < NB; ++i) *reinterpret_cast<dc_f32x4*>(st + i * 16) = s[i];
+}
+
+// (3) the read-out and, for up to 128 value channels, the head norm and gate (obuf null)
+template <typename T, int D>
+__global__ void __launch_bounds__(512, 4)
+delta_block_out_kernel(const float* __restrict__ ws, const int* __restrict__ seq,
+                       const int* __restrict__ nvalid, float* __restrict__ obuf,
+                       const T* __restrict__ gate, long gstride, const float* __restrict__ norm_w,
+                       float eps, T* __restrict__ out, int t_base, int nblk, int S, int H, int Dv,
+                       int gate_silu, int wide) {
+    constexpr int OS = 132;                      // rows of the result in LDS
+    __shared__ __attribute__((aligned(16))) float qs[DB_T * OS];
+    const int blk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    const int t0 = t_base + blk * DB_T, n = seq[b] < 0 ? 0 : nvalid[b];
+    const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // gates of the tokens and channels that this thread norms, on their way beside the last products
+    DbRow<T, 8> gates[2];
+    const int nt = tid >> 4, nc = (tid & 15) * 8;
+    auto load_gates = [&]() {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            gates[e] = *reinterpret_cast<const DbRow<T, 8>*>(
+                gate + ((long)b * S + min(t0 + nt + e * 32, n - 1)) * gstride + (long)h * Dv + min(nc, Dv - 8));
+    };
+    const float* o = ws + (((long)b * nblk + blk) * H + h) * db_unit(D, Dv);
+    const float *oq = o + 64L * D, *ou = o + 192L * D, *op = ou + 64L * Dv, *os = op + 2560 + D;
+    if (t0 < n) {
+        for (int at = tid; at < DB_T * D / 4; at += 512)
+            reinterpret_cast<float4*>(qs)[at] = reinterpret_cast<const float4*>(oq)[at];
+        __syncthreads();
+        for (int c0 = 0; c0 < Dv / 16; c0 += 8) {
+            dc_f32x4 O[4];                       // a wave has 16 channels
+            const int ct = c0 + wid;
+            if (ct >= Dv / 16 && !obuf) load_gates();
+            if (ct < Dv / 16) {
+                dc_f32x4 s[D / 16], u[4];
+#pragma unroll
+                for (int kk = 0; kk < D / 16; ++kk)
+                    s[kk] = *reinterpret_cast<const dc_f32x4*>(os + (kk * (Dv / 16) + ct) * 256 + lane * 4);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    u[i] = *reinterpret_cast<const dc_f32x4*>(
+                        ou + (long)i * Dv * 16 + (ct * 16 + r16) * 16 + g * 4);
+                    O[i] = {0.f, 0.f, 0.f, 0.f};
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int kk = 0; kk < D / 16; ++kk) {
+                    dc_f32x4 x[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        x[i] = *reinterpret_cast<const dc_f32x4*>(qs + ((i * (D / 16) + kk) * 64 + lane) * 4);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            O[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i][r], s[kk][r], O[i], 0, 0, 0);
+                    if (kk & 1) __builtin_amdgcn_sched_barrier(0);
+                }
+                if (!obuf) load_gates();
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    dc_f32x4 p[4];
+#pragma unroll
+                    for (int j = 0; j <= i; ++j)
+                        p[j] = *reinterpret_cast<const dc_f32x4*>(op + (i * (i + 1) / 2 + j) * 256 + lane * 4);
+                    dc_f32x4 oo = O[i];
+#pragma unroll
+                    for (int j = 0; j < i; ++j)  // an update that is not finite is NaN to later tokens
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            oo = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                p[j][r], fmaf(u[j][r], 0.f, u[j][r]), oo, 0, 0, 0);
+                    if (__any(!((u[i][0] + u[i][1]) * 0.f + (u[i][2] + u[i][3]) * 0.f == 0.f))) {
+                        // P is 0 for the tokens before it, but 0 * NaN is not. Row by row, over the
+                        // tokens that each one sees
+                        for (int w = 0; w < 4; ++w)
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) {
+                                const float us = __shfl(u[i][q], r16 + 16 * w, WAVE);
+                                // (an infinite update makes infinities of both signs in the state)
+                                const float later = us + us * 0.f;
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) {
+                                    const float ps = __shfl(p[i][q], g * 4 + r + 16 * w, WAVE);
+                                    const int over = g * 4 + r - (w * 4 + q);
+                                    if (over >= 0) oo[r] += ps * (over ? later : us);
+                                }
+                            }
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            oo = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i][r], u[i][r], oo, 0, 0, 0);
+                    }
+                    O[i] = oo;
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (!obuf) __syncthreads();          // q is read
+            if (ct < Dv / 16) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int t = i * 16 + g * 4 + r, c = ct * 16 + r16;
+                        if (!obuf) qs[t * OS + c] = O[i][r];
+                        else if (t0 + t < n) obuf[(((long)b * S + t0 + t) * H + h) * Dv + c] = O[i][r];
+                    }
+            }
+        }
+    }
+    if (obuf) return;
+    __syncthreads();
+    // as gated_rmsnorm_vec_kernel: 16 lanes a token, 8 channels each
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const int t = nt + e * 32;
+        if (t0 + t >= S) continue;               // (the same for the 16 lanes)
+        T* to = out + (((long)b * S + t0 + t) * H + h) * Dv + nc;
+        float v[8] = {}, ss = 0.f;
+        const bool mine = nc < Dv, live = t0 + t < n;
+        if (live && mine) {
+            load8<float>(qs + t * OS + nc, v);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) ss += v[i] * v[i];
+        }
+        ss = part_sum<16>(ss);
+        if (!mine) continue;
+        if (live) {
+            const float inv = 1.f / sqrtf(ss / Dv + eps);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float gt = ldf<T>(&gates[e].v[i]);
+                v[i] = v[i] * inv * norm_w[nc + i] * (gate_silu ? gt * sigmoidf_(gt) : sigmoidf_(gt));
+            }
+        }
+        if (wide) {
+            store8<T>(to, v);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) stf<T>(to + i, v[i]);
+        }
+    }
 }
 
 // per-head RMS norm over the value channels, shared weight, sigmoid gate: pad tokens produce zeros.
@@ -6088,29 +6448,45 @@ int nx_gated_delta(const float* qkv, long cstride, const void* beta, long bstrid
     if (D > 256 || H % G != 0 || (!ws && PS < (long)(2 * G + H) * D + H + G)) return -1;
     const long ntok = (long)B * S;
     if (ws) {
-        // in chunks, as many of them at a time as the workspace holds
+        // in blocks, as many of them and of the rows at a time as the workspace holds
         if ((D != 64 && D != 128) || Dv % 16 || cstride % 4) return -1;
-        const long per = (long)B * H * dc_unit(D, Dv);
-        const int span = (int)(ws_floats / per < 1024 ? ws_floats / per : 1024);
-        if (span < 1) return -1;
-        for (int t = 0; t < S; t += span * DC_T) {
-            const int nch = (S - t + DC_T - 1) / DC_T < span ? (S - t + DC_T - 1) / DC_T : span;
-            dim3 ga(nch, H, B), gb(H, Dv / 16, B), blk(256), blk6(6 * WAVE);
-#define DCA(TT, DD) delta_chunk_kernel<TT, DD><<<ga, blk, 0, st>>>( \
-            qkv, cstride, (const TT*)beta, bstride, (const TT*)a, astride, dt_bias, a_log, seq, \
-            nvalid, ws, t, nch, S, H, G, Dv, per_head)
-            if (in_bf16) { if (D == 64) DCA(bf16, 64); else DCA(bf16, 128); }
-            else { if (D == 64) DCA(float, 64); else DCA(float, 128); }
-#undef DCA
-            int rc = (int)hipGetLastError();
-            if (rc) return rc;
-            if (D == 64) delta_chunk_scan_kernel<64><<<gb, blk6, 0, st>>>(
-                ws, state, pos, seq, nvalid, obuf, t, nch, S, H, Dv);
-            else delta_chunk_scan_kernel<128><<<gb, blk6, 0, st>>>(
-                ws, state, pos, seq, nvalid, obuf, t, nch, S, H, Dv);
-            rc = (int)hipGetLastError();
-            if (rc) return rc;
-        }
+        const bool fused = Dv <= 128;
+        const int lds1 = D == 64 ? db_lds<64>() : db_lds<128>(), lds2 = 4 * DB_T * D * 4 + 2 * 4096 + 16384;
+        const int wide = (uintptr_t)out % 16 == 0;
+        const long units = ws_floats / ((long)H * db_unit(D, Dv));
+        if (units < 1) return -1;
+        const int rows = (int)(units < B ? units : B), most = (int)(units / rows < 1024 ? units / rows : 1024);
+        for (int b0 = 0; b0 < B; b0 += rows)
+            for (int t = 0; t < S; t += most * DB_T) {
+                const int left = (S - t + DB_T - 1) / DB_T, nblk = left < most ? left : most;
+                const int nr = B - b0 < rows ? B - b0 : rows;
+                const long r0 = (long)b0 * S;
+                const dim3 ga(nblk, H, nr), gb(H, Dv / 16, nr);
+                float* const ob = fused ? nullptr : obuf + r0 * H * Dv;
+#define DBK(TT, DD)                                                                                     \
+    do {                                                                                                \
+        if (hipFuncSetAttribute((const void*)delta_block_kernel<TT, DD>,                                \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, lds1) != hipSuccess ||      \
+            hipFuncSetAttribute((const void*)delta_block_scan_kernel<DD>,                               \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, lds2) != hipSuccess)        \
+            return (int)hipGetLastError();                                                              \
+        delta_block_kernel<TT, DD><<<ga, 1024, lds1, st>>>(                                             \
+            qkv + r0 * cstride, cstride, (const TT*)beta + r0 * bstride, bstride,                       \
+            (const TT*)a + r0 * astride, astride, dt_bias, a_log, seq + b0, nvalid + b0, ws, t, nblk, S, \
+            H, G, Dv, per_head);                                                                        \
+        delta_block_scan_kernel<DD><<<gb, 512, lds2, st>>>(ws, state, pos + r0, seq + b0, nvalid + b0, t, \
+                                                           nblk, S, H, Dv);                             \
+        delta_block_out_kernel<TT, DD><<<ga, 512, 0, st>>>(                                             \
+            ws, seq + b0, nvalid + b0, ob, (const TT*)gate + r0 * gstride, gstride, norm_w, eps,        \
+            (TT*)out + r0 * H * Dv, t, nblk, S, H, Dv, gate_silu, wide);                                \
+    } while (0)
+                if (in_bf16) { if (D == 64) DBK(bf16, 64); else DBK(bf16, 128); }
+                else { if (D == 64) DBK(float, 64); else DBK(float, 128); }
+#undef DBK
+                const int rc = (int)hipGetLastError();
+                if (rc) return rc;
+            }
+        if (fused) return 0;
     } else {
         const long waves = ntok * (2 * G + H);
         dim3 g0((unsigned)((waves + 3) / 4)), b0(4 * WAVE);

@@ -426,22 +426,23 @@ def window_bias_attention(q, k_cache, v_cache, step: StepLayout, block_table,
                            gate=gate, out_dtype=out_dtype, new_rows=new_rows)
 
 
-# Portions of at least this many tokens run in chunks; shorter ones token by token. At 32 tokens
-# of 16 heads of 128 the two are even (31 and 33 us for one row, 36 and 38 for 4, 78 and 77 for
-# 16); at 128 tokens the chunks take 57 us for the scan's 81 (4 rows) and 163 for 227 (16 rows).
+# Portions of at least this many tokens run in blocks of 64; shorter ones token by token. At 64 tokens
+# of 16 heads of 128 the two are even for one row and for 4 (37 and 36 us, 43 and 46; 71 and 119 for 16);
+# at 32 the blocks take 36 us for the scan's 24, at 128 41 for 60 and 50 for 76 (4 rows).
 DELTA_CHUNK_MIN_TOKENS = 64
-# Bytes of chunk operands kept between the two chunk kernels, at most. More tokens go in spans, which
+# Bytes of block operands kept between the block kernels, at most. More tokens go in spans, which
 # are not worth their ends even where a span's operands stay in the last-level cache: the chain
 # fills the chip badly, and starts and stops with each. With 128, 256, 512 MB, 1 and 2 GB, us: one row of
-# 4031 tokens of 16 heads of 128 369, 347, 347, 346, 347, of 60000 5100, 5058, 4953, 4952, 4957;
-# 13 of 1000 884, 822, 779, 779, 778; 64 of 200 of 32 heads 4350, 2618, 1898, 1650, 1651.
-DELTA_CHUNK_WORKSPACE = 1 << 30
+# 4031 tokens of 16 heads of 128 299, 259, 256, 255, 256, of 60000 4074, 3910, 3864, 3712, 3635;
+# 13 of 1000 833, 761, 737, 695, 695; 64 of 200 of 32 heads 2406, 2330, 2325, 1907, 1713.
+DELTA_CHUNK_WORKSPACE = 2 << 30
 # and where there is no room for that, or a capture's pool would hold it for good
 DELTA_CHUNK_LEAST = 128 << 20
 
 
 def _delta_workspace(chunks: int, floats: int, device) -> torch.Tensor:
-    """Room for the operands of up to that many chunks, of so many floats each, and of one at least."""
+    """Room for the operands of up to that many blocks of a row, of so many floats each, and of one at
+    least."""
     def room(limit):
         return torch.empty(max(1, min(chunks, limit // (4 * floats))) * floats, dtype=torch.float32,
                            device=device)
@@ -474,18 +475,19 @@ def gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps: float,
         out = torch.empty(B, S, H * vdim, dtype=out_dtype, device=qkv.device)
         PS = (2 * kv_heads + H) * dim + H + kv_heads
         obuf = prep = ws = None
-        unit = 49 * dim + 16 * vdim + 256          # floats of one 16-token chunk of a head
+        # floats of one 64-token block of a head (csrc/seqmix.hip db_unit)
+        unit = 193 * dim + 64 * vdim + 2560 + dim * vdim
         wide = (dim in (64, 128) and _rows_view(qkv) % 4 == 0 and qkv.data_ptr() % 16 == 0
                 and state.data_ptr() % 16 == 0)
         one = wide and S == 1 and vdim <= 128 and B < 65536
-        if not one:
-            obuf = torch.empty(B, S, H * vdim, dtype=torch.float32, device=qkv.device)
         if one:
             pass                                   # one launch, nothing in between
         elif wide and S >= DELTA_CHUNK_MIN_TOKENS and vdim % 16 == 0:
-            ws = _delta_workspace(-(-S // 16), B * H * unit, qkv.device)
+            ws = _delta_workspace(B * -(-S // 64), H * unit, qkv.device)
         else:
             prep = torch.empty(B, S, PS, dtype=torch.float32, device=qkv.device)
+        if prep is not None or (ws is not None and vdim > 128):
+            obuf = torch.empty(B, S, H * vdim, dtype=torch.float32, device=qkv.device)
         _check(lib.nx_gated_delta(
             _p(qkv), ctypes.c_long(_rows_view(qkv)), _p(beta),
             ctypes.c_long(_rows_view(beta)), _p(a), ctypes.c_long(_rows_view(a)),

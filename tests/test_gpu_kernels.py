@@ -2101,6 +2101,18 @@ def test_attention_decode_values_not_finite(D, gq, dtype, Sq, window, kind):
     _same_but_not_finite(got, want, 2.0 ** (-8.5 if dtype == torch.bfloat16 else -11.5))
 
 
+@pytest.mark.parametrize("S,D,Dv,H,G,per_head,dtype", [
+    (64, 128, 128, 2, 2, False, torch.float32), (65, 64, 144, 2, 1, False, torch.bfloat16),
+    (127, 128, 160, 2, 2, True, torch.float32), (128, 64, 64, 9, 3, False, torch.bfloat16),
+    (129, 128, 32, 2, 2, False, torch.bfloat16), (81, 64, 272, 1, 1, False, torch.float32),
+])
+@pytest.mark.parametrize("room", ["row", "all"])
+def test_gated_delta_blocks(S, D, Dv, H, G, per_head, dtype, room, monkeypatch):
+    """Blocks of 64 tokens at their edges and at those of the groups of 4 and 16 in them, value channels
+    above the 128 that a workgroup norms, one row's block at a time and all at once."""
+    test_gated_delta_chunks(S, D, Dv, H, G, per_head, dtype, "one" if room == "row" else "all", monkeypatch)
+
+
 @pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float32)])
 @pytest.mark.parametrize("part,bad", [("v", 0), ("v", 37), ("v", 99), ("q", 37), ("k", 50), ("a", 64),
                                       ("beta", 15), ("gate", 16)])
