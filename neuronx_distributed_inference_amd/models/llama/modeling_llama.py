@@ -112,7 +112,8 @@ class LlamaDecoderLayer(nn.Module):
     fused_forward = forward        # what modules/fused_layer.py stands for, of these parts
 
     def fused_parts(self):
-        return self.self_attn, self.mlp
+        parts = self._modules
+        return parts["self_attn"], parts["mlp"]
 
 
 class LlamaModel(DecoderModel):

@@ -73,6 +73,12 @@ class DecoderModel(nn.Module):
     """The device graph body. Subclasses implement `build_layers` and
     (optionally) `build_rotary`."""
 
+    # what a program may set; asked in every step, and slow to miss on a module (1.2 us each)
+    _layer_post_fns = None
+    eagle3_capture_layers = None
+    multimodal_ctx = None
+    spec_capture_topk = 0
+
     def __init__(self, config: InferenceConfig):
         super().__init__()
         ec = config.neuron_config

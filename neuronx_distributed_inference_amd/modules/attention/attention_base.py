@@ -204,7 +204,8 @@ class AttentionBase(nn.Module):
                      sequence_parallel: bool = False):
         """Cache rows (keys, values) that the fused front end of whole prompts (see attend_fused)
         writes and reads, None where it does not serve the call."""
-        if phase != PHASE_CTE or not self.qkv_proj.fused:
+        # (asked of every layer before the first one runs: its entry, see fused_layer._sub)
+        if phase != PHASE_CTE or not (self._modules.get("qkv_proj") or self.qkv_proj).fused:
             return None
         norms = self._front_norms(hidden)
         if not (
