@@ -453,7 +453,12 @@ struct TgPlan {
 //   512     34.9 / 38.2   25.5 / 29.7     123 /   105   62.1 / 89.2   442 / 375
 // so up to 256 rows, unless the tiles of more than 128 rows need a second round of the chip, and
 // up to 512 rows where the tiles of the outputs alone leave CUs idle. Parts of K fill the 256 CUs
-// once, each with 2 chunks or more.
+// once, each with 4 chunks or more, and 6 where there are more than 8 of them: a part is as many
+// bytes to write and to read as it has of weights at 128 rows and 4 chunks. Product and the norm
+// that adds up, with 2 chunks or more / so: 93 rows (2048, 2048) 15.2 / 12.9 us, 128 rows
+// (1024, 2048) 14.2 / 12.2, 64 rows (1024, 3072) 9.9 / 9.4, 256 rows (1024, 1024) 13.1 / 10.9,
+// 1 row (2048, 1024) 6.5 / 6.0; 128 rows (1024, 4096) in 16 / 10 / 8 parts 15.5 / 14.4 / 14.6,
+// 256 rows 15.0 / 14.5 / 16.0.
 // From 128 rows on what bounds them is what a CU takes in, x and w together: 40 to 43 GB/s in every
 // tile tried (chunks of x laid out in a row changed nothing, deeper rings of either no more), so a
 // tile of 192 rows, which reads w once for them, and x apart from w in time: 129 to 192 rows
@@ -500,7 +505,7 @@ TgPlan tg_plan(long M, long N, long K, bool glu, bool whole) {
     const long tiles = (M + p.bm - 1) / p.bm * ((N + p.bn - 1) / p.bn);
     if (M > 128 && tiles > 256) return p;
     if (M > 256 && (tiles > 128 || glu)) return p;
-    p.splits = glu ? 1 : (int)std::max(1L, std::min({256 / tiles, K / 128, 16L}));
+    p.splits = glu ? 1 : (int)std::max(1L, std::min({256 / tiles, std::max(std::min(8L, K / 256), K / 384), 16L}));
     return p;
 }
 
