@@ -3185,18 +3185,20 @@ __global__ void gated_rmsnorm_kernel(const float* __restrict__ o, const T* __res
 
 // ---- the recurrence and its norm for one token a row, all in one launch
 // Bound by the state, once in and once out. A workgroup per (head, row): its 8 waves have the whole
-// state of the head (D <= 128, Dv <= 128) on the way before they prepare q, k and the decays (each
-// 16 lanes for themselves, 8 key channels a lane, four value channels a wave at a time), so the
-// small chains of the preparation hide behind it; the norm over the value channels goes through
-// LDS. 48 rows of 16 heads of 128 x 128 (101 MB): 26 us; the three kernels above took 56. The state
+// state of the head (D <= 128, Dv <= 128) on the way before they prepare q and k (each 16 lanes
+// for themselves, 8 key channels a lane, four value channels a wave at a time), so the small chains
+// of the preparation hide behind it; the norm over the value channels goes through LDS. 48 rows of
+// 16 heads of 128 x 128 (101 MB): 26 us; the three kernels above took 56. The state
 // passes the caches by, which nothing reads before the next token and which others' weights want: 100
 // rows of 16 heads 51.4 -> 47.6, of 32 91.7 -> 83.3, 48 of 32 47 -> 43; in a model of four such
-// layers (48 rows) 493 -> 469 a step.
+// layers (48 rows) 493 -> 469 a step. The decays are two waves' work, a key channel a thread, and
+// not every 16 lanes' for themselves: 79 registers a lane for 90, with which three workgroups fit a
+// CU for two (768 workgroups are one round of the chip): 27.8 -> 21.5 us, the step 469 -> 448.
 // With TAPS the short convolution and silu of q, k and v come first, of the raw projections (in T)
 // and the carried tail, a channel a thread, where every head has a q and k of its own: q, k and v are
-// neither written nor read in 32 bits. The same 48 rows, 4 taps: 5.4 + 26.6 us apart, 30.0 so.
+// neither written nor read in 32 bits. The same 48 rows, 4 taps: 5.4 + 26.6 us apart, 30.0 so (before the decays were shared).
 template <typename T, int D, int TAPS>
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(512, 6)
 delta_step_kernel(const std::conditional_t<(TAPS > 0), T, float>* __restrict__ qkv, long cstride,
                   const float* __restrict__ cw, float* __restrict__ tail, const T* __restrict__ beta,
                   long bstride, const T* __restrict__ a, long astride,
@@ -3208,6 +3210,7 @@ delta_step_kernel(const std::conditional_t<(TAPS > 0), T, float>* __restrict__ q
     constexpr int F = D / 64, NI = 4;            // float4s of a lane in a state row; rows of a lane
     __shared__ float os[32 * NI];
     __shared__ __attribute__((aligned(16))) float cs[TAPS > 0 ? 2 * D + 128 : 4];   // q, k, v
+    __shared__ __attribute__((aligned(16))) float ds[D];                            // decays
     const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
     const int slot = seq[b], p = pos[b];
     T* op = out + ((long)b * H + h) * Dv;
@@ -3245,20 +3248,19 @@ delta_step_kernel(const std::conditional_t<(TAPS > 0), T, float>* __restrict__ q
         if constexpr (TAPS == 0) v[i] = qkv[(long)b * cstride + 2L * G * D + (long)h * Dv + r];
     }
     float4 q[F], k[F], dec[F];
-    const T* ap = a + (long)b * astride + (per_head ? h : (long)h * D + part * 4);
-    const float* bp = dt_bias + (per_head ? h : h * D + part * 4);
-    float av[4 * F], bv[4 * F];
+    // decays: a key channel a thread of the last two waves
+    const int dch = tid - 384;
+    float av = 0.f, bv = 0.f;
+    if (dch >= 0 && dch < D) {
+        av = ldf<T>(a + (long)b * astride + (per_head ? h : (long)h * D + dch));
+        bv = dt_bias[per_head ? h : h * D + dch];
+    }
 #pragma unroll
     for (int f = 0; f < F; ++f) {
         if constexpr (TAPS == 0) {
             const float* qp = qkv + (long)b * cstride + (long)g * D + part * 4;
             q[f] = *reinterpret_cast<const float4*>(qp + f * 64);
             k[f] = *reinterpret_cast<const float4*>(qp + (long)G * D + f * 64);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            av[4 * f + e] = ldf<T>(ap + (per_head ? 0 : f * 64 + e));
-            bv[4 * f + e] = bp[per_head ? 0 : f * 64 + e];
         }
     }
     const float bt = sigmoidf_(ldf<T>(beta + (long)b * bstride + h));
@@ -3277,10 +3279,13 @@ delta_step_kernel(const std::conditional_t<(TAPS > 0), T, float>* __restrict__ q
             acc += cwv[R] * ccur;
             cs[tid] = acc * sigmoidf_(acc);
         }
-        // (the state's loads stay in flight over it)
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+    }
+    if (dch >= 0 && dch < D) ds[dch] = expf(neg_rate * softplusf_(av + bv));
+    // (the state's loads stay in flight over it)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if constexpr (TAPS > 0) {
 #pragma unroll
         for (int f = 0; f < F; ++f) {
             q[f] = *reinterpret_cast<const float4*>(cs + part * 4 + f * 64);
@@ -3294,11 +3299,7 @@ delta_step_kernel(const std::conditional_t<(TAPS > 0), T, float>* __restrict__ q
     for (int f = 0; f < F; ++f) {
         sq += q[f].x * q[f].x + q[f].y * q[f].y + q[f].z * q[f].z + q[f].w * q[f].w;
         sk += k[f].x * k[f].x + k[f].y * k[f].y + k[f].z * k[f].z + k[f].w * k[f].w;
-        float* d = &dec[f].x;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (per_head && (f || e)) d[e] = dec[0].x;
-            else d[e] = expf(neg_rate * softplusf_(av[4 * f + e] + bv[4 * f + e]));
+        dec[f] = *reinterpret_cast<const float4*>(ds + part * 4 + f * 64);
     }
     const float iq = 1.f / sqrtf(part_sum<16>(sq) + 1e-6f) * (1.f / sqrtf((float)D));
     const float ik = 1.f / sqrtf(part_sum<16>(sk) + 1e-6f);
