@@ -325,6 +325,7 @@ WINDOWED = [
     (127, 4, 1, 64, 64, 5, dict(window=64, keep_first=80, r=True)),
     (128, 8, 8, 128, 16, 0, dict(chunk=48, sink=True, gate="head")),
     (300, 16, 4, 128, 64, 0, dict(window=100, keep_first=4, r=True, gate="full")),
+    (77, 6, 2, 64, 16, 40, dict(window=50, gate="full")),
     (65, 16, 1, 64, 24, 611, dict(window=1, slopes=True, q_temp=(0.3, 64))),
     (130, 6, 2, 128, 16, 70, dict(window=130, keep_first=64, chunk=90, softcap=20.0, r=True)),
     (64, 2, 2, 64, 64, 1000, dict(softcap=5.0, sink=True, slopes=True)),
