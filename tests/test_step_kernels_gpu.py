@@ -1068,3 +1068,21 @@ def test_layers_are_asked_once_a_prompt(moe, monkeypatch):
     with torch.inference_mode():
         lm(input_ids=ids, position_ids=torch.arange(70, device="cuda").repeat(2, 1))
     assert asked == [True]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D", [(1, 32, 8, 1024, 64), (1, 32, 8, 1025, 64), (1, 32, 8, 2048, 128),
+                                          (3, 12, 3, 1791, 64), (100, 3, 3, 70, 64), (2, 8, 1, 2060, 128)])
+def test_prompts_of_one_round_of_workgroups(B, Hq, Hkv, S, D):
+    """256 workgroups, 264, 512, 504 of 9 heads, more heads than CUs, 258 of 2 heads: every row of the
+    prompts, against 32-bit products: the result's rounding (2^-9) and as much for P's 16 bits."""
+    g = torch.Generator(device="cuda").manual_seed(S)
+    q, k, v = (torch.randn(B, h, S, D, device="cuda", generator=g).bfloat16() for h in (Hq, Hkv, Hkv))
+    out = torch.full_like(q, float("nan"))
+    ops._C.flash_prefill(out, q, k, v, D ** -0.5, 0, None)
+    seen = torch.ones(S, S, dtype=torch.bool, device="cuda").tril()
+    for b in range(B):
+        kk, vv = (t[b].float().repeat_interleave(Hq // Hkv, 0) for t in (k, v))
+        p = (q[b].float() @ kk.transpose(1, 2).contiguous() * D ** -0.5).masked_fill(~seen, float("-inf"))
+        want = torch.softmax(p, -1) @ vv
+        err = (out[b].float() - want).norm(dim=-1) / want.norm(dim=-1)
+        assert out[b].isfinite().all() and err.max() < 2.0 ** -7 and err.square().mean().sqrt() < 2.0 ** -8
