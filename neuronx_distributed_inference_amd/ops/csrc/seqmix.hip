@@ -436,22 +436,23 @@ __global__ void __launch_bounds__(LN_THREADS) stream_step_kernel(const StreamArg
 }
 
 // ------------------------------------------------------------ paged KV write
-template <typename T>
+// T: an element, or 16 bytes of them where rows, strides and caches allow it (4000 tokens of 4 + 4 heads
+// of 128, 16 MB moved: 12.6 -> 5.7 us); I: of as many as there are.
+template <typename T, typename I>
 __global__ void paged_kv_write_kernel(T* __restrict__ kc, T* __restrict__ vc,
                                       const T* __restrict__ k, long kstride,
                                       const T* __restrict__ v, long vstride,
-                                      const int* __restrict__ slots, long N, int GDk, int GDv,
+                                      const int* __restrict__ slots, I total, int GDk, int GDv,
                                       long nslots) {
-    const int per = GDk + GDv;
-    const long total = N * per;
-    for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-         idx += (long)gridDim.x * blockDim.x) {
-        const long tok = idx / per;
-        const int e = idx % per;
+    const I per = GDk + GDv;
+    for (I idx = (I)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
+         idx += (I)gridDim.x * blockDim.x) {
+        const I tok = idx / per;
+        const int e = (int)(idx - tok * per);
         const int s = slots[tok];
         if (s < 0 || s >= nslots) continue;
-        if (e < GDk) kc[(long)s * GDk + e] = k[tok * kstride + e];
-        else vc[(long)s * GDv + (e - GDk)] = v[tok * vstride + (e - GDk)];   // GDv = 0: no V
+        if (e < GDk) kc[(long)s * GDk + e] = k[(long)tok * kstride + e];
+        else vc[(long)s * GDv + (e - GDk)] = v[(long)tok * vstride + (e - GDk)];   // GDv = 0: no V
     }
 }
 
@@ -6273,13 +6274,16 @@ int nx_paged_kv_write(void* kc, void* vc, const void* k, long kstride, const voi
                       long nslots, hipStream_t st) {
     const long total = N * (GDk + GDv);
     if (total <= 0) return 0;
-    dim3 grid(grid_for(total, 256)), block(256);
-    if (is_bf16) paged_kv_write_kernel<bf16><<<grid, block, 0, st>>>(
-        (bf16*)kc, (bf16*)vc, (const bf16*)k, kstride, (const bf16*)v, vstride, slots, N, GDk,
-        GDv, nslots);
-    else paged_kv_write_kernel<float><<<grid, block, 0, st>>>(
-        (float*)kc, (float*)vc, (const float*)k, kstride, (const float*)v, vstride, slots, N,
-        GDk, GDv, nslots);
+    const int n = is_bf16 ? 8 : 4;                        // of 16 bytes
+    const bool wide = GDk % n == 0 && GDv % n == 0 && kstride % n == 0 && (GDv == 0 || vstride % n == 0) &&
+                      (((uintptr_t)kc | (uintptr_t)k | (GDv ? (uintptr_t)vc | (uintptr_t)v : 0)) % 16) == 0;
+#define PKW(T, I, M) paged_kv_write_kernel<T, I><<<dim3(grid_for(total / M, 256)), dim3(256), 0, st>>>( \
+        (T*)kc, (T*)vc, (const T*)k, kstride / M, (const T*)v, vstride / M, slots, (I)(total / M), GDk / M, \
+        GDv / M, nslots)
+    if (wide && total / n < (1L << 31)) PKW(uint4, unsigned, n);
+    else if (is_bf16) PKW(bf16, long, 1);
+    else PKW(float, long, 1);
+#undef PKW
     return (int)hipGetLastError();
 }
 

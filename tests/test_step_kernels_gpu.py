@@ -1086,3 +1086,28 @@ def test_prompts_of_one_round_of_workgroups(B, Hq, Hkv, S, D):
         want = torch.softmax(p, -1) @ vv
         err = (out[b].float() - want).norm(dim=-1) / want.norm(dim=-1)
         assert out[b].isfinite().all() and err.max() < 2.0 ** -7 and err.square().mean().sqrt() < 2.0 ** -8
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,G,Dk,Dv,off,values", [
+    (1, 1, 8, 8, 0, True), (700, 4, 128, 128, 0, True), (33, 2, 64, 64, 3, True), (70, 3, 12, 20, 0, True),
+    (5, 1, 576, 0, 8, False), (9, 1, 7, 0, 0, False), (300, 2, 16, 32, 16, True)])
+def test_paged_rows_are_written(N, G, Dk, Dv, off, values, dtype):
+    """Whole 16 bytes and elements, rows that start off 16 bytes, no values, tokens without a slot:
+    bit for bit."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    g = torch.Generator(device="cuda").manual_seed(N)
+    rows = torch.randn(N, off + G * (Dk + Dv) + 8, device="cuda", generator=g).to(dtype)
+    k, v = rows[:, off:off + G * Dk], rows[:, off + G * Dk:off + G * (Dk + Dv)]
+    kc, vc = (torch.randn(N // 16 + 2, 16, G, d, device="cuda", generator=g).to(dtype) for d in (Dk, Dv))
+    slots = torch.randperm(kc.shape[0] * 16, device="cuda", generator=g)[:N].to(torch.int32)
+    slots[N // 2::3] = -1
+    slots[N // 3:N // 3 + 1] = kc.shape[0] * 16
+    want = kc.clone(), vc.clone()
+    there = (slots >= 0) & (slots < kc.shape[0] * 16)
+    for c, x, d in zip(want, (k, v), (Dk, Dv)):
+        if d:
+            c.view(-1, G * d)[slots[there].long()] = x[there]
+    seqmix.paged_kv_write(kc, vc if values else None, k, v if values else None, slots)
+    assert torch.equal(kc, want[0]) and torch.equal(vc, want[1])
