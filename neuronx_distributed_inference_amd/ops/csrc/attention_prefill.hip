@@ -35,7 +35,7 @@
 //     over 3500 in pages of 64 90 -> 74 us, 64 tokens 24 -> 18. Other page sizes keep the row form.
 //   * Over a cache a wave has priority while it multiplies with V: its SIMD's other wave then
 //     computes exponentials beside it (74.6 -> 72.4 us; 200 tokens over 2000, heads of 64, 29.6 ->
-//     27.7). Prompts from an empty cache gain at 8192 tokens what they lose at 2048 (2 %): without.
+//     27.7). Prompts from an empty cache have it where flash_run says so.
 //
 // Rows with few tiles to share (short chunks over a long cache) are split over the keys as
 // well: fp32 partial sums per split and a small combining kernel.
@@ -150,7 +150,8 @@ struct FaArgs {
 // where the keys are: a row of a linear cache, pages, or pages that hold whole tiles
 enum FaKeys { ROWS, PAGES, TILE_PAGES };
 
-template <typename T, int D, int KEYS, bool HILO>
+// FIRST: a wave has priority while it multiplies with V
+template <typename T, int D, int KEYS, bool HILO, bool FIRST>
 __global__ __launch_bounds__(256, 2) void flash_kernel(
     T* __restrict__ out, const T* __restrict__ q, const T* __restrict__ k,
     const T* __restrict__ v, const FaArgs a) {
@@ -454,7 +455,7 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
             }
         // (this wave before the other of its SIMD: that one's exponentials are to run beside these
         // products, and not both waves' products in turns)
-        if constexpr (HILO) __builtin_amdgcn_s_setprio(1);
+        if constexpr (FIRST) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
             vec8 p[NP];
@@ -495,7 +496,7 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(
             __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
         }
         __builtin_amdgcn_sched_group_barrier(0x008, 4 * NP, 1);
-        if constexpr (HILO) __builtin_amdgcn_s_setprio(0);
+        if constexpr (FIRST) __builtin_amdgcn_s_setprio(0);
     }
 
     // ---- epilogue: rows of 4 channels from 8*(r>>2) + 4*half ----
@@ -624,14 +625,14 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(T* __restrict__ out,
     for (int j = 0; j < PER; ++j) po[j] = VecTraits<T>::from_float(acc[j] * inv);
 }
 
-template <typename T, int D, int KEYS, bool HILO>
+template <typename T, int D, int KEYS, bool HILO, bool FIRST = HILO>
 void flash_launch(torch::Tensor& out, const torch::Tensor& q, const torch::Tensor& k,
                   const torch::Tensor& v, FaArgs& a, hipStream_t stream) {
     const int gq = a.Hq / a.Hkv;
     a.nqt = (int)(((long)gq * a.S + QROWS - 1) / QROWS);
     const size_t lds = 4 * KT * D * 2 + 8 * sizeof(int) + (KEYS == PAGES ? 2 * (KT + 1) * sizeof(int) : 0);
     // a limit of the function on the device at hand, the same in every call
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_kernel<T, D, KEYS, HILO>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&flash_kernel<T, D, KEYS, HILO, FIRST>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const long blocks = (long)a.B * a.Hkv * a.nqt * a.nsplit;
     // Workgroups that are all there at once, two to a CU: the second ones in the other order, so that a
@@ -642,7 +643,7 @@ void flash_launch(torch::Tensor& out, const torch::Tensor& q, const torch::Tenso
     const long heads = (long)a.B * a.Hkv;
     a.turned = !HILO && a.window == 0 && blocks > CUS && blocks <= 2 * CUS ? (int)(CUS / heads) : 0;
     TORCH_CHECK(blocks < (1l << 31), "flash attention: too many query rows");
-    hipLaunchKernelGGL((flash_kernel<T, D, KEYS, HILO>), dim3((unsigned)blocks), dim3(256), lds, stream,
+    hipLaunchKernelGGL((flash_kernel<T, D, KEYS, HILO, FIRST>), dim3((unsigned)blocks), dim3(256), lds, stream,
                        (T*)out.data_ptr(), (const T*)q.data_ptr(), (const T*)k.data_ptr(),
                        (const T*)v.data_ptr(), a);
     HIP_CHECK_KERNEL();
@@ -695,11 +696,19 @@ void flash_run(torch::Tensor& out, const torch::Tensor& q, const torch::Tensor& 
     auto stream = at::hip::getCurrentHIPStream();
     const bool paged = a.block_table != nullptr, tiles = paged && a.block_size % KT == 0;
     const bool extend = a.positions != nullptr;
+    // Priority for prompts: between one and a half and two rounds of workgroups a CU's second place is
+    // filled all the way, and it pays as it does over a cache. Heads of 128, 768 workgroups (3072 tokens,
+    // 3 prompts of 1024) 92.5 -> 88.6 us and 42.4 -> 39.0, 880 118 -> 108, 1024 151 -> 142. 576 and 640 lose
+    // 2 and 4 %, 1256 to 1504 between +1 and -3; heads of 64 lose up to 6. (A kernel of its own: a
+    // branch around it in one kernel costs the others 1 to 3 %.)
+    const long groups = ((long)a.Hq / a.Hkv * a.S + QROWS - 1) / QROWS * a.B * a.Hkv;
+    const bool first = groups > 700 && groups <= 1024;
 #define FA_D(T, D)                                                                        \
     do {                                                                                  \
         if (tiles) flash_launch<T, D, TILE_PAGES, true>(out, q, k, v, a, stream);         \
         else if (paged) flash_launch<T, D, PAGES, true>(out, q, k, v, a, stream);         \
         else if (extend) flash_launch<T, D, ROWS, true>(out, q, k, v, a, stream);         \
+        else if (D == 128 && first) flash_launch<T, 128, ROWS, false, true>(out, q, k, v, a, stream); \
         else flash_launch<T, D, ROWS, false>(out, q, k, v, a, stream);                    \
     } while (0)
 #define FA_GO(T)                                                                          \

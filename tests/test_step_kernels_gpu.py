@@ -1071,10 +1071,11 @@ def test_layers_are_asked_once_a_prompt(moe, monkeypatch):
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,S,D", [(1, 32, 8, 1024, 64), (1, 32, 8, 1025, 64), (1, 32, 8, 2048, 128),
-                                          (3, 12, 3, 1791, 64), (100, 3, 3, 70, 64), (2, 8, 1, 2060, 128)])
+                                          (3, 12, 3, 1791, 64), (100, 3, 3, 70, 64), (2, 8, 1, 2060, 128),
+                                          (3, 32, 8, 1001, 128), (11, 32, 8, 255, 128)])
 def test_prompts_of_one_round_of_workgroups(B, Hq, Hkv, S, D):
-    """256 workgroups, 264, 512, 504 of 9 heads, more heads than CUs, 258 of 2 heads: every row of the
-    prompts, against 32-bit products: the result's rounding (2^-9) and as much for P's 16 bits."""
+    """256 workgroups, 264, 512, 504 of 9 heads, more heads than CUs, 258 of 2 heads, and 768 and 704, of
+    waves with priority: every row of the prompts, against 32-bit products: the result's rounding (2^-9) and as much for P's 16 bits."""
     g = torch.Generator(device="cuda").manual_seed(S)
     q, k, v = (torch.randn(B, h, S, D, device="cuda", generator=g).bfloat16() for h in (Hq, Hkv, Hkv))
     out = torch.full_like(q, float("nan"))
