@@ -21,6 +21,7 @@ from neuronx_distributed_inference_amd.models.model_base import CausalLMBase, De
 from neuronx_distributed_inference_amd.modules.attention.attention_base import AttentionBase
 from neuronx_distributed_inference_amd.modules.mlp import GatedMLP
 from neuronx_distributed_inference_amd.modules.norm import RMSNorm
+from neuronx_distributed_inference_amd.parallel.layers import entry
 
 
 def fuse_qkv_keys(sd: Dict[str, torch.Tensor]) -> Dict[str, torch.Tensor]:
@@ -112,8 +113,7 @@ class LlamaDecoderLayer(nn.Module):
     fused_forward = forward        # what modules/fused_layer.py stands for, of these parts
 
     def fused_parts(self):
-        parts = self._modules
-        return parts["self_attn"], parts["mlp"]
+        return entry(self, "self_attn"), entry(self, "mlp")
 
 
 class LlamaModel(DecoderModel):

@@ -30,7 +30,7 @@ from neuronx_distributed_inference_amd.modules.attention.gqa import (
 from neuronx_distributed_inference_amd.modules.norm import RMSNorm
 from neuronx_distributed_inference_amd.modules.rope import RotaryEmbedding
 from neuronx_distributed_inference_amd.parallel import state as ps
-from neuronx_distributed_inference_amd.parallel.layers import plain_linear
+from neuronx_distributed_inference_amd.parallel.layers import entry, plain_linear
 
 PHASE_CTE = "context_encoding"
 PHASE_TKG = "token_generation"
@@ -204,8 +204,7 @@ class AttentionBase(nn.Module):
                      sequence_parallel: bool = False):
         """Cache rows (keys, values) that the fused front end of whole prompts (see attend_fused)
         writes and reads, None where it does not serve the call."""
-        # (asked of every layer before the first one runs: its entry, see fused_layer._sub)
-        if phase != PHASE_CTE or not (self._modules.get("qkv_proj") or self.qkv_proj).fused:
+        if phase != PHASE_CTE or not entry(self, "qkv_proj").fused:
             return None
         norms = self._front_norms(hidden)
         if not (

@@ -23,7 +23,7 @@ from neuronx_distributed_inference_amd.modules.attention.attention_base import (
 from neuronx_distributed_inference_amd.modules.attention.gqa import GroupQueryAttentionO
 from neuronx_distributed_inference_amd.modules.mlp import GatedMLP
 from neuronx_distributed_inference_amd.modules.norm import RMSNorm
-from neuronx_distributed_inference_amd.parallel.layers import plain_linear
+from neuronx_distributed_inference_amd.parallel.layers import entry, plain_linear
 
 
 # what the loop does in their place, by heart: a class whose forward was replaced is not plain
@@ -39,15 +39,6 @@ def _plain_norm(norm, h: torch.Tensor) -> bool:
     weight = norm._parameters.get("weight")
     return (_plain(norm, RMSNorm) and weight is not None and weight.dtype == h.dtype
             and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
-
-
-def _sub(module, name: str):
-    """module.name of a part: its entry, not the search through the class that nn.Module's own access
-    begins with (0.1 us for 0.65). Some 130 of them stood before the first layer of a prompt of 4
-    layers, which waits for the host: 93 tokens of a 1B model, alone 527 -> 478 us (the host 341 ->
-    291 us a prompt; one prompt after the other 341 -> 333, the GPU's)."""
-    part = module._modules.get(name)
-    return getattr(module, name) if part is None else part
 
 
 def _own_attend(attn) -> bool:
@@ -77,11 +68,11 @@ def fusable(layers, final_norm, h: torch.Tensor, attention_mask, phase: str) -> 
                 and type(attn).attend_fused is AttentionBase.attend_fused
                 and not _hooked(attn)):
             return False
-        out = _sub(attn, "o_proj")
+        out = entry(attn, "o_proj")
         if not (_plain(out, GroupQueryAttentionO)
-                and plain_linear(_sub(out, "o_proj"), h)
-                and _plain_norm(_sub(layer, "input_layernorm"), h)
-                and _plain_norm(_sub(layer, "post_attention_layernorm"), h)):
+                and plain_linear(entry(out, "o_proj"), h)
+                and _plain_norm(entry(layer, "input_layernorm"), h)
+                and _plain_norm(entry(layer, "post_attention_layernorm"), h)):
             return False
     return True
 
@@ -89,7 +80,7 @@ def fusable(layers, final_norm, h: torch.Tensor, attention_mask, phase: str) -> 
 def _plain_mlp(mlp, x: torch.Tensor) -> bool:
     return (_plain(mlp, GatedMLP) and mlp.fused
             and mlp.act_mul_fused is ops.silu_mul_fused
-            and plain_linear(_sub(mlp, "gate_up_proj"), x) and plain_linear(_sub(mlp, "down_proj"), x))
+            and plain_linear(entry(mlp, "gate_up_proj"), x) and plain_linear(entry(mlp, "down_proj"), x))
 
 
 def _feed_forward(mlp, x: torch.Tensor) -> torch.Tensor:
@@ -121,17 +112,16 @@ def prompt_operands(layers, final_norm, x, cos, kv_mgr, seq_ids):
         attn, mlp = layer.fused_parts()
         if _own_attend(attn) or attn.q_norm is not None or attn.k_norm is not None:
             return None
-        qkv = _sub(attn, "qkv_proj")
+        qkv = entry(attn, "qkv_proj")
         rows = attn.prompt_front(x, cos, kv_mgr, PHASE_CTE, seq_ids)
         if (rows is None or not attn.use_rope or attn.sinks is not None
-                or _hooked(qkv) or not plain_linear(_sub(qkv, "qkv"), x) or not _plain_mlp(mlp, x)):
+                or _hooked(qkv) or not plain_linear(entry(qkv, "qkv"), x) or not _plain_mlp(mlp, x)):
             return None
-        norm = _sub(layer, "post_attention_layernorm")
-        following = _sub(after, "input_layernorm") if after is not None else final_norm
-        # (plain modules: what they hold as their weight is it)
-        weights += [m._parameters["weight"] for m in (
-            _sub(qkv, "qkv"), _sub(_sub(attn, "o_proj"), "o_proj"), norm, _sub(mlp, "gate_up_proj"),
-            _sub(mlp, "down_proj"), following)]
+        norm = entry(layer, "post_attention_layernorm")
+        following = entry(after, "input_layernorm") if after is not None else final_norm
+        weights += [m.weight for m in (
+            entry(qkv, "qkv"), entry(entry(attn, "o_proj"), "o_proj"), norm, entry(mlp, "gate_up_proj"),
+            entry(mlp, "down_proj"), following)]
         weights += rows
         sizes += [attn.num_heads_per_rank, attn.num_kv_heads_per_rank, int(attn.sliding_window)]
         numbers += [norm.variance_epsilon, following.variance_epsilon, float(attn.scale)]

@@ -224,6 +224,26 @@ def _linear(x: torch.Tensor, weight: torch.Tensor,
     return F.linear(x, weight, bias)
 
 
+_GETATTR = nn.Module.__getattr__
+_NONE = object()
+
+
+def entry(module: nn.Module, name: str, default=_NONE):
+    """getattr(module, name[, default]) of a module, without the failing search through the instance and
+    its class that nn.Module's own access begins with: what stands in the instance or on the class (a
+    part that a program replaced, a property) still comes first, and then what is registered. A part
+    0.33 us for 0.57, a name that is not there 0.40 for 0.78; a prompt, which waits for the host, asks
+    for some 20 parts a layer."""
+    own, cls = module.__dict__, type(module)
+    if name not in own and cls.__getattr__ is _GETATTR and not hasattr(cls, name):
+        for kind in ("_modules", "_parameters", "_buffers"):
+            if name in own[kind]:
+                return own[kind][name]
+        if default is not _NONE:
+            return default
+    return getattr(module, name) if default is _NONE else getattr(module, name, default)
+
+
 def plain_linear(mod: nn.Module, x: torch.Tensor) -> bool:
     """Whether calling the module on x is no more than x @ weight^T in 16 bits on the GPU, so that
     a fused kernel may stand for it: no bias, 8-bit weight, tensor parallelism, hook (of its

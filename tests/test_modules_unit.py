@@ -731,3 +731,58 @@ def test_moe_dense_does_not_copy_tokens_per_expert(dtype, monkeypatch):
             got = m._forward_dense_16bit(x, gates)
             tol = 1e-6 if dtype == torch.float32 else 2.0 ** -6
             assert (got - want).float().norm() < tol * want.float().norm()
+
+
+def _replace_part(module, name, part, how):
+    """The ways in which a program puts a part of its own in the place of a registered one."""
+    if how == "property":
+        module.__class__ = type("Own", (type(module),), {name: property(lambda self: part)})
+    elif how == "instance":
+        module.__dict__[name] = part
+    elif how == "deleted":
+        delattr(module, name)
+        setattr(module, name, part)
+    else:
+        module.__class__ = type("Own", (type(module),), {
+            "__getattr__": lambda self, n: part if n == name else torch.nn.Module.__getattr__(self, n)})
+        del module._modules[name]
+
+
+@pytest.mark.parametrize("how", ["property", "instance", "deleted", "getattr"])
+def test_replaced_parts_of_layers_are_seen(how, tiny_llama_config):
+    """What stands in a part's place is what a fused layer asks and a cache reads, as in the module's
+    own forward."""
+    from neuronx_distributed_inference_amd.models.llama.modeling_llama import LlamaForCausalLM
+
+    model = LlamaForCausalLM(tiny_llama_config).model
+    layer, kv, attn = model.layers[0], model.kv_mgr, model.layers[1].self_attn
+    assert layer.fused_parts() == (layer.self_attn, layer.mlp)
+    assert kv.get_cache(0)[0] is kv.k_caches[0]
+    own = lambda x: x  # noqa: E731
+    _replace_part(layer, "mlp", own, how)
+    assert layer.mlp is own and layer.fused_parts()[1] is own
+    caches = [torch.zeros(1, 1, 4, 8), torch.ones(1, 1, 4, 8)]
+    _replace_part(kv, "k_caches", caches, how)
+    assert kv.get_cache(1)[0] is caches[1]
+    front = type("Front", (), {"fused": False})()
+    _replace_part(attn, "qkv_proj", front, how)
+    assert attn.prompt_front(torch.zeros(1, 1, 8), None, kv, "context_encoding", None) is None
+
+
+@pytest.mark.parametrize("kind", ["part", "weight", "buffer", "plain"])
+def test_entry_is_getattr(kind):
+    from neuronx_distributed_inference_amd.parallel.layers import entry
+
+    m = torch.nn.Module()
+    assert entry(m, "x", None) is None and entry(m, "x", 3) == 3
+    with pytest.raises(AttributeError):
+        entry(m, "x")
+    value = {"part": torch.nn.Identity(), "weight": torch.nn.Parameter(torch.zeros(2)),
+             "buffer": torch.zeros(2), "plain": object()}[kind]
+    if kind == "buffer":
+        m.register_buffer("x", value)
+    else:
+        m.x = value
+    assert entry(m, "x") is entry(m, "x", None) is m.x is value
+    m.__dict__["x"] = other = object()
+    assert entry(m, "x") is m.x is other

@@ -1112,3 +1112,43 @@ def test_paged_rows_are_written(N, G, Dk, Dv, off, values, dtype):
             c.view(-1, G * d)[slots[there].long()] = x[there]
     seqmix.paged_kv_write(kc, vc if values else None, k, v if values else None, slots)
     assert torch.equal(kc, want[0]) and torch.equal(vc, want[1])
+
+
+@pytest.mark.parametrize("how", ["property", "instance", "deleted"])
+@pytest.mark.parametrize("rows", [0, 200])
+def test_feed_forwards_of_their_own_are_called(how, rows, monkeypatch):
+    """A layer whose feed-forward a program has replaced, in a prompt and in a step: as the chain of
+    modules, which calls it."""
+    from neuronx_distributed_inference_amd.models import model_base
+    from neuronx_distributed_inference_amd.modules import fused_layer
+
+    monkeypatch.setattr(fused_layer, "PROMPT_ROWS", rows)
+    lm = _small_llama("float16")
+    layer, calls = lm.model.layers[1], []
+    inner = layer.mlp
+
+    def own(x, *a, **kw):
+        calls.append(1)
+        return -2.0 * inner(x, *a, **kw)
+
+    if how == "property":
+        layer.__class__ = type("Own", (type(layer),), {"mlp": property(lambda self: own)})
+    elif how == "instance":
+        layer.__dict__["mlp"] = own
+    else:
+        del layer.mlp
+        layer.mlp = own
+    ids = torch.randint(0, 512, (2, 70), device="cuda")
+    step = torch.randint(0, 512, (2, 1), device="cuda")
+
+    def run():
+        lm.reset()
+        with torch.inference_mode():
+            return (lm(input_ids=ids).logits.float(),
+                    lm(input_ids=step, position_ids=torch.full((2, 1), 70, device="cuda")).logits.float())
+
+    got = run()
+    assert len(calls) == 2
+    monkeypatch.setattr(model_base, "fusable", lambda *a: False)
+    # (16-bit activations of two layers, rounded at other places)
+    assert all((a - b).norm() <= 0.004 * b.norm() for a, b in zip(got, run()))
