@@ -51,6 +51,7 @@ from neuronx_distributed_inference_amd.parallel import state as ps
 from neuronx_distributed_inference_amd.parallel.layers import (
     ColumnParallelLinear,
     ParallelEmbedding,
+    entry,
 )
 
 logger = logging.getLogger("nxdi_amd")
@@ -72,12 +73,6 @@ class ModelOutput:
 class DecoderModel(nn.Module):
     """The device graph body. Subclasses implement `build_layers` and
     (optionally) `build_rotary`."""
-
-    # what a program may set; asked in every step, and slow to miss on a module (1.2 us each)
-    _layer_post_fns = None
-    eagle3_capture_layers = None
-    multimodal_ctx = None
-    spec_capture_topk = 0
 
     def __init__(self, config: InferenceConfig):
         super().__init__()
@@ -236,7 +231,7 @@ class DecoderModel(nn.Module):
         """Whether ops.step_start makes what comes before the first layer's attention: nothing but
         the plain modules would, and the layers run fused."""
         emb, rot = self.embed_tokens, self.rotary
-        mm = getattr(self, "multimodal_ctx", None)
+        mm = entry(self, "multimodal_ctx", None)
         if (mm and phase == PHASE_CTE) or getattr(self, "_cos_sin_fn", None) is not None:
             return False
         if (self._own("embed") or self._own("prepare_hidden")
@@ -266,8 +261,8 @@ class DecoderModel(nn.Module):
                               rot._cos_cached, rot._sin_cached, norm.weight, norm.variance_epsilon)
 
     def _may_fuse(self) -> bool:
-        return (not getattr(self, "_layer_post_fns", None)
-                and not getattr(self, "eagle3_capture_layers", None)
+        return (not entry(self, "_layer_post_fns", None)
+                and not entry(self, "eagle3_capture_layers", None)
                 and not self._own("before_layer_run")
                 and not coarse_rows(self.dtype, getattr(self.kv_mgr, "dtype", self.dtype)))
 
@@ -338,7 +333,7 @@ class DecoderModel(nn.Module):
             self.ec.sequence_parallel_enabled
             and phase == PHASE_CTE and tp > 1 and S % tp == 0 and S >= tp
         )
-        post_fns = getattr(self, "_layer_post_fns", None)
+        post_fns = entry(self, "_layer_post_fns", None)
         runs = self.layer_runs()
         fused = [layer for _, layer in runs]
         may_fuse = not sp_active and self._may_fuse()
@@ -352,7 +347,7 @@ class DecoderModel(nn.Module):
         # multimodal splice (llava/pixtral pattern): projected vision
         # features replace the image-placeholder token embeddings. The mask
         # derives from input_ids, so bucket padding is handled for free.
-        mm = getattr(self, "multimodal_ctx", None)
+        mm = entry(self, "multimodal_ctx", None)
         if mm and phase == PHASE_CTE and not sp_active and start is None:
             # one splice per modality: [(placeholder_token_id, features), ...]
             # (single image/videos: qwen2-vl passes both in one prefill)
@@ -405,7 +400,7 @@ class DecoderModel(nn.Module):
                 h = post_fns[li](h, input_ids, phase)
             # EAGLE-3 conditions the draft on SEVERAL target layers'
             # hiddens (ref model_base.py:1402-1437: 3 layers concatenated)
-            cap = getattr(self, "eagle3_capture_layers", None)
+            cap = entry(self, "eagle3_capture_layers", None)
             if cap and li in cap:
                 if li == cap[0]:
                     self.eagle3_hiddens = {}
@@ -469,7 +464,7 @@ class DecoderModel(nn.Module):
         # target_probs flow, model_base.py:1678-1759); stored as an
         # attribute so FusedSpeculationModel can read it inside the same
         # graph capture (same pattern as last_hidden)
-        if getattr(self, "spec_capture_topk", 0):
+        if entry(self, "spec_capture_topk", 0):
             from neuronx_distributed_inference_amd.parallel.ops import (
                 distributed_topk,
             )

@@ -786,3 +786,24 @@ def test_entry_is_getattr(kind):
     assert entry(m, "x") is entry(m, "x", None) is m.x is value
     m.__dict__["x"] = other = object()
     assert entry(m, "x") is m.x is other
+
+
+@pytest.mark.parametrize("name", ["_layer_post_fns", "eagle3_capture_layers", "multimodal_ctx",
+                                  "spec_capture_topk"])
+def test_what_a_program_sets_on_a_model_is_kept(name, tiny_llama_config):
+    """A module, a weight and a buffer of these names read back as themselves; a model that nothing was
+    set on has none of them."""
+    from neuronx_distributed_inference_amd.models.llama.modeling_llama import LlamaForCausalLM
+
+    model = LlamaForCausalLM(tiny_llama_config).model
+    assert not hasattr(model, name)
+    assert model._may_fuse()
+    setattr(model, name, module := torch.nn.ModuleDict({"0": torch.nn.Identity()}))
+    assert getattr(model, name) is module and name in dict(model.named_children())
+    assert model._may_fuse() == (name not in ("_layer_post_fns", "eagle3_capture_layers"))
+    delattr(model, name)
+    setattr(model, name, weight := torch.nn.Parameter(torch.zeros(1)))
+    assert getattr(model, name) is weight
+    delattr(model, name)
+    model.register_buffer(name, buffer := torch.ones(1))
+    assert getattr(model, name) is buffer and name in dict(model.named_buffers())
