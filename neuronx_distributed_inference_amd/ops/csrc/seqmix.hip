@@ -2446,8 +2446,12 @@ gated_delta_kernel(const float* __restrict__ qkv, long cstride, const float* __r
 // 4000 tokens of 16 heads of 128, us: (1) 100, its phases one after the other in 16 waves of a CU; (2)
 // 117, 3600 cycles a block of which the matrix cores have 2050; (3) 59, 173 MB and 17 us of products. In
 // blocks of 16 tokens with the read-out on the chain 125 + 228, and 16 the norm. 64 tokens 37 (29), 256
-// 47 (43), 512 55 (62), 16 rows of 100 113 (140): a few tokens' wait is longer now. Error against 64 bits
-// 4.2e-7 (3.5e-7, the scan 3.0e-7).
+// 47 (43), 512 55 (62), 16 rows of 100 113 (140): a few tokens' wait is longer now.
+// Every sum begins at 0 and what it is added to, the larger one, comes last: U0 and the state and the right
+// sides take one rounding for a block's product and not one for each step of it, and long sums run in
+// two or four. Error against 64 bits of 64 tokens, of 1000 and of 4000, result / state: 2.0 / 2.0e-7, 2.4 /
+// 2.3, 2.4 / 2.2; with chunks of 16 tokens 2.0 / 2.1, 2.4 / 2.4, 2.4 / 2.4, token by token 1.9 / 2.0, 2.3 / 2.5,
+// 2.3 / 2.3; with sums onto the larger value 2.8 / 3.0, 3.3 / 3.2, 3.3 / 3.0.
 #define DB_T 64
 typedef float dc_f32x4 __attribute__((ext_vector_type(4)));
 
@@ -2462,8 +2466,8 @@ template <int D> constexpr int db_lds() {        // bytes of delta_block_kernel'
 }
 
 // e^x, and log(1 + e^x) as max(x, 0) + 2 atanh(z / (2 + z)) with z = e^-|x|, to one or two units of
-// the last place: the decays' error is that of expf and log1pf (3.0e-7 over rates of 1 to 16)
-// in a fifth of their instructions
+// the last place, in a fifth of the instructions of expf and log1pf: with those the result's and the
+// state's errors above are the same to three digits, and 4000 tokens take 282 us for 267
 DEV float exp_near(float x) {
     if (!(fabsf(x) < 80.f)) return expf(x);
     const float y = x * 1.44269502f, r = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269502f, -y));
@@ -2743,16 +2747,16 @@ delta_block_kernel(const float* __restrict__ qkv, long cstride, const T* __restr
             for (int t = 0; t < 16; ++t) x[t] = col[t * step];
 #pragma unroll
             for (int t = 0; t < 16; ++t) {
-                float v = x[t];
+                float v = 0.f;
 #pragma unroll
                 for (int s = 0; s < t; s += 4) {
                     const float4 l4 = *reinterpret_cast<const float4*>(L + t * 20 + s);
-                    v -= l4.x * x[s];
-                    if (s + 1 < t) v -= l4.y * x[s + 1];
-                    if (s + 2 < t) v -= l4.z * x[s + 2];
-                    if (s + 3 < t) v -= l4.w * x[s + 3];
+                    v += l4.x * x[s];
+                    if (s + 1 < t) v += l4.y * x[s + 1];
+                    if (s + 2 < t) v += l4.z * x[s + 2];
+                    if (s + 3 < t) v += l4.w * x[s + 3];
                 }
-                x[t] = bt[t] * v;
+                x[t] = bt[t] * (x[t] - v);
             }
 #pragma unroll
             for (int t = 0; t < 16; ++t) col[t * step] = x[t];
@@ -2765,7 +2769,7 @@ delta_block_kernel(const float* __restrict__ qkv, long cstride, const T* __restr
                 const int pair = wid % 6, i = pair < 1 ? 1 : pair < 3 ? 2 : 3, j = pair - i * (i - 1) / 2;
                 const float* A = (wid < 6 ? ks : qs) + (i * 16 + r16) * RS + q4 * 4;
                 const float* B = ds + (j * 16 + r16) * RS + q4 * 4;
-                dc_f32x4 c[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+                dc_f32x4 c[4] = {};
 #pragma unroll
                 for (int kk = 0; kk < D / 16; ++kk) {
                     dc_f32x4 x = *reinterpret_cast<const dc_f32x4*>(A + kk * 16);
@@ -2774,9 +2778,9 @@ delta_block_kernel(const float* __restrict__ qkv, long cstride, const T* __restr
                         x *= *reinterpret_cast<const dc_f32x4*>(gb + m * D + kk * 16 + q4 * 4);
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        c[r & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[r], y[r], c[r & 1], 0, 0, 0);
+                        c[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[r], y[r], c[r], 0, 0, 0);
                 }
-                c[0] += c[1];
+                c[0] = (c[0] + c[2]) + (c[1] + c[3]);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int t = q4 * 4 + r;
@@ -2802,14 +2806,16 @@ delta_block_kernel(const float* __restrict__ qkv, long cstride, const T* __restr
                     gg *= gb[(i - 1) * D + tile * 16 + r16];
                     X[i] *= gg;
                 }
+                dc_f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int j = 0; j < i; ++j) {
                     const dc_f32x4 m = -*reinterpret_cast<const dc_f32x4*>(
                         Ms + (i * (i - 1) / 2 + j) * 320 + r16 * 20 + q4 * 4);
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        X[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[r], X[j][r], X[i], 0, 0, 0);
+                        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(m[r], X[j][r], sum, 0, 0, 0);
                 }
+                X[i] += sum;
                 if (isw) {                       // (out in whole lines, below)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) ks[(i * 16 + q4 * 4 + r) * RS + tile * 16 + r16] = -X[i][r];
@@ -2952,11 +2958,12 @@ delta_block_scan_kernel(float* __restrict__ ws, float* __restrict__ state,
     read_w(0);
     for (int c = 0; c < nb; ++c) {
         float* o = base + c * hop;
-        dc_f32x4 u[4], v[2][4];
+        dc_f32x4 u[4], v[2][4], more[NB];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) more[i] = dc_f32x4{0.f, 0.f, 0.f, 0.f};
         // this wave's rows of U0 - W S: of 16 tokens and the next, their products in turns
         auto ahead = [&](int t) {
-            u[t] = __builtin_bit_cast(dc_f32x4, __builtin_bit_cast(u32x4, u0) & own[t]);
-            u[t + 1] = __builtin_bit_cast(dc_f32x4, __builtin_bit_cast(u32x4, u0) & own[t + 1]);
+            u[t] = u[t + 1] = dc_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -2964,6 +2971,8 @@ delta_block_scan_kernel(float* __restrict__ ws, float* __restrict__ state,
                     u[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][i][r], s[i][r], u[t], 0, 0, 0);
                     u[t + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t + 1][i][r], s[i][r], u[t + 1], 0, 0, 0);
                 }
+            u[t] += __builtin_bit_cast(dc_f32x4, __builtin_bit_cast(u32x4, u0) & own[t]);
+            u[t + 1] += __builtin_bit_cast(dc_f32x4, __builtin_bit_cast(u32x4, u0) & own[t + 1]);
         };
         auto sums = [&](int t) {
 #pragma unroll
@@ -2980,7 +2989,7 @@ delta_block_scan_kernel(float* __restrict__ ws, float* __restrict__ state,
             for (int r = 0; r < 4; ++r)
 #pragma unroll
                 for (int i = 0; i < NB; ++i)
-                    s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[t][i][r], u[t][r], s[i], 0, 0, 0);
+                    more[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[t][i][r], u[t][r], more[i], 0, 0, 0);
         };
         ahead(0);
         // while the products run
@@ -2998,8 +3007,6 @@ delta_block_scan_kernel(float* __restrict__ ws, float* __restrict__ state,
         ex[(2 * 4 + wid) * 64 + lane] = u[2];
         ex[(3 * 4 + wid) * 64 + lane] = u[3];
         read_k(c, 1);
-#pragma unroll
-        for (int i = 0; i < NB; ++i) s[i] *= gm[i];
         add(0);
         update(0);
         barrier();
@@ -3014,6 +3021,10 @@ delta_block_scan_kernel(float* __restrict__ ws, float* __restrict__ state,
         update(2);
         update(3);
         __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[i][r] = fmaf(s[i][r], gm[i][r], more[i][r]);
         const u32x4 mine = (__builtin_bit_cast(u32x4, u[0]) & own[0]) | (__builtin_bit_cast(u32x4, u[1]) & own[1]) |
                            (__builtin_bit_cast(u32x4, u[2]) & own[2]) | (__builtin_bit_cast(u32x4, u[3]) & own[3]);
         *reinterpret_cast<u32x4*>(o + au) = mine;
@@ -3063,24 +3074,28 @@ delta_block_out_kernel(const float* __restrict__ ws, const int* __restrict__ seq
                 for (int kk = 0; kk < D / 16; ++kk)
                     s[kk] = *reinterpret_cast<const dc_f32x4*>(os + (kk * (Dv / 16) + ct) * 256 + lane * 4);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
+                for (int i = 0; i < 4; ++i)
                     u[i] = *reinterpret_cast<const dc_f32x4*>(
                         ou + (long)i * Dv * 16 + (ct * 16 + r16) * 16 + g * 4);
-                    O[i] = {0.f, 0.f, 0.f, 0.f};
-                }
-                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int kk = 0; kk < D / 16; ++kk) {
-                    dc_f32x4 x[4];
+                for (int i = 0; i < 4; i += 2) {     // (all four at once do not fit the registers)
+                    dc_f32x4 y[2][2];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        x[i] = *reinterpret_cast<const dc_f32x4*>(qs + ((i * (D / 16) + kk) * 64 + lane) * 4);
+                    for (int e = 0; e < 2; ++e) y[e][0] = y[e][1] = dc_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)
+                    for (int kk = 0; kk < D / 16; ++kk) {
+                        dc_f32x4 x[2];
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            O[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i][r], s[kk][r], O[i], 0, 0, 0);
-                    if (kk & 1) __builtin_amdgcn_sched_barrier(0);
+                        for (int e = 0; e < 2; ++e)
+                            x[e] = *reinterpret_cast<const dc_f32x4*>(qs + (((i + e) * (D / 16) + kk) * 64 + lane) * 4);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+#pragma unroll
+                            for (int e = 0; e < 2; ++e)
+                                y[e][r & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e][r], s[kk][r], y[e][r & 1], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) O[i + e] = y[e][0] + y[e][1];
                 }
                 if (!obuf) load_gates();
                 __builtin_amdgcn_sched_barrier(0);
@@ -3090,7 +3105,7 @@ delta_block_out_kernel(const float* __restrict__ ws, const int* __restrict__ seq
 #pragma unroll
                     for (int j = 0; j <= i; ++j)
                         p[j] = *reinterpret_cast<const dc_f32x4*>(op + (i * (i + 1) / 2 + j) * 256 + lane * 4);
-                    dc_f32x4 oo = O[i];
+                    dc_f32x4 oo = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int j = 0; j < i; ++j)  // an update that is not finite is NaN to later tokens
 #pragma unroll
@@ -3118,7 +3133,7 @@ delta_block_out_kernel(const float* __restrict__ ws, const int* __restrict__ seq
                         for (int r = 0; r < 4; ++r)
                             oo = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i][r], u[i][r], oo, 0, 0, 0);
                     }
-                    O[i] = oo;
+                    O[i] += oo;
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }

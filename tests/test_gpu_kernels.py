@@ -2534,3 +2534,41 @@ def test_decode_captured_outside_of_inference_mode(do_sample):
                      position_ids=torch.full((B, 1), at, device=dev))
             tok = out.tokens.clone()
             assert torch.equal(tok.view(-1), out.logits.view(B, -1).argmax(-1))
+
+
+@pytest.mark.parametrize("S,D,Dv,rate", [(64, 128, 128, 0.0), (257, 128, 128, 2.7), (200, 64, 64, 1.0),
+                                         (100, 128, 144, 4.0)])
+def test_gated_delta_blocks_lose_no_precision(S, D, Dv, rate, monkeypatch):
+    """Blocks of 64 tokens against 64 bits, beside the recurrence token by token: result and state are
+    no further off than by a quarter more (sums of 32 bits in another order: 1.06 and 0.97 measured,
+    and 1.5 where a block's products were added to the larger value one by one)."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    dev, f64, B, H = _dev(), torch.float64, 2, 8
+    g = torch.Generator(device=dev).manual_seed(S)
+    r = lambda *s: torch.randn(*s, device=dev, generator=g)  # noqa: E731
+    qkv, beta, a, gate = r(B, S, H * (2 * D + Dv)), r(B, S, H), r(B, S, H * D), r(B, S, H * Dv)
+    A, dt, w, state = torch.linspace(0, rate, H, device=dev), r(H * D) - 4, r(Dv).abs() + 0.5, r(B, H, Dv, D) * 0.3
+    unit = lambda t: t * torch.rsqrt(t.square().sum(-1, keepdim=True) + 1e-6)  # noqa: E731
+    x = qkv.to(f64)
+    q = unit(x[..., :H * D].view(B, S, H, 1, D)) * D ** -0.5
+    k = unit(x[..., H * D:2 * H * D].view(B, S, H, 1, D))
+    v, M = x[..., 2 * H * D:].view(B, S, H, Dv), state.to(f64)
+    dec = torch.exp(-A.to(f64).exp().view(H, 1) * torch.nn.functional.softplus(a.to(f64) + dt.to(f64)).view(B, S, H, D))
+    want = torch.empty(B, S, H, Dv, dtype=f64, device=dev)
+    for t in range(S):
+        M = dec[:, t].unsqueeze(2) * M
+        u = torch.sigmoid(beta[:, t].to(f64)).unsqueeze(-1) * (v[:, t] - (M * k[:, t]).sum(-1))
+        M = M + u.unsqueeze(-1) * k[:, t]
+        want[:, t] = (M * q[:, t]).sum(-1)
+    want = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + 1e-5) * w.to(f64)
+    want = want.view(B, S, H * Dv) * torch.sigmoid(gate.to(f64))
+    pos = torch.arange(3, S + 3, device=dev).expand(B, S)
+    err = []
+    for least in (64, 1 << 30):
+        monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN_TOKENS", least)
+        st = state.clone()
+        out = seqmix.gated_delta_rule(qkv, beta, a, dt, A, gate, w, 1e-5, st,
+                                      seqmix.StepLayout(pos, torch.arange(B, device=dev)), H, D, Dv)
+        err.append([float((got.to(f64) - ref).norm() / ref.norm()) for got, ref in ((out, want), (st, M))])
+    assert all(got <= 1.25 * ref for got, ref in zip(*err)), err
