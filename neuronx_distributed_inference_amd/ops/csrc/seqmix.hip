@@ -2413,13 +2413,403 @@ gated_delta_kernel(const float* __restrict__ qkv, long cstride, const float* __r
     }
 }
 
-// ---- the same recurrence in blocks of 64 tokens, matrix cores in 32 bits
+// ---- the same recurrence in chunks of 16 tokens, matrix cores in 32 bits
 // Portions of several tokens: the scan above is a chain of two lane reductions a token (0.32 us,
-// 128 of 256 CUs for one prompt of 16 heads). With Gam_t the product of the decays from the block's
-// start to t, Gam_{s,t} that from after s to t, and S0 the state at the start, the block is
+// 128 of 256 CUs for one prompt of 16 heads). With Gam_t the product of the decays from the chunk's
+// start to t, Gam_{s,t} that from after s to t, and S0 the state at the start, the chunk is
 //   (I + L) U = beta (V - (Gam k) S0),  L_ts = beta_t k_t' diag(Gam_{s,t}) k_s   (s < t)
 //   O = (Gam q) S0 + P U,               P_ts = q_t' diag(Gam_{s,t}) k_s          (s <= t)
-//   S = diag(Gam_64) S0 + sum_s (Gam_{s,64} k_s) u_s'
+//   S = diag(Gam_16) S0 + sum_s (Gam_{s,16} k_s) u_s'
+// All but U, O and S is independent of the state:
+// (1) delta_chunk_kernel, a workgroup per (chunk, head): unit q and k, decays, the products
+//     (running ones, never a quotient or an exponential of a difference: strong decays go to
+//     zero as they do in the scan), L, P, and W = (I+L)^-1 beta Gam k, U0 = (I+L)^-1 beta V by
+//     forward substitution, a thread per column. It reads the projections itself: no prep pass.
+// (2) delta_chunk_scan_kernel, a workgroup per (row, head, 16 value channels): the chain over
+//     chunks, U = U0 - W S0 and so on, three products of 16x16 and D on 16x16x4 fp32 matrix
+//     instructions (the scan's precision; 16-bit parts would need six products). Waves split the
+//     D rows of the state, which stay in registers: the C layout of its update is the B layout
+//     of the next product when the key channels of A are taken in the same order. One LDS
+//     exchange and one barrier a chunk. A fifth wave reads the outputs out, off the chain; a
+//     sixth pulls the operands into L2 eight chunks ahead, the others into registers three ahead.
+// The head is the fastest grid index of (2): the 8 workgroups that read a head's W, q, k share an
+// XCD's L2. Chunks go through a workspace of bounded size, a span of tokens at a time.
+// For portions where the blocks below leave most CUs without work, or would work on padding for a
+// quarter of their time (the rule and both sides' times: ops/seqmix.py, delta_unit_tokens). A chunk is
+// a workgroup of 4 waves and its chain 0.9 us. Prep pass and scan took 1397 us for 4000 tokens of 16
+// heads of 128, these 347. Error against 64 bits: with the blocks' below.
+#define DC_T 16
+#define DC_AHEAD 8     // chunks
+typedef float dc_f32x4 __attribute__((ext_vector_type(4)));
+
+// floats of one (chunk, head): W 16D | Gam q 16D | (Gam k)' D16 | U0' Dv16 | P 256 | Gam_16 D
+__host__ DEV long dc_unit(int D, int Dv) { return 49L * D + 16L * Dv + 256; }
+
+template <typename T, int D>
+__global__ void __launch_bounds__(256)
+delta_chunk_kernel(const float* __restrict__ qkv, long cstride, const T* __restrict__ beta,
+                   long bstride, const T* __restrict__ a, long astride,
+                   const float* __restrict__ dt_bias, const float* __restrict__ a_log,
+                   const int* __restrict__ seq, const int* __restrict__ nvalid,
+                   float* __restrict__ ws, int t_base, int nchunk, int S, int H, int G, int Dv,
+                   int per_head) {
+    constexpr int PC = D / 16;                   // channels of a thread
+    constexpr int KS = DC_T + 1, LS = DC_T + 4;   // rows of L in whole float4s
+    __shared__ __attribute__((aligned(16))) float qs[DC_T * D], ks[DC_T * D], ds[DC_T * D];
+    __shared__ float gam[DC_T * D], kh[D * KS], Ps[DC_T * KS], bs[DC_T];
+    __shared__ __attribute__((aligned(16))) float Ls[DC_T * LS];
+    const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    const int n = nvalid[b], t0 = t_base + chunk * DC_T;
+    if (seq[b] < 0 || t0 >= n) return;           // uniform over the workgroup
+    const int tid = threadIdx.x, tk = tid >> 4, ln = tid & 15, c0 = ln * PC;
+    const int g = h / (H / G);
+    const bool valid = t0 + tk < n;
+    const long row = (long)b * S + min(t0 + tk, n - 1);   // padding repeats the last row: no
+                                                          // branch around a load
+    {
+        float qv[PC], kv[PC], av[PC], bv[PC], sq = 0.f, sk = 0.f;
+        const float* qp = qkv + row * cstride + (long)g * D + c0;
+        const T* ap = a + row * astride + (per_head ? h : (long)h * D + c0);
+        const float* bp = dt_bias + (per_head ? h : h * D + c0);
+#pragma unroll
+        for (int i = 0; i < PC; i += 4) {
+            const float4 x = *reinterpret_cast<const float4*>(qp + i);
+            const float4 y = *reinterpret_cast<const float4*>(qp + (long)G * D + i);
+            qv[i] = x.x; qv[i + 1] = x.y; qv[i + 2] = x.z; qv[i + 3] = x.w;
+            kv[i] = y.x; kv[i + 1] = y.y; kv[i + 2] = y.z; kv[i + 3] = y.w;
+        }
+#pragma unroll
+        for (int i = 0; i < PC; ++i) {
+            av[i] = ldf<T>(ap + (per_head ? 0 : i));
+            bv[i] = bp[per_head ? 0 : i];
+        }
+        const float braw = ldf<T>(beta + row * bstride + h);
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < PC; ++i) {
+            qv[i] = valid ? qv[i] : 0.f;
+            kv[i] = valid ? kv[i] : 0.f;
+            sq += qv[i] * qv[i];
+            sk += kv[i] * kv[i];
+        }
+        const float iq = 1.f / sqrtf(part_sum<16>(sq) + 1e-6f) * (1.f / sqrtf((float)D));
+        const float ik = 1.f / sqrtf(part_sum<16>(sk) + 1e-6f);
+        const float neg_rate = -expf(a_log[h]);
+        float dec = expf(neg_rate * softplusf_(av[0] + bv[0]));
+#pragma unroll
+        for (int i = 0; i < PC; ++i) {
+            if (i > 0 && !per_head) dec = expf(neg_rate * softplusf_(av[i] + bv[i]));
+            av[i] = valid ? dec : 1.f;           // padding: decay 1, q = k = beta = 0
+        }
+#pragma unroll
+        for (int i = 0; i < PC; i += 4) {
+            const int at = tk * D + c0 + i;
+            *reinterpret_cast<float4*>(qs + at) =
+                float4{qv[i] * iq, qv[i + 1] * iq, qv[i + 2] * iq, qv[i + 3] * iq};
+            *reinterpret_cast<float4*>(ks + at) =
+                float4{kv[i] * ik, kv[i + 1] * ik, kv[i + 2] * ik, kv[i + 3] * ik};
+            *reinterpret_cast<float4*>(ds + at) = float4{av[i], av[i + 1], av[i + 2], av[i + 3]};
+        }
+        if (ln == 0) bs[tk] = valid ? sigmoidf_(braw) : 0.f;
+        Ls[tk * LS + ln] = 0.f;
+        Ps[tk * KS + ln] = 0.f;
+    }
+    __syncthreads();
+    if (tid < D) {
+        float p = 1.f;
+#pragma unroll
+        for (int t = 0; t < DC_T; ++t) {
+            p *= ds[t * D + tid];
+            gam[t * D + tid] = p;
+        }
+    }
+    {
+        const int s = tk;                        // 16 lanes carry Gam_{s,t} k_s over t
+        float w[PC];
+#pragma unroll
+        for (int i = 0; i < PC; ++i) w[i] = ks[s * D + c0 + i];
+        for (int t = (tid >> 6) * 4; t < DC_T; ++t) {
+            float al = 0.f, ap = 0.f;
+#pragma unroll
+            for (int i = 0; i < PC; ++i) {
+                if (t > s) w[i] *= ds[t * D + c0 + i];
+                al += ks[t * D + c0 + i] * w[i];
+                ap += qs[t * D + c0 + i] * w[i];
+            }
+            al = part_sum<16>(al);
+            ap = part_sum<16>(ap);
+            if (ln == 0 && t >= s) {
+                Ps[t * KS + s] = ap;
+                if (t > s) Ls[t * LS + s] = al;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < PC; ++i) kh[(c0 + i) * KS + s] = w[i];
+    }
+    __syncthreads();
+    float* o = ws + (((long)b * nchunk + chunk) * H + h) * dc_unit(D, Dv);
+    for (int col = tid; col < D + Dv; col += 256) {
+        const float* vp = qkv + ((long)b * S + t0) * cstride + 2L * G * D + (long)h * Dv + (col - D);
+        float x[DC_T];
+        if (col < D) {
+#pragma unroll
+            for (int t = 0; t < DC_T; ++t) x[t] = ks[t * D + col] * gam[t * D + col];
+        } else {
+#pragma unroll
+            for (int t = 0; t < DC_T; ++t) x[t] = vp[(long)min(t, n - 1 - t0) * cstride];
+#pragma unroll
+            for (int t = 0; t < DC_T; ++t) x[t] = t0 + t < n ? x[t] : 0.f;
+        }
+#pragma unroll
+        for (int t = 0; t < DC_T; ++t) {
+            float v = x[t];
+#pragma unroll
+            for (int s = 0; s < t; s += 4) {
+                const float4 L = *reinterpret_cast<const float4*>(&Ls[t * LS + s]);
+                v -= L.x * x[s];
+                if (s + 1 < t) v -= L.y * x[s + 1];
+                if (s + 2 < t) v -= L.z * x[s + 2];
+                if (s + 3 < t) v -= L.w * x[s + 3];
+            }
+            x[t] = bs[t] * v;
+        }
+        if (col < D) {
+#pragma unroll
+            for (int t = 0; t < DC_T; ++t) o[t * D + col] = x[t];
+        } else {
+            float* u = o + 48L * D + (long)(col - D) * DC_T;
+#pragma unroll
+            for (int t = 0; t < DC_T; t += 4)
+                *reinterpret_cast<float4*>(u + t) = float4{x[t], x[t + 1], x[t + 2], x[t + 3]};
+        }
+    }
+    for (int i = tid; i < DC_T * D; i += 256) {
+        o[16 * D + i] = qs[i] * gam[i];
+        o[32 * D + i] = kh[(i >> 4) * KS + (i & 15)];
+    }
+    o[48L * D + 16L * Dv + tid] = Ps[tk * KS + ln];
+    if (tid < D) o[48L * D + 16L * Dv + 256 + tid] = gam[(DC_T - 1) * D + tid];
+}
+
+template <int D>
+__global__ void __launch_bounds__(6 * WAVE)
+delta_chunk_scan_kernel(const float* __restrict__ ws, float* __restrict__ state,
+                        const int* __restrict__ pos, const int* __restrict__ seq,
+                        const int* __restrict__ nvalid, float* __restrict__ obuf, int t_base,
+                        int nchunk, int S, int H, int Dv) {
+    constexpr int NB = D / 64;                   // 16-row blocks of the state a wave holds
+    __shared__ dc_f32x4 exu[2][4][WAVE], exo[2][4][WAVE];   // parity, wave, lane
+    __shared__ dc_f32x4 scratch[WAVE];
+    const int h = blockIdx.x, col0 = blockIdx.y * 16, b = blockIdx.z;
+    const int slot = seq[b], n = nvalid[b];
+    if (slot < 0 || n <= t_base) return;         // uniform over the workgroup
+    const int nch = min(nchunk, (n - t_base + DC_T - 1) / DC_T);
+    const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long unit = dc_unit(D, Dv);
+    const char* base = reinterpret_cast<const char*>(ws + ((long)b * nchunk * H + h) * unit);
+    const long hop = (long)H * unit * 4;         // bytes from chunk to chunk
+    const unsigned au = (48 * D + (col0 + r16) * 16 + g * 4) * 4;
+    const unsigned ap = (48 * D + 16 * Dv + r16 * 16 + g * 4) * 4;
+    auto barrier = [] {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+
+    if (wid == 5) {
+        // the runner ahead: pulls this workgroup's share of the chunk after next few into L2, so
+        // that the 3 chunks that fit the registers cover what is left of the way. The loads go
+        // to a scratch kilobyte of LDS and nothing waits for them until the end.
+        const unsigned lds = __builtin_amdgcn_readfirstlane(
+            (unsigned)(size_t)(__attribute__((address_space(3))) char*)scratch);
+        for (int c = 0; c <= nch; ++c) {
+            const char* o = base + min(c + DC_AHEAD, nch - 1) * hop;
+            for (int at = blockIdx.y * 1024; at < (int)unit * 4; at += gridDim.y * 1024) {
+                const char* from = o + min(at + lane * 16, (int)unit * 4 - 16);
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                             :: "s"(lds), "v"(from) : "memory", "m0");
+            }
+            __builtin_amdgcn_s_barrier();
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
+    }
+    if (wid == 4) {
+        // the read-out: after barrier c, U of chunk c from exu and O of chunk c - 1 (whose exo
+        // the state waves completed before that barrier) to memory
+        struct Ops {
+            dc_f32x4 u0, p;
+        };
+        auto load = [&](Ops& x, int c) {
+            const char* o = base + min(c, nch - 1) * hop;
+            x.u0 = *reinterpret_cast<const dc_f32x4*>(o + au);
+            x.p = *reinterpret_cast<const dc_f32x4*>(o + ap);
+            asm volatile("" ::: "memory");       // in flight from here on
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        dc_f32x4 uu = {0.f, 0.f, 0.f, 0.f};
+        float* op = obuf + (((long)b * S + t_base + g * 4) * H + h) * Dv + col0 + r16;
+        auto sums = [&](const Ops& cur, int c) {
+            dc_f32x4 u = cur.u0;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) u -= exu[c & 1][w][lane];
+            return u;
+        };
+        auto read_out = [&](const Ops& prev, int c) {
+            dc_f32x4 oo = exo[c & 1][0][lane];
+#pragma unroll
+            for (int w = 1; w < 4; ++w) oo += exo[c & 1][w][lane];
+            if (__any(!((uu[0] + uu[1]) * 0.f + (uu[2] + uu[3]) * 0.f == 0.f))) {
+                // a token whose update is not finite: P is 0 for the tokens before it, but
+                // 0 * NaN is not. Row by row, over the tokens that each one sees
+                for (int w = 0; w < 4; ++w)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float us = __shfl(uu[e], r16 + 16 * w, WAVE);
+                        // (an infinite update makes infinities of both signs in the state)
+                        const float later = us + us * 0.f;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const float ps = __shfl(prev.p[e], g * 4 + r + 16 * w, WAVE);
+                            const int over = g * 4 + r - (w * 4 + e);
+                            if (over >= 0) oo[r] += ps * (over ? later : us);
+                        }
+                    }
+                return oo;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                oo = __builtin_amdgcn_mfma_f32_16x16x4f32(prev.p[r], uu[r], oo, 0, 0, 0);
+            return oo;
+        };
+        // chunks before the last are whole: their stores are unconditional, or the compiler
+        // cannot count them and waits for the stores of the turn before
+        auto step = [&](const Ops& cur, const Ops& prev, int c) {
+            barrier();
+            const dc_f32x4 un = sums(cur, c), oo = read_out(prev, c - 1);
+            float* o = op + (long)(c - 1) * DC_T * H * Dv;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[(long)r * H * Dv] = oo[r];
+            uu = un;
+        };
+        auto last = [&](const Ops& prev) {
+            barrier();
+            const dc_f32x4 oo = read_out(prev, nch - 1);
+            const int left = n - t_base - (nch - 1) * DC_T - g * 4;
+            float* o = op + (long)(nch - 1) * DC_T * H * Dv;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (r < left) o[(long)r * H * Dv] = oo[r];
+        };
+        Ops x0, x1, x2, x3;
+        load(x0, 0);
+        load(x1, 1);
+        load(x2, 2);
+        barrier();
+        uu = sums(x0, 0);
+        for (int c = 1;;) {
+            if (c >= nch) { last(x0); break; }
+            load(x3, c + 2);
+            step(x1, x0, c);
+            if (++c >= nch) { last(x1); break; }
+            load(x0, c + 2);
+            step(x2, x1, c);
+            if (++c >= nch) { last(x2); break; }
+            load(x1, c + 2);
+            step(x3, x2, c);
+            if (++c >= nch) { last(x3); break; }
+            load(x2, c + 2);
+            step(x0, x3, c);
+            ++c;
+        }
+        return;
+    }
+
+    // state waves: NB blocks of 16 rows each, C layout
+    float* st = state + (((long)slot * H + h) * Dv + col0 + r16) * D + wid * (NB * 16) + g * 4;
+    const bool carry = t_base > 0 || pos[(long)b * S] > 0;
+    dc_f32x4 s[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+        s[i] = carry ? *reinterpret_cast<const dc_f32x4*>(st + i * 16) : dc_f32x4{0.f, 0.f, 0.f, 0.f};
+    struct Ops {
+        dc_f32x4 w[NB], q[NB], k[NB], gm[NB], u0;
+    };
+    const unsigned aw = (r16 * D + wid * NB * 16 + g * 4) * 4;
+    const unsigned ak = (32 * D + (wid * NB * 16 + r16) * 16 + g * 4) * 4;
+    const unsigned ag = (48 * D + 16 * Dv + 256 + wid * NB * 16 + g * 4) * 4;
+    auto load = [&](Ops& x, int c) {
+        const char* o = base + min(c, nch - 1) * hop;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            x.w[i] = *reinterpret_cast<const dc_f32x4*>(o + aw + i * 64);
+            x.q[i] = *reinterpret_cast<const dc_f32x4*>(o + aw + 16 * D * 4 + i * 64);
+            x.k[i] = *reinterpret_cast<const dc_f32x4*>(o + ak + i * 1024);
+            x.gm[i] = *reinterpret_cast<const dc_f32x4*>(o + ag + i * 64);
+        }
+        x.u0 = *reinterpret_cast<const dc_f32x4*>(o + au);
+        asm volatile("" ::: "memory");           // in flight from here on
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto step = [&](const Ops& x, int c) {
+        const int par = c & 1;
+        dc_f32x4 u[NB], o[NB], v[4];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) u[i] = o[i] = dc_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+                u[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w[i][r], s[i][r], u[i], 0, 0, 0);
+#pragma unroll
+        for (int i = 1; i < NB; ++i) u[0] += u[i];
+        exu[par][wid][lane] = u[0];
+        barrier();
+#pragma unroll
+        for (int w = 0; w < 4; ++w) v[w] = exu[par][w][lane];
+        // while the sums arrive
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+                o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][r], s[i][r], o[i], 0, 0, 0);
+        const dc_f32x4 uu = x.u0 - ((v[0] + v[1]) + (v[2] + v[3]));
+#pragma unroll
+        for (int i = 0; i < NB; ++i) s[i] *= x.gm[i];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+                s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i][r], uu[r], s[i], 0, 0, 0);
+#pragma unroll
+        for (int i = 1; i < NB; ++i) o[0] += o[i];
+        exo[par][wid][lane] = o[0];
+    };
+    Ops x0, x1, x2, x3;
+    load(x0, 0);
+    load(x1, 1);
+    load(x2, 2);
+    for (int c = 0;;) {
+        load(x3, c + 3);
+        step(x0, c);
+        if (++c >= nch) break;
+        load(x0, c + 3);
+        step(x1, c);
+        if (++c >= nch) break;
+        load(x1, c + 3);
+        step(x2, c);
+        if (++c >= nch) break;
+        load(x2, c + 3);
+        step(x3, c);
+        if (++c >= nch) break;
+    }
+    barrier();                                   // the read-out's last turn
+#pragma unroll
+    for (int i = 0; i < NB; ++i) *reinterpret_cast<dc_f32x4*>(st + i * 16) = s[i];
+}
+
+// ---- and in blocks of 64 tokens, the same equations for t up to 64
 // All but U, O and S is independent of the state:
 // (1) delta_block_kernel, a workgroup of 16 waves per (block, head): unit q and k, decays, the products
 //     (running ones, never a quotient or an exponential of a difference: strong decays go to
@@ -2443,18 +2833,15 @@ gated_delta_kernel(const float* __restrict__ qkv, long cstride, const float* __r
 //     matrix cores for a third of their time, on half of the CUs.
 // The head is the fastest grid index of (2): the 8 workgroups that read a head's W and k share an
 // XCD's L2. Blocks go through a workspace of bounded size, a span of tokens at a time.
-// 4000 tokens of 16 heads of 128, us: (1) 100, its phases one after the other in 16 waves of a CU; (2)
-// 117, 3600 cycles a block of which the matrix cores have 2050; (3) 59, 173 MB and 17 us of products. In
-// blocks of 16 tokens with the read-out on the chain 125 + 228, and 16 the norm. 64 tokens 37 (29), 256
-// 47 (43), 512 55 (62), 16 rows of 100 113 (140): a few tokens' wait is longer now.
+// 4000 tokens of 16 heads of 128, us: (1) 97, its phases one after the other in 16 waves of a CU; (2)
+// 115, 3600 cycles a block of which the matrix cores have 2050; (3) 48, 173 MB and 17 us of products. In
+// chunks of 16 tokens 121 + 224, and 16 the norm.
 // Every sum begins at 0 and what it is added to, the larger one, comes last: U0 and the state and the right
 // sides take one rounding for a block's product and not one for each step of it, and long sums run in
 // two or four. Error against 64 bits of 64 tokens, of 1000 and of 4000, result / state: 2.0 / 2.0e-7, 2.4 /
 // 2.3, 2.4 / 2.2; with chunks of 16 tokens 2.0 / 2.1, 2.4 / 2.4, 2.4 / 2.4, token by token 1.9 / 2.0, 2.3 / 2.5,
 // 2.3 / 2.3; with sums onto the larger value 2.8 / 3.0, 3.3 / 3.2, 3.3 / 3.0.
 #define DB_T 64
-typedef float dc_f32x4 __attribute__((ext_vector_type(4)));
-
 
 // floats of one (block, head): -W 64D | Gam q 64D | (Gam k)' 64D | U' 4 x Dv16 | P 10 x 256 | Gam_64 D |
 // the state at its start. W, q, k, P and the state are in pieces of 16 x 16 as a wave holds them: a
@@ -6500,7 +6887,7 @@ int nx_gated_delta(const float* qkv, long cstride, const void* beta, long bstrid
                    const float* a_log, const float* norm_w, float eps, float* state,
                    const int* pos, const int* seq, const int* nvalid, float* prep, long PS,
                    float* obuf, void* out, int in_bf16, int B, int S, int H, int G, int D,
-                   int Dv, int per_head, int gate_silu, float* ws, long ws_floats,
+                   int Dv, int per_head, int gate_silu, float* ws, long ws_floats, int unit_tokens,
                    hipStream_t st) {
     if (B <= 0 || S <= 0) return 0;
     if (!ws && !prep) {
@@ -6519,9 +6906,33 @@ int nx_gated_delta(const float* qkv, long cstride, const void* beta, long bstrid
     }
     if (D > 256 || H % G != 0 || (!ws && PS < (long)(2 * G + H) * D + H + G)) return -1;
     const long ntok = (long)B * S;
-    if (ws) {
+    if (ws && ((D != 64 && D != 128) || Dv % 16 || cstride % 4)) return -1;
+    if (ws && unit_tokens == DC_T) {
+        // in chunks, as many of them at a time as the workspace holds
+        const long per = (long)B * H * dc_unit(D, Dv);
+        const int span = (int)(ws_floats / per < 1024 ? ws_floats / per : 1024);
+        if (span < 1 || !obuf) return -1;
+        for (int t = 0; t < S; t += span * DC_T) {
+            const int nch = (S - t + DC_T - 1) / DC_T < span ? (S - t + DC_T - 1) / DC_T : span;
+            dim3 ga(nch, H, B), gb(H, Dv / 16, B), blk(256), blk6(6 * WAVE);
+#define DCA(TT, DD) delta_chunk_kernel<TT, DD><<<ga, blk, 0, st>>>( \
+            qkv, cstride, (const TT*)beta, bstride, (const TT*)a, astride, dt_bias, a_log, seq, \
+            nvalid, ws, t, nch, S, H, G, Dv, per_head)
+            if (in_bf16) { if (D == 64) DCA(bf16, 64); else DCA(bf16, 128); }
+            else { if (D == 64) DCA(float, 64); else DCA(float, 128); }
+#undef DCA
+            int rc = (int)hipGetLastError();
+            if (rc) return rc;
+            if (D == 64) delta_chunk_scan_kernel<64><<<gb, blk6, 0, st>>>(
+                ws, state, pos, seq, nvalid, obuf, t, nch, S, H, Dv);
+            else delta_chunk_scan_kernel<128><<<gb, blk6, 0, st>>>(
+                ws, state, pos, seq, nvalid, obuf, t, nch, S, H, Dv);
+            rc = (int)hipGetLastError();
+            if (rc) return rc;
+        }
+    } else if (ws) {
         // in blocks, as many of them and of the rows at a time as the workspace holds
-        if ((D != 64 && D != 128) || Dv % 16 || cstride % 4) return -1;
+        if (unit_tokens != DB_T || (Dv > 128 && !obuf)) return -1;
         const bool fused = Dv <= 128;
         const int lds1 = D == 64 ? db_lds<64>() : db_lds<128>(), lds2 = 4 * DB_T * D * 4 + 2 * 4096 + 16384;
         const int wide = (uintptr_t)out % 16 == 0;

@@ -426,23 +426,48 @@ def window_bias_attention(q, k_cache, v_cache, step: StepLayout, block_table,
                            gate=gate, out_dtype=out_dtype, new_rows=new_rows)
 
 
-# Portions of at least this many tokens run in blocks of 64; shorter ones token by token. At 64 tokens
-# of 16 heads of 128 the two are even for one row and for 4 (37 and 36 us, 43 and 46; 71 and 119 for 16);
-# at 32 the blocks take 36 us for the scan's 24, at 128 41 for 60 and 50 for 76 (4 rows).
+# Portions of at least this many tokens run in chunks of 16 or in blocks of 64, shorter ones token by
+# token. At 32 tokens of 16 heads of 128 the scan and the chunks are even (31 and 33 us for one row, 36
+# and 38 for 4, 78 and 77 for 16), at 64 the chunks take 28 us for the scan's 36, 39 for 46 and 102 for 119.
 DELTA_CHUNK_MIN_TOKENS = 64
-# Bytes of block operands kept between the block kernels, at most. More tokens go in spans, which
+# Bytes of their operands kept between the kernels, at most. More tokens go in spans, which
 # are not worth their ends even where a span's operands stay in the last-level cache: the chain
-# fills the chip badly, and starts and stops with each. With 128, 256, 512 MB, 1 and 2 GB, us: one row of
-# 4031 tokens of 16 heads of 128 299, 259, 256, 255, 256, of 60000 4074, 3910, 3864, 3712, 3635;
-# 13 of 1000 833, 761, 737, 695, 695; 64 of 200 of 32 heads 2406, 2330, 2325, 1907, 1713.
+# fills the chip badly, and starts and stops with each. Blocks with 1 GB and with 2, us: one row of
+# 4000 tokens of 16 heads of 128 248 and 249, of 60000 3675 and 3602, 13 of 1000 683 and 686, 64 of 256 of 32
+# heads 1928 and 1697 (chunks 4960, 780 and 2234 with 1 GB); with 128 MB 4031 tokens take 299.
 DELTA_CHUNK_WORKSPACE = 2 << 30
 # and where there is no room for that, or a capture's pool would hold it for good
 DELTA_CHUNK_LEAST = 128 << 20
 
 
+def _delta_floats(tokens: int, dim: int, vdim: int) -> int:
+    """Floats of a chunk of 16 or a block of 64 tokens of a head (csrc/seqmix.hip dc_unit, db_unit)."""
+    return 49 * dim + 16 * vdim + 256 if tokens == 16 else 193 * dim + 64 * vdim + 2560 + dim * vdim
+
+
+def delta_unit_tokens(rows: int, tokens: int, heads: int, dim: int, vdim: int) -> int:
+    """Whether rows of so many tokens run in chunks of 16 or in blocks of 64, by what the two take (us).
+    Chunks: a start, and the work that is there. Blocks: one at a time on a CU, so rounds of the
+    chip, full or not, and the work, of padding too; a tenth more where the operands go in spans. Chunks /
+    blocks of heads of 128 channels: one row of 64 tokens of 16 heads 27.7 / 34.7, of 128 32 / 39, of 256 41.5 /
+    45.7, of 320 49.4 / 47.4, of 512 61 / 54, of 4000 347 / 248; 2 rows of 200 44.9 / 47.6, of 256 47.8 / 47.3; 8 of
+    64 58.8 / 53.5; 12 of 144 131 / 137; 64 of 80 416 / 491, of 96 472 / 498, of 128 583 / 502. Of 336 shapes
+    of 1 to 64 rows of 64 to 4000 tokens of 16 and 32 heads of 64 and 128 channels, and of 256 value channels, it
+    takes in 10 the one that is slower by 2 to 6 %, else one that is not. (In a capture more shapes go in
+    spans: 7 rows of 333 of 16 heads 168 / 188.)"""
+    pairs, blocks = rows * heads, -(-tokens // 64)
+    chunked = 5 + 0.14 * dim + -(-tokens // 16) * (0.04 + pairs * vdim / 2250)
+    whole = (10.5 + 0.1 * blocks * -(-pairs * vdim // 4096)
+             + vdim * (0.2 * -(-pairs * blocks // 256) + pairs * blocks / 1450))
+    # (also where a capture or a full GPU leaves less: the same sums there)
+    if pairs * blocks * _delta_floats(64, dim, vdim) * 4 > DELTA_CHUNK_WORKSPACE:
+        whole *= 1.1
+    return 16 if chunked < whole else 64
+
+
 def _delta_workspace(chunks: int, floats: int, device) -> torch.Tensor:
-    """Room for the operands of up to that many blocks of a row, of so many floats each, and of one at
-    least."""
+    """Room for the operands of up to that many chunks of all rows or blocks of one, of so many floats
+    each, and of one at least."""
     def room(limit):
         return torch.empty(max(1, min(chunks, limit // (4 * floats))) * floats, dtype=torch.float32,
                            device=device)
@@ -475,18 +500,20 @@ def gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps: float,
         out = torch.empty(B, S, H * vdim, dtype=out_dtype, device=qkv.device)
         PS = (2 * kv_heads + H) * dim + H + kv_heads
         obuf = prep = ws = None
-        # floats of one 64-token block of a head (csrc/seqmix.hip db_unit)
-        unit = 193 * dim + 64 * vdim + 2560 + dim * vdim
+        unit = 0
         wide = (dim in (64, 128) and _rows_view(qkv) % 4 == 0 and qkv.data_ptr() % 16 == 0
                 and state.data_ptr() % 16 == 0)
         one = wide and S == 1 and vdim <= 128 and B < 65536
         if one:
             pass                                   # one launch, nothing in between
         elif wide and S >= DELTA_CHUNK_MIN_TOKENS and vdim % 16 == 0:
-            ws = _delta_workspace(B * -(-S // 64), H * unit, qkv.device)
+            unit = delta_unit_tokens(B, S, H, dim, vdim)
+            floats, units = H * _delta_floats(unit, dim, vdim), -(-S // unit)
+            ws = (_delta_workspace(units, B * floats, qkv.device) if unit == 16 else
+                  _delta_workspace(B * units, floats, qkv.device))
         else:
             prep = torch.empty(B, S, PS, dtype=torch.float32, device=qkv.device)
-        if prep is not None or (ws is not None and vdim > 128):
+        if prep is not None or unit == 16 or (unit == 64 and vdim > 128):
             obuf = torch.empty(B, S, H * vdim, dtype=torch.float32, device=qkv.device)
         _check(lib.nx_gated_delta(
             _p(qkv), ctypes.c_long(_rows_view(qkv)), _p(beta),
@@ -497,7 +524,7 @@ def gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps: float,
             ctypes.c_long(PS), _p(obuf), _p(out),
             _is_bf16(beta), B, S, H, kv_heads, dim, vdim, int(per_head),
             int(gate_act == "silu"), _p(ws), ctypes.c_long(0 if ws is None else ws.numel()),
-            _stream()), "gated_delta_rule")
+            unit, _stream()), "gated_delta_rule")
         return out
     return ref.gated_delta_rule(qkv, beta, a, dt_bias, a_log, gate, norm_w, eps,
                                 state, step.positions, step.seq_ids, kv_heads,

@@ -1532,11 +1532,11 @@ def test_attention_decode_short_rows_of_long_cache(cap, kind, window):
 ])
 @pytest.mark.parametrize("span", ["one", "all"])
 def test_gated_delta_chunks(S, D, Dv, H, G, per_head, dtype, span, monkeypatch):
-    """The delta rule in 16-token chunks, against the recurrence in 64 bits: rows of every length
-    around a chunk, a carried and a fresh state, a row without a slot, heads that share keys,
-    decays from next to none to total, one chunk a span and all in one. Products and sums are
-    32-bit: what a token's result is off by grows with the chain of 128 additions and the
-    16 substitutions, not with the length; 4e-6 (2-norm) is four times what the token-by-token
+    """The delta rule in chunks of 16 tokens (or blocks of 64, see delta_unit_tokens), against the
+    recurrence in 64 bits: rows of every length around a chunk, a carried and a fresh state, a row
+    without a slot, heads that share keys, decays from next to none to total, one chunk a span and
+    all in one. Products and sums are 32-bit: what a token's result is off by grows with the chain of
+    128 additions and the substitutions of a chunk, not with the length; 4e-6 (2-norm) is four times what the token-by-token
     kernel shows. In bf16 the result's own rounding (2^-9) comes on top."""
     from neuronx_distributed_inference_amd.ops import seqmix
 
@@ -2565,6 +2565,7 @@ def test_gated_delta_blocks_lose_no_precision(S, D, Dv, rate, monkeypatch):
     want = want.view(B, S, H * Dv) * torch.sigmoid(gate.to(f64))
     pos = torch.arange(3, S + 3, device=dev).expand(B, S)
     err = []
+    monkeypatch.setattr(seqmix, "delta_unit_tokens", lambda *a: 64)
     for least in (64, 1 << 30):
         monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN_TOKENS", least)
         st = state.clone()
@@ -2572,3 +2573,31 @@ def test_gated_delta_blocks_lose_no_precision(S, D, Dv, rate, monkeypatch):
                                       seqmix.StepLayout(pos, torch.arange(B, device=dev)), H, D, Dv)
         err.append([float((got.to(f64) - ref).norm() / ref.norm()) for got, ref in ((out, want), (st, M))])
     assert all(got <= 1.25 * ref for got, ref in zip(*err)), err
+
+
+@pytest.mark.parametrize("unit", [16, 64])
+@pytest.mark.parametrize("S,D,Dv,H,G,per_head,dtype,units", [
+    (64, 128, 128, 2, 2, False, torch.float32, 1), (65, 64, 144, 2, 1, False, torch.bfloat16, 100),
+    (127, 128, 160, 2, 2, True, torch.float32, 3), (128, 64, 64, 9, 3, False, torch.bfloat16, 3),
+    (257, 128, 32, 2, 2, False, torch.bfloat16, 14), (257, 64, 272, 1, 1, False, torch.float32, 17),
+    (400, 128, 16, 1, 1, True, torch.bfloat16, 100)])
+def test_gated_delta_in_both_units(S, D, Dv, H, G, per_head, dtype, unit, units, monkeypatch):
+    """Chunks and blocks, whichever the sizes would run in, with room for one unit, for some of the 7
+    rows (groups of 3, 3 and 1), for all rows in spans of two blocks and a last one, and for everything."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    monkeypatch.setattr(seqmix, "delta_unit_tokens", lambda *a: unit)
+    monkeypatch.setattr(seqmix, "DELTA_CHUNK_WORKSPACE", 4 * units * H * seqmix._delta_floats(unit, D, Dv))
+    test_gated_delta_chunks(S, D, Dv, H, G, per_head, dtype, "all", monkeypatch)
+
+
+@pytest.mark.parametrize("unit", [16, 64])
+@pytest.mark.parametrize("part,bad", [("v", 0), ("v", 37), ("v", 99), ("q", 37), ("k", 50), ("a", 64),
+                                      ("beta", 15), ("gate", 16)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_gated_delta_units_not_finite(part, bad, value, unit, monkeypatch):
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    monkeypatch.setattr(seqmix, "delta_unit_tokens", lambda *a: unit)
+    for D, dtype in ((128, torch.bfloat16), (64, torch.float32)):
+        test_gated_delta_chunks_not_finite(D, dtype, part, bad, value, monkeypatch)

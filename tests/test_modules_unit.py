@@ -807,3 +807,17 @@ def test_what_a_program_sets_on_a_model_is_kept(name, tiny_llama_config):
     delattr(model, name)
     model.register_buffer(name, buffer := torch.ones(1))
     assert getattr(model, name) is buffer and name in dict(model.named_buffers())
+
+
+@pytest.mark.parametrize("rows,tokens,heads,dim,vdim,unit", [
+    (1, 64, 16, 128, 128, 16), (1, 200, 32, 128, 128, 16), (1, 256, 16, 128, 128, 16),
+    (1, 256, 16, 64, 64, 16), (1, 384, 16, 128, 256, 16), (4, 96, 16, 128, 128, 16),
+    (64, 80, 16, 128, 128, 16), (64, 200, 32, 128, 128, 16), (12, 144, 16, 128, 128, 16),
+    (1, 384, 16, 128, 128, 64), (1, 512, 16, 64, 64, 64), (8, 64, 16, 128, 128, 64),
+    (4, 200, 16, 128, 128, 64), (16, 96, 16, 128, 128, 64), (64, 64, 16, 128, 128, 64),
+    (64, 256, 32, 128, 128, 64), (1, 4000, 16, 128, 128, 64), (1, 60000, 16, 128, 128, 64)])
+def test_delta_rule_runs_in_the_faster_unit(rows, tokens, heads, dim, vdim, unit):
+    """At shapes where one of the two took at least 3 % less."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    assert seqmix.delta_unit_tokens(rows, tokens, heads, dim, vdim) == unit
