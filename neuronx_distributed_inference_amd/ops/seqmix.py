@@ -435,7 +435,7 @@ DELTA_CHUNK_MIN_TOKENS = 64
 # fills the chip badly, and starts and stops with each. Blocks with 1 GB and with 2, us: one row of
 # 4000 tokens of 16 heads of 128 248 and 249, of 60000 3675 and 3602, 13 of 1000 683 and 686, 64 of 256 of 32
 # heads 1928 and 1697 (chunks 4960, 780 and 2234 with 1 GB); with 128 MB 4031 tokens take 299.
-DELTA_CHUNK_WORKSPACE = 2 << 30
+DELTA_CHUNK_WORKSPACE = 1 << 30
 # and where there is no room for that, or a capture's pool would hold it for good
 DELTA_CHUNK_LEAST = 128 << 20
 

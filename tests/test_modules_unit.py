@@ -821,3 +821,27 @@ def test_delta_rule_runs_in_the_faster_unit(rows, tokens, heads, dim, vdim, unit
     from neuronx_distributed_inference_amd.ops import seqmix
 
     assert seqmix.delta_unit_tokens(rows, tokens, heads, dim, vdim) == unit
+
+
+def test_delta_rule_keeps_a_gigabyte_at_most(monkeypatch):
+    """Room for the operands of chunks and blocks: all of them where they fit 1 GB, never more, one at
+    least, and 128 MB in a capture or where that fails."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    asked = []
+
+    def empty(n, **kw):
+        asked.append(4 * n)
+        if full and len(asked) == 1:
+            raise torch.cuda.OutOfMemoryError
+        return n
+
+    monkeypatch.setattr(torch, "empty", empty)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capture)
+    for full, capture, limit in ((False, False, 1 << 30), (True, False, 128 << 20), (False, True, 128 << 20)):
+        for units, floats in ((3, 1000), (10000, 829440), (1, 1 << 29), (1 << 20, 1 << 14)):
+            asked.clear()
+            got = seqmix._delta_workspace(units, floats, "cpu") * 4
+            assert got % (4 * floats) == 0 and got >= 4 * floats
+            assert got == 4 * floats * units or got <= max(limit, 4 * floats) < got + 4 * floats
+            assert got <= max(limit, 4 * floats)
