@@ -1203,11 +1203,11 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, long qstride, const bf16* __r
 //     all rows see whole take no mask.
 //   * The accumulator is rescaled only when a maximum grew by more than 2^8.
 //   * The result is laid into LDS at the end, in 32 bits, and leaves in whole rows, the gate comes
-//     in whole rows ahead of that: 8 bytes from 32 rows at a time took 10 us of 86, and the gate's
-//     division to the last bit, for a result of 16, 3 more.
+//     in whole rows ahead of that: 8 bytes from 32 rows at a time took 10 us of 86. (The hardware's
+//     exponential and reciprocal for the gate's sigmoid save 2 us and give 0 below -87.)
 //   * K is read four products ahead, and a wave has priority while it multiplies with V (86 -> 82).
-// 4000 tokens, 16 heads of 128 on 4 KV heads, window of 1024, log-distance bias, gate: 76 us (window
-// of 64: 26, before 33).
+// 4000 tokens, 16 heads of 128 on 4 KV heads, window of 1024, log-distance bias, gate: 90 -> 82 us (window
+// of 64: 32 -> 28).
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
@@ -1230,9 +1230,6 @@ DEV float wf_half_swap(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
     return __builtin_bit_cast(float, (threadIdx.x & 32) ? r[0] : r[1]);
 }
-
-// (2^-22 off at most near 0 and about |x| 2^-24 away from it: for results of 16 bits)
-DEV float wf_sigmoid(float x) { return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-LOG2E * x)); }
 
 struct WfArgs {
     const bf16* q;
@@ -1573,7 +1570,7 @@ __global__ void __launch_bounds__(256, 2) window_flash_kernel(const WfArgs a) {
             const float gv[4] = {__uint_as_float(gt[i].x << 16), __uint_as_float(gt[i].x & 0xffff0000u),
                                  __uint_as_float(gt[i].y << 16), __uint_as_float(gt[i].y & 0xffff0000u)};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] *= wf_sigmoid(gv[e]);
+            for (int e = 0; e < 4; ++e) v[e] *= sigmoidf_(gv[e]);
         }
         bf16x4_t y;
 #pragma unroll

@@ -1152,3 +1152,20 @@ def test_feed_forwards_of_their_own_are_called(how, rows, monkeypatch):
     monkeypatch.setattr(model_base, "fusable", lambda *a: False)
     # (16-bit activations of two layers, rounded at other places)
     assert all((a - b).norm() <= 0.004 * b.norm() for a, b in zip(got, run()))
+
+
+def test_gate_of_windowed_portions_is_the_plain_sigmoid():
+    """Rows that see one key, with values of 1: the result is the gate's sigmoid, 1 / (1 + exp(-x)) of 32
+    bits rounded once, for every gate of 16 bits in which it is neither 0 nor 1, and for the others."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    S, H, D = 128, 4, 128
+    gate = torch.arange(2 ** 16).to(torch.int16).view(torch.bfloat16).view(1, S, H * D).cuda()
+    kc = torch.randn(S // 16, 16, 1, D, device="cuda").bfloat16()
+    step = seqmix.StepLayout(torch.arange(S, device="cuda").view(1, S), torch.zeros(1, dtype=torch.long, device="cuda"))
+    got = seqmix.paged_attention(torch.randn(1, S, H * D, device="cuda").bfloat16(), kc, torch.ones_like(kc), step,
+                                 torch.arange(S // 16, device="cuda").view(1, -1).int(), D ** -0.5, H, window=1,
+                                 gate=gate)
+    want = (1 / (1 + torch.exp(-gate.float()))).bfloat16()
+    same = (got == want) | (got.isnan() & want.isnan())
+    assert same.all(), (int((~same).sum()), gate[~same][:8], got[~same][:8], want[~same][:8])
