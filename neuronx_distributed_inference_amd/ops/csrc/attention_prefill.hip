@@ -627,7 +627,7 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(T* __restrict__ out,
 
 template <typename T, int D, int KEYS, bool HILO, bool FIRST = HILO>
 void flash_launch(torch::Tensor& out, const torch::Tensor& q, const torch::Tensor& k,
-                  const torch::Tensor& v, FaArgs& a, hipStream_t stream) {
+                  const torch::Tensor& v, FaArgs& a, bool even, hipStream_t stream) {
     const int gq = a.Hq / a.Hkv;
     a.nqt = (int)(((long)gq * a.S + QROWS - 1) / QROWS);
     const size_t lds = 4 * KT * D * 2 + 8 * sizeof(int) + (KEYS == PAGES ? 2 * (KT + 1) * sizeof(int) : 0);
@@ -641,7 +641,7 @@ void flash_launch(torch::Tensor& out, const torch::Tensor& q, const torch::Tenso
     // 512 take the places that come free, longest first. Windows make rows alike (20.3 -> 20.6).
     constexpr int CUS = 256;
     const long heads = (long)a.B * a.Hkv;
-    a.turned = !HILO && a.window == 0 && blocks > CUS && blocks <= 2 * CUS ? (int)(CUS / heads) : 0;
+    a.turned = !HILO && even && a.window == 0 && blocks > CUS && blocks <= 2 * CUS ? (int)(CUS / heads) : 0;
     TORCH_CHECK(blocks < (1l << 31), "flash attention: too many query rows");
     hipLaunchKernelGGL((flash_kernel<T, D, KEYS, HILO, FIRST>), dim3((unsigned)blocks), dim3(256), lds, stream,
                        (T*)out.data_ptr(), (const T*)q.data_ptr(), (const T*)k.data_ptr(),
@@ -696,20 +696,27 @@ void flash_run(torch::Tensor& out, const torch::Tensor& q, const torch::Tensor& 
     auto stream = at::hip::getCurrentHIPStream();
     const bool paged = a.block_table != nullptr, tiles = paged && a.block_size % KT == 0;
     const bool extend = a.positions != nullptr;
-    // Priority for prompts: between one and a half and two rounds of workgroups a CU's second place is
-    // filled all the way, and it pays as it does over a cache. Heads of 128, 768 workgroups (3072 tokens,
-    // 3 prompts of 1024) 92.5 -> 88.6 us and 42.4 -> 39.0, 880 118 -> 108, 1024 151 -> 142. 576 and 640 lose
-    // 2 and 4 %, 1256 to 1504 between +1 and -3; heads of 64 lose up to 6. (A kernel of its own: a
-    // branch around it in one kernel costs the others 1 to 3 %.)
+    // Packed prompts of several lengths: the grid counts the longest's tiles for each, and says neither
+    // how many workgroups have work nor which of them are long.
+    const bool even = !a.starts || q.size(0) == (long)a.B * a.S;
+    // Priority for prompts: between 1.4 and two rounds of workgroups a CU's second place is filled all the
+    // way, and it pays as it does over a cache, where rows are long. Heads of 128, one prompt of 2816, 2880,
+    // 2944, 3072, 3584, 4096 tokens (704 to 1024 workgroups) 81.1 / 82.0, 83.4 / 83.3, 86.5 / 85.3, 94.6 / 90.5,
+    // 126 / 115, 156 / 146 us; 3 of 940 and of 1300 40.3 / 37.8 and 61.0 / 58.1, 4 of 900 46.2 / 44.5, but 5 of
+    // 700 39.8 / 39.5, 6 of 600 37.8 / 38.3, 8 of 370 26.9 / 28.9, 12 of 250 25.7 / 26.2. Chunks of 512 and 2048
+    // keys 41.1 / 39.8 and 87.9 / 82.8 (4096 tokens); a window has short rows: of 512 38.1 / 39.2 (3 of 1024), of
+    // 1024 59.8 / 63.1 (2848 tokens). 576 and 640 workgroups lose 2 and 4 %, 1256 to 1504 between +1 and -3;
+    // heads of 64 up to 6. (A kernel of its own: a branch around it in one kernel costs the others 1 to 3 %.)
     const long groups = ((long)a.Hq / a.Hkv * a.S + QROWS - 1) / QROWS * a.B * a.Hkv;
-    const bool first = groups > 700 && groups <= 1024;
+    const bool first = even && groups >= 720 && groups <= 1024 && a.S >= 900 &&
+                       (a.window <= 0 || a.window >= a.S);
 #define FA_D(T, D)                                                                        \
     do {                                                                                  \
-        if (tiles) flash_launch<T, D, TILE_PAGES, true>(out, q, k, v, a, stream);         \
-        else if (paged) flash_launch<T, D, PAGES, true>(out, q, k, v, a, stream);         \
-        else if (extend) flash_launch<T, D, ROWS, true>(out, q, k, v, a, stream);         \
-        else if (D == 128 && first) flash_launch<T, 128, ROWS, false, true>(out, q, k, v, a, stream); \
-        else flash_launch<T, D, ROWS, false>(out, q, k, v, a, stream);                    \
+        if (tiles) flash_launch<T, D, TILE_PAGES, true>(out, q, k, v, a, even, stream);   \
+        else if (paged) flash_launch<T, D, PAGES, true>(out, q, k, v, a, even, stream);   \
+        else if (extend) flash_launch<T, D, ROWS, true>(out, q, k, v, a, even, stream);   \
+        else if (D == 128 && first) flash_launch<T, 128, ROWS, false, true>(out, q, k, v, a, even, stream); \
+        else flash_launch<T, D, ROWS, false>(out, q, k, v, a, even, stream);              \
     } while (0)
 #define FA_GO(T)                                                                          \
     do {                                                                                  \

@@ -1074,8 +1074,8 @@ def test_layers_are_asked_once_a_prompt(moe, monkeypatch):
                                           (3, 12, 3, 1791, 64), (100, 3, 3, 70, 64), (2, 8, 1, 2060, 128),
                                           (3, 32, 8, 1001, 128), (11, 32, 8, 255, 128)])
 def test_prompts_of_one_round_of_workgroups(B, Hq, Hkv, S, D):
-    """256 workgroups, 264, 512, 504 of 9 heads, more heads than CUs, 258 of 2 heads, and 768 and 704, of
-    waves with priority: every row of the prompts, against 32-bit products: the result's rounding (2^-9) and as much for P's 16 bits."""
+    """256 workgroups, 264, 512, 504 of 9 heads, more heads than CUs, 258 of 2 heads, 768 of waves with
+    priority and 704 of short rows without: every row of the prompts, against 32-bit products: the result's rounding (2^-9) and as much for P's 16 bits."""
     g = torch.Generator(device="cuda").manual_seed(S)
     q, k, v = (torch.randn(B, h, S, D, device="cuda", generator=g).bfloat16() for h in (Hq, Hkv, Hkv))
     out = torch.full_like(q, float("nan"))
@@ -1169,3 +1169,28 @@ def test_gate_of_windowed_portions_is_the_plain_sigmoid():
     want = (1 / (1 + torch.exp(-gate.float()))).bfloat16()
     same = (got == want) | (got.isnan() & want.isnan())
     assert same.all(), (int((~same).sum()), gate[~same][:8], got[~same][:8], want[~same][:8])
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,lens", [
+    (32, 8, 128, (1001, 1001, 1001)), (32, 8, 128, (1001, 33, 700)), (8, 2, 128, (1100, 1100)),
+    (32, 8, 64, (256, 256, 1, 255)), (32, 8, 128, (400,) + (40,) * 9), (16, 4, 128, (901, 900, 3, 128, 129))])
+@pytest.mark.parametrize("window", [0, 300, -256])
+def test_packed_prompts_of_any_lengths(Hq, Hkv, D, lens, window):
+    """Prompts without padding, of one length (where the order and the priority of workgroups are those of
+    padded ones) and of several: each as it is by itself, but for the order of 32-bit sums of one
+    tile, which is the same: bit for bit."""
+    g = torch.Generator(device="cuda").manual_seed(len(lens))
+    rows, B, S = sum(lens), len(lens), max(lens)
+    q = torch.randn(rows, Hq, 1, D, device="cuda", generator=g).bfloat16()
+    kc, vc = (torch.randn(B + 2, Hkv, S + 5, D, device="cuda", generator=g).bfloat16() for _ in range(2))
+    sid = torch.randperm(B + 2, device="cuda", generator=g)[:B].to(torch.int32)
+    starts = torch.tensor((0,) + lens, device="cuda").cumsum(0).to(torch.int32)
+    out = torch.full_like(q, float("nan"))
+    ops._C.flash_prefill_packed(out, q, kc, vc, sid, starts, S, D ** -0.5, window)
+    at = 0
+    for b, n in enumerate(lens):
+        one = q[at:at + n, :, 0].transpose(0, 1).unsqueeze(0).contiguous()
+        want = torch.empty_like(one)
+        ops._C.flash_prefill_cached(want, one, kc, vc, sid[b:b + 1], D ** -0.5, window, None)
+        assert torch.equal(out[at:at + n, :, 0].transpose(0, 1), want[0]), (b, n)
+        at += n
