@@ -437,8 +437,15 @@ enum TgTile { T16, T16N, T32, T32N, T64, T64N, T64W, T128, T128N, T128W, T128B, 
 
 struct TgPlan {
     TgTile tile;
-    int bm, bn, splits;
+    int bm, bn, splits, tiles;
 };
+
+// parts of K that are worth their sum, see below
+long tg_parts(long M, long K, long tiles, bool whole) {
+    const bool small = whole ? M > 64 && M <= 128 && K >= 512 : true;
+    if (small && K <= 768 && tiles * (K / 128) <= (M <= 16 ? 128 : 64)) return K / 128;
+    return std::min(16L, std::max(std::min(8L, K / 256), K / 384));
+}
 
 // What is not taken (splits == 0) goes to the library. Times of 16-bit products on weights that
 // are not in a cache, 32-bit parts left to the next kernel, here / library (or the kernels with a
@@ -458,7 +465,12 @@ struct TgPlan {
 // that adds up, with 2 chunks or more / so: 93 rows (2048, 2048) 15.2 / 12.9 us, 128 rows
 // (1024, 2048) 14.2 / 12.2, 64 rows (1024, 3072) 9.9 / 9.4, 256 rows (1024, 1024) 13.1 / 10.9,
 // 1 row (2048, 1024) 6.5 / 6.0; 128 rows (1024, 4096) in 16 / 10 / 8 parts 15.5 / 14.4 / 14.6,
-// 256 rows 15.0 / 14.5 / 16.0.
+// 256 rows 15.0 / 14.5 / 16.0. A K of up to 768 in parts of 2 chunks, where these are at most 64 workgroups
+// (128 for up to 16 rows): parts of 2 / of 4, 1 row (2048, 512) 5.4 / 5.7 us, (1024, 256) 5.1 / 5.5, 93 rows (512, 256) 7.7 / 8.7, (1024, 512) 8.6 / 9.3,
+// (768, 768) 9.2 / 9.7, 64 rows (1024, 512) 6.7 / 6.9; with more of them 93 rows (4096, 512) 11.4 / 10.9, 400
+// (1024, 512) 11.6 / 11.1, (2048, 256) 12.0 / 10.4, 48 (768, 768) even, and of K 64 (512, 1024) 7.5 / 6.9. Where the sum is a launch of
+// its own, below, of a K from 512 on and for 65 to 128 rows: 93 (512, 512) 7.8 / 8.2, (2048, 512) 8.4 / 9.0; else
+// 48 (512, 512) 5.8 / 5.6, 1 (768, 768) 5.4 / 5.0, and one part 93 (512, 256) 7.1 / 6.2, 1 (1024, 256) 4.4 / 3.2.
 // From 128 rows on what bounds them is what a CU takes in, x and w together: 40 to 43 GB/s in every
 // tile tried (chunks of x laid out in a row changed nothing, deeper rings of either no more), so a
 // tile of 192 rows, which reads w once for them, and x apart from w in time: 129 to 192 rows
@@ -505,7 +517,8 @@ TgPlan tg_plan(long M, long N, long K, bool glu, bool whole) {
     const long tiles = (M + p.bm - 1) / p.bm * ((N + p.bn - 1) / p.bn);
     if (M > 128 && tiles > 256) return p;
     if (M > 256 && (tiles > 128 || glu)) return p;
-    p.splits = glu ? 1 : (int)std::max(1L, std::min({256 / tiles, std::max(std::min(8L, K / 256), K / 384), 16L}));
+    p.tiles = (int)tiles;
+    p.splits = glu ? 1 : (int)std::max(1L, std::min(256 / tiles, tg_parts(M, K, tiles, whole)));
     return p;
 }
 

@@ -845,3 +845,19 @@ def test_delta_rule_keeps_a_gigabyte_at_most(monkeypatch):
             assert got % (4 * floats) == 0 and got >= 4 * floats
             assert got == 4 * floats * units or got <= max(limit, 4 * floats) < got + 4 * floats
             assert got <= max(limit, 4 * floats)
+
+
+@pytest.mark.parametrize("M,N,K,parts,whole", [
+    (93, 512, 256, 2, 1), (1, 1024, 256, 2, 1), (400, 2048, 256, 1, 1), (93, 1024, 512, 4, 4),
+    (48, 1024, 512, 4, 2), (93, 4096, 512, 2, 2), (1, 2048, 512, 4, 2), (93, 768, 768, 6, 6),
+    (128, 1024, 640, 5, 5), (48, 768, 768, 3, 3), (16, 512, 128, 0, 1), (64, 512, 1024, 4, 4),
+    (128, 1024, 2048, 8, 8), (128, 2048, 2048, 8, 8), (64, 1024, 4096, 10, 10), (256, 4096, 4096, 4, 4)])
+def test_parts_of_products(M, N, K, parts, whole):
+    """Parts of K that a product is planned in, where the next kernel adds them up and where nobody does:
+    the faster of both sides of each line."""
+    from neuronx_distributed_inference_amd import ops
+
+    if not ops.extension_available():
+        pytest.skip("extension not built")
+    assert ops._C.tile_gemm_splits(M, N, K, 0, False) == parts
+    assert ops._C.tile_gemm_splits(M, N, K, 0, True) == whole
