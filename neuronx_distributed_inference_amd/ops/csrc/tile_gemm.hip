@@ -657,7 +657,11 @@ torch::Tensor tile_gemm_pair(torch::Tensor x, torch::Tensor w, torch::Tensor x2,
     a.N = w.size(0);
     const TgPlan plan = tg_plan(a.M, a.N, a.K, false, false);
     TORCH_CHECK(plan.splits > 0, "tile_gemm_pair: shape not taken");
-    a.splits = std::max(1, plan.splits / 2);
+    // the two fill the CUs together; 4 parts each where K has 4 chunks for each, and from there on half as
+    // many as one product takes (product and the norm that adds up, 2 / 4 parts each of K 1024: 16 rows
+    // (512, 1024) 8.0 / 6.9 us, 100 rows (1024, 1024) 12.9 / 11.5; 4 / 8 of K 2048: 100 rows (2048, 2048)
+    // 16.3 / 19.0, 48 rows (1024, 2048) 9.6 / 10.3)
+    a.splits = (int)std::max(1L, std::min(128L / plan.tiles, std::max(std::min(4L, (long)a.K / 256), tg_parts(a.M, a.K, 256, false) / 2)));
     torch::Tensor part = torch::empty({2 * a.splits, a.M, a.N}, x.options().dtype(torch::kFloat32));
     a.part = part.data_ptr<float>();
     a.x = x.data_ptr();

@@ -411,3 +411,18 @@ def test_delta_rule_where_memory_is_short(monkeypatch):
     assert want[2] > 200 << 20 and got[2] == captured[2] <= 128 << 20
     for other in (got, captured):
         assert torch.equal(other[0], want[0]) and torch.equal(other[1], want[1])
+
+
+@pytest.mark.parametrize("M,N,K,parts", [
+    (16, 512, 256, 1), (16, 512, 512, 2), (1, 512, 1024, 4), (100, 1024, 1024, 4), (48, 1536, 1536, 4),
+    (48, 1024, 2048, 4), (100, 2048, 2048, 4), (100, 2048, 4096, 5), (48, 4096, 2048, 2), (64, 16384, 512, 1)])
+def test_parts_of_pairs_of_products(M, N, K, parts):
+    """Parts that two products are taken in together, at both ends of what limits them, and their sums."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x, w, x2, w2 = (torch.empty(*s, device="cuda").normal_(0, 1, generator=g).to(BF)
+                    for s in ((M, K), (N, K)) * 2)
+    got = ops._C.tile_gemm_pair(x, w, x2, w2)
+    assert got.shape == (2 * parts, M, N)
+    for y, a, b in ((got[:parts], x, w), (got[parts:], x2, w2)):
+        limit = K * 2.0 ** -24 * (a.to(F64).abs() @ b.to(F64).abs().t())
+        assert ((y.to(F64).sum(0) - a.to(F64) @ b.to(F64).t()).abs() <= limit + 1e-30).all()
