@@ -1103,10 +1103,12 @@ def test_paged_rows_are_written(N, G, Dk, Dv, off, values, dtype):
     k, v = rows[:, off:off + G * Dk], rows[:, off + G * Dk:off + G * (Dk + Dv)]
     kc, vc = (torch.randn(N // 16 + 2, 16, G, d, device="cuda", generator=g).to(dtype) for d in (Dk, Dv))
     slots = torch.randperm(kc.shape[0] * 16, device="cuda", generator=g)[:N].to(torch.int32)
-    slots[N // 2::3] = -1
-    slots[N // 3:N // 3 + 1] = kc.shape[0] * 16
+    if N > 2:                                        # (a token alone has one)
+        slots[N // 2::3] = -1
+        slots[N // 3:N // 3 + 1] = kc.shape[0] * 16
     want = kc.clone(), vc.clone()
     there = (slots >= 0) & (slots < kc.shape[0] * 16)
+    assert there.any()
     for c, x, d in zip(want, (k, v), (Dk, Dv)):
         if d:
             c.view(-1, G * d)[slots[there].long()] = x[there]
