@@ -2110,6 +2110,9 @@ def test_attention_decode_values_not_finite(D, gq, dtype, Sq, window, kind):
 def test_gated_delta_blocks(S, D, Dv, H, G, per_head, dtype, room, monkeypatch):
     """Blocks of 64 tokens at their edges and at those of the groups of 4 and 16 in them, value channels
     above the 128 that a workgroup norms, one row's block at a time and all at once."""
+    from neuronx_distributed_inference_amd.ops import seqmix
+
+    monkeypatch.setattr(seqmix, "delta_unit_tokens", lambda *a: 64)
     test_gated_delta_chunks(S, D, Dv, H, G, per_head, dtype, "one" if room == "row" else "all", monkeypatch)
 
 
