@@ -465,12 +465,14 @@ long tg_parts(long M, long K, long tiles, bool whole) {
 // that adds up, with 2 chunks or more / so: 93 rows (2048, 2048) 15.2 / 12.9 us, 128 rows
 // (1024, 2048) 14.2 / 12.2, 64 rows (1024, 3072) 9.9 / 9.4, 256 rows (1024, 1024) 13.1 / 10.9,
 // 1 row (2048, 1024) 6.5 / 6.0; 128 rows (1024, 4096) in 16 / 10 / 8 parts 15.5 / 14.4 / 14.6,
-// 256 rows 15.0 / 14.5 / 16.0. A K of up to 768 in parts of 2 chunks, where these are at most 64 workgroups
-// (128 for up to 16 rows): parts of 2 / of 4, 1 row (2048, 512) 5.4 / 5.7 us, (1024, 256) 5.1 / 5.5, 93 rows (512, 256) 7.7 / 8.7, (1024, 512) 8.6 / 9.3,
-// (768, 768) 9.2 / 9.7, 64 rows (1024, 512) 6.7 / 6.9; with more of them 93 rows (4096, 512) 11.4 / 10.9, 400
-// (1024, 512) 11.6 / 11.1, (2048, 256) 12.0 / 10.4, 48 (768, 768) even, and of K 64 (512, 1024) 7.5 / 6.9. Where the sum is a launch of
-// its own, below, of a K from 512 on and for 65 to 128 rows: 93 (512, 512) 7.8 / 8.2, (2048, 512) 8.4 / 9.0; else
-// 48 (512, 512) 5.8 / 5.6, 1 (768, 768) 5.4 / 5.0, and one part 93 (512, 256) 7.1 / 6.2, 1 (1024, 256) 4.4 / 3.2.
+// 256 rows 15.0 / 14.5 / 16.0. A K of up to 768 in parts of 2 chunks, where these are at most 64
+// workgroups (128 for up to 16 rows): parts of 2 / of 4, 1 row (2048, 512) 5.4 / 5.7 us, (1024, 256)
+// 5.1 / 5.5, 93 rows (512, 256) 7.7 / 8.7, (1024, 512) 8.6 / 9.3, (768, 768) 9.2 / 9.7, 64 rows (1024, 512)
+// 6.7 / 6.9; with more of them 93 rows (4096, 512) 11.4 / 10.9, 400 (1024, 512) 11.6 / 11.1, (2048, 256)
+// 12.0 / 10.4, 48 (768, 768) even, and of a longer K 64 (512, 1024) 7.5 / 6.9. Where the sum is a launch of its
+// own, see below, only of a K from 512 on and for 65 to 128 rows: 93 (512, 512) 7.8 / 8.2, (2048, 512)
+// 8.4 / 9.0; else 48 (512, 512) 5.8 / 5.6, 1 (768, 768) 5.4 / 5.0, and 2 parts / one 93 (512, 256) 7.1 / 6.2,
+// 1 (1024, 256) 4.4 / 3.2.
 // From 128 rows on what bounds them is what a CU takes in, x and w together: 40 to 43 GB/s in every
 // tile tried (chunks of x laid out in a row changed nothing, deeper rings of either no more), so a
 // tile of 192 rows, which reads w once for them, and x apart from w in time: 129 to 192 rows
@@ -661,7 +663,8 @@ torch::Tensor tile_gemm_pair(torch::Tensor x, torch::Tensor w, torch::Tensor x2,
     // many as one product takes (product and the norm that adds up, 2 / 4 parts each of K 1024: 16 rows
     // (512, 1024) 8.0 / 6.9 us, 100 rows (1024, 1024) 12.9 / 11.5; 4 / 8 of K 2048: 100 rows (2048, 2048)
     // 16.3 / 19.0, 48 rows (1024, 2048) 9.6 / 10.3)
-    a.splits = (int)std::max(1L, std::min(128L / plan.tiles, std::max(std::min(4L, (long)a.K / 256), tg_parts(a.M, a.K, 256, false) / 2)));
+    const long worth = std::max(std::min(4L, (long)a.K / 256), tg_parts(a.M, a.K, 256, false) / 2);
+    a.splits = (int)std::max(1L, std::min(128L / plan.tiles, worth));
     torch::Tensor part = torch::empty({2 * a.splits, a.M, a.N}, x.options().dtype(torch::kFloat32));
     a.part = part.data_ptr<float>();
     a.x = x.data_ptr();
